@@ -19,8 +19,8 @@ PROBE_LIB = os.path.join(HERE, 'libmbx_probe.so')
 # the library with per-tile time stamps in the grouped-GEMM kernels (csrc/gmm_dma.h, MBX_TICKS), for bench.py --tile-ticks
 TICKS_LIB = os.path.join(HERE, 'libmbx_ticks.so')
 PROBE_SOURCE = 'probe.hip'
-SOURCES = ['routing.hip', 'permute.hip', 'gmm.hip', 'elementwise.hip', 'router.hip']
-HEADERS = [os.path.join(CSRC, 'common.h'), os.path.join(CSRC, 'gmm_dma.h'),
+SOURCES = ['routing.hip', 'permute.hip', 'gmm.hip', 'gmm_f32.hip', 'elementwise.hip', 'router.hip']
+HEADERS = [os.path.join(CSRC, 'common.h'), os.path.join(CSRC, 'gmm_dma.h'), os.path.join(CSRC, 'gmm_common.h'),
            os.path.join(os.path.dirname(HERE), 'include', 'mbx.h'), os.path.join(os.path.dirname(HERE), 'include', 'mbx_probe.h')]
 ARCH = 'gfx950'
 # -packed-fp32-ops is switched off: hipcc must not form v_pk_*_f32 from scalar float code.

@@ -13,16 +13,13 @@
 // values of its column.  The tile -> (expert, row tile) schedule is computed on the device
 // from the inclusive row bins, so no host copy of the group sizes is needed and empty
 // experts cost nothing (NN/NT) or produce an all-zero block (TN).
-#include "common.h"
+#include "gmm_common.h"
 
 #include <cstdlib>
 
 namespace mbx {
 namespace {
 
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
 typedef short s16x4_t __attribute__((ext_vector_type(4)));
@@ -34,8 +31,6 @@ __device__ __forceinline__ f32x16 mfma32(const u32x4& a, const u32x4& b, const f
   else
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8_t, a), __builtin_bit_cast(f16x8_t, b), c, 0, 0, 0);
 }
-
-typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 template <int DT>
 __device__ __forceinline__ f32x4 mfma16(const u32x4& a, const u32x4& b, const f32x4& c) {
@@ -145,17 +140,6 @@ __device__ __forceinline__ u32x4 read_frag(const uint16_t* lds, int r, int ks) {
   }
 }
 
-typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
-typedef float f32x2_t __attribute__((ext_vector_type(2)));
-
-template <int DT>
-__device__ __forceinline__ uint32_t pack2(float a, float b) {
-  const f32x2_t v = {a, b};
-  if (DT == MBX_BF16) return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2_t));  // v_cvt_pk_bf16_f32, RNE
-  return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, f16x2_t));
-}
-
 // The workgroup-level product: acc += A_tile(k) * B_tile(k) over k in [k_begin, k_end),
 // then c[m0.., n0..] = acc for rows < m_lim and columns < n_lim.
 template <int DT, bool A_MC, bool B_MC, typename T>
@@ -263,27 +247,6 @@ __device__ __forceinline__ void block_gemm(const Operand& opa, const Operand& op
   }
 }
 
-// Workgroups are dispatched to the 8 XCDs round-robin by workgroup id, and every XCD has its own
-// L2.  The logical tile order is cut into runs of kXcdRun tiles and run r goes to XCD r % 8, so
-// the workgroups resident on one XCD at a time form a compact block of tiles (same expert, a few
-// row tiles x a few column tiles) whose operand panels are fetched into that L2 once.
-constexpr int kXcds = 8;
-constexpr int kXcdRun = 32;
-
-__device__ __forceinline__ int xcd_tile_id(int block, int run = kXcdRun) {
-  const int xcd = block % kXcds, l = block / kXcds;
-  return ((l / run) * kXcds + xcd) * run + (l % run);
-}
-
-static inline int64_t xcd_grid(int64_t tiles, int run = kXcdRun) {
-  const int64_t q = (int64_t)kXcds * run;
-  return (tiles + q - 1) / q * q;
-}
-
-// A row bound read from the bins, kept inside [lo, rows]: a table that does not belong to the operands can make
-// the result wrong but never an access out of range.
-__device__ __forceinline__ int clamp_bound(int v, int lo, int rows) { return v < lo ? lo : (v > rows ? rows : v); }
-
 // ---- NN / NT: row tiles follow the expert bins --------------------------------------
 // Logical tile id -> (expert, column tile, row tile inside the expert), row tiles fastest.
 template <int DT, bool B_MC, typename T>
@@ -334,6 +297,7 @@ gmm_tn_kernel(const uint16_t* __restrict__ a, const uint16_t* __restrict__ b, ui
 #include "gmm_dma.h"
 
 // ---- any shape, any alignment, fp32 included ------------------------------------------
+// (fp32 operands of whole 16-byte pieces go to gmm_f32.hip.)
 // c(m, n) = sum_r a(m, r) b(r, n) with element-wise addressing and bounds checks, the products and sums
 // in fp32 on the matrix cores (v_mfma_f32_32x32x2_f32 is an IEEE fp32 multiply-add; 16-bit inputs are
 // widened exactly).  128 x 128 tile per workgroup, four waves of 64 x 64, K tiles of 16 staged through a
@@ -502,11 +466,6 @@ constexpr size_t lds_bytes() {
          (size_t)(OperandLds<A_MC, T::BM, T::BK, T::PAD_KC, T::PAD_MC>::ELEMS + OperandLds<B_MC, T::BN, T::BK, T::PAD_KC, T::PAD_MC>::ELEMS);
 }
 
-template <typename K>
-int allow_lds(K kernel, size_t bytes) {
-  return (int)hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
-}
-
 template <int DT, typename T>
 int gmm_mfma(const void* a, const void* b, void* c, const int32_t* bins, int num_groups, int64_t rows, int k, int n,
              int layout, hipStream_t s) {
@@ -544,21 +503,6 @@ int gmm_mfma(const void* a, const void* b, void* c, const int32_t* bins, int num
   return launch_status();
 }
 
-// One persistent workgroup per compute unit (a multiple of 8, so that every XCD gets the same number),
-// fewer when there are not that many tiles.
-static inline int persistent_grid(int64_t tiles_upper_bound) {
-  static int cus[64];
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = 0;
-  if (cus[dev] == 0) {
-    int n = 0;
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n < kXcds) n = 256;
-    cus[dev] = n / kXcds * kXcds;
-  }
-  const int64_t need = (tiles_upper_bound + kXcds - 1) / kXcds * kXcds;
-  return (int)(need < cus[dev] ? need : cus[dev]);
-}
-
 // Launch of the direct-to-LDS kernels (k a multiple of 64 for NN / NT; sizes as dma_sizes_ok() allows).
 // TS is the tile the tail of an NN / NT launch is cut into (TS = T: never cut).
 // a2 / b2 non-null (NN / NT only): c = a @ b[e] + a2 @ b2[e], the second pair shaped like the first.
@@ -574,12 +518,6 @@ struct CombineRows {
   int tokens = 0;
 };
 
-// kWorkspaceCounters int32 counters, zero before the launch and zero again after it, then room for fp32 tiles.
-constexpr size_t kWorkspaceCounters = 1024, kWorkspacePartBytes = (size_t)256 * 256 * 4, kWorkspaceParts = 320;
-struct Workspace {
-  void* base = nullptr;
-  size_t bytes = 0;
-};
 struct GatherRows {
   const int32_t* slots = nullptr;      // non-null: a (NT) / b (TN) is [src_rows, .], read through the row map
   const int32_t* src_bins = nullptr;
@@ -672,17 +610,10 @@ int gmm_dma(const void* a, const void* b, void* c, const int32_t* bins, int num_
   uint32_t gather_magic = 0;
   int gather_shift = 0;
   if (gather.slots) dma::gather_divisor(gather.top_k, gather_magic, gather_shift);
-  // the workspace as the kernel takes it: counters, parts (16-byte aligned), how many parts of a T tile fit
-  int32_t* ws_counters = nullptr;
-  float* ws_parts = nullptr;
-  int ws_capacity = 0;
-  if (ws.base && ((uintptr_t)ws.base & 15u) == 0 && ws.bytes > kWorkspaceCounters * sizeof(int32_t) && (int)grid / 2 <= (int)kWorkspaceCounters) {
-    ws_counters = (int32_t*)ws.base;
-    ws_parts = (float*)((char*)ws.base + kWorkspaceCounters * sizeof(int32_t));
-    const size_t fit = (ws.bytes - kWorkspaceCounters * sizeof(int32_t)) / ((size_t)T::BM * T::BN * sizeof(float));
-    ws_capacity = (int)(fit > 0x7fffffff ? 0x7fffffff : fit);
-    if (ws_capacity < 2) ws_parts = nullptr;
-  }
+  const WorkspaceParts lent(ws, (size_t)T::BM * T::BN * sizeof(float));
+  int32_t* const ws_counters = lent.counters;
+  float* const ws_parts = (int)grid / 2 <= (int)kWorkspaceCounters ? lent.parts : nullptr;
+  const int ws_capacity = lent.capacity;
 #define MBX_LAUNCH_ROWS_G(B_MC, DUAL, EPI, GATHER)                                                    \
   do {                                                                                                \
     auto kern = dma::gmm_rows_kernel<DT, B_MC, T, TS, DUAL, EPI, GATHER>;                             \
@@ -759,8 +690,6 @@ int gmm_generic(const void* a, const void* b, void* c, const int32_t* bins, int 
   gmm_generic_kernel<DT><<<dim3((unsigned)gx, (unsigned)gy, (unsigned)num_groups), 256, 0, s>>>(a, b, c, bins, layout, (int)rows, k, n);
   return launch_status();
 }
-
-static inline bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
 
 // The direct-to-LDS kernels address with 32-bit byte offsets from a base they set per tile (the tile's first
 // row of a and c in NN / NT), per expert (its weights; its [k, n] product in TN) or per segment of an
@@ -843,6 +772,10 @@ static int gmm_ws(const void* a, const void* b, void* c, int dtype, const int32_
     if (dtype == MBX_BF16) return gmm_mfma<MBX_BF16, TileBig>(a, b, c, bins, num_groups, rows, k, n, layout, s);
     return gmm_mfma<MBX_F16, TileBig>(a, b, c, bins, num_groups, rows, k, n, layout, s);
   }
+  if (dtype == MBX_F32) {
+    const int rc = gmm_f32(a, b, nullptr, nullptr, c, bins, num_groups, rows, k, n, layout, ws.base, ws.bytes, s);
+    if (rc != MBX_EUNSUPPORTED) return rc;
+  }
   switch (dtype) {
     case MBX_BF16: return gmm_generic<MBX_BF16>(a, b, c, bins, num_groups, rows, k, n, layout, s);
     case MBX_F16: return gmm_generic<MBX_F16>(a, b, c, bins, num_groups, rows, k, n, layout, s);
@@ -879,6 +812,7 @@ static int gmm_dual_ws(const void* a, const void* b, const void* a2, const void*
   if (num_groups == 0 || rows == 0 || n == 0) return 0;
   if (!bins || !c || (k > 0 && (!a || !b || !a2 || !b2))) return MBX_EINVAL;
   if (rows > 0x7fffffff) return MBX_ERANGE;
+  if (dtype == MBX_F32) return gmm_f32(a, b, a2, b2, c, bins, num_groups, rows, k, n, layout, ws.base, ws.bytes, as_stream(stream));
   // only the direct-to-LDS kernels reduce over two operand pairs: whole K tiles, at least four per pair
   const bool ok = dtype != MBX_F32 && aligned16(a) && aligned16(b) && aligned16(a2) && aligned16(b2) && aligned16(c) &&
                   k % TileDma::BK == 0 && k >= 4 * TileDma::BK && n % 8 == 0 && dma_sizes_ok(k, n);

@@ -1,0 +1,98 @@
+// What the translation units of the grouped GEMM share: vector types, the mapping of tiles to XCDs, the workspace a
+// caller lends, launch helpers.
+#pragma once
+
+#include "common.h"
+
+namespace mbx {
+namespace {
+
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
+typedef float f32x2_t __attribute__((ext_vector_type(2)));
+
+template <int DT>
+__device__ __forceinline__ uint32_t pack2(float a, float b) {
+  const f32x2_t v = {a, b};
+  if (DT == MBX_BF16) return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2_t));  // v_cvt_pk_bf16_f32, RNE
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, f16x2_t));
+}
+
+// Workgroups are dispatched to the 8 XCDs round-robin by workgroup id, and every XCD has its own
+// L2.  The logical tile order is cut into runs of kXcdRun tiles and run r goes to XCD r % 8, so
+// the workgroups resident on one XCD at a time form a compact block of tiles (same expert, a few
+// row tiles x a few column tiles) whose operand panels are fetched into that L2 once.
+constexpr int kXcds = 8;
+constexpr int kXcdRun = 32;
+
+__device__ __forceinline__ int xcd_tile_id(int block, int run = kXcdRun) {
+  const int xcd = block % kXcds, l = block / kXcds;
+  return ((l / run) * kXcds + xcd) * run + (l % run);
+}
+
+static inline int64_t xcd_grid(int64_t tiles, int run = kXcdRun) {
+  const int64_t q = (int64_t)kXcds * run;
+  return (tiles + q - 1) / q * q;
+}
+
+// A row bound read from the bins, kept inside [lo, rows]: a table that does not belong to the operands can make
+// the result wrong but never an access out of range.
+__device__ __forceinline__ int clamp_bound(int v, int lo, int rows) { return v < lo ? lo : (v > rows ? rows : v); }
+
+// kWorkspaceCounters int32 counters, zero before the launch and zero again after it, then room for fp32 tiles.
+constexpr size_t kWorkspaceCounters = 1024, kWorkspacePartBytes = (size_t)256 * 256 * 4, kWorkspaceParts = 320;
+struct Workspace {
+  void* base = nullptr;
+  size_t bytes = 0;
+};
+// The workspace as the kernels take it: counters, then parts of `part_bytes` each, 16-byte aligned; parts null where it
+// cannot hold two.
+struct WorkspaceParts {
+  int32_t* counters = nullptr;
+  float* parts = nullptr;
+  int capacity = 0;
+  WorkspaceParts(const Workspace& ws, size_t part_bytes) {
+    const size_t head = kWorkspaceCounters * sizeof(int32_t);
+    if (!ws.base || ((uintptr_t)ws.base & 15u) != 0 || ws.bytes < head + 2 * part_bytes) return;
+    const size_t fit = (ws.bytes - head) / part_bytes;
+    counters = (int32_t*)ws.base;
+    parts = (float*)((char*)ws.base + head);
+    capacity = (int)(fit > 0x7fffffff ? 0x7fffffff : fit);
+  }
+};
+
+static inline bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
+
+template <typename K>
+int allow_lds(K kernel, size_t bytes) {
+  return (int)hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+}
+
+// One persistent workgroup per compute unit (a multiple of 8, so that every XCD gets the same number),
+// fewer when there are not that many tiles.
+static inline int persistent_grid(int64_t tiles_upper_bound) {
+  static int cus[64];
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = 0;
+  if (cus[dev] == 0) {
+    int n = 0;
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n < kXcds) n = 256;
+    cus[dev] = n / kXcds * kXcds;
+  }
+  const int64_t need = (tiles_upper_bound + kXcds - 1) / kXcds * kXcds;
+  return (int)(need < cus[dev] ? need : cus[dev]);
+}
+
+}  // namespace
+
+// gmm_f32.hip: fp32 products of whole 16-byte pieces; MBX_EUNSUPPORTED where the operands are not.  a2 / b2 non-null
+// (NN / NT): c = a @ b[e] + a2 @ b2[e].
+int gmm_f32(const void* a, const void* b, const void* a2, const void* b2, void* c, const int32_t* bins, int num_groups,
+            int64_t rows, int k, int n, int layout, void* workspace, size_t workspace_bytes, hipStream_t s);
+
+}  // namespace mbx

@@ -891,3 +891,54 @@ def test_gmm_on_gathered_rows_with_assignments_out_of_range(gg):
     assert gg.gmm_gather(gg.GatheredRows(x[:, :72].contiguous(), indices, bin_ids, bins, None, top_k, tokens * top_k),
                          w1[:, :, :72].contiguous(), tpe) is None
     assert gg.gmm_gather(gg.GatheredRows(x, indices.long(), bin_ids, bins, None, top_k, tokens * top_k), w1, tpe) is None
+
+
+@pytest.mark.parametrize('groups,rows,k,n', [
+    (4, 1000, 36, 132),      # K tail of one 16-byte piece, a column tile of one piece
+    (3, 65 * 3, 32, 4),      # one K tile, the narrowest output; experts around the 64-row tile
+    (8, 8 * 129, 260, 260),  # experts around the full tile
+    (1, 300, 2052, 128),     # a handful of tiles, long reduction: cut along K (with and without a workspace)
+    (2, 4100, 128, 384),     # TN: few tiles, long reduction
+    (70, 2000, 64, 128),     # several experts per lane of the tile lookup, unranked TN
+    (5, 40, 128, 4100),      # many column tiles, a few rows per expert
+])
+@pytest.mark.parametrize('mode', ['nn', 'nt', 'tn', 'dual_nn', 'dual_nt'])
+def test_gmm_fp32_on_the_matrix_cores(gg, monkeypatch, groups, rows, k, n, mode):
+    """The fp32 kernels against fp64.  Each of an output's r products and partial sums is rounded once, errors of random
+    sign: 2^-24 sqrt(r) relative to the terms' root sum square, with a factor of four to spare."""
+    torch.manual_seed(rows + k)
+    sizes = _sizes(groups, rows, seed=groups + rows, empty=(0,) if groups > 2 else ())
+    trans_b, dual = mode.endswith('nt'), mode.startswith('dual')
+    a, a2 = (torch.randn(rows, k, device='cuda') for _ in range(2))
+    wshape = (groups, n, k) if trans_b else (groups, k, n)
+    b, b2 = (torch.randn(rows, n, device='cuda') if mode == 'tn' else torch.randn(wshape, device='cuda') for _ in range(2))
+    # a row that must not leak into its neighbours: the pieces past the end of a row's reduction read as zeros
+    bad = rows // 2
+    if mode != 'tn':
+        a[bad] = float('inf')
+    ok = torch.arange(rows, device='cuda') != bad
+
+    def product(x, w):
+        outs, start = [], 0
+        for e, c in enumerate(sizes.tolist()):
+            xe = x[start:start + c].double()
+            outs.append(xe.t() @ w[start:start + c].double() if mode == 'tn' else
+                        xe @ (w[e].double().t() if trans_b else w[e].double()))
+            start += c
+        return torch.stack(outs) if mode == 'tn' else torch.cat(outs)
+
+    want = product(a, b) + (product(a2, b2) if dual else 0)
+    length = int(sizes.max()) if mode == 'tn' else k * (2 if dual else 1)
+    tol = 4 * 2.0 ** -24 * math.sqrt(max(length, 16))
+    got = []
+    for lend in (True, False):
+        monkeypatch.setattr(gg, 'GMM_WORKSPACE', lend)
+        for _ in range(2):
+            out = gg.gmm_dual(a, b, a2, b2, sizes, trans_b=trans_b) if dual else \
+                gg.backend.gmm(a, b, sizes, trans_a=mode == 'tn', trans_b=trans_b)
+            if mode == 'tn':
+                assert max_block_err(out, want) < tol
+            else:
+                assert max_block_err(out[ok], want[ok]) < tol and not bool(torch.isfinite(out[bad]).any())
+            got.append(out)
+        assert torch.equal(got[-1].nan_to_num(), got[-2].nan_to_num())
