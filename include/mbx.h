@@ -216,15 +216,15 @@ int mbx_gmm(const void* a, const void* b, void* c, int dtype, const int32_t* bin
  * (`gmm(dsdd_out, w1, c=dx); dx += gmm(dv1_out, v1)`), as one reduction over both operand pairs:
  *   MBX_NN: c[r_e] = a[r_e] @ b[e] + a2[r_e] @ b2[e]      MBX_NT: ... @ b[e]^T + ... @ b2[e]^T
  * with a2 / b2 shaped like a / b.  One rounding of the fp32 sum instead of the reference's three.
- * Handles bf16 / f16 with k a multiple of 64 and at least 256, 16-byte aligned operands (n a multiple
- * of 8 for MBX_NN), any number of rows, one expert's weights below 2 GiB; anything else returns MBX_EUNSUPPORTED and the caller issues the
+ * Handles bf16 / f16 with k a multiple of 8 above 192 and n of 8, fp32 with k and n multiples of 4, 16-byte aligned operands,
+ * any number of rows, one expert's weights below 2 GiB; anything else returns MBX_EUNSUPPORTED and the caller issues the
  * two mbx_gmm calls and the addition itself. */
 int mbx_gmm_dual(const void* a, const void* b, const void* a2, const void* b2, void* c, int dtype,
                  const int32_t* bins, int num_groups, int64_t rows, int k, int n, int layout,
                  mbx_stream_t stream);
 
 /* mbx_gmm (a2 == b2 == NULL) / mbx_gmm_dual with a workspace: device memory the launch may use to cut the tiles of its
- * last, partly filled round of workgroups along the reduction (MBX_NN with long reductions: a Mixtral-shaped second
+ * last, partly filled round of workgroups along the reduction (16-bit MBX_NN with long reductions, fp32: a Mixtral-shaped second
  * product has 4.25 rounds of tiles on 256 compute units, and the quarter round costs as much as a whole one).  Parts
  * of a tile are summed in a fixed order: results do not change from run to run, but differ in the last bits from
  * those of a launch without workspace.  grouped_gemm.backend.gmm allocates what it needs through torch; this library
@@ -242,7 +242,7 @@ int mbx_gmm_ws(const void* a, const void* b, const void* a2, const void* b2, voi
  *   c[r_e] = a[r_e] @ b[e]^T (b is [E, n, k]),   c_act = act(c)
  * where act is applied in the product's epilogue to c as stored (rounded to `dtype`), i.e. to the value the
  * reference's separate activation kernel reads.  Both outputs are [rows, n].  act: MBX_ACT_GELU_TANH.
- * MBX_EUNSUPPORTED (the caller runs mbx_gmm and the activation itself): fp32, another activation, k not a multiple of 64,
+ * MBX_EUNSUPPORTED (the caller runs mbx_gmm and the activation itself): fp32, another activation, k not a multiple of 8,
  * n not a multiple of 8, operands or outputs not 16-byte aligned, one expert's weights of 2 GiB or more. */
 int mbx_gmm_act(const void* a, const void* b, void* c, void* c_act, int dtype, const int32_t* bins,
                 int num_groups, int64_t rows, int k, int n, int act, mbx_stream_t stream);
@@ -293,7 +293,7 @@ int mbx_gmm_gather(const void* x, int64_t x_rows, const int32_t* indices, int to
  * for every row r of the product (rows == tokens * 1: the unpadded grouped layout).  indices: the sorted assignments
  * (int32 [rows]); weights: [tokens] of type w_dtype (an mbx_dtype).  The roundings are those of mbx_gmm followed by
  * mbx_scatter: the results are bit-identical.  A row whose assignment is outside [0, tokens) is not combined.  out rows
- * that no assignment names are left as they are.  MBX_EUNSUPPORTED: fp32, k not a multiple of 64, unaligned, an
+ * that no assignment names are left as they are.  MBX_EUNSUPPORTED: fp32, k not a multiple of 8, unaligned, an
  * expert's weights of 2 GiB or more -- multiply, then scatter. */
 int mbx_gmm_scatter(const void* a, const void* b, void* c, void* out, int dtype, const int32_t* bins, int num_groups,
                     int64_t rows, int k, int n, const int32_t* indices, const void* weights, int w_dtype, int64_t tokens,

@@ -19,8 +19,9 @@ PROBE_LIB = os.path.join(HERE, 'libmbx_probe.so')
 # the library with per-tile time stamps in the grouped-GEMM kernels (csrc/gmm_dma.h, MBX_TICKS), for bench.py --tile-ticks
 TICKS_LIB = os.path.join(HERE, 'libmbx_ticks.so')
 PROBE_SOURCE = 'probe.hip'
-SOURCES = ['routing.hip', 'permute.hip', 'gmm.hip', 'gmm_f32.hip', 'elementwise.hip', 'router.hip']
-HEADERS = [os.path.join(CSRC, 'common.h'), os.path.join(CSRC, 'gmm_dma.h'), os.path.join(CSRC, 'gmm_common.h'),
+SOURCES = ['routing.hip', 'permute.hip', 'gmm.hip', 'gmm_rows.hip', 'gmm_rows_tail.hip', 'gmm_f32.hip', 'elementwise.hip', 'router.hip']
+TICKS_SOURCES = ['gmm.hip', 'gmm_rows.hip', 'gmm_rows_tail.hip']
+HEADERS = [os.path.join(CSRC, 'common.h'), os.path.join(CSRC, 'gmm_dma.h'), os.path.join(CSRC, 'gmm_common.h'), os.path.join(CSRC, 'gmm_rows.h'),
            os.path.join(os.path.dirname(HERE), 'include', 'mbx.h'), os.path.join(os.path.dirname(HERE), 'include', 'mbx_probe.h')]
 ARCH = 'gfx950'
 # -packed-fp32-ops is switched off: hipcc must not form v_pk_*_f32 from scalar float code.
@@ -59,14 +60,16 @@ def build(force: bool = False, verbose: bool = False) -> str:
             if verbose:
                 print(' '.join(cmd), flush=True)
             procs.append((cmd, subprocess.Popen(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)))
-    # gmm.hip a second time with the time stamps compiled in
-    gmm_src, ticks_obj = os.path.join(CSRC, 'gmm.hip'), os.path.join(BUILD, 'gmm_ticks.o')
-    ticks_stale = force or not os.path.exists(ticks_obj) or os.path.getmtime(ticks_obj) < max(os.path.getmtime(gmm_src), newest_header)
-    if ticks_stale:
-        cmd = [hipcc] + FLAGS + ['-DMBX_TICKS', '-c', gmm_src, '-o', ticks_obj]
-        if verbose:
-            print(' '.join(cmd), flush=True)
-        procs.append((cmd, subprocess.Popen(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)))
+    # the 16-bit grouped-GEMM sources a second time with the time stamps compiled in
+    ticks_objs = {}
+    for src in TICKS_SOURCES:
+        s, o = os.path.join(CSRC, src), os.path.join(BUILD, src.replace('.hip', '_ticks.o'))
+        ticks_objs[os.path.join(BUILD, src.replace('.hip', '.o'))] = o
+        if force or not os.path.exists(o) or os.path.getmtime(o) < max(os.path.getmtime(s), newest_header):
+            cmd = [hipcc] + FLAGS + ['-DMBX_TICKS', '-c', s, '-o', o]
+            if verbose:
+                print(' '.join(cmd), flush=True)
+            procs.append((cmd, subprocess.Popen(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)))
     probe_src = os.path.join(CSRC, PROBE_SOURCE)
     probe_cmd = None
     if force or not os.path.exists(PROBE_LIB) or os.path.getmtime(PROBE_LIB) < max(os.path.getmtime(probe_src), newest_header):
@@ -81,7 +84,7 @@ def build(force: bool = False, verbose: bool = False) -> str:
     if [c for c, _ in procs if c is not probe_cmd] or force or not os.path.exists(LIB) or not os.path.exists(TICKS_LIB):
         _run([hipcc, '-shared', '-fPIC', f'--offload-arch={ARCH}', '-o', LIB] + objs)
         _run([hipcc, '-shared', '-fPIC', f'--offload-arch={ARCH}', '-o', TICKS_LIB] +
-             [ticks_obj if o.endswith(os.sep + 'gmm.o') else o for o in objs])
+             [ticks_objs.get(o, o) for o in objs])
     return LIB
 
 

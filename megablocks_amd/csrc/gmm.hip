@@ -453,13 +453,6 @@ __global__ void __launch_bounds__(256) gelu_backward_vec_kernel(void* __restrict
 // Tile shapes.  256x256x64 with four waves (2x2, 128x128 each) keeps the accumulators in
 // 256 registers per lane and needs 144 KiB of the 160 KiB LDS for two stages.
 typedef Tile<256, 256, 64, 2, 2, 8, 32> TileBig;
-// The tiles of the direct-to-LDS kernels (gmm_dma.h): 256 x 256 x 64, four waves of 128 x 128, three A and two B
-// stages of 32 KiB; and the half-height tile (NN / NT only: the row tile follows the expert's row count) for the last
-// row tile of an expert when it is at most half full, for the tail of a launch, and for launches of small experts;
-// its smaller stages allow a three-deep ring (4 x 16 KiB + 3 x 32 KiB).
-typedef dma::Tile<256, 256, 2, 2, 64, 2> TileDma;
-typedef dma::Tile<128, 256, 1, 4, 64, 3> TileDmaSmallM;
-
 template <int DT, bool A_MC, bool B_MC, typename T>
 constexpr size_t lds_bytes() {
   return 2 * sizeof(uint16_t) *
@@ -503,180 +496,79 @@ int gmm_mfma(const void* a, const void* b, void* c, const int32_t* bins, int num
   return launch_status();
 }
 
-// Launch of the direct-to-LDS kernels (k a multiple of 64 for NN / NT; sizes as dma_sizes_ok() allows).
-// TS is the tile the tail of an NN / NT launch is cut into (TS = T: never cut).
-// a2 / b2 non-null (NN / NT only): c = a @ b[e] + a2 @ b2[e], the second pair shaped like the first.
-// epi / extra (NT, one operand pair only): dma::kEpiAct with the second output, dma::kEpiDact with the second input.
-// Rows of `a` gathered on the fly (NT; no epilogue, kEpiAct or kEpiGlu*): see GatherRows.
-// Device memory a launch may use for the parts of tiles it cuts along the reduction (gmm_rows_kernel's split-K tail):
-// The weighted combine in the epilogue (kEpiCombine): the sorted assignments (top_k = 1: tokens) of the product's rows,
-// the weights by token (or null) and their type, the row count of the combined output.
-struct CombineRows {
-  const int32_t* indices = nullptr;
-  const void* weights = nullptr;
-  int w_dtype = 0;
-  int tokens = 0;
-};
-
-struct GatherRows {
-  const int32_t* slots = nullptr;      // non-null: a (NT) / b (TN) is [src_rows, .], read through the row map
-  const int32_t* src_bins = nullptr;
-  int top_k = 1, src_rows = 0;
-  // TN only: the table of row offsets the kernel reads (4 bytes per sorted assignment, n_slots of them), and whether an
-  // earlier call with the same slots, top_k, src_rows and n has already filled it
-  uint32_t* row_table = nullptr;
-  int64_t n_slots = 0;
-  bool table_ready = false;
-};
+// TN launch of the direct-to-LDS kernels.  TS is the tile of a product's last row of tiles when that is at most half full
+// (TS = T: always T).
 template <int DT, typename T, typename TS>
-int gmm_dma(const void* a, const void* b, void* c, const int32_t* bins, int num_groups, int64_t rows, int k, int n,
-            int layout, hipStream_t s, const void* a2 = nullptr, const void* b2 = nullptr, int epi = dma::kEpiNone,
-            void* extra = nullptr, void* out2 = nullptr, GatherRows gather = GatherRows(), Workspace ws = Workspace(),
-            CombineRows combine = CombineRows()) {
-  const uint16_t* ap = (const uint16_t*)a;
-  const uint16_t* bp = (const uint16_t*)b;
-  const uint16_t* ap2 = (const uint16_t*)a2;
-  const uint16_t* bp2 = (const uint16_t*)b2;
-  const bool dual = a2 != nullptr && !dma::epi_is_dglu(epi) && !dma::epi_is_glu(epi);
-  uint16_t* cp = (uint16_t*)c;
-  if (layout == MBX_TN) {
-    constexpr size_t lds = T::LDS_BYTES > TS::LDS_BYTES ? T::LDS_BYTES : TS::LDS_BYTES;
-    const int tiles_m = (int)ceil_div(k, T::BM), tiles_n = (int)ceil_div(n, T::BN);
-    // rows per segment of a reduction: each operand's share stays below 2 GiB (whole K tiles)
-    const int64_t seg_rows = (((int64_t)1 << 31) - 1) / ((int64_t)(k > n ? k : n) * 2) / T::BK * T::BK;
-    const bool segmented = rows > seg_rows;
-    // the last row tile of the product as a TS tile when it is at most half full
-    const bool mixed = T::BM != TS::BM && k % T::BM != 0 && k % T::BM <= TS::BM;
-    auto kern = mixed ? (segmented ? dma::gmm_tn_kernel<DT, T, TS, true> : dma::gmm_tn_kernel<DT, T, TS, false>)
-                      : (segmented ? dma::gmm_tn_kernel<DT, T, T, true> : dma::gmm_tn_kernel<DT, T, T, false>);
-    int rc = allow_lds(kern, lds);
-    if (rc) return rc;
-    // short reductions (few rows per expert): several tiles per workgroup
-    const int64_t avg_rows = rows / (num_groups > 0 ? num_groups : 1);
-    int chunk = avg_rows >= 1024 ? 1 : avg_rows >= 512 ? 2 : 4;
-    // Reductions of a few dozen K tiles still gain from fewer workgroup launches (c3: 2 % of the launch with four
-    // tiles per workgroup), but only where an expert brings every XCD many tiles: with the six tiles per expert and
-    // XCD of a skewed c4, four to a workgroup leave most compute units idle behind the largest expert (2.4 x slower).
-    const dma::TnBlocks shape = dma::tn_block_shape(tiles_m, tiles_n);
-    if (avg_rows >= 1024 && avg_rows < 4096 && dma::tn_tiles_per_group(tiles_m, tiles_n, shape) / kXcds >= 64) chunk = 4;
-    const int64_t grid = dma::tn_grid(tiles_m, tiles_n, shape, num_groups, chunk);
-    if (grid > 0x7fffffff) return MBX_ERANGE;
-    // whole experts per XCD (if the kernel finds them balanced): for reductions of a few K tiles only
-    const int whole_ok = avg_rows < 1024 ? 1 : 0;
-    if (gather.slots) {
-      // the rows of b picked through the sorted assignments: the full tile only, one segment
-      if (!gather.src_bins || !gather.row_table || gather.top_k <= 0 || gather.n_slots > 0x7fffffff) return MBX_EINVAL;
-      if (segmented || !std::is_same<T, TS>::value) return MBX_EUNSUPPORTED;
-      if (!gather.table_ready) {
-        uint32_t magic = 0;
-        int shift = 0;
-        dma::gather_divisor(gather.top_k, magic, shift);
-        dma::gather_row_table_kernel<<<(unsigned)ceil_div(dma::row_table_entries(gather.n_slots, num_groups), 256), 256, 0, s>>>(
-            gather.slots, gather.src_bins, num_groups, (int)gather.n_slots, gather.src_rows, (uint32_t)n * 2u, magic, shift, gather.row_table);
-      }
-      if constexpr (T::BM == 256 && T::SB == 2) {
-        auto gkern = dma::gmm_tn_kernel<DT, T, T, false, true>;
-        int grc = allow_lds(gkern, lds);
-        if (grc) return grc;
-        gkern<<<(unsigned)grid, T::THREADS, lds, s>>>(ap, bp, cp, bins, num_groups, (int)rows, k, n, tiles_m, tiles_n, shape.bm, shape.bn, chunk, (int)seg_rows, whole_ok, gather.row_table, gather.src_bins, gather.src_rows, (int)gather.n_slots);
-        return launch_status();
-      } else {
-        return MBX_EUNSUPPORTED;
-      }
-    }
-    kern<<<(unsigned)grid, T::THREADS, lds, s>>>(ap, bp, cp, bins, num_groups, (int)rows, k, n, tiles_m, tiles_n, shape.bm, shape.bn, chunk, (int)seg_rows, whole_ok, nullptr, nullptr, 0, 0);
-    return launch_status();
-  }
+int launch_tn(const DmaCall& call) {
+  const int32_t* const bins = call.bins;
+  const int num_groups = call.num_groups, k = call.k, n = call.n;
+  const int64_t rows = call.rows;
+  const hipStream_t s = call.stream;
+  const uint16_t *ap = (const uint16_t*)call.a, *bp = (const uint16_t*)call.b;
+  uint16_t* cp = (uint16_t*)call.c;
+  const GatherRows& gather = call.gather;
   constexpr size_t lds = T::LDS_BYTES > TS::LDS_BYTES ? T::LDS_BYTES : TS::LDS_BYTES;
-  // a [w1 | v1] tile covers half as many output columns
-  const int tiles_n = (int)ceil_div(n, dma::epi_is_glu(epi) ? T::BN / 2 : T::BN);
-  const int64_t tiles = (ceil_div(rows, T::BM) + num_groups) * tiles_n;   // the row counts are only known on the device
-  if (tiles > 0x7fffffff) return MBX_ERANGE;
-  const unsigned grid = (unsigned)persistent_grid(tiles);
-  // An expert's last row tile, when at most half full, is computed with the half-height tile -- unless a row of tiles is
-  // longer than the run of tiles an XCD's workgroups take per round: the half-height tiles of such a row fill whole
-  // rounds of some XCDs, those finish early, and from then on the XCD's workgroups are no longer within the few K tiles
-  // of each other that the L2 holds (c3's NT launches, 112 and 56 column tiles against runs of 32: L2 misses 5.8 ->
-  // 3.3 GB; the launches themselves take 1 % longer for the padding they multiply, the step is 0.7 % shorter, the
-  // launches after them running at a higher clock).  With shorter rows of tiles the half-height tile wins (every
-  // launch of c2, c4 and c5: 0.7 - 2.8 % per step), and with few row tiles per expert the padding would be a large
-  // part of the work.  MBX_FULL_SHORT_FROM=N overrides the column-tile count from which
-  // the full tile is used (measurements).
-  static const int full_short_from = [] { const char* v = getenv("MBX_FULL_SHORT_FROM"); return v ? atoi(v) : -1; }();
-  const int run_tiles = (int)grid / kXcds;
-  // ... and only for experts of eight row tiles and more on average, where the padding is a few percent of the work
-  const bool long_experts = rows >= (int64_t)num_groups * 8 * T::BM;
-  const int half_limit = (full_short_from >= 0 ? tiles_n >= full_short_from : tiles_n > run_tiles && long_experts) ? 0 : TS::BM;
-  uint32_t gather_magic = 0;
-  int gather_shift = 0;
-  if (gather.slots) dma::gather_divisor(gather.top_k, gather_magic, gather_shift);
-  const WorkspaceParts lent(ws, (size_t)T::BM * T::BN * sizeof(float));
-  int32_t* const ws_counters = lent.counters;
-  float* const ws_parts = (int)grid / 2 <= (int)kWorkspaceCounters ? lent.parts : nullptr;
-  const int ws_capacity = lent.capacity;
-#define MBX_LAUNCH_ROWS_G(B_MC, DUAL, EPI, GATHER)                                                    \
-  do {                                                                                                \
-    auto kern = dma::gmm_rows_kernel<DT, B_MC, T, TS, DUAL, EPI, GATHER>;                             \
-    int rc = allow_lds(kern, lds);                                                                    \
-    if (rc) return rc;                                                                                \
-    kern<<<grid, T::THREADS, lds, s>>>(ap, bp, cp, bins, num_groups, rows, k, n, tiles_n, ap2, bp2, (uint16_t*)extra, (uint16_t*)out2,  \
-                                       gather.slots, gather.src_bins, gather.top_k, gather.src_rows, gather_magic, gather_shift, half_limit,  \
-                                       ws_counters, ws_parts, ws_capacity, combine.weights, combine.w_dtype, combine.tokens);  \
-  } while (0)
-#define MBX_LAUNCH_ROWS(B_MC, DUAL, EPI) MBX_LAUNCH_ROWS_G(B_MC, DUAL, EPI, false)
-  // the combine epilogue takes the sorted assignments where the gathered launches take theirs
-#define MBX_LAUNCH_ROWS_C(B_MC, DUAL, EPI)                                                            \
-  do {                                                                                                \
-    auto kern = dma::gmm_rows_kernel<DT, B_MC, T, TS, DUAL, EPI, false>;                              \
-    int rc = allow_lds(kern, lds);                                                                    \
-    if (rc) return rc;                                                                                \
-    kern<<<grid, T::THREADS, lds, s>>>(ap, bp, cp, bins, num_groups, rows, k, n, tiles_n, ap2, bp2, (uint16_t*)extra, (uint16_t*)out2,  \
-                                       combine.indices, nullptr, 1, 0, 0u, 0, half_limit, nullptr, nullptr, 0,          \
-                                       combine.weights, combine.w_dtype, combine.tokens);             \
-  } while (0)
+  const int tiles_m = (int)ceil_div(k, T::BM), tiles_n = (int)ceil_div(n, T::BN);
+  // rows per segment of a reduction: each operand's share stays below 2 GiB (whole K tiles)
+  const int64_t seg_rows = (((int64_t)1 << 31) - 1) / ((int64_t)(k > n ? k : n) * 2) / T::BK * T::BK;
+  const bool segmented = rows > seg_rows;
+  // the last row tile of the product as a TS tile when it is at most half full
+  const bool mixed = T::BM != TS::BM && k % T::BM != 0 && k % T::BM <= TS::BM;
+  auto kern = mixed ? (segmented ? dma::gmm_tn_kernel<DT, T, TS, true> : dma::gmm_tn_kernel<DT, T, TS, false>)
+                    : (segmented ? dma::gmm_tn_kernel<DT, T, T, true> : dma::gmm_tn_kernel<DT, T, T, false>);
+  int rc = allow_lds(kern, lds);
+  if (rc) return rc;
+  // short reductions (few rows per expert): several tiles per workgroup
+  const int64_t avg_rows = rows / (num_groups > 0 ? num_groups : 1);
+  int chunk = avg_rows >= 1024 ? 1 : avg_rows >= 512 ? 2 : 4;
+  // Reductions of a few dozen K tiles still gain from fewer workgroup launches (c3: 2 % of the launch with four
+  // tiles per workgroup), but only where an expert brings every XCD many tiles: with the six tiles per expert and
+  // XCD of a skewed c4, four to a workgroup leave most compute units idle behind the largest expert (2.4 x slower).
+  const dma::TnBlocks shape = dma::tn_block_shape(tiles_m, tiles_n);
+  if (avg_rows >= 1024 && avg_rows < 4096 && dma::tn_tiles_per_group(tiles_m, tiles_n, shape) / kXcds >= 64) chunk = 4;
+  const int64_t grid = dma::tn_grid(tiles_m, tiles_n, shape, num_groups, chunk);
+  if (grid > 0x7fffffff) return MBX_ERANGE;
+  // whole experts per XCD (if the kernel finds them balanced): for reductions of a few K tiles only
+  const int whole_ok = avg_rows < 1024 ? 1 : 0;
   if (gather.slots) {
-    if (layout != MBX_NT || a2 || !gather.src_bins || gather.top_k <= 0) return MBX_EINVAL;
-    switch (epi) {
-      case dma::kEpiNone: MBX_LAUNCH_ROWS_G(false, false, dma::kEpiNone, true); break;
-      case dma::kEpiAct: if (!extra) return MBX_EINVAL; MBX_LAUNCH_ROWS_G(false, false, dma::kEpiAct, true); break;
-      case dma::kEpiGluSilu: if (!extra || !b2 || !out2) return MBX_EINVAL; MBX_LAUNCH_ROWS_G(false, false, dma::kEpiGluSilu, true); break;
-      case dma::kEpiGluGelu: if (!extra || !b2 || !out2) return MBX_EINVAL; MBX_LAUNCH_ROWS_G(false, false, dma::kEpiGluGelu, true); break;
-      default: return MBX_EINVAL;
+    // the rows of b picked through the sorted assignments: the full tile only, one segment
+    if (!gather.src_bins || !gather.row_table || gather.top_k <= 0 || gather.n_slots > 0x7fffffff) return MBX_EINVAL;
+    if (segmented || !std::is_same<T, TS>::value) return MBX_EUNSUPPORTED;
+    if (!gather.table_ready) {
+      uint32_t magic = 0;
+      int shift = 0;
+      dma::gather_divisor(gather.top_k, magic, shift);
+      dma::gather_row_table_kernel<<<(unsigned)ceil_div(dma::row_table_entries(gather.n_slots, num_groups), 256), 256, 0, s>>>(
+          gather.slots, gather.src_bins, num_groups, (int)gather.n_slots, gather.src_rows, (uint32_t)n * 2u, magic, shift, gather.row_table);
     }
-    return launch_status();
+    if constexpr (T::BM == 256 && T::SB == 2) {
+      auto gkern = dma::gmm_tn_kernel<DT, T, T, false, true>;
+      int grc = allow_lds(gkern, lds);
+      if (grc) return grc;
+      gkern<<<(unsigned)grid, T::THREADS, lds, s>>>(ap, bp, cp, bins, num_groups, (int)rows, k, n, tiles_m, tiles_n, shape.bm, shape.bn, chunk, (int)seg_rows, whole_ok, gather.row_table, gather.src_bins, gather.src_rows, (int)gather.n_slots);
+      return launch_status();
+    } else {
+      return MBX_EUNSUPPORTED;
+    }
   }
-  if (dma::epi_is_glu(epi)) {
-    // b2 is the second matrix of the [w1 | v1] tiles (not a second operand pair)
-    if (layout != MBX_NT || !extra || !b2 || !out2 || a2) return MBX_EINVAL;
-    if (epi == dma::kEpiGluSilu) MBX_LAUNCH_ROWS(false, false, dma::kEpiGluSilu); else MBX_LAUNCH_ROWS(false, false, dma::kEpiGluGelu);
-    return launch_status();
-  }
-  if (dma::epi_is_dglu(epi)) {
-    // a2 carries x2 of the gated activation (not a second operand pair)
-    if (layout != MBX_NT || !extra || !a2 || !out2) return MBX_EINVAL;
-    if (epi == dma::kEpiDgluSilu) MBX_LAUNCH_ROWS(false, false, dma::kEpiDgluSilu); else MBX_LAUNCH_ROWS(false, false, dma::kEpiDgluGelu);
-    return launch_status();
-  }
-  if (epi == dma::kEpiCombine) {
-    // extra is the combined output [tokens, n]; c (the product itself) may be absent
-    if (layout != MBX_NN || a2 || !extra || !combine.indices) return MBX_EINVAL;
-    MBX_LAUNCH_ROWS_C(true, false, dma::kEpiCombine);
-    return launch_status();
-  }
-  if (epi != dma::kEpiNone) {
-    if (layout != MBX_NT || dual || !extra) return MBX_EINVAL;
-    if (epi == dma::kEpiAct) MBX_LAUNCH_ROWS(false, false, dma::kEpiAct); else MBX_LAUNCH_ROWS(false, false, dma::kEpiDact);
-    return launch_status();
-  }
-  if (layout == MBX_NT) {
-    if (dual) MBX_LAUNCH_ROWS(false, true, dma::kEpiNone); else MBX_LAUNCH_ROWS(false, false, dma::kEpiNone);
-  } else {
-    if (dual) MBX_LAUNCH_ROWS(true, true, dma::kEpiNone); else MBX_LAUNCH_ROWS(true, false, dma::kEpiNone);
-  }
-#undef MBX_LAUNCH_ROWS
-#undef MBX_LAUNCH_ROWS_C
-#undef MBX_LAUNCH_ROWS_G
+  kern<<<(unsigned)grid, T::THREADS, lds, s>>>(ap, bp, cp, bins, num_groups, (int)rows, k, n, tiles_m, tiles_n, shape.bm, shape.bn, chunk, (int)seg_rows, whole_ok, nullptr, nullptr, 0, 0);
   return launch_status();
+}
+
+// The direct-to-LDS kernels for 16-bit operands: the row tiles of NN / NT by whether the reduction is whole K tiles, TN
+// here (the half-height tile only when the product has at most 128 rows: it is slower otherwise).
+static int gmm_dma(const DmaCall& call) {
+  if (call.layout != MBX_TN) return call.k % dma::TileMain::BK == 0 ? gmm_rows(call) : gmm_rows_tail(call);
+  if (call.gather.slots) {   // gathered rows: the full tile only
+    if (call.dtype == MBX_BF16) return launch_tn<MBX_BF16, dma::TileMain, dma::TileMain>(call);
+    return launch_tn<MBX_F16, dma::TileMain, dma::TileMain>(call);
+  }
+  if (call.k <= dma::TileSmallM::BM) {
+    if (call.dtype == MBX_BF16) return launch_tn<MBX_BF16, dma::TileSmallM, dma::TileSmallM>(call);
+    return launch_tn<MBX_F16, dma::TileSmallM, dma::TileSmallM>(call);
+  }
+  if (call.dtype == MBX_BF16) return launch_tn<MBX_BF16, dma::TileMain, dma::TileSmallM>(call);
+  return launch_tn<MBX_F16, dma::TileMain, dma::TileSmallM>(call);
 }
 
 template <int DT>
@@ -697,20 +589,7 @@ int gmm_generic(const void* a, const void* b, void* c, const int32_t* bins, int 
 // or product and 256 rows of any operand (a 64-row K tile in TN).
 static inline bool dma_sizes_ok(int k, int n) {
   const int64_t lim = (int64_t)1 << 31;
-  return (int64_t)k * n * 2 < lim && (int64_t)k * 2 * TileDma::BM < lim && (int64_t)n * 2 * TileDma::BM < lim;
-}
-
-// NN / NT: whether to tile a launch with the half-height tile only.  With about one such tile per expert
-// (up to 144 rows on average) the full tile would mostly multiply padding.  Up to 320 rows the mix of
-// full tiles and a half-height last tile moves fewer weight bytes through the compute units (the
-// weights are streamed once per row tile), but its tiles cost unequal time, and a launch of fewer than
-// three rounds of them does not balance over the statically assigned workgroups.
-static inline bool half_height_only(int64_t rows, int num_groups, int n) {
-  const int64_t avg = rows / (num_groups > 0 ? num_groups : 1);
-  if (avg <= 144) return true;
-  if (avg > 320) return false;
-  const int64_t mixed_tiles = (ceil_div(rows, TileDma::BM) + num_groups / 2) * ceil_div(n, TileDma::BN);
-  return mixed_tiles < 3 * (int64_t)persistent_grid((int64_t)1 << 30);
+  return (int64_t)k * n * 2 < lim && (int64_t)k * 2 * dma::TileMain::BM < lim && (int64_t)n * 2 * dma::TileMain::BM < lim;
 }
 
 }  // namespace
@@ -723,6 +602,8 @@ extern "C" {
 #ifdef MBX_TICKS
 // libmbx_ticks.so only: where the kernels of gmm_dma.h put their per-tile time stamps (see there); NULL: nowhere.
 int mbx_debug_set_ticks(void* buffer) {
+  if (const int rc = gmm_rows_set_ticks(buffer)) return rc;
+  if (const int rc = gmm_rows_tail_set_ticks(buffer)) return rc;
   return (int)hipMemcpyToSymbol(HIP_SYMBOL(dma::g_ticks), &buffer, sizeof(buffer));
 }
 #endif
@@ -755,19 +636,11 @@ static int gmm_ws(const void* a, const void* b, void* c, int dtype, const int32_
   if (layout == MBX_NN) fast = fast && k % 8 == 0 && n % 8 == 0;
   if (layout == MBX_TN) fast = fast && k % 8 == 0 && n % 8 == 0;
   if (fast) {
-    // direct-to-LDS kernels: whole K tiles (NN / NT); their epilogue writes 16-byte pieces of the output's rows
-    bool dma_ok = dma_sizes_ok(k, n) && aligned16(c) && n % 8 == 0;
-    if (layout != MBX_TN) dma_ok = dma_ok && k % TileDma::BK == 0;
-    if (dma_ok) {
-      // TN: the half-height tile only when the product has at most 128 rows (it is slower otherwise)
-      const bool small_m = layout == MBX_TN ? k <= TileDmaSmallM::BM : half_height_only(rows, num_groups, n);
-      const GatherRows none;
-      if (small_m) {
-        if (dtype == MBX_BF16) return gmm_dma<MBX_BF16, TileDmaSmallM, TileDmaSmallM>(a, b, c, bins, num_groups, rows, k, n, layout, s, nullptr, nullptr, dma::kEpiNone, nullptr, nullptr, none, ws);
-        return gmm_dma<MBX_F16, TileDmaSmallM, TileDmaSmallM>(a, b, c, bins, num_groups, rows, k, n, layout, s, nullptr, nullptr, dma::kEpiNone, nullptr, nullptr, none, ws);
-      }
-      if (dtype == MBX_BF16) return gmm_dma<MBX_BF16, TileDma, TileDmaSmallM>(a, b, c, bins, num_groups, rows, k, n, layout, s, nullptr, nullptr, dma::kEpiNone, nullptr, nullptr, none, ws);
-      return gmm_dma<MBX_F16, TileDma, TileDmaSmallM>(a, b, c, bins, num_groups, rows, k, n, layout, s, nullptr, nullptr, dma::kEpiNone, nullptr, nullptr, none, ws);
+    // direct-to-LDS kernels: their epilogue writes 16-byte pieces of the output's rows
+    if (dma_sizes_ok(k, n) && aligned16(c) && n % 8 == 0) {
+      DmaCall call{a, b, c, dtype, bins, num_groups, rows, k, n, layout, s};
+      call.ws = ws;
+      return gmm_dma(call);
     }
     if (dtype == MBX_BF16) return gmm_mfma<MBX_BF16, TileBig>(a, b, c, bins, num_groups, rows, k, n, layout, s);
     return gmm_mfma<MBX_F16, TileBig>(a, b, c, bins, num_groups, rows, k, n, layout, s);
@@ -813,19 +686,15 @@ static int gmm_dual_ws(const void* a, const void* b, const void* a2, const void*
   if (!bins || !c || (k > 0 && (!a || !b || !a2 || !b2))) return MBX_EINVAL;
   if (rows > 0x7fffffff) return MBX_ERANGE;
   if (dtype == MBX_F32) return gmm_f32(a, b, a2, b2, c, bins, num_groups, rows, k, n, layout, ws.base, ws.bytes, as_stream(stream));
-  // only the direct-to-LDS kernels reduce over two operand pairs: whole K tiles, at least four per pair
-  const bool ok = dtype != MBX_F32 && aligned16(a) && aligned16(b) && aligned16(a2) && aligned16(b2) && aligned16(c) &&
-                  k % TileDma::BK == 0 && k >= 4 * TileDma::BK && n % 8 == 0 && dma_sizes_ok(k, n);
+  // only the direct-to-LDS kernels reduce over two operand pairs: at least four K tiles per pair
+  const bool ok = aligned16(a) && aligned16(b) && aligned16(a2) && aligned16(b2) && aligned16(c) && k % 8 == 0 &&
+                  k > 3 * dma::TileMain::BK && n % 8 == 0 && dma_sizes_ok(k, n);
   if (!ok) return MBX_EUNSUPPORTED;
-  hipStream_t s = as_stream(stream);
-  const bool small_m = half_height_only(rows, num_groups, n);
-  const GatherRows none;
-  if (small_m) {
-    if (dtype == MBX_BF16) return gmm_dma<MBX_BF16, TileDmaSmallM, TileDmaSmallM>(a, b, c, bins, num_groups, rows, k, n, layout, s, a2, b2, dma::kEpiNone, nullptr, nullptr, none, ws);
-    return gmm_dma<MBX_F16, TileDmaSmallM, TileDmaSmallM>(a, b, c, bins, num_groups, rows, k, n, layout, s, a2, b2, dma::kEpiNone, nullptr, nullptr, none, ws);
-  }
-  if (dtype == MBX_BF16) return gmm_dma<MBX_BF16, TileDma, TileDmaSmallM>(a, b, c, bins, num_groups, rows, k, n, layout, s, a2, b2, dma::kEpiNone, nullptr, nullptr, none, ws);
-  return gmm_dma<MBX_F16, TileDma, TileDmaSmallM>(a, b, c, bins, num_groups, rows, k, n, layout, s, a2, b2, dma::kEpiNone, nullptr, nullptr, none, ws);
+  DmaCall call{a, b, c, dtype, bins, num_groups, rows, k, n, layout, as_stream(stream)};
+  call.a2 = a2;
+  call.b2 = b2;
+  call.ws = ws;
+  return gmm_dma(call);
 }
 
 // The NT product with an activation epilogue (epi: dma::kEpiAct / dma::kEpiDact), for the shapes the direct-to-LDS
@@ -846,17 +715,18 @@ static int gmm_nt_epilogue(const void* a, const void* b, void* c, void* extra, i
   if (!bins || !c || (!extra && !plain) || (k > 0 && (!a || !b)) || (dglu && (!pre2 || !out2)) || (glu && (!out2 || (k > 0 && !b2)))) return MBX_EINVAL;
   if (rows > 0x7fffffff) return MBX_ERANGE;
   bool ok = dtype != MBX_F32 && aligned16(a) && aligned16(b) && aligned16(c) && aligned16(extra) && k > 0 &&
-            k % TileDma::BK == 0 && n % 8 == 0 && dma_sizes_ok(k, n) && (!dglu || (aligned16(pre2) && aligned16(out2)));
+            k % 8 == 0 && n % 8 == 0 && dma_sizes_ok(k, n) && (!dglu || (aligned16(pre2) && aligned16(out2)));
   // the second matrix is addressed from half a tile before its first row: that much more must fit below 2 GiB
-  if (glu) ok = ok && aligned16(b2) && aligned16(out2) && dma_sizes_ok(k, n + TileDma::BN / 2);
+  if (glu) ok = ok && aligned16(b2) && aligned16(out2) && dma_sizes_ok(k, n + dma::TileMain::BN / 2);
   if (!ok) return MBX_EUNSUPPORTED;
-  hipStream_t s = as_stream(stream);
-  if (half_height_only(rows, num_groups, n)) {
-    if (dtype == MBX_BF16) return gmm_dma<MBX_BF16, TileDmaSmallM, TileDmaSmallM>(a, b, c, bins, num_groups, rows, k, n, MBX_NT, s, pre2, b2, epi, extra, out2, gather);
-    return gmm_dma<MBX_F16, TileDmaSmallM, TileDmaSmallM>(a, b, c, bins, num_groups, rows, k, n, MBX_NT, s, pre2, b2, epi, extra, out2, gather);
-  }
-  if (dtype == MBX_BF16) return gmm_dma<MBX_BF16, TileDma, TileDmaSmallM>(a, b, c, bins, num_groups, rows, k, n, MBX_NT, s, pre2, b2, epi, extra, out2, gather);
-  return gmm_dma<MBX_F16, TileDma, TileDmaSmallM>(a, b, c, bins, num_groups, rows, k, n, MBX_NT, s, pre2, b2, epi, extra, out2, gather);
+  DmaCall call{a, b, c, dtype, bins, num_groups, rows, k, n, MBX_NT, as_stream(stream)};
+  call.a2 = pre2;
+  call.b2 = b2;
+  call.epi = epi;
+  call.extra = extra;
+  call.out2 = out2;
+  call.gather = gather;
+  return gmm_dma(call);
 }
 
 int mbx_gmm_act(const void* a, const void* b, void* c, void* c_act, int dtype, const int32_t* bins, int num_groups,
@@ -884,8 +754,8 @@ int mbx_gmm_gather(const void* x, int64_t x_rows, const int32_t* indices, int to
   if (b2 ? (act != MBX_ACT_SILU && act != MBX_ACT_GELU_TANH) || !c2 || !h : c2 != nullptr) return MBX_EINVAL;
   if (h && !b2 && act != MBX_ACT_GELU_TANH) return MBX_EUNSUPPORTED;
   if (!indices || (k > 0 && !x && x_rows > 0)) return MBX_EINVAL;
-  // the row map is indexed with 32 bits and the rows of x are addressed with 31 (bit 31 marks a row of zeros)
-  if (x_rows * top_k > 0x7fffffff || x_rows * (int64_t)k * 2 >= ((int64_t)1 << 31)) return MBX_EUNSUPPORTED;
+  // the row map is indexed with 32 bits and the rows of x are addressed with 31 (bit 31 marks a row of zeros); whole K tiles
+  if (k % dma::TileMain::BK != 0 || x_rows * top_k > 0x7fffffff || x_rows * (int64_t)k * 2 >= ((int64_t)1 << 31)) return MBX_EUNSUPPORTED;
   if (x_rows == 0 && rows > 0) x = b1;   // no row is read; the buffer descriptor still wants an address
   GatherRows gather;
   gather.slots = indices;
@@ -905,25 +775,21 @@ int mbx_gmm_scatter(const void* a, const void* b, void* c, void* out, int dtype,
   if (num_groups == 0 || rows == 0 || n == 0) return 0;
   if (!out || !bins || !indices || (k > 0 && (!a || !b))) return MBX_EINVAL;
   if (rows > 0x7fffffff || tokens > 0x7fffffff) return MBX_ERANGE;
-  // the direct-to-LDS NN kernel (16-bit types, whole K tiles, 16-byte pieces of rows); the combined output is addressed
+  // the direct-to-LDS NN kernel (16-bit types, 16-byte pieces of rows); the combined output is addressed
   // with 64 bits
   const bool ok = dtype != MBX_F32 && aligned16(a) && aligned16(b) && (!c || aligned16(c)) && aligned16(out) && k > 0 &&
-                  k % TileDma::BK == 0 && n % 8 == 0 && dma_sizes_ok(k, n);
+                  k % 8 == 0 && n % 8 == 0 && dma_sizes_ok(k, n);
   if (!ok) return MBX_EUNSUPPORTED;
   CombineRows combine;
   combine.indices = indices;
   combine.weights = weights;
   combine.w_dtype = w_dtype;
   combine.tokens = (int)tokens;
-  hipStream_t s = as_stream(stream);
-  const GatherRows none;
-  const Workspace no_ws;
-  if (half_height_only(rows, num_groups, n)) {
-    if (dtype == MBX_BF16) return gmm_dma<MBX_BF16, TileDmaSmallM, TileDmaSmallM>(a, b, c, bins, num_groups, rows, k, n, MBX_NN, s, nullptr, nullptr, dma::kEpiCombine, out, nullptr, none, no_ws, combine);
-    return gmm_dma<MBX_F16, TileDmaSmallM, TileDmaSmallM>(a, b, c, bins, num_groups, rows, k, n, MBX_NN, s, nullptr, nullptr, dma::kEpiCombine, out, nullptr, none, no_ws, combine);
-  }
-  if (dtype == MBX_BF16) return gmm_dma<MBX_BF16, TileDma, TileDmaSmallM>(a, b, c, bins, num_groups, rows, k, n, MBX_NN, s, nullptr, nullptr, dma::kEpiCombine, out, nullptr, none, no_ws, combine);
-  return gmm_dma<MBX_F16, TileDma, TileDmaSmallM>(a, b, c, bins, num_groups, rows, k, n, MBX_NN, s, nullptr, nullptr, dma::kEpiCombine, out, nullptr, none, no_ws, combine);
+  DmaCall call{a, b, c, dtype, bins, num_groups, rows, k, n, MBX_NN, as_stream(stream)};
+  call.epi = dma::kEpiCombine;
+  call.extra = out;
+  call.combine = combine;
+  return gmm_dma(call);
 }
 
 size_t mbx_gmm_tn_gather_table_bytes(int64_t x_rows, int top_k, int num_groups) {
@@ -942,7 +808,7 @@ int mbx_gmm_tn_gather(const void* a, const void* x, int64_t x_rows, const int32_
   const int64_t n_slots = x_rows * top_k;
   // the kernel with the full tile, 16-byte pieces of rows, one segment of the reduction, row offsets of 31 bits
   const bool ok = dtype != MBX_F32 && aligned16(a) && aligned16(x) && aligned16(c) && k % 8 == 0 && n % 8 == 0 && dma_sizes_ok(k, n) &&
-                  k > TileDmaSmallM::BM && n_slots <= 0x7fffffff && x_rows * (int64_t)n * 2 < ((int64_t)1 << 31) &&
+                  k > dma::TileSmallM::BM && n_slots <= 0x7fffffff && x_rows * (int64_t)n * 2 < ((int64_t)1 << 31) &&
                   rows * (int64_t)(k > n ? k : n) * 2 < ((int64_t)1 << 31);
   if (!ok) return MBX_EUNSUPPORTED;
   if (!row_table || row_table_bytes < mbx_gmm_tn_gather_table_bytes(x_rows, top_k, num_groups) || ((uintptr_t)row_table & 15u)) return MBX_ESCRATCH;
@@ -955,9 +821,9 @@ int mbx_gmm_tn_gather(const void* a, const void* x, int64_t x_rows, const int32_
   gather.row_table = (uint32_t*)row_table;
   gather.n_slots = n_slots;
   gather.table_ready = table_ready != 0;
-  hipStream_t s = as_stream(stream);
-  if (dtype == MBX_BF16) return gmm_dma<MBX_BF16, TileDma, TileDma>(a, x, c, bins, num_groups, rows, k, n, MBX_TN, s, nullptr, nullptr, dma::kEpiNone, nullptr, nullptr, gather);
-  return gmm_dma<MBX_F16, TileDma, TileDma>(a, x, c, bins, num_groups, rows, k, n, MBX_TN, s, nullptr, nullptr, dma::kEpiNone, nullptr, nullptr, gather);
+  DmaCall call{a, x, c, dtype, bins, num_groups, rows, k, n, MBX_TN, as_stream(stream)};
+  call.gather = gather;
+  return gmm_dma(call);
 }
 
 int mbx_gmm_dglu(const void* a, const void* b, const void* x1, const void* x2, void* d1, void* d2, int dtype,

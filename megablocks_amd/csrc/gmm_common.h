@@ -5,6 +5,66 @@
 #include "common.h"
 
 namespace mbx {
+
+// kWorkspaceCounters int32 counters, zero before the launch and zero again after it, then room for fp32 tiles.
+constexpr size_t kWorkspaceCounters = 1024, kWorkspacePartBytes = (size_t)256 * 256 * 4, kWorkspaceParts = 320;
+struct Workspace {
+  void* base = nullptr;
+  size_t bytes = 0;
+};
+
+// The weighted combine in the epilogue (kEpiCombine): the sorted assignments (top_k = 1: tokens) of the product's rows,
+// the weights by token (or null) and their type, the row count of the combined output.
+struct CombineRows {
+  const int32_t* indices = nullptr;
+  const void* weights = nullptr;
+  int w_dtype = 0;
+  int tokens = 0;
+};
+
+// Rows of an operand gathered on the fly.
+struct GatherRows {
+  const int32_t* slots = nullptr;      // non-null: a (NT) / b (TN) is [src_rows, .], read through the row map
+  const int32_t* src_bins = nullptr;
+  int top_k = 1, src_rows = 0;
+  // TN only: the table of row offsets the kernel reads (4 bytes per sorted assignment, n_slots of them), and whether an
+  // earlier call with the same slots, top_k, src_rows and n has already filled it
+  uint32_t* row_table = nullptr;
+  int64_t n_slots = 0;
+  bool table_ready = false;
+};
+
+// A launch of the direct-to-LDS kernels on 16-bit operands (gmm_dma.h).
+//   a2 / b2 non-null (no epilogue): c = a @ b[e] + a2 @ b2[e], the second pair shaped like the first;
+//   epi / extra / out2: an epilogue (dma::kEpi*) and its second output / input, third output; kEpiDglu*: a2 is x2; kEpiGlu*: b2 is
+//   the second matrix;
+//   gather: rows of `a` (NT; no epilogue, kEpiAct or kEpiGlu*) or of `b` (TN) picked through the sorted assignments;
+//   ws: device memory the launch may use for the parts of tiles it cuts along the reduction (NN without epilogue).
+struct DmaCall {
+  const void *a, *b;
+  void* c;
+  int dtype;
+  const int32_t* bins;
+  int num_groups;
+  int64_t rows;
+  int k, n, layout;
+  hipStream_t stream;
+  const void *a2 = nullptr, *b2 = nullptr;
+  int epi = 0;
+  void *extra = nullptr, *out2 = nullptr;
+  GatherRows gather{};
+  Workspace ws{};
+  CombineRows combine{};
+};
+
+// NN / NT launches, k a multiple of 64 (gmm_rows.hip) and of 8 only (gmm_rows_tail.hip).
+int gmm_rows(const DmaCall& call);
+int gmm_rows_tail(const DmaCall& call);
+#ifdef MBX_TICKS
+int gmm_rows_set_ticks(void* buffer);
+int gmm_rows_tail_set_ticks(void* buffer);
+#endif
+
 namespace {
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
@@ -44,12 +104,6 @@ static inline int64_t xcd_grid(int64_t tiles, int run = kXcdRun) {
 // the result wrong but never an access out of range.
 __device__ __forceinline__ int clamp_bound(int v, int lo, int rows) { return v < lo ? lo : (v > rows ? rows : v); }
 
-// kWorkspaceCounters int32 counters, zero before the launch and zero again after it, then room for fp32 tiles.
-constexpr size_t kWorkspaceCounters = 1024, kWorkspacePartBytes = (size_t)256 * 256 * 4, kWorkspaceParts = 320;
-struct Workspace {
-  void* base = nullptr;
-  size_t bytes = 0;
-};
 // The workspace as the kernels take it: counters, then parts of `part_bytes` each, 16-byte aligned; parts null where it
 // cannot hold two.
 struct WorkspaceParts {

@@ -1,7 +1,8 @@
 // Grouped-GEMM main loop with direct-to-LDS global loads and LDS rings of K tiles, and the kernels
 // that walk the tiles of a launch with it.
 //
-// Included by gmm.hip (uses its u32x4 / f32x4 types, pack2 and the XCD constants).
+// Included, inside the anonymous namespace of a translation unit, by gmm.hip (TN), gmm_rows.h (NN / NT) and gmm_f32.hip (the
+// helpers); uses the types, pack2 and the XCD constants of gmm_common.h.
 //
 // Why: with 256x256 output tiles a compute unit has to pull 64 bytes of operands per 16
 // MFMA-cycles.  Loads that pass through registers can only run one tile ahead and cost 64
@@ -62,6 +63,13 @@ struct Tile {
   static_assert(WAVES % 2 == 0, "the swizzles need the parity of a wave's load index to be fixed");
   static_assert((SB - 1) * (LA + LB) + LA + LB / 2 < 64, "vmcnt is a 6-bit counter");
 };
+
+// The tiles: 256 x 256 x 64, four waves of 128 x 128, three A and two B
+// stages of 32 KiB; and the half-height tile (NN / NT only: the row tile follows the expert's row count) for the last
+// row tile of an expert when it is at most half full, for the tail of a launch, and for launches of small experts;
+// its smaller stages allow a three-deep ring (4 x 16 KiB + 3 x 32 KiB).
+typedef Tile<256, 256, 2, 2, 64, 2> TileMain;
+typedef Tile<128, 256, 1, 4, 64, 3> TileSmallM;
 
 typedef __attribute__((address_space(3))) char* lds_ptr;
 
@@ -218,6 +226,9 @@ struct Args {
   // the entries of this lane's loads of K tiles 0 and 1, fetched by the caller while the tile before was computed.
   uint32_t gather_row2[8];
   u32x4 row_table;
+  // KTAIL instantiations: the K tiles (of this call) that hold the end of an operand pair's reduction, and how many of
+  // its elements (a multiple of 8) they hold.  -1: none.
+  int tail1, tail2, k_last;
   int tick_ordinal = -1;                  // MBX_TICKS builds: which tile of the workgroup this is
 };
 
@@ -276,7 +287,11 @@ __device__ __forceinline__ void mfma16_settle() { asm volatile("s_nop 15\n\ts_no
 // GATHER_B: the rows of the B tile (MC operand of 256 columns: the reduction runs over its rows) are gathered rows of a
 // matrix: each of a lane's LB loads of a K tile takes the byte offset of its row from a table (Args::row_table), which
 // it fetches a K tile ahead -- right after the load that used the entry for the K tile before, into the same register.
-template <int DT, bool A_MC, bool B_MC, typename T, bool DUAL = false, bool GLU = false, bool GATHER = false, bool GATHER_B = false>
+// KTAIL: the reduction is not a whole number of K tiles.  In the last K tile of an operand pair the 16-byte pieces of a
+// row (KC operand) past the end of the reduction are requested with bit 31 of the offset set and read as zeros; what
+// follows in memory is the next row, whose values may be infinite.  A lane fetches the same piece in all its loads of an
+// operand, so one register per operand carries the bit.  (The rows of an MC operand past the end are past its buffer.)
+template <int DT, bool A_MC, bool B_MC, typename T, bool DUAL = false, bool GLU = false, bool GATHER = false, bool GATHER_B = false, bool KTAIL = false>
 __device__ __forceinline__ void block_multiply16(const Args& g, typename T::Acc (&acc)[T::TM][T::TN], bool clear, char* lds_generic) {
   static_assert(T::KS == 2, "two k-steps of 32 per K tile");
   static_assert(!GLU || (!B_MC && !DUAL && T::LB % 2 == 0), "two matrices side by side in the B tile");
@@ -296,6 +311,10 @@ __device__ __forceinline__ void block_multiply16(const Args& g, typename T::Acc 
   const uint32_t b_lane = load_lane_offset<B_MC, BK, T::BN>(wave, g.b_r0, g.b_ld_bytes, false);
   const uint32_t a_lane1 = A_QDEP ? load_lane_offset<A_MC, BK, T::BM>(wave, g.a_r0, g.a_ld_bytes, true) : a_lane;
   const uint32_t b_lane1 = B_QDEP ? load_lane_offset<B_MC, BK, T::BN>(wave, g.b_r0, g.b_ld_bytes, true) : b_lane;
+  static_assert(!KTAIL || (!A_MC && !GATHER), "K tails: rows of a contiguous first operand, as they are");
+  const uint32_t piece_past = KTAIL && 8 * ((lane_id() & 7) ^ ((4 * (wave & 1) + (lane_id() >> 4)) & 7)) >= g.k_last ? 0x80000000u : 0u;
+  uint32_t a_tail = 0u, b_tail = 0u;   // piece_past when the loads issued next are those of a tail, else zero
+  auto tail_of = [&](int kt) -> uint32_t { return kt == g.tail1 || kt == g.tail2 ? piece_past : 0u; };
   const uint32_t a_step = A_MC ? BK * g.a_ld_bytes : BK * 2;   // bytes per K tile
   const uint32_t b_step = B_MC ? BK * g.b_ld_bytes : BK * 2;
   constexpr uint32_t A_ROWS = (uint32_t)(1024 / ((A_MC ? T::BM : BK) * 2)), B_ROWS = (uint32_t)(1024 / ((B_MC ? T::BN : BK) * 2));
@@ -334,10 +353,10 @@ __device__ __forceinline__ void block_multiply16(const Args& g, typename T::Acc 
       if constexpr (GATHER_B) {
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (__attribute__((address_space(3))) void*)(lds + dst), 16, (int)(b_row[GATHER_B ? q : 0] + (odd ? b_col1 : b_col)), 0, 0, 0);
       } else {
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(GLU && upper ? rb_upper : rb, (__attribute__((address_space(3))) void*)(lds + dst), 16, (int)((odd ? b_lane1 : b_lane) + sc), 0, 0, 0);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(GLU && upper ? rb_upper : rb, (__attribute__((address_space(3))) void*)(lds + dst), 16, (int)(((odd ? b_lane1 : b_lane) + sc) | (KTAIL && !B_MC ? b_tail : 0u)), 0, 0, 0);
       }
     } else {
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (__attribute__((address_space(3))) void*)(lds + dst), 16, (int)((GATHER ? a_row[GATHER ? q : 0] : odd ? a_lane1 : a_lane) + sc), 0, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (__attribute__((address_space(3))) void*)(lds + dst), 16, (int)(((GATHER ? a_row[GATHER ? q : 0] : odd ? a_lane1 : a_lane) + sc) | (KTAIL ? a_tail : 0u)), 0, 0, 0);
     }
   };
   auto issue_group = [&](bool is_b, int kt, int stage, int q0, int count) {   // prologue
@@ -468,6 +487,7 @@ __device__ __forceinline__ void block_multiply16(const Args& g, typename T::Acc 
   if (nk > 0) {
 #pragma unroll
     for (int t = 0; t < SB; ++t) {
+      if constexpr (KTAIL) a_tail = b_tail = tail_of(t);
       issue_group(false, t, t, 0, LA);
       if constexpr (GATHER_B) {
         if (t == 1) {
@@ -511,6 +531,7 @@ __device__ __forceinline__ void block_multiply16(const Args& g, typename T::Acc 
     uint32_t past = SB < nk ? 0u : 0x80000000u;
     uint32_t sc_a = a_sc0 | past, dst_a = a_dst0, sc_b = 0, dst_b = 0;
     if (DUAL) ra = SB >= g.nk1 ? g.rsrc_a2 : g.rsrc_a;
+    if constexpr (KTAIL) a_tail = tail_of(SB);
     constexpr int A_EVERY = (NP - NF - 3) / LA, B_EVERY = (NP - 4) / LB > 5 ? 5 : (NP - 4) / LB;
     for (int kt = 0; kt < nk; ++kt) {
       // k-step 0: the A loads (offsets set up in the iteration before); p0 / p1 prepare the B loads of k-step 1,
@@ -518,6 +539,7 @@ __device__ __forceinline__ void block_multiply16(const Args& g, typename T::Acc 
       auto p0 = [&]() {
         sc_b = b_sc0 | past;
         dst_b = b_dst0;
+        if constexpr (KTAIL && !B_MC) b_tail = tail_of(kt + SB);
       };
       auto p1 = [&]() {
         if (DUAL) rb = kt + SB >= g.nk1 ? g.rsrc_b2 : g.rsrc_b;
@@ -552,6 +574,7 @@ __device__ __forceinline__ void block_multiply16(const Args& g, typename T::Acc 
         sc_a = a_sc0 | past;
         dst_a = a_dst0;
         if (DUAL) ra = kt + 1 + SB >= g.nk1 ? g.rsrc_a2 : g.rsrc_a;
+        if constexpr (KTAIL) a_tail = tail_of(kt + 1 + SB);
       };
       uint32_t a_rd_nn = 0, b_rd_nn = 0;
       auto q2 = [&]() {
@@ -580,9 +603,9 @@ __device__ __forceinline__ void block_multiply16(const Args& g, typename T::Acc 
 #undef MBX_STEP16
 }
 
-template <int DT, bool A_MC, bool B_MC, typename T, bool DUAL = false, bool GLU = false, bool GATHER = false, bool GATHER_B = false>
+template <int DT, bool A_MC, bool B_MC, typename T, bool DUAL = false, bool GLU = false, bool GATHER = false, bool GATHER_B = false, bool KTAIL = false>
 __device__ __forceinline__ void block_multiply(const Args& g, typename T::Acc (&acc)[T::TM][T::TN], bool clear, char* lds) {
-  block_multiply16<DT, A_MC, B_MC, T, DUAL, GLU, GATHER, GATHER_B>(g, acc, clear, lds);
+  block_multiply16<DT, A_MC, B_MC, T, DUAL, GLU, GATHER, GATHER_B, KTAIL>(g, acc, clear, lds);
 }
 
 // ---- activation in the epilogue (tanh-GELU: megablocks/layers/arguments.py:19, megablocks/layers/gelu.py:9-13) ----
@@ -1083,13 +1106,13 @@ __device__ __forceinline__ void block_store(const typename T::Acc (&acc)[T::TM][
 }
 
 // c = A_tile * B_tile over all K tiles (the whole product of one output tile)
-template <int DT, bool A_MC, bool B_MC, typename T, bool DUAL = false, int EPI = kEpiNone, bool GATHER = false>
+template <int DT, bool A_MC, bool B_MC, typename T, bool DUAL = false, int EPI = kEpiNone, bool GATHER = false, bool KTAIL = false>
 __device__ __forceinline__ void block_gemm(const Args& g, uint16_t* __restrict__ c, int64_t ldc, int m_base, int m_lim,
                                            int n_base, int n_lim, char* lds, uint16_t* __restrict__ extra = nullptr,
                                            const uint16_t* __restrict__ pre2 = nullptr, uint16_t* __restrict__ out2 = nullptr,
                                            const Combine& combine = Combine()) {
   typename T::Acc acc[T::TM][T::TN];
-  block_multiply<DT, A_MC, B_MC, T, DUAL, epi_is_glu(EPI), GATHER>(g, acc, true, lds);
+  block_multiply<DT, A_MC, B_MC, T, DUAL, epi_is_glu(EPI), GATHER, false, KTAIL>(g, acc, true, lds);
   MBX_TICK(g.tick_ordinal, 2);
   block_store<DT, T, EPI>(acc, c, ldc, m_base, m_lim, n_base, n_lim, lds, extra, pre2, out2, combine);
   MBX_TICK(g.tick_ordinal, 4);
@@ -1266,7 +1289,8 @@ struct RowTiles {
 // launch decides).
 // slot / top_k is computed as (slot * top_k_magic) >> (32 + top_k_shift) (see gather_divisor(); top_k = 1: magic 0),
 // a division per row and tile being a few hundred dependent instructions on a wave that has its SIMD to itself.
-template <int DT, bool B_MC, typename T, typename TS, bool DUAL = false, int EPI = kEpiNone, bool GATHER = false>
+// KTAIL: k is a multiple of 8 but not of the K tile (see block_multiply16).
+template <int DT, bool B_MC, typename T, typename TS, bool DUAL = false, int EPI = kEpiNone, bool GATHER = false, bool KTAIL = false>
 __global__ void __launch_bounds__(T::THREADS)
 gmm_rows_kernel(const uint16_t* __restrict__ a, const uint16_t* __restrict__ b, uint16_t* __restrict__ c,
                 const int32_t* __restrict__ bins, int num_groups, int64_t rows, int k, int n, int tiles_n,
@@ -1291,9 +1315,15 @@ gmm_rows_kernel(const uint16_t* __restrict__ a, const uint16_t* __restrict__ b, 
   Args g;
   g.a_ld_bytes = (uint32_t)k * 2;
   g.b_ld_bytes = (uint32_t)(B_MC ? n : k) * 2;
-  const int nk1 = k / T::BK, nk_all = DUAL ? 2 * nk1 : nk1;
+  const int nk1 = (k + (KTAIL ? T::BK - 1 : 0)) / T::BK, nk_all = DUAL ? 2 * nk1 : nk1;
   g.nk1 = nk1;
   g.nk = nk_all;
+  auto set_tails = [&](int t0) {   // for a call that starts at K tile t0
+    g.tail1 = nk1 - 1 - t0;
+    g.tail2 = DUAL ? 2 * nk1 - 1 - t0 : -1;
+    g.k_last = k - (nk1 - 1) * T::BK;
+  };
+  if constexpr (KTAIL) set_tails(0);
   g.a_r0 = 0;   // the buffers of a and c start at the tile's first row: byte offsets stay small whatever the row count
   // The last, partly filled round.  Its `rest` tiles leave P - rest compute units idle for a whole tile's time, which
   // with long reductions and few rounds is a large part of the launch (a Mixtral-shaped second product: 1088 tiles on
@@ -1344,9 +1374,9 @@ gmm_rows_kernel(const uint16_t* __restrict__ a, const uint16_t* __restrict__ b, 
     // the last row tile of an expert, when at most half full, is computed as a half-height tile as well
     use_ts = kSplit && (use_ts || end - row0 <= half_limit);
     if (use_ts) {
-      block_gemm<DT, false, B_MC, TS, DUAL, EPI, GATHER>(g, c_tile, n, 0, end - row0, g.b_r0, n, lds, e_tile, p_tile, o_tile);
+      block_gemm<DT, false, B_MC, TS, DUAL, EPI, GATHER, KTAIL>(g, c_tile, n, 0, end - row0, g.b_r0, n, lds, e_tile, p_tile, o_tile);
     } else {
-      block_gemm<DT, false, B_MC, T, DUAL, EPI, GATHER>(g, c_tile, n, 0, end - row0, g.b_r0, n, lds, e_tile, p_tile, o_tile);
+      block_gemm<DT, false, B_MC, T, DUAL, EPI, GATHER, KTAIL>(g, c_tile, n, 0, end - row0, g.b_r0, n, lds, e_tile, p_tile, o_tile);
     }
     tile_done();
   };
@@ -1406,10 +1436,12 @@ gmm_rows_kernel(const uint16_t* __restrict__ a, const uint16_t* __restrict__ b, 
           g.nk1 = DUAL && !second && t1 > nk1 ? nk1 - t0 : 0x3fffffff;
           g.b_r0 = tn * kTileCols;
           typename T::Acc acc[T::TM][T::TN];
-          block_multiply<DT, false, B_MC, T, DUAL>(g, acc, true, lds);
+          if constexpr (KTAIL) set_tails(t0);
+          block_multiply<DT, false, B_MC, T, DUAL, false, false, false, KTAIL>(g, acc, true, lds);
           MBX_TICK(r, 2);
           g.nk = nk_all;
           g.nk1 = nk1;
+          if constexpr (KTAIL) set_tails(0);
           // The part's accumulators as they lie in the registers: 16 bytes per lane and product tile, addressed as a
           // buffer with the lane's offset in a register and the product tile's in a scalar (64-bit addresses per
           // store would take two registers each, which this kernel does not have).  Eight tiles at a time, so that the
@@ -1518,9 +1550,9 @@ gmm_rows_kernel(const uint16_t* __restrict__ a, const uint16_t* __restrict__ b, 
         combine.token = slots[combine.row_exists ? row : end - 1];
       }
       if (use_ts) {
-        block_gemm<DT, false, B_MC, TS, DUAL, EPI>(g, c_tile, n, 0, end - row0, g.b_r0, n, lds, e_tile, p_tile, o_tile, combine);
+        block_gemm<DT, false, B_MC, TS, DUAL, EPI, false, KTAIL>(g, c_tile, n, 0, end - row0, g.b_r0, n, lds, e_tile, p_tile, o_tile, combine);
       } else {
-        block_gemm<DT, false, B_MC, T, DUAL, EPI>(g, c_tile, n, 0, end - row0, g.b_r0, n, lds, e_tile, p_tile, o_tile, combine);
+        block_gemm<DT, false, B_MC, T, DUAL, EPI, false, KTAIL>(g, c_tile, n, 0, end - row0, g.b_r0, n, lds, e_tile, p_tile, o_tile, combine);
       }
       tile_done();
       MBX_TICK(r, 5);

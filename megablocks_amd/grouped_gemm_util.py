@@ -221,7 +221,7 @@ def _nt_operands(a, b, batch_sizes, what):
 def gmm_act(a, b, batch_sizes, fuse=None):
     """(c, gelu_tanh(c)) with c[r_e] = a[r_e] @ b[e].T: the first product of the expert MLP and its activation
     (mlp.py:521-522), the activation applied in the product's epilogue where the library has a kernel for the shape
-    (16-bit types, k a multiple of 64, n of 8) and the output is large enough for that to pay (`fuse` None; True /
+    (16-bit types, k and n multiples of 8) and the output is large enough for that to pay (`fuse` None; True /
     False force the choice), else as a separate element-wise pass."""
     a, b, bins = _nt_operands(a, b, batch_sizes, 'gmm_act')
     rows, k, n, groups = a.shape[0], a.shape[1], b.shape[1], bins.shape[0]

@@ -97,8 +97,11 @@ class _RouterLinear(torch.autograd.Function):
             from megablocks_amd import grouped_gemm_util as gg
             sizes = _RouterLinear.piece_sizes(x.shape[0])
             pieces = sizes.shape[0]
+            experts = grad.shape[1]
+            if experts % 8:   # the pipelined kernels read whole 16-byte pieces of rows
+                grad = torch.nn.functional.pad(grad, (0, -experts % 8))
             parts = gg.gmm(grad.contiguous(), x.contiguous(), sizes, trans_a=True, _record_as='router_wgrad')   # [pieces, E, h]
-            dw = (parts[0] if pieces == 1 else parts.sum(0, dtype=torch.float32)).to(ctx.weight_dtype)
+            dw = (parts[0] if pieces == 1 else parts.sum(0, dtype=torch.float32))[:experts].to(ctx.weight_dtype)
         return dx, dw
 
 

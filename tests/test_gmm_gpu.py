@@ -942,3 +942,62 @@ def test_gmm_fp32_on_the_matrix_cores(gg, monkeypatch, groups, rows, k, n, mode)
                 assert max_block_err(out[ok], want[ok]) < tol and not bool(torch.isfinite(out[bad]).any())
             got.append(out)
         assert torch.equal(got[-1].nan_to_num(), got[-2].nan_to_num())
+
+
+@pytest.mark.parametrize('groups,rows,k,n', [(3, 700, 8, 136), (4, 900, 72, 264), (5, 1500, 200, 512), (8, 3000, 1032, 2728),
+                                             (2, 40, 312, 1032), (12, 3600, 2728, 1032), (1, 260, 4104, 64)])
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])
+def test_gmm_reductions_that_end_inside_a_k_tile(gg, monkeypatch, groups, rows, k, n, dtype):
+    """k a multiple of 8 but not of 64, every NN / NT form, against fp32.  One row of the first operand and one weight row
+    are infinite: nothing of them may reach the products of the rows in front of them, whose last pieces end where
+    these begin in memory."""
+    torch.manual_seed(k)
+    sizes = _sizes(groups, rows, seed=k + rows, empty=(0,) if groups > 2 else ())
+    a, a2 = (torch.randn(rows, k, device='cuda').to(dtype) for _ in range(2))
+    wt, wt2 = ((torch.randn(groups, n, k, device='cuda') / k ** 0.5).to(dtype) for _ in range(2))      # NT
+    w, w2 = ((torch.randn(groups, k, n, device='cuda') / k ** 0.5).to(dtype) for _ in range(2))        # NN
+    bad_row, bad_col = rows // 2, n - 1
+    a[bad_row] = float('inf')
+    wt[:, bad_col] = float('inf')
+    keep = torch.ones(rows, n, dtype=torch.bool, device='cuda')
+    keep[bad_row] = False
+    nt_keep = keep.clone()
+    nt_keep[:, bad_col] = False
+
+    def check(got, want, mask):
+        got, want = (torch.where(mask, t.float(), torch.zeros((), device='cuda')) for t in (got, want))
+        assert max_block_err(got, want) < TOL
+
+    nt, nn = _ref_gpu(a, wt, sizes, False, True), _ref_gpu(a, w, sizes, False, False)
+    nt2, nn2 = _ref_gpu(a2, wt2, sizes, False, True), _ref_gpu(a2, w2, sizes, False, False)
+    for lend in (True, False):
+        monkeypatch.setattr(gg, 'GMM_WORKSPACE', lend)
+        check(gg.backend.gmm(a, wt, sizes, trans_b=True), nt, nt_keep)
+        check(gg.backend.gmm(a, w, sizes), nn, keep)
+        check(gg.gmm_dual(a, wt, a2, wt2, sizes, trans_b=True), nt + nt2, nt_keep)
+        check(gg.gmm_dual(a, w, a2, w2, sizes), nn + nn2, keep)
+    gelu = lambda t: torch.nn.functional.gelu(t.to(dtype).float(), approximate='tanh')   # noqa: E731
+    pre, act = gg.gmm_act(a, wt, sizes, fuse=True)
+    check(pre, nt, nt_keep)
+    check(act, gelu(pre), nt_keep)
+    x1, x2, h = gg.gmm_glu(a, wt, wt2, sizes, 1, fuse=True)
+    x2_ref = _ref_gpu(a, wt2, sizes, False, True)
+    check(x1, nt, nt_keep)
+    check(x2, x2_ref, keep)
+    check(h, gelu(x1) * x2.float(), nt_keep)
+    saved, saved2 = (torch.randn(rows, n, device='cuda').to(dtype) for _ in range(2))
+    check(gg.gmm_dact(a, wt, saved, sizes, fuse=True), gg.gmm_dact(a, wt, saved, sizes, fuse=False), nt_keep)
+    for got, want in zip(gg.gmm_dglu(a, wt, saved, saved2, sizes, 0, fuse=True), gg.gmm_dglu(a, wt, saved, saved2, sizes, 0, fuse=False)):
+        check(got, want, nt_keep)
+    # the combine in the store phase
+    order = torch.randperm(rows, device='cuda').int()
+    bins = torch.cumsum(sizes.cuda(), 0).int()
+    bin_ids = torch.repeat_interleave(torch.arange(groups), sizes).int().cuda()
+    weights = torch.rand(rows, device='cuda').to(dtype)
+    y, out = gg.gmm_scatter(a, w, sizes, gg.CombinedRows(order, bin_ids, bins, weights))
+    check(y, nn, keep)
+    want = torch.zeros_like(out)
+    want[order.long()] = (y.float() * weights[order.long()].float()[:, None]).to(dtype)
+    placed = torch.ones_like(keep)
+    placed[order[bad_row].long()] = False
+    assert torch.equal(torch.where(placed, out, 0), torch.where(placed, want, 0))
