@@ -1,0 +1,268 @@
+// NN / NT products of 16-bit operands where an expert has a handful of rows: decoding, short prompts, small batches
+// over many experts.
+//
+// What bounds them: the reading of the weights, once.  A row of the output costs no arithmetic to speak of (a matrix
+// instruction multiplies 16 rows whether they exist or not), so the tiles of gmm_dma.h, 256 columns by one workgroup per
+// compute unit, only make the launch coarse: 26 experts with a [2816, 2048] first product are 286 tiles on 256 compute
+// units, and their second product, 8 tiles of 22 K tiles each, is a chain of memory latencies on two thirds of the chip.
+//
+// Here the unit of work is 64 output columns of one expert by 16 of its rows.  A workgroup of eight waves walks a list of
+// units; its waves take every eighth 64-element chunk of a unit's reduction, so that they read neighbouring memory.  The
+// weights go from memory to registers as the matrix instruction wants them and are used once.  No wave waits for another
+// until the end of a unit, where the eight partial sums meet in LDS (added in wave order: results do not depend on
+// timing), and by then the loads of the workgroup's next unit are under way: two chunks per wave are in flight at all
+// times, 256 KiB per compute unit with its two workgroups.
+//
+//   NT ([n][k] weights): lane (c = l % 16, g = l / 16) reads 32 contiguous bytes of row c of a 16-row fragment, two 16-byte
+//   loads; 16 lines of 128 bytes per pair of loads.
+//   NN ([k][n] weights): lane (c, g) reads four columns (8 bytes) of eight rows k, whole 128-byte lines again, and swaps
+//   the 8 x 4 values into k order with byte permutes (32 of them per 8 KiB).
+// In a chunk, lane group g holds k = 16 g + 8 s .. + 7 for instruction s, in both operands.
+#include "gmm_common.h"
+
+#include <cstdlib>
+#include <type_traits>
+
+namespace mbx {
+namespace {
+
+#include "gmm_dma.h"   // buffer descriptors, tile list, activations
+
+namespace few {
+
+using dma::clip_bytes;
+using dma::make_rsrc;
+
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
+
+constexpr int kRows = 16, kCols = 64, kChunk = 64;
+constexpr int kPitch = kCols + 4;                                   // floats per row of a partial sum in LDS
+constexpr uint32_t kNone = 0x80000000u;   // an offset past every buffer: the load brings zeros
+
+template <int DT>
+__device__ __forceinline__ f32x4 mfma(const u32x4& a, const u32x4& b, const f32x4& c) {
+  if (DT == MBX_BF16) return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
+  return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, a), __builtin_bit_cast(f16x8_t, b), c, 0, 0, 0);
+}
+
+// One chunk's operands of a lane.
+template <bool B_MC> struct Chunk;
+template <> struct Chunk<false> { u32x4 a[2], b[2][4]; };
+template <> struct Chunk<true> { u32x4 a[2]; u32x2 b[2][8]; };
+
+// EPI: dma::kEpiNone, kEpiAct, kEpiGlu* (NT), kEpiCombine (NN).  GATHER (NT): as in gmm_dma.h's gmm_rows_kernel.
+// c / out2 may be null where only the activation (or the combine) is wanted.
+template <int DT, bool B_MC, int EPI, bool GATHER, int kWaves>
+__global__ void __launch_bounds__(kWaves * kWave, 4)
+gmm_few_kernel(const uint16_t* __restrict__ a, const uint16_t* __restrict__ b, uint16_t* __restrict__ c,
+               const int32_t* __restrict__ bins, int num_groups, int rows, int k, int n, int tiles_n,
+               const uint16_t* __restrict__ b2, uint16_t* __restrict__ extra, uint16_t* __restrict__ out2,
+               const int32_t* __restrict__ slots, const int32_t* __restrict__ src_bins, int top_k, int src_rows,
+               const void* __restrict__ combine_weights, int combine_w_dtype, int combine_tokens) {
+  __shared__ __attribute__((aligned(16))) float sums[kWaves * kRows * kPitch];
+  constexpr bool kGlu = dma::epi_is_glu(EPI);
+  constexpr int kTileCols = kGlu ? kCols / 2 : kCols;
+  const dma::RowTiles<kRows> tiles(bins, num_groups, tiles_n, rows, false, 8);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = lane_id(), col = lane & 15, g = lane >> 4;
+  const uint32_t pitch = (uint32_t)k * 2u;
+  const int chunks = (k + kChunk - 1) / kChunk;
+  const int steps = (chunks + 2 * kWaves - 1) / (2 * kWaves) * 2;   // chunks per wave, an even number; those past the last are not fetched
+
+  struct Unit { int e, start, row0, end, n0; };
+  auto locate = [&](int id) {
+    Unit u;
+    int tm, tn;
+    tiles.find(id, u.e, u.start, u.end, tm, tn);
+    u.row0 = u.start + tm * kRows;
+    u.n0 = tn * kTileCols;
+    return u;
+  };
+  auto slot_of = [&](const Unit& u) -> int {   // GATHER: the assignment of this lane's row
+    const int src_start = u.e > 0 ? src_bins[u.e - 1] : 0;
+    const int64_t slots_end = (int64_t)src_rows * top_k;
+    const int limit = (int)(src_bins[u.e] < slots_end ? src_bins[u.e] : slots_end);
+    const int j = (src_start < 0 ? 0 : src_start) + (u.row0 - u.start) + col;
+    return u.row0 + col < u.end && j < limit ? slots[j] : -1;
+  };
+  // where the loads issued now read from
+  __amdgpu_buffer_rsrc_t rsrc_a = make_rsrc(a, GATHER ? clip_bytes((int64_t)src_rows * k * 2) : 0u), rsrc_b = rsrc_a, rsrc_b2 = rsrc_a;
+  uint32_t a_off = kNone, b_off = 0;
+  auto aim = [&](const Unit& u, int slot) {
+    if constexpr (GATHER) {
+      const int row = slot >= 0 ? slot / top_k : src_rows;
+      a_off = row < src_rows ? (uint32_t)row * pitch + (uint32_t)g * 32u : kNone;
+    } else {
+      rsrc_a = make_rsrc(a + (int64_t)u.row0 * k, clip_bytes((int64_t)(u.end - u.row0) * k * 2));
+      a_off = u.row0 + col < u.end ? (uint32_t)col * pitch + (uint32_t)g * 32u : kNone;
+    }
+    rsrc_b = make_rsrc(b + (int64_t)u.e * k * n, (uint32_t)((int64_t)k * n * 2));
+    rsrc_b2 = kGlu ? make_rsrc(b2 + (int64_t)u.e * k * n, (uint32_t)((int64_t)k * n * 2)) : rsrc_b;
+    b_off = B_MC ? (uint32_t)(16 * g) * (uint32_t)n * 2u + (uint32_t)(u.n0 + col * 4) * 2u : (uint32_t)(u.n0 + col) * pitch + (uint32_t)g * 32u;
+  };
+  auto fetch = [&](Chunk<B_MC>& x, int step) {
+    const int ch = wave + step * kWaves;
+    const uint32_t byte0 = (uint32_t)ch * (kChunk * 2), none = ch < chunks ? 0u : kNone;
+    uint32_t b_at = B_MC ? (b_off + (uint32_t)ch * kChunk * (uint32_t)n * 2u) | none : b_off + byte0;
+    asm volatile("" : "+v"(b_at));   // the loads' addresses are sums with scalars, not sixteen registers carried through the loop
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      // pieces past the end of the reduction read as zeros (k is a multiple of 8); NN: rows past k are past the buffer
+      const uint32_t past = ch * kChunk + 16 * g + 8 * s < k ? none : kNone;
+      x.a[s] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc_a, (int)((a_off + byte0 + 16u * s) | past | (a_off & kNone)), 0, 0));
+      if constexpr (B_MC) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+          x.b[s][i] = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(rsrc_b, (int)(b_at + (8u * s + i) * (uint32_t)n * 2u), 0, 0));
+      } else {
+#pragma unroll
+        for (int f = 0; f < 4; ++f) {
+          const uint32_t rows_on = kGlu ? (uint32_t)(f & 1) * 16u : (uint32_t)f * 16u;
+          x.b[s][f] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(kGlu && f >= 2 ? rsrc_b2 : rsrc_b, (int)((b_at + rows_on * pitch + 16u * s) | past), 0, 0));
+        }
+      }
+    }
+  };
+  f32x4 acc[4];
+  auto multiply = [&](const Chunk<B_MC>& x) {
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+#pragma unroll
+      for (int f = 0; f < 4; ++f) {
+        u32x4 bf;
+        if constexpr (B_MC) {   // fragment f: columns 4 (lane % 16) + f
+          const uint32_t sel = f & 1 ? 0x07060302u : 0x05040100u;
+#pragma unroll
+          for (int w = 0; w < 4; ++w) bf[w] = __builtin_amdgcn_perm(x.b[s][2 * w + 1][f >> 1], x.b[s][2 * w][f >> 1], sel);
+        } else {
+          bf = x.b[s][f];
+        }
+        acc[f] = mfma<DT>(bf, x.a[s], acc[f]);
+      }
+  };
+  // eight columns of a row of the finished unit
+  auto total = [&](int m, int ch8, float (&f)[8]) {
+#pragma unroll
+    for (int t = 0; t < 8; ++t) f[t] = 0.f;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) {
+      const f32x4* p = (const f32x4*)(sums + (size_t)(w * kRows + m) * kPitch + ch8 * 8);
+      const f32x4 lo = p[0], hi = p[1];
+#pragma unroll
+      for (int t = 0; t < 4; ++t) { f[t] += lo[t]; f[4 + t] += hi[t]; }
+    }
+  };
+
+  if ((int)blockIdx.x >= tiles.total) return;
+  const Unit cur = locate(blockIdx.x);
+  aim(cur, GATHER ? slot_of(cur) : 0);
+  Chunk<B_MC> x0, x1;
+  fetch(x0, 0);
+#pragma unroll
+  for (int f = 0; f < 4; ++f) acc[f] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int step = 0; step < steps; step += 2) {
+    fetch(x1, step + 1);
+    __builtin_amdgcn_sched_barrier(0);   // a chunk's loads are all issued before the products of the one before it
+    multiply(x0);
+    __builtin_amdgcn_sched_barrier(0);
+    fetch(x0, step + 2);
+    __builtin_amdgcn_sched_barrier(0);
+    multiply(x1);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+    // partial sums: sums[wave][row][column]
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      // NT: fragment q, columns 16 q + 4 g + r.  NN: register q of the four fragments, columns 4 (4 g + q) + f.
+      f32x4 v;
+      if constexpr (B_MC) {
+#pragma unroll
+        for (int f = 0; f < 4; ++f) v[f] = acc[f][q];
+      } else {
+        v = acc[q];
+      }
+      *(f32x4*)(sums + (size_t)(wave * kRows + col) * kPitch + (B_MC ? 16 * g + 4 * q : 16 * q + 4 * g)) = v;
+    }
+    __syncthreads();
+    constexpr int kItems = kTileCols / 8;
+    const int m = threadIdx.x / kItems, ch8 = threadIdx.x % kItems, row = cur.row0 + m, cn = cur.n0 + ch8 * 8;
+    if (m < kRows && row < cur.end && cn < n) {   // n is a multiple of 8
+      const int64_t at = (int64_t)row * n + cn;
+      float f[8];
+      total(m, ch8, f);
+      const u32x4 v = dma::pack8<DT>(f);
+      if constexpr (kGlu) {
+        total(m, ch8 + kItems, f);
+        const u32x4 v2 = dma::pack8<DT>(f);
+        if (c != nullptr) {
+          *(u32x4*)(c + at) = v;
+          *(u32x4*)(out2 + at) = v2;
+        }
+        *(u32x4*)(extra + at) = dma::glu_chunk<DT, EPI == dma::kEpiGluGelu>(v, v2);
+      } else {
+        if (c != nullptr) *(u32x4*)(c + at) = v;
+        if constexpr (EPI == dma::kEpiAct) *(u32x4*)(extra + at) = dma::gelu_fwd_chunk<DT>(v);
+        if constexpr (EPI == dma::kEpiCombine) {
+          dma::Combine cb;
+          cb.weights = combine_weights;
+          cb.w_dtype = combine_w_dtype;
+          cb.tokens = combine_tokens;
+          cb.token = slots[row];
+          cb.row_exists = true;
+          const int token = dma::combine_token(cb);
+          if (token >= 0) *(u32x4*)(extra + (int64_t)token * n + cn) = dma::scale_chunk<DT>(v, dma::combine_weight(cb, token));
+        }
+      }
+    }
+}
+
+}  // namespace few
+
+template <int DT, bool B_MC, int EPI, bool GATHER, int W>
+int launch_few_w(const DmaCall& q, const int32_t* slots) {
+  const int cols = dma::epi_is_glu(EPI) ? few::kCols / 2 : few::kCols;
+  const int tiles_n = (int)ceil_div(q.n, cols);
+  const int64_t row_tiles = (q.rows < q.num_groups ? q.rows : q.num_groups) + q.rows / few::kRows;
+  if (row_tiles * tiles_n > 0x7fffffff) return MBX_ERANGE;
+  few::gmm_few_kernel<DT, B_MC, EPI, GATHER, W><<<(unsigned)(row_tiles * tiles_n), W * kWave, 0, q.stream>>>(
+      (const uint16_t*)q.a, (const uint16_t*)q.b, (uint16_t*)q.c, q.bins, q.num_groups, (int)q.rows, q.k, q.n, tiles_n,
+      (const uint16_t*)q.b2, (uint16_t*)q.extra, (uint16_t*)q.out2, slots, q.gather.src_bins, q.gather.top_k, q.gather.src_rows,
+      q.combine.weights, q.combine.w_dtype, q.combine.tokens);
+  return launch_status();
+}
+
+template <int DT, bool B_MC, int EPI, bool GATHER>
+int launch_few(const DmaCall& q, const int32_t* slots) {
+  static const int w = [] { const char* v = getenv("MBX_FEW_W"); return v ? atoi(v) : 4; }();
+  return w == 4 ? launch_few_w<DT, B_MC, EPI, GATHER, 4>(q, slots) : launch_few_w<DT, B_MC, EPI, GATHER, 8>(q, slots);
+}
+
+template <int DT>
+int dispatch_few(const DmaCall& q) {
+  if (q.layout == MBX_NN) {
+    if (q.epi == dma::kEpiCombine) return launch_few<DT, true, dma::kEpiCombine, false>(q, q.combine.indices);
+    return launch_few<DT, true, dma::kEpiNone, false>(q, nullptr);
+  }
+#define MBX_FEW_NT(EPI) (q.gather.slots ? launch_few<DT, false, EPI, true>(q, q.gather.slots) : launch_few<DT, false, EPI, false>(q, nullptr))
+  switch (q.epi) {
+    case dma::kEpiNone: return MBX_FEW_NT(dma::kEpiNone);
+    case dma::kEpiAct: return MBX_FEW_NT(dma::kEpiAct);
+    case dma::kEpiGluSilu: return MBX_FEW_NT(dma::kEpiGluSilu);
+    default: return MBX_FEW_NT(dma::kEpiGluGelu);
+  }
+#undef MBX_FEW_NT
+}
+
+}  // namespace
+
+bool gmm_few_takes(const DmaCall& q) {
+  const bool form = q.layout == MBX_NN ? (q.epi == dma::kEpiNone || q.epi == dma::kEpiCombine)
+                                       : (q.layout == MBX_NT && (q.epi == dma::kEpiNone || q.epi == dma::kEpiAct || dma::epi_is_glu(q.epi)));
+  if (!form || (q.a2 && !dma::epi_is_glu(q.epi))) return false;
+  static const int limit = [] { const char* v = getenv("MBX_FEW"); return v ? atoi(v) : 8; }();
+  return q.rows <= (int64_t)limit * q.num_groups;
+}
+
+int gmm_few(const DmaCall& q) { return q.dtype == MBX_BF16 ? dispatch_few<MBX_BF16>(q) : dispatch_few<MBX_F16>(q); }
+
+}  // namespace mbx
