@@ -1352,6 +1352,13 @@ gmm_rows_kernel(const uint16_t* __restrict__ a, const uint16_t* __restrict__ b, 
   const int items = big_rounds + ((ksplit > 1 || (kSplit && split)) ? 1 : 0);
   // first K tile of part p of a reduction cut into ksplit parts; with two operand pairs a cut within SB K tiles of the
   // pairs' boundary moves onto it (the main loop changes pairs at least SB + 1 K tiles into a call)
+  // Item `m` (this workgroup's place among its XCD's members) of the `count` items of the last, partly filled round, dealt
+  // to the XCDs in equal consecutive shares; -1: none.  (Dealt in whole runs they would leave the last XCDs idle while
+  // the first ones stream their operands through one L2 each.)
+  auto shared_out = [&](int count, int m) -> int {
+    const int first = (int)((int64_t)xcd * count / kXcds), next = (int)((int64_t)(xcd + 1) * count / kXcds);
+    return m < next - first ? first + m : -1;
+  };
   auto part_begin = [&](int p_) -> int {
     int t_ = (int)((int64_t)p_ * nk_all / ksplit);
     if (DUAL && t_ - nk1 < T::SB + 1 && nk1 - t_ < T::SB + 1) t_ = nk1;
@@ -1385,14 +1392,17 @@ gmm_rows_kernel(const uint16_t* __restrict__ a, const uint16_t* __restrict__ b, 
   auto locate = [&](int r, int& e, int& start, int& end, int& tn, int& row0, bool& tail_half) -> bool {
     int id, half = 0;
     tail_half = false;
-    if (r < big_rounds) {
+    if (r < full_rounds) {
       // Rotated by one member per round: where full and half-height tiles alternate along the list, a
       // workgroup would otherwise be dealt the same kind in every round.
       id = (r * kXcds + xcd) * run + (member + r) % run;
-      if (id >= total) return false;
+    } else if (r < big_rounds) {
+      const int j = shared_out(rest, (member + r) % run);
+      if (j < 0) return false;
+      id = full_rounds * P + j;
     } else {
-      const int j = xcd * run + member;   // half tile j: tile j / 2 of the tail, rows half j % 2
-      if (j >= 2 * rest) return false;
+      const int j = shared_out(2 * rest, member);   // half tile j: tile j / 2 of the tail, rows half j % 2
+      if (j < 0) return false;
       id = full_rounds * P + j / 2;
       half = j & 1;
       tail_half = true;
@@ -1406,14 +1416,17 @@ gmm_rows_kernel(const uint16_t* __restrict__ a, const uint16_t* __restrict__ b, 
     for (int r = 0; r < items; ++r) {
       int id, half = 0;
       bool use_ts = false;
-      if (r < big_rounds) {
+      if (r < full_rounds) {
         id = (r * kXcds + xcd) * run + (member + r) % run;   // as in locate()
-        if (id >= total) break;
+      } else if (r < big_rounds) {
+        const int j = shared_out(rest, (member + r) % run);
+        if (j < 0) break;
+        id = full_rounds * P + j;
       } else if (kSplitK && ksplit > 1) {
         if constexpr (kSplitK) {
           // part `part` of tail tile `tile`: consecutive workgroups of an XCD take the same part of consecutive tiles
-          const int j = xcd * run + member;
-          if (j >= ksplit * rest) break;
+          const int j = shared_out(ksplit * rest, member);
+          if (j < 0) break;
           const int tile = j % rest, part = j / rest;
           g.tick_ordinal = r;
           MBX_TICK(r, 0);
@@ -1512,8 +1525,8 @@ gmm_rows_kernel(const uint16_t* __restrict__ a, const uint16_t* __restrict__ b, 
         }
         continue;
       } else {
-        const int j = xcd * run + member;
-        if (j >= 2 * rest) break;
+        const int j = shared_out(2 * rest, member);
+        if (j < 0) break;
         id = full_rounds * P + j / 2;
         half = j & 1;
         use_ts = true;
