@@ -57,6 +57,10 @@ struct DmaCall {
   CombineRows combine{};
 };
 
+// NN / NT launches with a handful of rows per expert (gmm_few.hip), and whether a launch is one of them.
+bool gmm_few_takes(const DmaCall& call);
+int gmm_few(const DmaCall& call);
+
 // NN / NT launches, k a multiple of 64 (gmm_rows.hip) and of 8 only (gmm_rows_tail.hip).
 int gmm_rows(const DmaCall& call);
 int gmm_rows_tail(const DmaCall& call);

@@ -6,12 +6,21 @@
 // compute unit, only make the launch coarse: 26 experts with a [2816, 2048] first product are 286 tiles on 256 compute
 // units, and their second product, 8 tiles of 22 K tiles each, is a chain of memory latencies on two thirds of the chip.
 //
-// Here the unit of work is 64 output columns of one expert by 16 of its rows.  A workgroup of eight waves walks a list of
-// units; its waves take every eighth 64-element chunk of a unit's reduction, so that they read neighbouring memory.  The
-// weights go from memory to registers as the matrix instruction wants them and are used once.  No wave waits for another
-// until the end of a unit, where the eight partial sums meet in LDS (added in wave order: results do not depend on
-// timing), and by then the loads of the workgroup's next unit are under way: two chunks per wave are in flight at all
-// times, 256 KiB per compute unit with its two workgroups.
+// Here a workgroup of four waves takes 64 output columns of one expert and 16 of its rows, and each wave a quarter of the
+// reduction in chunks of 64.  The weights go from memory to registers as the matrix instruction wants them and are used
+// once; no wave waits for another until the end, where the four partial sums meet in LDS (added in wave order: results do
+// not depend on timing).  Two chunks per wave are in flight, and four workgroups share a compute unit: 256 KiB of weights
+// under way.  (Eight waves per workgroup: 2 - 12 % slower where the reduction is short, no faster elsewhere.  Workgroups
+// that walk a list of units with the next unit's loads under way: the registers for two units' addresses spill, 82
+// against 71 us on 64 experts of 4 rows, [1408, 2048].  32 or 64 rows at a time: the registers of one workgroup leave
+// too few loads in flight, 3.8 against 5.0 TB/s.)
+//
+// Measured (bf16, TB/s of the weights of the experts that got rows, gmm_dma.h's kernel / this one; a plain read reaches 5.8):
+//   8 experts x 4 rows, [14336, 4096]: gated first products 4.8 - 5.4 (by placement) / 5.6, second product 5.17 / 5.52
+//   64 x 4, [1408, 2048]: 5.21 / 5.32, 5.58 / 5.59;  25 of 64 experts with a row or two: 3.88 / 4.73, 4.66 / 4.76
+//   64 x 4, [3840, 1024]: 5.29 / 5.37, 5.62 / 5.66;  6 of 64 experts: 4.19 / 5.07, 1.52 / 3.75
+//   32 x 4, [2816, 3072]: 5.33 / 4.80, 4.85 / 5.12;  3 of 32 experts: 2.34 / 3.51, 1.66 / 4.29
+//   16 x 4, [1408, 1024]: 4.32 / 3.91, 1.98 / 3.78
 //
 //   NT ([n][k] weights): lane (c = l % 16, g = l / 16) reads 32 contiguous bytes of row c of a 16-row fragment, two 16-byte
 //   loads; 16 lines of 128 bytes per pair of loads.
@@ -20,7 +29,7 @@
 // In a chunk, lane group g holds k = 16 g + 8 s .. + 7 for instruction s, in both operands.
 #include "gmm_common.h"
 
-#include <cstdlib>
+#include <cmath>
 #include <type_traits>
 
 namespace mbx {
@@ -36,7 +45,7 @@ using dma::make_rsrc;
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
 
-constexpr int kRows = 16, kCols = 64, kChunk = 64;
+constexpr int kWaves = 4, kThreads = kWaves * kWave, kRows = 16, kCols = 64, kChunk = 64;
 constexpr int kPitch = kCols + 4;                                   // floats per row of a partial sum in LDS
 constexpr uint32_t kNone = 0x80000000u;   // an offset past every buffer: the load brings zeros
 
@@ -52,9 +61,9 @@ template <> struct Chunk<false> { u32x4 a[2], b[2][4]; };
 template <> struct Chunk<true> { u32x4 a[2]; u32x2 b[2][8]; };
 
 // EPI: dma::kEpiNone, kEpiAct, kEpiGlu* (NT), kEpiCombine (NN).  GATHER (NT): as in gmm_dma.h's gmm_rows_kernel.
-// c / out2 may be null where only the activation (or the combine) is wanted.
-template <int DT, bool B_MC, int EPI, bool GATHER, int kWaves>
-__global__ void __launch_bounds__(kWaves * kWave, 4)
+// c (with the gate: and out2) may be null where only the epilogue's output is wanted.
+template <int DT, bool B_MC, int EPI, bool GATHER>
+__global__ void __launch_bounds__(kThreads, 4)
 gmm_few_kernel(const uint16_t* __restrict__ a, const uint16_t* __restrict__ b, uint16_t* __restrict__ c,
                const int32_t* __restrict__ bins, int num_groups, int rows, int k, int n, int tiles_n,
                const uint16_t* __restrict__ b2, uint16_t* __restrict__ extra, uint16_t* __restrict__ out2,
@@ -67,7 +76,7 @@ gmm_few_kernel(const uint16_t* __restrict__ a, const uint16_t* __restrict__ b, u
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = lane_id(), col = lane & 15, g = lane >> 4;
   const uint32_t pitch = (uint32_t)k * 2u;
   const int chunks = (k + kChunk - 1) / kChunk;
-  const int steps = (chunks + 2 * kWaves - 1) / (2 * kWaves) * 2;   // chunks per wave, an even number; those past the last are not fetched
+  const int steps = (chunks + 2 * kWaves - 1) / (2 * kWaves) * 2;   // chunks per wave, an even number; those past the last chunk are not fetched
 
   struct Unit { int e, start, row0, end, n0; };
   auto locate = [&](int id) {
@@ -100,9 +109,15 @@ gmm_few_kernel(const uint16_t* __restrict__ a, const uint16_t* __restrict__ b, u
     rsrc_b2 = kGlu ? make_rsrc(b2 + (int64_t)u.e * k * n, (uint32_t)((int64_t)k * n * 2)) : rsrc_b;
     b_off = B_MC ? (uint32_t)(16 * g) * (uint32_t)n * 2u + (uint32_t)(u.n0 + col * 4) * 2u : (uint32_t)(u.n0 + col) * pitch + (uint32_t)g * 32u;
   };
+  // A wave's chunks are a quarter of the reduction, and the columns start at different places in it and go round: started
+  // together at its beginning, the workgroups would all read the first bytes of rows that are a power of two apart, and
+  // which memory channels those fall on is a matter of where the weights lie (the same launch took 341 to 456 us on
+  // different copies of the same weights; now 335 to 336).
+  int turn = 0;
   auto fetch = [&](Chunk<B_MC>& x, int step) {
-    const int ch = wave + step * kWaves;
-    const uint32_t byte0 = (uint32_t)ch * (kChunk * 2), none = ch < chunks ? 0u : kNone;
+    const int at = step + turn < steps ? step + turn : step + turn - steps;
+    const int ch = wave * steps + at;
+    const uint32_t byte0 = (uint32_t)ch * (kChunk * 2), none = step < steps && ch < chunks ? 0u : kNone;
     uint32_t b_at = B_MC ? (b_off + (uint32_t)ch * kChunk * (uint32_t)n * 2u) | none : b_off + byte0;
     asm volatile("" : "+v"(b_at));   // the loads' addresses are sums with scalars, not sixteen registers carried through the loop
 #pragma unroll
@@ -156,6 +171,7 @@ gmm_few_kernel(const uint16_t* __restrict__ a, const uint16_t* __restrict__ b, u
   if ((int)blockIdx.x >= tiles.total) return;
   const Unit cur = locate(blockIdx.x);
   aim(cur, GATHER ? slot_of(cur) : 0);
+  turn = (int)(((uint32_t)(cur.n0 / kCols) * 5u + (uint32_t)cur.e * 3u) % (uint32_t)steps);
   Chunk<B_MC> x0, x1;
   fetch(x0, 0);
 #pragma unroll
@@ -218,23 +234,18 @@ gmm_few_kernel(const uint16_t* __restrict__ a, const uint16_t* __restrict__ b, u
 
 }  // namespace few
 
-template <int DT, bool B_MC, int EPI, bool GATHER, int W>
-int launch_few_w(const DmaCall& q, const int32_t* slots) {
+template <int DT, bool B_MC, int EPI, bool GATHER>
+int launch_few(const DmaCall& q, const int32_t* slots) {
   const int cols = dma::epi_is_glu(EPI) ? few::kCols / 2 : few::kCols;
   const int tiles_n = (int)ceil_div(q.n, cols);
+  // an upper bound: the row counts are only known on the device
   const int64_t row_tiles = (q.rows < q.num_groups ? q.rows : q.num_groups) + q.rows / few::kRows;
   if (row_tiles * tiles_n > 0x7fffffff) return MBX_ERANGE;
-  few::gmm_few_kernel<DT, B_MC, EPI, GATHER, W><<<(unsigned)(row_tiles * tiles_n), W * kWave, 0, q.stream>>>(
+  few::gmm_few_kernel<DT, B_MC, EPI, GATHER><<<(unsigned)(row_tiles * tiles_n), few::kThreads, 0, q.stream>>>(
       (const uint16_t*)q.a, (const uint16_t*)q.b, (uint16_t*)q.c, q.bins, q.num_groups, (int)q.rows, q.k, q.n, tiles_n,
       (const uint16_t*)q.b2, (uint16_t*)q.extra, (uint16_t*)q.out2, slots, q.gather.src_bins, q.gather.top_k, q.gather.src_rows,
       q.combine.weights, q.combine.w_dtype, q.combine.tokens);
   return launch_status();
-}
-
-template <int DT, bool B_MC, int EPI, bool GATHER>
-int launch_few(const DmaCall& q, const int32_t* slots) {
-  static const int w = [] { const char* v = getenv("MBX_FEW_W"); return v ? atoi(v) : 4; }();
-  return w == 4 ? launch_few_w<DT, B_MC, EPI, GATHER, 4>(q, slots) : launch_few_w<DT, B_MC, EPI, GATHER, 8>(q, slots);
 }
 
 template <int DT>
@@ -255,12 +266,22 @@ int dispatch_few(const DmaCall& q) {
 
 }  // namespace
 
+// Up to eight rows per expert on average (beyond, experts of more than 16 rows read their weights twice: 16 rows per expert
+// cost 20 - 40 %).  NN: wherever gmm_dma.h's tiles would leave the chip partly idle.  NT: that kernel keeps up as long as
+// its rounds of tiles are about three quarters full (32 experts, [2816, 3072]: 195 against 216 us with 0.86 of them full,
+// 124 against 134 with 0.77; 25 of 64 experts, [1408, 2048]: 74 against 61 with 0.54), with short reductions, sixteen
+// chunks of which are four per wave here, longer still (16 experts, [1408, 1024]: 21 against 24 us with 0.69), and with
+// long ones it depends on where the weights lie (8 experts, [14336, 4096]: 347 - 398 against 335 us).
+// The number of experts that get rows is an expectation: rows that choose evenly.  The epilogues do not enter the rule: the
+// product of a launch with one is the plain launch's, bit for bit.
 bool gmm_few_takes(const DmaCall& q) {
-  const bool form = q.layout == MBX_NN ? (q.epi == dma::kEpiNone || q.epi == dma::kEpiCombine)
-                                       : (q.layout == MBX_NT && (q.epi == dma::kEpiNone || q.epi == dma::kEpiAct || dma::epi_is_glu(q.epi)));
-  if (!form || (q.a2 && !dma::epi_is_glu(q.epi))) return false;
-  static const int limit = [] { const char* v = getenv("MBX_FEW"); return v ? atoi(v) : 8; }();
-  return q.rows <= (int64_t)limit * q.num_groups;
+  const bool nn = q.layout == MBX_NN && (q.epi == dma::kEpiNone || q.epi == dma::kEpiCombine) && !q.a2;
+  const bool nt = q.layout == MBX_NT && (q.epi == dma::kEpiAct || dma::epi_is_glu(q.epi) || (q.epi == dma::kEpiNone && !q.a2));
+  if (!(nn || nt) || q.rows > 8 * (int64_t)q.num_groups) return false;
+  const double experts = q.num_groups * (1.0 - pow(1.0 - 1.0 / q.num_groups, (double)q.rows));
+  const double rounds = experts * (double)ceil_div(q.n, nn ? 256 : 128) / persistent_grid((int64_t)1 << 30);
+  const double filled = rounds / ceil(rounds);
+  return nn ? filled < 0.92 : q.k >= 4096 || filled < (q.k >= 2048 ? 0.7 : 0.5);
 }
 
 int gmm_few(const DmaCall& q) { return q.dtype == MBX_BF16 ? dispatch_few<MBX_BF16>(q) : dispatch_few<MBX_F16>(q); }

@@ -1001,3 +1001,63 @@ def test_gmm_reductions_that_end_inside_a_k_tile(gg, monkeypatch, groups, rows, 
     placed = torch.ones_like(keep)
     placed[order[bad_row].long()] = False
     assert torch.equal(torch.where(placed, out, 0), torch.where(placed, want, 0))
+
+
+@pytest.mark.parametrize('counts,k,n', [
+    ([0, 1, 16, 17, 33, 2, 0, 0, 3, 5, 1, 0], 2048, 136),      # experts around the 16 rows a workgroup takes
+    ([1] + [0] * 7, 4096, 1024), ([3, 0, 0, 1] + [0] * 60, 2048, 1408), ([2] * 16, 200, 264), ([1, 2, 1, 4] * 20, 2728, 72),
+    ([5] * 8, 64, 64), ([8] * 3, 8, 8),
+])
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])
+def test_gmm_with_a_handful_of_rows_per_expert(gg, counts, k, n, dtype):
+    """The kernels for a few rows per expert, every form they take, against fp32; k also inside a chunk, where a row's last
+    piece ends in front of a row of infinities; the forms' products equal bit for bit, and from run to run."""
+    torch.manual_seed(k + n)
+    sizes = torch.tensor(counts)
+    groups, rows = len(counts), int(sizes.sum())
+    a = torch.randn(rows, k, device='cuda').to(dtype)
+    w1, v1 = ((torch.randn(groups, n, k, device='cuda') / k ** 0.5).to(dtype) for _ in range(2))
+    w2 = (torch.randn(groups, k, n, device='cuda') / k ** 0.5).to(dtype)
+    bad = rows // 2
+    w1[:, n - 1] = float('inf')
+    keep = torch.ones(rows, n, dtype=torch.bool, device='cuda')
+    if rows > 1:
+        a[bad] = float('inf')
+        keep[bad] = False
+    nt_keep = keep.clone()
+    nt_keep[:, n - 1] = False
+
+    def check(got, want, mask):
+        got, want = (torch.where(mask, t.float(), torch.zeros((), device='cuda')) for t in (got, want))
+        assert rel_err(got, want) < TOL and max_block_err(got, want, 8, 32) < 4 * TOL
+
+    c = gg.backend.gmm(a, w1, sizes, trans_b=True)
+    check(c, _ref_gpu(a, w1, sizes, False, True), nt_keep)
+    assert torch.equal(c[:, :n - 1][keep[:, :n - 1]], gg.backend.gmm(a, w1, sizes, trans_b=True)[:, :n - 1][keep[:, :n - 1]])
+    finite = lambda t: torch.where(nt_keep, t, torch.zeros((), dtype=dtype, device='cuda'))   # noqa: E731
+    pre, act = gg.gmm_act(a, w1, sizes, fuse=True)
+    assert torch.equal(finite(pre), finite(c))
+    check(act, torch.nn.functional.gelu(c.float(), approximate='tanh'), nt_keep)
+    for code, fn in ((0, torch.nn.functional.silu), (1, lambda t: torch.nn.functional.gelu(t, approximate='tanh'))):
+        x1, x2, h = gg.gmm_glu(a, w1, v1, sizes, code, fuse=True)
+        assert torch.equal(finite(x1), finite(c))
+        check(x2, _ref_gpu(a, v1, sizes, False, True), keep)
+        check(h, fn(x1.float()).to(dtype).float() * x2.float(), nt_keep)
+    y = gg.backend.gmm(a, w2, sizes)
+    check(y, _ref_gpu(a, w2, sizes, False, False), keep)
+    # one expert per token: the rows picked from, and combined to, the tokens' places
+    order = torch.randperm(rows, device='cuda').int()
+    bins = torch.cumsum(sizes.cuda(), 0).int()
+    bin_ids = torch.repeat_interleave(torch.arange(groups), sizes).int().cuda()
+    weights = torch.rand(rows, device='cuda').to(dtype)
+    y2, out = gg.gmm_scatter(a, w2, sizes, gg.CombinedRows(order, bin_ids, bins, weights))
+    assert torch.equal(y2[keep], y[keep])
+    placed = torch.ones(rows, dtype=torch.bool, device='cuda')
+    placed[order[bad].long()] = rows == 1
+    want = gg.CombinedRows(order, bin_ids, bins, weights).scatter(y)
+    assert torch.equal(out[placed], want[placed])
+    if k % 64 == 0:
+        src = gg.GatheredRows(a, order, bin_ids, bins, None, 1, rows)
+        (g,) = gg.gmm_gather(src, w1, sizes)
+        mask = keep[order.long()] & nt_keep[0]
+        assert torch.equal(g[mask], gg.backend.gmm(src.materialize(), w1, sizes, trans_b=True)[mask])
