@@ -114,8 +114,14 @@ constexpr int kRadixBits = 8;
 constexpr int kRadix = 1 << kRadixBits;
 constexpr int kSortThreads = 256;
 constexpr int kSortWaves = kSortThreads / kWave;
-constexpr int kSortItems = 8;                                  // rounds of 64 keys per wave
-constexpr int kSortTile = kSortThreads * kSortItems;           // keys per block
+// Rounds of 64 keys per wave: the rounds of a wave are a serial chain (ballots, a cursor in LDS), and 2048 keys to a block
+// leave a batch of 16384 assignments on eight compute units (count + scan + scatter of 64 experts: 24 us; with two rounds
+// 11 us).  From 64 Ki keys on there are blocks enough, and the longer count table would cost the scan more than
+// the shorter chains give.
+constexpr int kSortItemsShort = 2, kSortItemsLong = 8;
+static inline int sort_items(int64_t n) { return n <= 65536 ? kSortItemsShort : kSortItemsLong; }
+static inline int sort_tile(int64_t n) { return kSortThreads * sort_items(n); }   // keys per block
+constexpr int kSortTileMax = kSortThreads * kSortItemsLong;
 
 template <typename T> struct UnsignedOf;
 template <> struct UnsignedOf<int16_t> { typedef uint16_t type; };
@@ -132,14 +138,14 @@ __device__ __forceinline__ uint32_t digit_of(T key, int shift, uint32_t mask) {
 }
 
 // Pass step 1: digit counts of every tile, stored digit-major: counts[d * nblocks + block].
-template <typename T>
+template <typename T, int kSortItems>
 __global__ void __launch_bounds__(kSortThreads)
 radix_count_kernel(const T* __restrict__ keys, int64_t n, int shift, uint32_t mask, int nbits,
                    int32_t* __restrict__ counts, int nblocks) {
   __shared__ int32_t hist[kRadix];
   hist[threadIdx.x] = 0;
   __syncthreads();
-  const int64_t base = (int64_t)blockIdx.x * kSortTile;
+  const int64_t base = (int64_t)blockIdx.x * (kSortThreads * kSortItems);
 #pragma unroll
   for (int it = 0; it < kSortItems; ++it) {
     const int64_t i = base + it * kSortThreads + threadIdx.x;
@@ -152,25 +158,35 @@ radix_count_kernel(const T* __restrict__ keys, int64_t n, int shift, uint32_t ma
   counts[(int64_t)threadIdx.x * nblocks + blockIdx.x] = hist[threadIdx.x];
 }
 
-// Pass step 2: exclusive scan, in place, of the digit-major count table (one block of 1024 threads).
+// Pass step 2: exclusive scan, in place, of the digit-major count table (one block of 1024 threads, four entries per
+// thread and round: the table of 196608 keys of 64 experts, 6144 entries, in two rounds instead of six).
 __device__ __forceinline__ void block_exclusive_scan_i32(int32_t* __restrict__ data, int64_t n) {
   __shared__ int32_t wave_tot[16];
-  __shared__ int32_t carry_s;
-  if (threadIdx.x == 0) carry_s = 0;
-  __syncthreads();
   const int lane = lane_id(), wave = threadIdx.x / kWave;
-  for (int64_t base = 0; base < n; base += 1024) {
-    const int64_t i = base + threadIdx.x;
-    const int32_t v = i < n ? data[i] : 0;
-    int32_t inc = wave_inclusive_scan(v);
+  int32_t carry = 0;
+  for (int64_t base = 0; base < n; base += 4096) {
+    const int64_t i = base + (int64_t)threadIdx.x * 4;
+    int32_t v[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) v[q] = i + q < n ? data[i + q] : 0;
+    const int32_t mine = v[0] + v[1] + v[2] + v[3];
+    const int32_t inc = wave_inclusive_scan(mine);
     if (lane == 63) wave_tot[wave] = inc;
     __syncthreads();
-    int32_t wave_off = 0;
-    for (int w = 0; w < wave; ++w) wave_off += wave_tot[w];
-    const int32_t carry = carry_s;
-    if (i < n) data[i] = carry + wave_off + inc - v;
-    __syncthreads();
-    if (threadIdx.x == 1023) carry_s = carry + wave_off + inc;
+    int32_t before = 0, all = 0;
+#pragma unroll
+    for (int w = 0; w < 16; ++w) {
+      const int32_t t = wave_tot[w];
+      before += w < wave ? t : 0;
+      all += t;
+    }
+    int32_t run = carry + before + inc - mine;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      if (i + q < n) data[i + q] = run;
+      run += v[q];
+    }
+    carry += all;
     __syncthreads();
   }
 }
@@ -216,7 +232,7 @@ route_scan_kernel(int32_t* __restrict__ table, int ndigits, int nblocks, int32_t
 // that holds it: p itself, or with padded_bins the row p - bins[e - 1] + padded_bins[e - 1] of expert e's padded
 // block (-1 for a key whose digit is at or past num_bins) -- the map inverse_map_kernel of the permutation kernels
 // builds.
-template <typename T, bool IOTA>
+template <typename T, bool IOTA, int kSortItems>
 __global__ void __launch_bounds__(kSortThreads)
 radix_scatter_kernel(const T* __restrict__ keys_in, const T* __restrict__ vals_in, int64_t n,
                      int shift, uint32_t mask, int nbits, const int32_t* __restrict__ offsets,
@@ -228,7 +244,7 @@ radix_scatter_kernel(const T* __restrict__ keys_in, const T* __restrict__ vals_i
   for (int w = 0; w < kSortWaves; ++w) wave_hist[w][threadIdx.x] = 0;
   __syncthreads();
 
-  const int64_t wave_base = (int64_t)blockIdx.x * kSortTile + (int64_t)wave * (kWave * kSortItems);
+  const int64_t wave_base = (int64_t)blockIdx.x * (kSortThreads * kSortItems) + (int64_t)wave * (kWave * kSortItems);
   T key[kSortItems];
   uint32_t dig[kSortItems];
 #pragma unroll
@@ -283,6 +299,88 @@ radix_scatter_kernel(const T* __restrict__ keys_in, const T* __restrict__ vals_i
   }
 }
 
+// The whole of mbx_route in one launch for short lists (decoding, short prompts): a block of 16 waves, wave w owning
+// rounds of 64 consecutive keys, `rounds` of them, as in radix_scatter_kernel; the counts never leave LDS.  30 assignments
+// of 64 experts: 15.0 us and two gaps between launches -> 3.2; 2001: 22.7 -> 8.4.  Beyond four rounds
+// the three launches, which spread over the chip, are the faster way.
+constexpr int kRouteThreads = 1024, kRouteWaves = kRouteThreads / kWave, kRouteRounds = 4;
+constexpr int64_t kRouteOneBlock = (int64_t)kRouteThreads * kRouteRounds;
+__global__ void __launch_bounds__(kRouteThreads)
+route_one_block_kernel(const int32_t* __restrict__ ids, int n, uint32_t mask, int nbits, int num_experts, int pad,
+                       int32_t* __restrict__ indices, int32_t* __restrict__ bin_ids, int32_t* __restrict__ tokens_per_expert,
+                       int32_t* __restrict__ bins, int32_t* __restrict__ padded_bins, int32_t* __restrict__ slot_rows) {
+  __shared__ int32_t cursor[kRouteWaves][kRadix];
+  __shared__ int32_t shift_of[kRadix];                          // from a sorted position to its row of the padded buffer
+  __shared__ int32_t scan_tot[2][kRadix / kWave];
+  const int lane = lane_id(), wave = threadIdx.x / kWave;
+  const int rounds = (n + kRouteThreads - 1) / kRouteThreads;   // uniform
+  for (int i = threadIdx.x; i < kRouteWaves * kRadix; i += kRouteThreads) (&cursor[0][0])[i] = 0;
+  __syncthreads();
+  volatile int32_t* const cur = cursor[wave];
+  int32_t key[kRouteRounds];
+  uint64_t peers[kRouteRounds];
+  const int wave_base = wave * kWave * rounds;
+#pragma unroll
+  for (int it = 0; it < kRouteRounds; ++it) {
+    if (it >= rounds) break;
+    const int i = wave_base + it * kWave + lane;
+    const bool valid = i < n;
+    key[it] = valid ? ids[i] : 0;
+    const uint32_t d = (uint32_t)key[it] & mask;
+    peers[it] = match_peers(d, valid, nbits);
+    if (valid && (peers[it] & lanemask_lt()) == 0) cur[d] += (int32_t)__popcll(peers[it]);   // one lane per digit; the wave's own row
+    __builtin_amdgcn_wave_barrier();
+  }
+  __syncthreads();
+  // thread d: the count of digit d, its exclusive prefix, and the padded one
+  int32_t count = 0, padded = 0, inc = 0, pinc = 0;
+  const int d = threadIdx.x;
+  if (d < kRadix) {
+#pragma unroll
+    for (int w = 0; w < kRouteWaves; ++w) count += cursor[w][d];
+    padded = pad > 0 && d < num_experts ? (count + pad - 1) / pad * pad : 0;
+    inc = wave_inclusive_scan(count);
+    pinc = wave_inclusive_scan(padded);
+    if (lane == 63) { scan_tot[0][wave] = inc; scan_tot[1][wave] = pinc; }
+  }
+  __syncthreads();
+  if (d < kRadix) {
+    for (int w = 0; w < wave; ++w) { inc += scan_tot[0][w]; pinc += scan_tot[1][w]; }
+    int32_t run = inc - count;
+    if (d < num_experts) {
+      tokens_per_expert[d] = count;
+      bins[d] = inc;
+      if (padded_bins != nullptr) padded_bins[d] = pinc;
+    }
+    shift_of[d] = padded_bins != nullptr ? (pinc - padded) - run : 0;
+#pragma unroll
+    for (int w = 0; w < kRouteWaves; ++w) {
+      const int32_t c = cursor[w][d];
+      cursor[w][d] = run;
+      run += c;
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int it = 0; it < kRouteRounds; ++it) {
+    if (it >= rounds) break;
+    const int i = wave_base + it * kWave + lane;
+    const bool valid = i < n;
+    const uint32_t dg = (uint32_t)key[it] & mask;
+    int32_t pos = 0;
+    if (valid) pos = cur[dg] + (int32_t)__popcll(peers[it] & lanemask_lt());
+    __builtin_amdgcn_wave_barrier();
+    if (valid && (peers[it] & lanemask_lt()) == 0) cur[dg] += (int32_t)__popcll(peers[it]);
+    __builtin_amdgcn_wave_barrier();
+    if (valid) {
+      bin_ids[pos] = key[it];
+      indices[pos] = i;
+      // as in radix_scatter_kernel: a digit at or past num_experts has no row of the padded buffer
+      if (slot_rows != nullptr) slot_rows[i] = padded_bins == nullptr ? pos : (int)dg >= num_experts ? -1 : pos + shift_of[dg];
+    }
+  }
+}
+
 template <typename T>
 __global__ void copy_iota_kernel(const T* __restrict__ x, int64_t n, T* __restrict__ keys_out, T* __restrict__ vals_out) {
   int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -298,7 +396,7 @@ template <typename T>
 int sort_impl(const T* x, int64_t n, int end_bit, T* keys_out, T* perm_out, void* scratch,
               size_t scratch_bytes, hipStream_t s) {
   if (n == 0) return 0;
-  if (n > 0x7fffffff - kSortTile) return MBX_ERANGE;
+  if (n > 0x7fffffff - kSortTileMax) return MBX_ERANGE;
   const int bits = (int)sizeof(T) * 8;
   if (end_bit > bits) end_bit = bits;
   const int passes = sort_passes(end_bit);
@@ -306,7 +404,8 @@ int sort_impl(const T* x, int64_t n, int end_bit, T* keys_out, T* perm_out, void
     copy_iota_kernel<T><<<(unsigned)(ceil_div(n, 256) < 2048 ? ceil_div(n, 256) : 2048), 256, 0, s>>>(x, n, keys_out, perm_out);
     return launch_status();
   }
-  const int nblocks = (int)ceil_div(n, kSortTile);
+  const int nblocks = (int)ceil_div(n, sort_tile(n));
+  const bool short_rounds = sort_items(n) == kSortItemsShort;
   const size_t counts_bytes = align256((size_t)kRadix * nblocks * sizeof(int32_t));
   const size_t buf_bytes = align256((size_t)n * sizeof(T));
   const size_t need = counts_bytes + (passes > 1 ? 2 * buf_bytes : 0);
@@ -324,12 +423,18 @@ int sort_impl(const T* x, int64_t n, int end_bit, T* keys_out, T* perm_out, void
     const bool to_final = ((passes - 1 - p) % 2) == 0;
     T* kout = to_final ? keys_out : tmp_keys;
     T* vout = to_final ? perm_out : tmp_vals;
-    radix_count_kernel<T><<<nblocks, kSortThreads, 0, s>>>(kin, n, shift, mask, pass_bits, counts, nblocks);
-    exclusive_scan_i32_kernel<<<1, 1024, 0, s>>>(counts, ((int64_t)1 << pass_bits) * nblocks);   // digit-major: digits the pass cannot produce come last
-    if (p == 0)
-      radix_scatter_kernel<T, true><<<nblocks, kSortThreads, 0, s>>>(kin, nullptr, n, shift, mask, pass_bits, counts, nblocks, kout, vout);
-    else
-      radix_scatter_kernel<T, false><<<nblocks, kSortThreads, 0, s>>>(kin, vin, n, shift, mask, pass_bits, counts, nblocks, kout, vout);
+#define MBX_SORT_PASS(ITEMS)                                                                                              \
+  do {                                                                                                                    \
+    radix_count_kernel<T, ITEMS><<<nblocks, kSortThreads, 0, s>>>(kin, n, shift, mask, pass_bits, counts, nblocks);       \
+    /* digit-major: digits the pass cannot produce come last */                                                           \
+    exclusive_scan_i32_kernel<<<1, 1024, 0, s>>>(counts, ((int64_t)1 << pass_bits) * nblocks);                            \
+    if (p == 0)                                                                                                           \
+      radix_scatter_kernel<T, true, ITEMS><<<nblocks, kSortThreads, 0, s>>>(kin, nullptr, n, shift, mask, pass_bits, counts, nblocks, kout, vout); \
+    else                                                                                                                  \
+      radix_scatter_kernel<T, false, ITEMS><<<nblocks, kSortThreads, 0, s>>>(kin, vin, n, shift, mask, pass_bits, counts, nblocks, kout, vout);    \
+  } while (0)
+    if (short_rounds) MBX_SORT_PASS(kSortItemsShort); else MBX_SORT_PASS(kSortItemsLong);
+#undef MBX_SORT_PASS
     kin = kout;
     vin = vout;
   }
@@ -458,7 +563,7 @@ size_t mbx_sort_scratch_bytes(int64_t n, int itype, int end_bit) {
   if (end_bit > bits) end_bit = bits;
   const int passes = sort_passes(end_bit);
   if (passes == 0) return 0;
-  const size_t nblocks = (size_t)ceil_div(n, kSortTile);
+  const size_t nblocks = (size_t)ceil_div(n, sort_tile(n));
   size_t need = align256((size_t)kRadix * nblocks * sizeof(int32_t));
   if (passes > 1) need += 2 * align256((size_t)n * itype_bytes(itype));
   return need;
@@ -486,21 +591,28 @@ int mbx_route(const int32_t* expert_ids, int64_t n, int num_experts, int end_bit
   if (end_bit > kRadixBits || num_experts > (1 << end_bit)) return MBX_EUNSUPPORTED;
   if (!tokens_per_expert || !bins || (pad > 0 && !padded_bins)) return MBX_EINVAL;
   if (n > 0 && (!expert_ids || !indices || !bin_ids)) return MBX_EINVAL;
-  if (n > 0x7fffffff - kSortTile) return MBX_ERANGE;
+  if (n > 0x7fffffff - kSortTileMax) return MBX_ERANGE;
   hipStream_t s = as_stream(stream);
-  const int nblocks = n > 0 ? (int)ceil_div(n, kSortTile) : 1;
-  if (scratch_bytes < (size_t)kRadix * nblocks * sizeof(int32_t) || scratch == nullptr) return MBX_ESCRATCH;
-  int32_t* counts = (int32_t*)scratch;
   const uint32_t mask = (1u << end_bit) - 1u;
   const int ndigits = 1 << end_bit;
-  // (n = 0: a table of zeros makes every count and bound zero)
-  radix_count_kernel<int32_t><<<nblocks, kSortThreads, 0, s>>>(expert_ids, n, 0, mask, end_bit, counts, nblocks);
-  route_scan_kernel<<<1, 1024, 0, s>>>(counts, ndigits, nblocks, (int32_t)n, num_experts, pad, tokens_per_expert, bins,
-                                       pad > 0 ? padded_bins : nullptr);
-  if (n > 0)
-    radix_scatter_kernel<int32_t, true><<<nblocks, kSortThreads, 0, s>>>(expert_ids, nullptr, n, 0, mask, end_bit, counts, nblocks,
-                                                                        bin_ids, indices, slot_rows, bins,
-                                                                        pad > 0 ? padded_bins : nullptr, num_experts);
+  int32_t* const pbins = pad > 0 ? padded_bins : nullptr;
+  if (n <= kRouteOneBlock) {
+    route_one_block_kernel<<<1, 1024, 0, s>>>(expert_ids, (int)n, mask, end_bit, num_experts, pad, indices, bin_ids,
+                                              tokens_per_expert, bins, pbins, slot_rows);
+    return launch_status();
+  }
+  const int nblocks = (int)ceil_div(n, sort_tile(n));
+  if (scratch_bytes < (size_t)kRadix * nblocks * sizeof(int32_t) || scratch == nullptr) return MBX_ESCRATCH;
+  int32_t* counts = (int32_t*)scratch;
+#define MBX_ROUTE_PASS(ITEMS)                                                                                             \
+  do {                                                                                                                    \
+    radix_count_kernel<int32_t, ITEMS><<<nblocks, kSortThreads, 0, s>>>(expert_ids, n, 0, mask, end_bit, counts, nblocks); \
+    route_scan_kernel<<<1, 1024, 0, s>>>(counts, ndigits, nblocks, (int32_t)n, num_experts, pad, tokens_per_expert, bins, pbins); \
+    radix_scatter_kernel<int32_t, true, ITEMS><<<nblocks, kSortThreads, 0, s>>>(expert_ids, nullptr, n, 0, mask, end_bit, counts, nblocks, \
+                                                                                bin_ids, indices, slot_rows, bins, pbins, num_experts);    \
+  } while (0)
+  if (sort_items(n) == kSortItemsShort) MBX_ROUTE_PASS(kSortItemsShort); else MBX_ROUTE_PASS(kSortItemsLong);
+#undef MBX_ROUTE_PASS
   return launch_status();
 }
 

@@ -501,6 +501,44 @@ def test_route_equals_the_separate_routing_ops(n, experts, blocking):
         assert torch.equal(kept[:n], built[:n])
 
 
+@pytest.mark.parametrize('n', [1, 63, 65, 1024, 1025, 4095, 4096, 4097, 65536, 65537])
+@pytest.mark.parametrize('experts', [3, 64, 256])
+def test_route_at_the_edges_of_its_launches(n, experts):
+    """One block up to 4096 assignments (rounds of 1024), three launches with short tiles up to 65536, long ones above;
+    the two-pass sort changes its tiles at the same size."""
+    for blocking in (0, 128):
+        test_route_equals_the_separate_routing_ops(n, experts, blocking)
+    keys = torch.randint(0, 1 << 12, (n,), generator=torch.Generator().manual_seed(n), dtype=torch.int32)
+    from megablocks_amd import ops
+    got, perm = ops.sort(keys.cuda(), 12)
+    want, want_perm = torch.sort(keys, stable=True)
+    assert torch.equal(got.cpu(), want) and torch.equal(perm.cpu(), want_perm.int())
+
+
+@pytest.mark.parametrize('tokens', [1, 5, 1023, 1024])
+@pytest.mark.parametrize('hidden', [512, 520, 1031, 2056])
+@pytest.mark.parametrize('top_k', [1, 2, 6, 9])
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float32])
+def test_combine_of_few_tokens_by_row_segments(tokens, hidden, top_k, dtype):
+    """Below 1024 tokens a row's 512-column segments go to waves of their own: products rounded to the type, then summed in
+    fp32 in the order of the experts, so the result is exact."""
+    from megablocks_amd import ops
+    g = torch.Generator().manual_seed(tokens + hidden + top_k)
+    top = torch.randint(0, 16, (tokens * top_k,), generator=g, dtype=torch.int32).cuda()
+    bin_ids, indices = ops.sort(top, 4)
+    bins = ops.inclusive_cumsum(ops.histogram(top, 16), 0)
+    x = torch.randn(tokens * top_k, hidden, generator=g).to(dtype).cuda()
+    w = torch.rand(tokens * top_k, generator=g).to(dtype).cuda()
+    got = ops.scatter(x, indices, bin_ids, w, bins, top_k)
+    rows = torch.empty_like(x)
+    rows[indices.long()] = x
+    rows = (rows * w[:, None]).view(tokens, top_k, hidden).float()
+    want = rows[:, 0].clone()
+    for j in range(1, top_k):
+        want += rows[:, j]
+    assert torch.equal(got, want.to(dtype))
+
+
 def test_route_falls_back_where_it_does_not_apply():
     from megablocks_amd.ops import routing
     ids = torch.zeros(8, dtype=torch.int32, device='cuda')
