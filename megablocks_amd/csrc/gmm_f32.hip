@@ -1,26 +1,30 @@
-// Grouped GEMM in fp32 on the fp32 matrix instruction (v_mfma_f32_16x16x4_f32: IEEE fp32 products and sums).
+// Grouped GEMM in fp32 on the bf16 matrix instruction: every value is split into three bf16 parts (24 bits, Split below), and the
+// six products of parts that reach 2^-18 of a product are summed in fp32 (v_mfma_f32_16x16x32_bf16).
 //
-// What bounds it: the matrix cores (157 TFLOP/s at 2.4 GHz; an instruction of 2048 FLOP lasts 32 cycles).  The
-// 16 x 16 x 4 form moves half the accumulator registers per FLOP of the 32 x 32 x 2 form and so draws less power: alone,
-// one wave per SIMD on random operands, 151 against 141 TFLOP/s.  Everything else is cheap next to them, provided that a
-// lane spends no vector-ALU work per element: the element-wise kernel of gmm.hip, which serves every alignment, checks
-// bounds and computes a 64-bit address for each 4-byte load and reached 71 TFLOP/s on 8 experts of 1024 +- 30 rows, hidden
-// 1024, ffn 4096 (961 us per product).  This one takes k and n that are multiples of 4 on 16-byte aligned operands and
-// moves whole 16-byte pieces global -> LDS without registers: 550 / 558 / 532 us NT / NN / TN there (125 TFLOP/s; the
-// padding of the ragged row tiles is 5 % of the work, the tail 7 %), 141 - 147 on 4096^3 and 8192^3 (the vendor library:
-// 134 - 153).
+// What bounds it: the matrix cores and the power they draw.  The fp32 instruction (v_mfma_f32_16x16x4_f32) does 256 FLOP
+// per cycle and compute unit, the bf16 one 4096, a sixth of which is 683.  Next to the 96 products of a K tile, 1536 cycles
+// of a SIMD, a wave spends 352 vector-ALU instructions, 1408 cycles, on the splitting; two waves share a SIMD, and what
+// one converts the other multiplies.  8 experts of 1024 +- 30 rows, hidden 1024, ffn 4096: 416 / 380 / 366 us NT / NN / TN
+// against 533 / 545 / 522 on the fp32 instruction and 961 in the element-wise kernel of gmm.hip, which serves every
+// alignment; 195 TFLOP/s on 4096^3 against 141.  Half the conversion instructions (v_dot2c_f32_bf16) changed nothing;
+// cutting the parts off instead of rounding them is 3 % faster and up to a third less exact.
+//
+// How exact: the parts leave 2^-27 of a value, the three products not taken 2^-26 of a product, and an accumulator is rounded six
+// times per 32 k instead of 32 times.  Relative error (2-norm) against fp64: 4.8e-7 over k = 1024, 9.8e-7 over 4096, where
+// a chain of fp32 fused multiply-adds shows 5.7e-7 and 1.15e-6.  Sums that the parts do not serve (infinities, NaN, values
+// next to the largest or the smallest) are formed again on the fp32 instruction: multiply().
 //
 // Tile: 128 x 128 (64 x 128 for short experts) per workgroup of four waves (2 x 2), K tiles of 32, two stages of
-// 32 KiB, so two workgroups share a compute unit and one multiplies while the other waits at its barrier or stores.  A
-// K tile is 128 matrix instructions per wave, 4096 cycles: the loads of a K tile are issued that long before they are
-// needed, and one barrier per K tile is enough.
+// 32 KiB, so two workgroups share a compute unit and one multiplies while the other converts, waits at its barrier or
+// stores.  Operands go global -> LDS without registers as whole 16-byte pieces (k and n multiples of 4, 16-byte aligned
+// operands); the loads of a K tile are issued a K tile before they are needed, and one barrier per K tile is enough.
 //
 // LDS layouts: an operand whose reduction dimension is contiguous (KC) is [row][32 k], 128-byte rows, 16-byte chunk c of row r
 // at position c ^ ((r >> 1) & 7) (gmm_dma.h's layout of 64 16-bit values, byte for byte); one ds_read_b128 gives a
 // lane its row's operand of four instructions.  An operand whose reduction dimension is strided (MC) is [k][128 columns],
 // the column XORed by 16 ((k >> 2) & 3), so that the four quarter waves, which read rows four apart, use different
 // banks; a lane reads two rows per ds_read2st64_b32.  Step j (of 4) of group s (of 2) of a K tile multiplies
-// k = 16 s + 4 (lane / 16) + j of both operands.
+// k = 16 s + 4 (lane / 16) + j of both operands; the bf16 instruction takes both groups' four as a lane's eight.
 #include "gmm_common.h"
 
 namespace mbx {
@@ -37,7 +41,7 @@ using dma::make_rsrc;
 using dma::RowTiles;
 using dma::tile_done;
 
-constexpr int kBN = 128, kBK = 32, kThreads = 256, kGroups = kBK / 16;
+constexpr int kBN = 128, kBK = 32, kThreads = 256;
 constexpr uint32_t kOperandBytes = 128 * kBK * 4, kStageBytes = 2 * kOperandBytes;
 constexpr size_t kLdsBytes = 2 * kStageBytes;
 constexpr size_t kPartBytes = (size_t)128 * kBN * 4;       // one tile's accumulators in the workspace
@@ -74,6 +78,35 @@ template <> struct Frag<true> {
   __device__ __forceinline__ void tie() { asm volatile("" : "+v"(v[0]), "+v"(v[1])); }
 };
 
+// Eight fp32 values as three bf16 parts each, v = part 0 + part 1 + part 2 up to 2^-27 |v|: every part is the rest the parts
+// before it leave (the differences are exact), rounded to nearest.  In kSteps steps of a few instructions, to be put between
+// products: step 3 p + q forms part q of the values 2 p and 2 p + 1.
+struct Split {
+  static constexpr int kSteps = 12;
+  u32x4 part[3];
+  float rest[2];
+  template <int X, bool MC>
+  __device__ __forceinline__ void step(const Frag<MC>& low, const Frag<MC>& high) {
+    constexpr int p = X / 3, q = X % 3, v = 2 * (p & 1);
+    if constexpr (q == 0) {
+      rest[0] = p < 2 ? low.at(v) : high.at(v);
+      rest[1] = p < 2 ? low.at(v + 1) : high.at(v + 1);
+    }
+    const uint32_t both = pack2<MBX_BF16>(rest[0], rest[1]);
+    part[q][p] = both;
+    if constexpr (q < 2) {
+      rest[0] -= __uint_as_float(both << 16);
+      rest[1] -= __uint_as_float(both & 0xffff0000u);
+    }
+  }
+};
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+
+__device__ __forceinline__ f32x4 mfma(u32x4 a, u32x4 b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+}
+
 template <int N>
 __device__ __forceinline__ void wait_lgkm() {   // at most N LDS reads of this wave still in flight
   static_assert(N < 16, "lgkmcnt is a 4-bit counter");
@@ -87,8 +120,8 @@ __device__ __forceinline__ void wait_lgkm() {   // at most N LDS reads of this w
 template <int BM> using Acc = f32x4[BM / 32][4];
 
 // acc += A_tile * B_tile over K tiles [g.kt0, g.kt1)
-template <bool A_MC, bool B_MC, int BM, bool DUAL>
-__device__ __forceinline__ void multiply(const Args& g, Acc<BM>& acc, char* lds_generic) {
+template <bool A_MC, bool B_MC, int BM, bool DUAL, bool FP32>
+__device__ __forceinline__ void multiply_as(const Args& g, Acc<BM>& acc, char* lds_generic) {
   constexpr int TM = BM / 32, TN = 4;
   static_assert(!A_MC || BM == 128, "a strided first operand: full tiles");
   const lds_ptr lds = (lds_ptr)lds_generic;
@@ -140,53 +173,93 @@ __device__ __forceinline__ void multiply(const Args& g, Acc<BM>& acc, char* lds_
 
   Frag<A_MC> fa[2][TM];
   Frag<B_MC> fb[2][TN];
-  constexpr int READS = (A_MC ? 2 : 1) * TM + (B_MC ? 2 : 1) * TN;
-  // read instruction r of the READS of group s: an operand of a KC fragment (four k) or half of one of an MC fragment (two)
-  auto read_one = [&](auto si, auto ri, int buf, uint32_t base) {
-    constexpr int s = decltype(si)::value, r = decltype(ri)::value, NA = (A_MC ? 2 : 1) * TM;
-    if constexpr (r < NA) {
-      constexpr int i = A_MC ? r / 2 : r;
-      if constexpr (A_MC) fa[buf][i].v[r % 2] = lds_read2_rows<16 * s + 2 * (r % 2)>(base + fa_off[i]);
-      else fa[buf][i].v = dma::read_frag_kc<s, i * 16 * 128>(base, fa_off[0]);
-    } else {
-      constexpr int q = r - NA, j = B_MC ? q / 2 : q;
-      if constexpr (B_MC) fb[buf][j].v[q % 2] = lds_read2_rows<16 * s + 2 * (q % 2)>(base + fb_off[j]);
-      else fb[buf][j].v = dma::read_frag_kc<s, j * 16 * 128>(base, fb_off[0]);
-    }
-  };
-  // the values of a group as registers written at this point: orders their users behind the wait in front of it
-  auto tie = [&](int buf) {
-#pragma unroll
-    for (int i = 0; i < TM; ++i) fa[buf][i].tie();
-#pragma unroll
-    for (int j = 0; j < TN; ++j) fb[buf][j].tie();
-  };
-  // The products of a group in register buffer `buf`, 16 TM of them; behind every product comes one of the reads of the
-  // next group (into the other buffer) or, with LOADS, one of the loads of a K tile, until all are issued: issued in one
-  // go they hold the wave's next product back (a wave-wide load takes the address unit some 20 cycles, and four waves
-  // issue theirs at the same time): 136 - 141 TFLOP/s on 8192^3 instead of 143 - 147.
-  constexpr int NP = 4 * TM * TN;
-  auto products = [&](auto bi, auto next_group, auto loads, uint32_t next_base) {
-    constexpr int buf = decltype(bi)::value, NL = decltype(loads)::value ? LA + LB : 0, EVERY = NP / (READS + NL) > 2 ? 2 : 1;
-    static_assert(READS + NL <= NP, "one instruction per product");
-    __builtin_amdgcn_sched_barrier(0);
-    dma::static_for<NP>([&](auto mi) {
-      constexpr int m = decltype(mi)::value, t = m / (TM * TN), i = m / TN % TM, j = m % TN;
-      acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(fb[buf][j].at(t), fa[buf][i].at(t), acc[i][j], 0, 0, 0);
-      if constexpr (m % EVERY == 0) {
-        constexpr int x = m / EVERY;
-        if constexpr (x < READS) read_one(next_group, std::integral_constant<int, x>{}, buf ^ 1, next_base);
-        else if constexpr (x - READS < NL) load_one(std::integral_constant<int, x - READS>{});
-      }
-      __builtin_amdgcn_sched_barrier(0);
+  // the read instructions of group s of one fragment: one of a KC fragment (four k), two of an MC fragment (two each)
+  auto read_a = [&](auto ii, uint32_t base) {
+    constexpr int i = decltype(ii)::value;
+    dma::static_for<2>([&](auto si) {
+      constexpr int s = decltype(si)::value;
+      if constexpr (A_MC) { fa[s][i].v[0] = lds_read2_rows<16 * s>(base + fa_off[i]); fa[s][i].v[1] = lds_read2_rows<16 * s + 2>(base + fa_off[i]); }
+      else fa[s][i].v = dma::read_frag_kc<s, i * 16 * 128>(base, fa_off[0]);
     });
   };
-  // The barrier of a K tile sits in front of the products of its last group, when every wave has that group in
-  // registers: the stage is free from then on and takes K tile kt + 2, and the first group of K tile kt + 1, which has
-  // landed, is read behind the last group's products.
+  auto read_b = [&](auto ji, uint32_t base) {
+    constexpr int j = decltype(ji)::value;
+    dma::static_for<2>([&](auto si) {
+      constexpr int s = decltype(si)::value;
+      if constexpr (B_MC) { fb[s][j].v[0] = lds_read2_rows<16 * s>(base + fb_off[j]); fb[s][j].v[1] = lds_read2_rows<16 * s + 2>(base + fb_off[j]); }
+      else fb[s][j].v = dma::read_frag_kc<s, j * 16 * 128>(base, fb_off[0]);
+    });
+  };
+  // the values of a K tile as registers written at this point: orders their users behind the wait in front of it
+  auto tie = [&] {
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+#pragma unroll
+      for (int i = 0; i < TM; ++i) fa[s][i].tie();
+#pragma unroll
+      for (int j = 0; j < TN; ++j) fb[s][j].tie();
+    }
+  };
+  // The products of a K tile on its split operands.  Fragments of A go in pairs, so that twelve products on two
+  // accumulators stand between the conversions; what is converted behind the products of (pair, j) is the next fragment
+  // of B, or the next pair of A.  The fragments of the next K tile are read behind the products of the last pair, when
+  // the conversions are done (with one pair: as soon as a fragment is converted), so that their registers serve the
+  // parts until then; one of the loads of K tile kt + 2 goes out behind every second product.
+  Split sa[2][2], sb[TN];
+  auto products = [&](uint32_t next_base) {
+    constexpr int PAIRS = TM / 2;
+    auto convert_a = [&](auto ii, auto xi) {
+      constexpr int i = decltype(ii)::value, x = decltype(xi)::value;
+      sa[i / 2 % 2][i % 2].template step<x>(fa[0][i], fa[1][i]);
+      if constexpr (PAIRS == 1 && x == Split::kSteps - 1) { __builtin_amdgcn_sched_barrier(0); read_a(ii, next_base); }
+    };
+    auto convert_b = [&](auto ji, auto xi) {
+      constexpr int j = decltype(ji)::value, x = decltype(xi)::value;
+      sb[j].template step<x>(fb[0][j], fb[1][j]);
+      if constexpr (PAIRS == 1 && x == Split::kSteps - 1) { __builtin_amdgcn_sched_barrier(0); read_b(ji, next_base); }
+    };
+    constexpr std::integral_constant<int, 0> c0{};
+    constexpr std::integral_constant<int, 1> c1{};
+    dma::static_for<Split::kSteps>([&](auto xi) { convert_a(c0, xi); convert_b(c0, xi); convert_a(c1, xi); });
+    dma::static_for<PAIRS * TN>([&](auto pj) {
+      constexpr int p = decltype(pj)::value / TN, j = decltype(pj)::value % TN;
+      dma::static_for<12>([&](auto mi) {
+        constexpr int m = decltype(mi)::value, t = m / 2, i = m % 2;
+        constexpr int pa[6] = {0, 2, 1, 0, 1, 0}, pb[6] = {2, 0, 1, 1, 0, 0};   // the small products first
+        acc[2 * p + i][j] = mfma(sb[j].part[pb[t]], sa[p % 2][i].part[pa[t]], acc[2 * p + i][j]);
+        if constexpr (p == 0 && j + 1 < TN) convert_b(std::integral_constant<int, j + 1>{}, mi);
+        if constexpr (p + 1 < PAIRS && j >= TN - 2) convert_a(std::integral_constant<int, 2 * p + 2 + j - (TN - 2)>{}, mi);
+        if constexpr (p == 1 && m % 6 == 5) {
+          if constexpr (j < 2) read_a(std::integral_constant<int, 2 * j + m / 6>{}, next_base);
+          else { read_b(std::integral_constant<int, 2 * (j - 2) + m / 6>{}, next_base); }
+        }
+        constexpr int load = (decltype(pj)::value * 12 + m) / 2;
+        if constexpr (m % 2 == 1 && load < LA + LB) load_one(std::integral_constant<uint32_t, load>{});
+        __builtin_amdgcn_sched_barrier(0);
+      });
+    });
+  };
+  // The same products on the fp32 instruction.
+  auto products_fp32 = [&](uint32_t next_base) {
+    dma::static_for<2>([&](auto si) {
+      dma::static_for<4>([&](auto ti) {
+        constexpr int s = decltype(si)::value, t = decltype(ti)::value;
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+          for (int j = 0; j < TN; ++j)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(fb[s][j].at(t), fa[s][i].at(t), acc[i][j], 0, 0, 0);
+      });
+    });
+    __builtin_amdgcn_sched_barrier(0);
+    dma::static_for<LA + LB>(load_one);
+    dma::static_for<TM>([&](auto ii) { read_a(ii, next_base); });
+    dma::static_for<TN>([&](auto ji) { read_b(ji, next_base); });
+  };
+  // A K tile's values are in registers when its iteration begins.  The barrier stands where every wave has read its
+  // stage, which takes K tile kt + 2 from then on, and where K tile kt + 1 has landed in the other, to be read during
+  // the products.
   if (g.kt0 >= g.kt1) return;
-  constexpr std::integral_constant<int, 0> c0{};
-  constexpr std::integral_constant<int, 1> c1{};
   load_at(g.kt0, 0);
   dma::static_for<LA + LB>(load_one);
   load_at(g.kt0 + 1, kStageBytes);
@@ -194,21 +267,18 @@ __device__ __forceinline__ void multiply(const Args& g, Acc<BM>& acc, char* lds_
   dma::wait_vmcnt<LA + LB>();
   __builtin_amdgcn_s_barrier();
   uint32_t stage = 0;
-  dma::static_for<READS>([&](auto ri) { read_one(c0, ri, 0, lds_base); });
+  dma::static_for<TM>([&](auto ii) { read_a(ii, lds_base); });
+  dma::static_for<TN>([&](auto ji) { read_b(ji, lds_base); });
   wait_lgkm<0>();
-  tie(0);
-  static_assert(kGroups == 2, "two groups per K tile");
+  tie();
   for (int kt = g.kt0; kt < g.kt1; ++kt) {
-    products(c0, c1, std::false_type{}, lds_base + stage);
-    load_at(kt + 2, stage);
-    wait_lgkm<0>();
-    tie(1);
     dma::wait_vmcnt<0>();
     __builtin_amdgcn_s_barrier();
-    products(c1, c0, std::true_type{}, lds_base + (stage ^ kStageBytes));   // past the last K tile: reads of stale LDS into dead registers
+    load_at(kt + 2, stage);
     stage ^= kStageBytes;
+    if constexpr (FP32) products_fp32(lds_base + stage); else products(lds_base + stage);   // past the last K tile: reads of stale LDS into dead registers
     wait_lgkm<0>();
-    tie(0);
+    tie();
   }
   dma::wait_vmcnt<0>();
 }
@@ -219,6 +289,34 @@ __device__ __forceinline__ void clear(Acc<BM>& acc) {
   for (int i = 0; i < BM / 32; ++i)
 #pragma unroll
     for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+}
+
+// acc = A_tile * B_tile over K tiles [g.kt0, g.kt1), on the split operands; where a sum comes out infinite, NaN or of a
+// magnitude below kTiny, a second time on the fp32 instruction, which takes such operands as they are.  The splitting of an
+// infinity, or of a value that rounds to one, leaves NaN parts, so no such sum stays unnoticed; parts of a value below
+// 2^-102 can fall below the normal range, and a sum that holds nothing larger is small itself.
+constexpr float kTiny = 0x1p-64f;
+
+template <bool A_MC, bool B_MC, int BM, bool DUAL>
+__device__ __forceinline__ void multiply(const Args& g, Acc<BM>& acc, char* lds) {
+  clear<BM>(acc);
+  multiply_as<A_MC, B_MC, BM, DUAL, false>(g, acc, lds);
+  uint32_t largest = 0, smallest = 0xffffffffu;   // of the magnitudes as integers; less one, which leaves zeros out
+#pragma unroll
+  for (int i = 0; i < BM / 32; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const uint32_t u = __float_as_uint(acc[i][j][r]) & 0x7fffffffu;
+        largest = largest > u ? largest : u;
+        smallest = smallest < u - 1u ? smallest : u - 1u;
+      }
+  const bool again = largest >= 0x7f800000u || smallest < __float_as_uint(kTiny) - 1u;
+  if (__syncthreads_or(again)) {
+    clear<BM>(acc);
+    multiply_as<A_MC, B_MC, BM, DUAL, true>(g, acc, lds);
+  }
 }
 
 // c[m][n] = acc for the tile's rows below m_lim and columns below n (n a multiple of 4, c 16-byte aligned)
@@ -337,7 +435,6 @@ gmm_f32_rows_kernel(const float* __restrict__ a, const float* __restrict__ b, fl
     g.kt0 = cut ? (int)((int64_t)part * nk / ksplit) : 0;
     g.kt1 = cut ? (int)((int64_t)(part + 1) * nk / ksplit) : nk;
     Acc<BM> acc;
-    clear<BM>(acc);
     multiply<false, B_MC, BM, DUAL>(g, acc, lds);
     if (!cut || join_parts<BM>(acc, id - full_rounds * P, rest, part, ksplit, ws_counters, ws_parts, lds))
       store<BM>(acc, c + (int64_t)row0 * n, n, end - row0, g.b_r0, n);
@@ -393,7 +490,6 @@ gmm_f32_tn_kernel(const float* __restrict__ a, const float* __restrict__ b, floa
   g.kt0 = (int)((int64_t)part * nk / ksplit);
   g.kt1 = (int)((int64_t)(part + 1) * nk / ksplit);
   Acc<128> acc;
-  clear<128>(acc);
   multiply<true, true, 128, false>(g, acc, lds);
   if (ksplit > 1 && !join_parts<128>(acc, tile, total, part, ksplit, ws_counters, ws_parts, lds)) return;
   store<128>(acc, c + ((int64_t)e * k + g.a_r0) * n, n, k - g.a_r0, g.b_r0, n);
@@ -411,7 +507,8 @@ static inline bool f32_ok(const void* a, const void* b, const void* c, int64_t r
 }
 
 // Tiles of 64 rows up to 192 rows per expert on average: of full ones an expert of that many leaves a quarter and more of
-// the multiplications to padding, which this kernel, bound by the matrix cores, pays in full.
+// the multiplications to padding, which this kernel, bound by the matrix cores, pays in full (64 experts of 100 - 156 rows,
+// 1024 x 1408: 228 us NT).
 constexpr int64_t kF32ShortRows = 192;
 
 }  // namespace

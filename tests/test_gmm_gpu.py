@@ -944,6 +944,32 @@ def test_gmm_fp32_on_the_matrix_cores(gg, monkeypatch, groups, rows, k, n, mode)
         assert torch.equal(got[-1].nan_to_num(), got[-2].nan_to_num())
 
 
+@pytest.mark.parametrize('k', [36, 64, 2052])
+@pytest.mark.parametrize('mode', ['nn', 'nt', 'tn'])
+def test_gmm_fp32_at_the_ends_of_the_range(gg, k, mode):
+    """Output rows from operands next to the largest and the smallest fp32 values, which are not the sum of three bf16 values
+    there, against fp64.  Every row is held to the error of a sum of k terms, 2^-24 sqrt(k) of its largest entry with a
+    factor of four to spare, plus what underflow leaves of a product."""
+    torch.manual_seed(k)
+    rows, n = 300, 132
+    a = torch.randn(rows, k, device='cuda')
+    b = torch.randn(k, n, device='cuda').clamp_(-3, 3)
+    a *= torch.exp2(-torch.arange(rows, device='cuda').float() / 2.25).unsqueeze(1)   # down to 2^-133: subnormals
+    a[7], a[8], a[9] = 0.0, 0.0, 0.0
+    largest = torch.finfo(torch.float32).max
+    a[7, 3], a[8, k - 1], a[200, k // 2] = largest, -largest, largest
+    b[3], b[k - 1], b[k // 2] = b[3] / 4, b[k - 1] / 4, b[k // 2] / 4
+    want = a.double() @ b.double()
+    sizes = torch.tensor([rows])
+    if mode == 'tn':
+        got = gg.backend.gmm(a.t().contiguous(), b, torch.tensor([k]), trans_a=True)[0]
+    else:
+        got = gg.backend.gmm(a, (b.t() if mode == 'nt' else b).contiguous()[None], sizes, trans_b=mode == 'nt')
+    tol = 4 * 2.0 ** -24 * math.sqrt(k) * want.abs().amax(1) + k * 2.0 ** -149
+    assert bool(((got.double() - want).abs().amax(1) <= tol).all())
+    assert not bool(got[9].any())
+
+
 @pytest.mark.parametrize('groups,rows,k,n', [(3, 700, 8, 136), (4, 900, 72, 264), (5, 1500, 200, 512), (8, 3000, 1032, 2728),
                                              (2, 40, 312, 1032), (12, 3600, 2728, 1032), (1, 260, 4104, 64)])
 @pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])
