@@ -3,7 +3,7 @@
 //
 // What bounds it: the matrix cores and the power they draw.  The fp32 instruction (v_mfma_f32_16x16x4_f32) does 256 FLOP
 // per cycle and compute unit, the bf16 one 4096, a sixth of which is 683.  Next to the 96 products of a K tile, 1536 cycles
-// of a SIMD, a wave spends 352 vector-ALU instructions, 1408 cycles, on the splitting; two waves share a SIMD, and what
+// of a SIMD, a wave spends 384 vector-ALU instructions, 1536 cycles, on the splitting; two waves share a SIMD, and what
 // one converts the other multiplies.  8 experts of 1024 +- 30 rows, hidden 1024, ffn 4096: 416 / 380 / 366 us NT / NN / TN
 // against 533 / 545 / 522 on the fp32 instruction and 961 in the element-wise kernel of gmm.hip, which serves every
 // alignment; 195 TFLOP/s on 4096^3 against 141.  Half the conversion instructions (v_dot2c_f32_bf16) changed nothing;
@@ -86,11 +86,12 @@ struct Split {
   u32x4 part[3];
   float rest[2];
   template <int X, bool MC>
-  __device__ __forceinline__ void step(const Frag<MC>& low, const Frag<MC>& high) {
+  __device__ __forceinline__ void step(const Frag<MC>& low, const Frag<MC>& high, float& largest) {   // largest: magnitude seen
     constexpr int p = X / 3, q = X % 3, v = 2 * (p & 1);
     if constexpr (q == 0) {
       rest[0] = p < 2 ? low.at(v) : high.at(v);
       rest[1] = p < 2 ? low.at(v + 1) : high.at(v + 1);
+      asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(largest) : "v"(rest[0]), "v"(rest[1]));
     }
     const uint32_t both = pack2<MBX_BF16>(rest[0], rest[1]);
     part[q][p] = both;
@@ -119,9 +120,9 @@ __device__ __forceinline__ void wait_lgkm() {   // at most N LDS reads of this w
 // of the workgroup's tile (the operands are swapped, so a lane owns runs of four consecutive columns).
 template <int BM> using Acc = f32x4[BM / 32][4];
 
-// acc += A_tile * B_tile over K tiles [g.kt0, g.kt1)
+// acc += A_tile * B_tile over K tiles [g.kt0, g.kt1); largest: the largest magnitude among the operands (unless FP32)
 template <bool A_MC, bool B_MC, int BM, bool DUAL, bool FP32>
-__device__ __forceinline__ void multiply_as(const Args& g, Acc<BM>& acc, char* lds_generic) {
+__device__ __forceinline__ void multiply_as(const Args& g, Acc<BM>& acc, char* lds_generic, float& largest) {
   constexpr int TM = BM / 32, TN = 4;
   static_assert(!A_MC || BM == 128, "a strided first operand: full tiles");
   const lds_ptr lds = (lds_ptr)lds_generic;
@@ -210,12 +211,12 @@ __device__ __forceinline__ void multiply_as(const Args& g, Acc<BM>& acc, char* l
     constexpr int PAIRS = TM / 2;
     auto convert_a = [&](auto ii, auto xi) {
       constexpr int i = decltype(ii)::value, x = decltype(xi)::value;
-      sa[i / 2 % 2][i % 2].template step<x>(fa[0][i], fa[1][i]);
+      sa[i / 2 % 2][i % 2].template step<x>(fa[0][i], fa[1][i], largest);
       if constexpr (PAIRS == 1 && x == Split::kSteps - 1) { __builtin_amdgcn_sched_barrier(0); read_a(ii, next_base); }
     };
     auto convert_b = [&](auto ji, auto xi) {
       constexpr int j = decltype(ji)::value, x = decltype(xi)::value;
-      sb[j].template step<x>(fb[0][j], fb[1][j]);
+      sb[j].template step<x>(fb[0][j], fb[1][j], largest);
       if constexpr (PAIRS == 1 && x == Split::kSteps - 1) { __builtin_amdgcn_sched_barrier(0); read_b(ji, next_base); }
     };
     constexpr std::integral_constant<int, 0> c0{};
@@ -292,15 +293,17 @@ __device__ __forceinline__ void clear(Acc<BM>& acc) {
 }
 
 // acc = A_tile * B_tile over K tiles [g.kt0, g.kt1), on the split operands; where a sum comes out infinite, NaN or of a
-// magnitude below kTiny, a second time on the fp32 instruction, which takes such operands as they are.  The splitting of an
-// infinity, or of a value that rounds to one, leaves NaN parts, so no such sum stays unnoticed; parts of a value below
-// 2^-102 can fall below the normal range, and a sum that holds nothing larger is small itself.
-constexpr float kTiny = 0x1p-64f;
+// magnitude below kTiny, or an operand is kHuge or more, a second time on the fp32 instruction, which takes such operands as
+// they are.  The splitting of an infinity, or of a value that rounds to one, leaves NaN parts, so no such sum stays
+// unnoticed.  Parts of a value below 2^-102 can fall below the normal range: next to operands below kHuge its products are
+// below kTiny, and what they lose (2^-134 of the value, 2^-96 of a product) is 2^-32 of any sum that stays.
+constexpr float kTiny = 0x1p-64f, kHuge = 0x1p38f;
 
 template <bool A_MC, bool B_MC, int BM, bool DUAL>
 __device__ __forceinline__ void multiply(const Args& g, Acc<BM>& acc, char* lds) {
   clear<BM>(acc);
-  multiply_as<A_MC, B_MC, BM, DUAL, false>(g, acc, lds);
+  float operand = 0.f;
+  multiply_as<A_MC, B_MC, BM, DUAL, false>(g, acc, lds, operand);
   uint32_t largest = 0, smallest = 0xffffffffu;   // of the magnitudes as integers; less one, which leaves zeros out
 #pragma unroll
   for (int i = 0; i < BM / 32; ++i)
@@ -312,10 +315,10 @@ __device__ __forceinline__ void multiply(const Args& g, Acc<BM>& acc, char* lds)
         largest = largest > u ? largest : u;
         smallest = smallest < u - 1u ? smallest : u - 1u;
       }
-  const bool again = largest >= 0x7f800000u || smallest < __float_as_uint(kTiny) - 1u;
+  const bool again = operand >= kHuge || largest >= 0x7f800000u || smallest < __float_as_uint(kTiny) - 1u;
   if (__syncthreads_or(again)) {
     clear<BM>(acc);
-    multiply_as<A_MC, B_MC, BM, DUAL, true>(g, acc, lds);
+    multiply_as<A_MC, B_MC, BM, DUAL, true>(g, acc, lds, operand);
   }
 }
 

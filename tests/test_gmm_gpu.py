@@ -970,6 +970,23 @@ def test_gmm_fp32_at_the_ends_of_the_range(gg, k, mode):
     assert not bool(got[9].any())
 
 
+@pytest.mark.parametrize('power', [37, 110, 126])
+@pytest.mark.parametrize('mode', ['nn', 'nt', 'tn'])
+def test_gmm_fp32_of_small_by_large_values(gg, mode, power):
+    """Values around 2^-power times values around 2^power, sums around 1, against fp64: the small ones have parts below the
+    normal range of bf16 from about 2^-102 on.  The error bound of a sum of k terms, with a factor of four to spare."""
+    torch.manual_seed(power)
+    rows, k, n = 200, 96, 132
+    a = torch.randn(rows, k, device='cuda').clamp_(-3, 3) * 2.0 ** -power
+    b = torch.randn(k, n, device='cuda').clamp_(-1.9, 1.9) * 2.0 ** power
+    want = a.double() @ b.double()
+    if mode == 'tn':
+        got = gg.backend.gmm(a.t().contiguous(), b, torch.tensor([k]), trans_a=True)[0]
+    else:
+        got = gg.backend.gmm(a, (b.t() if mode == 'nt' else b).contiguous()[None], torch.tensor([rows]), trans_b=mode == 'nt')
+    assert max_block_err(got, want) < 4 * 2.0 ** -24 * math.sqrt(k)
+
+
 @pytest.mark.parametrize('groups,rows,k,n', [(3, 700, 8, 136), (4, 900, 72, 264), (5, 1500, 200, 512), (8, 3000, 1032, 2728),
                                              (2, 40, 312, 1032), (12, 3600, 2728, 1032), (1, 260, 4104, 64)])
 @pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])
