@@ -246,6 +246,10 @@ int mbx_gmm_ws(const void* a, const void* b, const void* a2, const void* b2, voi
  * n not a multiple of 8, operands or outputs not 16-byte aligned, one expert's weights of 2 GiB or more. */
 int mbx_gmm_act(const void* a, const void* b, void* c, void* c_act, int dtype, const int32_t* bins,
                 int num_groups, int64_t rows, int k, int n, int act, mbx_stream_t stream);
+/* The same with b as [E, k, n], c[r_e] = a[r_e] @ b[e]: the batched MLP of the capacity-factor layer,
+ * megablocks/layers/mlp.py:162-167 (`activation_fn(torch.bmm(x, w1))`). */
+int mbx_gmm_act_nn(const void* a, const void* b, void* c, void* c_act, int dtype, const int32_t* bins,
+                   int num_groups, int64_t rows, int k, int n, int act, mbx_stream_t stream);
 
 /* The activation gradient of the expert MLP's backward, megablocks/layers/mlp.py:478-483 with
  * megablocks/layers/gelu.py:9-13 (`dact = gmm(ddsd_out, w2, trans_b=True); dsdd_out = gelu_backward_(dact, sdd_out)`),

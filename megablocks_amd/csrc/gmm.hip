@@ -698,15 +698,15 @@ static int gmm_dual_ws(const void* a, const void* b, const void* a2, const void*
   return gmm_dma(call);
 }
 
-// The NT product with an activation epilogue (epi: dma::kEpiAct / dma::kEpiDact), for the shapes the direct-to-LDS
+// The product with an activation epilogue (epi: dma::kEpiAct / dma::kEpiDact), for the shapes the direct-to-LDS
 // kernels take; anything else is MBX_EUNSUPPORTED and the caller runs the product and the element-wise pass.
 // (kEpiDglu*: pre2 = x2, out2 = the second output.)
 // (kEpiGlu*: b2 = the second matrix, extra = the gated activation, out2 = the second product.)
 // gather.slots non-null: `a` is read through the row map (no epilogue, kEpiAct and kEpiGlu* only; `extra` may then be
-// null for no epilogue).
-static int gmm_nt_epilogue(const void* a, const void* b, void* c, void* extra, int dtype, const int32_t* bins, int num_groups,
+// null for no epilogue).  layout: MBX_NT, or MBX_NN with kEpiAct.
+static int gmm_epilogue(const void* a, const void* b, void* c, void* extra, int dtype, const int32_t* bins, int num_groups,
                            int64_t rows, int k, int n, int act, int epi, mbx_stream_t stream, const void* pre2 = nullptr,
-                           void* out2 = nullptr, const void* b2 = nullptr, GatherRows gather = GatherRows()) {
+                           void* out2 = nullptr, const void* b2 = nullptr, GatherRows gather = GatherRows(), int layout = MBX_NT) {
   if (num_groups < 0 || rows < 0 || k < 0 || n < 0) return MBX_EINVAL;
   if (dtype != MBX_BF16 && dtype != MBX_F16 && dtype != MBX_F32) return MBX_EINVAL;
   const bool dglu = dma::epi_is_dglu(epi), glu = dma::epi_is_glu(epi);
@@ -720,7 +720,7 @@ static int gmm_nt_epilogue(const void* a, const void* b, void* c, void* extra, i
   // the second matrix is addressed from half a tile before its first row: that much more must fit below 2 GiB
   if (glu) ok = ok && aligned16(b2) && aligned16(out2) && dma_sizes_ok(k, n + dma::TileMain::BN / 2);
   if (!ok) return MBX_EUNSUPPORTED;
-  DmaCall call{a, b, c, dtype, bins, num_groups, rows, k, n, MBX_NT, as_stream(stream)};
+  DmaCall call{a, b, c, dtype, bins, num_groups, rows, k, n, layout, as_stream(stream)};
   call.a2 = pre2;
   call.b2 = b2;
   call.epi = epi;
@@ -732,18 +732,24 @@ static int gmm_nt_epilogue(const void* a, const void* b, void* c, void* extra, i
 
 int mbx_gmm_act(const void* a, const void* b, void* c, void* c_act, int dtype, const int32_t* bins, int num_groups,
                 int64_t rows, int k, int n, int act, mbx_stream_t stream) {
-  return gmm_nt_epilogue(a, b, c, c_act, dtype, bins, num_groups, rows, k, n, act, dma::kEpiAct, stream);
+  return gmm_epilogue(a, b, c, c_act, dtype, bins, num_groups, rows, k, n, act, dma::kEpiAct, stream);
+}
+
+int mbx_gmm_act_nn(const void* a, const void* b, void* c, void* c_act, int dtype, const int32_t* bins, int num_groups,
+                   int64_t rows, int k, int n, int act, mbx_stream_t stream) {
+  return gmm_epilogue(a, b, c, c_act, dtype, bins, num_groups, rows, k, n, act, dma::kEpiAct, stream, nullptr, nullptr, nullptr,
+                      GatherRows(), MBX_NN);
 }
 
 int mbx_gmm_dact(const void* a, const void* b, const void* pre, void* c, int dtype, const int32_t* bins, int num_groups,
                  int64_t rows, int k, int n, int act, mbx_stream_t stream) {
-  return gmm_nt_epilogue(a, b, c, (void*)pre, dtype, bins, num_groups, rows, k, n, act, dma::kEpiDact, stream);
+  return gmm_epilogue(a, b, c, (void*)pre, dtype, bins, num_groups, rows, k, n, act, dma::kEpiDact, stream);
 }
 
 int mbx_gmm_glu(const void* a, const void* b1, const void* b2, void* x1, void* x2, void* h, int dtype, const int32_t* bins,
                 int num_groups, int64_t rows, int k, int n, int act, mbx_stream_t stream) {
   if (act != MBX_ACT_SILU && act != MBX_ACT_GELU_TANH) return MBX_EINVAL;
-  return gmm_nt_epilogue(a, b1, x1, h, dtype, bins, num_groups, rows, k, n, act,
+  return gmm_epilogue(a, b1, x1, h, dtype, bins, num_groups, rows, k, n, act,
                          act == MBX_ACT_SILU ? dma::kEpiGluSilu : dma::kEpiGluGelu, stream, nullptr, x2, b2);
 }
 
@@ -764,7 +770,7 @@ int mbx_gmm_gather(const void* x, int64_t x_rows, const int32_t* indices, int to
   gather.top_k = top_k;
   gather.src_rows = (int)x_rows;
   const int epi = b2 ? (act == MBX_ACT_SILU ? dma::kEpiGluSilu : dma::kEpiGluGelu) : h ? dma::kEpiAct : dma::kEpiNone;
-  return gmm_nt_epilogue(x, b1, c, h, dtype, bins, num_groups, rows, k, n, act, epi, stream, nullptr, c2, b2, gather);
+  return gmm_epilogue(x, b1, c, h, dtype, bins, num_groups, rows, k, n, act, epi, stream, nullptr, c2, b2, gather);
 }
 
 int mbx_gmm_scatter(const void* a, const void* b, void* c, void* out, int dtype, const int32_t* bins, int num_groups,
@@ -830,7 +836,7 @@ int mbx_gmm_tn_gather(const void* a, const void* x, int64_t x_rows, const int32_
 int mbx_gmm_dglu(const void* a, const void* b, const void* x1, const void* x2, void* d1, void* d2, int dtype,
                  const int32_t* bins, int num_groups, int64_t rows, int k, int n, int act, mbx_stream_t stream) {
   if (act != MBX_ACT_SILU && act != MBX_ACT_GELU_TANH) return MBX_EINVAL;
-  return gmm_nt_epilogue(a, b, d1, (void*)x1, dtype, bins, num_groups, rows, k, n, act,
+  return gmm_epilogue(a, b, d1, (void*)x1, dtype, bins, num_groups, rows, k, n, act,
                          act == MBX_ACT_SILU ? dma::kEpiDgluSilu : dma::kEpiDgluGelu, stream, x2, d2);
 }
 

@@ -207,35 +207,43 @@ def _use_epilogue(fuse, a, rows, n):
     return bool(fuse)
 
 
-def _nt_operands(a, b, batch_sizes, what):
+def activation_epilogues(*operands):
+    """Whether products of these operands can have an activation in their epilogue: 16-bit tensors of one type on the GPU."""
+    return ACTIVATION_EPILOGUES and all(t.is_cuda and t.dtype == operands[0].dtype for t in operands) and \
+        operands[0].dtype in (torch.bfloat16, torch.float16)
+
+
+def _nt_operands(a, b, batch_sizes, what, trans_b=True):
     _lib.require_cuda(a, b)
     if a.ndim != 2 or b.ndim != 3 or a.dtype != b.dtype:
-        raise ValueError(f'{what}: a must be [rows, k] and b [num_groups, n, k] of the same dtype')
+        raise ValueError(f'{what}: a must be [rows, k] and b [num_groups, {"n, k" if trans_b else "k, n"}] of the same dtype')
     a, b = a.contiguous(), b.contiguous()
     bins = _device_bins(batch_sizes, a.device, a.shape[0])
-    if b.shape[0] != bins.shape[0] or b.shape[2] != a.shape[1]:
+    if b.shape[0] != bins.shape[0] or b.shape[2 if trans_b else 1] != a.shape[1]:
         raise ValueError(f'{what}: b does not match a and batch_sizes')
     return a, b, bins
 
 
-def gmm_act(a, b, batch_sizes, fuse=None):
-    """(c, gelu_tanh(c)) with c[r_e] = a[r_e] @ b[e].T: the first product of the expert MLP and its activation
-    (mlp.py:521-522), the activation applied in the product's epilogue where the library has a kernel for the shape
-    (16-bit types, k and n multiples of 8) and the output is large enough for that to pay (`fuse` None; True /
-    False force the choice), else as a separate element-wise pass."""
-    a, b, bins = _nt_operands(a, b, batch_sizes, 'gmm_act')
-    rows, k, n, groups = a.shape[0], a.shape[1], b.shape[1], bins.shape[0]
+def gmm_act(a, b, batch_sizes, fuse=None, trans_b=True):
+    """(c, gelu_tanh(c)) with c[r_e] = a[r_e] @ b[e].T (`trans_b` False: @ b[e]): the first product of the expert MLP and
+    its activation (mlp.py:521-522; mlp.py:165-166), the activation applied in the product's epilogue where the library
+    has a kernel for the shape (16-bit types, k and n multiples of 8) and the output is large enough for that to pay
+    (`fuse` None; True / False force the choice), else as a separate element-wise pass."""
+    a, b, bins = _nt_operands(a, b, batch_sizes, 'gmm_act', trans_b)
+    rows, k, n, groups = a.shape[0], a.shape[1], b.shape[1 if trans_b else 2], bins.shape[0]
     c = torch.empty((rows, n), dtype=a.dtype, device=a.device)
     c_act = torch.empty_like(c)
     rc = _lib.EUNSUPPORTED
     if _use_epilogue(fuse, a, rows, n):
-        with _lib.device_of(a), _lib.record('gmm_nt_act', rows=rows, k=k, n=n, elem=a.element_size(), groups=groups) as rec:
-            rc = lib.mbx_gmm_act(_lib.ptr(a), _lib.ptr(b), _lib.ptr(c), _lib.ptr(c_act), _lib.dtype_of(a), _lib.ptr(bins),
-                                 groups, rows, k, n, ACT_GELU_TANH, _lib.stream())
+        launch = lib.mbx_gmm_act if trans_b else lib.mbx_gmm_act_nn
+        with _lib.device_of(a), _lib.record('gmm_nt_act' if trans_b else 'gmm_nn_act', rows=rows, k=k, n=n,
+                                            elem=a.element_size(), groups=groups) as rec:
+            rc = launch(_lib.ptr(a), _lib.ptr(b), _lib.ptr(c), _lib.ptr(c_act), _lib.dtype_of(a), _lib.ptr(bins),
+                        groups, rows, k, n, ACT_GELU_TANH, _lib.stream())
             if rc == _lib.EUNSUPPORTED:
                 rec.cancel()
     if rc == _lib.EUNSUPPORTED:
-        gmm(a, b, batch_sizes, trans_b=True, c=c)
+        gmm(a, b, batch_sizes, trans_b=trans_b, c=c)
         return c, torch.nn.functional.gelu(c, approximate='tanh')
     _lib.check(rc, 'gmm_act')
     return c, c_act

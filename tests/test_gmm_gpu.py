@@ -1104,3 +1104,38 @@ def test_gmm_with_a_handful_of_rows_per_expert(gg, counts, k, n, dtype):
         (g,) = gg.gmm_gather(src, w1, sizes)
         mask = keep[order.long()] & nt_keep[0]
         assert torch.equal(g[mask], gg.backend.gmm(src.materialize(), w1, sizes, trans_b=True)[mask])
+
+
+@pytest.mark.parametrize('groups,rows,k,n', [(1, 1, 8, 8), (3, 130, 64, 256), (5, 1280, 72, 264), (8, 8 * 257, 128, 1032), (32, 4096, 192, 768)])
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])
+def test_batched_mlp_with_activation_epilogues(gg, groups, rows, k, n, dtype):
+    """The capacity-factor layer's products with the activation in their epilogues against the plain product and an
+    element-wise pass: the product bit for bit unless the plain launch cuts its last tiles along the reduction, the
+    activation of the stored product within the rounding of two tanh evaluations; and every gradient against the node
+    autograd builds from the parts."""
+    from megablocks_amd.layers.mlp import BatchedGeluMLP
+    torch.manual_seed(rows)
+    sizes = _sizes(groups, rows, seed=rows, empty=(1,) if groups > 2 else ()).cuda()
+    x = torch.randn(rows, k, device='cuda').to(dtype)
+    w1 = (torch.randn(groups, k, n, device='cuda') / k ** 0.5).to(dtype)
+    w2 = (torch.randn(groups, n, k, device='cuda') / n ** 0.5).to(dtype)
+    pre, act = gg.gmm_act(x, w1, sizes, fuse=True, trans_b=False)
+    assert max_block_err(pre, _ref_gpu(x, w1, sizes.cpu(), False, False)) < TOL
+    assert rel_err(act, torch.nn.functional.gelu(pre.float(), approximate='tanh')) < TOL
+    grad = torch.randn(rows, k, device='cuda').to(dtype)
+    results = []
+    for fused in (True, False):
+        ts = [t.clone().requires_grad_(True) for t in (x, w1, w2)]
+        if fused:
+            y = BatchedGeluMLP.apply(*ts, sizes)
+        else:
+            h = torch.nn.functional.gelu(gg.ops.gmm(ts[0], ts[1], sizes), approximate='tanh')
+            y = gg.ops.gmm(h, ts[2], sizes)
+        y.backward(grad)
+        results.append([y] + [t.grad for t in ts])
+    for got, want in zip(*results):
+        assert rel_err(got, want) < TOL
+    # inputs without a gradient: nothing is computed for them
+    w = w2.clone().requires_grad_(True)
+    BatchedGeluMLP.apply(x, w1, w, sizes).backward(grad)
+    assert torch.equal(w.grad, results[0][3])
