@@ -364,7 +364,14 @@ int mbx_router_forward(const void* logits, int dtype, int64_t tokens, int num_ex
                        void* scores, void* weights, int64_t* indices, int32_t* indices32, float* lse,
                        mbx_stream_t stream);
 
-/* Backward of the above as autograd derives it for router.py:98-106: grad_logits from grad_weights
+/* The linear layer in front of it as well, megablocks/layers/router.py:96-106, for 16-bit types in one launch:
+ * logits = round(x @ weight^T) with x [tokens, hidden], weight [num_experts, hidden], then the above (the logits are not
+ * written).  Meant for a few tokens.  MBX_EUNSUPPORTED: fp32, hidden not a multiple of 8, x or weight not 16-byte
+ * aligned, more than 128 experts, top_k above 64. */
+int mbx_router_linear_forward(const void* x, const void* weight, int dtype, int64_t tokens, int hidden, int num_experts, int top_k,
+                              float norm_p, void* scores, void* weights, int64_t* indices, int32_t* indices32, mbx_stream_t stream);
+
+/* Backward of mbx_router_forward as autograd derives it for router.py:98-106: grad_logits from grad_weights
  * [tokens, top_k] (NULL: none) and, optionally, a gradient that reaches `scores` directly (NULL: none;
  * e.g. from the load-balancing loss, moe.py:32-89), given the forward's scores and indices.  grad_lse (NULL: none): a
  * gradient that reaches the forward's `lse` ([tokens], fp32; from the z-loss, router.py:25-42); it adds

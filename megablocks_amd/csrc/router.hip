@@ -24,81 +24,167 @@ __device__ __forceinline__ float wave_pnorm(float w, bool live, float p) {
   return p == 1.f ? sum : (p == 2.f ? sqrtf(sum) : powf(sum, 1.f / p));
 }
 
-// scores = softmax(logits) rounded to the storage type (computed in fp32: exp(x - max) / sum, as
+// One token's scores, choices and weights, by one wave: lane l has the logits of experts l, l + 64, ... in x (-inf past the
+// last).  scores = softmax(logits) rounded to the storage type (computed in fp32: exp(x - max) / sum, as
 // torch's softmax does for 16-bit inputs); the k largest rounded scores in descending order, ties to the
 // lower expert index (NaN scores first); weights = those scores, divided by their rounded p-norm if p > 0
 // (each of torch's two operations rounds to the storage type).
 template <int DT, int R>
+__device__ __forceinline__ void route_token(float (&x)[R], int64_t t, int num_experts, int top_k, float p,
+                                            typename Elem<DT>::type* __restrict__ scores, typename Elem<DT>::type* __restrict__ weights,
+                                            int64_t* __restrict__ indices, int32_t* __restrict__ indices32, float* __restrict__ lse) {
+  typedef typename Elem<DT>::type E;
+  const int lane = lane_id();
+  float m = -INFINITY;
+#pragma unroll
+  for (int r = 0; r < R; ++r) m = fmaxf(m, x[r]);
+  m = wave_max(m);
+  float sum = 0.f;
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    x[r] = lane + r * kWave < num_experts ? expf(x[r] - m) : 0.f;
+    sum += x[r];
+  }
+  sum = wave_sum(sum);
+  // logsumexp of the row, the term of the router z-loss (router.py:37): an infinite maximum is the result itself
+  if (lse && lane == 0) lse[t] = (m == INFINITY || m == -INFINITY) ? m : m + logf(sum);
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int e = lane + r * kWave;
+    const E s = Elem<DT>::from_f32(x[r] / sum);
+    if (e < num_experts) scores[t * num_experts + e] = s;
+    // The selection key: the rounded score; -1 marks "not a candidate" (scores are >= 0).  A NaN score (a NaN
+    // or +inf logit makes the whole row NaN) ranks above every number, as torch.topk ranks it, so that the
+    // indices written are always experts: +inf, which no score can be, stands for it.
+    const float v = Elem<DT>::to_f32(s);
+    x[r] = e < num_experts ? (v != v ? INFINITY : v) : -1.f;
+  }
+  float my_w = 0.f;
+  int my_i = 0;
+  for (int j = 0; j < top_k; ++j) {
+    float best = -1.f;
+    int best_e = 0x7fffffff;
+#pragma unroll
+    for (int r = 0; r < R; ++r)   // ascending expert index: a later equal value does not replace an earlier one
+      if (x[r] > best) { best = x[r]; best_e = lane + r * kWave; }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+      const float ov = __shfl_xor(best, off, 64);
+      const int oe = __shfl_xor(best_e, off, 64);
+      if (ov > best || (ov == best && oe < best_e)) { best = ov; best_e = oe; }
+    }
+    if (lane == j) { my_w = best == INFINITY ? NAN : best; my_i = best_e; }
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+      if (lane + r * kWave == best_e) x[r] = -1.f;
+  }
+  const bool live = lane < top_k;
+  if (p > 0.f) {
+    const float norm = Elem<DT>::to_f32(Elem<DT>::from_f32(wave_pnorm(my_w, live, p)));
+    my_w = my_w / norm;
+  }
+  if (live) {
+    weights[t * top_k + lane] = Elem<DT>::from_f32(my_w);
+    indices[t * top_k + lane] = my_i;
+    if (indices32) indices32[t * top_k + lane] = my_i;   // what the routing kernels take, without a cast pass
+  }
+}
+
+template <int DT, int R>
 __global__ void __launch_bounds__(kTokenThreads)
 router_forward_kernel(const void* __restrict__ logits_, int64_t tokens, int num_experts, int top_k, float p,
-                      void* __restrict__ scores_, void* __restrict__ weights_, int64_t* __restrict__ indices,
+                      void* __restrict__ scores, void* __restrict__ weights, int64_t* __restrict__ indices,
                       int32_t* __restrict__ indices32, float* __restrict__ lse) {
   typedef typename Elem<DT>::type E;
   const E* logits = (const E*)logits_;
-  E* scores = (E*)scores_;
-  E* weights = (E*)weights_;
   const int lane = lane_id(), wave = threadIdx.x / kWave;
   for (int64_t t = (int64_t)blockIdx.x * kTokenWaves + wave; t < tokens; t += (int64_t)gridDim.x * kTokenWaves) {
-    const E* row = logits + t * num_experts;
     float x[R];
-    float m = -INFINITY;
 #pragma unroll
     for (int r = 0; r < R; ++r) {
       const int e = lane + r * kWave;
-      x[r] = e < num_experts ? Elem<DT>::to_f32(row[e]) : -INFINITY;
-      m = fmaxf(m, x[r]);
+      x[r] = e < num_experts ? Elem<DT>::to_f32(logits[t * num_experts + e]) : -INFINITY;
     }
-    m = wave_max(m);
-    float sum = 0.f;
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-      x[r] = lane + r * kWave < num_experts ? expf(x[r] - m) : 0.f;
-      sum += x[r];
-    }
-    sum = wave_sum(sum);
-    // logsumexp of the row, the term of the router z-loss (router.py:37): an infinite maximum is the result itself
-    if (lse && lane == 0) lse[t] = (m == INFINITY || m == -INFINITY) ? m : m + logf(sum);
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-      const int e = lane + r * kWave;
-      const E s = Elem<DT>::from_f32(x[r] / sum);
-      if (e < num_experts) scores[t * num_experts + e] = s;
-      // The selection key: the rounded score; -1 marks "not a candidate" (scores are >= 0).  A NaN score (a NaN
-      // or +inf logit makes the whole row NaN) ranks above every number, as torch.topk ranks it, so that the
-      // indices written are always experts: +inf, which no score can be, stands for it.
-      const float v = Elem<DT>::to_f32(s);
-      x[r] = e < num_experts ? (v != v ? INFINITY : v) : -1.f;
-    }
-    float my_w = 0.f;
-    int my_i = 0;
-    for (int j = 0; j < top_k; ++j) {
-      float best = -1.f;
-      int best_e = 0x7fffffff;
-#pragma unroll
-      for (int r = 0; r < R; ++r)   // ascending expert index: a later equal value does not replace an earlier one
-        if (x[r] > best) { best = x[r]; best_e = lane + r * kWave; }
-#pragma unroll
-      for (int off = 32; off > 0; off >>= 1) {
-        const float ov = __shfl_xor(best, off, 64);
-        const int oe = __shfl_xor(best_e, off, 64);
-        if (ov > best || (ov == best && oe < best_e)) { best = ov; best_e = oe; }
-      }
-      if (lane == j) { my_w = best == INFINITY ? NAN : best; my_i = best_e; }
-#pragma unroll
-      for (int r = 0; r < R; ++r)
-        if (lane + r * kWave == best_e) x[r] = -1.f;
-    }
-    const bool live = lane < top_k;
-    if (p > 0.f) {
-      const float norm = Elem<DT>::to_f32(Elem<DT>::from_f32(wave_pnorm(my_w, live, p)));
-      my_w = my_w / norm;
-    }
-    if (live) {
-      weights[t * top_k + lane] = Elem<DT>::from_f32(my_w);
-      indices[t * top_k + lane] = my_i;
-      if (indices32) indices32[t * top_k + lane] = my_i;   // what the routing kernels take, without a cast pass
-    }
+    route_token<DT, R>(x, t, num_experts, top_k, p, (E*)scores, (E*)weights, indices, indices32, lse);
   }
+}
+
+// The router's linear layer and the above in one launch, for a few tokens: logits[t][e] = x[t] . weight[e], summed in fp32 and
+// rounded to the storage type.  One workgroup of sixteen waves per token: wave w has experts w, w + 16, ..., a lane eight
+// columns of every 512, so that a load of a wave is 1 KiB of one row.
+//
+// What bounds it: the latency of reading the weights (64 experts of 2048: 256 KiB) through one compute unit, and of the chain
+// of waits behind it.  The vendor library's product and router_forward_kernel / this kernel, us, 5 tokens: 8 experts of 4096:
+// 12.4 / 6.8, 12 of 1032: 10.8 / 7.8, 64 of 2048: 11.1 / 9.1, 64 of 4096: 13.6 / 11.1, 128 of 2048: 11.6 / 11.7, 128 of 4096:
+// 14.0 / 16.1; 256 tokens (one per compute unit): 12.8 / 7.4, 11.7 / 8.4, 11.4 / 10.4, 14.0 / 12.7, 12.0 / 13.7.  (On the matrix
+// instruction, 16 tokens per workgroup, whose loads take 16 rows at a stride of often a power of two: 64 of 2048 16 - 21.)
+constexpr int kLinearWaves = 16;
+constexpr int kLinearMaxExperts = 8 * kLinearWaves;
+
+typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+
+// PER: experts per wave
+template <int DT, int PER>
+__global__ void __launch_bounds__(kLinearWaves * kWave)
+router_linear_kernel(const uint16_t* __restrict__ x_, const uint16_t* __restrict__ weight, int hidden, int num_experts,
+                     int top_k, float p, void* __restrict__ scores, void* __restrict__ weights, int64_t* __restrict__ indices,
+                     int32_t* __restrict__ indices32) {
+  typedef typename Elem<DT>::type E;
+  constexpr int kAhead = PER >= 8 ? 2 : PER >= 4 ? 4 : 8;   // pieces of a row under way, next to those of the other experts
+  constexpr int R = PER <= 4 ? 1 : 2;
+  __shared__ float logits[PER * kLinearWaves < kWave ? kWave : PER * kLinearWaves];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = lane_id();
+  const int64_t t = blockIdx.x;
+  // pieces past the end of a row and experts past the last (bit 31: out of range) read as zeros
+  const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc((void*)(x_ + t * hidden), 0, hidden * 2, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc((void*)weight, 0, num_experts * hidden * 2, 0x00020000);
+  auto unpack = [](uint32_t v, float& lo, float& hi) {
+    lo = Elem<DT>::to_f32(__builtin_bit_cast(E, (uint16_t)v));
+    hi = Elem<DT>::to_f32(__builtin_bit_cast(E, (uint16_t)(v >> 16)));
+  };
+  float acc[PER];
+#pragma unroll
+  for (int i = 0; i < PER; ++i) acc[i] = 0.f;
+  const uint32_t pitch = (uint32_t)hidden * 2u;
+  for (int k0 = lane * 8; k0 - lane * 8 < hidden; k0 += 512 * kAhead) {
+    u32x4_t xv[kAhead], wv[kAhead][PER];
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) {
+      const uint32_t at = 2u * (uint32_t)(k0 + 512 * u) | (k0 + 512 * u < hidden ? 0u : 0x80000000u);
+      xv[u] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rx, (int)at, 0, 0));
+#pragma unroll
+      for (int i = 0; i < PER; ++i)
+        wv[u][i] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rw, (int)(at + (uint32_t)(wave + kLinearWaves * i) * pitch), 0, 0));
+    }
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u)
+#pragma unroll
+      for (int w = 0; w < 4; ++w) {
+        float x0, x1;
+        unpack(xv[u][w], x0, x1);
+#pragma unroll
+        for (int i = 0; i < PER; ++i) {
+          float w0, w1;
+          unpack(wv[u][i][w], w0, w1);
+          acc[i] = fmaf(x0, w0, acc[i]);
+          acc[i] = fmaf(x1, w1, acc[i]);
+        }
+      }
+  }
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    const float sum = wave_sum(acc[i]);
+    if (lane == 0) logits[wave + kLinearWaves * i] = sum;
+  }
+  __syncthreads();
+  if (wave != 0) return;
+  float v[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int e = lane + r * kWave;
+    v[r] = e < num_experts ? Elem<DT>::to_f32(Elem<DT>::from_f32(logits[e])) : -INFINITY;
+  }
+  route_token<DT, R>(v, t, num_experts, top_k, p, (E*)scores, (E*)weights, indices, indices32, nullptr);
 }
 
 // grad_logits = d(loss)/d(logits) given d/d(weights) (and optionally d/d(scores) from other users of the
@@ -211,6 +297,32 @@ int mbx_router_forward(const void* logits, int dtype, int64_t tokens, int num_ex
   if (!logits || !scores || !weights || !indices) return MBX_EINVAL;
   hipStream_t s = as_stream(stream);
   MBX_ROUTER_DISPATCH(router_forward_kernel, logits, tokens, num_experts, top_k, norm_p, scores, weights, indices, indices32, lse);
+  return launch_status();
+}
+
+int mbx_router_linear_forward(const void* x, const void* weight, int dtype, int64_t tokens, int hidden, int num_experts, int top_k,
+                              float norm_p, void* scores, void* weights, int64_t* indices, int32_t* indices32, mbx_stream_t stream) {
+  if (tokens < 0 || hidden <= 0 || num_experts <= 0 || top_k <= 0 || top_k > num_experts || !(norm_p >= 0.f)) return MBX_EINVAL;
+  if (dtype != MBX_BF16 && dtype != MBX_F16 && dtype != MBX_F32) return MBX_EINVAL;
+  if (dtype == MBX_F32 || hidden % 8 || num_experts > kLinearMaxExperts || top_k > kWave || (int64_t)num_experts * hidden * 2 >= ((int64_t)1 << 30) ||
+      tokens > 0x7fffffff || (((uintptr_t)x | (uintptr_t)weight) & 15u)) return MBX_EUNSUPPORTED;
+  if (tokens == 0) return 0;
+  if (!x || !weight || !scores || !weights || !indices) return MBX_EINVAL;
+  hipStream_t s = as_stream(stream);
+#define MBX_ROUTER_LINEAR(PER)                                                                                              \
+  do {                                                                                                                      \
+    if (dtype == MBX_BF16)                                                                                                  \
+      router_linear_kernel<MBX_BF16, PER><<<(unsigned)tokens, kLinearWaves * kWave, 0, s>>>(                                \
+          (const uint16_t*)x, (const uint16_t*)weight, hidden, num_experts, top_k, norm_p, scores, weights, indices, indices32); \
+    else                                                                                                                    \
+      router_linear_kernel<MBX_F16, PER><<<(unsigned)tokens, kLinearWaves * kWave, 0, s>>>(                                 \
+          (const uint16_t*)x, (const uint16_t*)weight, hidden, num_experts, top_k, norm_p, scores, weights, indices, indices32); \
+  } while (0)
+  if (num_experts <= kLinearWaves) MBX_ROUTER_LINEAR(1);
+  else if (num_experts <= 2 * kLinearWaves) MBX_ROUTER_LINEAR(2);
+  else if (num_experts <= 4 * kLinearWaves) MBX_ROUTER_LINEAR(4);
+  else MBX_ROUTER_LINEAR(8);
+#undef MBX_ROUTER_LINEAR
   return launch_status();
 }
 

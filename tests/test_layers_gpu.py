@@ -255,6 +255,42 @@ def _softmax_topk_reference(logits, top_k, norm_p):
     return scores, w, i
 
 
+@pytest.mark.parametrize('tokens,hidden,experts,top_k,norm_p', [
+    (1, 8, 1, 1, None), (5, 2048, 64, 6, 1), (16, 4096, 8, 2, 1), (17, 1032, 12, 3, 2), (33, 520, 65, 4, 1), (256, 1024, 128, 8, None),
+    (15, 264, 127, 2, 1), (31, 72, 16, 1, None)])
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])
+def test_router_with_its_linear_layer_in_one_kernel(tokens, hidden, experts, top_k, norm_p, dtype):
+    """The fused kernel against softmax and choice on logits computed in fp64 and rounded: another order of the sums moves a
+    logit by one rounding step now and then, so scores are held to two steps of it, and the choices to the scores."""
+    from megablocks_amd.layers import router as r
+    torch.manual_seed(tokens + experts)
+    layer = torch.nn.Linear(hidden, experts, bias=False, device='cuda', dtype=dtype)
+    with torch.no_grad():
+        layer.weight.normal_(0, 0.5 / hidden ** 0.5)
+    x = torch.randn(tokens, hidden, device='cuda').to(dtype)
+    with torch.no_grad():
+        assert r._LinearSoftmaxTopK.supported(x, layer, top_k)
+        scores, weights, indices, indices32 = r._LinearSoftmaxTopK.apply(x, layer.weight, top_k, norm_p or 0)
+    logits = (x.double() @ layer.weight.detach().double().t()).to(dtype)
+    want = logits.double().softmax(-1)
+    step = torch.finfo(dtype).eps
+    assert float(((scores.double() - want).abs() / want).max()) < 2 * step * (1 + float(logits.abs().max()))
+    order = scores.double().sort(dim=-1, descending=True, stable=True)
+    assert torch.equal(indices, order.indices[:, :top_k]) and torch.equal(indices32.long(), indices)
+    picked = order.values[:, :top_k].detach()
+    if norm_p:
+        picked = picked / picked.norm(p=norm_p, dim=-1, keepdim=True)
+    assert float(((weights.double() - picked).abs() / picked).max()) < 2 * step
+    # what the kernel does not take stays with the layer's own call
+    hook = layer.register_forward_hook(lambda *_: None)
+    with torch.no_grad():
+        assert not r._LinearSoftmaxTopK.supported(x, layer, top_k)
+        hook.remove()
+        assert not r._LinearSoftmaxTopK.supported(x.float(), layer, top_k)
+        assert not r._LinearSoftmaxTopK.supported(x.repeat(257, 1), layer, top_k)
+    assert not r._LinearSoftmaxTopK.supported(x, layer, top_k)
+
+
 @pytest.mark.parametrize('tokens,experts,top_k', [(1, 1, 1), (300, 8, 2), (257, 64, 1), (200, 65, 6), (100, 128, 8),
                                                   (50, 512, 64), (1000, 16, 4)])
 @pytest.mark.parametrize('norm_p', [0, 1, 2, 3.0])
