@@ -534,13 +534,7 @@ int launch_tn(const DmaCall& call) {
     // the rows of b picked through the sorted assignments: the full tile only, one segment
     if (!gather.src_bins || !gather.row_table || gather.top_k <= 0 || gather.n_slots > 0x7fffffff) return MBX_EINVAL;
     if (segmented || !std::is_same<T, TS>::value) return MBX_EUNSUPPORTED;
-    if (!gather.table_ready) {
-      uint32_t magic = 0;
-      int shift = 0;
-      dma::gather_divisor(gather.top_k, magic, shift);
-      dma::gather_row_table_kernel<<<(unsigned)ceil_div(dma::row_table_entries(gather.n_slots, num_groups), 256), 256, 0, s>>>(
-          gather.slots, gather.src_bins, num_groups, (int)gather.n_slots, gather.src_rows, (uint32_t)n * 2u, magic, shift, gather.row_table);
-    }
+    if (!gather.table_ready) dma::build_row_table(call);
     if constexpr (T::BM == 256 && T::SB == 2) {
       auto gkern = dma::gmm_tn_kernel<DT, T, T, false, true>;
       int grc = allow_lds(gkern, lds);
@@ -560,6 +554,7 @@ int launch_tn(const DmaCall& call) {
 static int gmm_dma(const DmaCall& call) {
   if (gmm_few_takes(call)) return gmm_few(call);
   if (call.layout != MBX_TN) return call.k % dma::TileMain::BK == 0 ? gmm_rows(call) : gmm_rows_tail(call);
+  if (gmm_tn_short_takes(call)) return gmm_tn_short(call);
   if (call.gather.slots) {   // gathered rows: the full tile only
     if (call.dtype == MBX_BF16) return launch_tn<MBX_BF16, dma::TileMain, dma::TileMain>(call);
     return launch_tn<MBX_F16, dma::TileMain, dma::TileMain>(call);

@@ -61,6 +61,10 @@ struct DmaCall {
 bool gmm_few_takes(const DmaCall& call);
 int gmm_few(const DmaCall& call);
 
+// TN launches with few rows per expert (gmm_tn_short.hip), and whether a launch is one of them.
+bool gmm_tn_short_takes(const DmaCall& call);
+int gmm_tn_short(const DmaCall& call);
+
 // NN / NT launches, k a multiple of 64 (gmm_rows.hip) and of 8 only (gmm_rows_tail.hip).
 int gmm_rows(const DmaCall& call);
 int gmm_rows_tail(const DmaCall& call);

@@ -1956,3 +1956,12 @@ __global__ void gather_row_table_kernel(const int32_t* __restrict__ slots, const
 }
 
 }  // namespace dma
+// The table of a gathered TN launch, written by a launch in front of it.
+static inline void build_row_table(const DmaCall& q) {
+  uint32_t magic = 0;
+  int shift = 0;
+  gather_divisor(q.gather.top_k, magic, shift);
+  gather_row_table_kernel<<<(unsigned)ceil_div(row_table_entries(q.gather.n_slots, q.num_groups), 256), 256, 0, q.stream>>>(
+      q.gather.slots, q.gather.src_bins, q.num_groups, (int)q.gather.n_slots, q.gather.src_rows, (uint32_t)q.n * 2u, magic, shift, q.gather.row_table);
+}
+

@@ -1139,3 +1139,43 @@ def test_batched_mlp_with_activation_epilogues(gg, groups, rows, k, n, dtype):
     w = w2.clone().requires_grad_(True)
     BatchedGeluMLP.apply(x, w1, w, sizes).backward(grad)
     assert torch.equal(w.grad, results[0][3])
+
+
+@pytest.mark.parametrize('groups,rows,k,n,skew', [(1, 1, 8, 8, False), (1, 1024, 128, 136, False), (3, 0, 64, 128, False),
+                                                  (4, 257, 136, 120, False), (8, 8 * 63, 264, 1032, True), (64, 64 * 130, 256, 384, True),
+                                                  (70, 70 * 40, 72, 264, True), (130, 900, 128, 2056, False),
+                                                  (5, 5 * 256, 1032, 4616, False), (16, 16 * 257, 1024, 2056, True)])
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])
+def test_gmm_tn_with_few_rows_per_expert(gg, groups, rows, k, n, skew, dtype):
+    """Weight gradients with short reductions, on both sides of the line where the kernel for them takes over, alike and
+    skewed experts, plain and on gathered rows, against fp32; rows of infinities past an expert's last (its neighbour's) must not
+    reach it."""
+    torch.manual_seed(rows + k)
+    if skew:
+        p = torch.arange(1, groups + 1).float() ** -1.2
+        sizes = (p / p.sum() * rows).floor().long()
+        sizes[0] += rows - int(sizes.sum())
+        sizes = sizes[torch.randperm(groups)]
+    else:
+        sizes = _sizes(groups, rows, seed=k, empty=(0,) if groups > 2 and rows else ())
+    a = torch.randn(rows, k, device='cuda').to(dtype)
+    x = torch.randn(max(rows, 1), n, device='cuda').to(dtype)[:rows]
+    b = x.clone()
+    ends = torch.cumsum(sizes, 0)
+    bad = int(torch.nonzero(sizes)[0]) if rows > 1 and int((sizes > 0).sum()) > 1 else -1
+    if bad >= 0:
+        b[int(ends[bad] - sizes[bad]):int(ends[bad])] = float('inf')
+    keep = [e for e in range(groups) if e != bad]
+    want = torch.stack([a[int(ends[e] - sizes[e]):int(ends[e])].float().t() @ b[int(ends[e] - sizes[e]):int(ends[e])].float()
+                        for e in keep]) if keep else torch.zeros(0, k, n, device='cuda')
+    got = gg.backend.gmm(a, b, sizes, trans_a=True)
+    assert torch.isfinite(got[keep]).all() and (not keep or rel_err(got[keep], want) < TOL)
+    assert not got[(sizes == 0).cuda()].any()
+    if keep and float(want.abs().max()) > 0:
+        assert max_block_err(got[keep], want) < TOL
+    if rows and k > 128:   # one expert per token: row r is row order[r] of the tokens
+        order = torch.randperm(rows, device='cuda').int()
+        bins = ends.cuda().int()
+        bin_ids = torch.repeat_interleave(torch.arange(groups), sizes).int().cuda()
+        src = gg.GatheredRows(x, order, bin_ids, bins, None, 1, rows)
+        assert torch.equal(gg.gmm_tn_gather(a, src, sizes.cuda()), gg.backend.gmm(a, x[order.long()], sizes, trans_a=True))
