@@ -1965,3 +1965,4 @@ static inline void build_row_table(const DmaCall& q) {
       q.gather.slots, q.gather.src_bins, q.num_groups, (int)q.gather.n_slots, q.gather.src_rows, (uint32_t)q.n * 2u, magic, shift, q.gather.row_table);
 }
 
+}  // namespace dma
