@@ -1955,7 +1955,6 @@ __global__ void gather_row_table_kernel(const int32_t* __restrict__ slots, const
   table[s] = v;
 }
 
-}  // namespace dma
 // The table of a gathered TN launch, written by a launch in front of it.
 static inline void build_row_table(const DmaCall& q) {
   uint32_t magic = 0;
