@@ -286,6 +286,13 @@ int mbx_gmm_gather(const void* x, int64_t x_rows, const int32_t* indices, int to
                    const void* b1, const void* b2, void* c, void* c2, void* h, int dtype, const int32_t* bins,
                    int num_groups, int64_t rows, int k, int n, int act, mbx_stream_t stream);
 
+/* The activation output alone, where nothing will be differentiated: h of mbx_gmm_gather (indices NULL: of mbx_gmm_act,
+ * or with b2 of mbx_gmm_glu, x then [rows, k]; x_rows, top_k and x_bins are ignored), bit for bit; the products are not
+ * written.  Same restrictions. */
+int mbx_gmm_hidden(const void* x, int64_t x_rows, const int32_t* indices, int top_k, const int32_t* x_bins, const void* b1,
+                   const void* b2, void* h, int dtype, const int32_t* bins, int num_groups, int64_t rows, int k, int n, int act,
+                   mbx_stream_t stream);
+
 /* The experts' second product and the weighted combine in one launch, for top_k = 1: megablocks/layers/mlp.py:523 /
  * glu.py:205 (`gmm(x, w2, batch_sizes)`) followed by megablocks/layers/dmoe.py:280 (`ops.scatter(x, indices, bin_ids,
  * expert_weights, bins, top_k)`, megablocks/backend/kernels.py:173-207).  With one expert per token an output row is one

@@ -698,17 +698,20 @@ static int gmm_dual_ws(const void* a, const void* b, const void* a2, const void*
 // (kEpiDglu*: pre2 = x2, out2 = the second output.)
 // (kEpiGlu*: b2 = the second matrix, extra = the gated activation, out2 = the second product.)
 // gather.slots non-null: `a` is read through the row map (no epilogue, kEpiAct and kEpiGlu* only; `extra` may then be
-// null for no epilogue).  layout: MBX_NT, or MBX_NN with kEpiAct.
+// null for no epilogue).  layout: MBX_NT, or MBX_NN with kEpiAct.  only_extra (kEpiAct, kEpiGlu*): the products themselves are not
+// written (c, out2 null).
 static int gmm_epilogue(const void* a, const void* b, void* c, void* extra, int dtype, const int32_t* bins, int num_groups,
                            int64_t rows, int k, int n, int act, int epi, mbx_stream_t stream, const void* pre2 = nullptr,
-                           void* out2 = nullptr, const void* b2 = nullptr, GatherRows gather = GatherRows(), int layout = MBX_NT) {
+                           void* out2 = nullptr, const void* b2 = nullptr, GatherRows gather = GatherRows(), int layout = MBX_NT,
+                        bool only_extra = false) {
   if (num_groups < 0 || rows < 0 || k < 0 || n < 0) return MBX_EINVAL;
   if (dtype != MBX_BF16 && dtype != MBX_F16 && dtype != MBX_F32) return MBX_EINVAL;
   const bool dglu = dma::epi_is_dglu(epi), glu = dma::epi_is_glu(epi);
   const bool plain = epi == dma::kEpiNone;   // gathered rows only
   if (!dglu && !glu && !plain && act != MBX_ACT_GELU_TANH) return MBX_EUNSUPPORTED;
   if (num_groups == 0 || rows == 0 || n == 0) return 0;
-  if (!bins || !c || (!extra && !plain) || (k > 0 && (!a || !b)) || (dglu && (!pre2 || !out2)) || (glu && (!out2 || (k > 0 && !b2)))) return MBX_EINVAL;
+  if (!bins || (!c && !only_extra) || (!extra && !plain) || (k > 0 && (!a || !b)) || (dglu && (!pre2 || !out2)) ||
+      (glu && ((!out2 && !only_extra) || (k > 0 && !b2)))) return MBX_EINVAL;
   if (rows > 0x7fffffff) return MBX_ERANGE;
   bool ok = dtype != MBX_F32 && aligned16(a) && aligned16(b) && aligned16(c) && aligned16(extra) && k > 0 &&
             k % 8 == 0 && n % 8 == 0 && dma_sizes_ok(k, n) && (!dglu || (aligned16(pre2) && aligned16(out2)));
@@ -748,12 +751,13 @@ int mbx_gmm_glu(const void* a, const void* b1, const void* b2, void* x1, void* x
                          act == MBX_ACT_SILU ? dma::kEpiGluSilu : dma::kEpiGluGelu, stream, nullptr, x2, b2);
 }
 
-int mbx_gmm_gather(const void* x, int64_t x_rows, const int32_t* indices, int top_k, const int32_t* x_bins, const void* b1,
-                   const void* b2, void* c, void* c2, void* h, int dtype, const int32_t* bins, int num_groups, int64_t rows,
-                   int k, int n, int act, mbx_stream_t stream) {
+// mbx_gmm_gather and the gathered form of mbx_gmm_hidden (only_extra)
+static int gmm_gather(const void* x, int64_t x_rows, const int32_t* indices, int top_k, const int32_t* x_bins, const void* b1,
+                      const void* b2, void* c, void* c2, void* h, int dtype, const int32_t* bins, int num_groups, int64_t rows,
+                      int k, int n, int act, mbx_stream_t stream, bool only_extra) {
   if (x_rows < 0 || top_k <= 0 || k < 0 || num_groups < 0 || rows < 0 || n < 0) return MBX_EINVAL;
   if (num_groups == 0 || rows == 0 || n == 0) return 0;   // nothing to write (empty outputs may come as NULL)
-  if (b2 ? (act != MBX_ACT_SILU && act != MBX_ACT_GELU_TANH) || !c2 || !h : c2 != nullptr) return MBX_EINVAL;
+  if (b2 ? (act != MBX_ACT_SILU && act != MBX_ACT_GELU_TANH) || (!c2 && !only_extra) || !h : c2 != nullptr) return MBX_EINVAL;
   if (h && !b2 && act != MBX_ACT_GELU_TANH) return MBX_EUNSUPPORTED;
   if (!indices || (k > 0 && !x && x_rows > 0)) return MBX_EINVAL;
   // the row map is indexed with 32 bits and the rows of x are addressed with 31 (bit 31 marks a row of zeros); whole K tiles
@@ -765,7 +769,24 @@ int mbx_gmm_gather(const void* x, int64_t x_rows, const int32_t* indices, int to
   gather.top_k = top_k;
   gather.src_rows = (int)x_rows;
   const int epi = b2 ? (act == MBX_ACT_SILU ? dma::kEpiGluSilu : dma::kEpiGluGelu) : h ? dma::kEpiAct : dma::kEpiNone;
-  return gmm_epilogue(x, b1, c, h, dtype, bins, num_groups, rows, k, n, act, epi, stream, nullptr, c2, b2, gather);
+  return gmm_epilogue(x, b1, c, h, dtype, bins, num_groups, rows, k, n, act, epi, stream, nullptr, c2, b2, gather, MBX_NT, only_extra);
+}
+
+int mbx_gmm_gather(const void* x, int64_t x_rows, const int32_t* indices, int top_k, const int32_t* x_bins, const void* b1,
+                   const void* b2, void* c, void* c2, void* h, int dtype, const int32_t* bins, int num_groups, int64_t rows,
+                   int k, int n, int act, mbx_stream_t stream) {
+  return gmm_gather(x, x_rows, indices, top_k, x_bins, b1, b2, c, c2, h, dtype, bins, num_groups, rows, k, n, act, stream, false);
+}
+
+int mbx_gmm_hidden(const void* x, int64_t x_rows, const int32_t* indices, int top_k, const int32_t* x_bins, const void* b1,
+                   const void* b2, void* h, int dtype, const int32_t* bins, int num_groups, int64_t rows, int k, int n, int act,
+                   mbx_stream_t stream) {
+  if (num_groups == 0 || rows == 0 || n == 0) return 0;
+  if (!h) return MBX_EINVAL;
+  if (indices) return gmm_gather(x, x_rows, indices, top_k, x_bins, b1, b2, nullptr, nullptr, h, dtype, bins, num_groups, rows, k, n, act, stream, true);
+  if (b2 && act != MBX_ACT_SILU && act != MBX_ACT_GELU_TANH) return MBX_EINVAL;
+  const int epi = b2 ? (act == MBX_ACT_SILU ? dma::kEpiGluSilu : dma::kEpiGluGelu) : dma::kEpiAct;
+  return gmm_epilogue(x, b1, nullptr, h, dtype, bins, num_groups, rows, k, n, act, epi, stream, nullptr, nullptr, b2, GatherRows(), MBX_NT, true);
 }
 
 int mbx_gmm_scatter(const void* a, const void* b, void* c, void* out, int dtype, const int32_t* bins, int num_groups,

@@ -656,7 +656,7 @@ __device__ __forceinline__ void gelu_tanh_bwd8(float (&g)[8], const float (&x)[8
 
 // What the store of an output tile does besides storing it:
 //   kEpiNone      nothing;
-//   kEpiAct       also stores gelu_tanh of the (rounded) tile to a second output of the same shape;
+//   kEpiAct       also (or only, when c is null) stores gelu_tanh of the (rounded) tile to a second output of the same shape;
 //   kEpiDact      multiplies the (rounded) tile by d/dx gelu_tanh of a second input of the same shape before storing it;
 //   kEpiDgluSilu, kEpiDgluGelu   the tile g is the gradient of act(x1) * x2 (act = SiLU / tanh-GELU) with x1, x2 two
 //                 more inputs of the same shape: stores g * round(act(x1)) and round(g * x2) * act'(x1), two outputs,
@@ -670,6 +670,7 @@ __device__ __forceinline__ void gelu_tanh_bwd8(float (&g)[8], const float (&x)[8
 enum { kEpiNone = 0, kEpiAct = 1, kEpiDact = 2, kEpiDgluSilu = 3, kEpiDgluGelu = 4, kEpiGluSilu = 5, kEpiGluGelu = 6, kEpiCombine = 7 };
 constexpr bool epi_is_dglu(int epi) { return epi == kEpiDgluSilu || epi == kEpiDgluGelu; }
 constexpr bool epi_is_glu(int epi) { return epi == kEpiGluSilu || epi == kEpiGluGelu; }
+constexpr bool epi_c_optional(int epi) { return epi == kEpiAct || epi_is_glu(epi) || epi == kEpiCombine; }   // c (with the gate: and out2) may be null
 
 // the eight 16-bit values of a 16-byte chunk as fp32 and back (rounded)
 template <int DT>
@@ -918,7 +919,7 @@ __device__ __forceinline__ void block_store(const typename T::Acc (&acc)[T::TM][
       char* const cb = (char*)c;
       char* const hb = (char*)extra;
       char* const ob = (char*)out2;
-      const bool full_n = n_base + T::BN / 2 <= n_lim;      // uniform
+      const bool full_n = n_base + T::BN / 2 <= n_lim, keep = c != nullptr;      // uniform
 #pragma unroll 1
       for (int b = 0; b < ITERS; b += BATCH) {
         u32x4 v1[BATCH], v2[BATCH], h[BATCH];
@@ -935,15 +936,19 @@ __device__ __forceinline__ void block_store(const typename T::Acc (&acc)[T::TM][
           if (m + u * ROW_STEP >= m_lim || n >= n_lim) continue;
           const uint32_t o = off + (uint32_t)u * off_step;
           if (full_n || n + 8 <= n_lim) {
-            __builtin_nontemporal_store(v1[u], (u32x4*)(cb + o));
-            __builtin_nontemporal_store(v2[u], (u32x4*)(ob + o));
+            if (keep) {
+              __builtin_nontemporal_store(v1[u], (u32x4*)(cb + o));
+              __builtin_nontemporal_store(v2[u], (u32x4*)(ob + o));
+            }
             __builtin_nontemporal_store(h[u], (u32x4*)(hb + o));
           } else {
 #pragma unroll
             for (int t = 0; t < 8; ++t)
               if (n + t < n_lim) {
-                ((uint16_t*)(cb + o))[t] = (uint16_t)(v1[u][t >> 1] >> ((t & 1) * 16));
-                ((uint16_t*)(ob + o))[t] = (uint16_t)(v2[u][t >> 1] >> ((t & 1) * 16));
+                if (keep) {
+                  ((uint16_t*)(cb + o))[t] = (uint16_t)(v1[u][t >> 1] >> ((t & 1) * 16));
+                  ((uint16_t*)(ob + o))[t] = (uint16_t)(v2[u][t >> 1] >> ((t & 1) * 16));
+                }
                 ((uint16_t*)(hb + o))[t] = (uint16_t)(h[u][t >> 1] >> ((t & 1) * 16));
               }
           }
@@ -1001,6 +1006,7 @@ __device__ __forceinline__ void block_store(const typename T::Acc (&acc)[T::TM][
     }
     // the second output goes where kEpiAct's does (extra) or to out2 (kEpiDglu*: extra is an input there)
     constexpr bool kTwoOut = EPI == kEpiAct || kDglu;
+    const bool keep = EPI != kEpiAct || c != nullptr;   // uniform
     char* const second = kDglu ? ob : eb;
 #pragma unroll 1
     for (int b = 0; b < ITERS; b += BATCH) {
@@ -1075,7 +1081,7 @@ __device__ __forceinline__ void block_store(const typename T::Acc (&acc)[T::TM][
 #pragma unroll
         for (int u = 0; u < BATCH; ++u)
           if (m + u * ROW_STEP < m_lim) {
-            __builtin_nontemporal_store(v[u], (u32x4*)(cb + (off + (uint32_t)u * off_step)));
+            if (keep) __builtin_nontemporal_store(v[u], (u32x4*)(cb + (off + (uint32_t)u * off_step)));
             if constexpr (EPI == kEpiAct) y[u] = gelu_fwd_chunk<DT>(v[u]);
             if constexpr (kTwoOut) __builtin_nontemporal_store(y[u], (u32x4*)(second + (off + (uint32_t)u * off_step)));
           }
@@ -1087,13 +1093,13 @@ __device__ __forceinline__ void block_store(const typename T::Acc (&acc)[T::TM][
           if constexpr (EPI == kEpiAct) y[u] = gelu_fwd_chunk<DT>(v[u]);
           uint16_t* dst2 = (uint16_t*)(second + (off + (uint32_t)u * off_step));
           if (n + 8 <= n_lim) {
-            *(u32x4*)dst = v[u];
+            if (keep) *(u32x4*)dst = v[u];
             if constexpr (kTwoOut) *(u32x4*)dst2 = y[u];
           } else {
 #pragma unroll
             for (int t = 0; t < 8; ++t)
               if (n + t < n_lim) {
-                dst[t] = (uint16_t)(v[u][t >> 1] >> ((t & 1) * 16));
+                if (keep) dst[t] = (uint16_t)(v[u][t >> 1] >> ((t & 1) * 16));
                 if constexpr (kTwoOut) dst2[t] = (uint16_t)(y[kTwoOut ? u : 0][t >> 1] >> ((t & 1) * 16));
               }
           }
@@ -1374,7 +1380,7 @@ gmm_rows_kernel(const uint16_t* __restrict__ a, const uint16_t* __restrict__ b, 
     // the second matrix of a [w1 | v1] tile: rows BN / 2 .. BN - 1 of the tile are its rows b_r0 .. b_r0 + BN / 2 - 1
     if (epi_is_glu(EPI)) g.rsrc_b2 = make_rsrc(b2 + ((int64_t)e * n - T::BN / 2) * k, (uint32_t)(((int64_t)n + T::BN / 2) * k * 2));
     g.b_r0 = tn * kTileCols;
-    uint16_t* const c_tile = c + (int64_t)row0 * n;
+    uint16_t* const c_tile = epi_c_optional(EPI) && c == nullptr ? nullptr : c + (int64_t)row0 * n;
     uint16_t* const e_tile = EPI != kEpiNone ? extra + (int64_t)row0 * n : nullptr;
     const uint16_t* const p_tile = epi_is_dglu(EPI) ? a2 + (int64_t)row0 * n : nullptr;   // x2 of the gated activation
     uint16_t* const o_tile = epi_is_dglu(EPI) || epi_is_glu(EPI) ? out2 + (int64_t)row0 * n : nullptr;
@@ -1545,7 +1551,7 @@ gmm_rows_kernel(const uint16_t* __restrict__ a, const uint16_t* __restrict__ b, 
       // the second matrix of a [w1 | v1] tile: rows BN / 2 .. BN - 1 of the tile are its rows b_r0 .. b_r0 + BN / 2 - 1
       if (epi_is_glu(EPI)) g.rsrc_b2 = make_rsrc(b2 + ((int64_t)e * n - T::BN / 2) * k, (uint32_t)(((int64_t)n + T::BN / 2) * k * 2));
       g.b_r0 = tn * kTileCols;
-      uint16_t* const c_tile = EPI == kEpiCombine && c == nullptr ? nullptr : c + (int64_t)row0 * n;
+      uint16_t* const c_tile = epi_c_optional(EPI) && c == nullptr ? nullptr : c + (int64_t)row0 * n;
       uint16_t* const e_tile = EPI != kEpiNone && EPI != kEpiCombine ? extra + (int64_t)row0 * n : nullptr;
       const uint16_t* const p_tile = epi_is_dglu(EPI) ? a2 + (int64_t)row0 * n : nullptr;   // x2 of the gated activation
       uint16_t* const o_tile = epi_is_dglu(EPI) || epi_is_glu(EPI) ? out2 + (int64_t)row0 * n : nullptr;

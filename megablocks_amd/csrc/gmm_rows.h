@@ -94,15 +94,15 @@ int launch_rows(const DmaCall& call) {
     switch (epi) {
       case dma::kEpiNone: MBX_LAUNCH_ROWS_G(false, false, dma::kEpiNone, true); break;
       case dma::kEpiAct: if (!extra) return MBX_EINVAL; MBX_LAUNCH_ROWS_G(false, false, dma::kEpiAct, true); break;
-      case dma::kEpiGluSilu: if (!extra || !b2 || !out2) return MBX_EINVAL; MBX_LAUNCH_ROWS_G(false, false, dma::kEpiGluSilu, true); break;
-      case dma::kEpiGluGelu: if (!extra || !b2 || !out2) return MBX_EINVAL; MBX_LAUNCH_ROWS_G(false, false, dma::kEpiGluGelu, true); break;
+      case dma::kEpiGluSilu: if (!extra || !b2 || (!out2 && cp)) return MBX_EINVAL; MBX_LAUNCH_ROWS_G(false, false, dma::kEpiGluSilu, true); break;
+      case dma::kEpiGluGelu: if (!extra || !b2 || (!out2 && cp)) return MBX_EINVAL; MBX_LAUNCH_ROWS_G(false, false, dma::kEpiGluGelu, true); break;
       default: return MBX_EINVAL;
     }
     return launch_status();
   }
   if (dma::epi_is_glu(epi)) {
     // b2 is the second matrix of the [w1 | v1] tiles (not a second operand pair)
-    if (layout != MBX_NT || !extra || !b2 || !out2 || a2) return MBX_EINVAL;
+    if (layout != MBX_NT || !extra || !b2 || (!out2 && cp) || a2) return MBX_EINVAL;
     if (epi == dma::kEpiGluSilu) MBX_LAUNCH_ROWS(false, false, dma::kEpiGluSilu); else MBX_LAUNCH_ROWS(false, false, dma::kEpiGluGelu);
     return launch_status();
   }

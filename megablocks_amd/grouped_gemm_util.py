@@ -224,13 +224,38 @@ def _nt_operands(a, b, batch_sizes, what, trans_b=True):
     return a, b, bins
 
 
-def gmm_act(a, b, batch_sizes, fuse=None, trans_b=True):
+def _hidden(a, src, b1, b2, bins, rows, act):
+    """The activation output of the experts' first product(s) alone (`mbx_gmm_hidden`): gmm_act's, or with b2 gmm_glu's, of
+    the rows `a`, or with `src` (a GatheredRows; a = src.x) of the rows that describes.  None: no kernel for the shape."""
+    k, n, groups = a.shape[1], b1.shape[1], bins.shape[0]
+    h = torch.empty((rows, n), dtype=a.dtype, device=a.device)
+    indices = None if src is None else src.indices.contiguous()
+    x_bins = None if src is None or src.padded_bins is None else src.bins.contiguous()
+    with _lib.device_of(a), _lib.record('gmm_nt_act' if b2 is None else 'gmm_nt_glu', rows=rows, k=k, n=n * (1 if b2 is None else 2),
+                                        elem=a.element_size(), groups=groups) as rec:
+        rc = lib.mbx_gmm_hidden(_lib.ptr(a), a.shape[0], _lib.ptr(indices), 1 if src is None else src.top_k, _lib.ptr(x_bins),
+                                _lib.ptr(b1), _lib.ptr(b2), _lib.ptr(h), _lib.dtype_of(a), _lib.ptr(bins), groups, rows, k, n, act,
+                                _lib.stream())
+        if rc == _lib.EUNSUPPORTED:
+            rec.cancel()
+    if rc == _lib.EUNSUPPORTED:
+        return None
+    _lib.check(rc, 'gmm_hidden')
+    return h
+
+
+def gmm_act(a, b, batch_sizes, fuse=None, trans_b=True, keep_product=True):
     """(c, gelu_tanh(c)) with c[r_e] = a[r_e] @ b[e].T (`trans_b` False: @ b[e]): the first product of the expert MLP and
     its activation (mlp.py:521-522; mlp.py:165-166), the activation applied in the product's epilogue where the library
     has a kernel for the shape (16-bit types, k and n multiples of 8) and the output is large enough for that to pay
-    (`fuse` None; True / False force the choice), else as a separate element-wise pass."""
+    (`fuse` None; True / False force the choice), else as a separate element-wise pass.  keep_product False (nothing will
+    differentiate): c may come back as None, the launch then writes the activation only."""
     a, b, bins = _nt_operands(a, b, batch_sizes, 'gmm_act', trans_b)
     rows, k, n, groups = a.shape[0], a.shape[1], b.shape[1 if trans_b else 2], bins.shape[0]
+    if not keep_product and trans_b and _use_epilogue(fuse, a, rows, n):
+        h = _hidden(a, None, b, None, bins, rows, ACT_GELU_TANH)
+        if h is not None:
+            return None, h
     c = torch.empty((rows, n), dtype=a.dtype, device=a.device)
     c_act = torch.empty_like(c)
     rc = _lib.EUNSUPPORTED
@@ -277,10 +302,11 @@ def gmm_dact(a, b, pre, batch_sizes, c=None, fuse=None):
     return c
 
 
-def gmm_glu(a, b1, b2, batch_sizes, act, fuse=None):
+def gmm_glu(a, b1, b2, batch_sizes, act, fuse=None, keep_product=True):
     """(x1, x2, h) with x1 = a[r_e] @ b1[e].T, x2 = a[r_e] @ b2[e].T and h = activation(x1) * x2: the two first
     products of the GLU experts and their gated activation (glu.py:201-204) in one launch where the library has a
-    kernel for the shape, else as two `gmm` and the element-wise pass.  act: 0 = SiLU, 1 = tanh-GELU."""
+    kernel for the shape, else as two `gmm` and the element-wise pass.  act: 0 = SiLU, 1 = tanh-GELU.  keep_product
+    False (nothing will differentiate): x1 and x2 may come back as None, the launch then writes h only."""
     a, b1, bins = _nt_operands(a, b1, batch_sizes, 'gmm_glu')
     _lib.require_cuda(b2)
     if b2.shape != b1.shape or b2.dtype != b1.dtype:
@@ -288,6 +314,10 @@ def gmm_glu(a, b1, b2, batch_sizes, act, fuse=None):
     b2 = b2.contiguous()
     rows, k, n, groups = a.shape[0], a.shape[1], b1.shape[1], bins.shape[0]
     rc = _lib.EUNSUPPORTED
+    if not keep_product and _use_epilogue(fuse, a, rows, n):
+        h = _hidden(a, None, b1, b2, bins, rows, act)
+        if h is not None:
+            return None, None, h
     if _use_epilogue(fuse, a, rows, n):
         x1, x2, h = (torch.empty((rows, n), dtype=a.dtype, device=a.device) for _ in range(3))
         with _lib.device_of(a), _lib.record('gmm_nt_glu', rows=rows, k=k, n=2 * n, elem=a.element_size(), groups=groups) as rec:
@@ -346,12 +376,13 @@ class GatheredRows:
         return kernels.padded_scatter(grad, self.indices, self.bin_ids, None, self.bins, self.padded_bins, self.top_k)
 
 
-def gmm_gather(src: GatheredRows, b1, batch_sizes, b2=None, act=None):
+def gmm_gather(src: GatheredRows, b1, batch_sizes, b2=None, act=None, keep_product=True):
     """The first product(s) of the experts on the rows `src` describes, read from the ungathered tokens (one launch,
     `mbx_gmm_gather`): bit-identical to `src.materialize()` followed by
         b2 None, act None:  (gmm(a, b1, trans_b=True),)
         b2 None, act ACT_GELU_TANH:  gmm_act(a, b1)  -> (c, gelu_tanh(c))
         b2 given:  gmm_glu(a, b1, b2, act)  -> (x1, x2, h)
+    keep_product False (nothing will differentiate): the entries in front of the activation's may be None.
     Returns None where the library has no kernel for the operands: the caller then gathers and multiplies."""
     x = src.x
     if not (x.is_cuda and x.ndim == 2 and x.dtype in (torch.bfloat16, torch.float16) and b1.ndim == 3 and
@@ -372,6 +403,9 @@ def gmm_gather(src: GatheredRows, b1, batch_sizes, b2=None, act=None):
     groups = bins.shape[0]
     if b1.shape[0] != groups or src.bins.numel() != groups:
         return None
+    if act is not None and not keep_product:
+        h = _hidden(x, src, b1, b2, bins, rows, act)
+        return None if h is None else (None, h) if b2 is None else (None, None, h)
     x_bins = None if src.padded_bins is None else src.bins.contiguous()
     c = torch.empty((rows, n), dtype=x.dtype, device=x.device)
     c2 = None if b2 is None else torch.empty_like(c)

@@ -115,14 +115,16 @@ class GroupedGLUExperts(torch.autograd.Function):
 
     @staticmethod
     @torch.amp.custom_fwd(device_type='cuda')
-    def forward(ctx, x, w1, v1, w2, batch_sizes, act, c_indices=None, c_bin_ids=None, c_bins=None, c_weights=None):
+    def forward(ctx, x, w1, v1, w2, batch_sizes, act, c_indices=None, c_bin_ids=None, c_bins=None, c_weights=None, keep=True):
         # c_*: the layer's combine (`gg.CombinedRows`), when the node is to return the combined output
+        # keep False: no gradient is recorded, the first products themselves need not be written
         x = x.contiguous()
-        sdd_out, v1_out, activation_fn_out = gg.gmm_glu(x, w1, v1, batch_sizes, act)
+        sdd_out, v1_out, activation_fn_out = gg.gmm_glu(x, w1, v1, batch_sizes, act, keep_product=keep)
         ctx.act = act
         combine = None if c_indices is None else gg.CombinedRows(c_indices, c_bin_ids, c_bins, c_weights)
         out, kept = second_product(activation_fn_out, w2, batch_sizes, combine, ctx.needs_input_grad[9])
-        ctx.save_for_backward(x, w1, v1, w2, batch_sizes, sdd_out, v1_out, activation_fn_out, *kept)
+        if keep:
+            ctx.save_for_backward(x, w1, v1, w2, batch_sizes, sdd_out, v1_out, activation_fn_out, *kept)
         return out
 
     @staticmethod
@@ -131,7 +133,7 @@ class GroupedGLUExperts(torch.autograd.Function):
         x, w1, v1, w2, batch_sizes, sdd_out, v1_out, activation_fn_out, *kept = ctx.saved_tensors
         ddsd_out, dweights = second_product_grad(kept, grad, ctx.needs_input_grad[9])
         return (*_glu_experts_backward(ctx.needs_input_grad, x, w1, v1, w2, batch_sizes, sdd_out, v1_out,
-                                       activation_fn_out, ddsd_out, ctx.act), None, None, None, None, None, dweights)
+                                       activation_fn_out, ddsd_out, ctx.act), None, None, None, None, None, dweights, None)
 
 
 def _glu_experts_backward(needs, x, w1, v1, w2, batch_sizes, sdd_out, v1_out, activation_fn_out, ddsd_out, act):
@@ -164,19 +166,21 @@ class GatheredGLUExperts(torch.autograd.Function):
     @staticmethod
     @torch.amp.custom_fwd(device_type='cuda')
     def forward(ctx, x, w1, v1, w2, batch_sizes, act, indices, bin_ids, bins, padded_bins, top_k, rows, combined=False,
-                c_weights=None):
+                c_weights=None, keep=True):
+        # keep False: no gradient is recorded, the first products themselves need not be written
         # combined: the node returns the layer's combine of its output (top_k = 1; the same assignments, c_weights)
         x = x.contiguous()
         src = gg.GatheredRows(x, indices, bin_ids, bins, padded_bins, top_k, rows)
-        out = gg.gmm_gather(src, w1, batch_sizes, b2=v1, act=act)
+        out = gg.gmm_gather(src, w1, batch_sizes, b2=v1, act=act, keep_product=keep)
         if out is None:
-            out = gg.gmm_glu(src.materialize(), w1, v1, batch_sizes, act)
+            out = gg.gmm_glu(src.materialize(), w1, v1, batch_sizes, act, keep_product=keep)
         sdd_out, v1_out, activation_fn_out = out
         ctx.act, ctx.top_k, ctx.rows = act, top_k, rows
         combine = gg.CombinedRows(indices, bin_ids, bins, c_weights) if combined else None
         out, kept = second_product(activation_fn_out, w2, batch_sizes, combine, ctx.needs_input_grad[13])
-        ctx.save_for_backward(x, w1, v1, w2, batch_sizes, sdd_out, v1_out, activation_fn_out, indices, bin_ids, bins,
-                              padded_bins, *kept)
+        if keep:
+            ctx.save_for_backward(x, w1, v1, w2, batch_sizes, sdd_out, v1_out, activation_fn_out, indices, bin_ids, bins,
+                                  padded_bins, *kept)
         return out
 
     @staticmethod
@@ -190,7 +194,7 @@ class GatheredGLUExperts(torch.autograd.Function):
                                                   v1_out, activation_fn_out, ddsd_out, ctx.act)
         if dx is not None:
             dx = src.scatter_grad(dx)
-        return dx, dw1, dv1, dw2, None, None, None, None, None, None, None, None, None, dweights
+        return dx, dw1, dv1, dw2, None, None, None, None, None, None, None, None, None, dweights, None
 
 
 def _one_node(x, w1, v1, w2, act):
@@ -289,7 +293,7 @@ class SparseGLU(SparseMLP):
         operands = gg.autocast_operands(x, w1, v1, w2)
         if _one_node(*operands, act):
             c = (None, None, None, None) if combine is None else (combine.indices, combine.bin_ids, combine.bins, combine.weights)
-            return GroupedGLUExperts.apply(*operands, batch_sizes, act, *c)
+            return GroupedGLUExperts.apply(*operands, batch_sizes, act, *c, torch.is_grad_enabled())
         x1, x2 = GLUProjection.apply(*operands[:3], batch_sizes)
         x1 = gated_activation(self.args.activation_fn, x1, x2)
         return self._combined(gg.ops.gmm(x1, w2, batch_sizes), combine)
@@ -312,7 +316,7 @@ class SparseGLU(SparseMLP):
             return None
         return GatheredGLUExperts.apply(x, w1, v1, w2, batch_sizes, act, src.indices, src.bin_ids, src.bins,
                                         src.padded_bins, src.top_k, src.rows, combine is not None,
-                                        None if combine is None else combine.weights)
+                                        None if combine is None else combine.weights, torch.is_grad_enabled())
 
 
 class GroupedGLU(SparseGLU):

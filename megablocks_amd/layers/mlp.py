@@ -173,15 +173,17 @@ class GroupedGeluMLP(torch.autograd.Function):
 
     @staticmethod
     @torch.amp.custom_fwd(device_type='cuda')
-    def forward(ctx, x, w1, w2, batch_sizes, c_indices=None, c_bin_ids=None, c_bins=None, c_weights=None):
+    def forward(ctx, x, w1, w2, batch_sizes, c_indices=None, c_bin_ids=None, c_bins=None, c_weights=None, keep=True):
         # c_*: the layer's combine (`gg.CombinedRows`), when the node is to return the combined output
+        # keep False: no gradient is recorded, the first product itself need not be written
         if ctx._fwd_used_autocast:
             x, w1, w2 = x.to(ctx._dtype), w1.to(ctx._dtype), w2.to(ctx._dtype)
         x, w1, w2 = x.contiguous(), w1.contiguous(), w2.contiguous()
-        sdd_out, activation_fn_out = gg.gmm_act(x, w1, batch_sizes)
+        sdd_out, activation_fn_out = gg.gmm_act(x, w1, batch_sizes, keep_product=keep)
         combine = None if c_indices is None else gg.CombinedRows(c_indices, c_bin_ids, c_bins, c_weights)
         out, kept = second_product(activation_fn_out, w2, batch_sizes, combine, ctx.needs_input_grad[7])
-        ctx.save_for_backward(w1, w2, batch_sizes, x, sdd_out, activation_fn_out, *kept)
+        if keep:
+            ctx.save_for_backward(w1, w2, batch_sizes, x, sdd_out, activation_fn_out, *kept)
         return out
 
     @staticmethod
@@ -190,7 +192,7 @@ class GroupedGeluMLP(torch.autograd.Function):
         w1, w2, batch_sizes, x, sdd_out, activation_fn_out, *kept = ctx.saved_tensors
         ddsd_out, dweights = second_product_grad(kept, grad, ctx.needs_input_grad[7])
         return (*_gelu_mlp_backward(ctx.needs_input_grad, x, w1, w2, batch_sizes, sdd_out, activation_fn_out, ddsd_out),
-                None, None, None, None, dweights)
+                None, None, None, None, dweights, None)
 
 
 def _gelu_mlp_backward(needs, x, w1, w2, batch_sizes, sdd_out, activation_fn_out, ddsd_out):
@@ -253,21 +255,23 @@ class GatheredGeluMLP(torch.autograd.Function):
     @staticmethod
     @torch.amp.custom_fwd(device_type='cuda')
     def forward(ctx, x, w1, w2, batch_sizes, indices, bin_ids, bins, padded_bins, top_k, rows, combined=False,
-                c_weights=None):
+                c_weights=None, keep=True):
         # combined: the node returns the layer's combine of its output (top_k = 1; the same assignments, c_weights)
+        # keep False: no gradient is recorded, the first product itself need not be written
         if ctx._fwd_used_autocast:
             x, w1, w2 = x.to(ctx._dtype), w1.to(ctx._dtype), w2.to(ctx._dtype)
         x, w1, w2 = x.contiguous(), w1.contiguous(), w2.contiguous()
         src = gg.GatheredRows(x, indices, bin_ids, bins, padded_bins, top_k, rows)
-        out = gg.gmm_gather(src, w1, batch_sizes, act=gg.ACT_GELU_TANH)
+        out = gg.gmm_gather(src, w1, batch_sizes, act=gg.ACT_GELU_TANH, keep_product=keep)
         if out is None:
-            out = gg.gmm_act(src.materialize(), w1, batch_sizes)
+            out = gg.gmm_act(src.materialize(), w1, batch_sizes, keep_product=keep)
         sdd_out, activation_fn_out = out
         ctx.top_k, ctx.rows = top_k, rows
         combine = gg.CombinedRows(indices, bin_ids, bins, c_weights) if combined else None
         out, kept = second_product(activation_fn_out, w2, batch_sizes, combine, ctx.needs_input_grad[11])
-        ctx.save_for_backward(w1, w2, batch_sizes, x, sdd_out, activation_fn_out, indices, bin_ids, bins, padded_bins,
-                              *kept)
+        if keep:
+            ctx.save_for_backward(w1, w2, batch_sizes, x, sdd_out, activation_fn_out, indices, bin_ids, bins, padded_bins,
+                                  *kept)
         return out
 
     @staticmethod
@@ -280,13 +284,13 @@ class GatheredGeluMLP(torch.autograd.Function):
                                           activation_fn_out, ddsd_out)
         if dx is not None:
             dx = src.scatter_grad(dx)
-        return dx, dw1, dw2, None, None, None, None, None, None, None, None, dweights
+        return dx, dw1, dw2, None, None, None, None, None, None, None, None, dweights, None
 
 
 def grouped_gelu_mlp(x, w1, w2, batch_sizes, combine=None):
     """GroupedGeluMLP; with `combine` (a `gg.CombinedRows`) the node returns the layer's combine of its output."""
     c = (None, None, None, None) if combine is None else (combine.indices, combine.bin_ids, combine.bins, combine.weights)
-    return GroupedGeluMLP.apply(x, w1, w2, batch_sizes, *c)
+    return GroupedGeluMLP.apply(x, w1, w2, batch_sizes, *c, torch.is_grad_enabled())
 
 
 class MemoryOptimizedGroupedMLP(torch.autograd.Function):
@@ -416,7 +420,8 @@ class SparseMLP(torch.nn.Module):
             return None   # the memory-optimised schedule is a matter of what the backward keeps: without one, the same forward
         w1, w2 = self._expert_views(self.w1, self.w2)
         return GatheredGeluMLP.apply(src.x, w1, w2, batch_sizes, src.indices, src.bin_ids, src.bins, src.padded_bins,
-                                     src.top_k, src.rows, combine is not None, None if combine is None else combine.weights)
+                                     src.top_k, src.rows, combine is not None, None if combine is None else combine.weights,
+                                     torch.is_grad_enabled())
 
 
 class GroupedMLP(SparseMLP):

@@ -1141,6 +1141,41 @@ def test_batched_mlp_with_activation_epilogues(gg, groups, rows, k, n, dtype):
     assert torch.equal(w.grad, results[0][3])
 
 
+@pytest.mark.parametrize('groups,tokens,top_k,k,n', [(1, 1, 1, 64, 8), (4, 30, 2, 128, 264), (3, 130, 1, 72, 256), (8, 700, 2, 64, 1032),
+                                                     (5, 2000, 3, 128, 136), (2, 900, 2, 192, 512)])
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])
+def test_first_products_that_write_only_their_activation(gg, groups, tokens, top_k, k, n, dtype):
+    """Without gradients the launches leave the products themselves out: the activation bit for bit, for every form."""
+    torch.manual_seed(tokens)
+    rows = tokens * top_k
+    sizes = _sizes(groups, rows, seed=rows, empty=(0,) if groups > 2 else ()).cuda()
+    x = torch.randn(tokens, k, device='cuda').to(dtype)
+    b1, b2 = ((torch.randn(groups, n, k, device='cuda') / k ** 0.5).to(dtype) for _ in range(2))
+    order = torch.randperm(rows, device='cuda').int()
+    bins = torch.cumsum(sizes, 0).int()
+    bin_ids = torch.repeat_interleave(torch.arange(groups, device='cuda'), sizes.long()).int()
+    padded_sizes = ((sizes + 127) // 128 * 128).int()
+    padded = torch.cumsum(padded_sizes, 0).int()
+    for src, group_sizes in ((gg.GatheredRows(x, order, bin_ids, bins, None, top_k, rows), sizes),
+                             (gg.GatheredRows(x, order, bin_ids, bins, padded, top_k, int(padded[-1])), padded_sizes)):
+        a = src.materialize()
+        pre, act = gg.gmm_act(a, b1, group_sizes, fuse=True)
+        none, only = gg.gmm_act(a, b1, group_sizes, fuse=True, keep_product=False)
+        assert none is None and torch.equal(only, act)
+        both = gg.gmm_gather(src, b1, group_sizes, act=gg.ACT_GELU_TANH, keep_product=False)
+        assert (both is None) == (k % 64 != 0)
+        assert both is None or (both[0] is None and torch.equal(both[1], act))
+        for code in (0, 1):
+            h = gg.gmm_glu(a, b1, b2, group_sizes, code, fuse=True)[2]
+            none, none2, only = gg.gmm_glu(a, b1, b2, group_sizes, code, fuse=True, keep_product=False)
+            assert none is None and none2 is None and torch.equal(only, h)
+            got = gg.gmm_gather(src, b1, group_sizes, b2=b2, act=code, keep_product=False)
+            assert got is None if k % 64 else torch.equal(got[2], h)
+    # fp32: no such launch, the products come back
+    pre, act = gg.gmm_act(x.float(), b1.float(), _sizes(groups, tokens, seed=1).cuda(), keep_product=False)
+    assert pre.shape == act.shape
+
+
 @pytest.mark.parametrize('groups,rows,k,n,skew', [(1, 1, 8, 8, False), (1, 1024, 128, 136, False), (3, 0, 64, 128, False),
                                                   (4, 257, 136, 120, False), (8, 8 * 63, 264, 1032, True), (64, 64 * 130, 256, 384, True),
                                                   (70, 70 * 40, 72, 264, True), (130, 900, 128, 2056, False),
