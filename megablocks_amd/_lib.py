@@ -61,8 +61,8 @@ _SIGNATURES = {
     'mbx_glu_forward': (_i, [_vp, _vp, _vp, _i, _i, _i64, _vp]),
     'mbx_glu_backward': (_i, [_vp, _vp, _vp, _vp, _vp, _i, _i, _i64, _vp]),
     'mbx_router_forward': (_i, [_vp, _i, _i64, _i, _i, ctypes.c_float, _vp, _vp, _vp, _vp, _vp, _vp]),
-    'mbx_router_backward': (_i, [_vp, _vp, _vp, _vp, _i, _i64, _i, _i, ctypes.c_float, _vp, _vp, _vp]),
     'mbx_router_linear_forward': (_i, [_vp, _vp, _i, _i64, _i, _i, _i, ctypes.c_float, _vp, _vp, _vp, _vp, _vp]),
+    'mbx_router_backward': (_i, [_vp, _vp, _vp, _vp, _i, _i64, _i, _i, ctypes.c_float, _vp, _vp, _vp]),
 }
 
 
@@ -88,40 +88,62 @@ def check(code: int, what: str = 'mbx'):
 
 
 def ptr(t):
-    """Device address of a tensor (None -> NULL)."""
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    """Device address of a tensor (None -> NULL), as the ABI's pointer arguments take it: a plain integer (a c_void_p object
+    each costs three times as much, and a layer step passes hundreds)."""
+    return None if t is None else t.data_ptr()
 
 
 _raw_stream = getattr(torch._C, '_cuda_getCurrentRawStream', None)
+# torch.cuda.current_device() without its check for an initialised runtime: whoever launches holds a tensor on the GPU
+_current_device = getattr(torch._C, '_cuda_getDevice', torch.cuda.current_device)
 
 
 def stream():
     """The current stream of the current device as the ABI takes it.  Called once per launch: the raw handle
     straight from the binding where torch has one (several times cheaper than building a Stream object)."""
     if _raw_stream is not None:
-        return ctypes.c_void_p(_raw_stream(torch.cuda.current_device()))
+        return ctypes.c_void_p(_raw_stream(_current_device()))
     return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
 
 
-class device_of:
-    """`with device_of(tensor):` makes the tensor's device current for the launch (and restores the previous one);
-    nothing to do, and nearly free, when it already is."""
-    __slots__ = ('idx', 'prev')
-
-    def __init__(self, t):
-        self.idx, self.prev = t.device.index, -1
+class _Nothing:
+    """The context of a launch that needs none."""
+    __slots__ = ()
 
     def __enter__(self):
-        cur = torch.cuda.current_device()
-        if self.idx is not None and cur != self.idx:
-            self.prev = cur
-            torch.cuda.set_device(self.idx)
         return self
 
     def __exit__(self, *exc):
-        if self.prev >= 0:
-            torch.cuda.set_device(self.prev)
         return False
+
+    def cancel(self):
+        pass
+
+
+_NOTHING = _Nothing()
+
+
+class _Device:
+    __slots__ = ('idx', 'prev')
+
+    def __init__(self, idx):
+        self.idx = idx
+
+    def __enter__(self):
+        self.prev = _current_device()
+        torch.cuda.set_device(self.idx)
+        return self
+
+    def __exit__(self, *exc):
+        torch.cuda.set_device(self.prev)
+        return False
+
+
+def device_of(t):
+    """`with device_of(tensor):` makes the tensor's device current for the launch (and restores the previous one);
+    nothing to do, and nearly free, when it already is."""
+    idx = t.get_device()
+    return _NOTHING if idx < 0 or idx == _current_device() else _Device(idx)
 
 
 def autocast_gpu_dtype():
@@ -162,17 +184,15 @@ def as_i32(t):
 profile_hook = None
 
 
-class record:
-    """`with record('gmm_nt', rows=..., k=..., n=...):` around a launch."""
+class _Record:
     __slots__ = ('name', 'meta', 'ev0')
 
-    def __init__(self, name, **meta):
-        self.name, self.meta, self.ev0 = name, meta, None
+    def __init__(self, name, meta):
+        self.name, self.meta = name, meta
 
     def __enter__(self):
-        if profile_hook is not None:
-            self.ev0 = torch.cuda.Event(enable_timing=True)
-            self.ev0.record()
+        self.ev0 = torch.cuda.Event(enable_timing=True)
+        self.ev0.record()
         return self
 
     def cancel(self):
@@ -180,8 +200,13 @@ class record:
         self.ev0 = None
 
     def __exit__(self, *exc):
-        if self.ev0 is not None:
+        if self.ev0 is not None and profile_hook is not None:
             ev1 = torch.cuda.Event(enable_timing=True)
             ev1.record()
             profile_hook.append((self.name, self.meta, self.ev0, ev1))
         return False
+
+
+def record(name, **meta):
+    """`with record('gmm_nt', rows=..., k=..., n=...):` around a launch."""
+    return _NOTHING if profile_hook is None else _Record(name, meta)
