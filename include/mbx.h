@@ -329,6 +329,15 @@ int mbx_gmm_tn_gather(const void* a, const void* x, int64_t x_rows, const int32_
                       void* c, int dtype, const int32_t* bins, int num_groups, int64_t rows, int k, int n, void* row_table,
                       size_t row_table_bytes, int table_ready, mbx_stream_t stream);
 
+/* A weight gradient in fp32, for fp32 master weights under autocast: c[e] = a[r_e]^T @ b[r_e] (indices NULL; x_rows, top_k, x_bins
+ * and the table are ignored) or mbx_gmm_tn_gather's product (b = x), 16-bit operands, the fp32 sums stored as they are, where
+ * the reference's autograd casts a rounded product back.  MBX_EUNSUPPORTED (the caller multiplies in 16 bits and casts): fp32
+ * operands, k or n not multiples of 8, buffers not 16-byte aligned, an operand of 2 GiB or more; gathered: what
+ * mbx_gmm_tn_gather does not take. */
+int mbx_gmm_tn_f32(const void* a, const void* b, int64_t x_rows, const int32_t* indices, int top_k, const int32_t* x_bins, float* c,
+                   int dtype, const int32_t* bins, int num_groups, int64_t rows, int k, int n, void* row_table,
+                   size_t row_table_bytes, int table_ready, mbx_stream_t stream);
+
 /* The backward of the GLU experts' gated activation on the product that feeds it, megablocks/layers/glu.py:135-153
  * (`gmm(ddsd_out, w2, trans_b=True, c=dactivation_fn_out)`, then autograd's gradient of
  * `activation_fn(sdd_out) * v1_out`, glu.py:120-124), in one launch:

@@ -514,7 +514,9 @@ int launch_tn(const DmaCall& call) {
   const bool segmented = rows > seg_rows;
   // the last row tile of the product as a TS tile when it is at most half full
   const bool mixed = T::BM != TS::BM && k % T::BM != 0 && k % T::BM <= TS::BM;
-  auto kern = mixed ? (segmented ? dma::gmm_tn_kernel<DT, T, TS, true> : dma::gmm_tn_kernel<DT, T, TS, false>)
+  if (call.out32 && segmented) return MBX_EUNSUPPORTED;
+  auto kern = call.out32 ? (mixed ? dma::gmm_tn_kernel<DT, T, TS, false, false, true> : dma::gmm_tn_kernel<DT, T, T, false, false, true>)
+              : mixed ? (segmented ? dma::gmm_tn_kernel<DT, T, TS, true> : dma::gmm_tn_kernel<DT, T, TS, false>)
                     : (segmented ? dma::gmm_tn_kernel<DT, T, T, true> : dma::gmm_tn_kernel<DT, T, T, false>);
   int rc = allow_lds(kern, lds);
   if (rc) return rc;
@@ -536,7 +538,7 @@ int launch_tn(const DmaCall& call) {
     if (segmented || !std::is_same<T, TS>::value) return MBX_EUNSUPPORTED;
     if (!gather.table_ready) dma::build_row_table(call);
     if constexpr (T::BM == 256 && T::SB == 2) {
-      auto gkern = dma::gmm_tn_kernel<DT, T, T, false, true>;
+      auto gkern = call.out32 ? dma::gmm_tn_kernel<DT, T, T, false, true, true> : dma::gmm_tn_kernel<DT, T, T, false, true>;
       int grc = allow_lds(gkern, lds);
       if (grc) return grc;
       gkern<<<(unsigned)grid, T::THREADS, lds, s>>>(ap, bp, cp, bins, num_groups, (int)rows, k, n, tiles_m, tiles_n, shape.bm, shape.bn, chunk, (int)seg_rows, whole_ok, gather.row_table, gather.src_bins, gather.src_rows, (int)gather.n_slots);
@@ -820,9 +822,9 @@ size_t mbx_gmm_tn_gather_table_bytes(int64_t x_rows, int top_k, int num_groups) 
   return (size_t)dma::row_table_entries(x_rows * top_k, num_groups) * 4;
 }
 
-int mbx_gmm_tn_gather(const void* a, const void* x, int64_t x_rows, const int32_t* indices, int top_k, const int32_t* x_bins,
-                      void* c, int dtype, const int32_t* bins, int num_groups, int64_t rows, int k, int n, void* row_table,
-                      size_t row_table_bytes, int table_ready, mbx_stream_t stream) {
+static int gmm_tn_gather(const void* a, const void* x, int64_t x_rows, const int32_t* indices, int top_k, const int32_t* x_bins,
+                         void* c, int dtype, const int32_t* bins, int num_groups, int64_t rows, int k, int n, void* row_table,
+                         size_t row_table_bytes, int table_ready, mbx_stream_t stream, bool out32) {
   if (x_rows < 0 || top_k <= 0 || k < 0 || n < 0 || num_groups < 0 || rows < 0) return MBX_EINVAL;
   if (dtype != MBX_BF16 && dtype != MBX_F16 && dtype != MBX_F32) return MBX_EINVAL;
   if (num_groups == 0 || (int64_t)k * n == 0) return 0;
@@ -846,6 +848,28 @@ int mbx_gmm_tn_gather(const void* a, const void* x, int64_t x_rows, const int32_
   gather.table_ready = table_ready != 0;
   DmaCall call{a, x, c, dtype, bins, num_groups, rows, k, n, MBX_TN, as_stream(stream)};
   call.gather = gather;
+  call.out32 = out32;
+  return gmm_dma(call);
+}
+
+int mbx_gmm_tn_gather(const void* a, const void* x, int64_t x_rows, const int32_t* indices, int top_k, const int32_t* x_bins,
+                      void* c, int dtype, const int32_t* bins, int num_groups, int64_t rows, int k, int n, void* row_table,
+                      size_t row_table_bytes, int table_ready, mbx_stream_t stream) {
+  return gmm_tn_gather(a, x, x_rows, indices, top_k, x_bins, c, dtype, bins, num_groups, rows, k, n, row_table, row_table_bytes, table_ready, stream, false);
+}
+
+int mbx_gmm_tn_f32(const void* a, const void* b, int64_t x_rows, const int32_t* indices, int top_k, const int32_t* x_bins, float* c,
+                   int dtype, const int32_t* bins, int num_groups, int64_t rows, int k, int n, void* row_table,
+                   size_t row_table_bytes, int table_ready, mbx_stream_t stream) {
+  if (indices) return gmm_tn_gather(a, b, x_rows, indices, top_k, x_bins, c, dtype, bins, num_groups, rows, k, n, row_table, row_table_bytes, table_ready, stream, true);
+  if (num_groups < 0 || rows < 0 || k < 0 || n < 0) return MBX_EINVAL;
+  if (dtype != MBX_BF16 && dtype != MBX_F16 && dtype != MBX_F32) return MBX_EINVAL;
+  if (num_groups == 0 || (int64_t)k * n == 0) return 0;
+  if (!c || !bins || (rows > 0 && (!a || !b))) return MBX_EINVAL;
+  if (rows > 0x7fffffff) return MBX_ERANGE;
+  if (dtype == MBX_F32 || !aligned16(a) || !aligned16(b) || !aligned16(c) || k % 8 || n % 8 || !dma_sizes_ok(k, n)) return MBX_EUNSUPPORTED;
+  DmaCall call{a, b, c, dtype, bins, num_groups, rows, k, n, MBX_TN, as_stream(stream)};
+  call.out32 = true;
   return gmm_dma(call);
 }
 

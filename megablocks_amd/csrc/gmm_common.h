@@ -55,6 +55,7 @@ struct DmaCall {
   GatherRows gather{};
   Workspace ws{};
   CombineRows combine{};
+  bool out32 = false;   // TN: c is fp32
 };
 
 // NN / NT launches with a handful of rows per expert (gmm_few.hip), and whether a launch is one of them.

@@ -1111,6 +1111,23 @@ __device__ __forceinline__ void block_store(const typename T::Acc (&acc)[T::TM][
   }
 }
 
+// The tile's accumulators to an fp32 matrix (n_lim a multiple of 4, c 16-byte aligned rows), straight from the registers: a
+// lane owns runs of four columns, and two stores fill the 128 bytes of a row they share.
+template <typename T>
+__device__ __forceinline__ void block_store_f32(const typename T::Acc (&acc)[T::TM][T::TN], float* __restrict__ c, int64_t ldc,
+                                                int m_base, int m_lim, int n_base, int n_lim) {
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = lane_id();
+  const int m0 = m_base + (wave / T::WN) * T::WTM + (lane & 15), n0 = n_base + (wave % T::WN) * T::WTN + (lane >> 4) * 4;
+#pragma unroll
+  for (int i = 0; i < T::TM; ++i) {
+    if (m0 + i * T::MF >= m_lim) continue;
+    float* const row = c + (int64_t)(m0 + i * T::MF) * ldc + n0;
+#pragma unroll
+    for (int j = 0; j < T::TN; ++j)
+      if (n0 + j * T::MF < n_lim) *(f32x4*)(row + j * T::MF) = acc[i][j];
+  }
+}
+
 // c = A_tile * B_tile over all K tiles (the whole product of one output tile)
 template <int DT, bool A_MC, bool B_MC, typename T, bool DUAL = false, int EPI = kEpiNone, bool GATHER = false, bool KTAIL = false>
 __device__ __forceinline__ void block_gemm(const Args& g, uint16_t* __restrict__ c, int64_t ldc, int m_base, int m_lim,
@@ -1705,11 +1722,12 @@ static inline int64_t tn_grid(int tiles_m, int tiles_n, TnBlocks shape, int num_
 // c[e] = a[start:end]^T @ b[start:end].
 // GATHER: b is the matrix the rows are picked from (its buffer, g.rsrc_b, and the row table, g.row_table /
 // g.gather_row / g.gather_row2, are the caller's business).
-template <int DT, typename TT, bool SEGMENTED, bool GATHER = false>
+// OUT32: c is fp32.
+template <int DT, typename TT, bool SEGMENTED, bool GATHER = false, bool OUT32 = false>
 __device__ __forceinline__ void tn_tile(Args& g, const uint16_t* __restrict__ a, const uint16_t* __restrict__ b,
                                         uint16_t* __restrict__ c_e, int start, int end, int k, int n, int seg_rows,
                                         char* lds) {
-  static_assert(!(GATHER && SEGMENTED), "gathered rows: one segment");
+  static_assert(!((GATHER || OUT32) && SEGMENTED), "gathered rows, fp32 products: one segment");
   if constexpr (!SEGMENTED) {
     // the buffers cover exactly the rows of this expert: later rows read as zero
     const int64_t group_rows = end - start;
@@ -1719,7 +1737,8 @@ __device__ __forceinline__ void tn_tile(Args& g, const uint16_t* __restrict__ a,
     typename TT::Acc acc[TT::TM][TT::TN];
     block_multiply<DT, true, true, TT, false, false, false, GATHER>(g, acc, true, lds);
     MBX_TICK(g.tick_ordinal, 2);
-    block_store<DT, TT>(acc, c_e, n, g.a_r0, k, g.b_r0, n, lds);
+    if constexpr (OUT32) block_store_f32<TT>(acc, (float*)c_e, n, g.a_r0, k, g.b_r0, n);
+    else block_store<DT, TT>(acc, c_e, n, g.a_r0, k, g.b_r0, n, lds);
     MBX_TICK(g.tick_ordinal, 4);
   } else {
     // The reduction runs over the expert's rows in segments of at most seg_rows rows, each with buffers
@@ -1752,7 +1771,8 @@ __device__ __forceinline__ void tn_tile(Args& g, const uint16_t* __restrict__ a,
 // glu.py:128-166: `gmm(dsdd_out, x, batch_sizes, trans_a=True)` with x the gathered tokens).  row_table: one entry per
 // sorted assignment, the byte offset of its row in b with bit 31 flipped (gather_row_table_kernel); src_bins: the
 // inclusive bins of the sorted assignments (`bins` are the row bins of a, which may be padded per expert).
-template <int DT, typename T, typename TS, bool SEGMENTED, bool GATHER = false>
+// OUT32: c is fp32 (the products' sums as they are, for fp32 master weights).
+template <int DT, typename T, typename TS, bool SEGMENTED, bool GATHER = false, bool OUT32 = false>
 __global__ void __launch_bounds__(T::THREADS)
 gmm_tn_kernel(const uint16_t* __restrict__ a, const uint16_t* __restrict__ b, uint16_t* __restrict__ c,
               const int32_t* __restrict__ bins, int num_groups, int rows, int k, int n, int tiles_m, int tiles_n,
@@ -1855,11 +1875,11 @@ gmm_tn_kernel(const uint16_t* __restrict__ a, const uint16_t* __restrict__ b, ui
       MBX_TICK(g.tick_ordinal, 0);
       g.a_r0 = cur.tm * T::BM;
       g.b_r0 = cur.tn * T::BN;
-      uint16_t* const c_e = c + (int64_t)cur.e * k * n;
+      uint16_t* const c_e = c + (int64_t)cur.e * k * n * (OUT32 ? 2 : 1);
       if (kMixed && k - g.a_r0 <= TS::BM) {
-        tn_tile<DT, TS, SEGMENTED>(g, a, b, c_e, cur.start, cur.end, k, n, seg_rows, lds);
+        tn_tile<DT, TS, SEGMENTED, false, OUT32>(g, a, b, c_e, cur.start, cur.end, k, n, seg_rows, lds);
       } else {
-        tn_tile<DT, T, SEGMENTED>(g, a, b, c_e, cur.start, cur.end, k, n, seg_rows, lds);
+        tn_tile<DT, T, SEGMENTED, false, OUT32>(g, a, b, c_e, cur.start, cur.end, k, n, seg_rows, lds);
       }
       tile_done();
       MBX_TICK(g.tick_ordinal, 5);
@@ -1918,7 +1938,7 @@ gmm_tn_kernel(const uint16_t* __restrict__ a, const uint16_t* __restrict__ b, ui
       MBX_TICK(g.tick_ordinal, 0);
       g.a_r0 = cur.tm * T::BM;
       g.b_r0 = cur.tn * T::BN;
-      tn_tile<DT, T, false, true>(g, a, b, c + (int64_t)cur.e * k * n, cur.start, cur.end, k, n, seg_rows, lds);
+      tn_tile<DT, T, false, true, OUT32>(g, a, b, c + (int64_t)cur.e * k * n * (OUT32 ? 2 : 1), cur.start, cur.end, k, n, seg_rows, lds);
       arrived = g.nk > 0;
       tile_done();
       MBX_TICK(g.tick_ordinal, 5);

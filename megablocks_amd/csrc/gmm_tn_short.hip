@@ -44,8 +44,8 @@ __device__ __forceinline__ f32x4 mfma(const u32x4& a, const u32x4& b, const f32x
   return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, a), __builtin_bit_cast(f16x8_t, b), c, 0, 0, 0);
 }
 
-// GATHER: the rows of b are picked through gmm_dma.h's row table (there: gmm_tn_kernel).
-template <int DT, bool GATHER>
+// OUT32: c is fp32.  GATHER: the rows of b are picked through gmm_dma.h's row table (there: gmm_tn_kernel).
+template <int DT, bool GATHER, bool OUT32>
 __global__ void __launch_bounds__(T::THREADS, kPerCu)
 gmm_tn_short_kernel(const uint16_t* __restrict__ a, const uint16_t* __restrict__ b, uint16_t* __restrict__ c,
                     const int32_t* __restrict__ bins, int num_groups, int rows, int k, int n, int tiles_m, int tiles_n,
@@ -190,10 +190,11 @@ gmm_tn_short_kernel(const uint16_t* __restrict__ a, const uint16_t* __restrict__
     multiply();
   }
   dma::wait_vmcnt<0>();
-  dma::block_store<DT, T>(acc, c + (int64_t)e * k * n, n, tm * T::BM, k, tn * T::BN, n, lds_generic);
+  if constexpr (OUT32) dma::block_store_f32<T>(acc, (float*)c + (int64_t)e * k * n, n, tm * T::BM, k, tn * T::BN, n);
+  else dma::block_store<DT, T>(acc, c + (int64_t)e * k * n, n, tm * T::BM, k, tn * T::BN, n, lds_generic);
 }
 
-template <int DT>
+template <int DT, bool OUT32>
 int launch(const DmaCall& q) {
   const int tiles_m = (int)ceil_div(q.k, T::BM), tiles_n = (int)ceil_div(q.n, T::BN);
   const int64_t grid = ceil_div((int64_t)tiles_m * tiles_n, kXcds) * q.num_groups * kXcds;
@@ -202,9 +203,9 @@ int launch(const DmaCall& q) {
   if (q.gather.slots) {
     if (!q.gather.src_bins || !q.gather.row_table || q.gather.top_k <= 0 || q.gather.n_slots > 0x7fffffff) return MBX_EINVAL;
     if (!q.gather.table_ready) dma::build_row_table(q);
-    gmm_tn_short_kernel<DT, true><<<(unsigned)grid, T::THREADS, kLdsBytes, q.stream>>>(a, b, (uint16_t*)q.c, q.bins, q.num_groups, (int)q.rows, q.k, q.n, tiles_m, tiles_n, q.gather.row_table, q.gather.src_bins, q.gather.src_rows, (int)q.gather.n_slots);
+    gmm_tn_short_kernel<DT, true, OUT32><<<(unsigned)grid, T::THREADS, kLdsBytes, q.stream>>>(a, b, (uint16_t*)q.c, q.bins, q.num_groups, (int)q.rows, q.k, q.n, tiles_m, tiles_n, q.gather.row_table, q.gather.src_bins, q.gather.src_rows, (int)q.gather.n_slots);
   } else {
-    gmm_tn_short_kernel<DT, false><<<(unsigned)grid, T::THREADS, kLdsBytes, q.stream>>>(a, b, (uint16_t*)q.c, q.bins, q.num_groups, (int)q.rows, q.k, q.n, tiles_m, tiles_n, nullptr, nullptr, 0, 0);
+    gmm_tn_short_kernel<DT, false, OUT32><<<(unsigned)grid, T::THREADS, kLdsBytes, q.stream>>>(a, b, (uint16_t*)q.c, q.bins, q.num_groups, (int)q.rows, q.k, q.n, tiles_m, tiles_n, nullptr, nullptr, 0, 0);
   }
   return launch_status();
 }
@@ -223,6 +224,9 @@ bool gmm_tn_short_takes(const DmaCall& q) {
   return q.rows <= (int64_t)(tiles <= at_once ? 1024 : 256) * q.num_groups;
 }
 
-int gmm_tn_short(const DmaCall& q) { return q.dtype == MBX_BF16 ? tn_short::launch<MBX_BF16>(q) : tn_short::launch<MBX_F16>(q); }
+int gmm_tn_short(const DmaCall& q) {
+  if (q.out32) return q.dtype == MBX_BF16 ? tn_short::launch<MBX_BF16, true>(q) : tn_short::launch<MBX_F16, true>(q);
+  return q.dtype == MBX_BF16 ? tn_short::launch<MBX_BF16, false>(q) : tn_short::launch<MBX_F16, false>(q);
+}
 
 }  // namespace mbx

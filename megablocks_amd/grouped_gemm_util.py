@@ -357,15 +357,18 @@ class GatheredRows:
             return kernels.gather(self.x, self.indices, self.bin_ids, None, self.bins, self.top_k)
         return kernels.padded_gather(self.x, self.indices, self.bin_ids, None, self.bins, self.padded_bins, self.top_k)
 
-    def weight_gradient(self, d, batch_sizes):
+    def weight_gradient(self, d, batch_sizes, weight_dtype=None):
         """gmm(d, self.materialize(), batch_sizes, trans_a=True): the weight gradient of a product whose operand these
         rows were (mlp.py:485-491, glu.py:154-159), read from the ungathered tokens where the library has a kernel for
-        the shapes (`gmm_tn_gather`), else from the copy, which is then made once and kept for the next call."""
-        out = gmm_tn_gather(d, self, batch_sizes)
+        the shapes (`gmm_tn_gather`), else from the copy, which is then made once and kept for the next call.
+        weight_dtype: as for `weight_gradient`."""
+        out = gmm_tn_gather(d, self, batch_sizes, fp32_out=True) if _wants_fp32(d, weight_dtype) else None
+        if out is None:
+            out = gmm_tn_gather(d, self, batch_sizes)
         if out is None:
             if getattr(self, '_copy', None) is None:
                 self._copy = self.materialize()
-            out = gmm(d, self._copy, batch_sizes, trans_a=True)
+            out = weight_gradient(d, self._copy, batch_sizes, weight_dtype)
         return out
 
     def scatter_grad(self, grad):
@@ -424,11 +427,39 @@ def gmm_gather(src: GatheredRows, b1, batch_sizes, b2=None, act=None, keep_produ
     return (c,) if act is None else (c, h) if b2 is None else (c, c2, h)
 
 
-def gmm_tn_gather(a, src: GatheredRows, batch_sizes, c=None):
+def _wants_fp32(a, weight_dtype):
+    return weight_dtype == torch.float32 and a.is_cuda and a.dtype in (torch.bfloat16, torch.float16)
+
+
+def weight_gradient(a, b, batch_sizes, weight_dtype=None):
+    """gmm(a, b, batch_sizes, trans_a=True), the gradient of a weight of type `weight_dtype` (None: of a's): where 16-bit
+    operands meet an fp32 weight (autocast) the product's fp32 sums are stored as they are, in one launch, instead of
+    being rounded, stored, read and cast back (64 experts of 256 rows, [1024, 4096]: 352 us, the 16-bit product and the cast
+    514; 8 of 2048 rows, [2048, 8192]: 504, 546).  May come back in a's type: autograd then casts it."""
+    if not _wants_fp32(a, weight_dtype) or a.ndim != 2 or b.ndim != 2 or b.dtype != a.dtype or b.shape[0] != a.shape[0]:
+        return gmm(a, b, batch_sizes, trans_a=True)
+    a, b = a.contiguous(), b.contiguous()
+    rows, k, n = a.shape[0], a.shape[1], b.shape[1]
+    bins = _device_bins(batch_sizes, a.device, rows)
+    groups = bins.shape[0]
+    c = torch.empty((groups, k, n), dtype=torch.float32, device=a.device)
+    with _lib.device_of(a), _lib.record('gmm_tn', rows=rows, k=k, n=n, elem=a.element_size(), groups=groups) as rec:
+        rc = lib.mbx_gmm_tn_f32(_lib.ptr(a), _lib.ptr(b), 0, None, 1, None, _lib.ptr(c), _lib.dtype_of(a), _lib.ptr(bins), groups, rows,
+                                k, n, None, 0, 0, _lib.stream())
+        if rc == _lib.EUNSUPPORTED:
+            rec.cancel()
+    if rc == _lib.EUNSUPPORTED:
+        return gmm(a, b, batch_sizes, trans_a=True)
+    _lib.check(rc, 'gmm_tn_f32')
+    return c
+
+
+def gmm_tn_gather(a, src: GatheredRows, batch_sizes, c=None, fp32_out=False):
     """out[e] = a[r_e].T @ X[r_e] with X the rows `src` describes, read from the ungathered tokens (one launch,
     `mbx_gmm_tn_gather`; bit-identical to `gmm(a, src.materialize(), batch_sizes, trans_a=True)`).  The table of row
     offsets the kernel reads is built by the first call for a `src` and kept on it (the weight gradients of w1 and v1
-    share it).  Returns None where the library has no kernel for the operands: the caller gathers first."""
+    share it).  fp32_out: the fp32 sums as they are (`mbx_gmm_tn_f32`).  Returns None where the library has no kernel for
+    the operands: the caller gathers first."""
     x = src.x
     if not (x.is_cuda and x.ndim == 2 and x.dtype in (torch.bfloat16, torch.float16) and a.ndim == 2 and a.dtype == x.dtype
             and a.is_cuda and a.shape[0] == src.rows and src.indices.dtype == torch.int32 and src.bins.dtype == torch.int32):
@@ -445,9 +476,10 @@ def gmm_tn_gather(a, src: GatheredRows, batch_sizes, c=None):
     if src.bins.numel() != groups:
         return None
     x_bins = None if src.padded_bins is None else src.bins.contiguous()
+    out_dtype = torch.float32 if fp32_out else a.dtype
     if c is None:
-        c = torch.empty((groups, k, n), dtype=a.dtype, device=a.device)
-    elif tuple(c.shape) != (groups, k, n) or c.dtype != a.dtype or not c.is_contiguous():
+        c = torch.empty((groups, k, n), dtype=out_dtype, device=a.device)
+    elif tuple(c.shape) != (groups, k, n) or c.dtype != out_dtype or not c.is_contiguous():
         raise ValueError('gmm_tn_gather: c has the wrong shape, dtype or layout')
     table = getattr(src, '_row_table', None)
     ready = table is not None and table[1] == n
@@ -455,7 +487,8 @@ def gmm_tn_gather(a, src: GatheredRows, batch_sizes, c=None):
         table = (torch.empty(max(lib.mbx_gmm_tn_gather_table_bytes(x.shape[0], src.top_k, groups) // 4, 4), dtype=torch.int32,
                              device=x.device), n)
     with _lib.device_of(a), _lib.record('gmm_tn', rows=rows, k=k, n=n, elem=a.element_size(), groups=groups) as rec:
-        rc = lib.mbx_gmm_tn_gather(_lib.ptr(a), _lib.ptr(x), x.shape[0], _lib.ptr(src.indices.contiguous()), src.top_k,
+        launch = lib.mbx_gmm_tn_f32 if fp32_out else lib.mbx_gmm_tn_gather
+        rc = launch(_lib.ptr(a), _lib.ptr(x), x.shape[0], _lib.ptr(src.indices.contiguous()), src.top_k,
                                    _lib.ptr(x_bins), _lib.ptr(c), _lib.dtype_of(a), _lib.ptr(bins), groups, rows, k, n,
                                    _lib.ptr(table[0]), table[0].numel() * 4, 1 if ready else 0, _lib.stream())
         if rc == _lib.EUNSUPPORTED:

@@ -118,6 +118,9 @@ class GroupedGLUExperts(torch.autograd.Function):
     def forward(ctx, x, w1, v1, w2, batch_sizes, act, c_indices=None, c_bin_ids=None, c_bins=None, c_weights=None, keep=True):
         # c_*: the layer's combine (`gg.CombinedRows`), when the node is to return the combined output
         # keep False: no gradient is recorded, the first products themselves need not be written
+        ctx.weight_dtypes = w1.dtype, v1.dtype, w2.dtype
+        if ctx._fwd_used_autocast:
+            x, w1, v1, w2 = x.to(ctx._dtype), w1.to(ctx._dtype), v1.to(ctx._dtype), w2.to(ctx._dtype)
         x = x.contiguous()
         sdd_out, v1_out, activation_fn_out = gg.gmm_glu(x, w1, v1, batch_sizes, act, keep_product=keep)
         ctx.act = act
@@ -133,24 +136,24 @@ class GroupedGLUExperts(torch.autograd.Function):
         x, w1, v1, w2, batch_sizes, sdd_out, v1_out, activation_fn_out, *kept = ctx.saved_tensors
         ddsd_out, dweights = second_product_grad(kept, grad, ctx.needs_input_grad[9])
         return (*_glu_experts_backward(ctx.needs_input_grad, x, w1, v1, w2, batch_sizes, sdd_out, v1_out,
-                                       activation_fn_out, ddsd_out, ctx.act), None, None, None, None, None, dweights, None)
+                                       activation_fn_out, ddsd_out, ctx.act, ctx.weight_dtypes), None, None, None, None, None, dweights, None)
 
 
-def _glu_experts_backward(needs, x, w1, v1, w2, batch_sizes, sdd_out, v1_out, activation_fn_out, ddsd_out, act):
+def _glu_experts_backward(needs, x, w1, v1, w2, batch_sizes, sdd_out, v1_out, activation_fn_out, ddsd_out, act, weight_dtypes):
     """(dx, dw1, dv1, dw2) of GroupedGLUExperts from what its forward saved; needs = which of (x, w1, v1, w2) want a
     gradient.  x: the experts' input rows, or a `gg.GatheredRows` that describes them (the weight gradients then read
-    the rows from the ungathered tokens)."""
+    the rows from the ungathered tokens).  weight_dtypes: of w1, v1 and w2 before the casts of autocast."""
     ddsd_out = ddsd_out.contiguous()
     dx = dw1 = dv1 = dw2 = None
     if needs[3]:
-        dw2 = gg.backend.gmm(activation_fn_out, ddsd_out, batch_sizes, trans_a=True)
+        dw2 = gg.weight_gradient(activation_fn_out, ddsd_out, batch_sizes, weight_dtypes[2])
     if needs[0] or needs[1] or needs[2]:
         dsdd_out, dv1_out = gg.gmm_dglu(ddsd_out, w2, sdd_out, v1_out, batch_sizes, act)
-        wgrad = x.weight_gradient if isinstance(x, gg.GatheredRows) else (lambda d, sizes: gg.backend.gmm(d, x, sizes, trans_a=True))
+        wgrad = x.weight_gradient if isinstance(x, gg.GatheredRows) else (lambda d, *args: gg.weight_gradient(d, x, *args))
         if needs[1]:
-            dw1 = wgrad(dsdd_out, batch_sizes)
+            dw1 = wgrad(dsdd_out, batch_sizes, weight_dtypes[0])
         if needs[2]:
-            dv1 = wgrad(dv1_out, batch_sizes)
+            dv1 = wgrad(dv1_out, batch_sizes, weight_dtypes[1])
         if needs[0]:
             dx = gg.gmm_dual(dsdd_out, w1, dv1_out, v1, batch_sizes)
     return dx, dw1, dv1, dw2
@@ -169,6 +172,9 @@ class GatheredGLUExperts(torch.autograd.Function):
                 c_weights=None, keep=True):
         # keep False: no gradient is recorded, the first products themselves need not be written
         # combined: the node returns the layer's combine of its output (top_k = 1; the same assignments, c_weights)
+        ctx.weight_dtypes = w1.dtype, v1.dtype, w2.dtype
+        if ctx._fwd_used_autocast:
+            x, w1, v1, w2 = x.to(ctx._dtype), w1.to(ctx._dtype), v1.to(ctx._dtype), w2.to(ctx._dtype)
         x = x.contiguous()
         src = gg.GatheredRows(x, indices, bin_ids, bins, padded_bins, top_k, rows)
         out = gg.gmm_gather(src, w1, batch_sizes, b2=v1, act=act, keep_product=keep)
@@ -191,7 +197,7 @@ class GatheredGLUExperts(torch.autograd.Function):
         ddsd_out, dweights = second_product_grad(kept, grad, ctx.needs_input_grad[13])
         src = gg.GatheredRows(x, indices, bin_ids, bins, padded_bins, ctx.top_k, ctx.rows)
         dx, dw1, dv1, dw2 = _glu_experts_backward(ctx.needs_input_grad, src, w1, v1, w2, batch_sizes, sdd_out,
-                                                  v1_out, activation_fn_out, ddsd_out, ctx.act)
+                                                  v1_out, activation_fn_out, ddsd_out, ctx.act, ctx.weight_dtypes)
         if dx is not None:
             dx = src.scatter_grad(dx)
         return dx, dw1, dv1, dw2, None, None, None, None, None, None, None, None, None, dweights, None
@@ -199,9 +205,11 @@ class GatheredGLUExperts(torch.autograd.Function):
 
 def _one_node(x, w1, v1, w2, act):
     """Whether the experts can run as GroupedGLUExperts: an activation the library has, 16-bit operands of one type on
-    the GPU, rows the element-wise kernels take."""
-    return (act is not None and x.is_cuda and x.dtype in (torch.bfloat16, torch.float16) and
-            w1.dtype == v1.dtype == w2.dtype == x.dtype and (w1.shape[1] * x.element_size()) % 16 == 0 and
+    the GPU (under autocast: once the node has cast them), rows the element-wise kernels take."""
+    autocast = x.is_cuda and torch.is_autocast_enabled()
+    dtype = _lib.autocast_gpu_dtype() if autocast else x.dtype
+    return (act is not None and x.is_cuda and dtype in (torch.bfloat16, torch.float16) and
+            (autocast or w1.dtype == v1.dtype == w2.dtype == x.dtype) and w1.shape[1] % 8 == 0 and
             w1.is_contiguous() and v1.is_contiguous() and w2.is_contiguous())
 
 
@@ -211,6 +219,7 @@ class MemoryOptimizedGroupedGLU(torch.autograd.Function):
     @staticmethod
     @torch.amp.custom_fwd(device_type='cuda')
     def forward(ctx, x, w1, v1, w2, batch_sizes, activation_fn):
+        ctx.weight_dtypes = w1.dtype, v1.dtype, w2.dtype
         if ctx._fwd_used_autocast:
             x, w1, v1, w2 = x.to(ctx._dtype), w1.to(ctx._dtype), v1.to(ctx._dtype), w2.to(ctx._dtype)
         if not x.is_contiguous() or not w1.is_contiguous() or not v1.is_contiguous() or not w2.is_contiguous():
@@ -251,7 +260,7 @@ class MemoryOptimizedGroupedGLU(torch.autograd.Function):
                 v1_out = v1_out.detach().requires_grad_(True)
                 activation_fn_out = activation_fn(sdd_out) * v1_out
 
-        dw2 = gg.backend.gmm(activation_fn_out.detach(), ddsd_out, batch_sizes, trans_a=True)
+        dw2 = gg.weight_gradient(activation_fn_out.detach(), ddsd_out, batch_sizes, ctx.weight_dtypes[2])
         if fused:
             # one launch where the library has it; else the product (which then overwrites the recomputed activation,
             # glu.py:138) and the element-wise backward
@@ -261,8 +270,8 @@ class MemoryOptimizedGroupedGLU(torch.autograd.Function):
             activation_fn_out.backward(dactivation_fn_out)
             dsdd_out, dv1_out = sdd_out.grad, v1_out.grad
 
-        dw1 = gg.backend.gmm(dsdd_out, x, batch_sizes, trans_a=True)
-        dv1 = gg.backend.gmm(dv1_out, x, batch_sizes, trans_a=True)
+        dw1 = gg.weight_gradient(dsdd_out, x, batch_sizes, ctx.weight_dtypes[0])
+        dv1 = gg.weight_gradient(dv1_out, x, batch_sizes, ctx.weight_dtypes[1])
         dx = gg.gmm_dual(dsdd_out, w1, dv1_out, v1, batch_sizes, c=ddsd_out)   # reuses the ddsd_out allocation
         return dx, dw1, dv1, dw2, None, None
 
@@ -290,11 +299,10 @@ class SparseGLU(SparseMLP):
                     'Memory optimized implementation not yet supported with GLU with sparse kernels.')
             return self._combined(memory_optimized_grouped_glu(x, w1, v1, w2, batch_sizes, self.args.activation_fn), combine)
         act = _activation_code(self.args.activation_fn)
-        operands = gg.autocast_operands(x, w1, v1, w2)
-        if _one_node(*operands, act):
+        if _one_node(x, w1, v1, w2, act):
             c = (None, None, None, None) if combine is None else (combine.indices, combine.bin_ids, combine.bins, combine.weights)
-            return GroupedGLUExperts.apply(*operands, batch_sizes, act, *c, torch.is_grad_enabled())
-        x1, x2 = GLUProjection.apply(*operands[:3], batch_sizes)
+            return GroupedGLUExperts.apply(x, w1, v1, w2, batch_sizes, act, *c, torch.is_grad_enabled())
+        x1, x2 = GLUProjection.apply(*gg.autocast_operands(x, w1, v1), batch_sizes)
         x1 = gated_activation(self.args.activation_fn, x1, x2)
         return self._combined(gg.ops.gmm(x1, w2, batch_sizes), combine)
 
@@ -311,7 +319,7 @@ class SparseGLU(SparseMLP):
             return None
         act = _activation_code(self.args.activation_fn)
         w1, v1, w2 = self._expert_views(self.w1, self.v1, self.w2)
-        x, w1, v1, w2 = gg.autocast_operands(src.x, w1, v1, w2)
+        x = src.x
         if not _one_node(x, w1, v1, w2, act):
             return None
         return GatheredGLUExperts.apply(x, w1, v1, w2, batch_sizes, act, src.indices, src.bin_ids, src.bins,

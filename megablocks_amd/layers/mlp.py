@@ -176,6 +176,7 @@ class GroupedGeluMLP(torch.autograd.Function):
     def forward(ctx, x, w1, w2, batch_sizes, c_indices=None, c_bin_ids=None, c_bins=None, c_weights=None, keep=True):
         # c_*: the layer's combine (`gg.CombinedRows`), when the node is to return the combined output
         # keep False: no gradient is recorded, the first product itself need not be written
+        ctx.weight_dtypes = w1.dtype, w2.dtype
         if ctx._fwd_used_autocast:
             x, w1, w2 = x.to(ctx._dtype), w1.to(ctx._dtype), w2.to(ctx._dtype)
         x, w1, w2 = x.contiguous(), w1.contiguous(), w2.contiguous()
@@ -191,23 +192,23 @@ class GroupedGeluMLP(torch.autograd.Function):
     def backward(ctx: Any, grad: torch.Tensor):
         w1, w2, batch_sizes, x, sdd_out, activation_fn_out, *kept = ctx.saved_tensors
         ddsd_out, dweights = second_product_grad(kept, grad, ctx.needs_input_grad[7])
-        return (*_gelu_mlp_backward(ctx.needs_input_grad, x, w1, w2, batch_sizes, sdd_out, activation_fn_out, ddsd_out),
-                None, None, None, None, dweights, None)
+        return (*_gelu_mlp_backward(ctx.needs_input_grad, x, w1, w2, batch_sizes, sdd_out, activation_fn_out, ddsd_out,
+                                    ctx.weight_dtypes), None, None, None, None, dweights, None)
 
 
-def _gelu_mlp_backward(needs, x, w1, w2, batch_sizes, sdd_out, activation_fn_out, ddsd_out):
+def _gelu_mlp_backward(needs, x, w1, w2, batch_sizes, sdd_out, activation_fn_out, ddsd_out, weight_dtypes):
     """(dx, dw1, dw2) of GroupedGeluMLP from what its forward saved; needs = which of (x, w1, w2) want a gradient.
     x: the experts' input rows, or a `gg.GatheredRows` that describes them (the weight gradient then reads the rows from
-    the ungathered tokens)."""
+    the ungathered tokens).  weight_dtypes: of w1 and w2 before the casts of autocast."""
     ddsd_out = ddsd_out.contiguous()
     dx = dw1 = dw2 = None
     if needs[2]:
-        dw2 = gg.backend.gmm(activation_fn_out, ddsd_out, batch_sizes, trans_a=True)
+        dw2 = gg.weight_gradient(activation_fn_out, ddsd_out, batch_sizes, weight_dtypes[1])
     if needs[0] or needs[1]:
         dsdd_out = gg.gmm_dact(ddsd_out, w2, sdd_out, batch_sizes)
         if needs[1]:
-            dw1 = x.weight_gradient(dsdd_out, batch_sizes) if isinstance(x, gg.GatheredRows) else \
-                gg.backend.gmm(dsdd_out, x, batch_sizes, trans_a=True)
+            dw1 = x.weight_gradient(dsdd_out, batch_sizes, weight_dtypes[0]) if isinstance(x, gg.GatheredRows) else \
+                gg.weight_gradient(dsdd_out, x, batch_sizes, weight_dtypes[0])
         if needs[0]:
             dx = gg.backend.gmm(dsdd_out, w1, batch_sizes)
     return dx, dw1, dw2
@@ -258,6 +259,7 @@ class GatheredGeluMLP(torch.autograd.Function):
                 c_weights=None, keep=True):
         # combined: the node returns the layer's combine of its output (top_k = 1; the same assignments, c_weights)
         # keep False: no gradient is recorded, the first product itself need not be written
+        ctx.weight_dtypes = w1.dtype, w2.dtype
         if ctx._fwd_used_autocast:
             x, w1, w2 = x.to(ctx._dtype), w1.to(ctx._dtype), w2.to(ctx._dtype)
         x, w1, w2 = x.contiguous(), w1.contiguous(), w2.contiguous()
@@ -281,7 +283,7 @@ class GatheredGeluMLP(torch.autograd.Function):
         ddsd_out, dweights = second_product_grad(kept, grad, ctx.needs_input_grad[11])
         src = gg.GatheredRows(x, indices, bin_ids, bins, padded_bins, ctx.top_k, ctx.rows)
         dx, dw1, dw2 = _gelu_mlp_backward(ctx.needs_input_grad, src, w1, w2, batch_sizes, sdd_out,
-                                          activation_fn_out, ddsd_out)
+                                          activation_fn_out, ddsd_out, ctx.weight_dtypes)
         if dx is not None:
             dx = src.scatter_grad(dx)
         return dx, dw1, dw2, None, None, None, None, None, None, None, None, dweights, None
@@ -300,6 +302,7 @@ class MemoryOptimizedGroupedMLP(torch.autograd.Function):
     @staticmethod
     @torch.amp.custom_fwd(device_type='cuda')
     def forward(ctx, x, w1, w2, batch_sizes, activation_fn):
+        ctx.weight_dtypes = w1.dtype, w2.dtype
         if ctx._fwd_used_autocast:
             x, w1, w2 = x.to(ctx._dtype), w1.to(ctx._dtype), w2.to(ctx._dtype)
         if not x.is_contiguous() or not w1.is_contiguous() or not w2.is_contiguous():
@@ -335,7 +338,7 @@ class MemoryOptimizedGroupedMLP(torch.autograd.Function):
                 sdd_out = sdd_out.detach().requires_grad_(True)
                 activation_fn_out = activation_fn(sdd_out)
 
-        dw2 = gg.backend.gmm(activation_fn_out.detach(), ddsd_out, batch_sizes, trans_a=True)
+        dw2 = gg.weight_gradient(activation_fn_out.detach(), ddsd_out, batch_sizes, ctx.weight_dtypes[1])
 
         if default_act:
             # d(sdd_out) overwrites the recomputed activation: the product ddsd_out @ w2^T with the closed-form GELU
@@ -346,7 +349,7 @@ class MemoryOptimizedGroupedMLP(torch.autograd.Function):
             activation_fn_out.backward(dactivation_fn_out)
             dsdd_out = sdd_out.grad
 
-        dw1 = gg.backend.gmm(dsdd_out, x, batch_sizes, trans_a=True)
+        dw1 = gg.weight_gradient(dsdd_out, x, batch_sizes, ctx.weight_dtypes[0])
         dx = gg.backend.gmm(dsdd_out, w1, batch_sizes, c=ddsd_out)   # reuses the incoming gradient buffer
         return dx, dw1, dw2, None, None
 

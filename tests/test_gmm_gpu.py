@@ -1214,3 +1214,64 @@ def test_gmm_tn_with_few_rows_per_expert(gg, groups, rows, k, n, skew, dtype):
         bin_ids = torch.repeat_interleave(torch.arange(groups), sizes).int().cuda()
         src = gg.GatheredRows(x, order, bin_ids, bins, None, 1, rows)
         assert torch.equal(gg.gmm_tn_gather(a, src, sizes.cuda()), gg.backend.gmm(a, x[order.long()], sizes, trans_a=True))
+
+
+@pytest.mark.parametrize('groups,rows,k,n', [(1, 1, 8, 8), (3, 130, 64, 136), (5, 5 * 300, 264, 1032), (70, 900, 136, 256), (4, 4 * 1500, 392, 264),
+                                             (8, 8 * 2100, 1024, 640), (2, 0, 64, 64)])
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])
+def test_weight_gradients_of_fp32_weights(gg, groups, rows, k, n, dtype):
+    """The fp32 weight gradient of 16-bit operands: rounded it is the 16-bit product bit for bit, and against fp64 it shows
+    the error of an fp32 sum (2^-24 per term, random signs, a factor of four to spare).  Plain and on gathered rows."""
+    torch.manual_seed(rows + n)
+    sizes = _sizes(groups, rows, seed=k, empty=(0,) if groups > 2 and rows else ()).cuda()
+    a = torch.randn(rows, k, device='cuda').to(dtype)
+    x = torch.randn(rows, n, device='cuda').to(dtype)
+    got = gg.weight_gradient(a, x, sizes, torch.float32)
+    assert got.dtype == torch.float32 and torch.equal(got.to(dtype), gg.backend.gmm(a, x, sizes, trans_a=True))
+    start = 0
+    for e, c in enumerate(sizes.tolist()):
+        want = a[start:start + c].double().t() @ x[start:start + c].double()
+        assert rel_err(got[e].double(), want) <= 4 * 2.0 ** -24 * max(c, 16) ** 0.5 if c else not got[e].any()
+        start += c
+    assert gg.weight_gradient(a, x, sizes).dtype == dtype and gg.weight_gradient(a, x, sizes, dtype).dtype == dtype
+    if rows and k > 128:
+        order = torch.randperm(rows, device='cuda').int()
+        bins = torch.cumsum(sizes, 0).int()
+        bin_ids = torch.repeat_interleave(torch.arange(groups, device='cuda'), sizes.long()).int()
+        src = gg.GatheredRows(x, order, bin_ids, bins, None, 1, rows)
+        wide = src.weight_gradient(a, sizes, torch.float32)
+        assert wide.dtype == torch.float32 and torch.equal(wide.to(dtype), gg.gmm_tn_gather(a, src, sizes))
+
+
+@pytest.mark.parametrize('mlp', ['mlp', 'glu'])
+@pytest.mark.parametrize('memopt', [False, True])
+@pytest.mark.parametrize('top_k', [1, 4])
+def test_autocast_gradients_of_fp32_experts(gg, mlp, memopt, top_k):
+    """A layer with fp32 parameters under autocast: every gradient in fp32, the experts' without the rounding to bf16 the plain
+    route gives them, and within one rounding of that route's."""
+    from megablocks_amd.layers.arguments import Arguments
+    from megablocks_amd.layers.dmoe import dMoE
+    torch.manual_seed(3)
+    kw = dict(activation_fn=torch.nn.functional.silu) if mlp == 'glu' else {}
+    layer = dMoE(Arguments(hidden_size=136, ffn_hidden_size=264, moe_num_experts=8, moe_top_k=top_k, bias=False, mlp_type=mlp, mlp_impl='grouped',
+                           memory_optimized_mlp=memopt, moe_loss_weight=0.0, fp16=False, bf16=False, device=torch.device('cuda'), **kw))
+    x = torch.randn(200, 1, 136, device='cuda', requires_grad=True)
+    grad = torch.randn(200, 1, 136, device='cuda').bfloat16()
+    results = []
+    for wide in (True, False):
+        with pytest.MonkeyPatch.context() as patch:
+            if not wide:
+                patch.setattr(gg, '_wants_fp32', lambda *_: False)
+            layer.zero_grad(set_to_none=True)
+            x.grad = None
+            with torch.autocast('cuda', dtype=torch.bfloat16):
+                y = layer(x)
+            y.backward(grad)
+            results.append([x.grad] + [p.grad for p in layer.parameters()])
+    assert torch.equal(results[0][0], results[1][0])
+    rounded = 0
+    for got, want in zip(*results):
+        assert got.dtype == want.dtype == torch.float32
+        assert torch.equal(got, want) or torch.equal(got.bfloat16().float(), want)
+        rounded += not torch.equal(got, want)
+    assert rounded == (3 if mlp == 'glu' else 2)
