@@ -79,6 +79,9 @@ int mbx_route(const int32_t* expert_ids, int64_t n, int num_experts, int end_bit
               int32_t* bin_ids, int32_t* tokens_per_expert, int32_t* bins, int32_t* padded_bins,
               int32_t* slot_rows, void* scratch, size_t scratch_bytes, mbx_stream_t stream);
 
+/* megablocks/ops/round_up.py:7-14: out[i] = (x[i] + value - 1) / value * value in 32-bit arithmetic (division towards zero). */
+int mbx_round_up(const int32_t* x, int64_t n, int32_t value, int32_t* out, mbx_stream_t stream);
+
 /* csrc/cumsum.h:104-156 `inclusive_cumsum / exclusive_cumsum(x, dim=1, out)`: scan of
  * every row of x [rows, n]. */
 int mbx_cumsum(const void* x, int itype, int64_t rows, int64_t n, int exclusive, void* out,

@@ -32,25 +32,30 @@ constexpr int kHistLdsBins = 8192;
 
 // One block per (chunk, row).  Counts land in LDS; lanes holding the same id are merged
 // with ballots first when the id space is small, so an LDS atomic is issued once per
-// distinct id per wave instead of once per lane.
-template <typename T, bool DIRECT>
+// distinct id per wave instead of once per lane.  A block takes kHistThreads * ROUNDS ids, all of whose loads are under way
+// before the first is counted (65536 ids: 2.9 us; 7.0 with eight rounds one after the other).
+template <typename T, bool DIRECT, int ROUNDS>
 __global__ void __launch_bounds__(kHistThreads)
-histogram_kernel(const T* __restrict__ x, int64_t n, int num_bins, int nbits, int64_t chunk,
-                 int32_t* __restrict__ out) {
+histogram_kernel(const T* __restrict__ x, int64_t n, int num_bins, int nbits, int32_t* __restrict__ out) {
   extern __shared__ int32_t hist[];
   const int64_t row = blockIdx.y;
   const T* xr = x + row * n;
   int32_t* outr = out + row * (int64_t)num_bins;
+  const int64_t begin = (int64_t)blockIdx.x * (kHistThreads * ROUNDS);
+  T ids[ROUNDS];
+#pragma unroll
+  for (int r = 0; r < ROUNDS; ++r) {
+    const int64_t i = begin + r * kHistThreads + threadIdx.x;
+    ids[r] = i < n ? xr[i] : (T)-1;
+  }
   for (int b = threadIdx.x; b < num_bins; b += kHistThreads) hist[b] = 0;
   __syncthreads();
-  const int64_t begin = (int64_t)blockIdx.x * chunk;
-  const int64_t end = begin + chunk < n ? begin + chunk : n;
   // every lane of a wave runs the same number of rounds so the ballots see whole waves
-  for (int64_t base = begin; base < end; base += kHistThreads) {
-    const int64_t i = base + threadIdx.x;
-    bool valid = i < end;
-    int64_t v = valid ? (int64_t)xr[i] : 0;
-    valid = valid && v >= 0 && v < num_bins;
+#pragma unroll
+  for (int r = 0; r < ROUNDS; ++r) {
+    if (begin + r * kHistThreads >= n) break;
+    const int64_t v = (int64_t)ids[r];
+    const bool valid = v >= 0 && v < num_bins;
     if (nbits > 0) {
       const uint64_t peers = match_peers((uint32_t)v, valid, nbits);
       if (valid && (peers & lanemask_lt()) == 0) atomicAdd(&hist[v], (int32_t)__popcll(peers));
@@ -90,14 +95,17 @@ int histogram_impl(const T* x, int64_t rows, int64_t n, int num_bins, int32_t* o
   if (num_bins <= kHistLdsBins) {
     const size_t lds = (size_t)num_bins * sizeof(int32_t);
     if (n <= (int64_t)kHistThreads * 8) {  // one block per row writes its counts directly
-      histogram_kernel<T, true><<<dim3(1, (unsigned)rows), kHistThreads, lds, s>>>(x, n, num_bins, nbits, n > 0 ? n : 1, out);
+      histogram_kernel<T, true, 8><<<dim3(1, (unsigned)rows), kHistThreads, lds, s>>>(x, n, num_bins, nbits, out);
       return launch_status();
     }
     fill_i32_kernel<<<(unsigned)(ceil_div(total, 256) < 1024 ? ceil_div(total, 256) : 1024), 256, 0, s>>>(out, total, 0);
-    const int64_t chunk = (int64_t)kHistThreads * 8;
-    const int64_t blocks = ceil_div(n, chunk);
+    // two rounds to a block while that is no more than two blocks per compute unit
+    const bool few = ceil_div(n, (int64_t)kHistThreads * 2) * rows <= 512;
+    const int64_t blocks = ceil_div(n, (int64_t)kHistThreads * (few ? 2 : 8));
     if (blocks > 0x7fffffff) return MBX_ERANGE;
-    histogram_kernel<T, false><<<dim3((unsigned)blocks, (unsigned)rows), kHistThreads, lds, s>>>(x, n, num_bins, nbits, chunk, out);
+    const dim3 grid((unsigned)blocks, (unsigned)rows);
+    if (few) histogram_kernel<T, false, 2><<<grid, kHistThreads, lds, s>>>(x, n, num_bins, nbits, out);
+    else histogram_kernel<T, false, 8><<<grid, kHistThreads, lds, s>>>(x, n, num_bins, nbits, out);
     return launch_status();
   }
   fill_i32_kernel<<<(unsigned)(ceil_div(total, 256) < 1024 ? ceil_div(total, 256) : 1024), 256, 0, s>>>(out, total, 0);
@@ -107,6 +115,12 @@ int histogram_impl(const T* x, int64_t rows, int64_t n, int num_bins, int32_t* o
     histogram_global_kernel<T><<<dim3((unsigned)blocks, (unsigned)rows), 256, 0, s>>>(x, n, num_bins, out);
   }
   return launch_status();
+}
+
+// ------------------------------------------------------------------ round up
+__global__ void round_up_kernel(const int32_t* __restrict__ x, int64_t n, int32_t value, int32_t* __restrict__ out) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) out[i] = (int32_t)((uint32_t)((int32_t)((uint32_t)x[i] + (uint32_t)(value - 1)) / value) * (uint32_t)value);
 }
 
 // ------------------------------------------------------------------ radix sort
@@ -613,6 +627,16 @@ int mbx_route(const int32_t* expert_ids, int64_t n, int num_experts, int end_bit
   } while (0)
   if (sort_items(n) == kSortItemsShort) MBX_ROUTE_PASS(kSortItemsShort); else MBX_ROUTE_PASS(kSortItemsLong);
 #undef MBX_ROUTE_PASS
+  return launch_status();
+}
+
+int mbx_round_up(const int32_t* x, int64_t n, int32_t value, int32_t* out, mbx_stream_t stream) {
+  if (n < 0 || value <= 0) return MBX_EINVAL;
+  if (n == 0) return 0;
+  if (!x || !out) return MBX_EINVAL;
+  const int64_t blocks = ceil_div(n, 256);
+  if (blocks > 0x7fffffff) return MBX_ERANGE;
+  round_up_kernel<<<(unsigned)blocks, 256, 0, as_stream(stream)>>>(x, n, value, out);
   return launch_status();
 }
 

@@ -583,3 +583,23 @@ def test_route_with_ids_outside_the_experts_stays_in_range(blocking):
         want = torch.zeros_like(out)
         want[owned.cuda().long()] = x[((rows >= 0).nonzero().flatten() // top_k).cuda()]
         assert torch.equal(out, want)
+
+
+@pytest.mark.parametrize('n', [0, 1, 1023, 8192, 8193, 65536, 2 * 1024 * 513, 2 ** 21 + 5])
+@pytest.mark.parametrize('dtype', [torch.int16, torch.int32, torch.int64])
+def test_histogram_over_the_block_sizes(ops, n, dtype):
+    """One block, two rounds to a block, eight: sizes around the lines between them; ids outside the bins are not counted."""
+    torch.manual_seed(n)
+    ids = torch.randint(-2, 70, (n,)).to(dtype)
+    want = torch.bincount(ids[(ids >= 0) & (ids < 64)].long(), minlength=64)
+    assert torch.equal(ops.histogram(ids.cuda(), 64).cpu().long(), want)
+
+
+def test_round_up_in_one_launch(ops):
+    x = torch.randint(-1000, 100000, (1000,), dtype=torch.int32)
+    x[0] = 2 ** 31 - 5
+    for value in (1, 7, 128, 2 ** 30):
+        want = torch.div(x + (value - 1), value, rounding_mode='trunc') * value
+        assert torch.equal(ops.round_up(x.cuda(), value).cpu(), want)
+        assert torch.equal(ops.round_up(x.cuda()[::3], value).cpu(), want[::3])
+    assert ops.round_up(x[:0].cuda(), 128).shape == (0,) and ops.round_up(x.cuda().view(10, 100), 128).shape == (10, 100)
