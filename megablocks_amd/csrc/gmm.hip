@@ -555,6 +555,7 @@ int launch_tn(const DmaCall& call) {
 // here (the half-height tile only when the product has at most 128 rows: it is slower otherwise).
 static int gmm_dma(const DmaCall& call) {
   if (gmm_few_takes(call)) return gmm_few(call);
+  if (gmm_mid_takes(call)) return gmm_mid(call);
   if (call.layout != MBX_TN) return call.k % dma::TileMain::BK == 0 ? gmm_rows(call) : gmm_rows_tail(call);
   if (gmm_tn_short_takes(call)) return gmm_tn_short(call);
   if (call.gather.slots) {   // gathered rows: the full tile only

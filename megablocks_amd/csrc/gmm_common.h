@@ -62,6 +62,10 @@ struct DmaCall {
 bool gmm_few_takes(const DmaCall& call);
 int gmm_few(const DmaCall& call);
 
+// NT launches with a few dozen rows per expert (gmm_mid.hip), and whether a launch is one of them.
+bool gmm_mid_takes(const DmaCall& call);
+int gmm_mid(const DmaCall& call);
+
 // TN launches with few rows per expert (gmm_tn_short.hip), and whether a launch is one of them.
 bool gmm_tn_short_takes(const DmaCall& call);
 int gmm_tn_short(const DmaCall& call);

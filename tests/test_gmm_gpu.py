@@ -1275,3 +1275,59 @@ def test_autocast_gradients_of_fp32_experts(gg, mlp, memopt, top_k):
         assert torch.equal(got, want) or torch.equal(got.bfloat16().float(), want)
         rounded += not torch.equal(got, want)
     assert rounded == (3 if mlp == 'glu' else 2)
+
+
+@pytest.mark.parametrize('groups,rows,k,n', [(64, 640, 64, 1032), (70, 70 * 40, 72, 1288), (300, 12000, 128, 8), (9, 9 * 39, 520, 7688),
+                                             (8, 8 * 40 + 1, 192, 8456), (40, 40 * 30, 1032, 2056)])
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])
+def test_gmm_nt_with_a_few_dozen_rows_per_expert(gg, groups, rows, k, n, dtype):
+    """NT launches on both sides of the line where the kernel for them takes over, every form, against fp32; the forms' products
+    equal bit for bit.  Experts of 0 to more than 64 rows; an infinite expert must not reach its neighbours."""
+    torch.manual_seed(rows)
+    sizes = _sizes(groups, rows, seed=rows, empty=(1,))
+    ends = torch.cumsum(sizes, 0)
+    a = torch.randn(rows, k, device='cuda').to(dtype)
+    w, v = ((torch.randn(groups, n, k, device='cuda') / k ** 0.5).to(dtype) for _ in range(2))
+    w[2] = float('inf')   # an expert's weights: its rows only
+    keep = torch.ones(rows, 1, dtype=torch.bool, device='cuda')
+    keep[int(ends[1]):int(ends[2])] = False
+    zero = torch.zeros((), device='cuda')
+
+    def check(got, want):
+        got, want = (torch.where(keep, t.float(), zero) for t in (got, want))
+        assert rel_err(got, want) < TOL and max_block_err(got, want, 8, 32) < 4 * TOL
+
+    def same(x, y):
+        return torch.equal(torch.where(keep, x.float(), zero), torch.where(keep, y.float(), zero))
+
+    ref, ref_v = _ref_gpu(a, w, sizes, False, True), _ref_gpu(a, v, sizes, False, True)
+    sizes = sizes.cuda()
+    c = gg.backend.gmm(a, w, sizes, trans_b=True)
+    check(c, ref)
+    pre, act = gg.gmm_act(a, w, sizes, fuse=True)
+    assert same(pre, c)
+    check(act, torch.nn.functional.gelu(c.float(), approximate='tanh'))
+    saved, saved2 = torch.randn(rows, n, device='cuda').to(dtype), torch.randn(rows, n, device='cuda').to(dtype)
+    x = saved.float().requires_grad_(True)
+    torch.nn.functional.gelu(x, approximate='tanh').backward(torch.where(keep, c.float(), zero))
+    check(gg.gmm_dact(a, w, saved, sizes, fuse=True), x.grad)
+    for code, fn in ((0, torch.nn.functional.silu), (1, lambda t: torch.nn.functional.gelu(t, approximate='tanh'))):
+        x1, x2, h = gg.gmm_glu(a, w, v, sizes, code, fuse=True)
+        assert same(x1, c)
+        check(x2, ref_v)
+        check(h, fn(x1.float()).to(dtype).float() * x2.float())
+        p, q = saved.float().requires_grad_(True), saved2.float().requires_grad_(True)
+        (fn(p) * q).backward(torch.where(keep, c.float(), zero))
+        d1, d2 = gg.gmm_dglu(a, w, saved, saved2, sizes, code, fuse=True)
+        check(d1, p.grad)
+        check(d2, q.grad)
+    if k % 64 == 0:
+        order = torch.randperm(rows, device='cuda').int()
+        bins = ends.cuda().int()
+        bin_ids = torch.repeat_interleave(torch.arange(groups, device='cuda'), sizes.long()).int()
+        tokens = torch.empty_like(a)
+        tokens[order.long()] = a
+        src = gg.GatheredRows(tokens, order, bin_ids, bins, None, 1, rows)
+        assert same(gg.gmm_gather(src, w, sizes)[0], c)
+        assert same(gg.gmm_gather(src, w, sizes, b2=v, act=1)[2], h)
+        assert same(gg.gmm_gather(src, w, sizes, b2=v, act=1, keep_product=False)[2], h)
