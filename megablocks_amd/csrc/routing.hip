@@ -133,8 +133,13 @@ constexpr int kSortWaves = kSortThreads / kWave;
 // 11 us).  From 64 Ki keys on there are blocks enough, and the longer count table would cost the scan more than
 // the shorter chains give.
 constexpr int kSortItemsShort = 2, kSortItemsLong = 8;
-static inline int sort_items(int64_t n) { return n <= 65536 ? kSortItemsShort : kSortItemsLong; }
-static inline int sort_tile(int64_t n) { return kSortThreads * sort_items(n); }   // keys per block
+constexpr int64_t kSortShortMost = 65536;
+static inline int sort_blocks(int64_t n, int items) { return (int)ceil_div(n, kSortThreads * items); }
+static inline size_t sort_counts_bytes(int64_t n, int items) { return (size_t)kRadix * sort_blocks(n, items) * sizeof(int32_t); }
+// `room`: the bytes there are for the count table.  A buffer made for another size may hold only the table of long rounds.
+static inline int sort_items(int64_t n, size_t room) {
+  return n <= kSortShortMost && room >= sort_counts_bytes(n, kSortItemsShort) ? kSortItemsShort : kSortItemsLong;
+}
 constexpr int kSortTileMax = kSortThreads * kSortItemsLong;
 
 template <typename T> struct UnsignedOf;
@@ -418,12 +423,10 @@ int sort_impl(const T* x, int64_t n, int end_bit, T* keys_out, T* perm_out, void
     copy_iota_kernel<T><<<(unsigned)(ceil_div(n, 256) < 2048 ? ceil_div(n, 256) : 2048), 256, 0, s>>>(x, n, keys_out, perm_out);
     return launch_status();
   }
-  const int nblocks = (int)ceil_div(n, sort_tile(n));
-  const bool short_rounds = sort_items(n) == kSortItemsShort;
-  const size_t counts_bytes = align256((size_t)kRadix * nblocks * sizeof(int32_t));
-  const size_t buf_bytes = align256((size_t)n * sizeof(T));
-  const size_t need = counts_bytes + (passes > 1 ? 2 * buf_bytes : 0);
-  if (scratch_bytes < need || scratch == nullptr) return MBX_ESCRATCH;
+  const size_t buf_bytes = align256((size_t)n * sizeof(T)), bufs_bytes = passes > 1 ? 2 * buf_bytes : 0;
+  if (scratch_bytes < align256(sort_counts_bytes(n, kSortItemsLong)) + bufs_bytes || scratch == nullptr) return MBX_ESCRATCH;
+  const int items = sort_items(n, scratch_bytes - bufs_bytes), nblocks = sort_blocks(n, items);
+  const size_t counts_bytes = align256(sort_counts_bytes(n, items));   // a multiple of 1024: no padding
   int32_t* counts = (int32_t*)scratch;
   T* tmp_keys = (T*)((char*)scratch + counts_bytes);
   T* tmp_vals = (T*)((char*)scratch + counts_bytes + buf_bytes);
@@ -447,7 +450,7 @@ int sort_impl(const T* x, int64_t n, int end_bit, T* keys_out, T* perm_out, void
     else                                                                                                                  \
       radix_scatter_kernel<T, false, ITEMS><<<nblocks, kSortThreads, 0, s>>>(kin, vin, n, shift, mask, pass_bits, counts, nblocks, kout, vout);    \
   } while (0)
-    if (short_rounds) MBX_SORT_PASS(kSortItemsShort); else MBX_SORT_PASS(kSortItemsLong);
+    if (items == kSortItemsShort) MBX_SORT_PASS(kSortItemsShort); else MBX_SORT_PASS(kSortItemsLong);
 #undef MBX_SORT_PASS
     kin = kout;
     vin = vout;
@@ -577,8 +580,9 @@ size_t mbx_sort_scratch_bytes(int64_t n, int itype, int end_bit) {
   if (end_bit > bits) end_bit = bits;
   const int passes = sort_passes(end_bit);
   if (passes == 0) return 0;
-  const size_t nblocks = (size_t)ceil_div(n, sort_tile(n));
-  size_t need = align256((size_t)kRadix * nblocks * sizeof(int32_t));
+  // never less than for fewer keys: a buffer made for the longest list serves every list at full speed
+  const size_t longs = sort_counts_bytes(n, kSortItemsLong), shorts = sort_counts_bytes(n < kSortShortMost ? n : kSortShortMost, kSortItemsShort);
+  size_t need = align256(longs > shorts ? longs : shorts);
   if (passes > 1) need += 2 * align256((size_t)n * itype_bytes(itype));
   return need;
 }
@@ -610,13 +614,14 @@ int mbx_route(const int32_t* expert_ids, int64_t n, int num_experts, int end_bit
   const uint32_t mask = (1u << end_bit) - 1u;
   const int ndigits = 1 << end_bit;
   int32_t* const pbins = pad > 0 ? padded_bins : nullptr;
+  // the short lists need no scratch, but whether a call is accepted does not depend on the way it takes
+  if (scratch_bytes < sort_counts_bytes(n > 0 ? n : 1, kSortItemsLong) || scratch == nullptr) return MBX_ESCRATCH;
   if (n <= kRouteOneBlock) {
     route_one_block_kernel<<<1, 1024, 0, s>>>(expert_ids, (int)n, mask, end_bit, num_experts, pad, indices, bin_ids,
                                               tokens_per_expert, bins, pbins, slot_rows);
     return launch_status();
   }
-  const int nblocks = (int)ceil_div(n, sort_tile(n));
-  if (scratch_bytes < (size_t)kRadix * nblocks * sizeof(int32_t) || scratch == nullptr) return MBX_ESCRATCH;
+  const int items = sort_items(n, scratch_bytes), nblocks = sort_blocks(n, items);
   int32_t* counts = (int32_t*)scratch;
 #define MBX_ROUTE_PASS(ITEMS)                                                                                             \
   do {                                                                                                                    \
@@ -625,7 +630,7 @@ int mbx_route(const int32_t* expert_ids, int64_t n, int num_experts, int end_bit
     radix_scatter_kernel<int32_t, true, ITEMS><<<nblocks, kSortThreads, 0, s>>>(expert_ids, nullptr, n, 0, mask, end_bit, counts, nblocks, \
                                                                                 bin_ids, indices, slot_rows, bins, pbins, num_experts);    \
   } while (0)
-  if (sort_items(n) == kSortItemsShort) MBX_ROUTE_PASS(kSortItemsShort); else MBX_ROUTE_PASS(kSortItemsLong);
+  if (items == kSortItemsShort) MBX_ROUTE_PASS(kSortItemsShort); else MBX_ROUTE_PASS(kSortItemsLong);
 #undef MBX_ROUTE_PASS
   return launch_status();
 }

@@ -47,6 +47,9 @@ def test_error_strings_and_scratch_sizes():
     four = lib.mbx_sort_scratch_bytes(16384, 1, 32)             # four passes: plus two ping-pong buffers
     assert 0 < one < four and four >= one + 2 * 16384 * 4
     assert lib.mbx_sort_scratch_bytes(16384, 1, 0) == 0
+    for bits in (6, 32):                                        # a buffer for the longest list serves every list
+        sizes = [lib.mbx_sort_scratch_bytes(n, 1, bits) for n in (1, 512, 513, 16384, 65535, 65536, 65537, 262144, 262145, 1 << 20)]
+        assert sizes == sorted(sizes)
 
 
 def test_argument_errors_are_reported_without_touching_the_gpu():

@@ -515,6 +515,36 @@ def test_route_at_the_edges_of_its_launches(n, experts):
     assert torch.equal(got.cpu(), want) and torch.equal(perm.cpu(), want_perm.int())
 
 
+@pytest.mark.parametrize('n', [1, 4096, 4097, 30000, 65536, 65537])
+def test_sort_and_route_at_the_limits_of_the_scratch(n):
+    """A count table of 1024 bytes per 2048 keys is enough for either call (next to the two buffers of a sort of several passes),
+    whatever tiles it would take with more; with less, or none, both refuse."""
+    from megablocks_amd import _lib
+    lib = _lib.lib
+    ids = torch.randint(0, 64, (n,), generator=torch.Generator().manual_seed(n), dtype=torch.int32)
+    x, want = ids.cuda(), torch.sort(ids, stable=True)
+    keys, perm = torch.empty_like(x), torch.empty_like(x)
+    tpe, bins = torch.empty(64, dtype=torch.int32, device='cuda'), torch.empty(64, dtype=torch.int32, device='cuda')
+    table = (n + 2047) // 2048 * 1024
+    buffers = 2 * ((n * 4 + 255) // 256 * 256)
+
+    def calls(nbytes, bits, pass_scratch=True):
+        scratch = torch.empty(nbytes, dtype=torch.uint8, device='cuda') if pass_scratch else None
+        yield lambda: lib.mbx_sort(_lib.ptr(x), _lib.I32, n, bits, _lib.ptr(keys), _lib.ptr(perm), _lib.ptr(scratch), nbytes, _lib.stream())
+        if bits <= 8:
+            yield lambda: lib.mbx_route(_lib.ptr(x), n, 64, bits, 0, _lib.ptr(perm), _lib.ptr(keys), _lib.ptr(tpe), _lib.ptr(bins), None,
+                                        None, _lib.ptr(scratch), nbytes, _lib.stream())
+
+    for bits, least in ((6, table), (12, table + buffers)):
+        for nbytes in (least, lib.mbx_sort_scratch_bytes(n, _lib.I32, bits)):
+            for call in calls(nbytes, bits):
+                keys.fill_(-1), perm.fill_(-1)
+                assert call() == 0
+                assert torch.equal(keys.cpu(), want[0]) and torch.equal(perm.cpu(), want[1].int())
+        for call in [*calls(least - 1, bits), *calls(least, bits, pass_scratch=False)]:
+            assert call() == _lib.ESCRATCH
+
+
 @pytest.mark.parametrize('tokens', [1, 5, 1023, 1024])
 @pytest.mark.parametrize('hidden', [512, 520, 1031, 2056])
 @pytest.mark.parametrize('top_k', [1, 2, 6, 9])
