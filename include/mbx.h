@@ -56,7 +56,8 @@ int mbx_histogram(const void* x, int itype, int64_t rows, int64_t n, int num_bin
 
 /* csrc/sort.h:59-86 `sort(x, end_bit, x_out, iota_out)`: stable LSD radix sort of n keys
  * on bits [0, end_bit); the payload is 0..n-1 in the key type.  keys_out[i] =
- * x[perm_out[i]].  With end_bit equal to the key width the order is the signed order. */
+ * x[perm_out[i]].  With end_bit equal to the key width the order is the signed order.
+ * mbx_sort_scratch_bytes() is never less than for fewer keys: a buffer made for the longest list serves every list. */
 size_t mbx_sort_scratch_bytes(int64_t n, int itype, int end_bit);
 int mbx_sort(const void* x, int itype, int64_t n, int end_bit, void* keys_out,
              void* perm_out, void* scratch, size_t scratch_bytes, mbx_stream_t stream);
@@ -236,6 +237,9 @@ int mbx_gmm_dual(const void* a, const void* b, const void* a2, const void* b2, v
  *   first 4096 bytes are zero before the first launch that uses it.  Every launch leaves them zero again.  Launches
  *   that may run at the same time (different streams) need workspaces of their own. */
 size_t mbx_gmm_workspace_bytes(void);
+/* Which graph capture `stream` is part of, for callers that keep a workspace per capture: a number of its own for each
+ * capture, 0 outside of one. */
+int mbx_capture_id(mbx_stream_t stream, uint64_t* id);
 int mbx_gmm_ws(const void* a, const void* b, const void* a2, const void* b2, void* c, int dtype, const int32_t* bins,
                int num_groups, int64_t rows, int k, int n, int layout, void* workspace, size_t workspace_bytes,
                mbx_stream_t stream);

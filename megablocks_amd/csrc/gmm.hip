@@ -607,6 +607,15 @@ int mbx_debug_set_ticks(void* buffer) {
 }
 #endif
 
+int mbx_capture_id(mbx_stream_t stream, uint64_t* id) {
+  if (!id) return MBX_EINVAL;
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  unsigned long long number = 0;
+  MBX_HIP_CHECK(hipStreamGetCaptureInfo(as_stream(stream), &status, &number));
+  *id = status == hipStreamCaptureStatusNone ? 0 : number;
+  return 0;
+}
+
 size_t mbx_gmm_workspace_bytes(void) { return kWorkspaceCounters * sizeof(int32_t) + kWorkspaceParts * kWorkspacePartBytes; }
 
 static int gmm_dual_ws(const void* a, const void* b, const void* a2, const void* b2, void* c, int dtype, const int32_t* bins,

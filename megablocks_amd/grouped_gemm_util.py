@@ -5,6 +5,7 @@ bf16/f16 MFMA kernels of libmbx.so.
 `batch_sizes` may be the host int64 tensor the reference passes (mlp.py:502) or, to avoid
 the device-to-host copy, a device tensor of per-expert row counts.
 """
+import ctypes
 import os
 import types
 
@@ -83,24 +84,40 @@ def note_bins(batch_sizes: torch.Tensor, bins: torch.Tensor):
 # Device memory the NN products and all fp32 products lend the library for the parts of the tiles of their last round of workgroups
 # (`mbx_gmm_ws`): one buffer per device and stream, made at the first product on that stream and kept.  Launches on
 # one stream run one after the other, so they can share it; launches on different streams may overlap, so they do not.
-# A stream that is being captured gets its buffer from the capture's memory pool like any tensor made during a capture
-# (its zero-fill is a kernel of the graph; the buffer stays with this module, so later captures on a stream with the
-# same handle reuse it).  MBX_GMM_WORKSPACE=0: none (every tile is computed by one workgroup; results differ in the
-# last bits).
+# A stream that is being captured gets a buffer of its own for each capture, from the capture's memory pool (its counters
+# are cleared by a kernel of the graph): graphs may be replayed in any order, on any streams, next to each other and next
+# to eager work, and one that is never replayed clears nothing.  MBX_GMM_WORKSPACE=0: none (every tile is computed by one
+# workgroup; results differ in the last bits).
+_WORKSPACE_CLEARED = 4096   # bytes at its head that are zero before the first launch (`mbx_gmm_ws`)
 GMM_WORKSPACE = os.environ.get('MBX_GMM_WORKSPACE', '1') != '0'
 _workspaces = {}
+_captured_workspaces = {}   # (device, stream) -> (capture, buffer), of the last capture only: the memory is its graph's
 
 
 def _workspace(device):
     """(pointer, bytes) of the current stream's workspace on `device`; (None, 0) if switched off."""
     if not GMM_WORKSPACE:
         return None, 0
-    key = (device.index if device.index is not None else torch.cuda.current_device(), _lib.stream().value)
+    stream = _lib.stream()
+    key = (device.index if device.index is not None else torch.cuda.current_device(), stream.value)
+    if torch.cuda.is_current_stream_capturing():
+        return _captured_workspace(key, device, stream)
     ws = _workspaces.get(key)
     if ws is None:
         ws = torch.zeros(lib.mbx_gmm_workspace_bytes(), dtype=torch.uint8, device=device)
         _workspaces[key] = ws
     return _lib.ptr(ws), ws.numel()
+
+
+def _captured_workspace(key, device, stream):
+    capture = ctypes.c_uint64()
+    _lib.check(lib.mbx_capture_id(stream, ctypes.byref(capture)), 'capture_id')
+    kept = _captured_workspaces.get(key)
+    if kept is None or kept[0] != capture.value:
+        ws = torch.empty(lib.mbx_gmm_workspace_bytes(), dtype=torch.uint8, device=device)
+        ws[:_WORKSPACE_CLEARED].zero_()
+        kept = _captured_workspaces[key] = (capture.value, ws)
+    return _lib.ptr(kept[1]), kept[1].numel()
 
 
 def gmm(a, b, batch_sizes, trans_a=False, trans_b=False, c=None, _record_as=None):

@@ -970,6 +970,43 @@ def test_gmm_fp32_at_the_ends_of_the_range(gg, k, mode):
     assert not bool(got[9].any())
 
 
+@pytest.mark.parametrize('dtype,mode', [(torch.float32, 'nn'), (torch.float32, 'nt'), (torch.float32, 'tn'), (torch.bfloat16, 'nn')])
+def test_captures_have_workspaces_of_their_own(gg, dtype, mode):
+    """Two graphs captured one after the other on one stream, with products whose tiles are cut along the reduction: replayed
+    in either order, next to eager products, each gives the eager result bit for bit."""
+    torch.manual_seed(3)
+    groups, rows, k, n = 1, 256, 4096, 512
+    if mode == 'tn':
+        a, b, sizes = torch.randn(k, rows, device='cuda').to(dtype), torch.randn(k, n, device='cuda').to(dtype), [k]
+    else:
+        a = torch.randn(rows, k, device='cuda').to(dtype)
+        b, sizes = torch.randn(groups, *((n, k) if mode == 'nt' else (k, n)), device='cuda').to(dtype), [rows]
+    sizes = torch.tensor(sizes, device='cuda')
+
+    def product():
+        return gg.backend.gmm(a, b, sizes, trans_a=mode == 'tn', trans_b=mode == 'nt')
+
+    want = product()
+    torch.cuda.synchronize()
+    graphs, outs, used = [], [], [gg._workspace(a.device)[0]]
+    for _ in range(2):
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            outs.append((product(), product()))
+            used.append(gg._workspace(a.device)[0])
+            assert gg._workspace(a.device)[0] == used[-1]
+        graphs.append(graph)
+    assert len(set(used)) == 3
+    for order in ((1, 0), (0, 1), (1, 1, 0)):
+        for i in order:
+            for out in outs[i]:
+                out.zero_()
+            graphs[i].replay()
+            eager = product()
+            torch.cuda.synchronize()
+            assert all(torch.equal(out, want) for out in (*outs[i], eager))
+
+
 @pytest.mark.parametrize('power', [37, 110, 126])
 @pytest.mark.parametrize('mode', ['nn', 'nt', 'tn'])
 def test_gmm_fp32_of_small_by_large_values(gg, mode, power):
