@@ -141,16 +141,21 @@ class _SoftmaxTopK(torch.autograd.Function):
     @staticmethod
     def backward(ctx: Any, grad_scores, grad_weights, _grad_indices, _grad_indices32, grad_lse):
         scores, indices = ctx.saved_tensors
-        tokens, experts = scores.shape
-        grad_logits = torch.empty_like(scores)
-        gs = None if grad_scores is None else grad_scores.to(scores.dtype).contiguous()
-        gw = None if grad_weights is None else grad_weights.to(scores.dtype).contiguous()
-        gl = None if grad_lse is None else grad_lse.float().contiguous()
-        with _lib.device_of(scores):
-            _lib.check(_lib.lib.mbx_router_backward(_lib.ptr(gw), _lib.ptr(gs), _lib.ptr(scores), _lib.ptr(indices),
-                                                    _lib.dtype_of(scores), tokens, experts, ctx.top_k, ctx.norm_p,
-                                                    _lib.ptr(grad_logits), _lib.ptr(gl), _lib.stream()), 'router_backward')
-        return grad_logits, None, None, None
+        return _logits_gradient(scores, indices, ctx.top_k, ctx.norm_p, grad_scores, grad_weights, grad_lse), None, None, None
+
+
+def _logits_gradient(scores, indices, top_k, norm_p, grad_scores, grad_weights, grad_lse=None):
+    """The gradient of the logits behind _SoftmaxTopK's outputs (`mbx_router_backward`); the outputs' may be None."""
+    tokens, experts = scores.shape
+    grad_logits = torch.empty_like(scores)
+    gs = None if grad_scores is None else grad_scores.to(scores.dtype).contiguous()
+    gw = None if grad_weights is None else grad_weights.to(scores.dtype).contiguous()
+    gl = None if grad_lse is None else grad_lse.float().contiguous()
+    with _lib.device_of(scores):
+        _lib.check(_lib.lib.mbx_router_backward(_lib.ptr(gw), _lib.ptr(gs), _lib.ptr(scores), _lib.ptr(indices),
+                                                _lib.dtype_of(scores), tokens, experts, top_k, norm_p,
+                                                _lib.ptr(grad_logits), _lib.ptr(gl), _lib.stream()), 'router_backward')
+    return grad_logits
 
 
 class _LinearSoftmaxTopK(torch.autograd.Function):
@@ -162,10 +167,14 @@ class _LinearSoftmaxTopK(torch.autograd.Function):
 
     @staticmethod
     def supported(x: torch.Tensor, layer: torch.nn.Module, top_k: int) -> bool:
+        return not torch.is_grad_enabled() and _LinearSoftmaxTopK.fits(x, layer, top_k)
+
+    @staticmethod
+    def fits(x: torch.Tensor, layer: torch.nn.Module, top_k: int) -> bool:
         """Few tokens and a small layer: one launch instead of two (64 experts of 2048, 5 tokens: 11.1 -> 9.1 us on the GPU, and
         the vendor library's call alone is 25 us of host time; 512 tokens: 11.5 against 14.5, 128 experts of 4096: 14.0
         against 16.1)."""
-        if torch.is_grad_enabled() or type(layer) is not torch.nn.Linear or not x.is_cuda or x.shape[0] > _LinearSoftmaxTopK.MAX_TOKENS:
+        if type(layer) is not torch.nn.Linear or not x.is_cuda or x.shape[0] > _LinearSoftmaxTopK.MAX_TOKENS:
             return False
         weight = layer.weight
         return (x.dtype in (torch.bfloat16, torch.float16) and type(weight) is torch.nn.Parameter and weight.dtype == x.dtype and
@@ -187,6 +196,32 @@ class _LinearSoftmaxTopK(torch.autograd.Function):
                 _lib.ptr(weights), _lib.ptr(indices), _lib.ptr(indices32), _lib.stream()), 'router_linear_forward')
         ctx.mark_non_differentiable(indices, indices32)
         return scores, weights, indices, indices32
+
+
+class _RecordedLinearSoftmaxTopK(torch.autograd.Function):
+    """_LinearSoftmaxTopK where gradients are recorded.  The kernel sums a logit in another order than the vendor's product,
+    so both modes have to take it: a step that is recomputed (activation checkpointing runs the forward without gradients
+    first) must choose the experts, and weigh them, as the pass whose output it belongs to did."""
+
+    @staticmethod
+    def supported(x: torch.Tensor, layer: torch.nn.Module, top_k: int) -> bool:
+        return torch.is_grad_enabled() and _LinearSoftmaxTopK.fits(x, layer, top_k)
+
+    @staticmethod
+    def forward(ctx: Any, x: torch.Tensor, weight: torch.Tensor, top_k: int, norm_p: float):
+        scores, weights, indices, indices32 = _LinearSoftmaxTopK.forward(ctx, x, weight, top_k, norm_p)
+        ctx.save_for_backward(x, weight, scores, indices)
+        ctx.top_k, ctx.norm_p = top_k, float(norm_p)
+        ctx.set_materialize_grads(False)
+        return scores, weights, indices, indices32
+
+    @staticmethod
+    def backward(ctx: Any, grad_scores, grad_weights, _grad_indices, _grad_indices32):
+        x, weight, scores, indices = ctx.saved_tensors
+        grad = _logits_gradient(scores, indices, ctx.top_k, ctx.norm_p, grad_scores, grad_weights)
+        dx = grad @ weight if ctx.needs_input_grad[0] else None
+        dw = grad.t() @ x if ctx.needs_input_grad[1] else None
+        return dx, dw, None, None
 
 
 def _has_hooks(module: torch.nn.Module) -> bool:
@@ -240,9 +275,10 @@ class LearnedRouter(torch.nn.Module):
             x = x * self.jitter(x)
         x2d = x.view(-1, x.shape[-1])
         args = self.args
-        if FUSED_SOFTMAX_TOPK and args.moe_zloss_weight == 0 and not args.uniform_expert_assignment and \
-                _LinearSoftmaxTopK.supported(x2d, self.layer, args.moe_top_k):
-            return _LinearSoftmaxTopK.apply(x2d, self.layer.weight, args.moe_top_k, args.moe_normalize_expert_weights or 0)
+        if FUSED_SOFTMAX_TOPK and args.moe_zloss_weight == 0 and not args.uniform_expert_assignment:
+            for node in (_LinearSoftmaxTopK, _RecordedLinearSoftmaxTopK):   # without gradients, with
+                if node.supported(x2d, self.layer, args.moe_top_k):
+                    return node.apply(x2d, self.layer.weight, args.moe_top_k, args.moe_normalize_expert_weights or 0)
         if x2d.is_cuda and x2d.dtype in (torch.bfloat16, torch.float16) and x2d.shape[0] >= 4 * _RouterLinear.PIECE_ROWS:
             logits = _RouterLinear.apply(x2d, self.layer.weight)
         else:

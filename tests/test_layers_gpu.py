@@ -291,6 +291,65 @@ def test_router_with_its_linear_layer_in_one_kernel(tokens, hidden, experts, top
     assert not r._LinearSoftmaxTopK.supported(x, layer, top_k)
 
 
+@pytest.mark.parametrize('tokens', [1, 5, 256, 257])
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize('training', [True, False])
+def test_router_chooses_alike_with_and_without_gradients(tokens, dtype, training):
+    """A forward under no_grad and the one that records gradients give the same bits on both sides of the one-kernel limit (256
+    tokens), and the recorded one is differentiated as router.py:96-106 is by autograd, up to the rounding of its steps."""
+    from megablocks_amd.layers.arguments import Arguments
+    from megablocks_amd.layers.router import LearnedRouter
+    torch.manual_seed(tokens)
+    hidden, experts, top_k = 2048, 64, 6
+    args = Arguments(hidden_size=hidden, ffn_hidden_size=hidden, moe_num_experts=experts, moe_top_k=top_k, device='cuda',
+                     moe_normalize_expert_weights=1, bf16=dtype == torch.bfloat16, fp16=dtype == torch.float16)
+    router = LearnedRouter(args).train(training)
+    for _ in range(8 if tokens > 5 else 200):   # a logit in some ten thousand depends on the order of its sum
+        x = torch.randn(tokens, hidden, device='cuda').to(dtype).requires_grad_(True)
+        with torch.no_grad():
+            without = router(x)
+        scores, weights, indices = router(x)
+        for a, b in zip(without, (scores, weights, indices)):
+            assert torch.equal(a, b.detach())
+    gs, gw = torch.randn_like(scores), torch.randn_like(weights)
+    torch.autograd.backward([scores, weights], [gs, gw])
+    x32 = x.detach().float().requires_grad_(True)
+    w32 = router.layer.weight.detach().float().requires_grad_(True)
+    s32 = (x32 @ w32.t()).softmax(-1)
+    p32 = s32.gather(1, indices)
+    torch.autograd.backward([s32, p32 / p32.norm(p=1, dim=-1, keepdim=True)], [gs.float(), gw.float()])
+    assert router.layer.weight.grad.dtype == dtype
+    tol = 2e-2 if dtype == torch.bfloat16 else 5e-3   # scores and the logits' gradient are rounded to 16 bits on the way
+    assert rel_err(x.grad, x32.grad) < tol and rel_err(router.layer.weight.grad, w32.grad) < tol
+
+
+@pytest.mark.parametrize('tokens', [16, 200])
+def test_dmoe_under_reentrant_checkpointing_gives_the_plain_steps_gradients(tokens):
+    """Re-entrant activation checkpointing runs the forward without gradients and once more with them: every gradient and the
+    output equal those of the plain step, bit for bit."""
+    from torch.utils.checkpoint import checkpoint
+
+    from megablocks_amd.layers.arguments import Arguments
+    from megablocks_amd.layers.dmoe import dMoE
+    torch.manual_seed(tokens)
+    args = Arguments(hidden_size=2048, ffn_hidden_size=128, moe_num_experts=64, moe_top_k=6, device='cuda', mlp_type='glu',
+                     mlp_impl='grouped', activation_fn=F.silu, moe_normalize_expert_weights=1, moe_loss_weight=0.0, bias=False, fp16=False, bf16=True,
+                     init_method=partial(torch.nn.init.normal_, std=0.05))
+    layer = dMoE(args)
+
+    def step(run):
+        layer.zero_grad(set_to_none=True)
+        xr = x.clone().requires_grad_(True)
+        out = run(xr)
+        out.backward(grad)
+        return [out.detach(), xr.grad] + [p.grad for p in layer.parameters()]
+    for _ in range(4096 // tokens):
+        x = torch.randn(tokens, 1, 2048, device='cuda', dtype=torch.bfloat16)
+        grad = torch.randn_like(x)
+        for a, b in zip(step(layer), step(lambda t: checkpoint(layer, t, use_reentrant=True))):
+            assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize('tokens,experts,top_k', [(1, 1, 1), (300, 8, 2), (257, 64, 1), (200, 65, 6), (100, 128, 8),
                                                   (50, 512, 64), (1000, 16, 4)])
 @pytest.mark.parametrize('norm_p', [0, 1, 2, 3.0])
