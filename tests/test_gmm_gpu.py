@@ -618,6 +618,42 @@ def test_gmm_with_activation_epilogues(gg, groups, rows, k, n, dtype):
         gg.gmm_act(a, b[:, :, :k - 8].contiguous(), sizes)
 
 
+@pytest.mark.parametrize('k', [64, 72])
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])
+def test_gelu_epilogues_on_every_16_bit_value(gg, dtype, k):
+    """gelu_tanh and its derivative in the epilogues at every finite 16-bit value of the pre-activation (the product itself is
+    exactly 1, or the value): finite wherever the separate pass is, within a rounding step of the function in fp64, and
+    no more of them off the nearest 16-bit value than the separate pass has."""
+    x = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(dtype).cuda()
+    x = torch.where(torch.isfinite(x), x, torch.zeros_like(x)).view(256, 256)
+    x64 = x.double()
+    u = math.sqrt(2 / math.pi) * (x64 + 0.044715 * x64 ** 3)
+    q = 2 * math.sqrt(2 / math.pi) * (1 + 3 * 0.044715 * x64 ** 2)
+    tail = x64.abs() > 40     # there the derivative is 0 or 1 in any type
+    want_grad = torch.where(tail, (x64 > 0).double(), torch.sigmoid(2 * u) * (1 + x64 * torch.sigmoid(-2 * u) * q))
+    ones, rows = torch.zeros(256, k, device='cuda', dtype=dtype), torch.tensor([256], device='cuda')
+    ones[:, 0] = 1
+    values = torch.zeros(256, 256, k, device='cuda', dtype=dtype)
+    values[:, :, 0] = x
+    # a sigmoid below the normal fp32 range (2^-126) counts as zero; the derivative's other factor is below 2^8 there
+    step, least = torch.finfo(dtype).eps, max(torch.finfo(dtype).tiny * torch.finfo(dtype).eps, 2.0 ** -118)
+
+    def check(got, separate, want):
+        there = torch.isfinite(separate) & torch.isfinite(want.to(dtype))
+        assert bool(torch.isfinite(got[there]).all())
+        d = (got[there].double() - want[there]).abs()
+        # one step of the result; of 1 where the derivative crosses zero (its two terms are rounded in fp32: 2^-22 each)
+        assert bool((d <= step * want[there].abs() + torch.clamp(2.0 ** -21 * (x64[there].abs() < 2), min=least)).all())
+        assert int((got[there] != want[there].to(dtype)).sum()) <= int((separate[there] != want[there].to(dtype)).sum())
+    dact = [gg.gmm_dact(ones, ones[None], x, rows, fuse=fuse) for fuse in (True, False)]
+    check(*dact, want_grad)
+    one = torch.ones_like(x)
+    dglu = [gg.gmm_dglu(ones, ones[None], x, one, rows, 1, fuse=fuse) for fuse in (True, False)]
+    check(dglu[0][0], dglu[1][0], want_grad)
+    each = torch.ones(256, dtype=torch.int64, device='cuda')
+    check(gg.gmm_act(ones, values, each, fuse=True)[1], gg.gmm_act(ones, values, each, fuse=False)[1], x64 * torch.sigmoid(2 * u))
+
+
 @pytest.mark.parametrize('groups,rows,k,n', EPILOGUE)
 @pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16, torch.float32])
 @pytest.mark.parametrize('act', [0, 1], ids=['silu', 'gelu_tanh'])
