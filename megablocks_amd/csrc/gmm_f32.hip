@@ -429,7 +429,9 @@ gmm_f32_rows_kernel(const float* __restrict__ a, const float* __restrict__ b, fl
     int e, start, end, tm, tn;
     tiles.find(id, e, start, end, tm, tn);
     const int row0 = start + tm * BM;
-    const uint32_t a_bytes = clip_bytes((rows - row0) * k * 4), b_bytes = (uint32_t)((int64_t)k * n * 4);
+    // up to the expert's last row: the next expert's rows, or rows behind the last bin that nobody may have written, must not
+    // have a say in which instruction forms these sums
+    const uint32_t a_bytes = clip_bytes((int64_t)(end - row0) * k * 4), b_bytes = (uint32_t)((int64_t)k * n * 4);
     g.rsrc_a = make_rsrc(a + (int64_t)row0 * k, a_bytes);
     g.rsrc_b = make_rsrc(b + (int64_t)e * k * n, b_bytes);
     g.rsrc_a2 = DUAL ? make_rsrc(a2 + (int64_t)row0 * k, a_bytes) : g.rsrc_a;

@@ -980,6 +980,28 @@ def test_gmm_fp32_on_the_matrix_cores(gg, monkeypatch, groups, rows, k, n, mode)
         assert torch.equal(got[-1].nan_to_num(), got[-2].nan_to_num())
 
 
+@pytest.mark.parametrize('other', [float('inf'), float('nan'), 2.0 ** 40, 2.0 ** -80])
+@pytest.mark.parametrize('mode', ['nn', 'nt', 'dual_nn', 'dual_nt'])
+def test_gmm_fp32_rows_do_not_depend_on_the_rows_behind_them(gg, mode, other):
+    """An expert's rows give the same bits whatever the next expert's rows, and rows behind the last bin, hold: a row tile
+    reaches past the rows it belongs to (70 and 200 rows; tiles of 64 and 128)."""
+    torch.manual_seed(3)
+    k, n, trans_b, dual = 512, 260, mode.endswith('nt'), mode.startswith('dual')
+    for first, second, behind in ((70, 50, 40), (400, 300, 100)):
+        a, a2 = (torch.randn(first + second + behind, k, device='cuda') for _ in range(2))
+        b, b2 = (torch.randn((2, n, k) if trans_b else (2, k, n), device='cuda') for _ in range(2))
+        sizes = torch.tensor([first, second], device='cuda')     # on the device: their sum need not be the row count
+
+        def product(x, x2):
+            return gg.gmm_dual(x, b, x2, b2, sizes, trans_b=trans_b) if dual else gg.backend.gmm(x, b, sizes, trans_b=trans_b)
+        want = product(a, a2)[:first + second]
+        x, x2 = a.clone(), a2.clone()
+        x[first + second:], x2[first + second:] = other, other
+        assert torch.equal(product(x, x2)[:first + second], want)
+        x[first:], x2[first:] = other, other
+        assert torch.equal(product(x, x2)[:first], want[:first])
+
+
 @pytest.mark.parametrize('k', [36, 64, 2052])
 @pytest.mark.parametrize('mode', ['nn', 'nt', 'tn'])
 def test_gmm_fp32_at_the_ends_of_the_range(gg, k, mode):
