@@ -292,33 +292,98 @@ __device__ __forceinline__ void clear(Acc<BM>& acc) {
     for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 }
 
-// acc = A_tile * B_tile over K tiles [g.kt0, g.kt1), on the split operands; where a sum comes out infinite, NaN or of a
-// magnitude below kTiny, or an operand is kHuge or more, a second time on the fp32 instruction, which takes such operands as
-// they are.  The splitting of an infinity, or of a value that rounds to one, leaves NaN parts, so no such sum stays
-// unnoticed.  Parts of a value below 2^-102 can fall below the normal range: next to operands below kHuge its products are
-// below kTiny, and what they lose (2^-134 of the value, 2^-96 of a product) is 2^-32 of any sum that stays.
+// Whether one of the values a tile multiplies over K tiles [g.kt0, g.kt1) is so small that its parts lose some of it, zeros
+// apart.  Values of the same operand beyond the tile's last column count along.
+constexpr float kSmall = 0x1p-102f;
+
+template <bool MC, int R, bool DUAL>   // R: rows (KC) of the tile
+__device__ __forceinline__ bool any_small(const Args& g, const __amdgpu_buffer_rsrc_t& first, const __amdgpu_buffer_rsrc_t& second, int r0, uint32_t ld) {
+  // KC: eight lanes a row of 32 k;  MC: 32 lanes a row of 128 columns
+  const int t = threadIdx.x, piece = MC ? t % 32 : t % 8, row = MC ? t / 32 : t / 8;
+  constexpr int kStep = MC ? kThreads / 32 : kThreads / 8, kRows = MC ? kBK : R;
+  constexpr int kLoads = kRows / kStep, kAhead = 16 / kLoads;   // loads per K tile, K tiles under way
+  uint32_t smallest = 0xffffffffu;   // of the magnitudes as integers; less one, which leaves zeros out
+  for (int kt0 = g.kt0; kt0 < g.kt1; kt0 += kAhead) {
+    u32x4 v[kAhead][kLoads];
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) {
+      const int kt = kt0 + u;
+      const bool other = DUAL && kt >= g.nk1;
+      const int kk = (other ? kt - g.nk1 : kt) * kBK;
+      // a piece past the end of the reduction, a K tile past the last: zeros
+      const uint32_t past = kt < g.kt1 && (MC || kk + 4 * piece < g.k) ? 0u : 0x80000000u;
+#pragma unroll
+      for (int q = 0; q < kLoads; ++q) {
+        const uint32_t at = MC ? (uint32_t)(kk + row + q * kStep) * ld + (uint32_t)r0 * 4u + (uint32_t)piece * 16u
+                               : (uint32_t)(r0 + row + q * kStep) * ld + (uint32_t)(kk + 4 * piece) * 4u;
+        v[u][q] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(other ? second : first, (int)(at | past), 0, 0));
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u)
+#pragma unroll
+      for (int q = 0; q < kLoads; ++q)
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+          const uint32_t m = (v[u][q][w] & 0x7fffffffu) - 1u;
+          smallest = smallest < m ? smallest : m;
+        }
+  }
+  return smallest < __float_as_uint(kSmall) - 1u;
+}
+
+// acc = A_tile * B_tile over K tiles [g.kt0, g.kt1), on the split operands; a second time on the fp32 instruction, which takes
+// every value as it is, where
+//   * a sum comes out infinite, NaN or of a magnitude below kTiny, or an operand is kHuge or more.  The splitting of an
+//     infinity, or of a value that rounds to one, leaves NaN parts, so no such sum stays unnoticed.  Parts of a value below
+//     kSmall can fall below the normal range: next to operands below kHuge its products are below kTiny, and what they
+//     lose (2^-134 of the value, 2^-96 of a product) is 2^-32 of any sum that stays;
+//   * a sum comes out zero and the tile has such a value, whose parts may all have been zero.  Zero sums are common (rows that
+//     pad an expert), so the values are looked at before the tile is repeated.
+// Of the sums only those that are stored count: rows below m_lim, columns below n_lim.
 constexpr float kTiny = 0x1p-64f, kHuge = 0x1p38f;
 
 template <bool A_MC, bool B_MC, int BM, bool DUAL>
-__device__ __forceinline__ void multiply(const Args& g, Acc<BM>& acc, char* lds) {
+__device__ __forceinline__ void multiply(const Args& g, Acc<BM>& acc, int m_lim, int n_lim, char* lds) {
   clear<BM>(acc);
   float operand = 0.f;
   multiply_as<A_MC, B_MC, BM, DUAL, false>(g, acc, lds, operand);
-  uint32_t largest = 0, smallest = 0xffffffffu;   // of the magnitudes as integers; less one, which leaves zeros out
+  const int wave = threadIdx.x / kWave, lane = lane_id();
+  const int m0 = (wave / 2) * (BM / 2) + (lane & 15), n0 = (wave % 2) * 64 + 4 * (lane >> 4);
+  // twice the bits less one: no sign, zeros at the top; whether there is anything to look at more closely
+  uint32_t low = 0xffffffffu, high = 0;
 #pragma unroll
   for (int i = 0; i < BM / 32; ++i)
 #pragma unroll
     for (int j = 0; j < 4; ++j)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const uint32_t u = __float_as_uint(acc[i][j][r]) & 0x7fffffffu;
-        largest = largest > u ? largest : u;
-        smallest = smallest < u - 1u ? smallest : u - 1u;
+        const uint32_t t = __float_as_uint(acc[i][j][r]) * 2u - 1u;
+        low = low < t ? low : t;
+        high = high > t ? high : t;
       }
-  const bool again = operand >= kHuge || largest >= 0x7f800000u || smallest < __float_as_uint(kTiny) - 1u;
-  if (__syncthreads_or(again)) {
-    clear<BM>(acc);
-    multiply_as<A_MC, B_MC, BM, DUAL, true>(g, acc, lds, operand);
+  bool again = operand >= kHuge, zero = false;
+  if (low < 2u * __float_as_uint(kTiny) - 1u || high >= 2u * 0x7f800000u - 1u) {
+#pragma unroll
+    for (int i = 0; i < BM / 32; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const bool stored = m0 + 16 * i < m_lim && n0 + 16 * j < n_lim;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const float v = fabsf(acc[i][j][r]);
+          again |= stored && v != 0.f && !(v >= kTiny && v < INFINITY);
+          zero |= stored && v == 0.f;
+        }
+      }
+  }
+  if (__syncthreads_or(again || zero)) {
+    if (__syncthreads_or(zero))
+      again |= any_small<A_MC, BM, DUAL>(g, g.rsrc_a, g.rsrc_a2, g.a_r0, g.a_ld) || any_small<B_MC, 128, DUAL>(g, g.rsrc_b, g.rsrc_b2, g.b_r0, g.b_ld);
+    if (__syncthreads_or(again)) {
+      clear<BM>(acc);
+      multiply_as<A_MC, B_MC, BM, DUAL, true>(g, acc, lds, operand);
+    }
   }
 }
 
@@ -440,7 +505,7 @@ gmm_f32_rows_kernel(const float* __restrict__ a, const float* __restrict__ b, fl
     g.kt0 = cut ? (int)((int64_t)part * nk / ksplit) : 0;
     g.kt1 = cut ? (int)((int64_t)(part + 1) * nk / ksplit) : nk;
     Acc<BM> acc;
-    multiply<false, B_MC, BM, DUAL>(g, acc, lds);
+    multiply<false, B_MC, BM, DUAL>(g, acc, end - row0, n - g.b_r0, lds);
     if (!cut || join_parts<BM>(acc, id - full_rounds * P, rest, part, ksplit, ws_counters, ws_parts, lds))
       store<BM>(acc, c + (int64_t)row0 * n, n, end - row0, g.b_r0, n);
     tile_done();
@@ -495,7 +560,7 @@ gmm_f32_tn_kernel(const float* __restrict__ a, const float* __restrict__ b, floa
   g.kt0 = (int)((int64_t)part * nk / ksplit);
   g.kt1 = (int)((int64_t)(part + 1) * nk / ksplit);
   Acc<128> acc;
-  multiply<true, true, 128, false>(g, acc, lds);
+  multiply<true, true, 128, false>(g, acc, k - g.a_r0, n - g.b_r0, lds);
   if (ksplit > 1 && !join_parts<128>(acc, tile, total, part, ksplit, ws_counters, ws_parts, lds)) return;
   store<128>(acc, c + ((int64_t)e * k + g.a_r0) * n, n, k - g.a_r0, g.b_r0, n);
 }

@@ -1065,6 +1065,47 @@ def test_captures_have_workspaces_of_their_own(gg, dtype, mode):
             assert all(torch.equal(out, want) for out in (*outs[i], eager))
 
 
+@pytest.mark.parametrize('small,large', [(-128, 20), (-136, 30), (-149, 37), (-140, 100)])
+@pytest.mark.parametrize('mode', ['nn', 'nt', 'tn', 'dual_nn', 'dual_nt'])
+def test_gmm_fp32_of_values_without_bf16_parts(gg, mode, small, large):
+    """Values below the smallest bf16 value, whose three parts are all zero, times large ones, in either operand, among rows
+    of zeros: the sums, far inside the fp32 range, come out of the values themselves.  Bound of a sum of k terms, with a
+    factor of four to spare."""
+    torch.manual_seed(-small)
+    rows, k, n, trans_b, dual = 200, 68, 132, mode.endswith('nt'), mode.startswith('dual')
+    tiny = (torch.rand(rows, k, device='cuda', dtype=torch.float64) + 1) * 2.0 ** small
+    tiny = tiny.float()
+    tiny[rows // 2:rows // 2 + 20] = 0
+    big = (torch.rand(rows, n, device='cuda') + 1) * 2.0 ** large if mode == 'tn' else (torch.rand(1, k, n, device='cuda') + 1) * 2.0 ** large
+    sizes = torch.tensor([rows])
+    tol = 4 * 2.0 ** -24 * math.sqrt(2 * (rows if mode == 'tn' else k))
+
+    def product(x, w):
+        if mode == 'tn':
+            return gg.backend.gmm(x, w, sizes, trans_a=True)[0]
+        w = w.transpose(1, 2).contiguous() if trans_b else w
+        return gg.gmm_dual(x, w, x, w, sizes, trans_b=trans_b) if dual else gg.backend.gmm(x, w, sizes, trans_b=trans_b)
+
+    def exact(x, w):
+        return x.double().t() @ w.double() if mode == 'tn' else (2 if dual else 1) * (x.double() @ w[0].double())
+
+    def check(x, w):
+        want, got = exact(x, w), product(x, w).double()
+        assert float((got - want).norm() / want.norm()) < tol + 2.0 ** -149 / float(want.abs().max())
+        assert bool((got[want == 0] == 0).all())
+    check(tiny, big)
+    if mode == 'tn':
+        check(big, tiny)
+    else:   # the other way round: rows of large values, tiny weights
+        check((torch.rand(rows, k, device='cuda') + 1) * 2.0 ** large, (tiny[:k, :1].expand(k, n) * 1.0).unsqueeze(0).contiguous())
+    # next to values of ordinary size in the same tile, a row and a column of them
+    x, w = torch.randn_like(tiny), big.clone()
+    if mode != 'tn':
+        x[3] = tiny[3]
+        got, want = product(x, w).double(), exact(x, w)
+        assert float((got[3] - want[3]).norm() / want[3].norm()) < tol
+
+
 @pytest.mark.parametrize('power', [37, 110, 126])
 @pytest.mark.parametrize('mode', ['nn', 'nt', 'tn'])
 def test_gmm_fp32_of_small_by_large_values(gg, mode, power):
