@@ -9,10 +9,12 @@
 // alignment; 195 TFLOP/s on 4096^3 against 141.  Half the conversion instructions (v_dot2c_f32_bf16) changed nothing;
 // cutting the parts off instead of rounding them is 3 % faster and up to a third less exact.
 //
-// How exact: the parts leave 2^-27 of a value, the three products not taken 2^-26 of a product, and an accumulator is rounded six
-// times per 32 k instead of 32 times.  Relative error (2-norm) against fp64: 4.8e-7 over k = 1024, 9.8e-7 over 4096, where
-// a chain of fp32 fused multiply-adds shows 5.7e-7 and 1.15e-6.  Sums that the parts do not serve (infinities, NaN, values
-// next to the largest or the smallest) are formed again on the fp32 instruction: multiply().
+// How exact: three parts hold all 24 bits of a value; the three products of parts not taken come to less than 2^-25 of a product,
+// and an accumulator is rounded six times per 32 k instead of 32 times.  Relative error (2-norm) against fp64: 4.8e-7 over
+// k = 1024, 9.8e-7 over 4096, where a chain of fp32 fused multiply-adds shows 5.7e-7 and 1.15e-6; 3.4e-8 over eight terms (5.4e-8).
+// The error of a single product is larger than that chain's, up to 2.6 2^-24 of it instead of one: sums of one or two terms,
+// and those that the parts do not serve (infinities, NaN, values next to the largest or the smallest), are formed on the fp32
+// instruction: multiply().
 //
 // Tile: 128 x 128 (64 x 128 for short experts) per workgroup of four waves (2 x 2), K tiles of 32, two stages of
 // 32 KiB, so two workgroups share a compute unit and one multiplies while the other converts, waits at its barrier or
@@ -332,8 +334,8 @@ __device__ __forceinline__ bool any_small(const Args& g, const __amdgpu_buffer_r
   return smallest < __float_as_uint(kSmall) - 1u;
 }
 
-// acc = A_tile * B_tile over K tiles [g.kt0, g.kt1), on the split operands; a second time on the fp32 instruction, which takes
-// every value as it is, where
+// acc = A_tile * B_tile over K tiles [g.kt0, g.kt1), on the split operands (multiply()); a second time on the fp32 instruction,
+// which takes every value as it is, where
 //   * a sum comes out infinite, NaN or of a magnitude below kTiny, or an operand is kHuge or more.  The splitting of an
 //     infinity, or of a value that rounds to one, leaves NaN parts, so no such sum stays unnoticed.  Parts of a value below
 //     kSmall can fall below the normal range: next to operands below kHuge its products are below kTiny, and what they
@@ -344,10 +346,7 @@ __device__ __forceinline__ bool any_small(const Args& g, const __amdgpu_buffer_r
 constexpr float kTiny = 0x1p-64f, kHuge = 0x1p38f;
 
 template <bool A_MC, bool B_MC, int BM, bool DUAL>
-__device__ __forceinline__ void multiply(const Args& g, Acc<BM>& acc, int m_lim, int n_lim, char* lds) {
-  clear<BM>(acc);
-  float operand = 0.f;
-  multiply_as<A_MC, B_MC, BM, DUAL, false>(g, acc, lds, operand);
+__device__ __forceinline__ bool sums_need_fp32(const Args& g, const Acc<BM>& acc, float operand, int m_lim, int n_lim) {
   const int wave = threadIdx.x / kWave, lane = lane_id();
   const int m0 = (wave / 2) * (BM / 2) + (lane & 15), n0 = (wave % 2) * 64 + 4 * (lane >> 4);
   // twice the bits less one: no sign, zeros at the top; whether there is anything to look at more closely
@@ -380,11 +379,26 @@ __device__ __forceinline__ void multiply(const Args& g, Acc<BM>& acc, int m_lim,
   if (__syncthreads_or(again || zero)) {
     if (__syncthreads_or(zero))
       again |= any_small<A_MC, BM, DUAL>(g, g.rsrc_a, g.rsrc_a2, g.a_r0, g.a_ld) || any_small<B_MC, 128, DUAL>(g, g.rsrc_b, g.rsrc_b2, g.b_r0, g.b_ld);
-    if (__syncthreads_or(again)) {
-      clear<BM>(acc);
-      multiply_as<A_MC, B_MC, BM, DUAL, true>(g, acc, lds, operand);
-    }
+    return __syncthreads_or(again);
   }
+  return false;
+}
+
+// A reduction of one or two terms goes to the fp32 instruction at once: its result is rounded once or twice there, and the
+// products of parts that are left out, and what the bf16 instruction drops of a sum, are more than that (largest error over the
+// sum of the magnitudes, 2^-24: 1.0 / 2.6 over one term, 1.9 / 2.6 over two, 2.5 / 2.3 over three, 3.7 / 2.1 over eight).
+constexpr int kFewTerms = 2;
+
+template <bool A_MC, bool B_MC, int BM, bool DUAL>
+__device__ __forceinline__ void multiply(const Args& g, Acc<BM>& acc, int m_lim, int n_lim, char* lds) {
+  clear<BM>(acc);
+  float operand = 0.f;
+  if (!A_MC || g.k > kFewTerms) {   // NN / NT: k is a multiple of 4
+    multiply_as<A_MC, B_MC, BM, DUAL, false>(g, acc, lds, operand);
+    if (!sums_need_fp32<A_MC, B_MC, BM, DUAL>(g, acc, operand, m_lim, n_lim)) return;
+    clear<BM>(acc);
+  }
+  multiply_as<A_MC, B_MC, BM, DUAL, true>(g, acc, lds, operand);
 }
 
 // c[m][n] = acc for the tile's rows below m_lim and columns below n (n a multiple of 4, c 16-byte aligned)

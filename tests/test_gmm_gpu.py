@@ -1065,6 +1065,30 @@ def test_captures_have_workspaces_of_their_own(gg, dtype, mode):
             assert all(torch.equal(out, want) for out in (*outs[i], eager))
 
 
+@pytest.mark.parametrize('among', [0, 64, 300])
+def test_gmm_fp32_of_few_terms(gg, among):
+    """Weight gradients of experts with one to eight rows, by themselves and next to experts of `among` rows on average: the error
+    against fp64 is no larger than that of a chain of fp32 multiply-adds (one term: the product, rounded once)."""
+    torch.manual_seed(among)
+    k, n, terms = 260, 516, list(range(1, 9))
+    sizes = torch.tensor(terms + ([16 * among - 4] if among else []))
+    rows = int(sizes.sum())
+    a, b = torch.randn(rows, k, device='cuda'), torch.randn(rows, n, device='cuda')
+    out = gg.backend.gmm(a, b, sizes, trans_a=True)
+    start = 0
+    for e, r in enumerate(terms):
+        x, y = a[start:start + r].double(), b[start:start + r].double()
+        start += r
+        want, chain = x.t() @ y, torch.zeros(k, n, device='cuda')
+        for t in range(r):
+            chain = (chain.double() + x[t, :, None] * y[t, None, :]).float()   # exact product, one rounding
+        if r == 1:
+            assert torch.equal(out[e], chain)
+        total = x.abs().t() @ y.abs()
+        for norm in (lambda d: float(d.norm()), lambda d: float((d / total).abs().max())):
+            assert norm(out[e].double() - want) <= 1.05 * norm(chain.double() - want), (r, norm(out[e].double() - want), norm(chain.double() - want))
+
+
 @pytest.mark.parametrize('small,large', [(-128, 20), (-136, 30), (-149, 37), (-140, 100)])
 @pytest.mark.parametrize('mode', ['nn', 'nt', 'tn', 'dual_nn', 'dual_nt'])
 def test_gmm_fp32_of_values_without_bf16_parts(gg, mode, small, large):
