@@ -157,7 +157,8 @@ static inline int persistent_grid(int64_t tiles_upper_bound) {
 
 }  // namespace
 
-// gmm_f32.hip: fp32 products of whole 16-byte pieces; MBX_EUNSUPPORTED where the operands are not.  a2 / b2 non-null
+// gmm_f32.hip: fp32 products of whole 16-byte pieces; MBX_EUNSUPPORTED where the operands are not, and for TN launches with few
+// rows per expert.  a2 / b2 non-null
 // (NN / NT): c = a @ b[e] + a2 @ b2[e].
 int gmm_f32(const void* a, const void* b, const void* a2, const void* b2, void* c, const int32_t* bins, int num_groups,
             int64_t rows, int k, int n, int layout, void* workspace, size_t workspace_bytes, hipStream_t s);

@@ -590,6 +590,14 @@ static inline bool f32_ok(const void* a, const void* b, const void* c, int64_t r
   return (int64_t)k * n * 4 < lim && (int64_t)k * 4 * 128 < lim;
 }
 
+// TN launches left to gmm.hip's element-wise kernel, a chain of fp32 multiply-adds per sum: up to 24 rows per expert on average.
+// There is next to nothing to multiply, and three of its workgroups share a compute unit, which is what the stores want (us, that
+// kernel / this one; 64 experts, [1024, 4096]: 1 row 214 / 393, 16: 270 / 405, 32: 347 / 418, 64: 500 / 490;  8, [4096,
+// 4096]: 99 / 153, 123 / 153, 170 / 156, 254 / 197;  128, [768, 2048]: 162 / 211, 211 / 221, 269 / 217, 379 / 305).  The size limits are that kernel's.
+static inline bool f32_short_tn(int num_groups, int64_t rows, int k) {
+  return rows <= 24 * (int64_t)num_groups && ceil_div(k, 128) <= 65535 && num_groups <= 65535;
+}
+
 // Tiles of 64 rows up to 192 rows per expert on average: of full ones an expert of that many leaves a quarter and more of
 // the multiplications to padding, which this kernel, bound by the matrix cores, pays in full (64 experts of 100 - 156 rows,
 // 1024 x 1408: 228 us NT).
@@ -599,6 +607,7 @@ constexpr int64_t kF32ShortRows = 192;
 
 int gmm_f32(const void* a, const void* b, const void* a2, const void* b2, void* c, const int32_t* bins, int num_groups,
                    int64_t rows, int k, int n, int layout, void* workspace, size_t workspace_bytes, hipStream_t s) {
+  if (layout == MBX_TN && f32_short_tn(num_groups, rows, k)) return MBX_EUNSUPPORTED;
   if (!f32_ok(a, b, c, rows, k, n, layout) || (a2 && !f32_ok(a2, b2, c, rows, k, n, layout))) return MBX_EUNSUPPORTED;
   const float *ap = (const float*)a, *bp = (const float*)b, *ap2 = (const float*)a2, *bp2 = (const float*)b2;
   float* cp = (float*)c;
