@@ -83,6 +83,12 @@ gmm_few_kernel(const uint16_t* __restrict__ a, const uint16_t* __restrict__ b, u
     Unit u;
     int tm, tn;
     tiles.find(id, u.e, u.start, u.end, tm, tn);
+    // Eight column tiles, then the same eight with the expert's next rows: those workgroups follow on the same XCDs and find
+    // the weights in their L2s.
+    const int mt = (u.end - u.start + kRows - 1) / kRows, t = tn * mt + tm, first = t / (8 * mt) * 8, in = t - first * mt;
+    const int wide = tiles_n - first < 8 ? tiles_n - first : 8;
+    tm = in / wide;
+    tn = first + in % wide;
     u.row0 = u.start + tm * kRows;
     u.n0 = tn * kTileCols;
     return u;
@@ -267,20 +273,33 @@ int dispatch_few(const DmaCall& q) {
 }  // namespace
 
 // Up to eight rows per expert on average (beyond, experts of more than 16 rows read their weights twice: 16 rows per expert
-// cost 20 - 40 %).  NN: wherever gmm_dma.h's tiles would leave the chip partly idle.  NT: that kernel keeps up as long as
-// its rounds of tiles are about three quarters full (32 experts, [2816, 3072]: 195 against 216 us with 0.86 of them full,
-// 124 against 134 with 0.77; 25 of 64 experts, [1408, 2048]: 74 against 61 with 0.54), with short reductions, sixteen
-// chunks of which are four per wave here, longer still (16 experts, [1408, 1024]: 21 against 24 us with 0.69), and with
-// long ones it depends on where the weights lie (8 experts, [14336, 4096]: 347 - 398 against 335 us).
+// cost 20 - 40 %).
+// NN: wherever gmm_dma.h's tiles would leave the chip partly idle; with reductions of 3072 and more only up to half a round of
+// them, which that kernel does not cut into more than two parts (us, that kernel / this one, two rows per expert:
+// [14336, 4096] 8 experts 178 / 173, 9: 185 / 231, 12: 227 / 258;  [8192, 4096] 8: 104 / 115, 12: 134 / 172, 28: 311 / 400;
+// [4096, 2048] 16: 45 / 43, 24: 71 / 78;  [2816, 3072] 16: 46 / 44, 32: 112 / 103).
+// NT: that kernel keeps up as long as its rounds of tiles are about three quarters full (32 experts, [2816, 3072]: 195 against
+// 216 us with 0.86 of them full, 124 against 134 with 0.77; 25 of 64 experts, [1408, 2048]: 74 against 61 with 0.54), with
+// short reductions, sixteen chunks of which are four per wave here, longer still (16 experts, [1408, 1024]: 21 against 24 us
+// with 0.69), and with long ones it depends on where the weights lie (8 experts, [14336, 4096]: 347 - 398 against 335 us).
+// From four rows per expert on gmm_mid.hip's launches are its own: as fast with even rows, faster with skewed ones (us, this
+// kernel / that one, gated and plain, 8 rows on average, even, Zipf-distributed (exponent 1.2) and all on top_k experts: 8 experts
+// top-2, [14336, 4096]: 352, 173 / 343, 158;  376, 187 / 344, 158;  158, 81 / 94, 63;  64 top-6, [1408, 4096]: 282, 147 / 264,
+// 129;  303, 159 / 254, 122;  141, 85 / 68, 64).
+// Skewed rows where the launch stays here, against gmm_dma.h (Zipf and all on top_k, 8 rows): NN, 8 experts, [14336, 4096]: 192
+// / 215, 52 / 52;  16 top-4, [4096, 2048]: 47 / 53, 26 / 16;  32 top-2, [2816, 1024]: 34 / 35, 25 / 12;  NT gated, 16 top-2,
+// [4096, 4096]: 214 / 216, 58 / 79 (even: 227 / 203).
 // The number of experts that get rows is an expectation: rows that choose evenly.  The epilogues do not enter the rule: the
 // product of a launch with one is the plain launch's, bit for bit.
 bool gmm_few_takes(const DmaCall& q) {
   const bool nn = q.layout == MBX_NN && (q.epi == dma::kEpiNone || q.epi == dma::kEpiCombine) && !q.a2;
   const bool nt = q.layout == MBX_NT && (q.epi == dma::kEpiAct || dma::epi_is_glu(q.epi) || (q.epi == dma::kEpiNone && !q.a2));
   if (!(nn || nt) || q.rows > 8 * (int64_t)q.num_groups) return false;
+  if (nt && q.rows > 4 * (int64_t)q.num_groups && gmm_mid_takes(q)) return false;
   const double experts = q.num_groups * (1.0 - pow(1.0 - 1.0 / q.num_groups, (double)q.rows));
   const double rounds = experts * (double)ceil_div(q.n, nn ? 256 : 128) / persistent_grid((int64_t)1 << 30);
   const double filled = rounds / ceil(rounds);
+  if (nn && q.k >= 3072) return rounds <= 0.5;
   return nn ? filled < 0.92 : q.k >= 4096 || filled < (q.k >= 2048 ? 0.7 : 0.5);
 }
 

@@ -1266,6 +1266,17 @@ def test_gmm_with_a_handful_of_rows_per_expert(gg, counts, k, n, dtype):
         assert torch.equal(g[mask], gg.backend.gmm(src.materialize(), w1, sizes, trans_b=True)[mask])
 
 
+@pytest.mark.parametrize('counts,k,n', [
+    ([33, 1, 0, 70, 2, 0, 0, 1, 0, 0, 0, 0, 0, 0, 17, 4], 2048, 1096),      # columns that end inside a run of eight tiles
+    ([0] * 15 + [128], 2048, 512), ([0, 64] + [0] * 30, 2056, 72), ([7] * 8, 2816, 8448), ([56] + [0] * 7, 4096, 1032),
+    ([4] * 12, 3072, 4096), ([8, 8], 3072, 264),
+])
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])
+def test_gmm_with_a_handful_of_rows_on_average(gg, counts, k, n, dtype):
+    """The same where single experts have several row tiles of those kernels, and on both sides of the lines to the others."""
+    test_gmm_with_a_handful_of_rows_per_expert(gg, counts, k, n, dtype)
+
+
 @pytest.mark.parametrize('groups,rows,k,n', [(1, 1, 8, 8), (3, 130, 64, 256), (5, 1280, 72, 264), (8, 8 * 257, 128, 1032), (32, 4096, 192, 768)])
 @pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])
 def test_batched_mlp_with_activation_epilogues(gg, groups, rows, k, n, dtype):
