@@ -60,17 +60,17 @@ template <bool B_MC> struct Chunk;
 template <> struct Chunk<false> { u32x4 a[2], b[2][4]; };
 template <> struct Chunk<true> { u32x4 a[2]; u32x2 b[2][8]; };
 
-// EPI: dma::kEpiNone, kEpiAct, kEpiGlu* (NT), kEpiCombine (NN).  GATHER (NT): as in gmm_dma.h's gmm_rows_kernel.
-// c (with the gate: and out2) may be null where only the epilogue's output is wanted.
+// EPI: dma::kEpiNone, kEpiAct, kEpiGlu*, kEpiDact, kEpiDglu* (NT), kEpiCombine (NN).  GATHER (NT): as in gmm_dma.h's gmm_rows_kernel.
+// c (with the gate: and out2) may be null where only the epilogue's output is wanted.  a2: x2 of kEpiDglu*.
 template <int DT, bool B_MC, int EPI, bool GATHER>
 __global__ void __launch_bounds__(kThreads, 4)
 gmm_few_kernel(const uint16_t* __restrict__ a, const uint16_t* __restrict__ b, uint16_t* __restrict__ c,
                const int32_t* __restrict__ bins, int num_groups, int rows, int k, int n, int tiles_n,
-               const uint16_t* __restrict__ b2, uint16_t* __restrict__ extra, uint16_t* __restrict__ out2,
+               const uint16_t* __restrict__ a2, const uint16_t* __restrict__ b2, uint16_t* __restrict__ extra, uint16_t* __restrict__ out2,
                const int32_t* __restrict__ slots, const int32_t* __restrict__ src_bins, int top_k, int src_rows,
                const void* __restrict__ combine_weights, int combine_w_dtype, int combine_tokens) {
   __shared__ __attribute__((aligned(16))) float sums[kWaves * kRows * kPitch];
-  constexpr bool kGlu = dma::epi_is_glu(EPI);
+  constexpr bool kGlu = dma::epi_is_glu(EPI), kDglu = dma::epi_is_dglu(EPI);
   constexpr int kTileCols = kGlu ? kCols / 2 : kCols;
   const dma::RowTiles<kRows> tiles(bins, num_groups, tiles_n, rows, false, 8);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = lane_id(), col = lane & 15, g = lane >> 4;
@@ -192,50 +192,62 @@ gmm_few_kernel(const uint16_t* __restrict__ a, const uint16_t* __restrict__ b, u
     multiply(x1);
     __builtin_amdgcn_sched_barrier(0);
   }
-    // partial sums: sums[wave][row][column]
+  constexpr int kItems = kTileCols / 8;
+  const int m = threadIdx.x / kItems, ch8 = threadIdx.x % kItems, row = cur.row0 + m, cn = cur.n0 + ch8 * 8;
+  const bool mine = m < kRows && row < cur.end && cn < n;   // n is a multiple of 8
+  const int64_t at = (int64_t)row * n + cn;
+  u32x4 in1 = {0u, 0u, 0u, 0u}, in2 = in1;   // the epilogue's inputs, under way while the sums meet
+  if constexpr (EPI == dma::kEpiDact || kDglu)
+    if (mine) in1 = *(const u32x4*)(extra + at);
+  if constexpr (kDglu)
+    if (mine) in2 = *(const u32x4*)(a2 + at);
+  // partial sums: sums[wave][row][column]
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      // NT: fragment q, columns 16 q + 4 g + r.  NN: register q of the four fragments, columns 4 (4 g + q) + f.
-      f32x4 v;
-      if constexpr (B_MC) {
+  for (int q = 0; q < 4; ++q) {
+    // NT: fragment q, columns 16 q + 4 g + r.  NN: register q of the four fragments, columns 4 (4 g + q) + f.
+    f32x4 v;
+    if constexpr (B_MC) {
 #pragma unroll
-        for (int f = 0; f < 4; ++f) v[f] = acc[f][q];
-      } else {
-        v = acc[q];
-      }
-      *(f32x4*)(sums + (size_t)(wave * kRows + col) * kPitch + (B_MC ? 16 * g + 4 * q : 16 * q + 4 * g)) = v;
+      for (int f = 0; f < 4; ++f) v[f] = acc[f][q];
+    } else {
+      v = acc[q];
     }
-    __syncthreads();
-    constexpr int kItems = kTileCols / 8;
-    const int m = threadIdx.x / kItems, ch8 = threadIdx.x % kItems, row = cur.row0 + m, cn = cur.n0 + ch8 * 8;
-    if (m < kRows && row < cur.end && cn < n) {   // n is a multiple of 8
-      const int64_t at = (int64_t)row * n + cn;
-      float f[8];
-      total(m, ch8, f);
-      const u32x4 v = dma::pack8<DT>(f);
-      if constexpr (kGlu) {
-        total(m, ch8 + kItems, f);
-        const u32x4 v2 = dma::pack8<DT>(f);
-        if (c != nullptr) {
-          *(u32x4*)(c + at) = v;
-          *(u32x4*)(out2 + at) = v2;
-        }
-        *(u32x4*)(extra + at) = dma::glu_chunk<DT, EPI == dma::kEpiGluGelu>(v, v2);
-      } else {
-        if (c != nullptr) *(u32x4*)(c + at) = v;
-        if constexpr (EPI == dma::kEpiAct) *(u32x4*)(extra + at) = dma::gelu_fwd_chunk<DT>(v);
-        if constexpr (EPI == dma::kEpiCombine) {
-          dma::Combine cb;
-          cb.weights = combine_weights;
-          cb.w_dtype = combine_w_dtype;
-          cb.tokens = combine_tokens;
-          cb.token = slots[row];
-          cb.row_exists = true;
-          const int token = dma::combine_token(cb);
-          if (token >= 0) *(u32x4*)(extra + (int64_t)token * n + cn) = dma::scale_chunk<DT>(v, dma::combine_weight(cb, token));
-        }
-      }
+    *(f32x4*)(sums + (size_t)(wave * kRows + col) * kPitch + (B_MC ? 16 * g + 4 * q : 16 * q + 4 * g)) = v;
+  }
+  __syncthreads();
+  if (!mine) return;
+  float f[8];
+  total(m, ch8, f);
+  const u32x4 v = dma::pack8<DT>(f);
+  if constexpr (kGlu) {
+    total(m, ch8 + kItems, f);
+    const u32x4 v2 = dma::pack8<DT>(f);
+    if (c != nullptr) {
+      *(u32x4*)(c + at) = v;
+      *(u32x4*)(out2 + at) = v2;
     }
+    *(u32x4*)(extra + at) = dma::glu_chunk<DT, EPI == dma::kEpiGluGelu>(v, v2);
+  } else if constexpr (kDglu) {
+    u32x4 d1, d2;
+    dma::dglu_chunk<DT, EPI == dma::kEpiDgluGelu>(v, in1, in2, d1, d2);
+    *(u32x4*)(c + at) = d1;
+    *(u32x4*)(out2 + at) = d2;
+  } else if constexpr (EPI == dma::kEpiDact) {
+    *(u32x4*)(c + at) = dma::gelu_bwd_chunk<DT>(v, in1);
+  } else {
+    if (c != nullptr) *(u32x4*)(c + at) = v;
+    if constexpr (EPI == dma::kEpiAct) *(u32x4*)(extra + at) = dma::gelu_fwd_chunk<DT>(v);
+    if constexpr (EPI == dma::kEpiCombine) {
+      dma::Combine cb;
+      cb.weights = combine_weights;
+      cb.w_dtype = combine_w_dtype;
+      cb.tokens = combine_tokens;
+      cb.token = slots[row];
+      cb.row_exists = true;
+      const int token = dma::combine_token(cb);
+      if (token >= 0) *(u32x4*)(extra + (int64_t)token * n + cn) = dma::scale_chunk<DT>(v, dma::combine_weight(cb, token));
+    }
+  }
 }
 
 }  // namespace few
@@ -249,7 +261,7 @@ int launch_few(const DmaCall& q, const int32_t* slots) {
   if (row_tiles * tiles_n > 0x7fffffff) return MBX_ERANGE;
   few::gmm_few_kernel<DT, B_MC, EPI, GATHER><<<(unsigned)(row_tiles * tiles_n), few::kThreads, 0, q.stream>>>(
       (const uint16_t*)q.a, (const uint16_t*)q.b, (uint16_t*)q.c, q.bins, q.num_groups, (int)q.rows, q.k, q.n, tiles_n,
-      (const uint16_t*)q.b2, (uint16_t*)q.extra, (uint16_t*)q.out2, slots, q.gather.src_bins, q.gather.top_k, q.gather.src_rows,
+      (const uint16_t*)q.a2, (const uint16_t*)q.b2, (uint16_t*)q.extra, (uint16_t*)q.out2, slots, q.gather.src_bins, q.gather.top_k, q.gather.src_rows,
       q.combine.weights, q.combine.w_dtype, q.combine.tokens);
   return launch_status();
 }
@@ -258,6 +270,7 @@ template <int DT>
 int dispatch_few(const DmaCall& q) {
   if (q.layout == MBX_NN) {
     if (q.epi == dma::kEpiCombine) return launch_few<DT, true, dma::kEpiCombine, false>(q, q.combine.indices);
+    if (q.epi == dma::kEpiAct) return launch_few<DT, true, dma::kEpiAct, false>(q, nullptr);
     return launch_few<DT, true, dma::kEpiNone, false>(q, nullptr);
   }
 #define MBX_FEW_NT(EPI) (q.gather.slots ? launch_few<DT, false, EPI, true>(q, q.gather.slots) : launch_few<DT, false, EPI, false>(q, nullptr))
@@ -265,7 +278,10 @@ int dispatch_few(const DmaCall& q) {
     case dma::kEpiNone: return MBX_FEW_NT(dma::kEpiNone);
     case dma::kEpiAct: return MBX_FEW_NT(dma::kEpiAct);
     case dma::kEpiGluSilu: return MBX_FEW_NT(dma::kEpiGluSilu);
-    default: return MBX_FEW_NT(dma::kEpiGluGelu);
+    case dma::kEpiGluGelu: return MBX_FEW_NT(dma::kEpiGluGelu);
+    case dma::kEpiDact: return launch_few<DT, false, dma::kEpiDact, false>(q, nullptr);
+    case dma::kEpiDgluSilu: return launch_few<DT, false, dma::kEpiDgluSilu, false>(q, nullptr);
+    default: return launch_few<DT, false, dma::kEpiDgluGelu, false>(q, nullptr);
   }
 #undef MBX_FEW_NT
 }
@@ -292,9 +308,8 @@ int dispatch_few(const DmaCall& q) {
 // The number of experts that get rows is an expectation: rows that choose evenly.  The epilogues do not enter the rule: the
 // product of a launch with one is the plain launch's, bit for bit.
 bool gmm_few_takes(const DmaCall& q) {
-  const bool nn = q.layout == MBX_NN && (q.epi == dma::kEpiNone || q.epi == dma::kEpiCombine) && !q.a2;
-  const bool nt = q.layout == MBX_NT && (q.epi == dma::kEpiAct || dma::epi_is_glu(q.epi) || (q.epi == dma::kEpiNone && !q.a2));
-  if (!(nn || nt) || q.rows > 8 * (int64_t)q.num_groups) return false;
+  const bool nn = q.layout == MBX_NN, nt = q.layout == MBX_NT;
+  if (!(nn || nt) || (q.a2 && !dma::epi_is_dglu(q.epi)) || q.rows > 8 * (int64_t)q.num_groups) return false;
   if (nt && q.rows > 4 * (int64_t)q.num_groups && gmm_mid_takes(q)) return false;
   const double experts = q.num_groups * (1.0 - pow(1.0 - 1.0 / q.num_groups, (double)q.rows));
   const double rounds = experts * (double)ceil_div(q.n, nn ? 256 : 128) / persistent_grid((int64_t)1 << 30);

@@ -1277,6 +1277,41 @@ def test_gmm_with_a_handful_of_rows_on_average(gg, counts, k, n, dtype):
     test_gmm_with_a_handful_of_rows_per_expert(gg, counts, k, n, dtype)
 
 
+@pytest.mark.parametrize('counts,k,n', [
+    ([2] * 16, 4096, 1032), ([1, 0, 5, 4] * 8, 2048, 520), ([8] * 6, 200, 136),      # a handful of rows per expert
+    ([17, 24, 40] * 11, 264, 2056), ([130, 90, 200, 64], 136, 776), ([300] * 8, 1088, 264),
+])
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])
+def test_products_under_an_epilogue_are_the_plain_ones(gg, monkeypatch, counts, k, n, dtype):
+    """Every epilogue is applied to the product the plain launch forms, bit for bit, whichever kernel takes the sizes:
+    with activations where the derivative is 1 (gelu_tanh and SiLU far to the right) the gradient forms show it too."""
+    torch.manual_seed(n)
+    monkeypatch.setattr(gg, 'GMM_WORKSPACE', False)      # lent memory would let plain NN launches cut their last tiles
+    sizes = torch.tensor(counts)
+    groups, rows = len(counts), int(sizes.sum())
+    sizes = sizes.cuda()
+    a = torch.randn(rows, k, device='cuda').to(dtype)
+    w, v = ((torch.randn(groups, n, k, device='cuda') / k ** 0.5).to(dtype) for _ in range(2))
+    plain, plain_v = gg.backend.gmm(a, w, sizes, trans_b=True), gg.backend.gmm(a, v, sizes, trans_b=True)
+    right = torch.full((rows, n), 32.0, device='cuda', dtype=dtype)
+    assert torch.equal(gg.gmm_act(a, w, sizes, fuse=True)[0], plain)
+    assert torch.equal(gg.gmm_dact(a, w, right, sizes, fuse=True), plain)
+    for code in (0, 1):
+        x1, x2, _ = gg.gmm_glu(a, w, v, sizes, code, fuse=True)
+        assert torch.equal(x1, plain) and torch.equal(x2, plain_v)
+        d1, d2 = gg.gmm_dglu(a, w, right, torch.full_like(right, 0.5), sizes, code, fuse=True)
+        assert torch.equal(d1, plain * 0.5) and torch.equal(d2, plain * 32)
+    wn = w.transpose(1, 2).contiguous()
+    nn = gg.backend.gmm(a, wn, sizes)
+    pre, act = gg.gmm_act(a, wn, sizes, fuse=True, trans_b=False)
+    assert torch.equal(pre, nn)
+    assert rel_err(act, torch.nn.functional.gelu(pre.float(), approximate='tanh')) < 4e-3     # one rounding step
+    order = torch.arange(rows, device='cuda').int()
+    bin_ids = torch.repeat_interleave(torch.arange(groups, device='cuda'), sizes).int()
+    y, _ = gg.gmm_scatter(a, wn, sizes, gg.CombinedRows(order, bin_ids, torch.cumsum(sizes, 0).int(), None))
+    assert torch.equal(y, nn)
+
+
 @pytest.mark.parametrize('groups,rows,k,n', [(1, 1, 8, 8), (3, 130, 64, 256), (5, 1280, 72, 264), (8, 8 * 257, 128, 1032), (32, 4096, 192, 768)])
 @pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])
 def test_batched_mlp_with_activation_epilogues(gg, groups, rows, k, n, dtype):
