@@ -337,12 +337,47 @@ def operand_pattern_leg(w, inp):
     return res
 
 
+def tile_phases(t):
+    """tile_ticks_leg's figures of one launch from its stamps t [workgroups, tiles of a workgroup, stamps of a tile] in
+    microseconds (0: not written)."""
+    import torch
+
+    tiles = t.shape[1]
+    done = (t[:, :, 0] > 0) & (t[:, :, 1] > 0) & (t[:, :, 5] > 0)
+    n = int(done.sum())
+    if n == 0:   # a launch of kernels that stamp nothing (fp32, sizes the direct-to-LDS kernels do not take)
+        return dict(tiles=0, note='no stamped tiles')
+    phase = lambda x, y: float((t[:, :, y] - t[:, :, x])[done].mean())
+    nxt = torch.zeros_like(done)
+    nxt[:, :-1] = done[:, :-1] & done[:, 1:]
+    between = (t[:, 1:, 0] - t[:, :-1, 5])[nxt[:, :-1]]
+    start = t[:, :, 0][done].min()
+    # a workgroup's first tile has no stores of a tile before it in flight; its last one may be a part of a tile
+    # (mbx_gmm_ws: the tail of an NN launch) whose "stores" include the reduction of the parts
+    per_ordinal = {}
+    for o in range(min(tiles, 8)):
+        if int(done[:, o].sum()):
+            sel = done[:, o]
+            per_ordinal[str(o)] = [round(float((t[:, o, y] - t[:, o, x])[sel].mean()), 2) for x, y in ((0, 1), (1, 2), (2, 4))]
+    return dict(
+        tiles=n, workgroups=int(done.any(dim=1).sum()),
+        start_to_first_k_tile=round(phase(0, 1), 2),
+        of_which=dict(find_the_tile=round(phase(0, 6), 2), request_first_k_tiles=round(phase(6, 7), 2),
+                      clear_accumulators=round(phase(7, 3), 2), wait_for_first_k_tile=round(phase(3, 1), 2)),
+        main_loop=round(phase(1, 2), 2),
+        last_mfma_to_last_store_issued=round(phase(2, 4), 2), hand_over=round(phase(4, 5), 2),
+        between_tiles_of_a_workgroup=round(float(between.mean()), 2) if between.numel() else None,
+        tile_total=round(phase(0, 5), 2), by_ordinal_of_the_tile_in_its_workgroup_start_loop_store=per_ordinal,
+        first_tile_start_to_last_tile_end_ms=round(float(t[:, :, 5][done].max() - start) / 1000.0, 4))
+
+
 def tile_ticks_leg(w, inp):
     """Where the time of an output tile goes, for the three grouped products of this workload's shapes: the kernels of
     libmbx_ticks.so (the library compiled with -DMBX_TICKS; loaded instead of libmbx.so by this leg) stamp every tile
     with the constant-rate clock (100 MHz) when it starts, when its first K tile has landed, after its last MFMA, after
-    its last store has been issued and after the workgroup's LDS has been handed on.  One launch per product is read
-    back; times are microseconds per tile, averaged over the launch's tiles."""
+    its last store has been issued and after the workgroup's LDS has been handed on.  The kernels for few rows per expert
+    stamp nothing: that library leaves their launches to the stamped ones.  One launch per product is read back; times are
+    microseconds per tile, averaged over the launch's tiles."""
     import ctypes
 
     import torch
@@ -384,31 +419,8 @@ def tile_ticks_leg(w, inp):
         e1.record()
         torch.cuda.synchronize()
         _lib.check(set_ticks(None), 'set_ticks')
-        t = buf.view(workgroups, tiles, ids).cpu().double() / 100.0     # microseconds
-        done = (t[:, :, 0] > 0) & (t[:, :, 1] > 0) & (t[:, :, 5] > 0)
-        n = int(done.sum())
-        phase = lambda x, y: float((t[:, :, y] - t[:, :, x])[done].mean())
-        nxt = torch.zeros_like(done)
-        nxt[:, :-1] = done[:, :-1] & done[:, 1:]
-        between = (t[:, 1:, 0] - t[:, :-1, 5])[nxt[:, :-1]]
-        start = t[:, :, 0][done].min()
-        # a workgroup's first tile has no stores of a tile before it in flight; its last one may be a part of a tile
-        # (mbx_gmm_ws: the tail of an NN launch) whose "stores" include the reduction of the parts
-        per_ordinal = {}
-        for o in range(min(tiles, 8)):
-            if int(done[:, o].sum()):
-                sel = done[:, o]
-                per_ordinal[str(o)] = [round(float((t[:, o, y] - t[:, o, x])[sel].mean()), 2) for x, y in ((0, 1), (1, 2), (2, 4))]
-        res['products'][name] = dict(
-            launch_ms=round(e0.elapsed_time(e1), 4), tiles=n, workgroups=int(done.any(dim=1).sum()),
-            start_to_first_k_tile=round(phase(0, 1), 2),
-            of_which=dict(find_the_tile=round(phase(0, 6), 2), request_first_k_tiles=round(phase(6, 7), 2),
-                          clear_accumulators=round(phase(7, 3), 2), wait_for_first_k_tile=round(phase(3, 1), 2)),
-            main_loop=round(phase(1, 2), 2),
-            last_mfma_to_last_store_issued=round(phase(2, 4), 2), hand_over=round(phase(4, 5), 2),
-            between_tiles_of_a_workgroup=round(float(between.mean()), 2) if between.numel() else None,
-            tile_total=round(phase(0, 5), 2), by_ordinal_of_the_tile_in_its_workgroup_start_loop_store=per_ordinal,
-            first_tile_start_to_last_tile_end_ms=round(float(t[:, :, 5][done].max() - start) / 1000.0, 4))
+        res['products'][name] = dict(launch_ms=round(e0.elapsed_time(e1), 4),
+                                     **tile_phases(buf.view(workgroups, tiles, ids).cpu().double() / 100.0))   # microseconds
     return res
 
 

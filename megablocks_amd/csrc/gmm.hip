@@ -554,10 +554,15 @@ int launch_tn(const DmaCall& call) {
 // The direct-to-LDS kernels for 16-bit operands: the row tiles of NN / NT by whether the reduction is whole K tiles, TN
 // here (the half-height tile only when the product has at most 128 rows: it is slower otherwise).
 static int gmm_dma(const DmaCall& call) {
-  if (gmm_few_takes(call)) return gmm_few(call);
-  if (gmm_mid_takes(call)) return gmm_mid(call);
+#ifdef MBX_TICKS
+  constexpr bool kFewRows = false;   // the kernels for few rows per expert have no stamps
+#else
+  constexpr bool kFewRows = true;
+#endif
+  if (kFewRows && gmm_few_takes(call)) return gmm_few(call);
+  if (kFewRows && gmm_mid_takes(call)) return gmm_mid(call);
   if (call.layout != MBX_TN) return call.k % dma::TileMain::BK == 0 ? gmm_rows(call) : gmm_rows_tail(call);
-  if (gmm_tn_short_takes(call)) return gmm_tn_short(call);
+  if (kFewRows && gmm_tn_short_takes(call)) return gmm_tn_short(call);
   if (call.gather.slots) {   // gathered rows: the full tile only
     if (call.dtype == MBX_BF16) return launch_tn<MBX_BF16, dma::TileMain, dma::TileMain>(call);
     return launch_tn<MBX_F16, dma::TileMain, dma::TileMain>(call);
