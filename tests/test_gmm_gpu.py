@@ -1314,7 +1314,7 @@ def test_products_under_an_epilogue_are_the_plain_ones(gg, monkeypatch, counts, 
 
 @pytest.mark.parametrize('groups,rows,k,n', [(1, 1, 8, 8), (3, 130, 64, 256), (5, 1280, 72, 264), (8, 8 * 257, 128, 1032), (32, 4096, 192, 768)])
 @pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])
-def test_batched_mlp_with_activation_epilogues(gg, groups, rows, k, n, dtype):
+def test_batched_mlp_with_activation_epilogues(gg, monkeypatch, groups, rows, k, n, dtype):
     """The capacity-factor layer's products with the activation in their epilogues against the plain product and an
     element-wise pass: the product bit for bit unless the plain launch cuts its last tiles along the reduction, the
     activation of the stored product within the rounding of two tanh evaluations; and every gradient against the node
@@ -1328,6 +1328,9 @@ def test_batched_mlp_with_activation_epilogues(gg, groups, rows, k, n, dtype):
     pre, act = gg.gmm_act(x, w1, sizes, fuse=True, trans_b=False)
     assert max_block_err(pre, _ref_gpu(x, w1, sizes.cpu(), False, False)) < TOL
     assert rel_err(act, torch.nn.functional.gelu(pre.float(), approximate='tanh')) < TOL
+    monkeypatch.setattr(gg, 'GMM_WORKSPACE', False)
+    assert torch.equal(pre, gg.backend.gmm(x, w1, sizes))
+    monkeypatch.undo()
     grad = torch.randn(rows, k, device='cuda').to(dtype)
     results = []
     for fused in (True, False):
@@ -1537,3 +1540,34 @@ def test_gmm_nt_with_a_few_dozen_rows_per_expert(gg, groups, rows, k, n, dtype):
         assert same(gg.gmm_gather(src, w, sizes)[0], c)
         assert same(gg.gmm_gather(src, w, sizes, b2=v, act=1)[2], h)
         assert same(gg.gmm_gather(src, w, sizes, b2=v, act=1, keep_product=False)[2], h)
+
+
+@pytest.mark.parametrize('tokens,experts,top_k,k,n,blocking', [
+    (400, 64, 6, 128, 1288, 0), (640, 64, 2, 320, 1288, 0), (256, 128, 4, 64, 776, 0), (296, 40, 3, 192, 2056, 0), (75, 12, 5, 64, 5896, 0),
+    # padded rows: expert e's start at a multiple of 128 in the product and not in the list of assignments
+    (12, 80, 2, 128, 1800, 128), (6, 64, 3, 64, 1544, 128),
+])
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])
+def test_gathered_products_of_a_few_dozen_rows_per_expert(gg, tokens, experts, top_k, k, n, blocking, dtype):
+    """The kernel for a few dozen rows per expert (up to 40 on average, more 64 x 256 tiles than compute units) reading
+    its rows through the assignments: several experts per token, padded and not, every form, against the gathered copy and
+    the product on it, bit for bit."""
+    indices, bin_ids, bins, padded, tpe = _routing(tokens, experts, top_k, seed=tokens, blocking=blocking)
+    sizes = torch.diff(padded, prepend=padded.new_zeros(1)) if blocking else tpe
+    rows = int(sizes.sum())
+    assert rows <= 40 * experts and experts * ((n + 255) // 256) * 0.95 > 256
+    x = torch.randn(tokens, k, device='cuda').to(dtype)
+    w1, v1 = ((torch.randn(experts, n, k, device='cuda') / k ** 0.5).to(dtype) for _ in range(2))
+    src = gg.GatheredRows(x, indices, bin_ids, bins, padded, top_k, rows)
+    a = src.materialize()
+    (c,) = gg.gmm_gather(src, w1, sizes)
+    assert torch.equal(c, gg.backend.gmm(a, w1, sizes, trans_b=True))
+    assert max_block_err(c, _ref_gpu(a, w1, sizes.cpu(), False, True), 8, 32) < 4 * TOL
+    pre, act = gg.gmm_gather(src, w1, sizes, act=gg.ACT_GELU_TANH)
+    want_pre, want_act = gg.gmm_act(a, w1, sizes, fuse=True)
+    assert torch.equal(pre, c) and torch.equal(want_pre, c) and torch.equal(act, want_act)
+    assert torch.equal(gg.gmm_gather(src, w1, sizes, act=gg.ACT_GELU_TANH, keep_product=False)[1], act)
+    for code in (0, 1):
+        got, want = gg.gmm_gather(src, w1, sizes, b2=v1, act=code), gg.gmm_glu(a, w1, v1, sizes, code, fuse=True)
+        assert all(torch.equal(p, q) for p, q in zip(got, want)) and torch.equal(got[0], c)
+        assert torch.equal(gg.gmm_gather(src, w1, sizes, b2=v1, act=code, keep_product=False)[2], got[2])
