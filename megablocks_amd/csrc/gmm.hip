@@ -2,11 +2,14 @@
 //
 //   NN: c[r_e] = a[r_e] @ b[e]        NT: c[r_e] = a[r_e] @ b[e]^T       TN: c[e] = a[r_e]^T @ b[r_e]
 //
-// Two implementations.  The product path is the direct-to-LDS kernels of gmm_dma.h (v_mfma_f32_16x16x32, LDS rings
-// filled by buffer_load ... lds, persistent workgroups with an XCD-aware tile schedule).  This file holds their launch
-// logic, and, for the shapes they do not take, a register-staged kernel (v_mfma_f32_32x32x16, operand tiles loaded
-// into registers, stored to a double-buffered LDS tile) and an element-wise kernel for any shape, alignment and fp32.
-// In all of them an operand whose reduction dimension is contiguous in memory ("KC": a in NN/NT, b in NT) is kept as
+// The entry points and the choice of the kernel.  16-bit operands of whole 16-byte pieces go to the direct-to-LDS kernels of
+// gmm_dma.h (v_mfma_f32_16x16x32, LDS rings filled by buffer_load ... lds, persistent workgroups with an XCD-aware tile
+// schedule; NN / NT launched by gmm_rows.hip and gmm_rows_tail.hip, TN here) or, with few rows per expert, to those of
+// gmm_few.hip, gmm_mid.hip and gmm_tn_short.hip; fp32 ones to gmm_f32.hip.  This file also has what takes the rest: a
+// register-staged kernel (v_mfma_f32_32x32x16, operand tiles loaded into registers, stored to a double-buffered LDS
+// tile) for outputs the others cannot store and weights of 2 GiB and more, and an element-wise kernel for any shape,
+// alignment and type, which fp32 weight gradients of few rows per expert use too.
+// In those of gmm_dma.h and of this file an operand whose reduction dimension is contiguous in memory ("KC": a in NN/NT, b in NT) is kept as
 // [row][k] in LDS and read with 128-bit LDS loads; an operand whose reduction dimension is
 // strided ("MC": b in NN, both in TN) is kept as [k][col] and read with the gfx950
 // transposing LDS load (ds_read_b64_tr_b16), which hands every lane the four k-consecutive

@@ -291,9 +291,10 @@ int dispatch_few(const DmaCall& q) {
 // Up to eight rows per expert on average (beyond, experts of more than 16 rows read their weights twice: 16 rows per expert
 // cost 20 - 40 %).
 // NN: wherever gmm_dma.h's tiles would leave the chip partly idle; with reductions of 3072 and more only up to half a round of
-// them, which that kernel does not cut into more than two parts (us, that kernel / this one, two rows per expert:
-// [14336, 4096] 8 experts 178 / 173, 9: 185 / 231, 12: 227 / 258;  [8192, 4096] 8: 104 / 115, 12: 134 / 172, 28: 311 / 400;
-// [4096, 2048] 16: 45 / 43, 24: 71 / 78;  [2816, 3072] 16: 46 / 44, 32: 112 / 103).
+// them: there that kernel cuts its tiles along the reduction, and here a workgroup runs so long that a compute unit with one
+// more than the others ends late (8 experts of [14336, 4096], two to a compute unit, 174 us, 9 experts 235).  (us, that
+// kernel / this one, two rows per expert: [14336, 4096] 8 experts 178 / 173, 9: 185 / 231, 12: 227 / 258;  [8192, 4096] 8: 104 /
+// 115, 12: 134 / 172, 28: 311 / 400;  [4096, 2048] 16: 45 / 43, 24: 71 / 78;  [2816, 3072] 16: 46 / 44, 32: 112 / 103).
 // NT: that kernel keeps up as long as its rounds of tiles are about three quarters full (32 experts, [2816, 3072]: 195 against
 // 216 us with 0.86 of them full, 124 against 134 with 0.77; 25 of 64 experts, [1408, 2048]: 74 against 61 with 0.54), with
 // short reductions, sixteen chunks of which are four per wave here, longer still (16 experts, [1408, 1024]: 21 against 24 us

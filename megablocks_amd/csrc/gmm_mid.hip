@@ -13,8 +13,7 @@
 //   64 x 24, [4096, 1024]: 200 / 193, 105 / 99, 120 / 101;  128 x 24, [2048, 768]: 159 / 148, 86 / 77, 100 / 79
 // (369 MB of weights in 68 us: 5.4 TB/s.)
 //
-// Layouts are gmm_dma.h's: rows of 128 bytes for operands whose reduction is contiguous, [k][256] with transposing reads for NN
-// weights.
+// Layouts are gmm_dma.h's for operands whose reduction is contiguous: rows of 128 bytes.
 #include "gmm_common.h"
 
 #include <cmath>
@@ -190,7 +189,11 @@ int dispatch(const DmaCall& q) {
 // Up to 40 rows per expert on average (from 64 on an expert's weights are read twice: 64 experts, [4096, 1024], 107 / 101 us at
 // 40 rows, 108 / 111 at 52) and more tiles than compute units: with fewer a workgroup is alone on its compute unit and
 // waits out every stage, where gmm_dma.h's ring has three under way (16 experts, [2816, 1024], 176 tiles: 19.5 / 21.4; 16,
-// [1024, 3072], 64 tiles: 33 / 51).  The number of experts that get rows is an expectation: rows that choose evenly.
+// [1024, 3072], 64 tiles: 33 / 51).  The number of experts that get rows is an expectation: rows that choose evenly.  Skewed rows
+// (gated, plain, gradient, 16 and 38 rows on average): Zipf-distributed, exponent 1.2, like even ones (64 experts top-6, [1408,
+// 2048]: 172, 94, 101 / 135, 67, 69 and 194, 93, 99 / 153, 70, 73; 8 top-2, [14336, 4096]: 342, 205, 210 / 353, 160, 164
+// and 363, 216, 223 / 352, 168, 172); where a few experts get everything there are too few tiles again, and the launch is short
+// (all on top_k of them: 30, 28, 32 / 35, 33, 35 and 51, 29, 33 / 42, 34, 36; 86, 68, 72 / 98, 63, 66 and 126, 56, 63 / 136, 66, 82).
 // The epilogues do not enter the rule: the product of a launch with one is the plain launch's, bit for bit.  NN launches stay
 // with gmm_dma.h, which cuts their last round along the reduction (8 experts, [4096, 14336]: 210 / 314).
 bool gmm_mid_takes(const DmaCall& q) {
