@@ -83,12 +83,14 @@ gmm_few_kernel(const uint16_t* __restrict__ a, const uint16_t* __restrict__ b, u
     Unit u;
     int tm, tn;
     tiles.find(id, u.e, u.start, u.end, tm, tn);
-    // Eight column tiles, then the same eight with the expert's next rows: those workgroups follow on the same XCDs and find
-    // the weights in their L2s.
-    const int mt = (u.end - u.start + kRows - 1) / kRows, t = tn * mt + tm, first = t / (8 * mt) * 8, in = t - first * mt;
-    const int wide = tiles_n - first < 8 ? tiles_n - first : 8;
-    tm = in / wide;
-    tn = first + in % wide;
+    const int mt = (u.end - u.start + kRows - 1) / kRows;
+    if (mt > 1) {
+      // Eight column tiles, then the same eight with the expert's next rows: those workgroups follow on the same XCDs and find
+      // the weights in their L2s.
+      const int t = tn * mt + tm, first = t / (8 * mt) * 8, in = t - first * mt, wide = tiles_n - first < 8 ? tiles_n - first : 8;
+      tm = in / wide;
+      tn = first + in % wide;
+    }
     u.row0 = u.start + tm * kRows;
     u.n0 = tn * kTileCols;
     return u;
