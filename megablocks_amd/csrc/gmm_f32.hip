@@ -1,32 +1,36 @@
-// Grouped GEMM in fp32 on the bf16 matrix instruction: every value is split into three bf16 parts (24 bits, Split below), and the
+// Grouped GEMM in fp32 on the bf16 matrix instruction: every value is split into three bf16 parts (24 bits, Chunk below), and the
 // six products of parts that reach 2^-18 of a product are summed in fp32 (v_mfma_f32_16x16x32_bf16).
 //
 // What bounds it: the matrix cores and the power they draw.  The fp32 instruction (v_mfma_f32_16x16x4_f32) does 256 FLOP
-// per cycle and compute unit, the bf16 one 4096, a sixth of which is 683.  Next to the 96 products of a K tile, 1536 cycles
-// of a SIMD, a wave spends 384 vector-ALU instructions, 1536 cycles, on the splitting; two waves share a SIMD, and what
-// one converts the other multiplies.  8 experts of 1024 +- 30 rows, hidden 1024, ffn 4096: 416 / 380 / 366 us NT / NN / TN
-// against 533 / 545 / 522 on the fp32 instruction and 961 in the element-wise kernel of gmm.hip, which serves every
-// alignment; 195 TFLOP/s on 4096^3 against 141.  Half the conversion instructions (v_dot2c_f32_bf16) changed nothing;
+// per cycle and compute unit, the bf16 one 4096, a sixth of which is 683.  Next to a product there is room for two vector-ALU
+// instructions per SIMD (measured: 2 are free, 3 cost a fifth, 4 half of the rate), and a value takes six to become parts.  So a
+// workgroup converts a value once, on its way to the LDS, and its waves multiply parts: 1.7 instructions per product.  When every
+// wave converted what it read, 4 per product, the matrix cores were busy 45 - 50 % of the time, now 55 - 59 %, at 2.0 GHz instead
+// of 2.1.  8 experts of 1024 +- 30 rows, hidden 1024, ffn 4096: 374 / 348 / 325 us NT / NN / TN against 455 / 435 / 373 that way,
+// 533 / 545 / 522 on the fp32 instruction and 961 in the element-wise kernel of gmm.hip, which serves every alignment; 237 TFLOP/s
+// on 4096^3 (190; the vendor library 231).  Keeping the pipeline filled across a workgroup's tiles changed nothing (370 / 362 / 337);
 // cutting the parts off instead of rounding them is 3 % faster and up to a third less exact.
 //
 // How exact: three parts hold all 24 bits of a value; the three products of parts not taken come to less than 2^-25 of a product,
 // and an accumulator is rounded six times per 32 k instead of 32 times.  Relative error (2-norm) against fp64: 4.8e-7 over
-// k = 1024, 9.8e-7 over 4096, where a chain of fp32 fused multiply-adds shows 5.7e-7 and 1.15e-6; 3.4e-8 over eight terms (5.4e-8).
+// k = 1024, 9.8e-7 over 4096, where a chain of fp32 fused multiply-adds shows 5.7e-7 and 1.15e-6; 3.1e-8 over eight terms (5.4e-8).
+// The small tile, which puts its sums aside every 256 terms: 2.3e-7 over 1024 terms of which a launch that is cut into four parts made
+// 2.3e-7 too, 2.4e-7 over 4096 (3.5e-7 cut into eight).
 // The error of a single product is larger than that chain's, up to 2.6 2^-24 of it instead of one: sums of one or two terms,
 // and those that the parts do not serve (infinities, NaN, values next to the largest or the smallest), are formed on the fp32
 // instruction: multiply().
 //
-// Tile: 128 x 128 (64 x 128 for short experts) per workgroup of four waves (2 x 2), K tiles of 32, two stages of
-// 32 KiB, so two workgroups share a compute unit and one multiplies while the other converts, waits at its barrier or
-// stores.  Operands go global -> LDS without registers as whole 16-byte pieces (k and n multiples of 4, 16-byte aligned
-// operands); the loads of a K tile are issued a K tile before they are needed, and one barrier per K tile is enough.
+// Tile: 128 x 256 per workgroup of eight waves, two to a SIMD, K tiles of 32 in two stages of 72 KiB; 256 x 128 for TN products
+// whose edges it leaves less empty (12 experts of 500 rows, [2728, 1032]: 252 -> 212 us); 64 x 128, 36 KiB a stage and two
+// workgroups to a compute unit, for short experts and launches of few tiles (f32_small()).  Values pass through registers, a
+// K tile ahead: while K tile kt is multiplied, kt + 1 is converted and written to the other stage, and the loads of kt + 2 go
+// out into the registers that frees.  One barrier per K tile.
 //
-// LDS layouts: an operand whose reduction dimension is contiguous (KC) is [row][32 k], 128-byte rows, 16-byte chunk c of row r
-// at position c ^ ((r >> 1) & 7) (gmm_dma.h's layout of 64 16-bit values, byte for byte); one ds_read_b128 gives a
-// lane its row's operand of four instructions.  An operand whose reduction dimension is strided (MC) is [k][128 columns],
-// the column XORed by 16 ((k >> 2) & 3), so that the four quarter waves, which read rows four apart, use different
-// banks; a lane reads two rows per ds_read2st64_b32.  Step j (of 4) of group s (of 2) of a K tile multiplies
-// k = 16 s + 4 (lane / 16) + j of both operands; the bf16 instruction takes both groups' four as a lane's eight.
+// LDS layout: the three parts of an operand tile, each [row][32 k] bf16: 64-byte rows, the 16-byte chunk of k = 8 q .. 8 q + 7 of
+// row r at position q ^ x(r) (chunk_at), which neither the reads (16 rows, one chunk) nor the writes (64 rows of one chunk, or
+// 16 whole rows) find in the same banks; x = (r >> 2) & 3 alone costs 14 % of the cycles in conflicts.  An operand whose reduction
+// dimension is contiguous (KC) is loaded in 16-byte pieces, two to a chunk; one whose reduction dimension is strided (MC) in
+// dwords, 64 consecutive columns to a load and eight k to a chunk, so that both end up in the same layout.
 #include "gmm_common.h"
 
 namespace mbx {
@@ -43,11 +47,32 @@ using dma::make_rsrc;
 using dma::RowTiles;
 using dma::tile_done;
 
-constexpr int kBN = 128, kBK = 32, kThreads = 256;
-constexpr uint32_t kOperandBytes = 128 * kBK * 4, kStageBytes = 2 * kOperandBytes;
-constexpr size_t kLdsBytes = 2 * kStageBytes;
-constexpr size_t kPartBytes = (size_t)128 * kBN * 4;       // one tile's accumulators in the workspace
+constexpr int kBK = 32, kThreads = 512;
+constexpr uint32_t kRowBytes = kBK * 2;                    // a part of a row's K tile
 constexpr int kMaxKSplit = 8, kMinPartTiles = 8;           // parts of a reduction, K tiles per part
+
+// A tile of BM x BN and how the eight waves share it.
+template <int BM_, int BN_>
+struct Shape {
+  static constexpr int BM = BM_, BN = BN_;
+  static constexpr int WN = BM == 256 ? 2 : 4, WM = 8 / WN;                      // waves along the columns, the rows
+  static constexpr int TM = BM / WM / 16, TN = BN / WN / 16;                     // 16 x 16 accumulator tiles of a wave
+  static constexpr uint32_t kPlaneBytes = (BM + BN) * kRowBytes, kStageBytes = 3 * kPlaneBytes;
+  static constexpr size_t kLdsBytes = 2 * kStageBytes;
+  static constexpr size_t kPartBytes = (size_t)BM * BN * 4;                      // one tile's accumulators in the workspace
+  static constexpr int kPerUnit = kLdsBytes > 80 * 1024 ? 1 : 2;                 // workgroups that share a compute unit
+  // K tiles after which the sums so far are put aside and new ones begun (0: never).  Launches of few tiles get the small tile
+  // and with it are cut along the reduction less often; what that took off the error of a long sum this does.
+  static constexpr int kBlock = BM == 64 ? kMinPartTiles : 0;
+  // Accumulator tile (i, j), register r of lane l is row row(wave) + 16 i + l % 16, column column(wave) + 16 j + 4 (l / 16) + r
+  // of the workgroup's tile (the operands are swapped, so a lane owns runs of four consecutive columns).
+  typedef f32x4 Acc[TM][TN];
+  static __device__ __forceinline__ int row(int wave) { return wave / WN * (TM * 16); }
+  static __device__ __forceinline__ int column(int wave) { return wave % WN * (TN * 16); }
+};
+typedef Shape<128, 256> Wide;    // the main tile
+typedef Shape<256, 128> Tall;    // TN, where it leaves less of the product's edges empty
+typedef Shape<64, 128> Small;    // NN / NT launches of few rows per expert, and those that leave compute units idle
 
 // The operands of a tile: buffers (out-of-range bytes read as zero), row pitches in bytes, tile origins, the first and
 // one past the last K tile to multiply, the length of the whole reduction (pieces of a row past it read as zeros).
@@ -58,251 +83,283 @@ struct Args {
   int a_r0, b_r0, kt0, kt1, k, nk1;
 };
 
-template <int ROW>   // this lane's column in rows ROW and ROW + 1 of an MC tile
-__device__ __forceinline__ u32x2 lds_read2_rows(uint32_t addr) {
-  u32x2 v;
-  asm volatile("ds_read2st64_b32 %0, %1 offset0:%2 offset1:%3" : "=v"(v) : "v"(addr), "n"(2 * ROW), "n"(2 * ROW + 2));
-  return v;
-}
-
-// The operand of four matrix instructions of a 16-row (column) fragment, as the reads deliver it.  A read is under way from
-// its statement to the wait for it: nothing may touch its registers in between, so they are taken apart (at) only where a
-// product uses them, and every path from the reads to a loop's end or a use goes through the wait and tie().
-template <bool MC> struct Frag;
-template <> struct Frag<false> {
-  u32x4 v;
-  __device__ __forceinline__ float at(int t) const { return __uint_as_float(v[t]); }
-  __device__ __forceinline__ void tie() { asm volatile("" : "+v"(v)); }
-};
-template <> struct Frag<true> {
-  u32x2 v[2];
-  __device__ __forceinline__ float at(int t) const { return __uint_as_float(v[t / 2][t % 2]); }
-  __device__ __forceinline__ void tie() { asm volatile("" : "+v"(v[0]), "+v"(v[1])); }
-};
-
-// Eight fp32 values as three bf16 parts each, v = part 0 + part 1 + part 2 up to 2^-27 |v|: every part is the rest the parts
-// before it leave (the differences are exact), rounded to nearest.  In kSteps steps of a few instructions, to be put between
-// products: step 3 p + q forms part q of the values 2 p and 2 p + 1.
-struct Split {
-  static constexpr int kSteps = 12;
-  u32x4 part[3];
-  float rest[2];
-  template <int X, bool MC>
-  __device__ __forceinline__ void step(const Frag<MC>& low, const Frag<MC>& high, float& largest) {   // largest: magnitude seen
-    constexpr int p = X / 3, q = X % 3, v = 2 * (p & 1);
-    if constexpr (q == 0) {
-      rest[0] = p < 2 ? low.at(v) : high.at(v);
-      rest[1] = p < 2 ? low.at(v + 1) : high.at(v + 1);
-      asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(largest) : "v"(rest[0]), "v"(rest[1]));
-    }
-    const uint32_t both = pack2<MBX_BF16>(rest[0], rest[1]);
-    part[q][p] = both;
-    if constexpr (q < 2) {
-      rest[0] -= __uint_as_float(both << 16);
-      rest[1] -= __uint_as_float(both & 0xffff0000u);
-    }
-  }
-};
-
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef const __attribute__((address_space(3))) u32x4* lds_in;
+typedef __attribute__((address_space(3))) u32x4* lds_out;
+typedef __attribute__((address_space(3))) u32x2* lds_out_half;
 
 __device__ __forceinline__ f32x4 mfma(u32x4 a, u32x4 b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }
 
-template <int N>
-__device__ __forceinline__ void wait_lgkm() {   // at most N LDS reads of this wave still in flight
-  static_assert(N < 16, "lgkmcnt is a 4-bit counter");
-  asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(N) : "memory");
+// V (8 or 4) consecutive k of one row (column) of an operand on their way from memory to the LDS: the chunk of one thread.
+// step() forms the three bf16 parts, v = part 0 + part 1 + part 2 up to 2^-27 |v|: every part is the rest the parts before
+// it leave (the differences are exact), rounded to nearest.  In kSteps steps of a few instructions, to be put between
+// products: step V / 2 q + p forms part q of the values 2 p and 2 p + 1, the last of a part stores it.
+template <int V, uint32_t PLANE>
+struct Chunk {
+  static constexpr int kPairs = V / 2, kSteps = 3 * kPairs;
+  float v[V];
+  uint32_t part[kPairs];
+
+  template <int X>
+  __device__ __forceinline__ void step(float& largest, lds_ptr to) {   // largest: magnitude seen
+    constexpr int q = X / kPairs, p = X % kPairs;
+    if constexpr (q == 0) asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(largest) : "v"(v[2 * p]), "v"(v[2 * p + 1]));
+    const uint32_t both = pack2<MBX_BF16>(v[2 * p], v[2 * p + 1]);
+    part[p] = both;
+    if constexpr (q < 2) {
+      v[2 * p] -= __uint_as_float(both << 16);
+      v[2 * p + 1] -= __uint_as_float(both & 0xffff0000u);
+    }
+    if constexpr (p == kPairs - 1) {
+      if constexpr (V == 8) *(lds_out)(to + q * PLANE) = u32x4{part[0], part[1], part[2], part[3]};
+      else *(lds_out_half)(to + q * PLANE) = u32x2{part[0], part[1]};
+    }
+  }
+  // for the fp32 instruction: the values as they are, k 0 .. 3 of eight to one plane, 4 .. 7 to the next
+  __device__ __forceinline__ void store_as_is(lds_ptr to, int half) const {
+    if constexpr (V == 8) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        *(lds_out)(to + h * PLANE) = u32x4{__float_as_uint(v[4 * h]), __float_as_uint(v[4 * h + 1]), __float_as_uint(v[4 * h + 2]), __float_as_uint(v[4 * h + 3])};
+    } else {
+      *(lds_out)(to + half * ((int)PLANE - 8)) = u32x4{__float_as_uint(v[0]), __float_as_uint(v[1]), __float_as_uint(v[2]), __float_as_uint(v[3])};
+    }
+  }
+};
+
+template <typename S>
+__device__ __forceinline__ void clear(typename S::Acc& acc) {
+#pragma unroll
+  for (int i = 0; i < S::TM; ++i)
+#pragma unroll
+    for (int j = 0; j < S::TN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 }
 
-// The accumulators of a wave: (BM / 32) x 4 tiles of 16 x 16 of its (BM / 2) x 64 part of the tile.  Tile (i, j), register r of
-// lane l is
-//   row wm + 16 i + l % 16, column wn + 16 j + 4 (l / 16) + r
-// of the workgroup's tile (the operands are swapped, so a lane owns runs of four consecutive columns).
-template <int BM> using Acc = f32x4[BM / 32][4];
-
 // acc += A_tile * B_tile over K tiles [g.kt0, g.kt1); largest: the largest magnitude among the operands (unless FP32)
-template <bool A_MC, bool B_MC, int BM, bool DUAL, bool FP32>
-__device__ __forceinline__ void multiply_as(const Args& g, Acc<BM>& acc, char* lds_generic, float& largest) {
-  constexpr int TM = BM / 32, TN = 4;
-  static_assert(!A_MC || BM == 128, "a strided first operand: full tiles");
+template <bool A_MC, bool B_MC, typename S, bool DUAL, bool FP32>
+__device__ __forceinline__ void multiply_as(const Args& g, typename S::Acc& acc, char* lds_generic, float& largest) {
+  constexpr int TM = S::TM, TN = S::TN, kA = S::BM == 256 ? 2 : 1, kB = S::BN / 128, kChunks = kA + kB;   // chunks of a thread
+  constexpr int kAV = S::BM == 64 ? 4 : 8;
+  if (g.kt0 >= g.kt1) return;
   const lds_ptr lds = (lds_ptr)lds_generic;
-  const uint32_t lds_base = (uint32_t)(uintptr_t)lds;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = lane_id(), quarter = lane >> 4;
-  const int wm = (wave / 2) * (BM / 2), wn = (wave % 2) * 64;
-  constexpr int LA = BM / 32, LB = 4;   // wave-wide loads of a K tile per wave
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = lane_id();
 
-  // KC: load j = wave + 4 q holds rows 8 j .. 8 j + 7; a lane's 16-byte piece is the same for all q.
-  // MC: load j holds rows k = 2 j, 2 j + 1, whose (k >> 2) & 3 is (wave >> 1) + 2 (q & 1).
-  auto mc_offset = [&](int r0, uint32_t ld, int odd) -> uint32_t {
-    return (uint32_t)(lane >> 5) * ld + (uint32_t)r0 * 4u + (uint32_t)((lane & 31) ^ (4 * ((wave >> 1) + 2 * odd))) * 16u;
+  // This thread's chunks: k = 8 q .. 8 q + 7 of rows r and r + 128 of A and of B; BM = 64: one half of eight k of a row of A.
+  auto chunk_at = [&](int row, int q) -> uint32_t {
+    const int b = row >> 2 & 3, x = (((b << 1 ^ b) & 2) | b >> 1) ^ (row >> 1 & 1);
+    return (uint32_t)row * kRowBytes + (uint32_t)((q ^ x) << 4);
   };
-  const uint32_t a_lane = A_MC ? mc_offset(g.a_r0, g.a_ld, 0) : dma::load_lane_offset<false, 64, 128>(wave, g.a_r0, g.a_ld);
-  const uint32_t b_lane = B_MC ? mc_offset(g.b_r0, g.b_ld, 0) : dma::load_lane_offset<false, 64, 128>(wave, g.b_r0, g.b_ld);
-  const uint32_t a_odd = A_MC ? mc_offset(g.a_r0, g.a_ld, 1) - a_lane : 0u, b_odd = B_MC ? mc_offset(g.b_r0, g.b_ld, 1) - b_lane : 0u;
-  const uint32_t a_j = A_MC ? 2u * g.a_ld : 8u * g.a_ld, b_j = B_MC ? 2u * g.b_ld : 8u * g.b_ld;   // from load j to j + 1
+  const int kc_r = threadIdx.x >> 2, kc_q = threadIdx.x & 3;                    // four lanes a row: 128 bytes of it
+  const int half_r = A_MC ? lane : threadIdx.x >> 3, half_k = 4 * (A_MC ? wave : threadIdx.x & 7);   // eight lanes a row; 64 columns per load
+  const int mc_r = lane + 64 * (wave >> 2), mc_q = wave & 3;                    // 64 consecutive columns per load
+  const uint32_t a_to = kAV == 4 ? chunk_at(half_r, half_k >> 3) + (half_k & 4 ? 8u : 0u) : A_MC ? chunk_at(mc_r, mc_q) : chunk_at(kc_r, kc_q);
+  const uint32_t b_to = S::BM * kRowBytes + (B_MC ? chunk_at(mc_r, mc_q) : chunk_at(kc_r, kc_q));
+  const uint32_t a_lane = kAV == 4 ? (A_MC ? (uint32_t)half_k * g.a_ld + (uint32_t)(g.a_r0 + half_r) * 4u : (uint32_t)(g.a_r0 + half_r) * g.a_ld + (uint32_t)half_k * 4u)
+                          : A_MC ? (uint32_t)(8 * mc_q) * g.a_ld + (uint32_t)(g.a_r0 + mc_r) * 4u
+                                 : (uint32_t)(g.a_r0 + kc_r) * g.a_ld + (uint32_t)kc_q * 32u;
+  const uint32_t b_lane = B_MC ? (uint32_t)(8 * mc_q) * g.b_ld + (uint32_t)(g.b_r0 + mc_r) * 4u
+                               : (uint32_t)(g.b_r0 + kc_r) * g.b_ld + (uint32_t)kc_q * 32u;
   const uint32_t a_step = A_MC ? kBK * g.a_ld : kBK * 4u, b_step = B_MC ? kBK * g.b_ld : kBK * 4u;   // per K tile
-  const int piece_k = 4 * ((lane & 7) ^ ((4 * (wave & 1) + ((lane >> 3) >> 1)) & 7));   // first k of a KC lane's piece
-  // One of the LA + LB loads of a K tile: load_at() works out the K tile's addresses, load_one() issues number q.
-  uint32_t a0 = 0, b0 = 0, dst = 0;
+
+  typedef Chunk<kAV, S::kPlaneBytes> ChunkA;
+  typedef Chunk<8, S::kPlaneBytes> ChunkB;
+  ChunkA ca[kA];
+  ChunkB cb[kB];
+  uint32_t a_at = 0, b_at = 0, past_half = 0, past_low = 0, past_high = 0;
   __amdgpu_buffer_rsrc_t ra = g.rsrc_a, rb = g.rsrc_b;
-  auto load_at = [&](int kt, uint32_t stage) {
+  auto load_at = [&](int kt) {
     const bool second = DUAL && kt >= g.nk1;
     const int kk = second ? kt - g.nk1 : kt;
-    // k is a multiple of 4: a piece of a row lies inside the reduction or past it, where it has to read as zeros (the
-    // next row's values could be infinite); bit 31 puts it out of the buffer's range, as it does a K tile past the last
-    const uint32_t past = kk * kBK + piece_k < g.k ? 0u : 0x80000000u, none = kt < g.kt1 ? 0u : 0x80000000u;
+    // bit 31 puts a load out of its buffer's range, so that it reads zeros: a K tile past the last, and the pieces of a row
+    // past the end of the reduction (k is a multiple of 4), where the next row's values could be infinite
+    const uint32_t none = kt < g.kt1 ? 0u : 0x80000000u;
+    const int left = g.k - kk * kBK;
+    past_half = left > half_k ? 0u : 0x80000000u;
+    past_low = left > 8 * kc_q ? 0u : 0x80000000u;
+    past_high = left > 8 * kc_q + 4 ? 0u : 0x80000000u;
     if (DUAL) { ra = second ? g.rsrc_a2 : g.rsrc_a; rb = second ? g.rsrc_b2 : g.rsrc_b; }
-    a0 = (a_lane + (uint32_t)kk * a_step + (uint32_t)wave * a_j) | (A_MC ? none : past | none);
-    b0 = (b_lane + (uint32_t)kk * b_step + (uint32_t)wave * b_j) | (B_MC ? none : past | none);
-    dst = stage + (uint32_t)wave * 1024u;
+    a_at = (a_lane + (uint32_t)kk * a_step) | none;
+    b_at = (b_lane + (uint32_t)kk * b_step) | none;
   };
-  auto load_one = [&](auto qi) {
-    constexpr uint32_t q = decltype(qi)::value;
-    if constexpr (q < LA)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (__attribute__((address_space(3))) void*)(lds + dst + q * 4096u), 16, (int)(a0 + 4u * q * a_j + (q & 1 ? a_odd : 0u)), 0, 0, 0);
-    else
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (__attribute__((address_space(3))) void*)(lds + dst + kOperandBytes + (q - LA) * 4096u), 16, (int)(b0 + 4u * (q - LA) * b_j + ((q - LA) & 1 ? b_odd : 0u)), 0, 0, 0);
-  };
-
-  // LDS addresses of this lane's operands of group 0 in stage 0
-  auto mc_frag = [&](int r) -> uint32_t { return (uint32_t)(quarter * 4 * 512 + ((r + (lane & 15)) ^ (16 * quarter)) * 4); };
-  uint32_t fa_off[A_MC ? TM : 1], fb_off[B_MC ? TN : 1];
+  auto load_whole = [&](auto mc, ChunkB& to, const __amdgpu_buffer_rsrc_t& rsrc, uint32_t at, uint32_t ld, uint32_t number) {
+    if constexpr (decltype(mc)::value) {
+      at += number * (128 * 4);
 #pragma unroll
-  for (int i = 0; i < (A_MC ? TM : 1); ++i) fa_off[i] = A_MC ? mc_frag(wm + 16 * i) : dma::frag_lane_offset<false, 64, 128>(wm);
+      for (int u = 0; u < 8; ++u) to.v[u] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rsrc, (int)(at + u * ld), 0, 0));
+    } else {
+      at += number * (128 * ld);
+      const u32x4 low = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)(at | past_low), 0, 0));
+      const u32x4 high = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)((at + 16) | past_high), 0, 0));
 #pragma unroll
-  for (int j = 0; j < (B_MC ? TN : 1); ++j) fb_off[j] = kOperandBytes + (B_MC ? mc_frag(wn + 16 * j) : dma::frag_lane_offset<false, 64, 128>(wn));
-
-  Frag<A_MC> fa[2][TM];
-  Frag<B_MC> fb[2][TN];
-  // the read instructions of group s of one fragment: one of a KC fragment (four k), two of an MC fragment (two each)
-  auto read_a = [&](auto ii, uint32_t base) {
-    constexpr int i = decltype(ii)::value;
-    dma::static_for<2>([&](auto si) {
-      constexpr int s = decltype(si)::value;
-      if constexpr (A_MC) { fa[s][i].v[0] = lds_read2_rows<16 * s>(base + fa_off[i]); fa[s][i].v[1] = lds_read2_rows<16 * s + 2>(base + fa_off[i]); }
-      else fa[s][i].v = dma::read_frag_kc<s, i * 16 * 128>(base, fa_off[0]);
-    });
-  };
-  auto read_b = [&](auto ji, uint32_t base) {
-    constexpr int j = decltype(ji)::value;
-    dma::static_for<2>([&](auto si) {
-      constexpr int s = decltype(si)::value;
-      if constexpr (B_MC) { fb[s][j].v[0] = lds_read2_rows<16 * s>(base + fb_off[j]); fb[s][j].v[1] = lds_read2_rows<16 * s + 2>(base + fb_off[j]); }
-      else fb[s][j].v = dma::read_frag_kc<s, j * 16 * 128>(base, fb_off[0]);
-    });
-  };
-  // the values of a K tile as registers written at this point: orders their users behind the wait in front of it
-  auto tie = [&] {
-#pragma unroll
-    for (int s = 0; s < 2; ++s) {
-#pragma unroll
-      for (int i = 0; i < TM; ++i) fa[s][i].tie();
-#pragma unroll
-      for (int j = 0; j < TN; ++j) fb[s][j].tie();
+      for (int u = 0; u < 4; ++u) { to.v[u] = __uint_as_float(low[u]); to.v[4 + u] = __uint_as_float(high[u]); }
     }
   };
-  // The products of a K tile on its split operands.  Fragments of A go in pairs, so that twelve products on two
-  // accumulators stand between the conversions; what is converted behind the products of (pair, j) is the next fragment
-  // of B, or the next pair of A.  The fragments of the next K tile are read behind the products of the last pair, when
-  // the conversions are done (with one pair: as soon as a fragment is converted), so that their registers serve the
-  // parts until then; one of the loads of K tile kt + 2 goes out behind every second product.
-  Split sa[2][2], sb[TN];
-  auto products = [&](uint32_t next_base) {
-    constexpr int PAIRS = TM / 2;
-    auto convert_a = [&](auto ii, auto xi) {
-      constexpr int i = decltype(ii)::value, x = decltype(xi)::value;
-      sa[i / 2 % 2][i % 2].template step<x>(fa[0][i], fa[1][i], largest);
-      if constexpr (PAIRS == 1 && x == Split::kSteps - 1) { __builtin_amdgcn_sched_barrier(0); read_a(ii, next_base); }
-    };
-    auto convert_b = [&](auto ji, auto xi) {
-      constexpr int j = decltype(ji)::value, x = decltype(xi)::value;
-      sb[j].template step<x>(fb[0][j], fb[1][j], largest);
-      if constexpr (PAIRS == 1 && x == Split::kSteps - 1) { __builtin_amdgcn_sched_barrier(0); read_b(ji, next_base); }
-    };
-    constexpr std::integral_constant<int, 0> c0{};
-    constexpr std::integral_constant<int, 1> c1{};
-    dma::static_for<Split::kSteps>([&](auto xi) { convert_a(c0, xi); convert_b(c0, xi); convert_a(c1, xi); });
-    dma::static_for<PAIRS * TN>([&](auto pj) {
-      constexpr int p = decltype(pj)::value / TN, j = decltype(pj)::value % TN;
-      dma::static_for<12>([&](auto mi) {
-        constexpr int m = decltype(mi)::value, t = m / 2, i = m % 2;
-        constexpr int pa[6] = {0, 2, 1, 0, 1, 0}, pb[6] = {2, 0, 1, 1, 0, 0};   // the small products first
-        acc[2 * p + i][j] = mfma(sb[j].part[pb[t]], sa[p % 2][i].part[pa[t]], acc[2 * p + i][j]);
-        if constexpr (p == 0 && j + 1 < TN) convert_b(std::integral_constant<int, j + 1>{}, mi);
-        if constexpr (p + 1 < PAIRS && j >= TN - 2) convert_a(std::integral_constant<int, 2 * p + 2 + j - (TN - 2)>{}, mi);
-        if constexpr (p == 1 && m % 6 == 5) {
-          if constexpr (j < 2) read_a(std::integral_constant<int, 2 * j + m / 6>{}, next_base);
-          else { read_b(std::integral_constant<int, 2 * (j - 2) + m / 6>{}, next_base); }
-        }
-        constexpr int load = (decltype(pj)::value * 12 + m) / 2;
-        if constexpr (m % 2 == 1 && load < LA + LB) load_one(std::integral_constant<uint32_t, load>{});
-        __builtin_amdgcn_sched_barrier(0);
-      });
-    });
+  auto load_a = [&](int number, ChunkA& to) {
+    if constexpr (kAV == 4 && A_MC) {
+#pragma unroll
+      for (int u = 0; u < 4; ++u) to.v[u] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(ra, (int)(a_at + u * g.a_ld), 0, 0));
+    } else if constexpr (kAV == 4) {
+      const u32x4 w = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(ra, (int)(a_at | past_half), 0, 0));
+#pragma unroll
+      for (int u = 0; u < 4; ++u) to.v[u] = __uint_as_float(w[u]);
+    } else {
+      load_whole(std::integral_constant<bool, A_MC>{}, to, ra, a_at, g.a_ld, number);
+    }
   };
-  // The same products on the fp32 instruction.
-  auto products_fp32 = [&](uint32_t next_base) {
-    dma::static_for<2>([&](auto si) {
-      dma::static_for<4>([&](auto ti) {
-        constexpr int s = decltype(si)::value, t = decltype(ti)::value;
+  auto load_b = [&](int number, ChunkB& to) { load_whole(std::integral_constant<bool, B_MC>{}, to, rb, b_at, g.b_ld, number); };
+  auto a_chunk_to = [&](int number, uint32_t stage) -> lds_ptr { return lds + (a_to + stage) + number * (128 * kRowBytes); };
+  auto b_chunk_to = [&](int number, uint32_t stage) -> lds_ptr { return lds + (b_to + stage) + number * (128 * kRowBytes); };
+
+  const uint32_t frag_lane = chunk_at(lane & 15, lane >> 4);
+  const uint32_t fa_at = (uint32_t)S::row(wave) * kRowBytes + frag_lane;
+  const uint32_t fb_at = (uint32_t)(S::BM + S::column(wave)) * kRowBytes + frag_lane;
+  u32x4 fa[3][TM], fb[3][TN];
+  auto read_a = [&](auto qi, auto ii, uint32_t stage) {
+    constexpr int q = decltype(qi)::value, i = decltype(ii)::value;
+    fa[q][i] = *(lds_in)(lds + (fa_at + stage) + (q * S::kPlaneBytes + i * 16 * kRowBytes));
+  };
+  auto read_b = [&](auto qi, auto ji, uint32_t stage) {
+    constexpr int q = decltype(qi)::value, j = decltype(ji)::value;
+    fb[q][j] = *(lds_in)(lds + (fb_at + stage) + (q * S::kPlaneBytes + j * 16 * kRowBytes));
+  };
+  auto barrier = [&] {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+  };
+  constexpr std::integral_constant<int, 0> c0{};
+  constexpr std::integral_constant<int, 1> c1{};
+  constexpr std::integral_constant<int, 2> c2{};
+
+  // K tile kt0 into stage 0, K tile kt0 + 1 under way
+  {
+    ChunkA first_a[kA];
+    ChunkB first_b[kB];
+    load_at(g.kt0);
+#pragma unroll
+    for (int c = 0; c < kA; ++c) load_a(c, first_a[c]);
+#pragma unroll
+    for (int c = 0; c < kB; ++c) load_b(c, first_b[c]);
+    load_at(g.kt0 + 1);
+#pragma unroll
+    for (int c = 0; c < kA; ++c) load_a(c, ca[c]);
+#pragma unroll
+    for (int c = 0; c < kB; ++c) load_b(c, cb[c]);
+    dma::static_for<kA>([&](auto ci) {
+      constexpr int c = decltype(ci)::value;
+      if constexpr (FP32) first_a[c].store_as_is(a_chunk_to(c, 0), (half_k & 4) != 0);
+      else dma::static_for<ChunkA::kSteps>([&](auto xi) { first_a[c].template step<decltype(xi)::value>(largest, a_chunk_to(c, 0)); });
+    });
+    dma::static_for<kB>([&](auto ci) {
+      constexpr int c = decltype(ci)::value;
+      if constexpr (FP32) first_b[c].store_as_is(b_chunk_to(c, 0), 0);
+      else dma::static_for<ChunkB::kSteps>([&](auto xi) { first_b[c].template step<decltype(xi)::value>(largest, b_chunk_to(c, 0)); });
+    });
+  }
+  barrier();
+  uint32_t stage = 0;
+  typename S::Acc aside;
+  if constexpr (S::kBlock != 0) clear<S>(aside);
+  auto put_aside = [&](int kt) {   // behind K tile kt, and at the end
+    if constexpr (S::kBlock != 0) {
+      if ((kt + 1 - g.kt0) % S::kBlock != 0 && kt + 1 != g.kt1) return;
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+          aside[i][j] += acc[i][j];
+          acc[i][j] = kt + 1 == g.kt1 ? aside[i][j] : f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+    }
+  };
+  if constexpr (FP32) {
+    for (int kt = g.kt0; kt < g.kt1; ++kt) {
+      dma::static_for<TM>([&](auto ii) { read_a(c0, ii, stage); read_a(c1, ii, stage); });
+      dma::static_for<TN>([&](auto ji) { read_b(c0, ji, stage); read_b(c1, ji, stage); });
+      stage = S::kStageBytes - stage;
+      load_at(kt + 2);
+#pragma unroll
+      for (int c = 0; c < kA; ++c) { ca[c].store_as_is(a_chunk_to(c, stage), (half_k & 4) != 0); load_a(c, ca[c]); }
+#pragma unroll
+      for (int c = 0; c < kB; ++c) { cb[c].store_as_is(b_chunk_to(c, stage), 0); load_b(c, cb[c]); }
+#pragma unroll
+      for (int t = 0; t < 8; ++t)
 #pragma unroll
         for (int i = 0; i < TM; ++i)
 #pragma unroll
           for (int j = 0; j < TN; ++j)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(fb[s][j].at(t), fa[s][i].at(t), acc[i][j], 0, 0, 0);
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(fb[t / 4][j][t % 4]), __uint_as_float(fa[t / 4][i][t % 4]), acc[i][j], 0, 0, 0);
+      put_aside(kt);
+      barrier();
+    }
+    return;
+  }
+
+  // The products of a K tile go by pairs of parts, the small ones first.  Parts 1 are read ahead of the loop's head, the other
+  // parts a pass before the products that take them; between the products of the first five passes stand the conversions
+  // of K tile kt + 1 (and, when a chunk is converted, the loads of kt + 2 into its registers); the barrier stands where all
+  // waves have read this stage and written the other, with the last pass still to be multiplied behind it.
+  constexpr int kPass = TM * TN, kConvert = 5 * kPass - 2, kWorkA = kA * ChunkA::kSteps, kWork = kWorkA + kB * ChunkB::kSteps;
+  constexpr int pa[6] = {1, 0, 2, 0, 1, 0}, pb[6] = {1, 2, 0, 1, 0, 0};
+  dma::static_for<TM>([&](auto ii) { read_a(c1, ii, 0); });
+  dma::static_for<TN>([&](auto ji) { read_b(c1, ji, 0); });
+  for (int kt = g.kt0; kt < g.kt1; ++kt) {
+    const uint32_t next = S::kStageBytes - stage;
+    load_at(kt + 2);
+    dma::static_for<6>([&](auto pi) {
+      constexpr int pass = decltype(pi)::value;
+      if constexpr (pass == 5) barrier();
+      dma::static_for<kPass>([&](auto mi) {
+        constexpr int m = decltype(mi)::value, i = m / TN, j = m % TN, at = pass * kPass + m;
+        // the next pass's (pass 5: the next K tile's) operands: TM + TN reads over the pass
+        constexpr int f0 = m * (TM + TN) / kPass, f1 = (m + 1) * (TM + TN) / kPass;
+        if constexpr (pass < 2 || pass == 5)
+          dma::static_for<f1 - f0>([&](auto oi) {
+            constexpr int f = f0 + decltype(oi)::value;
+            if constexpr (f < TM) {
+              constexpr std::integral_constant<int, f> fi{};
+              if constexpr (pass == 0) read_a(c0, fi, stage);
+              if constexpr (pass == 1) read_a(c2, fi, stage);
+              if constexpr (pass == 5) read_a(c1, fi, next);
+            } else {
+              constexpr std::integral_constant<int, f - TM> fi{};
+              if constexpr (pass == 0) read_b(c2, fi, stage);
+              if constexpr (pass == 1) read_b(c0, fi, stage);
+              if constexpr (pass == 5) read_b(c1, fi, next);
+            }
+          });
+        acc[i][j] = mfma(fb[pb[pass]][j], fa[pa[pass]][i], acc[i][j]);
+        constexpr int x0 = at * kWork / kConvert, x1 = (at + 1) * kWork / kConvert < kWork ? (at + 1) * kWork / kConvert : kWork;
+        dma::static_for<(x1 > x0 ? x1 - x0 : 0)>([&](auto oi) {
+          constexpr int x = x0 + decltype(oi)::value;
+          if constexpr (x < kWorkA) {
+            constexpr int c = x / ChunkA::kSteps, y = x % ChunkA::kSteps;
+            ca[c].template step<y>(largest, a_chunk_to(c, next));
+            if constexpr (y == ChunkA::kSteps - 1) load_a(c, ca[c]);
+          } else {
+            constexpr int c = (x - kWorkA) / ChunkB::kSteps, y = (x - kWorkA) % ChunkB::kSteps;
+            cb[c].template step<y>(largest, b_chunk_to(c, next));
+            if constexpr (y == ChunkB::kSteps - 1) load_b(c, cb[c]);
+          }
+        });
+        __builtin_amdgcn_sched_barrier(0);
       });
     });
-    __builtin_amdgcn_sched_barrier(0);
-    dma::static_for<LA + LB>(load_one);
-    dma::static_for<TM>([&](auto ii) { read_a(ii, next_base); });
-    dma::static_for<TN>([&](auto ji) { read_b(ji, next_base); });
-  };
-  // A K tile's values are in registers when its iteration begins.  The barrier stands where every wave has read its
-  // stage, which takes K tile kt + 2 from then on, and where K tile kt + 1 has landed in the other, to be read during
-  // the products.
-  if (g.kt0 >= g.kt1) return;
-  load_at(g.kt0, 0);
-  dma::static_for<LA + LB>(load_one);
-  load_at(g.kt0 + 1, kStageBytes);
-  dma::static_for<LA + LB>(load_one);
-  dma::wait_vmcnt<LA + LB>();
-  __builtin_amdgcn_s_barrier();
-  uint32_t stage = 0;
-  dma::static_for<TM>([&](auto ii) { read_a(ii, lds_base); });
-  dma::static_for<TN>([&](auto ji) { read_b(ji, lds_base); });
-  wait_lgkm<0>();
-  tie();
-  for (int kt = g.kt0; kt < g.kt1; ++kt) {
-    dma::wait_vmcnt<0>();
-    __builtin_amdgcn_s_barrier();
-    load_at(kt + 2, stage);
-    stage ^= kStageBytes;
-    if constexpr (FP32) products_fp32(lds_base + stage); else products(lds_base + stage);   // past the last K tile: reads of stale LDS into dead registers
-    wait_lgkm<0>();
-    tie();
+    stage = next;
+    put_aside(kt);
   }
-  dma::wait_vmcnt<0>();
-}
-
-template <int BM>
-__device__ __forceinline__ void clear(Acc<BM>& acc) {
-#pragma unroll
-  for (int i = 0; i < BM / 32; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 }
 
 // Whether one of the values a tile multiplies over K tiles [g.kt0, g.kt1) is so small that its parts lose some of it, zeros
 // apart.  Values of the same operand beyond the tile's last column count along.
 constexpr float kSmall = 0x1p-102f;
 
-template <bool MC, int R, bool DUAL>   // R: rows (KC) of the tile
+template <bool MC, int R, bool DUAL>   // R: rows (columns) of the tile
 __device__ __forceinline__ bool any_small(const Args& g, const __amdgpu_buffer_rsrc_t& first, const __amdgpu_buffer_rsrc_t& second, int r0, uint32_t ld) {
-  // KC: eight lanes a row of 32 k;  MC: 32 lanes a row of 128 columns
-  const int t = threadIdx.x, piece = MC ? t % 32 : t % 8, row = MC ? t / 32 : t / 8;
-  constexpr int kStep = MC ? kThreads / 32 : kThreads / 8, kRows = MC ? kBK : R;
+  // KC: eight lanes a row of 32 k;  MC: R / 4 lanes a row of R columns
+  constexpr int kLanes = MC ? R / 4 : 8, kStep = kThreads / kLanes, kRows = MC ? kBK : R;
+  const int t = threadIdx.x, piece = t % kLanes, row = t / kLanes;
   constexpr int kLoads = kRows / kStep, kAhead = 16 / kLoads;   // loads per K tile, K tiles under way
   uint32_t smallest = 0xffffffffu;   // of the magnitudes as integers; less one, which leaves zeros out
   for (int kt0 = g.kt0; kt0 < g.kt1; kt0 += kAhead) {
@@ -347,16 +404,16 @@ __device__ __forceinline__ bool any_small(const Args& g, const __amdgpu_buffer_r
 // rows, [1024, 4096], instead of 403 / 406 / 371; the element-wise kernel takes 840 / 878 / 780 for any values.
 constexpr float kTiny = 0x1p-64f, kHuge = 0x1p38f;
 
-template <bool A_MC, bool B_MC, int BM, bool DUAL>
-__device__ __forceinline__ bool sums_need_fp32(const Args& g, const Acc<BM>& acc, float operand, int m_lim, int n_lim) {
+template <bool A_MC, bool B_MC, typename S, bool DUAL>
+__device__ __forceinline__ bool sums_need_fp32(const Args& g, const typename S::Acc& acc, float operand, int m_lim, int n_lim) {
   const int wave = threadIdx.x / kWave, lane = lane_id();
-  const int m0 = (wave / 2) * (BM / 2) + (lane & 15), n0 = (wave % 2) * 64 + 4 * (lane >> 4);
+  const int m0 = S::row(wave) + (lane & 15), n0 = S::column(wave) + 4 * (lane >> 4);
   // twice the bits less one: no sign, zeros at the top; whether there is anything to look at more closely
   uint32_t low = 0xffffffffu, high = 0;
 #pragma unroll
-  for (int i = 0; i < BM / 32; ++i)
+  for (int i = 0; i < S::TM; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+    for (int j = 0; j < S::TN; ++j)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const uint32_t t = __float_as_uint(acc[i][j][r]) * 2u - 1u;
@@ -366,9 +423,9 @@ __device__ __forceinline__ bool sums_need_fp32(const Args& g, const Acc<BM>& acc
   bool again = operand >= kHuge, zero = false;
   if (low < 2u * __float_as_uint(kTiny) - 1u || high >= 2u * 0x7f800000u - 1u) {
 #pragma unroll
-    for (int i = 0; i < BM / 32; ++i)
+    for (int i = 0; i < S::TM; ++i)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
+      for (int j = 0; j < S::TN; ++j) {
         const bool stored = m0 + 16 * i < m_lim && n0 + 16 * j < n_lim;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
@@ -380,7 +437,7 @@ __device__ __forceinline__ bool sums_need_fp32(const Args& g, const Acc<BM>& acc
   }
   if (__syncthreads_or(again || zero)) {
     if (__syncthreads_or(zero))
-      again |= any_small<A_MC, BM, DUAL>(g, g.rsrc_a, g.rsrc_a2, g.a_r0, g.a_ld) || any_small<B_MC, 128, DUAL>(g, g.rsrc_b, g.rsrc_b2, g.b_r0, g.b_ld);
+      again |= any_small<A_MC, S::BM, DUAL>(g, g.rsrc_a, g.rsrc_a2, g.a_r0, g.a_ld) || any_small<B_MC, S::BN, DUAL>(g, g.rsrc_b, g.rsrc_b2, g.b_r0, g.b_ld);
     return __syncthreads_or(again);
   }
   return false;
@@ -391,30 +448,30 @@ __device__ __forceinline__ bool sums_need_fp32(const Args& g, const Acc<BM>& acc
 // sum of the magnitudes, 2^-24: 1.0 / 2.6 over one term, 1.9 / 2.6 over two, 2.5 / 2.3 over three, 3.7 / 2.1 over eight).
 constexpr int kFewTerms = 2;
 
-template <bool A_MC, bool B_MC, int BM, bool DUAL>
-__device__ __forceinline__ void multiply(const Args& g, Acc<BM>& acc, int m_lim, int n_lim, char* lds) {
-  clear<BM>(acc);
+template <bool A_MC, bool B_MC, typename S, bool DUAL>
+__device__ __forceinline__ void multiply(const Args& g, typename S::Acc& acc, int m_lim, int n_lim, char* lds) {
+  clear<S>(acc);
   float operand = 0.f;
   if (!A_MC || g.k > kFewTerms) {   // NN / NT: k is a multiple of 4
-    multiply_as<A_MC, B_MC, BM, DUAL, false>(g, acc, lds, operand);
-    if (!sums_need_fp32<A_MC, B_MC, BM, DUAL>(g, acc, operand, m_lim, n_lim)) return;
-    clear<BM>(acc);
+    multiply_as<A_MC, B_MC, S, DUAL, false>(g, acc, lds, operand);
+    if (!sums_need_fp32<A_MC, B_MC, S, DUAL>(g, acc, operand, m_lim, n_lim)) return;
+    clear<S>(acc);
   }
-  multiply_as<A_MC, B_MC, BM, DUAL, true>(g, acc, lds, operand);
+  multiply_as<A_MC, B_MC, S, DUAL, true>(g, acc, lds, operand);
 }
 
 // c[m][n] = acc for the tile's rows below m_lim and columns below n (n a multiple of 4, c 16-byte aligned)
-template <int BM>
-__device__ __forceinline__ void store(const Acc<BM>& acc, float* __restrict__ c, int64_t ldc, int m_lim, int n0, int n) {
+template <typename S>
+__device__ __forceinline__ void store(const typename S::Acc& acc, float* __restrict__ c, int64_t ldc, int m_lim, int n0, int n) {
   const int wave = threadIdx.x / kWave, lane = lane_id();
-  const int wm = (wave / 2) * (BM / 2), wn = (wave % 2) * 64;
+  const int wm = S::row(wave), wn = S::column(wave);
 #pragma unroll
-  for (int i = 0; i < BM / 32; ++i) {
+  for (int i = 0; i < S::TM; ++i) {
     const int m = wm + 16 * i + (lane & 15);
     if (m >= m_lim) continue;
     float* const row = c + (int64_t)m * ldc;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
+    for (int j = 0; j < S::TN; ++j) {
       const int col = n0 + wn + 16 * j + 4 * (lane >> 4);
       if (col < n) *(f32x4*)(row + col) = acc[i][j];
     }
@@ -425,15 +482,15 @@ __device__ __forceinline__ void store(const Acc<BM>& acc, float* __restrict__ c,
 // the workspace and returns whether this workgroup was the tile's last, which then holds the sum of all parts in
 // `acc`, added in part order whoever came last.  The parts go past the caches (workgroups of a tile sit on different
 // XCDs), a part is counted in once its stores are acknowledged, and nobody waits for anybody: see gmm_dma.h.
-template <int BM>
-__device__ __forceinline__ bool join_parts(Acc<BM>& acc, int tile, int tiles, int part, int ksplit, int32_t* counters,
+template <typename S>
+__device__ __forceinline__ bool join_parts(typename S::Acc& acc, int tile, int tiles, int part, int ksplit, int32_t* counters,
                                            float* parts, char* lds) {
-  constexpr int kThroughCaches = 0x11, kPieces = BM / 32 * 4;   // sc0 | sc1; 16-byte pieces per lane
+  constexpr int kThroughCaches = 0x11, kPieces = S::TM * S::TN;   // sc0 | sc1; 16-byte pieces per lane
   const uint32_t lane_off = threadIdx.x * 16u;
-  const __amdgpu_buffer_rsrc_t mine = make_rsrc((const char*)parts + ((size_t)part * tiles + tile) * kPartBytes, (uint32_t)kPartBytes);
+  const __amdgpu_buffer_rsrc_t mine = make_rsrc((const char*)parts + ((size_t)part * tiles + tile) * S::kPartBytes, (uint32_t)S::kPartBytes);
 #pragma unroll
   for (int p = 0; p < kPieces; ++p)
-    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, acc[p / 4][p % 4]), mine, (int)lane_off, p * (kThreads * 16), kThroughCaches);
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, acc[p / S::TN][p % S::TN]), mine, (int)lane_off, p * (kThreads * 16), kThroughCaches);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
   int* const flag = (int*)lds;
@@ -446,7 +503,7 @@ __device__ __forceinline__ bool join_parts(Acc<BM>& acc, int tile, int tiles, in
     f32x4 sum[4];
 #pragma unroll 1
     for (int q = 0; q < ksplit; ++q) {
-      const __amdgpu_buffer_rsrc_t theirs = make_rsrc((const char*)parts + ((size_t)q * tiles + tile) * kPartBytes, (uint32_t)kPartBytes);
+      const __amdgpu_buffer_rsrc_t theirs = make_rsrc((const char*)parts + ((size_t)q * tiles + tile) * S::kPartBytes, (uint32_t)S::kPartBytes);
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
         const f32x4 w = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(theirs, (int)lane_off, (p + u) * (kThreads * 16), kThroughCaches));
@@ -454,25 +511,25 @@ __device__ __forceinline__ bool join_parts(Acc<BM>& acc, int tile, int tiles, in
       }
     }
 #pragma unroll
-    for (int u = 0; u < 4; ++u) acc[p / 4][u] = sum[u];
+    for (int u = 0; u < 4; ++u) acc[(p + u) / S::TN][(p + u) % S::TN] = sum[u];
   }
   if (threadIdx.x == 0) counters[tile] = 0;   // as the launch found it
   return true;
 }
 
 // ---- NN / NT ----
-// P = gridDim.x workgroups (two per compute unit) walk the list of tiles as those of gmm_dma.h's kernel do.  The tiles of a
+// P = gridDim.x workgroups (one per compute unit, two of the small tile) walk the list of tiles as those of gmm_dma.h's kernel do.  The tiles of a
 // last round that would leave at least half of the workgroups idle are cut along the reduction when there is a
 // workspace: with four and a half rounds of long reductions (8 experts of 1024 rows: 4.4 rounds NT, 1.1 NN) the tail
 // would otherwise take as long as a full round.
-template <bool B_MC, int BM, bool DUAL>
-__global__ void __launch_bounds__(kThreads, 2)
+template <bool B_MC, typename S, bool DUAL>
+__global__ void __launch_bounds__(kThreads, 2 * S::kPerUnit)
 gmm_f32_rows_kernel(const float* __restrict__ a, const float* __restrict__ b, float* __restrict__ c, const int32_t* __restrict__ bins,
                     int num_groups, int64_t rows, int k, int n, int tiles_n, const float* __restrict__ a2, const float* __restrict__ b2,
                     int32_t* __restrict__ ws_counters, float* ws_parts, int ws_capacity) {
   extern __shared__ __attribute__((aligned(1024))) char lds[];
   const int P = gridDim.x, run = P / kXcds, xcd = blockIdx.x % kXcds, member = blockIdx.x / kXcds;
-  const RowTiles<BM> tiles(bins, num_groups, tiles_n, (int)rows, false, 8);
+  const RowTiles<S::BM> tiles(bins, num_groups, tiles_n, (int)rows, false, 8);
   const int total = tiles.total, full_rounds = total / P, rest = total - full_rounds * P;
   Args g;
   g.a_ld = (uint32_t)k * 4u;
@@ -509,7 +566,7 @@ gmm_f32_rows_kernel(const float* __restrict__ a, const float* __restrict__ b, fl
     }
     int e, start, end, tm, tn;
     tiles.find(id, e, start, end, tm, tn);
-    const int row0 = start + tm * BM;
+    const int row0 = start + tm * S::BM;
     // up to the expert's last row: the next expert's rows, or rows behind the last bin that nobody may have written, must not
     // have a say in which instruction forms these sums
     const uint32_t a_bytes = clip_bytes((int64_t)(end - row0) * k * 4), b_bytes = (uint32_t)((int64_t)k * n * 4);
@@ -517,13 +574,13 @@ gmm_f32_rows_kernel(const float* __restrict__ a, const float* __restrict__ b, fl
     g.rsrc_b = make_rsrc(b + (int64_t)e * k * n, b_bytes);
     g.rsrc_a2 = DUAL ? make_rsrc(a2 + (int64_t)row0 * k, a_bytes) : g.rsrc_a;
     g.rsrc_b2 = DUAL ? make_rsrc(b2 + (int64_t)e * k * n, b_bytes) : g.rsrc_b;
-    g.b_r0 = tn * kBN;
+    g.b_r0 = tn * S::BN;
     g.kt0 = cut ? (int)((int64_t)part * nk / ksplit) : 0;
     g.kt1 = cut ? (int)((int64_t)(part + 1) * nk / ksplit) : nk;
-    Acc<BM> acc;
-    multiply<false, B_MC, BM, DUAL>(g, acc, end - row0, n - g.b_r0, lds);
-    if (!cut || join_parts<BM>(acc, id - full_rounds * P, rest, part, ksplit, ws_counters, ws_parts, lds))
-      store<BM>(acc, c + (int64_t)row0 * n, n, end - row0, g.b_r0, n);
+    typename S::Acc acc;
+    multiply<false, B_MC, S, DUAL>(g, acc, end - row0, n - g.b_r0, lds);
+    if (!cut || join_parts<S>(acc, id - full_rounds * P, rest, part, ksplit, ws_counters, ws_parts, lds))
+      store<S>(acc, c + (int64_t)row0 * n, n, end - row0, g.b_r0, n);
     tile_done();
   }
 }
@@ -531,13 +588,14 @@ gmm_f32_rows_kernel(const float* __restrict__ a, const float* __restrict__ b, fl
 // ---- TN ----
 // One workgroup per tile and part of its reduction; ksplit is the launch's (> 1: there are few tiles and a workspace).
 // Experts are taken longest reduction first (every wave ranks up to 64 of them), so that the last tiles are short ones.
-__global__ void __launch_bounds__(kThreads, 2)
+template <typename S>
+__global__ void __launch_bounds__(kThreads, 2 * S::kPerUnit)
 gmm_f32_tn_kernel(const float* __restrict__ a, const float* __restrict__ b, float* __restrict__ c, const int32_t* __restrict__ bins,
                   int num_groups, int rows, int k, int n, int tiles_m, int tiles_n, int ksplit, int32_t* __restrict__ ws_counters,
                   float* ws_parts) {
   extern __shared__ __attribute__((aligned(1024))) char lds[];
   const int per_group = tiles_m * tiles_n, total = per_group * num_groups;
-  const int id = xcd_tile_id(blockIdx.x, 2 * kXcdRun);
+  const int id = xcd_tile_id(blockIdx.x, S::kPerUnit * kXcdRun);
   if (id >= total * ksplit) return;
   const int tile = id % total, part = id / total;
   int e = tile / per_group;
@@ -546,7 +604,7 @@ gmm_f32_tn_kernel(const float* __restrict__ a, const float* __restrict__ b, floa
     const int mine = lane < num_groups ? bins[lane] - (lane > 0 ? bins[lane - 1] : 0) : -1;
     int rank = 0;
     for (int o = 0; o < num_groups; ++o) {
-      const int other = __shfl(mine, o, kWave);
+      const int other = __builtin_amdgcn_readlane(mine, o);
       rank += (other > mine || (other == mine && o < lane)) ? 1 : 0;
     }
     if (lane >= num_groups) rank = -1;
@@ -563,8 +621,8 @@ gmm_f32_tn_kernel(const float* __restrict__ a, const float* __restrict__ b, floa
   Args g;
   g.a_ld = (uint32_t)k * 4u;
   g.b_ld = (uint32_t)n * 4u;
-  g.a_r0 = tm * 128;
-  g.b_r0 = tn * kBN;
+  g.a_r0 = tm * S::BM;
+  g.b_r0 = tn * S::BN;
   g.k = end - start;
   const int nk = (end - start + kBK - 1) / kBK;
   g.nk1 = nk;
@@ -575,10 +633,49 @@ gmm_f32_tn_kernel(const float* __restrict__ a, const float* __restrict__ b, floa
   g.rsrc_b2 = g.rsrc_b;
   g.kt0 = (int)((int64_t)part * nk / ksplit);
   g.kt1 = (int)((int64_t)(part + 1) * nk / ksplit);
-  Acc<128> acc;
-  multiply<true, true, 128, false>(g, acc, k - g.a_r0, n - g.b_r0, lds);
-  if (ksplit > 1 && !join_parts<128>(acc, tile, total, part, ksplit, ws_counters, ws_parts, lds)) return;
-  store<128>(acc, c + ((int64_t)e * k + g.a_r0) * n, n, k - g.a_r0, g.b_r0, n);
+  typename S::Acc acc;
+  multiply<true, true, S, false>(g, acc, k - g.a_r0, n - g.b_r0, lds);
+  if (ksplit > 1 && !join_parts<S>(acc, tile, total, part, ksplit, ws_counters, ws_parts, lds)) return;
+  store<S>(acc, c + ((int64_t)e * k + g.a_r0) * n, n, k - g.a_r0, g.b_r0, n);
+}
+
+template <bool B_MC, typename S, bool DUAL>
+int launch_rows(const float* a, const float* b, float* c, const int32_t* bins, int num_groups, int64_t rows, int k, int n, const float* a2,
+                const float* b2, const Workspace& lent, int units, hipStream_t s) {
+  WorkspaceParts ws(lent, S::kPartBytes);
+  if (units > (int)kWorkspaceCounters) ws.parts = nullptr;   // at most half of the workgroups' tiles are cut
+  auto kern = gmm_f32_rows_kernel<B_MC, S, DUAL>;
+  const int rc = allow_lds(kern, S::kLdsBytes);
+  if (rc) return rc;
+  kern<<<(unsigned)(S::kPerUnit * units), kThreads, S::kLdsBytes, s>>>(a, b, c, bins, num_groups, rows, k, n, (int)ceil_div(n, S::BN), a2, b2,
+                                                                      ws.counters, ws.parts, ws.capacity);
+  return launch_status();
+}
+
+template <typename S>
+int launch_tn(const float* a, const float* b, float* c, const int32_t* bins, int num_groups, int64_t rows, int k, int n,
+              const Workspace& lent, int units, hipStream_t s) {
+  WorkspaceParts ws(lent, S::kPartBytes);
+  if (units > (int)kWorkspaceCounters) ws.parts = nullptr;
+  const int tiles_m = (int)ceil_div(k, S::BM), tiles_n = (int)ceil_div(n, S::BN);
+  const int64_t total = (int64_t)tiles_m * tiles_n * num_groups;
+  if (total * kMaxKSplit > 0x7fffff00) return MBX_ERANGE;
+  int64_t ksplit = 1;
+  const int slots = S::kPerUnit * units;
+  if (ws.parts && 2 * total <= slots) {
+    const int64_t nk = rows / num_groups / kBK;
+    ksplit = slots / total;
+    ksplit = ksplit > kMaxKSplit ? kMaxKSplit : ksplit;
+    ksplit = ksplit > nk / kMinPartTiles ? nk / kMinPartTiles : ksplit;
+    ksplit = ksplit * total > ws.capacity ? ws.capacity / total : ksplit;
+    ksplit = ksplit < 2 ? 1 : ksplit;
+  }
+  auto kern = gmm_f32_tn_kernel<S>;
+  const int rc = allow_lds(kern, S::kLdsBytes);
+  if (rc) return rc;
+  kern<<<(unsigned)xcd_grid(total * ksplit, S::kPerUnit * kXcdRun), kThreads, S::kLdsBytes, s>>>(a, b, c, bins, num_groups, (int)rows, k, n, tiles_m, tiles_n,
+                                                                         (int)ksplit, ws.counters, ws.parts);
+  return launch_status();
 }
 
 }  // namespace f32
@@ -600,10 +697,13 @@ static inline bool f32_short_tn(int num_groups, int64_t rows, int k) {
   return rows <= 24 * (int64_t)num_groups && ceil_div(k, 128) <= 65535 && num_groups <= 65535;
 }
 
-// Tiles of 64 rows up to 192 rows per expert on average: of full ones an expert of that many leaves a quarter and more of
-// the multiplications to padding, which this kernel, bound by the matrix cores, pays in full (64 experts of 100 - 156 rows,
-// 1024 x 1408: 228 us NT).
-constexpr int64_t kF32ShortRows = 192;
+// The small tile, two workgroups to a compute unit, where the main tile would leave three eighths of the compute units or more
+// without one (us, main / small tile: NT 8 experts of 256 rows, [1408, 512]: 40 / 29; 4 of 1500, [704, 4096], 144 tiles: 240 / 218; 32 of
+// 100, [1408, 1024], 192 tiles: 75 / 80.  TN 8 of 512, [1024, 512], 128 tiles: 41 / 31; 8 of 256, [1408, 512], 176 tiles: 29 / 34), and in
+// NN / NT launches of up to 64 rows per expert on average, whose tiles would be half empty (64 experts of 64, [1408, 1024]:
+// 140 / 118; of 100: 157 / 158).
+static inline bool f32_small(int64_t tiles, int units) { return 8 * tiles < 5 * (int64_t)units; }
+constexpr int64_t kF32SmallRows = 64;
 
 }  // namespace
 
@@ -613,40 +713,20 @@ int gmm_f32(const void* a, const void* b, const void* a2, const void* b2, void* 
   if (!f32_ok(a, b, c, rows, k, n, layout) || (a2 && !f32_ok(a2, b2, c, rows, k, n, layout))) return MBX_EUNSUPPORTED;
   const float *ap = (const float*)a, *bp = (const float*)b, *ap2 = (const float*)a2, *bp2 = (const float*)b2;
   float* cp = (float*)c;
-  WorkspaceParts ws(Workspace{workspace, workspace_bytes}, f32::kPartBytes);
-  const int slots = 2 * persistent_grid((int64_t)1 << 30);   // two workgroups per compute unit
-  if (slots / 2 > (int)kWorkspaceCounters) ws.parts = nullptr;
+  const Workspace lent{workspace, workspace_bytes};
+  const int units = persistent_grid((int64_t)1 << 30);
   if (layout == MBX_TN) {
-    const int tiles_m = (int)ceil_div(k, 128), tiles_n = (int)ceil_div(n, f32::kBN);
-    const int64_t total = (int64_t)tiles_m * tiles_n * num_groups;
-    if (total * f32::kMaxKSplit > 0x7fffff00) return MBX_ERANGE;
-    int64_t ksplit = 1;
-    if (ws.parts && 2 * total <= slots) {
-      const int64_t nk = rows / num_groups / f32::kBK;
-      ksplit = slots / total;
-      ksplit = ksplit > f32::kMaxKSplit ? f32::kMaxKSplit : ksplit;
-      ksplit = ksplit > nk / f32::kMinPartTiles ? nk / f32::kMinPartTiles : ksplit;
-      ksplit = ksplit * total > ws.capacity ? ws.capacity / total : ksplit;
-      ksplit = ksplit < 2 ? 1 : ksplit;
-    }
-    int rc = allow_lds(f32::gmm_f32_tn_kernel, f32::kLdsBytes);
-    if (rc) return rc;
-    f32::gmm_f32_tn_kernel<<<(unsigned)xcd_grid(total * ksplit, 2 * kXcdRun), f32::kThreads, f32::kLdsBytes, s>>>(
-        ap, bp, cp, bins, num_groups, (int)rows, k, n, tiles_m, tiles_n, (int)ksplit, ws.counters, ws.parts);
-    return launch_status();
+    const int64_t wide = ceil_div(k, 128) * ceil_div(n, 256), tall = ceil_div(k, 256) * ceil_div(n, 128);
+    if (f32_small(num_groups * (tall < wide ? tall : wide), units)) return f32::launch_tn<f32::Small>(ap, bp, cp, bins, num_groups, rows, k, n, lent, units, s);
+    return tall < wide ? f32::launch_tn<f32::Tall>(ap, bp, cp, bins, num_groups, rows, k, n, lent, units, s)
+                       : f32::launch_tn<f32::Wide>(ap, bp, cp, bins, num_groups, rows, k, n, lent, units, s);
   }
-  const int tiles_n = (int)ceil_div(n, f32::kBN);
-  const bool short_tiles = rows <= kF32ShortRows * num_groups;
-  if ((ceil_div(rows, 64) + num_groups) * tiles_n > 0x7fffffff) return MBX_ERANGE;
-#define MBX_LAUNCH_F32(B_MC, BM, DUAL)                                                                            \
-  do {                                                                                                            \
-    auto kern = f32::gmm_f32_rows_kernel<B_MC, BM, DUAL>;                                                         \
-    int rc = allow_lds(kern, f32::kLdsBytes);                                                                     \
-    if (rc) return rc;                                                                                            \
-    kern<<<(unsigned)slots, f32::kThreads, f32::kLdsBytes, s>>>(ap, bp, cp, bins, num_groups, rows, k, n, tiles_n, ap2, bp2, \
-                                                                ws.counters, ws.parts, ws.capacity);              \
-  } while (0)
-#define MBX_LAUNCH_F32_BM(B_MC, DUAL) do { if (short_tiles) MBX_LAUNCH_F32(B_MC, 64, DUAL); else MBX_LAUNCH_F32(B_MC, 128, DUAL); } while (0)
+  if ((ceil_div(rows, 64) + num_groups) * ceil_div(n, 128) > 0x7fffffff) return MBX_ERANGE;
+  // an expert's rows in whole tiles
+  const int64_t average = ceil_div(rows, num_groups), tiles = num_groups * ceil_div(average, 128) * ceil_div(n, 256);
+  const bool small = average <= kF32SmallRows || f32_small(tiles, units);
+#define MBX_LAUNCH_F32(B_MC, S, DUAL) return f32::launch_rows<B_MC, S, DUAL>(ap, bp, cp, bins, num_groups, rows, k, n, ap2, bp2, lent, units, s)
+#define MBX_LAUNCH_F32_BM(B_MC, DUAL) do { if (small) MBX_LAUNCH_F32(B_MC, f32::Small, DUAL); else MBX_LAUNCH_F32(B_MC, f32::Wide, DUAL); } while (0)
   if (layout == MBX_NT) {
     if (a2) MBX_LAUNCH_F32_BM(false, true); else MBX_LAUNCH_F32_BM(false, false);
   } else {
@@ -654,7 +734,6 @@ int gmm_f32(const void* a, const void* b, const void* a2, const void* b2, void* 
   }
 #undef MBX_LAUNCH_F32_BM
 #undef MBX_LAUNCH_F32
-  return launch_status();
 }
 
 }  // namespace mbx

@@ -980,6 +980,37 @@ def test_gmm_fp32_on_the_matrix_cores(gg, monkeypatch, groups, rows, k, n, mode)
         assert torch.equal(got[-1].nan_to_num(), got[-2].nan_to_num())
 
 
+@pytest.mark.parametrize('mode,rows,k,n', [
+    ('nn', 700, 68, 4100), ('nt', 700, 68, 4100), ('dual_nn', 700, 36, 4100), ('dual_nt', 641, 36, 4100),   # 128 x 256
+    ('nn', 321, 36, 4100), ('nt', 321, 36, 4100), ('nt', 1300, 68, 260),   # 64 x 128: few rows, few tiles
+    ('tn', 700, 260, 4100), ('tn', 700, 132, 4100), ('tn', 700, 132, 260),   # 128 x 256, 256 x 128, 64 x 128
+])
+def test_gmm_fp32_tiles_with_values_off_the_parts(gg, mode, rows, k, n):
+    """Every tile shape of the fp32 kernels, five experts, with rows of the product 2^-100 and 2^45 times the others (tiles formed
+    again on the fp32 instruction next to tiles that are not), row by row against fp64: a sum of r terms, with a factor of four to
+    spare."""
+    torch.manual_seed(rows + k)
+    trans_b, dual = mode.endswith('nt'), mode.startswith('dual')
+    sizes = _sizes(5, rows, seed=rows)
+    wshape = (rows, n) if mode == 'tn' else (5, n, k) if trans_b else (5, k, n)
+    a, a2 = (torch.randn(rows, k, device='cuda') for _ in range(2))
+    b, b2 = (torch.randn(wshape, device='cuda') for _ in range(2))
+    for x in (a, a2):
+        view = x.t() if mode == 'tn' else x
+        view[3] *= 2.0 ** -100
+        view[-2] *= 2.0 ** 45
+
+    def exact(x, w):
+        parts = list(zip(x.double().split(sizes.tolist()), w.double().split(sizes.tolist()) if mode == 'tn' else w.double()))
+        return torch.cat([p.t() @ q if mode == 'tn' else p @ (q.t() if trans_b else q) for p, q in parts])
+    want = exact(a, b) + (exact(a2, b2) if dual else 0)
+    got = gg.gmm_dual(a, b, a2, b2, sizes, trans_b=trans_b) if dual else gg.backend.gmm(a, b, sizes, trans_a=mode == 'tn', trans_b=trans_b)
+    got = got.double().reshape(want.shape)
+    length = int(sizes.max()) if mode == 'tn' else k * (2 if dual else 1)
+    error = (got - want).norm(dim=1) / want.norm(dim=1).clamp_min(1e-300)
+    assert float(error.max()) < 4 * 2.0 ** -24 * math.sqrt(max(length, 16)), error.argmax()
+
+
 @pytest.mark.parametrize('other', [float('inf'), float('nan'), 2.0 ** 40, 2.0 ** -80])
 @pytest.mark.parametrize('mode', ['nn', 'nt', 'dual_nn', 'dual_nt'])
 def test_gmm_fp32_rows_do_not_depend_on_the_rows_behind_them(gg, mode, other):
