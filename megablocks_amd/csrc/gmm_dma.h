@@ -1808,21 +1808,20 @@ gmm_tn_kernel(const uint16_t* __restrict__ a, const uint16_t* __restrict__ b, ui
   if (ranked) {
     const int lane = lane_id();
     const int mine = lane < num_groups ? bins[lane] - (lane > 0 ? bins[lane - 1] : 0) : -1;
-    rank = 0;
-    for (int o = 0; o < num_groups; ++o) {
-      const int other = __shfl(mine, o, kWave);
-      rank += (other > mine || (other == mine && o < lane)) ? 1 : 0;
-    }
-    if (lane >= num_groups) rank = -1;
+    rank = rank_by_rows(mine, num_groups);
     if (whole_ok && num_groups >= kXcds) {
       const int home = rank < 0 ? -1 : serpentine_xcd(rank);
-      int worst = 0, total = 0;
-      for (int x = 0; x < kXcds; ++x) {
-        int v = home == x ? (mine > 0 ? mine : 0) : 0;
+      int worst = 0, total = 0, load[kXcds];   // the sums of all XCDs step by step, so that their shuffles overlap
 #pragma unroll
-        for (int o = kWave / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, kWave);
-        worst = v > worst ? v : worst;
-        total += v;
+      for (int x = 0; x < kXcds; ++x) load[x] = home == x ? (mine > 0 ? mine : 0) : 0;
+#pragma unroll
+      for (int o = kWave / 2; o > 0; o >>= 1)
+#pragma unroll
+        for (int x = 0; x < kXcds; ++x) load[x] += __shfl_xor(load[x], o, kWave);
+#pragma unroll
+      for (int x = 0; x < kXcds; ++x) {
+        worst = load[x] > worst ? load[x] : worst;
+        total += load[x];
       }
       whole = (int64_t)worst * kXcds * 200 <= (int64_t)total * 203;
     }

@@ -601,13 +601,7 @@ gmm_f32_tn_kernel(const float* __restrict__ a, const float* __restrict__ b, floa
   int e = tile / per_group;
   if (num_groups <= kWave) {
     const int lane = lane_id();
-    const int mine = lane < num_groups ? bins[lane] - (lane > 0 ? bins[lane - 1] : 0) : -1;
-    int rank = 0;
-    for (int o = 0; o < num_groups; ++o) {
-      const int other = __builtin_amdgcn_readlane(mine, o);
-      rank += (other > mine || (other == mine && o < lane)) ? 1 : 0;
-    }
-    if (lane >= num_groups) rank = -1;
+    const int rank = rank_by_rows(lane < num_groups ? bins[lane] - (lane > 0 ? bins[lane - 1] : 0) : -1, num_groups);
     e = __builtin_amdgcn_readfirstlane((int)__builtin_ctzll(__ballot(rank == e)));
   }
   // tiles of an expert in bands of eight row tiles (the last band takes what is left), rows fastest
