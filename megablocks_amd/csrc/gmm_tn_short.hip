@@ -12,7 +12,7 @@
 //   8 experts, [4096, 14336]:   202 / 167,  222 / 192,  259 / 232,  265 / 228,  370 / 350
 //   128 experts, [768, 2048]:   88 / 66,  100 / 81,  121 / 99,  154 / 139,  174 / 146
 //   32 experts, [1032, 2728]:   62 / 60,  64 / 60,  70 / 62,  86 / 76,  92 / 81
-// (4 rows of the first: 537 MB stored, 6.2 TB/s.)  Neighbours that store to different rows cost that case 100 instead of 87 us.
+// (4 rows of the first: 537 MB stored, 6.2 TB/s; operands in the last-level cache, without Prefetch.)  Neighbours that store to different rows cost that case 100 instead of 87 us.
 //
 // Layouts are gmm_dma.h's for strided operands of 128 columns: [k][128] rows, transposing reads.
 #include "gmm_common.h"
@@ -44,8 +44,107 @@ __device__ __forceinline__ f32x4 mfma(const u32x4& a, const u32x4& b, const f32x
   return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, a), __builtin_bit_cast(f16x8_t, b), c, 0, 0, 0);
 }
 
+// Which tile the workgroups of an XCD take: at(member) for its `member`-th, in the order they start.
+// Experts that are alike go to the XCDs in whole runs: an expert's panels are then fetched into one L2.  With one of more
+// than twice the average every XCD takes a part of each, those experts first (up to 64 experts; more come as they are).
+struct Tiles {
+  struct Tile { int e, tm, tn; };
+  int num_groups, rows, tiles_m, tiles_n, xcd, mine = 0, wide;
+  bool alike;
+
+  __device__ __forceinline__ Tiles(const int32_t* __restrict__ bins, int num_groups_, int rows_, int tiles_m_, int tiles_n_)
+      : num_groups(num_groups_), rows(rows_), tiles_m(tiles_m_), tiles_n(tiles_n_), xcd(blockIdx.x % kXcds) {
+    int most = 0;
+    for (int e0 = 0; e0 < num_groups; e0 += kWave) {
+      const int e = e0 + lane_id();
+      mine = e < num_groups ? clamp_row(bins[e], rows) - (e > 0 ? clamp_row(bins[e - 1], rows) : 0) : -1;
+      most = mine > most ? mine : most;
+    }
+#pragma unroll
+    for (int o = kWave / 2; o > 0; o >>= 1) {
+      const int other = __shfl_xor(most, o, kWave);
+      most = other > most ? other : most;
+    }
+    alike = (int64_t)__builtin_amdgcn_readfirstlane(most) * num_groups <= 2 * (int64_t)rows;
+    // bands of column tiles whose panel of b takes an L2 1.5 MiB; of few panels in a part of an expert
+    const int average = (int)((int64_t)rows / num_groups) + 1, fits = 6144 / average;
+    wide = alike && fits > 8 ? fits : 8;
+    wide = wide < tiles_n ? wide : tiles_n;
+  }
+  // Tile t of an expert: in bands of column tiles, a band's columns fastest, so that neighbours store to the same rows.
+  __device__ __forceinline__ void place(int t, Tile& tile) const {
+    const int band = t / (wide * tiles_m), left = tiles_n - band * wide, w = left < wide ? left : wide, in = t - band * wide * tiles_m;
+    tile.tm = in / w;
+    tile.tn = band * wide + in % w;
+  }
+  __device__ __forceinline__ bool at(int member, Tile& tile) const {   // false: there is none
+    const int per_group = tiles_m * tiles_n;
+    if (alike) {
+      const int64_t total = (int64_t)per_group * num_groups, share = (total + kXcds - 1) / kXcds, id = xcd * share + member;
+      if (member >= share || id >= total) return false;
+      tile.e = (int)(id / per_group);
+      place((int)(id % per_group), tile);
+    } else {
+      const int share = (per_group + kXcds - 1) / kXcds;
+      tile.e = member / share;
+      const int t = xcd * share + member % share;
+      if (tile.e >= num_groups || t >= per_group) return false;
+      place(t, tile);
+      if (num_groups <= kWave) {
+        // a full ranking is a loop over the experts in every workgroup: 40 of 250 us for 64 experts of 256 rows
+        const int lane = lane_id();
+        const bool exists = lane < num_groups, large = exists && (int64_t)mine * num_groups > 2 * (int64_t)rows;
+        const uint64_t larger = __ballot(large), others = __ballot(exists && !large), before = ((uint64_t)1 << lane) - 1;
+        const int rank = !exists ? -1 : large ? __popcll(larger & before) : __popcll(larger) + __popcll(others & before);
+        tile.e = __builtin_amdgcn_readfirstlane((int)__builtin_ctzll(__ballot(rank == tile.e)));
+      }
+    }
+    return true;
+  }
+};
+
+// An expert's rows, inside [0, rows] and in order whatever the table holds.
+__device__ __forceinline__ void expert_rows(const int32_t* __restrict__ bins, int e, int rows, int& start, int& count) {
+  start = e > 0 ? clamp_row(bins[e - 1], rows) : 0;
+  const int end = clamp_row(bins[e], rows);
+  count = end < start ? 0 : end - start;
+}
+
+// The operands of the tile a workgroup of this XCD will start with when the ones running now are done, fetched into the L2 by
+// those: the rows of a (columns of its row tile) by the workgroups of the tiles beside it, a share each, and the rows of b likewise
+// where an expert begins.  A workgroup's first loads otherwise wait for memory that is busy with the stores of the others, a
+// few microseconds in each of its 10 to 20: 64 experts, [1024, 4096], operands and products not in the last-level cache: 128 rows
+// 184 -> 165 us, 256 rows 238 -> 210.  One dword a lane, a lane a 128-byte line; out of range: no access.
+template <int BM, int BN, int AHEAD>
+struct Prefetch {
+  __amdgpu_buffer_rsrc_t ra, rb;
+  uint32_t a_at = 0x80000000u, b_at = 0x80000000u, a = 0, b = 0;
+  // behind the workgroup's own first loads
+  __device__ __forceinline__ Prefetch(const Tiles& tiles, int e, const uint16_t* __restrict__ pa, const uint16_t* __restrict__ pb,
+                                      const int32_t* __restrict__ bins, int k, int n) {
+    Tiles::Tile next;
+    int start = 0, count = 0;
+    if (tiles.at(blockIdx.x / kXcds + AHEAD, next)) {
+      expert_rows(bins, next.e, tiles.rows, start, count);
+      constexpr int kLinesA = BM * 2 / 128, kLinesB = BN * 2 / 128;   // of a row
+      const int thread = threadIdx.x, line_a = next.tn % tiles.wide * 256 + thread;
+      const int line_b = next.tm % (AHEAD / 8) * 256 + thread;        // eight column tiles or more at a time
+      if (line_a / kLinesA < count) a_at = (uint32_t)(line_a / kLinesA) * (uint32_t)k * 2u + (uint32_t)(next.tm * kLinesA + line_a % kLinesA) * 128u;
+      if (line_b / kLinesB < count && next.e != e) b_at = (uint32_t)(line_b / kLinesB) * (uint32_t)n * 2u + (uint32_t)(next.tn * kLinesB + line_b % kLinesB) * 128u;
+    }
+    ra = make_rsrc(pa + (int64_t)start * k, (uint32_t)((int64_t)count * k * 2));
+    rb = make_rsrc(pb + (int64_t)start * n, (uint32_t)((int64_t)count * n * 2));
+  }
+  __device__ __forceinline__ void issue() {   // where no loads follow that are waited for
+    a = __builtin_amdgcn_raw_buffer_load_b32(ra, (int)a_at, 0, 0);
+    b = __builtin_amdgcn_raw_buffer_load_b32(rb, (int)b_at, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  __device__ __forceinline__ void arrived() const { asm volatile("" ::"v"(a), "v"(b)); }   // behind the stores
+};
+
 // OUT32: c is fp32.  GATHER: the rows of b are picked through gmm_dma.h's row table (there: gmm_tn_kernel).
-template <int DT, bool GATHER, bool OUT32>
+template <int DT, bool GATHER, bool OUT32, bool AHEAD>
 __global__ void __launch_bounds__(T::THREADS, kPerCu)
 gmm_tn_short_kernel(const uint16_t* __restrict__ a, const uint16_t* __restrict__ b, uint16_t* __restrict__ c,
                     const int32_t* __restrict__ bins, int num_groups, int rows, int k, int n, int tiles_m, int tiles_n,
@@ -54,60 +153,18 @@ gmm_tn_short_kernel(const uint16_t* __restrict__ a, const uint16_t* __restrict__
   const lds_ptr lds = (lds_ptr)lds_generic;
   const uint32_t lds_base = (uint32_t)(uintptr_t)lds;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = lane_id();
-  const int per_group = tiles_m * tiles_n, xcd = blockIdx.x % kXcds, member = blockIdx.x / kXcds;
-  // Experts that are alike go to the XCDs in whole runs: an expert's panels are then fetched into one L2.  With one of more
-  // than twice the average every XCD takes a part of each, those experts first (up to 64 experts; more come as they are).
-  int mine = 0, most = 0;
-  for (int e0 = 0; e0 < num_groups; e0 += kWave) {
-    const int e = e0 + lane;
-    mine = e < num_groups ? clamp_row(bins[e], rows) - (e > 0 ? clamp_row(bins[e - 1], rows) : 0) : -1;
-    most = mine > most ? mine : most;
-  }
-#pragma unroll
-  for (int o = kWave / 2; o > 0; o >>= 1) {
-    const int other = __shfl_xor(most, o, kWave);
-    most = other > most ? other : most;
-  }
-  most = __builtin_amdgcn_readfirstlane(most);
-  int e, tm, tn;
-  // Tile t of an expert: in bands of column tiles whose panel of b takes an L2 1.5 MiB, a band's columns fastest, so that
-  // neighbours store to the same rows.
-  const int average = (int)((int64_t)rows / num_groups) + 1, fits = 6144 / average;
-  int wide = fits > 8 ? fits : 8;
-  auto place = [&](int t) {
-    const int band = t / (wide * tiles_m), left = tiles_n - band * wide, w = left < wide ? left : wide, in = t - band * wide * tiles_m;
-    tm = in / w;
-    tn = band * wide + in % w;
-  };
-  if ((int64_t)most * num_groups <= 2 * (int64_t)rows) {
-    const int64_t total = (int64_t)per_group * num_groups, share = (total + kXcds - 1) / kXcds, id = xcd * share + member;
-    if (member >= share || id >= total) return;
-    e = (int)(id / per_group);
-    place((int)(id % per_group));
-  } else {
-    const int share = (per_group + kXcds - 1) / kXcds;
-    wide = 8;   // a part of few panels
-    e = member / share;
-    const int t = xcd * share + member % share;
-    if (e >= num_groups || t >= per_group) return;
-    place(t);
-    if (num_groups <= kWave) {
-      // a full ranking is a loop over the experts in every workgroup: 40 of 250 us for 64 experts of 256 rows
-      const bool exists = lane < num_groups, large = exists && (int64_t)mine * num_groups > 2 * (int64_t)rows;
-      const uint64_t larger = __ballot(large), others = __ballot(exists && !large), before = ((uint64_t)1 << lane) - 1;
-      const int rank = !exists ? -1 : large ? __popcll(larger & before) : __popcll(larger) + __popcll(others & before);
-      e = __builtin_amdgcn_readfirstlane((int)__builtin_ctzll(__ballot(rank == e)));
-    }
-  }
-  const int start = e > 0 ? clamp_row(bins[e - 1], rows) : 0;
-  int end = clamp_row(bins[e], rows);
-  end = end < start ? start : end;
-  const int nk = (end - start + T::BK - 1) / T::BK;
+  const Tiles tiles(bins, num_groups, rows, tiles_m, tiles_n);
+  Tiles::Tile tile;
+  if (!tiles.at(blockIdx.x / kXcds, tile)) return;
+  const int e = tile.e, tm = tile.tm, tn = tile.tn;
+  int start, count;
+  expert_rows(bins, e, rows, start, count);
+  const int nk = (count + T::BK - 1) / T::BK;
   const uint32_t a_ld = (uint32_t)k * 2u, b_ld = (uint32_t)n * 2u;
   // the buffers cover exactly the expert's rows: later ones read as zeros
-  const __amdgpu_buffer_rsrc_t ra = make_rsrc(a + (int64_t)start * k, (uint32_t)((int64_t)(end - start) * k * 2));
+  const __amdgpu_buffer_rsrc_t ra = make_rsrc(a + (int64_t)start * k, (uint32_t)((int64_t)(count) * k * 2));
   const __amdgpu_buffer_rsrc_t rb = GATHER ? make_rsrc(b, clip_bytes((int64_t)src_rows * n * 2))
-                                           : make_rsrc(b + (int64_t)start * n, (uint32_t)((int64_t)(end - start) * n * 2));
+                                           : make_rsrc(b + (int64_t)start * n, (uint32_t)((int64_t)(count) * n * 2));
   // load j = wave + 4 q (q < 4) of an operand holds rows 4 j .. 4 j + 3 of the K tile, 16 lanes a row
   const uint32_t a_lane = dma::load_lane_offset<true, T::BK, 128>(wave, tm * T::BM, a_ld) + (uint32_t)(4 * wave) * a_ld;
   const uint32_t b_lane = dma::load_lane_offset<true, T::BK, 128>(wave, tn * T::BN, GATHER ? 0u : b_ld) + (GATHER ? 0u : (uint32_t)(4 * wave) * b_ld);
@@ -130,7 +187,7 @@ gmm_tn_short_kernel(const uint16_t* __restrict__ a, const uint16_t* __restrict__
   };
   // Of a last K tile of at most 32 rows (half of the experts, where their rows vary around whole K tiles) the second half, all
   // zeros, is neither loaded nor multiplied (64 experts of 256 +- 16 rows, [1024, 4096]: 187 -> 181 us).
-  const int half_at = nk > 0 && end - start - (nk - 1) * T::BK <= 32 ? nk - 1 : -1;
+  const int half_at = nk > 0 && count - (nk - 1) * T::BK <= 32 ? nk - 1 : -1;
   auto load = [&](int kt) {
 #pragma unroll
     for (int q = 0; q < 4; ++q) {   // rows 16 q .. of the K tile
@@ -176,11 +233,13 @@ gmm_tn_short_kernel(const uint16_t* __restrict__ a, const uint16_t* __restrict__
   for (int i = 0; i < T::TM; ++i)
 #pragma unroll
     for (int j = 0; j < T::TN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  Prefetch<T::BM, T::BN, kPerCu * kXcdRun> prefetch(tiles, e, a, b, bins, k, n);
   for (int kt = 0; kt < nk; ++kt) {
     __builtin_amdgcn_sched_barrier(0);
     dma::wait_vmcnt<0>();
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
+    if (AHEAD && kt + 1 == nk) prefetch.issue();
     read(std::integral_constant<int, 0>{});
     multiply();
     __builtin_amdgcn_sched_barrier(0);
@@ -195,9 +254,127 @@ gmm_tn_short_kernel(const uint16_t* __restrict__ a, const uint16_t* __restrict__
       multiply();
     }
   }
-  dma::wait_vmcnt<0>();
   if constexpr (OUT32) dma::block_store_f32<T>(acc, (float*)c + (int64_t)e * k * n, n, tm * T::BM, k, tn * T::BN, n);
   else dma::block_store<DT, T>(acc, c + (int64_t)e * k * n, n, tm * T::BM, k, tn * T::BN, n, lds_generic);
+  if (AHEAD) prefetch.arrived();
+}
+
+// ---- up to a few hundred rows per expert, many tiles: takes_mid() ----
+// 256 x 128 tiles, two workgroups of four waves to a compute unit, each with three stages of 32 rows: two K tiles under way while one is
+// multiplied, one barrier per K tile.
+typedef dma::Tile<256, 128, 2, 2, 64, 2> TM;   // for its shape
+constexpr int kMidK = 32, kMidStages = 3, kMidPerCu = 2;
+constexpr uint32_t kMidA = TM::BM * kMidK * 2, kMidStage = kMidA + TM::BN * kMidK * 2;
+constexpr size_t kMidLds = TM::EPILOGUE_BYTES > kMidStages * kMidStage ? TM::EPILOGUE_BYTES : kMidStages * kMidStage;
+static_assert(kMidPerCu * kMidLds <= 160 * 1024, "workgroups per compute unit");
+
+template <int N>
+__device__ __forceinline__ void wait_lgkm() {
+  asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(N) : "memory");
+}
+
+template <int DT, bool OUT32>
+__global__ void __launch_bounds__(TM::THREADS, kMidPerCu)
+gmm_tn_mid_kernel(const uint16_t* __restrict__ a, const uint16_t* __restrict__ b, uint16_t* __restrict__ c,
+                  const int32_t* __restrict__ bins, int num_groups, int rows, int k, int n, int tiles_m, int tiles_n) {
+  extern __shared__ __attribute__((aligned(1024))) char lds_generic[];
+  const lds_ptr lds = (lds_ptr)lds_generic;
+  const uint32_t lds_base = (uint32_t)(uintptr_t)lds;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const Tiles tiles(bins, num_groups, rows, tiles_m, tiles_n);
+  Tiles::Tile tile;
+  if (!tiles.at(blockIdx.x / kXcds, tile)) return;
+  const int e = tile.e, tm = tile.tm, tn = tile.tn;
+  int start, count;
+  expert_rows(bins, e, rows, start, count);
+  const int nk = (count + kMidK - 1) / kMidK;
+  const uint32_t a_ld = (uint32_t)k * 2u, b_ld = (uint32_t)n * 2u;
+  // the buffers cover exactly the expert's rows: later ones read as zeros
+  const __amdgpu_buffer_rsrc_t ra = make_rsrc(a + (int64_t)start * k, (uint32_t)((int64_t)(count) * k * 2));
+  const __amdgpu_buffer_rsrc_t rb = make_rsrc(b + (int64_t)start * n, (uint32_t)((int64_t)(count) * n * 2));
+  // load j = wave + 4 q holds rows 2 j, 2 j + 1 of a (q < 4), rows 4 j .. 4 j + 3 of b (q < 2)
+  uint32_t a_at[2];
+#pragma unroll
+  for (int odd = 0; odd < 2; ++odd) a_at[odd] = dma::load_lane_offset<true, 64, 256>(wave, tm * TM::BM, a_ld, odd != 0) + (uint32_t)(2 * wave + 8 * odd) * a_ld;
+  uint32_t b_at = dma::load_lane_offset<true, 64, 128>(wave, tn * TM::BN, b_ld) + (uint32_t)(4 * wave) * b_ld;
+  auto load = [&](uint32_t stage) {   // the next K tile
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (__attribute__((address_space(3))) void*)(lds + (stage + (uint32_t)(wave + 4 * q) * 1024u)), 16,
+                                               (int)(a_at[q & 1] + (uint32_t)(q / 2) * 16u * a_ld), 0, 0, 0);
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (__attribute__((address_space(3))) void*)(lds + (stage + kMidA + (uint32_t)(wave + 4 * q) * 1024u)), 16,
+                                               (int)(b_at + (uint32_t)q * 16u * b_ld), 0, 0, 0);
+    a_at[0] += kMidK * a_ld;
+    a_at[1] += kMidK * a_ld;
+    b_at += kMidK * b_ld;
+  };
+  const int wm = (wave / TM::WN) * TM::WTM, wn = (wave % TM::WN) * TM::WTN;
+  // XOR moves from one fragment of a wave to the next (its 128 / 64 columns start at a multiple of as many)
+  const uint32_t fa0 = lds_base + dma::frag_lane_offset<true, 64, 256>(wm), fb0 = lds_base + kMidA + dma::frag_lane_offset<true, 64, 128>(wn);
+  typename TM::Acc acc[TM::TM][TM::TN];
+#pragma unroll
+  for (int i = 0; i < TM::TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TM::TN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  uint32_t at = 0, to = 2 * kMidStage;
+  if (nk > 0) load(0);
+  if (nk > 1) load(kMidStage);
+  Prefetch<TM::BM, TM::BN, kMidPerCu * kXcdRun> prefetch(tiles, e, a, b, bins, k, n);
+  for (int kt = 0; kt < nk; ++kt) {
+    __builtin_amdgcn_sched_barrier(0);
+    if (kt + 1 < nk) dma::wait_vmcnt<6>(); else dma::wait_vmcnt<0>();   // K tile kt is there, kt + 1 under way
+    __builtin_amdgcn_s_barrier();    // ... for every wave, and nobody reads the stage of K tile kt - 1 any more
+    __builtin_amdgcn_sched_barrier(0);
+    u32x2 pa[TM::TM][2], pb[TM::TN][2];
+#pragma unroll
+    for (int j = 0; j < TM::TN; ++j) {
+      pb[j][0] = dma::lds_read_tr16_b64<0>((fb0 + at) ^ (32u * j));
+      pb[j][1] = dma::lds_read_tr16_b64<4 * 128 * 2>((fb0 + at) ^ (32u * j));
+    }
+#pragma unroll
+    for (int i = 0; i < TM::TM; ++i) {
+      pa[i][0] = dma::lds_read_tr16_b64<0>((fa0 + at) ^ (32u * i));
+      pa[i][1] = dma::lds_read_tr16_b64<4 * 256 * 2>((fa0 + at) ^ (32u * i));
+    }
+    if (kt + 2 < nk) load(to);
+    if (kt + 1 == nk) prefetch.issue();
+    u32x4 fb[TM::TN];
+    dma::static_for<TM::TM>([&](auto ii) {
+      constexpr int i = decltype(ii)::value, left = 2 * (TM::TM - 1 - i);
+      wait_lgkm<left>();
+      asm volatile("" : "+v"(pa[i][0]), "+v"(pa[i][1]));
+      if constexpr (i == 0) {
+#pragma unroll
+        for (int j = 0; j < TM::TN; ++j) {
+          asm volatile("" : "+v"(pb[j][0]), "+v"(pb[j][1]));
+          fb[j] = u32x4{pb[j][0][0], pb[j][0][1], pb[j][1][0], pb[j][1][1]};
+        }
+      }
+      const u32x4 fa = {pa[i][0][0], pa[i][0][1], pa[i][1][0], pa[i][1][1]};
+#pragma unroll
+      for (int j = 0; j < TM::TN; ++j) acc[i][j] = mfma<DT>(fb[j], fa, acc[i][j]);
+      __builtin_amdgcn_sched_barrier(0);
+    });
+    at = at == (kMidStages - 1) * kMidStage ? 0 : at + kMidStage;
+    to = to == (kMidStages - 1) * kMidStage ? 0 : to + kMidStage;
+  }
+  if constexpr (OUT32) dma::block_store_f32<TM>(acc, (float*)c + (int64_t)e * k * n, n, tm * TM::BM, k, tn * TM::BN, n);
+  else dma::block_store<DT, TM>(acc, c + (int64_t)e * k * n, n, tm * TM::BM, k, tn * TM::BN, n, lds_generic);
+  prefetch.arrived();
+}
+
+template <int DT, bool OUT32>
+int launch_mid(const DmaCall& q) {
+  const int tiles_m = (int)ceil_div(q.k, TM::BM), tiles_n = (int)ceil_div(q.n, TM::BN);
+  const int64_t grid = ceil_div((int64_t)tiles_m * tiles_n, kXcds) * q.num_groups * kXcds;
+  if (grid > 0x7fffffff) return MBX_ERANGE;
+  auto kern = gmm_tn_mid_kernel<DT, OUT32>;
+  const int rc = allow_lds(kern, kMidLds);
+  if (rc) return rc;
+  kern<<<(unsigned)grid, TM::THREADS, kMidLds, q.stream>>>((const uint16_t*)q.a, (const uint16_t*)q.b, (uint16_t*)q.c, q.bins, q.num_groups, (int)q.rows, q.k, q.n, tiles_m, tiles_n);
+  return launch_status();
 }
 
 template <int DT, bool OUT32>
@@ -209,11 +386,23 @@ int launch(const DmaCall& q) {
   if (q.gather.slots) {
     if (!q.gather.src_bins || !q.gather.row_table || q.gather.top_k <= 0 || q.gather.n_slots > 0x7fffffff) return MBX_EINVAL;
     if (!q.gather.table_ready) dma::build_row_table(q);
-    gmm_tn_short_kernel<DT, true, OUT32><<<(unsigned)grid, T::THREADS, kLdsBytes, q.stream>>>(a, b, (uint16_t*)q.c, q.bins, q.num_groups, (int)q.rows, q.k, q.n, tiles_m, tiles_n, q.gather.row_table, q.gather.src_bins, q.gather.src_rows, (int)q.gather.n_slots);
+    gmm_tn_short_kernel<DT, true, OUT32, false><<<(unsigned)grid, T::THREADS, kLdsBytes, q.stream>>>(a, b, (uint16_t*)q.c, q.bins, q.num_groups, (int)q.rows, q.k, q.n, tiles_m, tiles_n, q.gather.row_table, q.gather.src_bins, q.gather.src_rows, (int)q.gather.n_slots);
   } else {
-    gmm_tn_short_kernel<DT, false, OUT32><<<(unsigned)grid, T::THREADS, kLdsBytes, q.stream>>>(a, b, (uint16_t*)q.c, q.bins, q.num_groups, (int)q.rows, q.k, q.n, tiles_m, tiles_n, nullptr, nullptr, 0, 0);
+    gmm_tn_short_kernel<DT, false, OUT32, true><<<(unsigned)grid, T::THREADS, kLdsBytes, q.stream>>>(a, b, (uint16_t*)q.c, q.bins, q.num_groups, (int)q.rows, q.k, q.n, tiles_m, tiles_n, nullptr, nullptr, 0, 0);
   }
   return launch_status();
+}
+
+
+// 256 x 128 tiles out of three small stages where there are five rounds of them, up to 512 rows per expert on average, and of few rows
+// where no half of a row of them is empty: they read a quarter less than 128 x 128 tiles and need a third fewer workgroups, but
+// their last round is longer (us, this / 128 x 128, gmm_dma.h's above 256 rows; operands and products not in the last-level cache:
+// 64 experts, [1024, 4096]: 64 rows 134 / 135, 128: 155 / 170, 256: 203 / 216, 512: 318 / 330;  8, [4096, 14336]: 250: 333 / 345, 500: 522 / 515,
+// 600: 603 / 574;  64, [2048, 1408]: 100: 106 / 99, 200: 134 / 133, 300: 172 / 176;  16 of 300, [2048, 1408], three rounds: 53 / 46).
+static bool takes_mid(const DmaCall& q) {
+  const int64_t average = q.rows / q.num_groups, tiles = ceil_div(q.k, TM::BM) * ceil_div(q.n, TM::BN) * q.num_groups;
+  if (q.gather.slots || average <= 64 || average > 512 || tiles < 5 * kMidPerCu * (int64_t)persistent_grid((int64_t)1 << 30)) return false;
+  return average > 256 || q.k % TM::BM == 0 || q.k % TM::BM > TM::BM / 2;
 }
 
 }  // namespace tn_short
@@ -227,11 +416,16 @@ bool gmm_tn_short_takes(const DmaCall& q) {
   const int64_t widest = q.k > q.n ? q.k : q.n;
   if (q.layout != MBX_TN || q.rows * widest * 2 >= ((int64_t)1 << 31)) return false;   // one buffer per operand
   const int64_t tiles = ceil_div(q.k, 128) * ceil_div(q.n, 128) * q.num_groups, at_once = tn_short::kPerCu * (int64_t)persistent_grid((int64_t)1 << 30);
-  return q.rows <= (int64_t)(tiles <= at_once ? 1024 : 256) * q.num_groups;
+  return q.rows <= (int64_t)(tiles <= at_once ? 1024 : 256) * q.num_groups || tn_short::takes_mid(q);
 }
 
 int gmm_tn_short(const DmaCall& q) {
-  if (q.out32) return q.dtype == MBX_BF16 ? tn_short::launch<MBX_BF16, true>(q) : tn_short::launch<MBX_F16, true>(q);
+  const bool mid = tn_short::takes_mid(q);
+  if (q.out32) {
+    if (mid) return q.dtype == MBX_BF16 ? tn_short::launch_mid<MBX_BF16, true>(q) : tn_short::launch_mid<MBX_F16, true>(q);
+    return q.dtype == MBX_BF16 ? tn_short::launch<MBX_BF16, true>(q) : tn_short::launch<MBX_F16, true>(q);
+  }
+  if (mid) return q.dtype == MBX_BF16 ? tn_short::launch_mid<MBX_BF16, false>(q) : tn_short::launch_mid<MBX_F16, false>(q);
   return q.dtype == MBX_BF16 ? tn_short::launch<MBX_BF16, false>(q) : tn_short::launch<MBX_F16, false>(q);
 }
 

@@ -1456,6 +1456,34 @@ def test_gmm_tn_with_few_rows_per_expert(gg, groups, rows, k, n, skew, dtype):
         assert torch.equal(gg.gmm_tn_gather(a, src, sizes.cuda()), gg.backend.gmm(a, x[order.long()], sizes, trans_a=True))
 
 
+@pytest.mark.parametrize('groups,rows,k,n', [(70, 70 * 80, 504, 2568), (64, 64 * 300, 520, 1672), (9, 9 * 270, 4600, 2056), (12, 12 * 100, 768, 1032)])
+@pytest.mark.parametrize('spread', ['alike', 'skewed'])
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])
+def test_gmm_tn_of_many_tiles(gg, groups, rows, k, n, spread, dtype):
+    """Weight gradients of up to a few hundred rows per expert in launches of many tiles, block by block against fp32, and bit for bit
+    those on gathered rows, which the general kernels form; an expert without rows."""
+    torch.manual_seed(rows + k)
+    if spread == 'alike':
+        sizes = rows // groups + torch.randint(-20, 21, (groups,))
+        sizes[1] += sizes[2]
+        sizes[2] = 0
+    else:
+        sizes = _sizes(groups, rows, seed=k, empty=(0, groups - 2))
+    rows = int(sizes.sum())
+    a, b = torch.randn(rows, k, device='cuda').to(dtype), torch.randn(rows, n, device='cuda').to(dtype)
+    got = gg.backend.gmm(a, b, sizes, trans_a=True)
+    wide = gg.weight_gradient(a, b, sizes.cuda(), torch.float32)
+    assert torch.equal(wide.to(dtype), got) and not got[(sizes == 0).cuda()].any()
+    ends = torch.cumsum(sizes, 0)
+    for e in range(groups):
+        s = slice(int(ends[e] - sizes[e]), int(ends[e]))
+        if sizes[e]:
+            assert max_block_err(got[e], a[s].float().t() @ b[s].float()) < TOL
+    bin_ids = torch.repeat_interleave(torch.arange(groups), sizes).int().cuda()
+    src = gg.GatheredRows(b, torch.arange(rows, device='cuda').int(), bin_ids, ends.cuda().int(), None, 1, rows)
+    assert torch.equal(gg.gmm_tn_gather(a, src, sizes.cuda()), got)
+
+
 @pytest.mark.parametrize('groups,rows,k,n', [(1, 1, 8, 8), (3, 130, 64, 136), (5, 5 * 300, 264, 1032), (70, 900, 136, 256), (4, 4 * 1500, 392, 264),
                                              (8, 8 * 2100, 1024, 640), (2, 0, 64, 64)])
 @pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])
