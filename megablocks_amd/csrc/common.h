@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "../../include/mbx.h"
 
 namespace mbx {
@@ -63,20 +65,67 @@ __device__ __forceinline__ float load_as_f32(const void* p, int64_t i, int dtype
 // ---- wave64 primitives ----
 __device__ __forceinline__ int lane_id() { return __lane_id(); }
 
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-  return v;
+// Between lanes without the LDS: a shuffle (ds_bpermute_b32) keeps a wave waiting some 100 cycles, a permute or DPP
+// operand two or three instructions, and a reduction is six of them in a chain.
+//
+// wave_butterfly(v, op): all lanes get v combined over the wave, op(v, v of the lane 32, 16, 8, 4, 2, 1 further) in turn, for a
+// commutative op.  The steps by 32 and 16 swap half waves and rows of 16; by 8 the row is rotated by 8, by 4 by 4 (its
+// halves are alike by then), by 2 and 1 quads are permuted.  All lanes must be active.
+template <int STEP>
+__device__ __forceinline__ uint32_t lane_xor_dpp(uint32_t v) {   // STEP 8 (4: lanes 8 apart are alike), 2, 1
+  constexpr int ctrl = STEP == 8 ? 0x128 : STEP == 4 ? 0x124 : STEP == 2 ? 0x4e : 0xb1;
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, ctrl, 0xf, 0xf, true);
 }
+template <typename T, typename F>
+__device__ __forceinline__ T wave_butterfly(T v, F&& op) {
+  static_assert(sizeof(T) == 4, "one register");
+  const auto bits = [](T x) { return __builtin_bit_cast(uint32_t, x); };
+  const auto value = [](uint32_t x) { return __builtin_bit_cast(T, x); };
+  const auto halves = __builtin_amdgcn_permlane32_swap(bits(v), bits(v), false, false);
+  v = op(value(halves[0]), value(halves[1]));
+  const auto rows = __builtin_amdgcn_permlane16_swap(bits(v), bits(v), false, false);
+  v = op(value(rows[0]), value(rows[1]));
+  v = op(v, value(lane_xor_dpp<8>(bits(v))));
+  v = op(v, value(lane_xor_dpp<4>(bits(v))));
+  v = op(v, value(lane_xor_dpp<2>(bits(v))));
+  return op(v, value(lane_xor_dpp<1>(bits(v))));
+}
+
+__device__ __forceinline__ float wave_sum(float v) {
+  return wave_butterfly(v, [](float a, float b) { return a + b; });
+}
+__device__ __forceinline__ float wave_max(float v) {
+  return wave_butterfly(v, [](float a, float b) { return fmaxf(a, b); });
+}
+__device__ __forceinline__ int wave_max(int v) {
+  return wave_butterfly(v, [](int a, int b) { return a > b ? a : b; });
+}
+
+// Lane `from`'s value, the same `from` in all lanes.
+__device__ __forceinline__ int lane_value(int v, int from) { return __builtin_amdgcn_readlane(v, from); }
+__device__ __forceinline__ float lane_value(float v, int from) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), from)); }
 
 // Inclusive prefix sum across the 64 lanes of a wave.
 template <typename T>
 __device__ __forceinline__ T wave_inclusive_scan(T v) {
-  const int lane = lane_id();
+  if constexpr (sizeof(T) == 4) {
+    const auto moved = [](T x, auto ctrl, auto rows) {   // zero where no lane is that far below, in the rows not named
+      return (T)__builtin_amdgcn_update_dpp(0, (int)x, decltype(ctrl)::value, decltype(rows)::value, 0xf, false);
+    };
+    typedef std::integral_constant<int, 0xf> all;
+    v += moved(v, std::integral_constant<int, 0x111>{}, all{});   // row_shr by 1, 2, 4, 8: inside the rows of 16
+    v += moved(v, std::integral_constant<int, 0x112>{}, all{});
+    v += moved(v, std::integral_constant<int, 0x114>{}, all{});
+    v += moved(v, std::integral_constant<int, 0x118>{}, all{});
+    v += moved(v, std::integral_constant<int, 0x142>{}, std::integral_constant<int, 0xa>{});   // row_bcast:15 to rows 1 and 3
+    v += moved(v, std::integral_constant<int, 0x143>{}, std::integral_constant<int, 0xc>{});   // row_bcast:31 to rows 2 and 3
+  } else {
+    const int lane = lane_id();
 #pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    T o = __shfl_up(v, off, 64);
-    if (lane >= off) v += o;
+    for (int off = 1; off < 64; off <<= 1) {
+      T o = __shfl_up(v, off, 64);
+      if (lane >= off) v += o;
+    }
   }
   return v;
 }

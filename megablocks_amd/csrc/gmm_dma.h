@@ -1216,12 +1216,7 @@ struct RowTiles {
       }
       lane_mt = span;
     }
-    int incl = span, sincl = shorts;
-#pragma unroll
-    for (int o = 1; o < kWave; o <<= 1) {
-      const int v = __shfl_up(incl, o, kWave), w = __shfl_up(sincl, o, kWave);
-      if (lane >= o) { incl += v; sincl += w; }
-    }
+    const int incl = wave_inclusive_scan(span), sincl = wave_inclusive_scan(shorts);
     lane_incl = incl;
     lane_short_incl = sincl;
     total_short = __builtin_amdgcn_readlane(sincl, kWave - 1) * tiles_n;
@@ -1811,17 +1806,12 @@ gmm_tn_kernel(const uint16_t* __restrict__ a, const uint16_t* __restrict__ b, ui
     rank = rank_by_rows(mine, num_groups);
     if (whole_ok && num_groups >= kXcds) {
       const int home = rank < 0 ? -1 : serpentine_xcd(rank);
-      int worst = 0, total = 0, load[kXcds];   // the sums of all XCDs step by step, so that their shuffles overlap
-#pragma unroll
-      for (int x = 0; x < kXcds; ++x) load[x] = home == x ? (mine > 0 ? mine : 0) : 0;
-#pragma unroll
-      for (int o = kWave / 2; o > 0; o >>= 1)
-#pragma unroll
-        for (int x = 0; x < kXcds; ++x) load[x] += __shfl_xor(load[x], o, kWave);
+      int worst = 0, total = 0;
 #pragma unroll
       for (int x = 0; x < kXcds; ++x) {
-        worst = load[x] > worst ? load[x] : worst;
-        total += load[x];
+        const int load = wave_butterfly(home == x && mine > 0 ? mine : 0, [](int a, int b) { return a + b; });
+        worst = load > worst ? load : worst;
+        total += load;
       }
       whole = (int64_t)worst * kXcds * 200 <= (int64_t)total * 203;
     }

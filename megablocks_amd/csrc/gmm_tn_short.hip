@@ -60,11 +60,7 @@ struct Tiles {
       mine = e < num_groups ? clamp_row(bins[e], rows) - (e > 0 ? clamp_row(bins[e - 1], rows) : 0) : -1;
       most = mine > most ? mine : most;
     }
-#pragma unroll
-    for (int o = kWave / 2; o > 0; o >>= 1) {
-      const int other = __shfl_xor(most, o, kWave);
-      most = other > most ? other : most;
-    }
+    most = wave_max(most);
     alike = (int64_t)__builtin_amdgcn_readfirstlane(most) * num_groups <= 2 * (int64_t)rows;
     // bands of column tiles whose panel of b takes an L2 1.5 MiB; of few panels in a part of an expert
     const int average = (int)((int64_t)rows / num_groups) + 1, fits = 6144 / average;

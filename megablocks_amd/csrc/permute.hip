@@ -265,9 +265,9 @@ gather_tokens_kernel(const void* __restrict__ x_, int64_t tokens, int hidden, in
         if (c < nvec) v[i] = src[c];
       }
       for (int j = 0; j < top_k; ++j) {
-        const int row = __shfl(my_row, j, kWave);
+        const int row = lane_value(my_row, j);
         if (row < 0) continue;
-        const float scale = __shfl(my_scale, j, kWave);
+        const float scale = lane_value(my_scale, j);
         u32x4* dst = (u32x4*)(out + (int64_t)row * hidden);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -347,10 +347,10 @@ combine_kernel(const void* __restrict__ x_, int64_t tokens, int hidden, int part
       bool live[BATCH];
 #pragma unroll
       for (int j = 0; j < BATCH; ++j) {
-        const int row = __shfl(my_row, j, kWave);
+        const int row = lane_value(my_row, j);
         live[j] = row >= 0;
         src[j] = (const u32x4*)(x + (int64_t)(live[j] ? row : 0) * hidden);
-        scale[j] = __shfl(my_scale, j, kWave);
+        scale[j] = lane_value(my_scale, j);
       }
       // eight 16-byte loads per lane in flight whatever top_k is: with two experts per token four columns of the
       // row are worked on together (two loads at a time leave a wave waiting on memory latency most of the time)
@@ -478,8 +478,8 @@ scatter_backward_kernel(const void* __restrict__ grad_, const void* __restrict__
     float scale[BATCH], acc[BATCH];
 #pragma unroll
     for (int j = 0; j < BATCH; ++j) {
-      row[j] = __shfl(my_row, j, kWave);
-      scale[j] = __shfl(my_scale, j, kWave);
+      row[j] = lane_value(my_row, j);
+      scale[j] = lane_value(my_scale, j);
       acc[j] = 0.f;
     }
     for (int c0 = 0; c0 < nvec; c0 += 4 * kWave) {

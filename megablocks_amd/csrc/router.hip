@@ -9,12 +9,6 @@ namespace {
 constexpr int kTokenThreads = 256;
 constexpr int kTokenWaves = kTokenThreads / kWave;
 
-__device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, 64));
-  return v;
-}
-
 // ||w||_p of the first top_k lanes' values (p > 0)
 __device__ __forceinline__ float wave_pnorm(float w, bool live, float p) {
   const float a = fabsf(w);
@@ -67,12 +61,10 @@ __device__ __forceinline__ void route_token(float (&x)[R], int64_t t, int num_ex
 #pragma unroll
     for (int r = 0; r < R; ++r)   // ascending expert index: a later equal value does not replace an earlier one
       if (x[r] > best) { best = x[r]; best_e = lane + r * kWave; }
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-      const float ov = __shfl_xor(best, off, 64);
-      const int oe = __shfl_xor(best_e, off, 64);
-      if (ov > best || (ov == best && oe < best_e)) { best = ov; best_e = oe; }
-    }
+    // the largest score, then the lowest expert that has it
+    const float top = wave_butterfly(best, [](float a, float b) { return a > b ? a : b; });
+    best_e = wave_butterfly(best == top ? best_e : 0x7fffffff, [](int a, int b) { return a < b ? a : b; });
+    best = top;
     if (lane == j) { my_w = best == INFINITY ? NAN : best; my_i = best_e; }
 #pragma unroll
     for (int r = 0; r < R; ++r)
@@ -226,8 +218,8 @@ router_backward_kernel(const void* __restrict__ grad_weights_, const void* __res
         dw = dy / n - dot / (n * n) * dn;
       }
       for (int j = 0; j < top_k; ++j) {
-        const int e = __shfl(my_i, j, 64);
-        const float v = __shfl(dw, j, 64);
+        const int e = lane_value(my_i, j);
+        const float v = lane_value(dw, j);
 #pragma unroll
         for (int r = 0; r < R; ++r)
           if (lane + r * kWave == e) ds[r] += v;
