@@ -564,6 +564,7 @@ static int gmm_dma(const DmaCall& call) {
 #endif
   if (kFewRows && gmm_few_takes(call)) return gmm_few(call);
   if (kFewRows && gmm_mid_takes(call)) return gmm_mid(call);
+  if (kFewRows && gmm_pair_takes(call)) return gmm_pair(call);
   if (call.layout != MBX_TN) return call.k % dma::TileMain::BK == 0 ? gmm_rows(call) : gmm_rows_tail(call);
   if (kFewRows && gmm_tn_short_takes(call)) return gmm_tn_short(call);
   if (call.gather.slots) {   // gathered rows: the full tile only

@@ -66,6 +66,14 @@ int gmm_few(const DmaCall& call);
 bool gmm_mid_takes(const DmaCall& call);
 int gmm_mid(const DmaCall& call);
 
+// NN launches with no full round of tiles are cut along the reduction from this many K tiles on: exchanging the parts takes some 20
+// us.  8 experts of 48 rows, [4096, 1024]: 61 -> 36 us; 4 of 500, [2816, 1024]: 58 -> 45; 8 of 256, [1408, 512]: 18 -> 21.
+constexpr int kMinCutTiles = 32;
+
+// NN / NT launches of few tiles (gmm_pair.hip), and whether a launch is one of them.
+bool gmm_pair_takes(const DmaCall& call);
+int gmm_pair(const DmaCall& call);
+
 // TN launches with few rows per expert (gmm_tn_short.hip), and whether a launch is one of them.
 bool gmm_tn_short_takes(const DmaCall& call);
 int gmm_tn_short(const DmaCall& call);

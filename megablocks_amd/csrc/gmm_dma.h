@@ -912,12 +912,11 @@ __device__ __forceinline__ void block_store(const typename T::Acc (&acc)[T::TM][
     __syncthreads();
     if constexpr (epi_is_glu(EPI)) {
       // The tile is [x1 | x2]: BN / 2 output columns from n_base on.  A lane takes the same 16-byte chunk of both
-      // halves of a row: 16 lanes a row, four rows per instruction; it stores the two chunks (to c and out2) and
-      // their gated activation (to extra).  Batches of four rows per lane: eight LDS reads in flight, twelve stores.
-      static_assert(T::BN == 256, "sixteen chunks per half row");
-      constexpr int RPI = 4, ITERS = T::BM / RPI / T::WAVES, BATCH = 4, ROW_STEP = T::WAVES * RPI;
+      // halves of a row: 16 (8) lanes a row, four (eight) rows per instruction; it stores the two chunks (to c and out2)
+      // and their gated activation (to extra).  Batches of four rows per lane: eight LDS reads in flight, twelve stores.
+      constexpr int LANES = T::BN / 16, RPI = kWave / LANES, ITERS = T::BM / RPI / T::WAVES, BATCH = 4, ROW_STEP = T::WAVES * RPI;
       static_assert(ITERS % BATCH == 0, "store batches");
-      const int rl = lane >> 4, ch = lane & 15;
+      const int rl = lane / LANES, ch = lane % LANES;
       const int n = n_base + ch * 8;
       const uint32_t rd_addr = lds_base + (uint32_t)((wave * RPI + rl) * ROW + ch * 16);
       int m = m_base + wave * RPI + rl;

@@ -45,7 +45,9 @@ int launch_rows(const DmaCall& call) {
   const int tiles_n = (int)ceil_div(n, dma::epi_is_glu(epi) ? T::BN / 2 : T::BN);
   const int64_t tiles = (ceil_div(rows, T::BM) + num_groups) * tiles_n;   // the row counts are only known on the device
   if (tiles > 0x7fffffff) return MBX_ERANGE;
-  const unsigned grid = (unsigned)persistent_grid(tiles);
+  // launches that may cut their tiles along the reduction want the compute units that have no tile for the parts
+  const bool may_cut = layout == MBX_NN && epi == dma::kEpiNone && ws.base != nullptr && (dual ? 2 : 1) * ceil_div(k, T::BK) >= kMinCutTiles;
+  const unsigned grid = (unsigned)persistent_grid(may_cut ? (int64_t)1 << 30 : tiles);
   // An expert's last row tile, when at most half full, is computed with the half-height tile -- unless a row of tiles is
   // longer than the run of tiles an XCD's workgroups take per round: the half-height tiles of such a row fill whole
   // rounds of some XCDs, those finish early, and from then on the XCD's workgroups are no longer within the few K tiles
