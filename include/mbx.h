@@ -403,6 +403,11 @@ int mbx_router_backward(const void* grad_weights, const void* grad_scores, const
                         int dtype, int64_t tokens, int num_experts, int top_k, float norm_p, void* grad_logits,
                         const float* grad_lse, mbx_stream_t stream);
 
+/* out[i] = parts[0][i] + ... + parts[num_parts - 1][i] for i < n, in fp32, rounded once to `dtype`; part p starts at parts + p pitch.
+ * The weight gradient of the router's linear layer from those of equal pieces of the batch (mbx_gmm_tn_f32, one group a
+ * piece). */
+int mbx_sum_parts(const float* parts, int num_parts, int64_t pitch, void* out, int dtype, int64_t n, mbx_stream_t stream);
+
 #ifdef __cplusplus
 }
 #endif

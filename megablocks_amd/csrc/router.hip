@@ -238,6 +238,47 @@ router_backward_kernel(const void* __restrict__ grad_weights_, const void* __res
   }
 }
 
+// out[i] = sum over the parts, in fp32, rounded once.  A block takes 64 runs of four values; each of its four waves adds up a
+// quarter of the parts, eight loads under way, and the first puts the quarters together, in order.  What bounds it: one reading of the
+// parts (64 of 64 x 1024, 16.8 MB: 5 us; torch's sum of as many 16-bit values 9.9, and the cast of its result 4.8).
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+template <int DT>
+__global__ void __launch_bounds__(kTokenThreads)
+sum_parts_kernel(const float* __restrict__ parts, int num_parts, int64_t pitch, void* __restrict__ out_, int64_t n) {
+  typedef typename Elem<DT>::type E;
+  __shared__ f32x4_t sums[kTokenWaves][kWave];
+  constexpr int kAhead = 8;
+  const int lane = lane_id(), wave = threadIdx.x / kWave;
+  const int64_t i = ((int64_t)blockIdx.x * kWave + lane) * 4;
+  const int first = (int)((int64_t)wave * num_parts / kTokenWaves), last = (int)((int64_t)(wave + 1) * num_parts / kTokenWaves);
+  f32x4_t sum = {0.f, 0.f, 0.f, 0.f};
+  if (i + 4 <= n && (pitch & 3) == 0) {
+    const f32x4_t* p = (const f32x4_t*)(parts + i);
+    for (int q = first; q < last; q += kAhead) {
+      f32x4_t v[kAhead];
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u)
+        if (q + u < last) v[u] = p[(int64_t)(q + u) * (pitch / 4)];
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u)
+        if (q + u < last) sum += v[u];
+    }
+  } else {
+    for (int q = first; q < last; ++q)
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+        if (i + t < n) sum[t] += parts[(int64_t)q * pitch + i + t];
+  }
+  sums[wave][lane] = sum;
+  __syncthreads();
+  if (wave != 0) return;
+#pragma unroll
+  for (int w = 1; w < kTokenWaves; ++w) sum += sums[w][lane];
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+    if (i + t < n) ((E*)out_)[i + t] = Elem<DT>::from_f32(sum[t]);
+}
+
 static inline unsigned token_grid(int64_t tokens) {
   int64_t blocks = ceil_div(tokens, kTokenWaves);
   if (blocks > 256 * 8) blocks = 256 * 8;
@@ -329,6 +370,20 @@ int mbx_router_backward(const void* grad_weights, const void* grad_scores, const
   hipStream_t s = as_stream(stream);
   MBX_ROUTER_DISPATCH(router_backward_kernel, grad_weights, grad_scores, scores, indices, tokens, num_experts, top_k,
                       norm_p, grad_logits, grad_lse);
+  return launch_status();
+}
+
+int mbx_sum_parts(const float* parts, int num_parts, int64_t pitch, void* out, int dtype, int64_t n, mbx_stream_t stream) {
+  if (num_parts <= 0 || n < 0 || pitch < n) return MBX_EINVAL;
+  if (dtype != MBX_BF16 && dtype != MBX_F16 && dtype != MBX_F32) return MBX_EINVAL;
+  if (n == 0) return 0;
+  if (!parts || !out || ((uintptr_t)parts & 15u)) return MBX_EINVAL;
+  const int64_t blocks = ceil_div(n, 4 * kWave);
+  if (blocks > 0x7fffffff) return MBX_ERANGE;
+  hipStream_t s = as_stream(stream);
+  if (dtype == MBX_BF16) sum_parts_kernel<MBX_BF16><<<(unsigned)blocks, kTokenThreads, 0, s>>>(parts, num_parts, pitch, out, n);
+  else if (dtype == MBX_F16) sum_parts_kernel<MBX_F16><<<(unsigned)blocks, kTokenThreads, 0, s>>>(parts, num_parts, pitch, out, n);
+  else sum_parts_kernel<MBX_F32><<<(unsigned)blocks, kTokenThreads, 0, s>>>(parts, num_parts, pitch, out, n);
   return launch_status();
 }
 

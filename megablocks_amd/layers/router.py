@@ -53,10 +53,11 @@ class _UniformExpertAssignment(torch.autograd.Function):
 
 
 class _RouterLinear(torch.autograd.Function):
-    """`x @ weight^T` of the router's `torch.nn.Linear` (router.py:96), with the weight gradient
-    `[E, T] @ [T, h]` (a short, wide output over a reduction as long as the batch: a handful of tiles for the
-    vendor GEMM) computed by the grouped TN kernel instead: the token range is cut into equal pieces, each
-    piece is one group, and the partial products are summed in fp32."""
+    """`x @ weight^T` of the router's `torch.nn.Linear` (router.py:96) with the gradients from the grouped kernels: the
+    weight's, `[E, T] @ [T, h]` (a short, wide output over a reduction as long as the batch: a handful of tiles for the
+    vendor GEMM), by the TN kernel over equal pieces of the token range, one group each, whose fp32 sums one kernel adds up
+    and rounds; the input's, a reduction of E, by the NN kernel.  (A call of the vendor library is some 50 us of host time,
+    one of these 15 - 20.  GPU, 16384 tokens of 1024, 64 experts: weight 14 + 10 + 5 -> 14 + 5 us, input 18 -> 13.)"""
 
     PIECE_ROWS = 256   # tokens per piece (four K tiles of the TN kernel)
     MAX_PIECES = 64
@@ -64,14 +65,14 @@ class _RouterLinear(torch.autograd.Function):
     _sizes = {}
 
     @staticmethod
-    def piece_sizes(tokens: int) -> torch.Tensor:
+    def piece_sizes(tokens: int, max_pieces: int = MAX_PIECES) -> torch.Tensor:
         """Rows per piece (kept per batch size: the grouped GEMM caches the device-side bins on this tensor)."""
-        sizes = _RouterLinear._sizes.get(tokens)
+        sizes = _RouterLinear._sizes.get((tokens, max_pieces))
         if sizes is None:
-            pieces = max(1, min(_RouterLinear.MAX_PIECES, tokens // _RouterLinear.PIECE_ROWS))
+            pieces = max(1, min(max_pieces, tokens // _RouterLinear.PIECE_ROWS))
             sizes = torch.full((pieces,), tokens // pieces, dtype=torch.int64)
             sizes[:tokens % pieces] += 1
-            _RouterLinear._sizes[tokens] = sizes
+            _RouterLinear._sizes[tokens, max_pieces] = sizes
         return sizes
 
     @staticmethod
@@ -90,19 +91,34 @@ class _RouterLinear(torch.autograd.Function):
     @torch.amp.custom_bwd(device_type='cuda')
     def backward(ctx: Any, grad: torch.Tensor):
         x, weight = ctx.saved_tensors
-        grad = grad.to(x.dtype)
-        dx = grad @ weight if ctx.needs_input_grad[0] else None
-        dw = None
-        if ctx.needs_input_grad[1]:
-            from megablocks_amd import grouped_gemm_util as gg
-            sizes = _RouterLinear.piece_sizes(x.shape[0])
-            pieces = sizes.shape[0]
-            experts = grad.shape[1]
-            if experts % 8:   # the pipelined kernels read whole 16-byte pieces of rows
-                grad = torch.nn.functional.pad(grad, (0, -experts % 8))
-            parts = gg.gmm(grad.contiguous(), x.contiguous(), sizes, trans_a=True, _record_as='router_wgrad')   # [pieces, E, h]
-            dw = (parts[0] if pieces == 1 else parts.sum(0, dtype=torch.float32))[:experts].to(ctx.weight_dtype)
-        return dx, dw
+        return _linear_gradients(grad.to(x.dtype), x, weight, ctx.weight_dtype, *ctx.needs_input_grad[:2])
+
+
+def _linear_gradients(grad, x, weight, weight_dtype, want_x, want_weight):
+    """(dx, dweight) of `x @ weight^T`, all 16-bit of one type on the GPU; dweight in `weight_dtype`."""
+    from megablocks_amd import grouped_gemm_util as gg
+    tokens, experts = grad.shape
+    grad = grad.contiguous()
+    dx = dw = None
+    if want_x:
+        # the kernels read whole 16-byte pieces of rows
+        dx = grad @ weight if experts % 8 or tokens == 0 else gg.gmm(
+            grad, weight.unsqueeze(0), _RouterLinear.piece_sizes(tokens, 1), _record_as='router_dgrad')
+    if want_weight:
+        sizes = _RouterLinear.piece_sizes(tokens)
+        pieces = sizes.shape[0]
+        if experts % 8:
+            grad = torch.nn.functional.pad(grad, (0, -experts % 8))
+        # [pieces, E, h]; a single piece's sums are rounded by the product itself
+        parts = gg.weight_gradient(grad, x.contiguous(), sizes, torch.float32 if pieces > 1 else None)
+        if pieces == 1 or parts.dtype != torch.float32:
+            dw = (parts[0] if pieces == 1 else parts.sum(0, dtype=torch.float32))[:experts].to(weight_dtype)
+        else:
+            dw = torch.empty((experts, x.shape[1]), dtype=weight_dtype, device=x.device)
+            with _lib.device_of(x):
+                _lib.check(_lib.lib.mbx_sum_parts(_lib.ptr(parts), pieces, parts.stride(0), _lib.ptr(dw), _lib.dtype_of(dw),
+                                                  dw.numel(), _lib.stream()), 'sum_parts')
+    return dx, dw
 
 
 class _SoftmaxTopK(torch.autograd.Function):
@@ -174,14 +190,14 @@ class _LinearSoftmaxTopK(torch.autograd.Function):
         """Few tokens and a small layer: one launch instead of two (64 experts of 2048, 5 tokens: 11.1 -> 9.1 us on the GPU, and
         the vendor library's call alone is 25 us of host time; 512 tokens: 11.5 against 14.5, 128 experts of 4096: 14.0
         against 16.1)."""
-        if type(layer) is not torch.nn.Linear or not x.is_cuda or x.shape[0] > _LinearSoftmaxTopK.MAX_TOKENS:
+        if not x.is_cuda or x.shape[0] > _LinearSoftmaxTopK.MAX_TOKENS or not _plain_linear(layer):
             return False
         weight = layer.weight
-        return (x.dtype in (torch.bfloat16, torch.float16) and type(weight) is torch.nn.Parameter and weight.dtype == x.dtype and
-                weight.device == x.device and layer.bias is None and x.shape[0] > 0 and x.shape[1] == weight.shape[1] and
+        return (x.dtype in (torch.bfloat16, torch.float16) and weight.dtype == x.dtype and
+                weight.device == x.device and x.shape[0] > 0 and x.shape[1] == weight.shape[1] and
                 x.shape[1] % 8 == 0 and weight.shape[0] <= 128 and weight.numel() <= _LinearSoftmaxTopK.MAX_WEIGHTS and 0 < top_k <= min(64, weight.shape[0]) and
                 x.is_contiguous() and weight.is_contiguous() and (x.data_ptr() | weight.data_ptr()) % 16 == 0 and
-                not torch.is_autocast_enabled() and not _has_hooks(layer))
+                not torch.is_autocast_enabled())
 
     @staticmethod
     def forward(ctx: Any, x: torch.Tensor, weight: torch.Tensor, top_k: int, norm_p: float):
@@ -219,9 +235,7 @@ class _RecordedLinearSoftmaxTopK(torch.autograd.Function):
     def backward(ctx: Any, grad_scores, grad_weights, _grad_indices, _grad_indices32):
         x, weight, scores, indices = ctx.saved_tensors
         grad = _logits_gradient(scores, indices, ctx.top_k, ctx.norm_p, grad_scores, grad_weights)
-        dx = grad @ weight if ctx.needs_input_grad[0] else None
-        dw = grad.t() @ x if ctx.needs_input_grad[1] else None
-        return dx, dw, None, None
+        return *_linear_gradients(grad, x, weight, weight.dtype, *ctx.needs_input_grad[:2]), None, None
 
 
 def _has_hooks(module: torch.nn.Module) -> bool:
@@ -230,6 +244,11 @@ def _has_hooks(module: torch.nn.Module) -> bool:
     return bool(module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks or
                 glob._global_forward_hooks or glob._global_forward_pre_hooks or glob._global_backward_hooks or
                 glob._global_backward_pre_hooks or 'forward' in module.__dict__)
+
+
+def _plain_linear(layer: torch.nn.Module) -> bool:
+    """Whether calling `layer` is a product with its weight and nothing else."""
+    return type(layer) is torch.nn.Linear and layer.bias is None and type(layer.weight) is torch.nn.Parameter and not _has_hooks(layer)
 
 
 def int32_indices(expert_indices: torch.Tensor) -> torch.Tensor:
@@ -279,7 +298,8 @@ class LearnedRouter(torch.nn.Module):
             for node in (_LinearSoftmaxTopK, _RecordedLinearSoftmaxTopK):   # without gradients, with
                 if node.supported(x2d, self.layer, args.moe_top_k):
                     return node.apply(x2d, self.layer.weight, args.moe_top_k, args.moe_normalize_expert_weights or 0)
-        if x2d.is_cuda and x2d.dtype in (torch.bfloat16, torch.float16) and x2d.shape[0] >= 4 * _RouterLinear.PIECE_ROWS:
+        if torch.is_grad_enabled() and x2d.is_cuda and x2d.dtype in (torch.bfloat16, torch.float16) and x2d.shape[0] > 0 and \
+                _plain_linear(self.layer):
             logits = _RouterLinear.apply(x2d, self.layer.weight)
         else:
             logits = self.layer(x2d)

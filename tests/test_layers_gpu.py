@@ -243,6 +243,27 @@ def test_router_linear_gradients(tokens, hidden, experts, dtype):
     assert int(sizes.sum()) == tokens and sizes.shape[0] == min(64, tokens // 256) and int(sizes.max() - sizes.min()) <= 1
 
 
+@pytest.mark.parametrize('tokens,hidden,experts', [(1, 8, 8), (255, 264, 12), (513, 1032, 64), (1024, 520, 8), (40000, 512, 128), (20000, 72, 5)])
+@pytest.mark.parametrize('dtype,weight_dtype', [(torch.bfloat16, torch.bfloat16), (torch.float16, torch.float16), (torch.bfloat16, torch.float32)])
+def test_router_linear_gradients_against_fp64(tokens, hidden, experts, dtype, weight_dtype):
+    """Both gradients of the router's linear layer against fp64: fp32 sums rounded once to 16 bits (half a step, 2^-9 or 2^-12, with a
+    factor of two to spare), and for fp32 weights not at all (2^-24 per term, random signs, a factor of four)."""
+    from megablocks_amd.layers.router import _RouterLinear
+    torch.manual_seed(tokens)
+    x = torch.randn(tokens, hidden, device='cuda').to(dtype).requires_grad_(True)
+    weight = torch.randn(experts, hidden, device='cuda').to(dtype).to(weight_dtype).requires_grad_(True)
+    g = torch.randn(tokens, experts, device='cuda').to(dtype)
+    with torch.autocast('cuda', dtype=dtype, enabled=weight_dtype != dtype):
+        _RouterLinear.apply(x, weight).backward(g)
+    assert x.grad.dtype == dtype and weight.grad.dtype == weight_dtype
+    rounding = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+    sums = 4 * 2.0 ** -24 * max(tokens, 16) ** 0.5
+    assert rel_err(x.grad.double(), g.double() @ weight.detach().double()) < rounding
+    # a batch of one piece, or of experts the kernels for fp32 sums do not take, may pass through 16 bits
+    exact = weight_dtype == torch.float32 and tokens >= 512
+    assert rel_err(weight.grad.double(), g.double().t() @ x.detach().double()) < (sums if exact else rounding)
+
+
 def _softmax_topk_reference(logits, top_k, norm_p):
     """router.py:87-106 with torch's own operations."""
     scores = logits.softmax(dim=-1)
