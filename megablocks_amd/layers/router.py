@@ -56,8 +56,9 @@ class _RouterLinear(torch.autograd.Function):
     """`x @ weight^T` of the router's `torch.nn.Linear` (router.py:96) with the gradients from the grouped kernels: the
     weight's, `[E, T] @ [T, h]` (a short, wide output over a reduction as long as the batch: a handful of tiles for the
     vendor GEMM), by the TN kernel over equal pieces of the token range, one group each, whose fp32 sums one kernel adds up
-    and rounds; the input's, a reduction of E, by the NN kernel.  (A call of the vendor library is some 50 us of host time,
-    one of these 15 - 20.  GPU, 16384 tokens of 1024, 64 experts: weight 14 + 10 + 5 -> 14 + 5 us, input 18 -> 13.)"""
+    and rounds; the input's, a reduction of E, by the NN kernel.  (GPU, 16384 tokens of 1024, 64 experts: weight 14 + 10 + 5 -> 14 + 5 us,
+    input 18 -> 14; the backward's host time with the router kernel's 102 -> 81 us.  At 600 tokens, where the vendor's
+    two products are as quick, a node of Python's in the forward is 5 us more than torch's own: from 1024 tokens.)"""
 
     PIECE_ROWS = 256   # tokens per piece (four K tiles of the TN kernel)
     MAX_PIECES = 64
@@ -190,14 +191,14 @@ class _LinearSoftmaxTopK(torch.autograd.Function):
         """Few tokens and a small layer: one launch instead of two (64 experts of 2048, 5 tokens: 11.1 -> 9.1 us on the GPU, and
         the vendor library's call alone is 25 us of host time; 512 tokens: 11.5 against 14.5, 128 experts of 4096: 14.0
         against 16.1)."""
-        if not x.is_cuda or x.shape[0] > _LinearSoftmaxTopK.MAX_TOKENS or not _plain_linear(layer):
+        if type(layer) is not torch.nn.Linear or not x.is_cuda or x.shape[0] > _LinearSoftmaxTopK.MAX_TOKENS:
             return False
         weight = layer.weight
-        return (x.dtype in (torch.bfloat16, torch.float16) and weight.dtype == x.dtype and
-                weight.device == x.device and x.shape[0] > 0 and x.shape[1] == weight.shape[1] and
+        return (x.dtype in (torch.bfloat16, torch.float16) and type(weight) is torch.nn.Parameter and weight.dtype == x.dtype and
+                weight.device == x.device and layer.bias is None and x.shape[0] > 0 and x.shape[1] == weight.shape[1] and
                 x.shape[1] % 8 == 0 and weight.shape[0] <= 128 and weight.numel() <= _LinearSoftmaxTopK.MAX_WEIGHTS and 0 < top_k <= min(64, weight.shape[0]) and
                 x.is_contiguous() and weight.is_contiguous() and (x.data_ptr() | weight.data_ptr()) % 16 == 0 and
-                not torch.is_autocast_enabled())
+                not torch.is_autocast_enabled() and not _has_hooks(layer))
 
     @staticmethod
     def forward(ctx: Any, x: torch.Tensor, weight: torch.Tensor, top_k: int, norm_p: float):
@@ -244,11 +245,6 @@ def _has_hooks(module: torch.nn.Module) -> bool:
     return bool(module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks or
                 glob._global_forward_hooks or glob._global_forward_pre_hooks or glob._global_backward_hooks or
                 glob._global_backward_pre_hooks or 'forward' in module.__dict__)
-
-
-def _plain_linear(layer: torch.nn.Module) -> bool:
-    """Whether calling `layer` is a product with its weight and nothing else."""
-    return type(layer) is torch.nn.Linear and layer.bias is None and type(layer.weight) is torch.nn.Parameter and not _has_hooks(layer)
 
 
 def int32_indices(expert_indices: torch.Tensor) -> torch.Tensor:
@@ -298,8 +294,7 @@ class LearnedRouter(torch.nn.Module):
             for node in (_LinearSoftmaxTopK, _RecordedLinearSoftmaxTopK):   # without gradients, with
                 if node.supported(x2d, self.layer, args.moe_top_k):
                     return node.apply(x2d, self.layer.weight, args.moe_top_k, args.moe_normalize_expert_weights or 0)
-        if torch.is_grad_enabled() and x2d.is_cuda and x2d.dtype in (torch.bfloat16, torch.float16) and x2d.shape[0] > 0 and \
-                _plain_linear(self.layer):
+        if x2d.is_cuda and x2d.dtype in (torch.bfloat16, torch.float16) and x2d.shape[0] >= 4 * _RouterLinear.PIECE_ROWS:
             logits = _RouterLinear.apply(x2d, self.layer.weight)
         else:
             logits = self.layer(x2d)

@@ -243,7 +243,7 @@ def test_router_linear_gradients(tokens, hidden, experts, dtype):
     assert int(sizes.sum()) == tokens and sizes.shape[0] == min(64, tokens // 256) and int(sizes.max() - sizes.min()) <= 1
 
 
-@pytest.mark.parametrize('tokens,hidden,experts', [(1, 8, 8), (255, 264, 12), (513, 1032, 64), (1024, 520, 8), (40000, 512, 128), (20000, 72, 5)])
+@pytest.mark.parametrize('tokens,hidden,experts', [(1, 8, 8), (255, 264, 12), (513, 1032, 64), (1024, 520, 8), (40000, 512, 128), (20000, 72, 5), (1100, 70, 16)])
 @pytest.mark.parametrize('dtype,weight_dtype', [(torch.bfloat16, torch.bfloat16), (torch.float16, torch.float16), (torch.bfloat16, torch.float32)])
 def test_router_linear_gradients_against_fp64(tokens, hidden, experts, dtype, weight_dtype):
     """Both gradients of the router's linear layer against fp64: fp32 sums rounded once to 16 bits (half a step, 2^-9 or 2^-12, with a
