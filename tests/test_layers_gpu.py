@@ -259,8 +259,8 @@ def test_router_linear_gradients_against_fp64(tokens, hidden, experts, dtype, we
     rounding = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
     sums = 4 * 2.0 ** -24 * max(tokens, 16) ** 0.5
     assert rel_err(x.grad.double(), g.double() @ weight.detach().double()) < rounding
-    # a batch of one piece, or of experts the kernels for fp32 sums do not take, may pass through 16 bits
-    exact = weight_dtype == torch.float32 and tokens >= 512
+    # a batch of one piece, or with rows the kernels for fp32 sums do not take, passes through 16 bits
+    exact = weight_dtype == torch.float32 and tokens >= 512 and hidden % 8 == 0
     assert rel_err(weight.grad.double(), g.double().t() @ x.detach().double()) < (sums if exact else rounding)
 
 
