@@ -317,6 +317,19 @@ int mbx_gmm_scatter(const void* a, const void* b, void* c, void* out, int dtype,
                     int64_t rows, int k, int n, const int32_t* indices, const void* weights, int w_dtype, int64_t tokens,
                     mbx_stream_t stream);
 
+/* What follows the router in the dropless layer's forward where no gradient is recorded (megablocks/layers/dmoe.py:239-280 over
+ * mlp.py:499-523 / glu.py:173-205), enqueued by one call: mbx_route, mbx_gmm_hidden, mbx_gmm_ws and mbx_scatter (with fused_combine
+ * and top_k == 1 mbx_gmm_scatter instead of the last two; mbx_gather first where the first product does not), with their results bit for bit.
+ * x: [tokens, hidden_size]; expert_ids: [tokens * top_k]; weights: the same, of type w_dtype (NULL: 1); w1, v1 (NULL: no gate), w2:
+ * [num_experts, ffn, hidden_size]; out: [tokens, hidden_size]; tokens_per_expert: [num_experts].  scratch:
+ * mbx_experts_forward_scratch_bytes() bytes, 16-byte aligned.  workspace: as for mbx_gmm_ws.  MBX_EUNSUPPORTED: no tokens, fp32, or
+ * what mbx_route or mbx_gmm_hidden do not take; out and tokens_per_expert are then undefined, and the caller issues the separate calls. */
+size_t mbx_experts_forward_scratch_bytes(int64_t tokens, int top_k, int num_experts, int end_bit, int hidden_size, int ffn, int dtype);
+int mbx_experts_forward(const void* x, int64_t tokens, int hidden_size, int dtype, const int32_t* expert_ids, int top_k,
+                        const void* weights, int w_dtype, int num_experts, int end_bit, const void* w1, const void* v1,
+                        const void* w2, int ffn, int act, int fused_combine, void* out, int32_t* tokens_per_expert, void* scratch,
+                        size_t scratch_bytes, void* workspace, size_t workspace_bytes, mbx_stream_t stream);
+
 /* The weight gradient of the experts' first product(s) on token rows that were never gathered: the backward's
  * `gmm(dsdd_out, x, batch_sizes, trans_a=True)` of megablocks/layers/mlp.py:485-491 / glu.py:154-159, where x is what
  * megablocks/layers/dmoe.py:219 / :273 gathered (`ops.padded_gather` / `ops.gather`), with that gather done by the

@@ -19,7 +19,7 @@ PROBE_LIB = os.path.join(HERE, 'libmbx_probe.so')
 # the library with per-tile time stamps in the grouped-GEMM kernels (csrc/gmm_dma.h, MBX_TICKS), for bench.py --tile-ticks
 TICKS_LIB = os.path.join(HERE, 'libmbx_ticks.so')
 PROBE_SOURCE = 'probe.hip'
-SOURCES = ['routing.hip', 'permute.hip', 'gmm.hip', 'gmm_rows.hip', 'gmm_rows_tail.hip', 'gmm_few.hip', 'gmm_f32.hip', 'gmm_mid.hip', 'gmm_pair.hip', 'gmm_tn_short.hip', 'elementwise.hip', 'router.hip']
+SOURCES = ['routing.hip', 'permute.hip', 'gmm.hip', 'gmm_rows.hip', 'gmm_rows_tail.hip', 'gmm_few.hip', 'gmm_f32.hip', 'gmm_mid.hip', 'gmm_pair.hip', 'gmm_tn_short.hip', 'elementwise.hip', 'router.hip', 'experts.hip']
 TICKS_SOURCES = ['gmm.hip', 'gmm_rows.hip', 'gmm_rows_tail.hip']
 HEADERS = [os.path.join(CSRC, 'common.h'), os.path.join(CSRC, 'gmm_dma.h'), os.path.join(CSRC, 'gmm_common.h'), os.path.join(CSRC, 'gmm_rows.h'),
            os.path.join(os.path.dirname(HERE), 'include', 'mbx.h'), os.path.join(os.path.dirname(HERE), 'include', 'mbx_probe.h')]

@@ -583,6 +583,56 @@ def gmm_scatter(a, b, batch_sizes, combine: CombinedRows, keep_product=True):
     return y, out
 
 
+# Assignments up to which `experts_forward` takes a pass: the routing is one launch, and with more the GPU's time is what counts either way.
+EXPERTS_FORWARD_MAX_SLOTS = 4096
+
+
+def experts_forward(x, expert_ids, expert_weights, num_experts, end_bit, top_k, w1, v1, w2, act):
+    """(out, tokens_per_expert) of the grouped dropless layer behind its router (dmoe.py:239-280) without gradients, from one call
+    of the library (`mbx_experts_forward`) that enqueues the launches of `ops.route`, `gmm_gather`, `gmm` and `ops.scatter`: the
+    same results bit for bit.  None: one of those does not take the operands in that form, or they are not plain tensors.
+    x: [tokens, hidden]; w1, v1 (None: no gate), w2: the experts' weights, num_experts x ffn x hidden elements each.
+    (The layer's pass where the host bounds it: 16 tokens, top-2 of 16 experts 119 -> 64 us, one token 102 -> 60; 300 tokens, top-2 of
+    32 experts 147 -> 90; the GPU's time: 4096 assignments, 8 experts of [1024, 2816], 84.)"""
+    tensors = (x, expert_ids, expert_weights, w1, w2) if v1 is None else (x, expert_ids, expert_weights, w1, v1, w2)
+    slots, dtype, device = expert_ids.numel(), x.dtype, x.device
+    if not 0 < slots <= EXPERTS_FORWARD_MAX_SLOTS or dtype not in (torch.bfloat16, torch.float16) or not x.is_cuda or \
+            x.shape[1] == 0 or FUSED_GATHER == '0' or _lib.profile_hook is not None:
+        return None
+    for t in tensors:
+        if (type(t) is not torch.Tensor and type(t) is not torch.nn.Parameter) or t.device != device:
+            return None
+    elements = w1.numel()
+    ffn = elements // (num_experts * x.shape[1])
+    for w in tensors[3:]:
+        if w.dtype != dtype or w.numel() != elements or not w.is_contiguous() or w.data_ptr() % 16:
+            return None
+    if x.shape[1] % 8 or ffn % 8 or ffn * x.shape[1] >= 1 << 30:   # rows and weights the kernels under the call take
+        return None
+    if ffn * num_experts * x.shape[1] != elements or x.shape[0] * top_k != slots or expert_ids.dtype != torch.int32 or \
+            expert_weights.numel() != slots or expert_weights.dtype not in _lib.DTYPE or not _use_epilogue(None, x, slots, ffn):
+        return None
+    x, expert_ids, expert_weights = x.contiguous(), expert_ids.contiguous(), expert_weights.contiguous()
+    if x.data_ptr() % 16:
+        return None
+    tokens, hidden = x.shape
+    code = _lib.DTYPE[dtype]
+    out = torch.empty_like(x)
+    tokens_per_expert = torch.empty(num_experts, dtype=torch.int32, device=device)
+    nbytes = lib.mbx_experts_forward_scratch_bytes(tokens, top_k, num_experts, end_bit, hidden, ffn, code)
+    scratch = torch.empty(nbytes, dtype=torch.uint8, device=device)
+    with _lib.device_of(x):
+        ws, ws_bytes = _workspace(device)
+        rc = lib.mbx_experts_forward(x.data_ptr(), tokens, hidden, code, expert_ids.data_ptr(), top_k, expert_weights.data_ptr(),
+                                     _lib.DTYPE[expert_weights.dtype], num_experts, end_bit, w1.data_ptr(), _lib.ptr(v1), w2.data_ptr(), ffn, act,
+                                     FUSED_COMBINE != '0', out.data_ptr(), tokens_per_expert.data_ptr(), scratch.data_ptr(), nbytes,
+                                     ws, ws_bytes, _lib.stream())
+    if rc == _lib.EUNSUPPORTED:
+        return None
+    _lib.check(rc, 'experts_forward')
+    return out, tokens_per_expert
+
+
 def gmm_dglu(a, b, x1, x2, batch_sizes, act, fuse=None):
     """The gradients (d x1, d x2) of `activation(x1) * x2` where the incoming gradient is g = a[r_e] @ b[e].T: the
     `gmm(ddsd_out, w2, trans_b=True)` of the GLU experts' backward and the backward of their gated activation

@@ -12,7 +12,12 @@ from megablocks_amd.ops import routing as ops_routing
 from megablocks_amd import grouped_gemm_util as gg
 from megablocks_amd.layers import common, dmlp_registry, moe, mpu
 from megablocks_amd.layers.arguments import Arguments
-from megablocks_amd.layers.mlp import Topology
+from megablocks_amd.layers.glu import GroupedGLU, _activation_code
+from megablocks_amd.layers.mlp import DEFAULT_ACTIVATION_FN, GroupedMLP, Topology
+
+
+# whether a torch.func transform is under way
+_transforms_active = getattr(torch._C, '_are_functorch_transforms_active', lambda: False)
 
 
 def promote_scalar(x):
@@ -151,10 +156,35 @@ class ParallelDroplessMLP(moe.ParallelMLP):
         x = self._sparse_experts(x, indices, bin_ids, bins, padded_bins, top_k)
         return ops.padded_scatter(x, indices, bin_ids, expert_weights, bins, padded_bins, top_k)
 
+    def _one_call_forward(self, x, expert_weights, top_experts):
+        """grouped_forward_once from one call of the library (gg.experts_forward), where the layer and its experts are the
+        built-in ones, nothing is traced or transformed and no gradient is recorded; else None."""
+        experts = self.mlp
+        if type(self) is not ParallelDroplessMLP or 'forward_tokens' in experts.__dict__ or \
+                not self.__dict__.keys().isdisjoint(('indices_and_bins', 'grouped_permute_and_compute', 'permute_and_compute')):
+            return None
+        if type(experts) is GroupedMLP:
+            act = gg.ACT_GELU_TANH if self.args.activation_fn is DEFAULT_ACTIVATION_FN else None
+            v1 = None
+        elif type(experts) is GroupedGLU:
+            act, v1 = _activation_code(self.args.activation_fn), experts.v1
+        else:
+            return None
+        if act is None or experts.gradient_scale is not None or mpu.experts_per_rank(self.args) != self.num_experts or \
+                torch.is_autocast_enabled() or torch.compiler.is_compiling() or _transforms_active() or \
+                torch.autograd.forward_ad._current_level >= 0 or torch._C._get_tracing_state() is not None:
+            return None
+        return gg.experts_forward(x.view(-1, x.shape[-1]), top_experts.int(), expert_weights, self.num_experts, self.sort_end_bit,
+                                  self.args.moe_top_k, experts.w1, v1, experts.w2, act)
+
     def grouped_forward_once(self, x, expert_weights, top_experts):
         """dmoe.py:239-258."""
         expert_weights = expert_weights.flatten()
         top_experts = top_experts.flatten()
+        if not torch.is_grad_enabled():
+            done = self._one_call_forward(x, expert_weights, top_experts)
+            if done is not None:
+                return done
         with torch.no_grad():
             indices, bin_ids, bins, tokens_per_expert = self.indices_and_bins(top_experts)
         out = self.grouped_permute_and_compute(x, tokens_per_expert, indices, bin_ids, expert_weights, bins, -1,

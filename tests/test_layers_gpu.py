@@ -1226,6 +1226,40 @@ def test_dmoe_forward_without_gradients_on_no_tokens_and_on_a_few(monkeypatch, m
 
 
 @pytest.mark.parametrize('mlp_type', ['mlp', 'glu'])
+@pytest.mark.parametrize('tokens,hs,ffn,ne,top_k,one_call', [(1, 64, 72, 1, 1, True), (5, 136, 264, 12, 6, True), (300, 256, 520, 8, 1, True), (4096, 64, 128, 128, 1, True),
+                                                             (683, 72, 200, 16, 6, False), (7, 64, 132, 4, 2, False), (7, 60, 128, 4, 2, False)])
+def test_dmoe_forward_from_one_call_is_the_separate_calls(monkeypatch, mlp_type, tokens, hs, ffn, ne, top_k, one_call):
+    """The layer behind its router in one call of the library, without gradients: bit for bit what the separate calls give, for
+    strided and int64 assignments and fp32 gate weights too, at the longest list it takes; longer lists and rows that are
+    not whole 16-byte pieces are left to the separate calls, and wrong sizes are refused as there."""
+    from megablocks_amd import grouped_gemm_util as gg
+    from megablocks_amd.layers.dmoe import dMoE
+    torch.manual_seed(tokens)
+    layer = dMoE(_args(hidden_size=hs, ffn_hidden_size=ffn, moe_num_experts=ne, moe_top_k=top_k, mlp_type=mlp_type))
+    x = torch.randn(tokens, 1, hs, device='cuda').bfloat16()
+    ids = torch.rand(tokens, ne, device='cuda').topk(top_k).indices
+    weights = torch.rand(tokens, top_k, device='cuda').bfloat16()
+    wide = torch.zeros(tokens, 2 * top_k, device='cuda', dtype=torch.int32)
+    wide[:, ::2] = ids
+    forms = [(x, weights, ids.int()), (x, weights.float(), ids), (x, weights.repeat_interleave(2, 1)[:, ::2], wide[:, ::2]),
+             (torch.cat([x, x], -1)[..., :hs], weights, ids.int())]
+    seen = []
+    call = gg.experts_forward
+    monkeypatch.setattr(gg, 'experts_forward', lambda *a: seen.append(call(*a)) or seen[-1])
+    with torch.no_grad():
+        got = [layer.experts(a, None, w, i) for a, w, i in forms]
+        counts = [layer.experts.forward_once(a, w, i)[1] for a, w, i in forms[:1]]
+        assert len(seen) == len(forms) + 1 and all((s is not None) == one_call for s in seen)
+        with pytest.raises(ValueError):
+            layer.experts(x, None, weights[:, :0], ids.int())
+        monkeypatch.setattr(gg, 'experts_forward', lambda *a: None)
+        for g, (a, w, i) in zip(got, forms):
+            assert torch.equal(g, layer.experts(a, None, w, i))
+        assert torch.equal(counts[0], layer.experts.forward_once(*forms[0])[1])
+    assert torch.equal(counts[0].long(), torch.bincount(ids.flatten(), minlength=ne))
+
+
+@pytest.mark.parametrize('mlp_type', ['mlp', 'glu'])
 def test_memory_optimized_dmoe_forward_without_gradients_gathers_in_the_first_product(syn, monkeypatch, mlp_type):
     """memory_optimized_mlp only changes what the backward keeps: without gradients the layer takes the same forward
     as the plain one, first product on the ungathered tokens included."""
