@@ -17,6 +17,8 @@
 // Layouts are gmm_dma.h's for strided operands of 128 columns: [k][128] rows, transposing reads.
 #include "gmm_common.h"
 
+#include <cmath>
+
 namespace mbx {
 namespace {
 
@@ -255,7 +257,7 @@ gmm_tn_short_kernel(const uint16_t* __restrict__ a, const uint16_t* __restrict__
   if (AHEAD) prefetch.arrived();
 }
 
-// ---- up to a few hundred rows per expert, many tiles: takes_mid() ----
+// ---- a few hundred rows per expert: choose() ----
 // 256 x 128 tiles, two workgroups of four waves to a compute unit, each with three stages of 32 rows: two K tiles under way while one is
 // multiplied, one barrier per K tile.
 typedef dma::Tile<256, 128, 2, 2, 64, 2> TM;   // for its shape
@@ -390,33 +392,63 @@ int launch(const DmaCall& q) {
 }
 
 
+enum Kernel { kDma, kShort, kMid };   // gmm_dma.h's 256 x 256 tiles, 128 x 128 of 64 rows, 256 x 128 of 32 rows
+
+// What the kernel's launch is estimated to take, us: rounds of tiles, each a start and so much per 64 rows, and no less than the
+// operands and products at the rate it moves them.  A last round that is not full costs `part` of one with the compute units' first
+// workgroups and grows from there to a whole one.  Fitted to 472 launches (4 - 128 experts of 280 - 1300 rows, [704 - 8192, 512 - 4096],
+// memory that is not in the last-level cache); rms 11 %.
+struct Cost {
+  int height, width, per_cu;
+  double start, tile, k_tile, part, rate;
+  double operator()(const DmaCall& q, double units, double average) const {
+    const double all = (double)ceil_div(q.k, height) * ceil_div(q.n, width) * q.num_groups / (per_cu * units), full = floor(all), rest = all - full;
+    const double one = 1.0 / per_cu, grown = per_cu == 1 ? rest : rest > one ? (rest - one) / (1 - one) : 0.0;
+    const double rounds = full + (rest > 0 ? part + (1 - part) * grown : 0.0);
+    const double mb = ((double)q.rows * (q.k + q.n) + (double)q.num_groups * q.k * q.n) * 2e-6;
+    return start + fmax(rounds * (tile + k_tile * average / 64), mb / rate);
+  }
+};
+constexpr Cost kCosts[] = {{256, 256, 1, 5.0, 6.2, 1.59, 0.58, 2.96}, {128, 128, kPerCu, 4.8, 0.75, 2.35, 0.46, 3.62}, {256, 128, kMidPerCu, 4.9, 3.3, 2.01, 0.53, 3.61}};
+
+// Up to 256 rows per expert on average 128 x 128 tiles: beyond, gmm_dma.h's tile hides its latencies behind its products, and its
+// wider tile reads less.  Up to 1024 rows where all of them run at once: 256 x 256 tiles would leave most compute units idle (8
+// experts, [576, 1024]: 18.6 against 12.8 us at 512 rows, 26.9 against 20.7 at 1024).
 // 256 x 128 tiles out of three small stages where there are five rounds of them, up to 512 rows per expert on average, and of few rows
 // where no half of a row of them is empty: they read a quarter less than 128 x 128 tiles and need a third fewer workgroups, but
 // their last round is longer (us, this / 128 x 128, gmm_dma.h's above 256 rows; operands and products not in the last-level cache:
 // 64 experts, [1024, 4096]: 64 rows 134 / 135, 128: 155 / 170, 256: 203 / 216, 512: 318 / 330;  8, [4096, 14336]: 250: 333 / 345, 500: 522 / 515,
 // 600: 603 / 574;  64, [2048, 1408]: 100: 106 / 99, 200: 134 / 133, 300: 172 / 176;  16 of 300, [2048, 1408], three rounds: 53 / 46).
-static bool takes_mid(const DmaCall& q) {
-  const int64_t average = q.rows / q.num_groups, tiles = ceil_div(q.k, TM::BM) * ceil_div(q.n, TM::BN) * q.num_groups;
-  if (q.gather.slots || average <= 64 || average > 512 || tiles < 5 * kMidPerCu * (int64_t)persistent_grid((int64_t)1 << 30)) return false;
-  return average > 256 || q.k % TM::BM == 0 || q.k % TM::BM > TM::BM / 2;
+// From 256 to 768 rows another kernel than these lines say where its estimate is shorter by a sixteenth: half-empty last rounds and
+// half-empty tiles decide there.  135 launches that the estimates were not fitted to (4 - 128 experts, [704 - 8192, 512 - 4096] at random): 256 - 320
+// rows 15 % shorter on the geometric mean, to 400 8 %, to 512 6 %, to 768 3 %, four of them 3 - 9 % longer; above 768 rows they gain nothing.
+// (From / to: 64 experts of 300, [1408, 512]: 59 / 43; 64 of 520, [2304, 576]: 148 / 108; 16 of 300, [3072, 768]: 44 / 36; 8 of 450, [1408, 2048]: 35 / 30;
+// 12 of 500, [1472, 1344]: 41 / 42; 32 of 670, [1664, 832]: 88 / 96.)
+static Kernel choose(const DmaCall& q) {
+  const double units = persistent_grid((int64_t)1 << 30);
+  const int64_t average = q.rows / q.num_groups, tiles = ceil_div(q.k, 128) * ceil_div(q.n, 128) * q.num_groups;
+  const int64_t mid_tiles = ceil_div(q.k, TM::BM) * ceil_div(q.n, TM::BN) * q.num_groups;
+  Kernel kernel = q.rows <= (int64_t)((double)tiles <= kPerCu * units ? 1024 : 256) * q.num_groups ? kShort : kDma;
+  if (q.gather.slots) return kernel;
+  if (average > 64 && average <= 512 && (double)mid_tiles >= 5 * kMidPerCu * units && (average > 256 || q.k % TM::BM == 0 || q.k % TM::BM > TM::BM / 2)) kernel = kMid;
+  if (average < 256 || average > 768) return kernel;
+  const double here = kCosts[kernel](q, units, (double)average);
+  for (Kernel other : {kDma, kShort, kMid})
+    if (kCosts[other](q, units, (double)average) < fmin(0.94 * here, kCosts[kernel](q, units, (double)average))) kernel = other;
+  return kernel;
 }
 
 }  // namespace tn_short
 }  // namespace
 
-// Up to 256 rows per expert on average: beyond, gmm_dma.h's tile hides its latencies behind its products, and its wider tile
-// reads less (64 experts, [1024, 4096]: 344 against 366 us at 512 rows; 8 experts, [4096, 14336]: 443 against 447 at 384).
-// Up to 1024 rows where all tiles run at once: 256 x 256 tiles would leave most compute units idle (8 experts, [576, 1024]:
-// 18.6 against 12.8 us at 512 rows, 26.9 against 20.7 at 1024).
 bool gmm_tn_short_takes(const DmaCall& q) {
   const int64_t widest = q.k > q.n ? q.k : q.n;
   if (q.layout != MBX_TN || q.rows * widest * 2 >= ((int64_t)1 << 31)) return false;   // one buffer per operand
-  const int64_t tiles = ceil_div(q.k, 128) * ceil_div(q.n, 128) * q.num_groups, at_once = tn_short::kPerCu * (int64_t)persistent_grid((int64_t)1 << 30);
-  return q.rows <= (int64_t)(tiles <= at_once ? 1024 : 256) * q.num_groups || tn_short::takes_mid(q);
+  return tn_short::choose(q) != tn_short::kDma;
 }
 
 int gmm_tn_short(const DmaCall& q) {
-  const bool mid = tn_short::takes_mid(q);
+  const bool mid = tn_short::choose(q) == tn_short::kMid;
   if (q.out32) {
     if (mid) return q.dtype == MBX_BF16 ? tn_short::launch_mid<MBX_BF16, true>(q) : tn_short::launch_mid<MBX_F16, true>(q);
     return q.dtype == MBX_BF16 ? tn_short::launch<MBX_BF16, true>(q) : tn_short::launch<MBX_F16, true>(q);

@@ -1497,7 +1497,8 @@ def test_gmm_tn_with_few_rows_per_expert(gg, groups, rows, k, n, skew, dtype):
         assert torch.equal(gg.gmm_tn_gather(a, src, sizes.cuda()), gg.backend.gmm(a, x[order.long()], sizes, trans_a=True))
 
 
-@pytest.mark.parametrize('groups,rows,k,n', [(70, 70 * 80, 504, 2568), (64, 64 * 300, 520, 1672), (9, 9 * 270, 4600, 2056), (12, 12 * 100, 768, 1032)])
+@pytest.mark.parametrize('groups,rows,k,n', [(70, 70 * 80, 504, 2568), (64, 64 * 300, 520, 1672), (9, 9 * 270, 4600, 2056), (12, 12 * 100, 768, 1032),
+                                             (16, 16 * 300, 1160, 648), (40, 40 * 520, 2312, 584), (6, 6 * 1024, 1416, 520), (4, 4 * 280, 2056, 1032)])
 @pytest.mark.parametrize('spread', ['alike', 'skewed'])
 @pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])
 def test_gmm_tn_of_many_tiles(gg, groups, rows, k, n, spread, dtype):
