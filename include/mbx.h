@@ -63,7 +63,7 @@ int mbx_sort(const void* x, int itype, int64_t n, int end_bit, void* keys_out,
              void* perm_out, void* scratch, size_t scratch_bytes, mbx_stream_t stream);
 
 /* The routing bookkeeping of one layer step, megablocks/layers/moe.py:152-183 (`indices_and_bins`) and
- * megablocks/layers/dmoe.py:131-154 (`indices_and_padded_bins`), in one launch up to 4096 ids, three above, instead of the seven of
+ * megablocks/layers/dmoe.py:131-154 (`indices_and_padded_bins`), in one launch up to 4096 ids, two above (three for count tables past 6144 entries), instead of the seven of
  * sort + histogram + the cumsums + mbx_slot_rows.  For int32 expert ids [n] in [0, num_experts):
  *   bin_ids, indices      = sort(expert_ids, end_bit)                      (csrc/sort.h:59)
  *   tokens_per_expert     = histogram(expert_ids, num_experts)             (csrc/histogram.h:61)

@@ -244,6 +244,57 @@ route_scan_kernel(int32_t* __restrict__ table, int ndigits, int nblocks, int32_t
   }
 }
 
+// Pass steps 2 and 3 in one launch for count tables of up to kFoldMost entries: every block of the scatter scans the whole table for
+// itself, a thread a run of it, and keeps what it needs: where its keys of each digit start (at) and where each digit starts
+// (first, first[ndigits] = n).  A launch of one workgroup less; us of the pass out of a graph, mbx_sort and mbx_route with pad: 65536
+// keys of 8 digits (1024 entries) 8.5 -> 7.4 and 9.9 -> 7.8, 16384 of 64 (2048) 9.8 -> 9.0 and 11.6 -> 9.5, 196608 of 64 (6144) 21.1 -> 21.1
+// and 24.9 -> 22.1; 65536 of 64 (8192) would be 13.5 -> 13.8.
+constexpr int kFoldMost = 6144, kFoldRun = kFoldMost / kSortThreads;
+__device__ __forceinline__ void fold_counts(const int32_t* __restrict__ table, int ndigits, int nblocks, int32_t* first, int32_t* at, int32_t* wave_tot) {
+  const int entries = ndigits * nblocks, run = (entries + kSortThreads - 1) / kSortThreads, i0 = (int)threadIdx.x * run, mine = (int)blockIdx.x;
+  int32_t v[kFoldRun];
+  int32_t sum = 0;
+#pragma unroll
+  for (int g = 0; g < kFoldRun; g += 8) {
+    if (g >= run) break;   // uniform
+#pragma unroll
+    for (int q = g; q < g + 8; ++q) v[q] = q < run && i0 + q < entries ? table[i0 + q] : 0;
+#pragma unroll
+    for (int q = g; q < g + 8; ++q) sum += v[q];
+  }
+  const int32_t inc = wave_inclusive_scan(sum);
+  if (lane_id() == 63) wave_tot[threadIdx.x / kWave] = inc;
+  __syncthreads();
+  int32_t before = inc - sum, all = 0;
+#pragma unroll
+  for (int w = 0; w < kSortWaves; ++w) {
+    before += w < (int)threadIdx.x / kWave ? wave_tot[w] : 0;
+    all += wave_tot[w];
+  }
+  int d = i0 / nblocks, b = i0 - d * nblocks;
+#pragma unroll
+  for (int g = 0; g < kFoldRun; g += 8) {
+    if (g >= run) break;
+#pragma unroll
+    for (int q = g; q < g + 8; ++q) {
+      if (q < run && i0 + q < entries) {
+        if (b == 0) first[d] = before;
+        if (b == mine) at[d] = before;
+        before += v[q];
+        if (++b == nblocks) { b = 0; ++d; }
+      }
+    }
+  }
+  if (threadIdx.x == 0) first[ndigits] = all;
+  __syncthreads();
+}
+
+// What the scatter of mbx_route writes besides, from the folded table (as route_scan_kernel's).
+struct RouteOut {
+  int32_t *tokens_per_expert, *bins, *padded_bins;
+  int num_experts, pad;
+};
+
 // Pass step 3: stable scatter.  Wave w of a block owns kSortItems consecutive rounds of 64
 // consecutive keys, so "earlier key" means earlier wave, then earlier round, then lower lane.
 // slot_rows (with IOTA, i.e. on the first pass, whose values are the key's positions in the input; NULL: not wanted):
@@ -251,15 +302,38 @@ route_scan_kernel(int32_t* __restrict__ table, int ndigits, int nblocks, int32_t
 // that holds it: p itself, or with padded_bins the row p - bins[e - 1] + padded_bins[e - 1] of expert e's padded
 // block (-1 for a key whose digit is at or past num_bins) -- the map inverse_map_kernel of the permutation kernels
 // builds.
-template <typename T, bool IOTA, int kSortItems>
+// FOLD: `offsets` is the table of counts, not yet scanned (fold_counts), and block 0 writes `route` (its pointers NULL: not wanted).
+template <typename T, bool IOTA, int kSortItems, bool FOLD>
 __global__ void __launch_bounds__(kSortThreads)
 radix_scatter_kernel(const T* __restrict__ keys_in, const T* __restrict__ vals_in, int64_t n,
                      int shift, uint32_t mask, int nbits, const int32_t* __restrict__ offsets,
                      int nblocks, T* __restrict__ keys_out, T* __restrict__ vals_out,
                      int32_t* __restrict__ slot_rows = nullptr, const int32_t* __restrict__ bins = nullptr,
-                     const int32_t* __restrict__ padded_bins = nullptr, int num_bins = 0) {
+                     const int32_t* __restrict__ padded_bins = nullptr, int num_bins = 0, RouteOut route = {}) {
   __shared__ int32_t wave_hist[kSortWaves][kRadix];
+  __shared__ int32_t first[FOLD ? kRadix + 1 : 1], at[FOLD ? kRadix : 1], shift_of[FOLD ? kRadix : 1], wave_tot[kSortWaves];
   const int lane = lane_id(), wave = threadIdx.x / kWave;
+  if constexpr (FOLD) {
+    const int ndigits = 1 << nbits, e = (int)threadIdx.x;
+    fold_counts(offsets, ndigits, nblocks, first, at, wave_tot);
+    if (route.bins != nullptr) {
+      const bool expert = e < route.num_experts;   // no more of them than digits
+      const int32_t count = expert ? first[e + 1] - first[e] : 0;
+      if (blockIdx.x == 0 && expert) {
+        route.tokens_per_expert[e] = count;
+        route.bins[e] = first[e + 1];
+      }
+      if (route.padded_bins != nullptr) {
+        const int32_t padded = (count + route.pad - 1) / route.pad * route.pad, inc = wave_inclusive_scan(padded);
+        if (lane == 63) wave_tot[wave] = inc;
+        __syncthreads();
+        int32_t end = inc;
+        for (int w = 0; w < wave; ++w) end += wave_tot[w];
+        if (blockIdx.x == 0 && expert) route.padded_bins[e] = end;
+        shift_of[e] = end - padded - (expert ? first[e] : 0);   // from a sorted position to its row of the padded buffer
+      }
+    }
+  }
   for (int w = 0; w < kSortWaves; ++w) wave_hist[w][threadIdx.x] = 0;
   __syncthreads();
 
@@ -278,7 +352,7 @@ radix_scatter_kernel(const T* __restrict__ keys_in, const T* __restrict__ vals_i
   __syncthreads();
   {  // thread d turns the per-wave counts of digit d into starting positions
     const int d = threadIdx.x;
-    int32_t run = offsets[(int64_t)d * nblocks + blockIdx.x];
+    int32_t run = FOLD ? (d < 1 << nbits ? at[d] : 0) : offsets[(int64_t)d * nblocks + blockIdx.x];
 #pragma unroll
     for (int w = 0; w < kSortWaves; ++w) {
       const int32_t c = wave_hist[w][d];
@@ -310,6 +384,7 @@ radix_scatter_kernel(const T* __restrict__ keys_in, const T* __restrict__ vals_i
           // of the padded buffer inside a bin so has exactly one slot or is padding.
           const int e = (int)dig[it];
           if (e >= num_bins) row = -1;
+          else if (FOLD) row = pos + shift_of[e];
           else if (e > 0) row = pos - bins[e - 1] + padded_bins[e - 1];
         }
         slot_rows[i] = row;
@@ -440,18 +515,28 @@ int sort_impl(const T* x, int64_t n, int end_bit, T* keys_out, T* perm_out, void
     const bool to_final = ((passes - 1 - p) % 2) == 0;
     T* kout = to_final ? keys_out : tmp_keys;
     T* vout = to_final ? perm_out : tmp_vals;
+    // digit-major: digits the pass cannot produce come last
+    const int64_t entries = ((int64_t)1 << pass_bits) * nblocks;
+#define MBX_SORT_SCATTER(ITEMS, FOLD)                                                                                     \
+  do {                                                                                                                    \
+    if (p == 0)                                                                                                           \
+      radix_scatter_kernel<T, true, ITEMS, FOLD><<<nblocks, kSortThreads, 0, s>>>(kin, nullptr, n, shift, mask, pass_bits, counts, nblocks, kout, vout); \
+    else                                                                                                                  \
+      radix_scatter_kernel<T, false, ITEMS, FOLD><<<nblocks, kSortThreads, 0, s>>>(kin, vin, n, shift, mask, pass_bits, counts, nblocks, kout, vout);    \
+  } while (0)
 #define MBX_SORT_PASS(ITEMS)                                                                                              \
   do {                                                                                                                    \
     radix_count_kernel<T, ITEMS><<<nblocks, kSortThreads, 0, s>>>(kin, n, shift, mask, pass_bits, counts, nblocks);       \
-    /* digit-major: digits the pass cannot produce come last */                                                           \
-    exclusive_scan_i32_kernel<<<1, 1024, 0, s>>>(counts, ((int64_t)1 << pass_bits) * nblocks);                            \
-    if (p == 0)                                                                                                           \
-      radix_scatter_kernel<T, true, ITEMS><<<nblocks, kSortThreads, 0, s>>>(kin, nullptr, n, shift, mask, pass_bits, counts, nblocks, kout, vout); \
-    else                                                                                                                  \
-      radix_scatter_kernel<T, false, ITEMS><<<nblocks, kSortThreads, 0, s>>>(kin, vin, n, shift, mask, pass_bits, counts, nblocks, kout, vout);    \
+    if (entries <= kFoldMost) {                                                                                           \
+      MBX_SORT_SCATTER(ITEMS, true);                                                                                      \
+    } else {                                                                                                              \
+      exclusive_scan_i32_kernel<<<1, 1024, 0, s>>>(counts, entries);                                                      \
+      MBX_SORT_SCATTER(ITEMS, false);                                                                                     \
+    }                                                                                                                     \
   } while (0)
     if (items == kSortItemsShort) MBX_SORT_PASS(kSortItemsShort); else MBX_SORT_PASS(kSortItemsLong);
 #undef MBX_SORT_PASS
+#undef MBX_SORT_SCATTER
     kin = kout;
     vin = vout;
   }
@@ -623,12 +708,18 @@ int mbx_route(const int32_t* expert_ids, int64_t n, int num_experts, int end_bit
   }
   const int items = sort_items(n, scratch_bytes), nblocks = sort_blocks(n, items);
   int32_t* counts = (int32_t*)scratch;
+  const RouteOut route{tokens_per_expert, bins, pbins, num_experts, pad};
 #define MBX_ROUTE_PASS(ITEMS)                                                                                             \
   do {                                                                                                                    \
     radix_count_kernel<int32_t, ITEMS><<<nblocks, kSortThreads, 0, s>>>(expert_ids, n, 0, mask, end_bit, counts, nblocks); \
-    route_scan_kernel<<<1, 1024, 0, s>>>(counts, ndigits, nblocks, (int32_t)n, num_experts, pad, tokens_per_expert, bins, pbins); \
-    radix_scatter_kernel<int32_t, true, ITEMS><<<nblocks, kSortThreads, 0, s>>>(expert_ids, nullptr, n, 0, mask, end_bit, counts, nblocks, \
+    if ((int64_t)ndigits * nblocks <= kFoldMost) {                                                                        \
+      radix_scatter_kernel<int32_t, true, ITEMS, true><<<nblocks, kSortThreads, 0, s>>>(expert_ids, nullptr, n, 0, mask, end_bit, counts, nblocks, \
+                                                                                bin_ids, indices, slot_rows, bins, pbins, num_experts, route);    \
+    } else {                                                                                                              \
+      route_scan_kernel<<<1, 1024, 0, s>>>(counts, ndigits, nblocks, (int32_t)n, num_experts, pad, tokens_per_expert, bins, pbins); \
+      radix_scatter_kernel<int32_t, true, ITEMS, false><<<nblocks, kSortThreads, 0, s>>>(expert_ids, nullptr, n, 0, mask, end_bit, counts, nblocks, \
                                                                                 bin_ids, indices, slot_rows, bins, pbins, num_experts);    \
+    }                                                                                                                     \
   } while (0)
   if (items == kSortItemsShort) MBX_ROUTE_PASS(kSortItemsShort); else MBX_ROUTE_PASS(kSortItemsLong);
 #undef MBX_ROUTE_PASS

@@ -515,6 +515,28 @@ def test_route_at_the_edges_of_its_launches(n, experts):
     assert torch.equal(got.cpu(), want) and torch.equal(perm.cpu(), want_perm.int())
 
 
+@pytest.mark.parametrize('n,experts', [(12288, 256), (12289, 256), (49152, 64), (49153, 64), (98304, 128), (98305, 128)])
+def test_route_at_the_longest_count_table_the_scatter_scans(n, experts):
+    """Count tables of 6144 entries, the longest that the scatter scans for itself, and one tile more; assignments outside the
+    experts' range there, and keys of two passes."""
+    test_route_at_the_edges_of_its_launches(n, experts)
+    from megablocks_amd.ops import routing
+    bits = experts.bit_length() - 1
+    ids = torch.randint(0, experts, (n,), generator=torch.Generator().manual_seed(n), dtype=torch.int32)
+    few = experts - 5                                               # the five last digits name no expert
+    indices, bin_ids, tpe, bins, pbins = routing.route(ids.cuda(), few, bits, 128)
+    want, order = torch.sort(ids, stable=True)
+    counts = torch.bincount(ids, minlength=experts)[:few]
+    ends = torch.cumsum((counts + 127) // 128 * 128, 0)
+    assert torch.equal(bin_ids.cpu(), want) and torch.equal(indices.cpu(), order.int())
+    assert torch.equal(tpe.cpu(), counts.int()) and torch.equal(bins.cpu(), torch.cumsum(counts, 0).int()) and torch.equal(pbins.cpu(), ends.int())
+    rows = torch.full((n,), -1, dtype=torch.int64)
+    named = want < few
+    starts = ends - (counts + 127) // 128 * 128
+    rows[order[named]] = (torch.arange(n) - (torch.cumsum(counts, 0) - counts)[want.clamp(max=few - 1).long()] + starts[want.clamp(max=few - 1).long()])[named]
+    assert torch.equal(indices._mbx_slot_rows[1][:n].cpu(), rows.int())
+
+
 @pytest.mark.parametrize('n', [1, 4096, 4097, 30000, 65536, 65537])
 def test_sort_and_route_at_the_limits_of_the_scratch(n):
     """A count table of 1024 bytes per 2048 keys is enough for either call (next to the two buffers of a sort of several passes),
