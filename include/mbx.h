@@ -201,6 +201,12 @@ int mbx_binned_scatter_wgrad(const void* x, const void* grad, int dtype, int64_t
                              int hidden, int top_k, const int32_t* indices, const int32_t* bins,
                              int num_bins, int capacity, void* wgrad, mbx_stream_t stream);
 
+/* Both gradients of binned_scatter (megablocks/ops/binned_scatter.py:34-56) in one pass over grad [tokens, hidden]: dx [num_bins,
+ * capacity, hidden] as mbx_binned_gather of grad with the weights writes it, and wgrad as mbx_binned_scatter_wgrad. */
+int mbx_binned_scatter_backward(const void* x, const void* grad, int dtype, int64_t tokens, int hidden, int top_k,
+                                const int32_t* indices, const int32_t* bins, int num_bins, int capacity, const void* weights,
+                                int w_dtype, void* dx, void* wgrad, mbx_stream_t stream);
+
 /* ------------------------------------------------------------------ grouped GEMM */
 
 /* grouped_gemm.backend.gmm(a, b, batch_sizes, trans_a, trans_b, c) as called through

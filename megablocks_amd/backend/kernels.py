@@ -333,3 +333,35 @@ def binned_scatter_wgrad(x, grad, indices, bins, top_k):
                                                 _lib.ptr(indices), _lib.ptr(bins), num_experts, expert_capacity,
                                                 _lib.ptr(out), _lib.stream()), 'binned_scatter_wgrad')
     return out
+
+
+def binned_scatter_backward(x, grad, indices, weights, bins, top_k):
+    """Both gradients of `binned_scatter` of `x`: (binned_gather of `grad` weighted, binned_scatter_wgrad), as
+    megablocks/ops/binned_scatter.py:34-56 computes them with two kernels, in one pass over `grad`."""
+    if grad.dtype != x.dtype:
+        return (binned_gather(grad, indices, weights, bins, x.shape[1], top_k),
+                binned_scatter_wgrad(x, grad, indices, bins, top_k))
+    assert_is_tensor(x, 3)
+    assert_is_matrix(grad)
+    assert_is_vector(indices)
+    assert_is_vector(bins)
+    assert_equal(bins.shape[0], x.shape[0])
+    _lib.require_cuda(x, grad, indices, bins, weights)
+    x, grad = x.contiguous(), grad.contiguous()
+    num_experts, expert_capacity, hidden_size = x.shape
+    assert_equal(grad.shape[1], hidden_size)
+    n_slots = indices.shape[0]
+    tokens = n_slots // top_k
+    assert_equal(grad.shape[0], tokens)
+    assert_equal(n_slots, tokens * top_k)
+    if weights is not None:
+        assert_equal(weights.shape[0], n_slots)
+    indices, bins = _lib.as_i32(indices), _lib.as_i32(bins)
+    wp, wdt, weights = _w(weights)
+    dgrad = torch.empty_like(x)
+    wgrad = torch.empty((n_slots,), dtype=x.dtype, device=x.device)
+    with _lib.device_of(x):
+        _lib.check(lib.mbx_binned_scatter_backward(_lib.ptr(x), _lib.ptr(grad), _lib.dtype_of(x), tokens, hidden_size, top_k,
+                                                   _lib.ptr(indices), _lib.ptr(bins), num_experts, expert_capacity, wp, wdt,
+                                                   _lib.ptr(dgrad), _lib.ptr(wgrad), _lib.stream()), 'binned_scatter_backward')
+    return dgrad, wgrad

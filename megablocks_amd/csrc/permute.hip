@@ -578,6 +578,58 @@ binned_wgrad_kernel(const void* __restrict__ x_, const void* __restrict__ grad_,
   }
 }
 
+// binned_gather_kernel of grad and binned_wgrad_kernel as one pass over the rows of grad: both read them, and the separate
+// pass is as long as the reading (16384 rows of 768, 32 experts, fp16: 17.9 + 9.2 -> 16.6 us).
+template <int DT>   // rows of whole 16-byte pieces
+__global__ void __launch_bounds__(kRowThreads)
+binned_scatter_backward_kernel(const void* __restrict__ x_, const void* __restrict__ grad_, int64_t tokens, int hidden, int top_k,
+                               const int32_t* __restrict__ indices, const int32_t* __restrict__ bins, int num_bins, int capacity,
+                               const void* __restrict__ weights, int w_dtype, void* __restrict__ dx_, void* __restrict__ wgrad_) {
+  typedef typename Elem<DT>::type E;
+  const E* grad = (const E*)grad_;
+  const int n_slots = (int)(tokens * top_k);
+  const int wave = threadIdx.x / kWave;
+  const int64_t total = (int64_t)num_bins * capacity;
+  for (int64_t r = (int64_t)blockIdx.x * kRowWaves + wave; r < total; r += (int64_t)gridDim.x * kRowWaves) {
+    const int e = (int)(r / capacity), j = (int)(r % capacity);
+    const int start = e > 0 ? bins[e - 1] : 0;
+    const E* x = (const E*)x_ + r * hidden;
+    E* dx = (E*)dx_ + r * hidden;
+    int s = -1;
+    if (start + j < bins[e] && start + j < n_slots) s = indices[start + j];
+    if (s < 0 || s >= n_slots) { wave_zero_row<DT, true>(dx, hidden); continue; }
+    const E* g = grad + (int64_t)(s / top_k) * hidden;
+    const float scale = weights ? load_as_f32(weights, s, w_dtype) : 1.f;
+    float d = 0.f;
+    // in the order of wave_dot_row
+    constexpr int EV = Vec16<DT>::kElems;
+    const int nvec = hidden / EV;
+    for (int c0 = lane_id(); c0 < nvec; c0 += 4 * kWave) {
+      u32x4 gv[4], xv[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (c0 + i * kWave < nvec) {
+          gv[i] = ((const u32x4*)g)[c0 + i * kWave];
+          xv[i] = __builtin_nontemporal_load((const u32x4*)x + c0 + i * kWave);
+        }
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (c0 + i * kWave < nvec) {
+          float fx[EV], fg[EV];
+          Vec16<DT>::unpack(xv[i], fx);
+          Vec16<DT>::unpack(gv[i], fg);
+#pragma unroll
+          for (int q = 0; q < EV; ++q) d += fx[q] * fg[q];
+#pragma unroll
+          for (int q = 0; q < EV; ++q) fg[q] *= scale;
+          ((u32x4*)dx)[c0 + i * kWave] = weights ? Vec16<DT>::pack(fg) : gv[i];
+        }
+    }
+    d = wave_sum(d);
+    if (lane_id() == 0) ((E*)wgrad_)[s] = Elem<DT>::from_f32(d);
+  }
+}
+
 template <typename T>
 __global__ void zero_kernel(T* __restrict__ p, int64_t n) {
   int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -879,6 +931,39 @@ int mbx_binned_scatter_wgrad(const void* x, const void* grad, int dtype, int64_t
 #define CALL(DT, V) binned_wgrad_kernel<DT, V><<<row_grid(total), kRowThreads, 0, s>>>(x, grad, tokens, hidden, top_k, indices, bins, num_bins, capacity, wgrad)
     MBX_DISPATCH_DT_VEC(dtype, vec, CALL)
 #undef CALL
+  }
+  return launch_status();
+}
+
+int mbx_binned_scatter_backward(const void* x, const void* grad, int dtype, int64_t tokens, int hidden, int top_k,
+                                const int32_t* indices, const int32_t* bins, int num_bins, int capacity, const void* weights,
+                                int w_dtype, void* dx, void* wgrad, mbx_stream_t stream) {
+  if (tokens < 0 || hidden < 0 || top_k <= 0 || num_bins < 0 || capacity < 0 || bad_dtype(dtype)) return MBX_EINVAL;
+  if (weights && bad_dtype(w_dtype)) return MBX_EINVAL;
+  const int64_t n_slots = tokens * top_k;
+  const int64_t total = (int64_t)num_bins * capacity;
+  if (n_slots > 0x7fffffff || total > 0x7fffffff) return MBX_ERANGE;
+  if ((tokens > 0 && (!wgrad || !indices)) || (num_bins > 0 && !bins) || (total > 0 && hidden > 0 && (!x || !dx || (tokens > 0 && !grad)))) return MBX_EINVAL;
+  hipStream_t s = as_stream(stream);
+  if (tokens > 0) {   // slots that were dropped
+    const unsigned fb = (unsigned)(ceil_div(n_slots, 256) < 2048 ? ceil_div(n_slots, 256) : 2048);
+    if (dtype_bytes(dtype) == 2) zero_kernel<uint16_t><<<fb, 256, 0, s>>>((uint16_t*)wgrad, n_slots);
+    else zero_kernel<uint32_t><<<fb, 256, 0, s>>>((uint32_t*)wgrad, n_slots);
+  }
+  if (total > 0 && hidden > 0) {
+    if (can_vec(dtype, hidden, x, grad ? grad : x, dx)) {
+#define CALL(DT, V) binned_scatter_backward_kernel<DT><<<row_grid(total), kRowThreads, 0, s>>>(x, grad, tokens, hidden, top_k, indices, bins, num_bins, capacity, weights, w_dtype, dx, wgrad)
+      MBX_DISPATCH_DT_VEC(dtype, true, CALL)
+#undef CALL
+    } else {   // each with the wide loads its own operands allow
+      const bool vec = can_vec(dtype, hidden, grad ? grad : dx, dx), vec_dot = can_vec(dtype, hidden, x, grad ? grad : x);
+#define CALL(DT, V) binned_gather_kernel<DT, V><<<row_grid(total), kRowThreads, 0, s>>>(grad, tokens, hidden, top_k, indices, bins, num_bins, capacity, weights, w_dtype, dx)
+      MBX_DISPATCH_DT_VEC(dtype, vec, CALL)
+#undef CALL
+#define CALL(DT, V) binned_wgrad_kernel<DT, V><<<row_grid(total), kRowThreads, 0, s>>>(x, grad, tokens, hidden, top_k, indices, bins, num_bins, capacity, wgrad)
+      MBX_DISPATCH_DT_VEC(dtype, vec_dot, CALL)
+#undef CALL
+    }
   }
   return launch_status();
 }

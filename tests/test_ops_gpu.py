@@ -237,6 +237,31 @@ def test_binned_ops(kernels, sl, hs, ne, top_k, cap_factor, dtype):
     assert rel_err(wg, oracle.binned_scatter_wgrad(want, grad, indices, bins, top_k)) < 1e-2
 
 
+@pytest.mark.parametrize('sl,hs,ne,top_k,cap', [(1, 8, 1, 1, 1), (77, 520, 3, 2, 5), (300, 2056, 8, 1, 60), (513, 129, 64, 4, 20), (2000, 768, 32, 1, 62)])
+@pytest.mark.parametrize('dtype,w_dtype', [(torch.bfloat16, torch.bfloat16), (torch.float16, torch.float32), (torch.float32, torch.float32), (torch.float16, None)])
+def test_both_gradients_of_binned_scatter_in_one_pass(kernels, sl, hs, ne, top_k, cap, dtype, w_dtype):
+    """What binned_gather (bit for bit) and binned_scatter_wgrad give, on aligned and unaligned rows, int64 assignments, experts with dropped
+    assignments and with empty places; a gradient of another type takes the two calls, and wrong sizes are refused."""
+    indices, bin_ids, bins, pbins = _routing(sl, ne, top_k, seed=sl)
+    indices, bins = dev(indices), dev(bins)
+    w = None if w_dtype is None else torch.rand(sl * top_k, device='cuda').to(w_dtype)
+    flat = torch.randn(ne * cap * hs + 1, device='cuda').to(dtype)
+    grad = torch.randn(sl, hs, device='cuda').to(dtype)
+    for x in (flat[:-1].view(ne, cap, hs), flat[1:].view(ne, cap, hs)):
+        for g, idx in ((grad, indices), (grad.float(), indices.long())):
+            dx, dw = kernels.binned_scatter_backward(x, g, idx, w, bins, top_k)
+            assert torch.equal(dx, kernels.binned_gather(g, idx, w, bins, cap, top_k))
+            # the same order; whether a product is rounded before it is added is the compiler's: 2^-24 of every product (their sizes
+            # average 0.64), and one step of the type where that crosses a rounding
+            want = kernels.binned_scatter_wgrad(x, g, idx, bins, top_k).float()
+            step = {torch.bfloat16: 2.0 ** -7, torch.float16: 2.0 ** -10, torch.float32: 0.0}[dtype]
+            assert dw.dtype == dtype and torch.allclose(dw.float(), want, rtol=step, atol=hs * 2.0 ** -23)
+    with pytest.raises(ValueError):
+        kernels.binned_scatter_backward(x, grad[1:], indices, w, bins, top_k)
+    with pytest.raises(ValueError):
+        kernels.binned_scatter_backward(x, grad[:, 1:], indices, w, bins, top_k)
+
+
 def test_shape_errors_are_value_errors(kernels):
     x = torch.randn(4, 8).cuda()
     idx = torch.zeros(4, dtype=torch.int32).cuda()
