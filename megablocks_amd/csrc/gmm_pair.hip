@@ -234,6 +234,10 @@ int dispatch(const DmaCall& q) {
 // geometric mean, one in twenty 3 - 12 % longer.  gmm_dma.h's kernel / this one: NT 4 experts of 500, [1408, 2048]: 42 / 23; 8 of 300, [4096,
 // 2048]: 66 / 58; 64 of 48, [4096, 2048]: 247 / 189; 12 of 500, [2728, 1032]: 62 / 65; 16 of 500, [4096, 2048]: 136 / 151.  NN 8 of 500, [1408, 512]: 32 /
 // 16; 16 of 300, [1408, 2048]: 56 / 41; 8 of 300, [4096, 1024], cut: 49 / 41; 4 of 100: 30 / 40; 32 of 500, [3072, 768]: 79 / 110.
+// Under the epilogues (111 launches each of 100 - 700 rows per expert, [512 - 2048, 1408 - 4096]) the choice is as good: 6 % (activation), 7 % (its
+// gradient, the gate's gradient, the activation alone) shorter than gmm_dma.h's, 1.5 % of the best of both at most; except with the gate on up
+// to 144 rows, whose half-height tiles are quicker than estimated (16 experts of 100, [4096, 1024]: 58 / 66; 64 of 100, [2816, 1024]: 159 / 173): there
+// only what is shorter by a fifth (nine of 111 launches 4 - 15 % longer before, two 5 % now).
 bool gmm_pair_takes(const DmaCall& q) {
   if (q.layout == MBX_TN || (q.gather.slots && q.k % pair::T::BK)) return false;
   const bool nn = q.layout == MBX_NN, dual = q.a2 && !dma::epi_is_dglu(q.epi), glu = dma::epi_is_glu(q.epi);
@@ -257,7 +261,7 @@ bool gmm_pair_takes(const DmaCall& q) {
     there += cut ? tile / parts + 21 : 2 * left <= units && full > 0 && !half ? 0.75 * tile : tile;
   }
   there = fmax(there, (nn ? 1.3 : 0.5) + mb / (nn ? 5.4 : 4.6));
-  return here < 0.94 * there;
+  return here < (glu && average <= 144 ? 0.8 : 0.94) * there;
 }
 
 int gmm_pair(const DmaCall& q) { return q.dtype == MBX_BF16 ? pair::dispatch<MBX_BF16>(q) : pair::dispatch<MBX_F16>(q); }
