@@ -400,8 +400,8 @@ __device__ __forceinline__ bool any_small(const Args& g, const __amdgpu_buffer_r
 //   * a sum comes out zero and the tile has such a value, whose parts may all have been zero.  Zero sums are common (rows that
 //     pad an expert), so the values are looked at before the tile is repeated.
 // Of the sums only those that are stored count: rows below m_lim, columns below n_lim.  A launch that is formed twice throughout
-// (operands of 2^-60 and less next to others of order one, or of 2^40) takes 920 / 911 / 838 us NT / NN / TN for 8 experts of 1024
-// rows, [1024, 4096], instead of 403 / 406 / 371; the element-wise kernel takes 840 / 878 / 780 for any values.
+// (operands of 2^-60 and less next to others of order one, or of 2^40) takes 824 / 810 / 836 us NT / NN / TN for 8 experts of 1024
+// rows, [1024, 4096], instead of 340 / 324 / 338; the element-wise kernel takes 840 / 878 / 780 for any values.
 constexpr float kTiny = 0x1p-64f, kHuge = 0x1p38f;
 
 template <bool A_MC, bool B_MC, typename S, bool DUAL>
