@@ -596,7 +596,7 @@ def experts_forward(x, expert_ids, expert_weights, num_experts, end_bit, top_k, 
     32 experts 147 -> 90; the GPU's time: 4096 assignments, 8 experts of [1024, 2816], 84.)"""
     tensors = (x, expert_ids, expert_weights, w1, w2) if v1 is None else (x, expert_ids, expert_weights, w1, v1, w2)
     slots, dtype, device = expert_ids.numel(), x.dtype, x.device
-    if not 0 < slots <= EXPERTS_FORWARD_MAX_SLOTS or dtype not in (torch.bfloat16, torch.float16) or not x.is_cuda or \
+    if not 0 < slots <= EXPERTS_FORWARD_MAX_SLOTS or end_bit > 8 or dtype not in (torch.bfloat16, torch.float16) or not x.is_cuda or \
             x.shape[1] == 0 or FUSED_GATHER == '0' or _lib.profile_hook is not None:
         return None
     for t in tensors:
