@@ -1,5 +1,5 @@
 """Learned top-k router: megablocks/layers/router.py:10-114.  The linear layer is torch's (a small dense
-GEMM), except for its weight gradient on large 16-bit batches, which goes through the grouped TN kernel;
+GEMM), except for its gradients on large 16-bit batches, which go through the grouped kernels;
 softmax, top-k and the renormalisation of the selected weights are one HIP kernel each way.  The outputs
 feed the HIP routing kernels."""
 from typing import Any
