@@ -344,6 +344,42 @@ def test_router_chooses_alike_with_and_without_gradients(tokens, dtype, training
     assert rel_err(x.grad, x32.grad) < tol and rel_err(router.layer.weight.grad, w32.grad) < tol
 
 
+def test_router_backward_of_a_few_tokens_is_captured_at_a_new_token_count():
+    """Up to 256 tokens a forward and backward of the router can be captured at a token count that never ran eagerly, and every
+    replay gives the eager step's bits."""
+    from megablocks_amd.layers.router import LearnedRouter
+    router = LearnedRouter(_args(hidden_size=512, ffn_hidden_size=512, moe_num_experts=16, moe_top_k=2))
+    params = [router.layer.weight]
+
+    def step(x, gs, gw):
+        scores, weights, _ = router(x)
+        return torch.autograd.grad([scores, weights], [x, *params], [gs, gw])
+
+    def inputs(tokens):
+        return [t.bfloat16() for t in (torch.randn(tokens, 512, device='cuda'), torch.randn(tokens, 16, device='cuda'),
+                                       torch.randn(tokens, 2, device='cuda'))]
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        x, gs, gw = inputs(40)
+        step(x.requires_grad_(True), gs, gw)
+    torch.cuda.current_stream().wait_stream(side)
+    held = inputs(41)
+    held[0].requires_grad_(True)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = step(*held)
+    for _ in range(4):
+        fresh = inputs(41)
+        with torch.no_grad():
+            for h, f in zip(held, fresh):
+                h.copy_(f)
+        graph.replay()
+        torch.cuda.synchronize()
+        want = step(fresh[0].requires_grad_(True), *fresh[1:])
+        assert all(torch.equal(a, b) for a, b in zip(out, want))
+
+
 @pytest.mark.parametrize('tokens', [16, 200])
 def test_dmoe_under_reentrant_checkpointing_gives_the_plain_steps_gradients(tokens):
     """Re-entrant activation checkpointing runs the forward without gradients and once more with them: every gradient and the
