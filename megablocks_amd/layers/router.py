@@ -62,19 +62,32 @@ class _RouterLinear(torch.autograd.Function):
 
     PIECE_ROWS = 256   # tokens per piece (four K tiles of the TN kernel)
     MAX_PIECES = 64
+    MAX_KEPT = 4096    # batch sizes; a captured graph may hold the bins of any of them, so none is given up for another
 
     _sizes = {}
 
     @staticmethod
-    def piece_sizes(tokens: int, max_pieces: int = MAX_PIECES) -> torch.Tensor:
-        """Rows per piece (kept per batch size: the grouped GEMM caches the device-side bins on this tensor)."""
-        sizes = _RouterLinear._sizes.get((tokens, max_pieces))
+    def piece_sizes(tokens: int) -> torch.Tensor:
+        """Rows per piece (kept for the first MAX_KEPT batch sizes: the grouped GEMM caches the device-side bins on this tensor)."""
+        sizes = _RouterLinear._sizes.get(tokens)
         if sizes is None:
-            pieces = max(1, min(max_pieces, tokens // _RouterLinear.PIECE_ROWS))
+            pieces = max(1, min(_RouterLinear.MAX_PIECES, tokens // _RouterLinear.PIECE_ROWS))
             sizes = torch.full((pieces,), tokens // pieces, dtype=torch.int64)
             sizes[:tokens % pieces] += 1
-            _RouterLinear._sizes[tokens, max_pieces] = sizes
+            if len(_RouterLinear._sizes) < _RouterLinear.MAX_KEPT:
+                _RouterLinear._sizes[tokens] = sizes
         return sizes
+
+    @staticmethod
+    def whole_batch(sizes: torch.Tensor, tokens: int, device) -> torch.Tensor:
+        """The pieces as one group, whose bin on the device is the last of theirs: a batch size met for the first time is
+        copied there once (a copy waits for the queue to drain)."""
+        whole = getattr(sizes, '_mbx_whole', None)
+        if whole is None:
+            from megablocks_amd import grouped_gemm_util as gg
+            whole = sizes._mbx_whole = torch.tensor([tokens])
+            gg._remember(whole, (gg._device_bins(sizes, device, tokens)[-1:], whole._version, tokens))
+        return whole
 
     @staticmethod
     @torch.amp.custom_fwd(device_type='cuda')
@@ -101,12 +114,12 @@ def _linear_gradients(grad, x, weight, weight_dtype, want_x, want_weight):
     tokens, experts = grad.shape
     grad = grad.contiguous()
     dx = dw = None
+    sizes = _RouterLinear.piece_sizes(tokens) if want_weight else None
     if want_x:
-        # the kernels read whole 16-byte pieces of rows
-        dx = grad @ weight if experts % 8 or tokens == 0 else gg.gmm(
-            grad, weight.unsqueeze(0), _RouterLinear.piece_sizes(tokens, 1), _record_as='router_dgrad')
+        # the kernels read whole 16-byte pieces of rows; the input's gradient alone is not worth the copy of a bin
+        dx = grad @ weight if sizes is None or experts % 8 or tokens == 0 else gg.gmm(
+            grad, weight.unsqueeze(0), _RouterLinear.whole_batch(sizes, tokens, x.device), _record_as='router_dgrad')
     if want_weight:
-        sizes = _RouterLinear.piece_sizes(tokens)
         pieces = sizes.shape[0]
         if experts % 8:
             grad = torch.nn.functional.pad(grad, (0, -experts % 8))

@@ -16,6 +16,33 @@ def no_grouped_products(monkeypatch):
     monkeypatch.setattr(gg, 'weight_gradient', refuse)
 
 
+@pytest.fixture
+def launched(monkeypatch):
+    """The grouped products as plain ones: (layout, bins as they reach the kernel) of each."""
+    calls = []
+
+    def gmm(a, b, batch_sizes, trans_a=False, _record_as=None, **_):
+        bins = gg._device_bins(batch_sizes, a.device, a.shape[0])
+        calls.append(('tn' if trans_a else 'nn', bins.tolist()))
+        if not trans_a:
+            return (a.float() @ b[0].float()).to(a.dtype)
+        cuts = bins[:-1].long()
+        return torch.stack([(p.float().t() @ q.float()).to(a.dtype) for p, q in zip(a.tensor_split(cuts), b.tensor_split(cuts))])
+    monkeypatch.setattr(gg, 'gmm', gmm)
+    monkeypatch.setattr(gg, 'weight_gradient', lambda a, b, sizes, weight_dtype=None, **_: gmm(a, b, sizes, trans_a=True))
+    monkeypatch.setattr(r._RouterLinear, '_sizes', {})
+    return calls
+
+
+@pytest.fixture
+def copies(monkeypatch):
+    """The batch sizes whose bins are copied to the device (`_device_bins` finds none kept)."""
+    made = []
+    cumsum = torch.cumsum
+    monkeypatch.setattr(torch, 'cumsum', lambda t, *a, **k: made.append(t.tolist()) or cumsum(t, *a, **k))
+    return made
+
+
 def _operands(tokens, hidden, experts, dtype=torch.bfloat16):
     torch.manual_seed(tokens)
     return [torch.randn(*s).to(dtype) for s in ((tokens, hidden), (experts, hidden), (tokens, experts))]
@@ -34,3 +61,25 @@ def test_gradients_of_a_few_tokens_are_the_two_plain_products(monkeypatch, no_gr
     assert rest == [None, None] and (dx is not None, dw is not None) == want
     assert dx is None or torch.equal(dx, grad @ weight)
     assert dw is None or torch.equal(dw, grad.t() @ x)
+
+
+def test_a_batch_size_is_copied_to_the_device_once(launched, copies):
+    """One copy for both gradients at the first batch of a size, none for later ones, and none at all where only the input's
+    gradient is wanted."""
+    x, weight, grad = _operands(1100, 16, 8)
+    dx, _ = r._linear_gradients(grad, x, weight, weight.dtype, True, False)
+    assert not copies and torch.equal(dx, grad @ weight)
+    for _ in range(2):
+        r._linear_gradients(grad, x, weight, weight.dtype, True, True)
+    assert copies == [[275] * 4]
+    assert launched == 2 * [('nn', [1100]), ('tn', [275, 550, 825, 1100])]
+
+
+def test_batch_sizes_are_kept_up_to_a_bound(monkeypatch, launched, copies):
+    """Sizes past the bound are worked out anew each time; those kept stay, as graphs may hold them."""
+    monkeypatch.setattr(r._RouterLinear, 'MAX_KEPT', 2, raising=False)
+    for tokens in (1024, 1100, 1200, 1300, 1024, 1200):
+        x, weight, grad = _operands(tokens, 16, 8)
+        r._linear_gradients(grad, x, weight, weight.dtype, True, True)
+    assert len(r._RouterLinear._sizes) == 2
+    assert [sum(c) for c in copies] == [1024, 1100, 1200, 1300, 1200]
