@@ -108,6 +108,10 @@ class _RouterLinear(torch.autograd.Function):
         return _linear_gradients(grad.to(x.dtype), x, weight, ctx.weight_dtype, *ctx.needs_input_grad[:2])
 
 
+def _whole_pieces(t: torch.Tensor) -> bool:
+    return t.shape[1] % 8 == 0 and t.is_contiguous() and t.data_ptr() % 16 == 0
+
+
 def _linear_gradients(grad, x, weight, weight_dtype, want_x, want_weight):
     """(dx, dweight) of `x @ weight^T`, all 16-bit of one type on the GPU; dweight in `weight_dtype`."""
     from megablocks_amd import grouped_gemm_util as gg
@@ -116,9 +120,10 @@ def _linear_gradients(grad, x, weight, weight_dtype, want_x, want_weight):
     dx = dw = None
     sizes = _RouterLinear.piece_sizes(tokens) if want_weight else None
     if want_x:
-        # the kernels read whole 16-byte pieces of rows; the input's gradient alone is not worth the copy of a bin
-        dx = grad @ weight if sizes is None or experts % 8 or tokens == 0 else gg.gmm(
-            grad, weight.unsqueeze(0), _RouterLinear.whole_batch(sizes, tokens, x.device), _record_as='router_dgrad')
+        # the grouped kernels for whole 16-byte pieces of rows; the input's gradient alone is not worth the copy of a bin
+        grouped = sizes is not None and tokens > 0 and _whole_pieces(grad) and _whole_pieces(weight)
+        dx = gg.gmm(grad, weight.unsqueeze(0), _RouterLinear.whole_batch(sizes, tokens, x.device), _record_as='router_dgrad') \
+            if grouped else grad @ weight
     if want_weight:
         pieces = sizes.shape[0]
         if experts % 8:

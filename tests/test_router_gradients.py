@@ -83,3 +83,19 @@ def test_batch_sizes_are_kept_up_to_a_bound(monkeypatch, launched, copies):
         r._linear_gradients(grad, x, weight, weight.dtype, True, True)
     assert len(r._RouterLinear._sizes) == 2
     assert [sum(c) for c in copies] == [1024, 1100, 1200, 1300, 1200]
+
+
+@pytest.mark.parametrize('form', ['hidden', 'experts', 'weight_offset', 'weight_strided', 'grad_offset'])
+def test_rows_that_are_no_whole_pieces_leave_the_input_gradient_to_the_plain_product(launched, form):
+    """The grouped product serves whole aligned 16-byte pieces of rows; others it would give to the element-wise kernel."""
+    tokens, hidden, experts = 1100, 70 if form == 'hidden' else 72, 12 if form == 'experts' else 16
+    x, weight, grad = _operands(tokens, hidden, experts)
+    if form == 'weight_offset':
+        weight = torch.cat([weight.new_zeros(1), weight.flatten()])[1:].view(experts, hidden)
+    elif form == 'weight_strided':
+        weight = weight.t().contiguous().t()
+    elif form == 'grad_offset':
+        grad = torch.cat([grad.new_zeros(1), grad.flatten()])[1:].view(tokens, experts)
+    dx, dw = r._linear_gradients(grad, x, weight, weight.dtype, True, True)
+    assert torch.equal(dx, grad @ weight) and [c[0] for c in launched] == ['tn']
+    assert (dw.double() - grad.double().t() @ x.double()).norm() < 2.0 ** -7 * dw.double().norm()
