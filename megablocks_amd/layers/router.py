@@ -112,9 +112,20 @@ def _whole_pieces(t: torch.Tensor) -> bool:
     return t.shape[1] % 8 == 0 and t.is_contiguous() and t.data_ptr() % 16 == 0
 
 
+def _has_memory(t: torch.Tensor) -> bool:
+    try:
+        t.data_ptr()
+    except RuntimeError:
+        return False
+    return True
+
+
 def _linear_gradients(grad, x, weight, weight_dtype, want_x, want_weight):
     """(dx, dweight) of `x @ weight^T`, all 16-bit of one type on the GPU; dweight in `weight_dtype`."""
     from megablocks_amd import grouped_gemm_util as gg
+    if torch.is_grad_enabled() or not _has_memory(grad):
+        # a backward that is differentiated itself (create_graph), or runs over a batch of gradients at once (is_grads_batched)
+        return grad @ weight if want_x else None, (grad.t() @ x).to(weight_dtype) if want_weight else None
     tokens, experts = grad.shape
     grad = grad.contiguous()
     dx = dw = None

@@ -25,9 +25,9 @@ def launched(monkeypatch):
         bins = gg._device_bins(batch_sizes, a.device, a.shape[0])
         calls.append(('tn' if trans_a else 'nn', bins.tolist()))
         if not trans_a:
-            return (a.float() @ b[0].float()).to(a.dtype)
+            return (a.double() @ b[0].double()).to(a.dtype)
         cuts = bins[:-1].long()
-        return torch.stack([(p.float().t() @ q.float()).to(a.dtype) for p, q in zip(a.tensor_split(cuts), b.tensor_split(cuts))])
+        return torch.stack([(p.double().t() @ q.double()).to(a.dtype) for p, q in zip(a.tensor_split(cuts), b.tensor_split(cuts))])
     monkeypatch.setattr(gg, 'gmm', gmm)
     monkeypatch.setattr(gg, 'weight_gradient', lambda a, b, sizes, weight_dtype=None, **_: gmm(a, b, sizes, trans_a=True))
     monkeypatch.setattr(r._RouterLinear, '_sizes', {})
@@ -63,6 +63,7 @@ def test_gradients_of_a_few_tokens_are_the_two_plain_products(monkeypatch, no_gr
     assert dw is None or torch.equal(dw, grad.t() @ x)
 
 
+@torch.no_grad()   # as a backward runs
 def test_a_batch_size_is_copied_to_the_device_once(launched, copies):
     """One copy for both gradients at the first batch of a size, none for later ones, and none at all where only the input's
     gradient is wanted."""
@@ -75,6 +76,7 @@ def test_a_batch_size_is_copied_to_the_device_once(launched, copies):
     assert launched == 2 * [('nn', [1100]), ('tn', [275, 550, 825, 1100])]
 
 
+@torch.no_grad()
 def test_batch_sizes_are_kept_up_to_a_bound(monkeypatch, launched, copies):
     """Sizes past the bound are worked out anew each time; those kept stay, as graphs may hold them."""
     monkeypatch.setattr(r._RouterLinear, 'MAX_KEPT', 2, raising=False)
@@ -86,6 +88,7 @@ def test_batch_sizes_are_kept_up_to_a_bound(monkeypatch, launched, copies):
 
 
 @pytest.mark.parametrize('form', ['hidden', 'experts', 'weight_offset', 'weight_strided', 'grad_offset'])
+@torch.no_grad()
 def test_rows_that_are_no_whole_pieces_leave_the_input_gradient_to_the_plain_product(launched, form):
     """The grouped product serves whole aligned 16-byte pieces of rows; others it would give to the element-wise kernel."""
     tokens, hidden, experts = 1100, 70 if form == 'hidden' else 72, 12 if form == 'experts' else 16
@@ -99,3 +102,30 @@ def test_rows_that_are_no_whole_pieces_leave_the_input_gradient_to_the_plain_pro
     dx, dw = r._linear_gradients(grad, x, weight, weight.dtype, True, True)
     assert torch.equal(dx, grad @ weight) and [c[0] for c in launched] == ['tn']
     assert (dw.double() - grad.double().t() @ x.double()).norm() < 2.0 ** -7 * dw.double().norm()
+
+
+def _linear(x, weight):
+    return r._RouterLinear.apply(x, weight)
+
+
+def test_gradients_of_the_linear_layer_can_be_differentiated(launched):
+    """Under create_graph the backward is made of products autograd knows: second derivatives are those of torch's own linear."""
+    x, weight, grad = (t.requires_grad_(True) for t in _operands(1100, 16, 8, torch.float64))
+
+    def second(linear):
+        launched.clear()
+        dx, dw = torch.autograd.grad(linear(x, weight).tanh(), [x, weight], grad, create_graph=True)
+        assert not launched
+        return torch.autograd.grad([dx.square().sum(), dw.square().sum()], [x, weight, grad])
+    for got, want in zip(second(_linear), second(torch.nn.functional.linear)):
+        torch.testing.assert_close(got, want)
+
+
+def test_gradients_of_the_linear_layer_over_a_batch_of_gradients(no_grouped_products):
+    """is_grads_batched hands the backward a tensor without memory of its own."""
+    x, weight, _ = (t.requires_grad_(True) for t in _operands(1100, 16, 8, torch.float64))
+    grads = torch.randn(3, 1100, 8, dtype=torch.float64)
+    for wanted in ([x], [weight], [x, weight]):
+        for got, want in zip(*(torch.autograd.grad(linear(x, weight), wanted, grads, is_grads_batched=True)
+                               for linear in (_linear, torch.nn.functional.linear))):
+            torch.testing.assert_close(got, want)
