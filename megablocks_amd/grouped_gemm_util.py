@@ -448,25 +448,25 @@ def _wants_fp32(a, weight_dtype):
     return weight_dtype == torch.float32 and a.is_cuda and a.dtype in (torch.bfloat16, torch.float16)
 
 
-def weight_gradient(a, b, batch_sizes, weight_dtype=None):
+def weight_gradient(a, b, batch_sizes, weight_dtype=None, _record_as=None):
     """gmm(a, b, batch_sizes, trans_a=True), the gradient of a weight of type `weight_dtype` (None: of a's): where 16-bit
     operands meet an fp32 weight (autocast) the product's fp32 sums are stored as they are, in one launch, instead of
     being rounded, stored, read and cast back (64 experts of 256 rows, [1024, 4096]: 352 us, the 16-bit product and the cast
-    514; 8 of 2048 rows, [2048, 8192]: 504, 546).  May come back in a's type: autograd then casts it."""
+    514; 8 of 2048 rows, [2048, 8192]: 504, 546).  May come back in a's type: autograd then casts it.  _record_as: as for `gmm`."""
     if not _wants_fp32(a, weight_dtype) or a.ndim != 2 or b.ndim != 2 or b.dtype != a.dtype or b.shape[0] != a.shape[0]:
-        return gmm(a, b, batch_sizes, trans_a=True)
+        return gmm(a, b, batch_sizes, trans_a=True, _record_as=_record_as)
     a, b = a.contiguous(), b.contiguous()
     rows, k, n = a.shape[0], a.shape[1], b.shape[1]
     bins = _device_bins(batch_sizes, a.device, rows)
     groups = bins.shape[0]
     c = torch.empty((groups, k, n), dtype=torch.float32, device=a.device)
-    with _lib.device_of(a), _lib.record('gmm_tn', rows=rows, k=k, n=n, elem=a.element_size(), groups=groups) as rec:
+    with _lib.device_of(a), _lib.record(_record_as or 'gmm_tn', rows=rows, k=k, n=n, elem=a.element_size(), groups=groups) as rec:
         rc = lib.mbx_gmm_tn_f32(_lib.ptr(a), _lib.ptr(b), 0, None, 1, None, _lib.ptr(c), _lib.dtype_of(a), _lib.ptr(bins), groups, rows,
                                 k, n, None, 0, 0, _lib.stream())
         if rc == _lib.EUNSUPPORTED:
             rec.cancel()
     if rc == _lib.EUNSUPPORTED:
-        return gmm(a, b, batch_sizes, trans_a=True)
+        return gmm(a, b, batch_sizes, trans_a=True, _record_as=_record_as)
     _lib.check(rc, 'gmm_tn_f32')
     return c
 

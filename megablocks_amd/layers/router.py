@@ -140,7 +140,7 @@ def _linear_gradients(grad, x, weight, weight_dtype, want_x, want_weight):
         if experts % 8:
             grad = torch.nn.functional.pad(grad, (0, -experts % 8))
         # [pieces, E, h]; a single piece's sums are rounded by the product itself
-        parts = gg.weight_gradient(grad, x.contiguous(), sizes, torch.float32 if pieces > 1 else None)
+        parts = gg.weight_gradient(grad, x.contiguous(), sizes, torch.float32 if pieces > 1 else None, _record_as='router_wgrad')
         if pieces == 1 or parts.dtype != torch.float32:
             dw = (parts[0] if pieces == 1 else parts.sum(0, dtype=torch.float32))[:experts].to(weight_dtype)
         else:

@@ -264,6 +264,20 @@ def test_router_linear_gradients_against_fp64(tokens, hidden, experts, dtype, we
     assert rel_err(weight.grad.double(), g.double().t() @ x.detach().double()) < (sums if exact else rounding)
 
 
+@pytest.mark.parametrize('tokens,hidden', [(4096, 256), (1100, 70)])
+def test_router_products_keep_out_of_the_experts_statistics(monkeypatch, tokens, hidden):
+    """Per-launch timing (bench.py) sums up launches by name: those of the router's gradients have names of their own."""
+    from megablocks_amd import _lib
+    from megablocks_amd.layers.router import _RouterLinear
+    x = torch.randn(tokens, hidden, device='cuda').bfloat16().requires_grad_(True)
+    weight = torch.randn(8, hidden, device='cuda').bfloat16().requires_grad_(True)
+    logits = _RouterLinear.apply(x, weight)
+    monkeypatch.setattr(_lib, 'profile_hook', [])
+    logits.backward(torch.randn_like(logits))
+    names = [entry[0] for entry in _lib.profile_hook]
+    assert 'router_wgrad' in names and set(names) <= {'router_wgrad', 'router_dgrad'}
+
+
 def _softmax_topk_reference(logits, top_k, norm_p):
     """router.py:87-106 with torch's own operations."""
     scores = logits.softmax(dim=-1)
