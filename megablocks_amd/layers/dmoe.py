@@ -16,8 +16,13 @@ from megablocks_amd.layers.glu import GroupedGLU, _activation_code
 from megablocks_amd.layers.mlp import DEFAULT_ACTIVATION_FN, GroupedMLP, Topology
 
 
-# whether a torch.func transform is under way
-_transforms_active = getattr(torch._C, '_are_functorch_transforms_active', lambda: False)
+def _only_computed() -> bool:
+    """Whether operations are carried out as they are called and nothing else: not traced, compiled, transformed (torch.func),
+    differentiated forward or cast (autocast), all of which act on torch's operators and see nothing of a raw launch.  A torch
+    that does not say counts as one that is doing it."""
+    return not (torch.is_autocast_enabled() or torch.compiler.is_compiling() or torch.jit.is_tracing() or
+                getattr(torch._C, '_are_functorch_transforms_active', lambda: True)() or
+                getattr(torch.autograd.forward_ad, '_current_level', 0) >= 0)   # -1: outside of any dual level
 
 
 def promote_scalar(x):
@@ -171,8 +176,7 @@ class ParallelDroplessMLP(moe.ParallelMLP):
         else:
             return None
         if act is None or experts.gradient_scale is not None or mpu.experts_per_rank(self.args) != self.num_experts or \
-                torch.is_autocast_enabled() or torch.compiler.is_compiling() or _transforms_active() or \
-                torch.autograd.forward_ad._current_level >= 0 or torch._C._get_tracing_state() is not None:
+                not _only_computed():
             return None
         return gg.experts_forward(x.view(-1, x.shape[-1]), top_experts.int(), expert_weights, self.num_experts, self.sort_end_bit,
                                   self.args.moe_top_k, experts.w1, v1, experts.w2, act)
