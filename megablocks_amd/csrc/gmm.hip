@@ -556,11 +556,19 @@ int launch_tn(const DmaCall& call) {
 
 // The direct-to-LDS kernels for 16-bit operands: the row tiles of NN / NT by whether the reduction is whole K tiles, TN
 // here (the half-height tile only when the product has at most 128 rows: it is slower otherwise).
+// mbx_debug_row_kernel's choice for the NN / NT launches of this thread: kByRule, or one kernel for all of them.
+enum RowKernel { kByRule, kGeneral, kPair };
+static thread_local int row_kernel = kByRule;
+
 static int gmm_dma(const DmaCall& call) {
 #ifdef MBX_TICKS
   constexpr bool kFewRows = false;   // the kernels for few rows per expert have no stamps
 #else
   constexpr bool kFewRows = true;
+  if (call.layout != MBX_TN && row_kernel != kByRule) {
+    if (row_kernel == kPair) return gmm_pair_can(call) ? gmm_pair(call) : MBX_EUNSUPPORTED;
+    return call.k % dma::TileMain::BK == 0 ? gmm_rows(call) : gmm_rows_tail(call);
+  }
 #endif
   if (kFewRows && gmm_few_takes(call)) return gmm_few(call);
   if (kFewRows && gmm_mid_takes(call)) return gmm_mid(call);
@@ -606,6 +614,16 @@ static inline bool dma_sizes_ok(int k, int n) {
 using namespace mbx;
 
 extern "C" {
+
+#ifndef MBX_TICKS
+// For tests and measurements: which kernel takes the 16-bit NN / NT launches of the calling thread from now on -- 0 what the rules say,
+// 1 gmm_dma.h's, 2 gmm_pair.hip's (MBX_EUNSUPPORTED where it cannot).  Returns what it was.
+int mbx_debug_row_kernel(int kernel) {
+  const int before = row_kernel;
+  row_kernel = kernel == kGeneral || kernel == kPair ? kernel : kByRule;
+  return before;
+}
+#endif
 
 #ifdef MBX_TICKS
 // libmbx_ticks.so only: where the kernels of gmm_dma.h put their per-tile time stamps (see there); NULL: nowhere.

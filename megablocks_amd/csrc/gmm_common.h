@@ -70,7 +70,8 @@ int gmm_mid(const DmaCall& call);
 // us.  8 experts of 48 rows, [4096, 1024]: 61 -> 36 us; 4 of 500, [2816, 1024]: 58 -> 45; 8 of 256, [1408, 512]: 18 -> 21.
 constexpr int kMinCutTiles = 32;
 
-// NN / NT launches of few tiles (gmm_pair.hip), and whether a launch is one of them.
+// NN / NT launches of few tiles (gmm_pair.hip): whether a launch could run there, and whether it is one of them.
+bool gmm_pair_can(const DmaCall& call);
 bool gmm_pair_takes(const DmaCall& call);
 int gmm_pair(const DmaCall& call);
 

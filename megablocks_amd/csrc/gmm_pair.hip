@@ -227,6 +227,9 @@ int dispatch(const DmaCall& q) {
 }  // namespace pair
 }  // namespace
 
+// Gathered rows: whole K tiles.
+bool gmm_pair_can(const DmaCall& q) { return q.layout != MBX_TN && !(q.gather.slots && q.k % pair::T::BK); }
+
 // Whether the launch is estimated to be shorter here than with gmm_dma.h's tiles, by a sixteenth at least.  Both estimates are
 // rounds of tiles times K tiles times what one takes, us, fitted to 206 NT and 206 NN launches (4 - 64 experts of 48 - 800 rows,
 // [512 - 2048, 1408 - 4096], operands out of memory; rms 11 - 12 %), and no less than the operands at the rate the kernel reads them.
@@ -239,7 +242,7 @@ int dispatch(const DmaCall& q) {
 // to 144 rows, whose half-height tiles are quicker than estimated (16 experts of 100, [4096, 1024]: 58 / 66; 64 of 100, [2816, 1024]: 159 / 173): there
 // only what is shorter by a fifth (nine of 111 launches 4 - 15 % longer before, two 5 % now).
 bool gmm_pair_takes(const DmaCall& q) {
-  if (q.layout == MBX_TN || (q.gather.slots && q.k % pair::T::BK)) return false;
+  if (!gmm_pair_can(q)) return false;
   const bool nn = q.layout == MBX_NN, dual = q.a2 && !dma::epi_is_dglu(q.epi), glu = dma::epi_is_glu(q.epi);
   const double units = persistent_grid((int64_t)1 << 30), experts = q.num_groups, average = (double)q.rows / experts;
   const double nk = (dual ? 2.0 : 1.0) * (double)ceil_div(q.k, pair::T::BK), n = q.n * (glu ? 2.0 : 1.0);

@@ -1237,45 +1237,64 @@ def test_gmm_reductions_that_end_inside_a_k_tile(gg, monkeypatch, groups, rows, 
     assert torch.equal(torch.where(placed, out, 0), torch.where(placed, want, 0))
 
 
-@pytest.mark.parametrize('counts,k,n', [([100, 0, 129, 128, 1, 300], 128, 136), ([257, 255, 64], 200, 520), ([200], 64, 8), ([90] * 16, 448, 1032),
-                                           ([60, 500], 8, 264), ([61] * 70, 64, 72)])
+@pytest.fixture
+def row_kernel():
+    """Names the kernel that takes this thread's NN / NT products: 1 the general one, 2 that of launches of few tiles (an error
+    where it cannot)."""
+    from megablocks_amd._lib import lib
+    yield lib.mbx_debug_row_kernel
+    lib.mbx_debug_row_kernel(0)
+
+
+@pytest.mark.parametrize('counts,k,n', [
+    ([100, 0, 129, 128, 1, 300], 128, 136), ([257, 255, 64], 200, 520), ([200], 64, 8), ([90] * 16, 448, 1032), ([60, 500], 8, 264),
+    ([61] * 70, 64, 72),
+    ([1], 8, 8), ([127, 1, 0, 128], 72, 128), ([300, 290, 310], 2728, 1032), ([1, 2, 3], 576, 2048)])
 @pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])
-def test_products_of_few_tiles_are_the_general_kernels(gg, monkeypatch, counts, k, n, dtype):
-    """Launches of few tiles have a kernel of their own, every form of which gives the bits of the general one's: the same rows at
-    the head of operands of so many that the launch is taken for a large one, and against fp32."""
+def test_products_of_few_tiles_are_the_general_kernels(gg, monkeypatch, row_kernel, counts, k, n, dtype):
+    """Launches of few tiles have a kernel of their own, every form of which gives the bits of the general one's: each is run by
+    both, at reductions that end inside a K tile, rows and columns inside a tile, more experts than a wave has lanes and operands
+    with rows behind the last expert's; the plain products also against fp32."""
     torch.manual_seed(k + n)
     monkeypatch.setattr(gg, 'GMM_WORKSPACE', False)   # no cut along the reduction
     sizes = torch.tensor(counts, device='cuda')       # on the device: their sum need not be the row count
-    groups, rows, many = len(counts), sum(counts), 90000
-    a, a2, p1, p2, g = ((torch.randn(many, w, device='cuda')).to(dtype) for w in (k, k, n, n, k))
+    groups, rows = len(counts), sum(counts)
+    m = rows + 37
+    a, a2, p1, p2 = ((torch.randn(m, w, device='cuda')).to(dtype) for w in (k, k, n, n))
     wt, wt2 = ((torch.randn(groups, n, k, device='cuda') / k ** 0.5).to(dtype) for _ in range(2))
     w, w2 = (t.transpose(1, 2).contiguous() for t in (wt, wt2))
     order = torch.randperm(rows, device='cuda').int()
     bins = torch.cumsum(sizes, 0).int()
     bin_ids = torch.repeat_interleave(torch.arange(groups, device='cuda'), sizes).int()
-    weights = torch.rand(many, device='cuda').to(dtype)
+    weights = torch.rand(m, device='cuda').to(dtype)
     tokens = torch.randn(rows, k, device='cuda').to(dtype)
 
-    def forms(m):
-        x, x2, s1, s2 = a[:m], a2[:m], p1[:m], p2[:m]
+    def forms():
         src = gg.GatheredRows(tokens, order, bin_ids, bins, None, 1, m)
-        out = [gg.backend.gmm(x, wt, sizes, trans_b=True), gg.backend.gmm(x, w, sizes), gg.gmm_dact(x, wt, s1, sizes, fuse=True)]
+        out = [gg.backend.gmm(a, wt, sizes, trans_b=True), gg.backend.gmm(a, w, sizes), gg.gmm_dact(a, wt, p1, sizes, fuse=True)]
         if k > 192:
-            out += [gg.gmm_dual(x, wt, x2, wt2, sizes, trans_b=True), gg.gmm_dual(x, w, x2, w2, sizes)]
-        out += [*gg.gmm_act(x, wt, sizes, fuse=True), *gg.gmm_act(x, w, sizes, fuse=True, trans_b=False)]
+            out += [gg.gmm_dual(a, wt, a2, wt2, sizes, trans_b=True), gg.gmm_dual(a, w, a2, w2, sizes)]
+        out += [*gg.gmm_act(a, wt, sizes, fuse=True), *gg.gmm_act(a, w, sizes, fuse=True, trans_b=False)]
         for act in (0, 1):
-            out += [*gg.gmm_glu(x, wt, wt2, sizes, act, fuse=True), *gg.gmm_dglu(x, wt, s1, s2, sizes, act, fuse=True)]
+            out += [*gg.gmm_glu(a, wt, wt2, sizes, act, fuse=True), *gg.gmm_dglu(a, wt, p1, p2, sizes, act, fuse=True)]
         if k % 64 == 0:
-            out += [*gg.gmm_gather(src, wt, sizes), *gg.gmm_gather(src, wt, sizes, act=1), *gg.gmm_gather(src, wt, sizes, b2=wt2, act=0)]
-        combine = gg.CombinedRows(torch.cat([order, torch.zeros(m - rows, dtype=torch.int32, device='cuda')]), bin_ids, bins, weights[:m])
-        y, combined = gg.gmm_scatter(x, w, sizes, combine)
+            for act, second in ((None, None), (1, None), (0, wt2), (1, wt2)):
+                out += [*gg.gmm_gather(src, wt, sizes, act=act, b2=second)]
+                if act is not None:
+                    out += [gg.gmm_gather(src, wt, sizes, act=act, b2=second, keep_product=False)[-1]]
+        combine = gg.CombinedRows(torch.cat([order, torch.zeros(m - rows, dtype=torch.int32, device='cuda')]), bin_ids, bins, weights)
+        y, combined = gg.gmm_scatter(a, w, sizes, combine)
         return [t[:rows] for t in out + [y] if t is not None], combined[order.long()]
-    small, placed = forms(rows)
-    large, placed_large = forms(many)
-    assert len(small) == len(large) and all(torch.equal(s, t) for s, t in zip(small, large))
-    assert torch.equal(placed, placed_large)
-    want = _ref_gpu(a[:rows], wt, sizes.cpu(), False, True)
-    assert max_block_err(small[0], want) < TOL and max_block_err(small[1], want) < TOL
+    row_kernel(1)
+    general, placed = forms()
+    assert row_kernel(2) == 1
+    here, placed_here = forms()
+    assert row_kernel(0) == 2
+    assert len(here) == len(general) and all(torch.equal(s, t) for s, t in zip(here, general))
+    assert torch.equal(placed, placed_here)
+    for layout, got in ((True, here[0]), (False, here[1])):
+        want = _ref_gpu(a[:rows], wt if layout else w, sizes.cpu(), False, layout)
+        assert max_block_err(got, want) < TOL
 
 
 @pytest.mark.parametrize('counts,k,n', [
