@@ -623,6 +623,18 @@ int mbx_debug_row_kernel(int kernel) {
   row_kernel = kernel == kGeneral || kernel == kPair ? kernel : kByRule;
   return before;
 }
+
+// For tests: which of them the rules give a 16-bit NN / NT launch to (0: one of those for few rows per expert).  dual: two operand pairs
+// (no epilogue); epi: one of gmm_dma.h's; workspace: whether one is lent.
+int mbx_debug_row_kernel_by_rule(int layout, int epi, int dual, int num_groups, int64_t rows, int k, int n, int workspace) {
+  static const int some = 0;   // nothing is read through it
+  DmaCall call{&some, &some, nullptr, MBX_BF16, nullptr, num_groups, rows, k, n, layout, nullptr};
+  call.epi = epi;
+  if (dual || dma::epi_is_dglu(epi)) call.a2 = &some;
+  if (dual || dma::epi_is_glu(epi)) call.b2 = &some;
+  if (workspace) call.ws.base = (void*)&some;
+  return gmm_few_takes(call) || gmm_mid_takes(call) ? 0 : gmm_pair_takes(call) ? kPair : kGeneral;
+}
 #endif
 
 #ifdef MBX_TICKS

@@ -69,6 +69,12 @@ int gmm_mid(const DmaCall& call);
 // NN launches with no full round of tiles are cut along the reduction from this many K tiles on: exchanging the parts takes some 20
 // us.  8 experts of 48 rows, [4096, 1024]: 61 -> 36 us; 4 of 500, [2816, 1024]: 58 -> 45; 8 of 256, [1408, 512]: 18 -> 21.
 constexpr int kMinCutTiles = 32;
+// A cut tile has up to kMaxKSplit parts of at least kMinPartTiles K tiles.
+constexpr int kMaxKSplit = 8, kMinPartTiles = 8;
+
+// NN / NT launches of gmm_dma.h's kernel are tiled with the half-height tile only up to kHalfHeightRows rows per expert on average, and
+// up to kMixedRows unless full tiles with a half-height last one make kMixedRounds rounds (gmm_rows.h).
+constexpr int kHalfHeightRows = 144, kMixedRows = 320, kMixedRounds = 3;
 
 // NN / NT launches of few tiles (gmm_pair.hip): whether a launch could run there, and whether it is one of them.
 bool gmm_pair_can(const DmaCall& call);

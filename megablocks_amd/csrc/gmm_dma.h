@@ -1359,7 +1359,6 @@ gmm_rows_kernel(const uint16_t* __restrict__ a, const uint16_t* __restrict__ b, 
   //     Nobody waits for anybody.  The tail then takes 1 / ksplit of a round plus the reduction;
   //   * else the tail's tiles are cut into two half-height tiles each (TS), which take 0.7 of a full tile's time.
   constexpr bool kSplitK = B_MC && EPI == kEpiNone && !GATHER;
-  constexpr int kMaxKSplit = 8, kMinPartTiles = 8;
   int ksplit = 1;
   if constexpr (kSplitK) {
     if (ws_parts != nullptr && rest > 0 && 2 * rest <= P) {

@@ -233,14 +233,25 @@ bool gmm_pair_can(const DmaCall& q) { return q.layout != MBX_TN && !(q.gather.sl
 // Whether the launch is estimated to be shorter here than with gmm_dma.h's tiles, by a sixteenth at least.  Both estimates are
 // rounds of tiles times K tiles times what one takes, us, fitted to 206 NT and 206 NN launches (4 - 64 experts of 48 - 800 rows,
 // [512 - 2048, 1408 - 4096], operands out of memory; rms 11 - 12 %), and no less than the operands at the rate the kernel reads them.
-// Of those launches this takes about half; as chosen they are 10 % (NT) and 18 % (NN, with the cut of gmm_rows.h) shorter on the
-// geometric mean, one in twenty 3 - 12 % longer.  gmm_dma.h's kernel / this one: NT 4 experts of 500, [1408, 2048]: 42 / 23; 8 of 300, [4096,
-// 2048]: 66 / 58; 64 of 48, [4096, 2048]: 247 / 189; 12 of 500, [2728, 1032]: 62 / 65; 16 of 500, [4096, 2048]: 136 / 151.  NN 8 of 500, [1408, 512]: 32 /
-// 16; 16 of 300, [1408, 2048]: 56 / 41; 8 of 300, [4096, 1024], cut: 49 / 41; 4 of 100: 30 / 40; 32 of 500, [3072, 768]: 79 / 110.
-// Under the epilogues (111 launches each of 100 - 700 rows per expert, [512 - 2048, 1408 - 4096]) the choice is as good: 6 % (activation), 7 % (its
-// gradient, the gate's gradient, the activation alone) shorter than gmm_dma.h's, 1.5 % of the best of both at most; except with the gate on up
-// to 144 rows, whose half-height tiles are quicker than estimated (16 experts of 100, [4096, 1024]: 58 / 66; 64 of 100, [2816, 1024]: 159 / 173): there
-// only what is shorter by a fifth (nine of 111 launches 4 - 15 % longer before, two 5 % now).
+// gmm_dma.h's kernel / this one: NT 4 experts of 500, [1408, 2048]: 42 / 23; 8 of 300, [4096, 2048]: 66 / 58; 64 of 48, [4096, 2048]: 247 /
+// 189; 12 of 500, [2728, 1032]: 62 / 65; 16 of 500, [4096, 2048]: 136 / 151.  NN 8 of 500, [1408, 512]: 32 / 16; 16 of 300, [1408, 2048]: 56 /
+// 41; 8 of 300, [4096, 1024], cut: 49 / 41; 4 of 100: 30 / 40; 32 of 500, [3072, 768]: 79 / 110.
+// Gated launches of up to kHalfHeightRows rows, whose half-height tiles are quicker than estimated (16 experts of 100, [4096, 1024]: 58 / 66; 64
+// of 100, [2816, 1024]: 159 / 173): only what is shorter by a fifth.
+//
+// Bounds, where the estimates no longer hold (1780 launches of 1 - 256 experts, 41 - 40000 rows, [64 - 14336, 64 - 14336]):
+//   * eight rounds; two with the gate, whose three outputs are not in the estimate; four with more than kManyExperts experts: the kernel's
+//     gain is the last round and what overlaps across it (up to half a round 28 - 40 % shorter, to one 7 - 24, to four 8 - 17, to eight 3 -
+//     13, beyond 16 4 % to -10 %, a quarter of them by more than 3 % longer; with the gate 2 - 4 rounds 2 %, then -8 to -22 %: 8 experts of
+//     13700, [128, 4328]: 1262 / 1824; activation, 16 of 17200, [128, 2960]: 886 / 1109);
+//   * NN products that gmm_dma.h's kernel may cut, of fewer than kMostCutTiles K tiles: cutting longer ones gains more than estimated (8 of
+//     2037, [9536, 240]: 109 / 146; 4 of 1700, [10880, 752]: 126 / 169; with the combine, which is not cut, 4 of 1200, [8640, 120]: 152 / 82);
+//   * more than kManyExperts experts: what is shorter by a fifth (160 of 75, [1536, 136], two pairs: 50 / 61; of 52, [704, 320]: 31 / 21).
+// As chosen, of 2000 launches that none of this was fitted to (400 each in the fitted range, of 800 - 40000 rows, of 96 - 256 experts, of
+// [64 - 14336, 64 - 14336], of 9 - 47 rows; plain, two pairs and every epilogue): 25 / 37 / 19 / 29 / 30 % shorter on the geometric mean than
+// gmm_dma.h's; 3.5 % of them by more than 3 % longer, most of those 3 - 15 % (8 of 499, [880, 3640]: 36 / 48).
+constexpr double kMostRounds = 8, kMostRoundsMany = 4, kMostRoundsGlu = 2, kMostCutTiles = 96, kManyExperts = 64;
+
 bool gmm_pair_takes(const DmaCall& q) {
   if (!gmm_pair_can(q)) return false;
   const bool nn = q.layout == MBX_NN, dual = q.a2 && !dma::epi_is_dglu(q.epi), glu = dma::epi_is_glu(q.epi);
@@ -250,21 +261,24 @@ bool gmm_pair_takes(const DmaCall& q) {
   auto row_tiles = [&](double height) { return experts * (average > 64 ? average / height + 0.5 : 1.0); };   // the row counts vary
   // here: a round is two tiles to a compute unit, which one by itself works off in little more than half the time
   const double tiles = row_tiles(128) * ceil(n / 128), rounds = floor(tiles / (2 * units)), rest = tiles / (2 * units) - rounds;
+  const bool many = experts > kManyExperts;
+  const bool may_cut = nn && q.epi == dma::kEpiNone && q.ws.base;
+  if (tiles > (glu ? kMostRoundsGlu : many ? kMostRoundsMany : kMostRounds) * 2 * units || (may_cut && nk >= kMostCutTiles)) return false;
   double here = 4.8 + rounds * nk * 1.2;
   if (rest > 0) here += nk * (rest <= 0.5 ? 0.56 : 0.56 + 0.64 * (2 * rest - 1));
   here = fmax(here, 4.8 + mb / 5.5);
   // there: gmm_rows.h's choice of the half-height tile, and the cut of a last round that is at most half full
-  const bool half = average <= 144 || (average <= 320 && row_tiles(256) * ceil(n / 256) < 3 * units);
+  const bool half = average <= kHalfHeightRows || (average <= kMixedRows && row_tiles(256) * ceil(n / 256) < kMixedRounds * units);
   const double tile = nk * (nn ? (half ? 1.03 : 1.57) : (half ? 0.9 : 1.4)) + (nn ? 0 : 5);
   const double all = row_tiles(half ? 128 : 256) * ceil(n / 256), full = floor(all / units), left = all - full * units;
   double there = (nn ? 1.3 : 0.5) + full * tile;
   if (left > 0) {
-    const double parts = fmin(fmin(8.0, floor(units / left)), floor(nk / 8));
-    const bool cut = nn && q.epi == dma::kEpiNone && q.ws.base && 2 * left <= units && (full > 0 || nk >= kMinCutTiles) && parts >= 2;
+    const double parts = fmin(fmin((double)kMaxKSplit, floor(units / left)), floor(nk / kMinPartTiles));
+    const bool cut = may_cut && 2 * left <= units && (full > 0 || nk >= kMinCutTiles) && parts >= 2;
     there += cut ? tile / parts + 21 : 2 * left <= units && full > 0 && !half ? 0.75 * tile : tile;
   }
   there = fmax(there, (nn ? 1.3 : 0.5) + mb / (nn ? 5.4 : 4.6));
-  return here < (glu && average <= 144 ? 0.8 : 0.94) * there;
+  return here < (glu && average <= kHalfHeightRows ? 0.8 : many ? 0.8 : 0.94) * there;
 }
 
 int gmm_pair(const DmaCall& q) { return q.dtype == MBX_BF16 ? pair::dispatch<MBX_BF16>(q) : pair::dispatch<MBX_F16>(q); }

@@ -12,16 +12,16 @@ namespace {
 #include "gmm_dma.h"
 
 // NN / NT: whether to tile a launch with the half-height tile only.  With about one such tile per expert
-// (up to 144 rows on average) the full tile would mostly multiply padding.  Up to 320 rows the mix of
+// (up to kHalfHeightRows rows on average) the full tile would mostly multiply padding.  Up to kMixedRows the mix of
 // full tiles and a half-height last tile moves fewer weight bytes through the compute units (the
 // weights are streamed once per row tile), but its tiles cost unequal time, and a launch of fewer than
-// three rounds of them does not balance over the statically assigned workgroups.
+// kMixedRounds rounds of them does not balance over the statically assigned workgroups.
 static inline bool half_height_only(int64_t rows, int num_groups, int n) {
   const int64_t avg = rows / (num_groups > 0 ? num_groups : 1);
-  if (avg <= 144) return true;
-  if (avg > 320) return false;
+  if (avg <= kHalfHeightRows) return true;
+  if (avg > kMixedRows) return false;
   const int64_t mixed_tiles = (ceil_div(rows, dma::TileMain::BM) + num_groups / 2) * ceil_div(n, dma::TileMain::BN);
-  return mixed_tiles < 3 * (int64_t)persistent_grid((int64_t)1 << 30);
+  return mixed_tiles < kMixedRounds * (int64_t)persistent_grid((int64_t)1 << 30);
 }
 
 // TS is the tile the tail of a launch is cut into (TS = T: never cut).

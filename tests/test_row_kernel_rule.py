@@ -1,0 +1,37 @@
+"""Which kernel the rules give NN / NT launches to, without a GPU (the rules then take 256 compute units)."""
+import ctypes
+
+import pytest
+
+from megablocks_amd import _lib
+
+FEW, GENERAL, FEW_TILES = 0, 1, 2
+PLAIN, ACT, DACT, GATE, COMBINE = 0, 1, 2, 5, 7
+
+
+@pytest.fixture
+def kernel():
+    f = _lib.lib.mbx_debug_row_kernel_by_rule
+    f.argtypes = [ctypes.c_int] * 4 + [ctypes.c_int64] + [ctypes.c_int] * 3
+
+    def ask(layout, experts, rows, k, n, epi=PLAIN, dual=False, workspace=True):
+        return f(layout, epi, dual, experts, experts * rows, k, n, workspace)
+    return ask
+
+
+@pytest.mark.parametrize('layout,experts,rows,k,n,epi', [
+    (_lib.NT, 4, 500, 1408, 2048, PLAIN), (_lib.NT, 8, 3234, 576, 72, PLAIN), (_lib.NT, 160, 52, 704, 320, PLAIN),
+    (_lib.NN, 8, 500, 1408, 512, PLAIN), (_lib.NT, 32, 43, 3176, 152, GATE), (_lib.NT, 16, 1530, 1536, 88, DACT),
+    (_lib.NN, 4, 1200, 8640, 120, COMBINE)])
+def test_launches_of_few_tiles(kernel, layout, experts, rows, k, n, epi):
+    assert kernel(layout, experts, rows, k, n, epi) == FEW_TILES
+
+
+@pytest.mark.parametrize('layout,experts,rows,k,n,epi,dual', [
+    (_lib.NT, 8, 13673, 128, 4328, GATE, False), (_lib.NT, 2, 15001, 128, 8848, GATE, False), (_lib.NT, 16, 17159, 128, 2960, ACT, False),
+    (_lib.NT, 128, 759, 256, 2824, ACT, False), (_lib.NT, 64, 353, 64, 13432, PLAIN, False), (_lib.NT, 90000, 1, 64, 4096, PLAIN, False),
+    (_lib.NN, 8, 2037, 9536, 240, PLAIN, False), (_lib.NN, 4, 1705, 10880, 752, PLAIN, False), (_lib.NN, 32, 288, 12512, 400, PLAIN, True),
+    (_lib.NN, 160, 75, 1536, 136, PLAIN, True), (_lib.NN, 96, 132, 2176, 224, PLAIN, False), (_lib.NT, 160, 282, 1024, 848, PLAIN, False)])
+def test_launches_outside_of_what_the_estimates_hold_for(kernel, layout, experts, rows, k, n, epi, dual):
+    """Measured 5 - 45 % longer in the kernel for few tiles than in the general one, or of the same kind."""
+    assert kernel(layout, experts, rows, k, n, epi, dual) in (FEW, GENERAL)
