@@ -635,6 +635,12 @@ int mbx_debug_row_kernel_by_rule(int layout, int epi, int dual, int num_groups, 
   if (workspace) call.ws.base = (void*)&some;
   return gmm_few_takes(call) || gmm_mid_takes(call) ? 0 : gmm_pair_takes(call) ? kPair : kGeneral;
 }
+
+// For tests: the tiles of a 16-bit TN launch, as gmm_tn_short_choice() numbers them.
+int mbx_debug_tn_kernel_by_rule(int num_groups, int64_t rows, int k, int n) {
+  static const int some = 0;
+  return gmm_tn_short_choice(DmaCall{&some, &some, nullptr, MBX_BF16, nullptr, num_groups, rows, k, n, MBX_TN, nullptr});
+}
 #endif
 
 #ifdef MBX_TICKS

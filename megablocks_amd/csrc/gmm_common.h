@@ -84,6 +84,8 @@ int gmm_pair(const DmaCall& call);
 // TN launches with few rows per expert (gmm_tn_short.hip), and whether a launch is one of them.
 bool gmm_tn_short_takes(const DmaCall& call);
 int gmm_tn_short(const DmaCall& call);
+// For tests: 0 gmm_dma.h's kernel, 1 128 x 128 tiles, 2 256 x 128 tiles, 3 128 x 128 tiles that fetch ahead.
+int gmm_tn_short_choice(const DmaCall& call);
 
 // NN / NT launches, k a multiple of 64 (gmm_rows.hip) and of 8 only (gmm_rows_tail.hip).
 int gmm_rows(const DmaCall& call);

@@ -257,6 +257,14 @@ gmm_tn_short_kernel(const uint16_t* __restrict__ a, const uint16_t* __restrict__
   if (AHEAD) prefetch.arrived();
 }
 
+// Products of up to kSplitRows rows per expert whose rows are no whole 64-byte pieces: tiles beside each other store parts of the same piece,
+// which leave the L2 one by one (59 experts of 35, [2376, 1736]: 13 - 15 % more written than the product has, 154 us; [2376, 1728]: 79).
+// From more than kSplitColumns columns on, what is fetched ahead next to such stores costs more than it saves, and so do 256 x 128 tiles, which
+// fetch ahead (us, with / without, 256 x 128: 185 / 154, 59 experts of 35; 52 of 82, [1400, 1832]: 104 / 92; 50 launches 9 % on the geometric
+// mean, 13 % above 24 column tiles; of up to kSplitColumns columns 5 % the other way, above kSplitRows rows 3 - 9 %, and with whole pieces 4 - 7 %).
+constexpr int kSplitRows = 128, kSplitColumns = 1024;
+static bool split_rows(const DmaCall& q) { return q.n % 32 != 0 && q.n > kSplitColumns && q.rows <= (int64_t)kSplitRows * q.num_groups; }
+
 // ---- a few hundred rows per expert: choose() ----
 // 256 x 128 tiles, two workgroups of four waves to a compute unit, each with three stages of 32 rows: two K tiles under way while one is
 // multiplied, one barrier per K tile.
@@ -385,12 +393,12 @@ int launch(const DmaCall& q) {
     if (!q.gather.src_bins || !q.gather.row_table || q.gather.top_k <= 0 || q.gather.n_slots > 0x7fffffff) return MBX_EINVAL;
     if (!q.gather.table_ready) dma::build_row_table(q);
     gmm_tn_short_kernel<DT, true, OUT32, false><<<(unsigned)grid, T::THREADS, kLdsBytes, q.stream>>>(a, b, (uint16_t*)q.c, q.bins, q.num_groups, (int)q.rows, q.k, q.n, tiles_m, tiles_n, q.gather.row_table, q.gather.src_bins, q.gather.src_rows, (int)q.gather.n_slots);
-  } else {
-    gmm_tn_short_kernel<DT, false, OUT32, true><<<(unsigned)grid, T::THREADS, kLdsBytes, q.stream>>>(a, b, (uint16_t*)q.c, q.bins, q.num_groups, (int)q.rows, q.k, q.n, tiles_m, tiles_n, nullptr, nullptr, 0, 0);
+    return launch_status();
   }
+  auto kern = split_rows(q) ? gmm_tn_short_kernel<DT, false, OUT32, false> : gmm_tn_short_kernel<DT, false, OUT32, true>;
+  kern<<<(unsigned)grid, T::THREADS, kLdsBytes, q.stream>>>(a, b, (uint16_t*)q.c, q.bins, q.num_groups, (int)q.rows, q.k, q.n, tiles_m, tiles_n, nullptr, nullptr, 0, 0);
   return launch_status();
 }
-
 
 enum Kernel { kDma, kShort, kMid };   // gmm_dma.h's 256 x 256 tiles, 128 x 128 of 64 rows, 256 x 128 of 32 rows
 
@@ -423,18 +431,22 @@ constexpr Cost kCosts[] = {{256, 256, 1, 5.0, 6.2, 1.59, 0.58, 2.96}, {128, 128,
 // half-empty tiles decide there.  135 launches that the estimates were not fitted to (4 - 128 experts, [704 - 8192, 512 - 4096] at random): 256 - 320
 // rows 15 % shorter on the geometric mean, to 400 8 %, to 512 6 %, to 768 3 %, four of them 3 - 9 % longer; above 768 rows they gain nothing.
 // (From / to: 64 experts of 300, [1408, 512]: 59 / 43; 64 of 520, [2304, 576]: 148 / 108; 16 of 300, [3072, 768]: 44 / 36; 8 of 450, [1408, 2048]: 35 / 30;
-// 12 of 500, [1472, 1344]: 41 / 42; 32 of 670, [1664, 832]: 88 / 96.)
+// 12 of 500, [1472, 1344]: 41 / 42; 32 of 670, [1664, 832]: 88 / 96.)  128 x 128 tiles only up to 512 rows: beyond, narrow products take
+// longer than estimated (54 of 755, [176, 6184]: 222 us against 170 with gmm_dma.h's; 93 of 648, [1392, 216]: 85 / 78).
+// All of this against the lines on rows alone and no fetching ahead, 500 launches that none of it was fitted to (2 - 128 experts of 20 - 1100
+// rows, [128 - 8192, 128 - 8192], half of them odd): 5 % shorter on the geometric mean, 35 by more than
+// 3 % longer (few rows and few column tiles, 92 experts of 27, [3072, 448]: 61 / 73; half-empty tiles, 84 of 478, [328, 7368]: 351 / 387).
 static Kernel choose(const DmaCall& q) {
   const double units = persistent_grid((int64_t)1 << 30);
   const int64_t average = q.rows / q.num_groups, tiles = ceil_div(q.k, 128) * ceil_div(q.n, 128) * q.num_groups;
   const int64_t mid_tiles = ceil_div(q.k, TM::BM) * ceil_div(q.n, TM::BN) * q.num_groups;
   Kernel kernel = q.rows <= (int64_t)((double)tiles <= kPerCu * units ? 1024 : 256) * q.num_groups ? kShort : kDma;
   if (q.gather.slots) return kernel;
-  if (average > 64 && average <= 512 && (double)mid_tiles >= 5 * kMidPerCu * units && (average > 256 || q.k % TM::BM == 0 || q.k % TM::BM > TM::BM / 2)) kernel = kMid;
+  if (average > 64 && average <= 512 && !split_rows(q) && (double)mid_tiles >= 5 * kMidPerCu * units && (average > 256 || q.k % TM::BM == 0 || q.k % TM::BM > TM::BM / 2)) kernel = kMid;
   if (average < 256 || average > 768) return kernel;
   const double here = kCosts[kernel](q, units, (double)average);
   for (Kernel other : {kDma, kShort, kMid})
-    if (kCosts[other](q, units, (double)average) < fmin(0.94 * here, kCosts[kernel](q, units, (double)average))) kernel = other;
+    if ((other != kShort || average <= 512) && kCosts[other](q, units, (double)average) < fmin(0.94 * here, kCosts[kernel](q, units, (double)average))) kernel = other;
   return kernel;
 }
 
@@ -445,6 +457,11 @@ bool gmm_tn_short_takes(const DmaCall& q) {
   const int64_t widest = q.k > q.n ? q.k : q.n;
   if (q.layout != MBX_TN || q.rows * widest * 2 >= ((int64_t)1 << 31)) return false;   // one buffer per operand
   return tn_short::choose(q) != tn_short::kDma;
+}
+
+int gmm_tn_short_choice(const DmaCall& q) {
+  const tn_short::Kernel kernel = gmm_tn_short_takes(q) ? tn_short::choose(q) : tn_short::kDma;
+  return kernel == tn_short::kShort && !tn_short::split_rows(q) ? 3 : (int)kernel;
 }
 
 int gmm_tn_short(const DmaCall& q) {

@@ -1,6 +1,7 @@
 """GPU parity tests of the grouped GEMM: against the CPU oracle at small sizes and against an
 fp32 torch formulation on the GPU at the benchmark shapes.  Tolerance: relative Frobenius
 error <= 1e-2 (bf16/f16 inputs, fp32 accumulation)."""
+import ctypes
 import math
 
 import pytest
@@ -1542,6 +1543,34 @@ def test_gmm_tn_of_many_tiles(gg, groups, rows, k, n, spread, dtype):
             assert max_block_err(got[e], a[s].float().t() @ b[s].float()) < TOL
     bin_ids = torch.repeat_interleave(torch.arange(groups), sizes).int().cuda()
     src = gg.GatheredRows(b, torch.arange(rows, device='cuda').int(), bin_ids, ends.cuda().int(), None, 1, rows)
+    assert torch.equal(gg.gmm_tn_gather(a, src, sizes.cuda()), got)
+
+
+@pytest.mark.parametrize('groups,rows,k,n,kernel', [(70, 24, 520, 616, 3), (70, 24, 136, 1544, 1), (33, 100, 1032, 1032, 1), (33, 100, 1032, 1056, 3),
+                                                    (80, 128, 1160, 1096, 1), (80, 129, 1160, 1096, 2), (80, 65, 1280, 1088, 2), (5, 513, 136, 2056, 3),
+                                                    (54, 600, 176, 1544, 2)])
+def test_gmm_tn_stores_of_whole_and_split_pieces(gg, groups, rows, k, n, kernel):
+    """Weight gradients on both sides of the lines between the kernels for few rows per expert, each in the kernel the rule names, block by
+    block against fp32 and bit for bit those on gathered rows; what lies around the product stays."""
+    from megablocks_amd import _lib
+    f = _lib.lib.mbx_debug_tn_kernel_by_rule
+    f.argtypes = [ctypes.c_int, ctypes.c_int64, ctypes.c_int, ctypes.c_int]
+    assert f(groups, groups * rows, k, n) == kernel
+    torch.manual_seed(rows + n)
+    sizes = torch.full((groups,), rows)
+    sizes[0], sizes[1] = 2 * rows, 0
+    a, b = torch.randn(groups * rows, k, device='cuda').bfloat16(), torch.randn(groups * rows, n, device='cuda').bfloat16()
+    around = torch.full((groups * k * n + 2 * n,), 7.0, device='cuda', dtype=torch.bfloat16)
+    got = around[n:-n].view(groups, k, n)
+    gg.backend.gmm(a, b, sizes, trans_a=True, c=got)
+    assert (around[:n] == 7).all() and (around[-n:] == 7).all() and not got[1].any()
+    ends = torch.cumsum(sizes, 0)
+    for e in range(groups):
+        s = slice(int(ends[e] - sizes[e]), int(ends[e]))
+        if sizes[e]:
+            assert max_block_err(got[e], a[s].float().t() @ b[s].float()) < TOL
+    bin_ids = torch.repeat_interleave(torch.arange(groups), sizes).int().cuda()
+    src = gg.GatheredRows(b, torch.arange(groups * rows, device='cuda').int(), bin_ids, ends.cuda().int(), None, 1, groups * rows)
     assert torch.equal(gg.gmm_tn_gather(a, src, sizes.cuda()), got)
 
 

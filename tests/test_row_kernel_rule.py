@@ -1,4 +1,4 @@
-"""Which kernel the rules give NN / NT launches to, without a GPU (the rules then take 256 compute units)."""
+"""Which kernel the rules give launches to, without a GPU (the rules then take 256 compute units)."""
 import ctypes
 
 import pytest
@@ -35,3 +35,23 @@ def test_launches_of_few_tiles(kernel, layout, experts, rows, k, n, epi):
 def test_launches_outside_of_what_the_estimates_hold_for(kernel, layout, experts, rows, k, n, epi, dual):
     """Measured 5 - 45 % longer in the kernel for few tiles than in the general one, or of the same kind."""
     assert kernel(layout, experts, rows, k, n, epi, dual) in (FEW, GENERAL)
+
+
+ROUNDS_OF_256, TILES_128, TILES_256_128, TILES_128_AHEAD = 0, 1, 2, 3
+
+
+@pytest.mark.parametrize('experts,rows,k,n,want', [
+    # whole 64-byte pieces, or few columns: fetched ahead, 256 x 128 tiles for many
+    (64, 64, 1024, 4096, TILES_128_AHEAD), (59, 35, 2376, 1728, TILES_128_AHEAD), (64, 128, 1024, 4096, TILES_256_128), (27, 72, 696, 7904, TILES_256_128),
+    (64, 1, 1024, 4096, TILES_128_AHEAD), (55, 121, 2568, 208, TILES_128_AHEAD), (54, 122, 4320, 1016, TILES_256_128), (4, 1, 8, 8, TILES_128_AHEAD),
+    # pieces that two of many tiles store parts of: neither, up to 128 rows
+    (59, 35, 2376, 1736, TILES_128), (9, 63, 5576, 5736, TILES_128), (27, 72, 696, 7912, TILES_128), (52, 82, 1400, 1832, TILES_128),
+    (69, 128, 872, 5112, TILES_128), (69, 129, 920, 5112, TILES_256_128), (69, 200, 360, 5112, TILES_128_AHEAD),
+    # above 512 rows no 128 x 128 tiles out of estimates
+    (54, 755, 176, 6184, TILES_256_128), (93, 648, 1392, 216, TILES_256_128), (64, 300, 1408, 512, TILES_128_AHEAD), (8, 1024, 576, 1024, TILES_128_AHEAD),
+    (64, 2000, 1024, 4096, ROUNDS_OF_256)])
+def test_weight_gradients_of_few_rows(experts, rows, k, n, want):
+    """On the far side of the lines between them the kernels were measured 5 - 30 % longer."""
+    f = _lib.lib.mbx_debug_tn_kernel_by_rule
+    f.argtypes = [ctypes.c_int, ctypes.c_int64, ctypes.c_int, ctypes.c_int]
+    assert f(experts, experts * rows, k, n) == want
