@@ -641,6 +641,9 @@ int mbx_debug_tn_kernel_by_rule(int num_groups, int64_t rows, int k, int n) {
   static const int some = 0;
   return gmm_tn_short_choice(DmaCall{&some, &some, nullptr, MBX_BF16, nullptr, num_groups, rows, k, n, MBX_TN, nullptr});
 }
+
+// For tests: whether an fp32 NN / NT launch takes the small tile.
+int mbx_debug_f32_small_by_rule(int num_groups, int64_t rows, int k, int n, int dual) { return gmm_f32_rows_small(num_groups, rows, k, n, dual != 0); }
 #endif
 
 #ifdef MBX_TICKS

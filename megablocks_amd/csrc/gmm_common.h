@@ -193,5 +193,7 @@ static inline int persistent_grid(int64_t tiles_upper_bound) {
 // (NN / NT): c = a @ b[e] + a2 @ b2[e].
 int gmm_f32(const void* a, const void* b, const void* a2, const void* b2, void* c, const int32_t* bins, int num_groups,
             int64_t rows, int k, int n, int layout, void* workspace, size_t workspace_bytes, hipStream_t s);
+// For tests: whether an NN / NT launch takes the small tile.
+bool gmm_f32_rows_small(int num_groups, int64_t rows, int k, int n, bool dual);
 
 }  // namespace mbx

@@ -6,10 +6,12 @@
 // instructions per SIMD (measured: 2 are free, 3 cost a fifth, 4 half of the rate), and a value takes six to become parts.  So a
 // workgroup converts a value once, on its way to the LDS, and its waves multiply parts: 1.7 instructions per product.  When every
 // wave converted what it read, 4 per product, the matrix cores were busy 45 - 50 % of the time, now 55 - 59 %, at 2.0 GHz instead
-// of 2.1.  8 experts of 1024 +- 30 rows, hidden 1024, ffn 4096: 374 / 348 / 325 us NT / NN / TN against 455 / 435 / 373 that way,
-// 533 / 545 / 522 on the fp32 instruction and 961 in the element-wise kernel of gmm.hip, which serves every alignment; 237 TFLOP/s
-// on 4096^3 (190; the vendor library 231).  Keeping the pipeline filled across a workgroup's tiles changed nothing (370 / 362 / 337);
-// cutting the parts off instead of rounding them is 3 % faster and up to a third less exact.
+// of 2.1.  8 experts of 1024 +- 30 rows, [1024, 4096], normal values: 376 / 379 / 352 us NT / NN / TN (operands in the last-level cache or
+// not) against 460 / 459 / 408 that way and 947 / 983 / 882 in the element-wise kernel of gmm.hip, which serves every alignment; 4096^3: 626 /
+// 643 / 646 us, 220 - 213 TFLOP/s, against 799 / 802 / 783 (torch.mm: 1067 - 1071).  On the fp32 instruction the first three were some 40 %
+// longer than here.  Reductions of a dozen K tiles or less in small launches, whose time is the latency of a K tile's way through registers and
+// LDS, are 1 - 3 us longer than when operands went to the LDS directly (24 experts of 74, [128, 256], NT: 13.3 / 10.5).  Keeping the
+// pipeline filled across a workgroup's tiles changed nothing; cutting the parts off instead of rounding them is 3 % faster and up to a third less exact.
 //
 // How exact: three parts hold all 24 bits of a value; the three products of parts not taken come to less than 2^-25 of a product,
 // and an accumulator is rounded six times per 32 k instead of 32 times.  Relative error (2-norm) against fp64: 4.8e-7 over
@@ -22,7 +24,7 @@
 //
 // Tile: 128 x 256 per workgroup of eight waves, two to a SIMD, K tiles of 32 in two stages of 72 KiB; 256 x 128 for TN products
 // whose edges it leaves less empty (12 experts of 500 rows, [2728, 1032]: 252 -> 212 us); 64 x 128, 36 KiB a stage and two
-// workgroups to a compute unit, for short experts and launches of few tiles (f32_small()).  Values pass through registers, a
+// workgroups to a compute unit, for short experts, launches of few tiles and columns that leave the wide one half empty (f32_small_rows()).  Values pass through registers, a
 // K tile ahead: while K tile kt is multiplied, kt + 1 is converted and written to the other stage, and the loads of kt + 2 go
 // out into the registers that frees.  One barrier per K tile.
 //
@@ -400,8 +402,8 @@ __device__ __forceinline__ bool any_small(const Args& g, const __amdgpu_buffer_r
 //   * a sum comes out zero and the tile has such a value, whose parts may all have been zero.  Zero sums are common (rows that
 //     pad an expert), so the values are looked at before the tile is repeated.
 // Of the sums only those that are stored count: rows below m_lim, columns below n_lim.  A launch that is formed twice throughout
-// (operands of 2^-60 and less next to others of order one, or of 2^40) takes 824 / 810 / 836 us NT / NN / TN for 8 experts of 1024
-// rows, [1024, 4096], instead of 340 / 324 / 338; the element-wise kernel takes 840 / 878 / 780 for any values.
+// (operands of 2^-60 and less next to others of order one, or of 2^40) takes 993 / 1013 / 954 us NT / NN / TN for 8 experts of 1024
+// rows, [1024, 4096], instead of 376 / 379 / 352; the element-wise kernel takes 947 / 983 / 882 for any values.
 constexpr float kTiny = 0x1p-64f, kHuge = 0x1p38f;
 
 template <bool A_MC, bool B_MC, typename S, bool DUAL>
@@ -685,21 +687,46 @@ static inline bool f32_ok(const void* a, const void* b, const void* c, int64_t r
 
 // TN launches left to gmm.hip's element-wise kernel, a chain of fp32 multiply-adds per sum: up to 24 rows per expert on average.
 // There is next to nothing to multiply, and three of its workgroups share a compute unit, which is what the stores want (us, that
-// kernel / this one; 64 experts, [1024, 4096]: 1 row 214 / 393, 16: 270 / 405, 32: 347 / 418, 64: 500 / 490;  8, [4096,
-// 4096]: 99 / 153, 123 / 153, 170 / 156, 254 / 197;  128, [768, 2048]: 162 / 211, 211 / 221, 269 / 217, 379 / 305).  The size limits are that kernel's.
+// kernel / this one; 64 experts, [1024, 4096]: 32 rows 347 / 397, 64: 500 / 467;  8, [4096, 4096]: 170 / 187, 254 / 224;  128, [768,
+// 2048]: 269 / 272, 379 / 323).  The size limits are that kernel's.  Up to some 190 rows the stores bound this kernel too, and one workgroup
+// to a compute unit overlaps them with little: a third of the launches of 25 - 190 rows are 3 - 15 % longer than two of half the tile
+// were (8 of 128, [4096, 4096]: 286 / 266; 128 of 128, [768, 2048]: 430 / 396), the others shorter (64 of 64, [1024, 4096]: 467 / 519), together 5 %.
 static inline bool f32_short_tn(int num_groups, int64_t rows, int k) {
   return rows <= 24 * (int64_t)num_groups && ceil_div(k, 128) <= 65535 && num_groups <= 65535;
 }
 
-// The small tile, two workgroups to a compute unit, where the main tile would leave three eighths of the compute units or more
-// without one (us, main / small tile: NT 8 experts of 256 rows, [1408, 512]: 40 / 29; 4 of 1500, [704, 4096], 144 tiles: 240 / 218; 32 of
-// 100, [1408, 1024], 192 tiles: 75 / 80.  TN 8 of 512, [1024, 512], 128 tiles: 41 / 31; 8 of 256, [1408, 512], 176 tiles: 29 / 34), and in
-// NN / NT launches of up to 64 rows per expert on average, whose tiles would be half empty (64 experts of 64, [1408, 1024]:
-// 140 / 118; of 100: 157 / 158).
+// TN: the small tile, two workgroups to a compute unit, where the main tile would leave three eighths of the compute units or more
+// without one (us, main / small tile: 8 of 512, [1024, 512], 128 tiles: 41 / 31; 8 of 256, [1408, 512], 176 tiles: 29 / 34).
 static inline bool f32_small(int64_t tiles, int units) { return 8 * tiles < 5 * (int64_t)units; }
+
+// NN / NT: the small tile (us, main / small tile)
+//   * up to 64 rows per expert on average, where main tiles would be half empty (64 experts of 64, [1408, 1024]: 140 / 118; of 100: 157 / 158);
+//   * for few tiles as above (NT 8 of 256, [1408, 512]: 40 / 29; 4 of 1500, [704, 4096], 144 tiles: 240 / 218; 32 of 100, [1408, 1024], 192
+//     tiles: 75 / 80).  Long reductions that only the main tile's launch has few enough tiles to be cut along are shorter there (NN 38 of
+//     209, [3520, 192]: 105 / 157), but less exact: the small tile puts its sums aside;
+//   * where it multiplies that much less padding: kShortArea in reductions of up to kShortTiles K tiles, which are mostly the first
+//     loads and the stores, whose latency the second workgroup hides (28 of 726, [320, 320]: 57 / 45; 68 of 101, [288, 816]: 59 / 43; 22 of
+//     109, [320, 4672]: 68 / 76), kLongArea in longer ones, where it multiplies at three quarters of the main tile's rate (45 of 165,
+//     [8192, 320]: 533 / 365; 19 of 768, [2496, 320]: 175 / 188).  13 of 500 launches (2 - 128 experts of 20 - 2000 rows, [128 - 8192, 128 -
+//     8192]) are 3 - 30 % shorter by this line, one 3 % longer.
 constexpr int64_t kF32SmallRows = 64;
+constexpr int kShortTiles = 12;
+constexpr double kShortArea = 1.25, kLongArea = 1.45;
+static bool f32_small_rows(int num_groups, int64_t rows, int n, int64_t nk, int units) {
+  const int64_t average = ceil_div(rows, num_groups);
+  if (average <= kF32SmallRows) return true;
+  // an expert's rows in whole tiles
+  const int64_t tiles = num_groups * ceil_div(average, f32::Wide::BM) * ceil_div(n, f32::Wide::BN);
+  if (f32_small(tiles, units)) return true;
+  const auto area = [&](int bm, int bn) { return ((double)average / bm + 0.5) * bm * (double)ceil_div(n, bn) * bn; };   // the row counts vary
+  return area(f32::Wide::BM, f32::Wide::BN) > (nk <= kShortTiles ? kShortArea : kLongArea) * area(f32::Small::BM, f32::Small::BN);
+}
 
 }  // namespace
+
+bool gmm_f32_rows_small(int num_groups, int64_t rows, int k, int n, bool dual) {
+  return f32_small_rows(num_groups, rows, n, (dual ? 2 : 1) * ceil_div(k, f32::kBK), persistent_grid((int64_t)1 << 30));
+}
 
 int gmm_f32(const void* a, const void* b, const void* a2, const void* b2, void* c, const int32_t* bins, int num_groups,
                    int64_t rows, int k, int n, int layout, void* workspace, size_t workspace_bytes, hipStream_t s) {
@@ -716,9 +743,7 @@ int gmm_f32(const void* a, const void* b, const void* a2, const void* b2, void* 
                        : f32::launch_tn<f32::Wide>(ap, bp, cp, bins, num_groups, rows, k, n, lent, units, s);
   }
   if ((ceil_div(rows, 64) + num_groups) * ceil_div(n, 128) > 0x7fffffff) return MBX_ERANGE;
-  // an expert's rows in whole tiles
-  const int64_t average = ceil_div(rows, num_groups), tiles = num_groups * ceil_div(average, 128) * ceil_div(n, 256);
-  const bool small = average <= kF32SmallRows || f32_small(tiles, units);
+  const bool small = f32_small_rows(num_groups, rows, n, (a2 ? 2 : 1) * ceil_div(k, f32::kBK), units);
 #define MBX_LAUNCH_F32(B_MC, S, DUAL) return f32::launch_rows<B_MC, S, DUAL>(ap, bp, cp, bins, num_groups, rows, k, n, ap2, bp2, lent, units, s)
 #define MBX_LAUNCH_F32_BM(B_MC, DUAL) do { if (small) MBX_LAUNCH_F32(B_MC, f32::Small, DUAL); else MBX_LAUNCH_F32(B_MC, f32::Wide, DUAL); } while (0)
   if (layout == MBX_NT) {

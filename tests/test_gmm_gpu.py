@@ -938,6 +938,8 @@ def test_gmm_on_gathered_rows_with_assignments_out_of_range(gg):
     (2, 4100, 128, 384),     # TN: few tiles, long reduction
     (70, 2000, 64, 128),     # several experts per lane of the tile lookup, unranked TN
     (5, 40, 128, 4100),      # many column tiles, a few rows per expert
+    (60, 12000, 288, 300),   # many small tiles for the columns' sake, a short reduction and a longer one
+    (60, 12000, 600, 300),
 ])
 @pytest.mark.parametrize('mode', ['nn', 'nt', 'tn', 'dual_nn', 'dual_nt'])
 def test_gmm_fp32_on_the_matrix_cores(gg, monkeypatch, groups, rows, k, n, mode):

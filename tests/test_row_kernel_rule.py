@@ -55,3 +55,13 @@ def test_weight_gradients_of_few_rows(experts, rows, k, n, want):
     f = _lib.lib.mbx_debug_tn_kernel_by_rule
     f.argtypes = [ctypes.c_int, ctypes.c_int64, ctypes.c_int, ctypes.c_int]
     assert f(experts, experts * rows, k, n) == want
+
+
+@pytest.mark.parametrize('experts,rows,k,n,small', [
+    (64, 64, 1408, 1024, True), (64, 100, 1408, 1024, False), (8, 256, 1408, 512, True), (1, 0, 64, 64, True), (8, 1024, 1024, 4096, False),
+    # the small tile for less padding, in short reductions from a quarter on, in long ones from 45 %
+    (28, 726, 320, 320, True), (68, 101, 288, 816, True), (19, 768, 2496, 320, False), (45, 165, 8192, 320, True), (106, 103, 192, 1024, False)])
+def test_fp32_tiles(experts, rows, k, n, small):
+    f = _lib.lib.mbx_debug_f32_small_by_rule
+    f.argtypes = [ctypes.c_int, ctypes.c_int64, ctypes.c_int, ctypes.c_int, ctypes.c_int]
+    assert bool(f(experts, experts * rows, k, n, 0)) == small
