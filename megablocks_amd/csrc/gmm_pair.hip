@@ -3,8 +3,8 @@
 // What bounds them: with gmm_dma.h's 256 x 256 tiles, one workgroup to a compute unit, the rounds.  12 experts of 500 rows with a
 // [2728, 1032] product are 264 tiles on 256 compute units, their other product is 130 tiles with reductions of 43 K tiles each, and
 // within a round the first loads and the stores of all tiles come at the same time.  Here a workgroup of four waves computes a
-// 128 x 128 tile, two workgroups share a compute unit, each with two stages of 32 KiB, and one stores or waits while the other
-// multiplies.
+// 128 x 128 tile, two workgroups share a compute unit, each with three 16 KiB stages of A and two of B (together all of the LDS), and
+// one stores or waits while the other multiplies.
 //
 // Layouts and the order of the sums are gmm_dma.h's: the products are bit for bit those of its kernels.
 #include "gmm_common.h"
