@@ -230,28 +230,37 @@ int dispatch(const DmaCall& q) {
 // Gathered rows: whole K tiles.
 bool gmm_pair_can(const DmaCall& q) { return q.layout != MBX_TN && !(q.gather.slots && q.k % pair::T::BK); }
 
-// Whether the launch is estimated to be shorter here than with gmm_dma.h's tiles, by a sixteenth at least.  Both estimates are
+// By which part the launch has to be estimated shorter here than with gmm_dma.h's tiles (0: never here), a sixteenth in general.  `rounds`: of
+// tiles, here.  What the estimates leave out, from 5300 launches (2 - 4000 experts of 4 - 12000 rows on average, even or popular as r^-0.6 or r^-1.2, [64 - 4096,
+// 64 - 12000], plain, two pairs and every epilogue but the combine; time here / gmm_dma.h's on the geometric mean):
+//   * up to eight rounds the sixteenth holds, whatever the number of experts (above 64: 0.88, the activation's gradient 0.83).  The gain is the last
+//     round and what overlaps across it.  Beyond, most launches are longer here (1.06; 8 experts of 13700, [128, 4328], with the gate: 1262 / 1824 us;
+//     activation, 16 of 17200, [128, 2960]: 886 / 1109), but not those of up to kHalfHeightRows rows (0.91 to 24 rounds) and the activation's
+//     gradient (0.95) that an eighth is expected from, nor where gmm_dma.h's tile is mostly padding (0.74);
+//   * the gate's three outputs are not in the estimates: four rounds (two to four 0.93, four to eight 0.99, then 1.12); and of up to kHalfHeightRows rows,
+//     where the half-height tiles are quicker than estimated (16 experts of 100, [4096, 1024]: 58 / 66 us), only what is shorter by a fifth;
+//   * cutting products of kLongCutTiles K tiles and more gains gmm_dma.h's kernel more than estimated (1.09; 8 of 2037, [9536, 240]: 109 / 146 us; 4 of 1700,
+//     [10880, 752]: 126 / 169), except where its tile is mostly padding (36 of 825, [7768, 64]: 218 / 144);
+//   * every workgroup looks its expert up anew: with more than kManyExperts four rounds (0.63, beyond 1.06).
+// As chosen, 1600 of the launches that none of this was fitted to are 10 % shorter than gmm_dma.h's, 2 - 64 experts 17 %, 65 - 256 3 %; 2.4 % of them are by more
+// than 3 % longer, none by more than 18 %.
+constexpr double kFewRounds = 8, kLowRounds = 24, kMostRounds = 32, kGluRounds = 4, kManyRounds = 4, kManyExperts = 1024, kLongCutTiles = 96;
+
+static double gain_line(const DmaCall& q, bool may_cut, double nk, double average, double rounds) {
+  const bool glu = dma::epi_is_glu(q.epi), low = average <= kHalfHeightRows;
+  if (rounds > kMostRounds || (glu && rounds > kGluRounds) || (q.num_groups > kManyExperts && rounds > kManyRounds)) return 0;
+  if (may_cut && nk >= kLongCutTiles) return 0.55;
+  if (glu && low) return 0.8;
+  if (rounds <= kFewRounds) return 0.94;
+  return q.epi == dma::kEpiDact || (low && rounds <= kLowRounds) ? 0.88 : 0.7;
+}
+
+// Whether the launch is estimated to be shorter here than with gmm_dma.h's tiles by enough (gain_line).  Both estimates are
 // rounds of tiles times K tiles times what one takes, us, fitted to 206 NT and 206 NN launches (4 - 64 experts of 48 - 800 rows,
 // [512 - 2048, 1408 - 4096], operands out of memory; rms 11 - 12 %), and no less than the operands at the rate the kernel reads them.
 // gmm_dma.h's kernel / this one: NT 4 experts of 500, [1408, 2048]: 42 / 23; 8 of 300, [4096, 2048]: 66 / 58; 64 of 48, [4096, 2048]: 247 /
 // 189; 12 of 500, [2728, 1032]: 62 / 65; 16 of 500, [4096, 2048]: 136 / 151.  NN 8 of 500, [1408, 512]: 32 / 16; 16 of 300, [1408, 2048]: 56 /
 // 41; 8 of 300, [4096, 1024], cut: 49 / 41; 4 of 100: 30 / 40; 32 of 500, [3072, 768]: 79 / 110.
-// Gated launches of up to kHalfHeightRows rows, whose half-height tiles are quicker than estimated (16 experts of 100, [4096, 1024]: 58 / 66; 64
-// of 100, [2816, 1024]: 159 / 173): only what is shorter by a fifth.
-//
-// Bounds, where the estimates no longer hold (1780 launches of 1 - 256 experts, 41 - 40000 rows, [64 - 14336, 64 - 14336]):
-//   * eight rounds; two with the gate, whose three outputs are not in the estimate; four with more than kManyExperts experts: the kernel's
-//     gain is the last round and what overlaps across it (up to half a round 28 - 40 % shorter, to one 7 - 24, to four 8 - 17, to eight 3 -
-//     13, beyond 16 4 % to -10 %, a quarter of them by more than 3 % longer; with the gate 2 - 4 rounds 2 %, then -8 to -22 %: 8 experts of
-//     13700, [128, 4328]: 1262 / 1824; activation, 16 of 17200, [128, 2960]: 886 / 1109);
-//   * NN products that gmm_dma.h's kernel may cut, of fewer than kMostCutTiles K tiles: cutting longer ones gains more than estimated (8 of
-//     2037, [9536, 240]: 109 / 146; 4 of 1700, [10880, 752]: 126 / 169; with the combine, which is not cut, 4 of 1200, [8640, 120]: 152 / 82);
-//   * more than kManyExperts experts: what is shorter by a fifth (160 of 75, [1536, 136], two pairs: 50 / 61; of 52, [704, 320]: 31 / 21).
-// As chosen, of 2000 launches that none of this was fitted to (400 each in the fitted range, of 800 - 40000 rows, of 96 - 256 experts, of
-// [64 - 14336, 64 - 14336], of 9 - 47 rows; plain, two pairs and every epilogue): 25 / 37 / 19 / 29 / 30 % shorter on the geometric mean than
-// gmm_dma.h's; 3.5 % of them by more than 3 % longer, most of those 3 - 15 % (8 of 499, [880, 3640]: 36 / 48).
-constexpr double kMostRounds = 8, kMostRoundsMany = 4, kMostRoundsGlu = 2, kMostCutTiles = 96, kManyExperts = 64;
-
 bool gmm_pair_takes(const DmaCall& q) {
   if (!gmm_pair_can(q)) return false;
   const bool nn = q.layout == MBX_NN, dual = q.a2 && !dma::epi_is_dglu(q.epi), glu = dma::epi_is_glu(q.epi);
@@ -261,9 +270,8 @@ bool gmm_pair_takes(const DmaCall& q) {
   auto row_tiles = [&](double height) { return experts * (average > 64 ? average / height + 0.5 : 1.0); };   // the row counts vary
   // here: a round is two tiles to a compute unit, which one by itself works off in little more than half the time
   const double tiles = row_tiles(128) * ceil(n / 128), rounds = floor(tiles / (2 * units)), rest = tiles / (2 * units) - rounds;
-  const bool many = experts > kManyExperts;
   const bool may_cut = nn && q.epi == dma::kEpiNone && q.ws.base;
-  if (tiles > (glu ? kMostRoundsGlu : many ? kMostRoundsMany : kMostRounds) * 2 * units || (may_cut && nk >= kMostCutTiles)) return false;
+  const double line = gain_line(q, may_cut, nk, average, tiles / (2 * units));
   double here = 4.8 + rounds * nk * 1.2;
   if (rest > 0) here += nk * (rest <= 0.5 ? 0.56 : 0.56 + 0.64 * (2 * rest - 1));
   here = fmax(here, 4.8 + mb / 5.5);
@@ -278,7 +286,7 @@ bool gmm_pair_takes(const DmaCall& q) {
     there += cut ? tile / parts + 21 : 2 * left <= units && full > 0 && !half ? 0.75 * tile : tile;
   }
   there = fmax(there, (nn ? 1.3 : 0.5) + mb / (nn ? 5.4 : 4.6));
-  return here < (glu && average <= kHalfHeightRows ? 0.8 : many ? 0.8 : 0.94) * there;
+  return here < line * there;
 }
 
 int gmm_pair(const DmaCall& q) { return q.dtype == MBX_BF16 ? pair::dispatch<MBX_BF16>(q) : pair::dispatch<MBX_F16>(q); }
