@@ -242,8 +242,8 @@ bool gmm_pair_can(const DmaCall& q) { return q.layout != MBX_TN && !(q.gather.sl
 //   * cutting products of kLongCutTiles K tiles and more gains gmm_dma.h's kernel more than estimated (1.09; 8 of 2037, [9536, 240]: 109 / 146 us; 4 of 1700,
 //     [10880, 752]: 126 / 169), except where its tile is mostly padding (36 of 825, [7768, 64]: 218 / 144);
 //   * every workgroup looks its expert up anew: with more than kManyExperts four rounds (0.63, beyond 1.06).
-// As chosen, 1600 of the launches that none of this was fitted to are 10 % shorter than gmm_dma.h's, 2 - 64 experts 17 %, 65 - 256 3 %; 2.4 % of them are by more
-// than 3 % longer, none by more than 18 %.
+// As chosen, 1400 other launches of 2 - 256 experts are 11 % shorter than gmm_dma.h's (up to 64 experts 17 %, above 3 %); 2.6 % of them are by more than 3 %
+// longer, none by more than 18 %.
 constexpr double kFewRounds = 8, kLowRounds = 24, kMostRounds = 32, kGluRounds = 4, kManyRounds = 4, kManyExperts = 1024, kLongCutTiles = 96;
 
 static double gain_line(const DmaCall& q, bool may_cut, double nk, double average, double rounds) {
