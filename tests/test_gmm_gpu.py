@@ -1062,6 +1062,55 @@ def test_gmm_fp32_at_the_ends_of_the_range(gg, k, mode):
     assert not bool(got[9].any())
 
 
+@pytest.mark.parametrize('r', [124, 132, 160, 700])   # on both sides of where two scaled parts a value take over from three; cut reductions
+@pytest.mark.parametrize('mode', ['nn', 'nt', 'tn', 'dual_nn', 'dual_nt'])
+def test_gmm_fp32_rows_whose_first_values_do_not_show_their_range(gg, mode, r):
+    """Rows of either operand whose scale cannot be told from the first values: zeros there, a late value 2^10 or 2^30 times as large, later values
+    2^-12 or 2^-40 of the first, one value only; a NaN; in a second run an infinity.  Every row (column) of the product against fp64 within the
+    error of a sum of r terms, 2^-24 sqrt(r) of its terms' root sum square, with a factor of four to spare; what is not finite is so in its own
+    row or column only."""
+    torch.manual_seed(r)
+    rows, n, trans_b, dual = 150, 260, mode.endswith('nt'), mode.startswith('dual')
+
+    def operand(count):     # [count, r]: a row of it is one reduction
+        x = torch.randn(count, r, device='cuda')
+        x[1, :64] = 0
+        x[2, r - 1], x[3, r - 1] = 2.0 ** 10, 2.0 ** 30
+        x[4, 64:] *= 2.0 ** -12
+        x[5, 64:] *= 2.0 ** -40
+        x[6] = 0
+        x[6, r - 3] = 2.0 ** -90
+        x[7, :] = 0
+        x[8] *= 2.0 ** 60
+        return x
+
+    def product(x, w, x2, w2):
+        if mode == 'tn':
+            return gg.backend.gmm(x.t().contiguous(), w.t().contiguous(), torch.tensor([r]), trans_a=True)[0]
+        w, w2 = ((v if trans_b else v.t().contiguous())[None] for v in (w, w2))
+        sizes = torch.tensor([rows])
+        return gg.gmm_dual(x, w, x2, w2, sizes, trans_b=trans_b) if dual else gg.backend.gmm(x, w, sizes, trans_b=trans_b)
+
+    a, b, a2, b2 = operand(rows), operand(n), operand(rows), operand(n)
+    want = a.double() @ b.double().t()
+    terms = (a.double() ** 2) @ (b.double() ** 2).t()
+    if dual:
+        want, terms = want + a2.double() @ b2.double().t(), terms + (a2.double() ** 2) @ (b2.double() ** 2).t()
+    tol = 4 * 2.0 ** -24 * math.sqrt(2 * r if dual else r)
+    got = product(a, b, a2, b2).double()
+    error, size = (got - want) ** 2, terms + 2.0 ** -200
+    for dim in (0, 1):
+        assert float((error.sum(dim) / size.sum(dim)).sqrt().max()) < tol
+    assert bool((got[7] == 0).all()) and bool((got[:, 7] == 0).all())
+    for value, at in ((float('nan'), r // 2), (float('inf'), r - 1)):
+        x = a.clone()
+        x[40, at] = value
+        got = product(x, b, a2, b2).double()
+        rest = torch.arange(rows, device='cuda') != 40
+        assert not bool(torch.isfinite(got[40, torch.arange(n, device='cuda') != 7]).any())
+        assert float((((got - want) ** 2)[rest].sum(1) / size[rest].sum(1)).sqrt().max()) < tol
+
+
 @pytest.mark.parametrize('dtype,mode', [(torch.float32, 'nn'), (torch.float32, 'nt'), (torch.float32, 'tn'), (torch.bfloat16, 'nn')])
 def test_captures_have_workspaces_of_their_own(gg, dtype, mode):
     """Two graphs captured one after the other on one stream, with products whose tiles are cut along the reduction: replayed
