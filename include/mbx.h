@@ -336,6 +336,32 @@ int mbx_experts_forward(const void* x, int64_t tokens, int hidden_size, int dtyp
                         const void* w2, int ffn, int act, int fused_combine, void* out, int32_t* tokens_per_expert, void* scratch,
                         size_t scratch_bytes, void* workspace, size_t workspace_bytes, mbx_stream_t stream);
 
+/* What follows the router in a training step of the dropless layer (megablocks/layers/dmoe.py:239-280 over mlp.py:499-523 /
+ * glu.py:173-205 and their backward passes), enqueued by one call each way: the launches of mbx_route, mbx_gather, mbx_gmm_act / mbx_gmm_glu
+ * (with MBX_STEP_GATHER mbx_gmm_gather), mbx_gmm_ws and mbx_scatter (with MBX_STEP_COMBINE and top_k == 1 mbx_gmm_scatter); of
+ * mbx_scatter_backward, mbx_gmm_dact / mbx_gmm_dglu, the weight gradients (mbx_gmm, mbx_gmm_tn_gather, mbx_gmm_tn_f32), mbx_gmm_ws and
+ * mbx_scatter; with their results bit for bit.  Operands as for mbx_experts_forward; 16-bit dtype.  flags:
+ *   MBX_STEP_GATHER        the experts' rows are read from the tokens and not copied
+ *   MBX_STEP_COMBINE       one expert per token: the second product writes the combined output
+ *   MBX_STEP_KEEP_PRODUCT  the second product is kept (the gradient of `weights` will be asked for)
+ *   MBX_STEP_FP32_WEIGHTS  w1, v1, w2 and their gradients are fp32: the weights are cast (and the casts kept) and may be NULL in the backward
+ *   MBX_STEP_GATE          (backward; in the forward v1 says it) the experts have a gate
+ * kept: mbx_experts_step_bytes(..., 0) bytes that the forward fills and the backward reads; scratch: (..., 1) bytes for the forward, (..., 2)
+ * for the backward; all 16-byte aligned.  Backward: grad [tokens, hidden_size] of type dtype; x only with MBX_STEP_GATHER; dx, dweights (of type
+ * dtype, [tokens * top_k]), dw1, dv1, dw2: NULL where not wanted.  workspace: as for mbx_gmm_ws.  MBX_EUNSUPPORTED (forward only): sizes, types or
+ * alignments that some launch of either pass does not take; out, tokens_per_expert and kept are then undefined. */
+enum { MBX_STEP_GATHER = 1, MBX_STEP_COMBINE = 2, MBX_STEP_KEEP_PRODUCT = 4, MBX_STEP_FP32_WEIGHTS = 8, MBX_STEP_GATE = 16 };
+size_t mbx_experts_step_bytes(int64_t tokens, int top_k, int num_experts, int end_bit, int hidden_size, int ffn, int gate, int flags, int which);
+int mbx_experts_step_forward(const void* x, int64_t tokens, int hidden_size, int dtype, const int32_t* expert_ids, int top_k,
+                             const void* weights, int w_dtype, int num_experts, int end_bit, const void* w1, const void* v1,
+                             const void* w2, int ffn, int act, int flags, void* out, int32_t* tokens_per_expert, void* kept,
+                             size_t kept_bytes, void* scratch, size_t scratch_bytes, void* workspace, size_t workspace_bytes,
+                             mbx_stream_t stream);
+int mbx_experts_step_backward(const void* grad, const void* x, int64_t tokens, int hidden_size, int dtype, int top_k, const void* weights,
+                              int w_dtype, int num_experts, int end_bit, const void* w1, const void* v1, const void* w2, int ffn, int act,
+                              int flags, const void* kept, size_t kept_bytes, void* dx, void* dweights, void* dw1, void* dv1, void* dw2,
+                              void* scratch, size_t scratch_bytes, void* workspace, size_t workspace_bytes, mbx_stream_t stream);
+
 /* The weight gradient of the experts' first product(s) on token rows that were never gathered: the backward's
  * `gmm(dsdd_out, x, batch_sizes, trans_a=True)` of megablocks/layers/mlp.py:485-491 / glu.py:154-159, where x is what
  * megablocks/layers/dmoe.py:219 / :273 gathered (`ops.padded_gather` / `ops.gather`), with that gather done by the

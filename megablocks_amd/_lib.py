@@ -63,6 +63,9 @@ _SIGNATURES = {
     'mbx_gmm_hidden': (_i, [_vp, _i64, _vp, _i, _vp, _vp, _vp, _vp, _i, _vp, _i, _i64, _i, _i, _i, _vp]),
     'mbx_experts_forward_scratch_bytes': (_sz, [_i64, _i, _i, _i, _i, _i, _i]),
     'mbx_experts_forward': (_i, [_vp, _i64, _i, _i, _vp, _i, _vp, _i, _i, _i, _vp, _vp, _vp, _i, _i, _i, _vp, _vp, _vp, _sz, _vp, _sz, _vp]),
+    'mbx_experts_step_bytes': (_sz, [_i64, _i, _i, _i, _i, _i, _i, _i, _i]),
+    'mbx_experts_step_forward': (_i, [_vp, _i64, _i, _i, _vp, _i, _vp, _i, _i, _i, _vp, _vp, _vp, _i, _i, _i, _vp, _vp, _vp, _sz, _vp, _sz, _vp, _sz, _vp]),
+    'mbx_experts_step_backward': (_i, [_vp, _vp, _i64, _i, _i, _i, _vp, _i, _i, _i, _vp, _vp, _vp, _i, _i, _i, _vp, _sz, _vp, _vp, _vp, _vp, _vp, _vp, _sz, _vp, _sz, _vp]),
     'mbx_gelu_backward_inplace': (_i, [_vp, _vp, _i, _i64, _vp]),
     'mbx_glu_forward': (_i, [_vp, _vp, _vp, _i, _i, _i64, _vp]),
     'mbx_glu_backward': (_i, [_vp, _vp, _vp, _vp, _vp, _i, _i, _i64, _vp]),

@@ -633,6 +633,117 @@ def experts_forward(x, expert_ids, expert_weights, num_experts, end_bit, top_k, 
     return out, tokens_per_expert
 
 
+# Bytes a step keeps and works in up to which `experts_step` takes it: beyond, the GPU's time is what counts, and the separate nodes give
+# their tensors back one by one.
+EXPERTS_STEP_MAX_BYTES = 1 << 29
+_STEP_GATHER, _STEP_COMBINE, _STEP_KEEP_PRODUCT, _STEP_FP32_WEIGHTS, _STEP_GATE = 1, 2, 4, 8, 16   # of include/mbx.h
+
+
+class _ExpertsStep(torch.autograd.Function):
+    """(out, tokens_per_expert) of `experts_step`; sizes: (num_experts, end_bit, top_k, ffn, act, flags, bytes kept)."""
+
+    @staticmethod
+    def forward(ctx, x, expert_weights, w1, v1, w2, expert_ids, sizes):
+        num_experts, end_bit, top_k, ffn, act, flags, nbytes = sizes
+        tokens, hidden = x.shape
+        device, code = x.device, _lib.DTYPE[x.dtype]
+        out = torch.empty_like(x)
+        tokens_per_expert = torch.empty(num_experts, dtype=torch.int32, device=device)
+        kept = torch.empty(nbytes, dtype=torch.uint8, device=device)
+        scratch = torch.empty(lib.mbx_experts_step_bytes(tokens, top_k, num_experts, end_bit, hidden, ffn, v1 is not None, flags, 1),
+                              dtype=torch.uint8, device=device)
+        with _lib.device_of(x):
+            ws, ws_bytes = _workspace(device)
+            _lib.check(lib.mbx_experts_step_forward(
+                x.data_ptr(), tokens, hidden, code, expert_ids.data_ptr(), top_k, expert_weights.data_ptr(), _lib.DTYPE[expert_weights.dtype],
+                num_experts, end_bit, w1.data_ptr(), _lib.ptr(v1), w2.data_ptr(), ffn, act, flags, out.data_ptr(), tokens_per_expert.data_ptr(),
+                kept.data_ptr(), nbytes, scratch.data_ptr(), scratch.numel(), ws, ws_bytes, _lib.stream()), 'experts_step_forward')
+        weights = (None, None, None) if flags & _STEP_FP32_WEIGHTS else (w1, v1, w2)   # their casts are kept
+        ctx.save_for_backward(kept, expert_weights, x if flags & _STEP_GATHER else None, *weights)
+        ctx.sizes, ctx.x_like, ctx.shapes = sizes, (x.shape, x.dtype), tuple(None if w is None else w.shape for w in (w1, v1, w2))
+        ctx.mark_non_differentiable(tokens_per_expert)
+        ctx.set_materialize_grads(False)
+        return out, tokens_per_expert
+
+    @staticmethod
+    def backward(ctx, grad, _grad_tokens_per_expert):
+        if grad is None:
+            return (None,) * 7
+        kept, expert_weights, x, w1, v1, w2 = (t if t is None else _aligned(t) for t in ctx.saved_tensors)
+        num_experts, end_bit, top_k, ffn, act, flags, _ = ctx.sizes
+        (tokens, hidden), dtype = ctx.x_like
+        grad = _aligned(grad.to(dtype))
+        device, code = grad.device, _lib.DTYPE[dtype]
+        needs = ctx.needs_input_grad
+        dx = torch.empty((tokens, hidden), dtype=dtype, device=device) if needs[0] else None
+        dweights = torch.empty(tokens * top_k, dtype=dtype, device=device) if needs[1] else None
+        w_dtype = torch.float32 if flags & _STEP_FP32_WEIGHTS else dtype
+        dw1, dv1, dw2 = (torch.empty(shape, dtype=w_dtype, device=device) if need else None for shape, need in zip(ctx.shapes, needs[2:5]))
+        gate = _STEP_GATE if ctx.shapes[1] is not None else 0
+        scratch = torch.empty(lib.mbx_experts_step_bytes(tokens, top_k, num_experts, end_bit, hidden, ffn, gate != 0, flags, 2), dtype=torch.uint8,
+                              device=device)
+        ptr = _lib.ptr
+        with _lib.device_of(grad):
+            ws, ws_bytes = _workspace(device)
+            _lib.check(lib.mbx_experts_step_backward(
+                ptr(grad), ptr(x), tokens, hidden, code, top_k, ptr(expert_weights), _lib.DTYPE[expert_weights.dtype], num_experts, end_bit,
+                ptr(w1), ptr(v1), ptr(w2), ffn, act, flags | gate, ptr(kept), kept.numel(), ptr(dx), ptr(dweights), ptr(dw1), ptr(dv1), ptr(dw2),
+                ptr(scratch), scratch.numel(), ws, ws_bytes, _lib.stream()), 'experts_step_backward')
+        return dx, dweights if dweights is None else dweights.view(expert_weights.shape), dw1, dv1, dw2, None, None
+
+
+def _aligned(t):
+    """`t` in whole 16-byte pieces (a hook on saved tensors, or whoever made the gradient, may hand over any layout)."""
+    t = t.contiguous()
+    return t if t.data_ptr() % 16 == 0 else t.clone()
+
+
+def experts_step(x, expert_ids, expert_weights, num_experts, end_bit, top_k, w1, v1, w2, act, gather):
+    """(out, tokens_per_expert) of the grouped dropless layer behind its router (dmoe.py:239-280) where a gradient is recorded: one node, and
+    one call of the library each way (`mbx_experts_step_forward` / `_backward`), in place of the nodes of ops.gather, the experts and ops.scatter;
+    the launches and the results are theirs, bit for bit.  None: some launch does not take the operands, or they are not plain tensors.
+    w1, v1 (None: no gate), w2 as for `experts_forward`; under autocast they may be fp32 (their gradients then are).  gather: whether the experts'
+    rows are read from the tokens (`FUSED_GATHER`).  (A step the host bounds: 572 tokens, top-2 of 4 experts of [696, 856], gated, 463 -> 246 us;
+    one the GPU bounds, 16384 tokens, 64 experts of [1024, 4096], 1364 -> 1363.)"""
+    tensors = (x, expert_ids, expert_weights, w1, w2) if v1 is None else (x, expert_ids, expert_weights, w1, v1, w2)
+    slots, dtype, device = expert_ids.numel(), x.dtype, x.device
+    if slots == 0 or end_bit > 8 or top_k > 8 or dtype not in (torch.bfloat16, torch.float16) or not x.is_cuda or _lib.profile_hook is not None:
+        return None
+    for t in tensors:
+        if (type(t) is not torch.Tensor and type(t) is not torch.nn.Parameter) or t.device != device:
+            return None
+    tokens, hidden = x.shape
+    elements, w_dtype = w1.numel(), w1.dtype
+    if hidden == 0 or elements % (num_experts * hidden) or tokens * top_k != slots or expert_ids.dtype != torch.int32 or \
+            expert_weights.numel() != slots or expert_weights.dtype not in _lib.DTYPE:
+        return None
+    ffn = elements // (num_experts * hidden)
+    if hidden % 8 or ffn % 8 or ffn <= 192 or ffn * hidden >= 1 << 29 or not _use_epilogue(None, x, slots, ffn):
+        return None
+    for w in tensors[3:]:
+        if w.dtype != w_dtype or w.numel() != elements or not w.is_contiguous() or w.data_ptr() % 16:
+            return None
+    flags = _STEP_GATHER if gather else 0
+    if torch.is_autocast_enabled():
+        if dtype != _lib.autocast_gpu_dtype() or w_dtype not in (dtype, torch.float32):
+            return None
+        if w_dtype == torch.float32:
+            flags |= _STEP_FP32_WEIGHTS
+    elif w_dtype != dtype:
+        return None
+    if top_k == 1 and FUSED_COMBINE != '0':
+        flags |= _STEP_COMBINE
+    if expert_weights.requires_grad:
+        flags |= _STEP_KEEP_PRODUCT
+    sizes = [lib.mbx_experts_step_bytes(tokens, top_k, num_experts, end_bit, hidden, ffn, v1 is not None, flags, which) for which in (0, 2)]
+    if not 0 < sum(sizes) <= EXPERTS_STEP_MAX_BYTES:
+        return None
+    x, expert_ids, expert_weights = x.contiguous(), expert_ids.contiguous(), expert_weights.contiguous()
+    if x.data_ptr() % 16:
+        return None
+    return _ExpertsStep.apply(x, expert_weights, w1, v1, w2, expert_ids, (num_experts, end_bit, top_k, ffn, act, flags, sizes[0]))
+
+
 def gmm_dglu(a, b, x1, x2, batch_sizes, act, fuse=None):
     """The gradients (d x1, d x2) of `activation(x1) * x2` where the incoming gradient is g = a[r_e] @ b[e].T: the
     `gmm(ddsd_out, w2, trans_b=True)` of the GLU experts' backward and the backward of their gated activation

@@ -10,17 +10,17 @@ import torch
 import megablocks_amd.ops as ops
 from megablocks_amd.ops import routing as ops_routing
 from megablocks_amd import grouped_gemm_util as gg
-from megablocks_amd.layers import common, dmlp_registry, moe, mpu
+from megablocks_amd.layers import common, dmlp_registry, moe, mpu, router
 from megablocks_amd.layers.arguments import Arguments
 from megablocks_amd.layers.glu import GroupedGLU, _activation_code
 from megablocks_amd.layers.mlp import DEFAULT_ACTIVATION_FN, GroupedMLP, Topology
 
 
-def _only_computed() -> bool:
+def _only_computed(autocast: bool = False) -> bool:
     """Whether operations are carried out as they are called and nothing else: not traced, compiled, transformed (torch.func),
-    differentiated forward or cast (autocast), all of which act on torch's operators and see nothing of a raw launch.  A torch
-    that does not say counts as one that is doing it."""
-    return not (torch.is_autocast_enabled() or torch.compiler.is_compiling() or torch.jit.is_tracing() or
+    differentiated forward or, unless `autocast` says that the caller sees to that, cast, all of which act on torch's operators and see
+    nothing of a raw launch.  A torch that does not say counts as one that is doing it."""
+    return not ((not autocast and torch.is_autocast_enabled()) or torch.compiler.is_compiling() or torch.jit.is_tracing() or
                 getattr(torch._C, '_are_functorch_transforms_active', lambda: True)() or
                 getattr(torch.autograd.forward_ad, '_current_level', 0) >= 0)   # -1: outside of any dual level
 
@@ -161,9 +161,9 @@ class ParallelDroplessMLP(moe.ParallelMLP):
         x = self._sparse_experts(x, indices, bin_ids, bins, padded_bins, top_k)
         return ops.padded_scatter(x, indices, bin_ids, expert_weights, bins, padded_bins, top_k)
 
-    def _one_call_forward(self, x, expert_weights, top_experts):
-        """grouped_forward_once from one call of the library (gg.experts_forward), where the layer and its experts are the
-        built-in ones, nothing is traced or transformed and no gradient is recorded; else None."""
+    def _one_call_experts(self):
+        """(act, w1, v1, w2) of the experts, v1 None without a gate, where the layer and its experts are the built-in ones, with an
+        activation the library has; else None."""
         experts = self.mlp
         if type(self) is not ParallelDroplessMLP or 'forward_tokens' in experts.__dict__ or \
                 not self.__dict__.keys().isdisjoint(('indices_and_bins', 'grouped_permute_and_compute', 'permute_and_compute')):
@@ -175,20 +175,39 @@ class ParallelDroplessMLP(moe.ParallelMLP):
             act, v1 = _activation_code(self.args.activation_fn), experts.v1
         else:
             return None
-        if act is None or experts.gradient_scale is not None or mpu.experts_per_rank(self.args) != self.num_experts or \
-                not _only_computed():
+        if act is None or experts.gradient_scale is not None or mpu.experts_per_rank(self.args) != self.num_experts:
             return None
+        return act, experts.w1, v1, experts.w2
+
+    def _one_call_forward(self, x, expert_weights, top_experts):
+        """grouped_forward_once from one call of the library (gg.experts_forward), where the layer and its experts are the
+        built-in ones, nothing is traced or transformed and no gradient is recorded; else None."""
+        known = self._one_call_experts()
+        if known is None or not _only_computed():
+            return None
+        act, w1, v1, w2 = known
         return gg.experts_forward(x.view(-1, x.shape[-1]), top_experts.int(), expert_weights, self.num_experts, self.sort_end_bit,
-                                  self.args.moe_top_k, experts.w1, v1, experts.w2, act)
+                                  self.args.moe_top_k, w1, v1, w2, act)
+
+    def _one_call_step(self, x, expert_weights, top_experts):
+        """grouped_forward_once as one node (gg.experts_step), where the layer and its experts are the built-in ones, nothing is traced
+        or transformed, nobody looks at the experts module by itself and a gradient is recorded; else None."""
+        known = None if self.args.memory_optimized_mlp else self._one_call_experts()
+        if known is None or router._has_hooks(self.mlp) or not _only_computed(autocast=True):
+            return None
+        act, w1, v1, w2 = known
+        if not any(t is not None and t.requires_grad for t in (x, expert_weights, w1, v1, w2)):
+            return None
+        return gg.experts_step(x.view(-1, x.shape[-1]), top_experts.int(), expert_weights, self.num_experts, self.sort_end_bit,
+                               self.args.moe_top_k, w1, v1, w2, act, self._fuse_gather(x, self.args.moe_top_k))
 
     def grouped_forward_once(self, x, expert_weights, top_experts):
         """dmoe.py:239-258."""
         expert_weights = expert_weights.flatten()
         top_experts = top_experts.flatten()
-        if not torch.is_grad_enabled():
-            done = self._one_call_forward(x, expert_weights, top_experts)
-            if done is not None:
-                return done
+        done = (self._one_call_step if torch.is_grad_enabled() else self._one_call_forward)(x, expert_weights, top_experts)
+        if done is not None:
+            return done
         with torch.no_grad():
             indices, bin_ids, bins, tokens_per_expert = self.indices_and_bins(top_experts)
         out = self.grouped_permute_and_compute(x, tokens_per_expert, indices, bin_ids, expert_weights, bins, -1,

@@ -1,6 +1,7 @@
 """GPU parity tests of the dMoE layer (forward and backward) against the CPU oracle, in the
 manner of the reference's tests/layers/{dmoe,glu,moe}_test.py.  Tolerance: relative Frobenius
 error <= 1e-2 for bf16/f16, 1e-4 for fp32."""
+import contextlib
 import dataclasses
 import math
 from functools import partial
@@ -1307,6 +1308,107 @@ def test_dmoe_forward_from_one_call_is_the_separate_calls(monkeypatch, mlp_type,
             assert torch.equal(g, layer.experts(a, None, w, i))
         assert torch.equal(counts[0], layer.experts.forward_once(*forms[0])[1])
     assert torch.equal(counts[0].long(), torch.bincount(ids.flatten(), minlength=ne))
+
+
+@pytest.mark.parametrize('mlp_type', ['mlp', 'glu'])
+@pytest.mark.parametrize('tokens,hs,ffn,ne,top_k,mode', [
+    (1, 64, 200, 1, 1, 'bf16'), (5, 136, 264, 12, 6, 'bf16'), (300, 256, 520, 8, 1, 'fp16'), (1029, 64, 704, 64, 8, 'bf16'),
+    (777, 72, 200, 16, 2, 'fp16'), (300, 256, 520, 8, 1, 'amp'), (5, 128, 264, 12, 6, 'amp'), (777, 72, 200, 16, 2, 'amp'),
+    (3, 64, 192, 4, 2, 'none'), (3, 60, 200, 4, 2, 'none'), (3, 64, 200, 16, 9, 'none')])
+def test_dmoe_step_from_one_call_is_the_separate_nodes(monkeypatch, mlp_type, tokens, hs, ffn, ne, top_k, mode):
+    """A training step's experts as one node and one call each way: the output and every gradient bit for bit those of the separate
+    nodes, whatever wants a gradient, with the row gather forced on and off, fp32 parameters under autocast, strided and int64
+    assignments, a strided gradient, saved tensors that hooks have moved about; a second backward through a kept graph; 'none': sizes
+    left to the separate nodes."""
+    from megablocks_amd import grouped_gemm_util as gg
+    from megablocks_amd.layers.dmoe import dMoE
+    torch.manual_seed(tokens)
+    amp, dtype = mode == 'amp', torch.float16 if mode == 'fp16' else torch.bfloat16
+    layer = dMoE(_args(hidden_size=hs, ffn_hidden_size=ffn, moe_num_experts=ne, moe_top_k=top_k, mlp_type=mlp_type, bf16=not amp and mode != 'fp16',
+                       fp16=mode == 'fp16'))
+    x = torch.randn(tokens, 1, hs, device='cuda').to(dtype)
+    ids = torch.rand(tokens, ne, device='cuda').topk(top_k).indices
+    weights = torch.rand(tokens, top_k, device='cuda').to(torch.float32 if amp else dtype)
+    grad = torch.randn(tokens, 1, 2 * hs, device='cuda').to(dtype)[..., ::2]
+    params = dict(layer.experts.mlp.named_parameters())
+
+    def step(wants, ids=ids, pack=None):
+        leaves = dict(x=x.clone(), weights=weights.clone())
+        for name, t in {**leaves, **params}.items():
+            t.grad = None
+            t.requires_grad_(wants == 'all' or name in wants)
+        hooks = torch.autograd.graph.saved_tensors_hooks(pack, lambda t: t) if pack else contextlib.nullcontext()
+        with torch.autocast('cuda', dtype=torch.bfloat16, enabled=amp), hooks:
+            y = layer.experts(leaves['x'], None, leaves['weights'], ids)
+        y.backward(grad, retain_graph=True)
+        first = [y] + [t.grad for t in (*leaves.values(), *params.values())]
+        if wants == 'all' and pack is None:
+            for t in (*leaves.values(), *params.values()):
+                t.grad = None
+            y.backward(grad)
+            assert all(torch.equal(a, t.grad) for a, t in zip(first[1:], (*leaves.values(), *params.values())))
+        return first
+
+    def misplaced(t):     # the same values at an address that is no multiple of 16, or strided
+        wide = torch.zeros(2 * t.numel() + 1, dtype=t.dtype, device=t.device)
+        view = wide[1:1 + t.numel()].view(t.shape) if t.numel() % 2 else wide[1::2].view(t.shape)
+        return view.copy_(t)
+
+    seen = []
+    call = gg.experts_step
+    wide_ids = torch.zeros(tokens, 2 * top_k, device='cuda', dtype=torch.int32)
+    wide_ids[:, ::2] = ids
+    forms = [('all', ids.int(), None), ('all', wide_ids[:, ::2], misplaced), (('x',), ids, None), (('weights',), ids, None),
+             (('w2',), ids, None), (('w1', 'weights'), ids, None), (('v1', 'x') if mlp_type == 'glu' else ('w1', 'x'), ids, None)]
+    for gather in ('auto', '1', '0'):
+        monkeypatch.setattr(gg, 'FUSED_GATHER', gather)
+        monkeypatch.setattr(gg, 'experts_step', lambda *a: seen.append(call(*a)) or seen[-1])
+        got = [step(*(form if mode != 'none' else form[:2])) for form in forms]
+        assert len(seen) == len(forms) and all((s is not None) == (mode != 'none') for s in seen)
+        seen.clear()
+        monkeypatch.setattr(gg, 'experts_step', lambda *a: None)
+        for form, values in zip(forms, got):
+            for g, w in zip(values, step(*form[:2])):
+                assert (g is None) == (w is None) and (g is None or (g.dtype == w.dtype and torch.equal(g, w))), (gather, form[0])
+
+
+@pytest.mark.parametrize('mlp_type', ['mlp', 'glu'])
+def test_dmoe_step_from_one_call_under_capture(monkeypatch, mlp_type):
+    """The one-call step recorded into a graph and replayed on new inputs, with eager steps in between: every replay the eager result."""
+    from megablocks_amd import grouped_gemm_util as gg
+    from megablocks_amd.layers.dmoe import dMoE
+    torch.manual_seed(0)
+    layer = dMoE(_args(hidden_size=128, ffn_hidden_size=264, moe_num_experts=8, moe_top_k=2, mlp_type=mlp_type))
+    calls = []
+    call = gg.experts_step
+    monkeypatch.setattr(gg, 'experts_step', lambda *a: calls.append(1) or call(*a))
+    inputs = [(torch.randn(200, 1, 128, device='cuda').bfloat16(), torch.rand(200, 2, device='cuda').bfloat16(),
+               torch.rand(200, 8, device='cuda').topk(2).indices.int()) for _ in range(3)]
+    grad = torch.randn(200, 1, 128, device='cuda').bfloat16()
+    x, weights, ids = (t.clone() for t in inputs[0])
+    x.requires_grad_(True)
+    weights.requires_grad_(True)
+
+    def step(x, weights, ids):
+        wanted = (x, weights, *layer.experts.parameters())
+        y = layer.experts(x, None, weights, ids)
+        return (y, *torch.autograd.grad(y, wanted, grad))
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        step(x, weights, ids)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        out = step(x, weights, ids)
+    for i in (1, 2, 0, 1):
+        with torch.no_grad():
+            for t, v in zip((x, weights, ids), inputs[i]):
+                t.copy_(v)
+        graph.replay()
+        torch.cuda.synchronize()
+        want = step(inputs[i][0].clone().requires_grad_(True), inputs[i][1].clone().requires_grad_(True), inputs[i][2])
+        assert all(torch.equal(a, b) for a, b in zip(out, want))
+    assert len(calls) == 6
 
 
 @pytest.mark.parametrize('mlp_type', ['mlp', 'glu'])

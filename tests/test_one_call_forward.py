@@ -145,3 +145,58 @@ def test_a_torch_that_does_not_say_takes_the_separate_calls(monkeypatch, called,
         with torch.no_grad():
             assert layer._one_call_forward(*_inputs()) is None
     assert not called and dmoe._only_computed()
+
+
+@pytest.fixture
+def stepped(monkeypatch):
+    calls = []
+
+    def experts_step(x, ids, weights, *args):
+        calls.append(args)
+        return x, ids
+    monkeypatch.setattr(gg, 'experts_step', experts_step)
+    return calls
+
+
+@pytest.mark.parametrize('kw', [dict(), dict(mlp_type='glu', activation_fn=F.silu)])
+@pytest.mark.parametrize('context', [contextlib.nullcontext, _autocast])
+def test_the_built_in_layers_step_is_one_call(stepped, kw, context):
+    with context():
+        assert _layer(**kw)._one_call_step(*_inputs()) is not None
+    assert len(stepped) == 1
+
+
+def _hooked(layer):
+    layer.mlp.register_forward_hook(lambda *_: None)
+
+
+def _frozen(layer):
+    layer.requires_grad_(False)
+
+
+@pytest.mark.parametrize('change', [_patched('indices_and_bins'), _patched('grouped_permute_and_compute'), _other_experts, _scaled, _experts_patched,
+                                    _hooked, _frozen])
+def test_other_layers_steps_are_not(stepped, change):
+    layer = _layer()
+    change(layer)
+    assert layer._one_call_step(*_inputs()) is None
+    assert not stepped
+
+
+@pytest.mark.parametrize('kw', [dict(cls=_Layer), dict(activation_fn=F.relu), dict(memory_optimized_mlp=True)])
+def test_steps_of_other_classes_activations_and_schedules_are_not(stepped, kw):
+    assert _layer(**kw)._one_call_step(*_inputs()) is None
+    assert not stepped
+
+
+@pytest.mark.parametrize('transform', [_traced, _vmapped, _jvp, _functional])
+@pytest.mark.filterwarnings('ignore')
+def test_a_traced_or_transformed_step_is_not(stepped, transform):
+    layer, (x, weights, ids) = _layer(), _inputs()
+    results = []
+
+    def f(t):
+        results.append(layer._one_call_step(t, weights, ids))
+        return t * 2
+    transform(f, x)
+    assert results and all(r is None for r in results) and not stepped
