@@ -345,12 +345,14 @@ int mbx_experts_forward(const void* x, int64_t tokens, int hidden_size, int dtyp
  *   MBX_STEP_COMBINE       one expert per token: the second product writes the combined output
  *   MBX_STEP_KEEP_PRODUCT  the second product is kept (the gradient of `weights` will be asked for)
  *   MBX_STEP_FP32_WEIGHTS  w1, v1, w2 and their gradients are fp32: the weights are cast (and the casts kept) and may be NULL in the backward
+ *   MBX_STEP_RECOMPUTE     the activation's output is not kept (megablocks/layers/mlp.py:397-493, glu.py:66-167): the backward makes it again
+ *                          (mbx_gelu_forward / mbx_glu_forward)
  *   MBX_STEP_GATE          (backward; in the forward v1 says it) the experts have a gate
  * kept: mbx_experts_step_bytes(..., 0) bytes that the forward fills and the backward reads; scratch: (..., 1) bytes for the forward, (..., 2)
  * for the backward; all 16-byte aligned.  Backward: grad [tokens, hidden_size] of type dtype; x only with MBX_STEP_GATHER; dx, dweights (of type
  * dtype, [tokens * top_k]), dw1, dv1, dw2: NULL where not wanted.  workspace: as for mbx_gmm_ws.  MBX_EUNSUPPORTED (forward only): sizes, types or
  * alignments that some launch of either pass does not take; out, tokens_per_expert and kept are then undefined. */
-enum { MBX_STEP_GATHER = 1, MBX_STEP_COMBINE = 2, MBX_STEP_KEEP_PRODUCT = 4, MBX_STEP_FP32_WEIGHTS = 8, MBX_STEP_GATE = 16 };
+enum { MBX_STEP_GATHER = 1, MBX_STEP_COMBINE = 2, MBX_STEP_KEEP_PRODUCT = 4, MBX_STEP_FP32_WEIGHTS = 8, MBX_STEP_GATE = 16, MBX_STEP_RECOMPUTE = 32 };
 size_t mbx_experts_step_bytes(int64_t tokens, int top_k, int num_experts, int end_bit, int hidden_size, int ffn, int gate, int flags, int which);
 int mbx_experts_step_forward(const void* x, int64_t tokens, int hidden_size, int dtype, const int32_t* expert_ids, int top_k,
                              const void* weights, int w_dtype, int num_experts, int end_bit, const void* w1, const void* v1,
@@ -404,6 +406,10 @@ int mbx_gmm_dglu(const void* a, const void* b, const void* x1, const void* x2, v
 /* megablocks/layers/gelu.py:9-13 `_gelu_backward_inplace(g, x)`: g *= d/dx gelu_tanh(x). */
 int mbx_gelu_backward_inplace(void* g, const void* x, int dtype, int64_t numel,
                               mbx_stream_t stream);
+
+/* out = gelu_tanh(x) (megablocks/layers/mlp.py:466-472 recomputes it in the backward of the memory-optimised experts), 16-bit types, the values
+ * mbx_gmm_act stores of the same x.  numel must be a multiple of 8 and the buffers 16-byte aligned (else MBX_EINVAL); fp32: MBX_EUNSUPPORTED. */
+int mbx_gelu_forward(const void* x, void* out, int dtype, int64_t numel, mbx_stream_t stream);
 
 /* The gated activation of the GLU experts, megablocks/layers/glu.py:89,204
  * (`activation_fn(x1) * x2`) in one pass: out = round(round(act(a)) * b), i.e. with the same two

@@ -41,8 +41,8 @@ struct Parts {
 struct StepParts {
   Layout kept, forward, backward;
   size_t indices, bin_ids, bins, slot_rows, weights[3], rows, x1, x2, hidden, product;   // kept
-  size_t sort, sort_bytes;                                                               // forward
-  size_t grad_rows, d1, d2, table, table_bytes;                                          // backward
+  size_t sort, sort_bytes, hidden_forward;                                               // forward
+  size_t grad_rows, d1, d2, table, table_bytes, hidden_again;                            // backward
   StepParts(int64_t tokens, int top_k, int num_experts, int end_bit, int hidden_size, int ffn, bool gate, int flags) {
     const size_t n = (size_t)(tokens * top_k), wide = n * (size_t)ffn * 2, narrow = n * (size_t)hidden_size * 2;
     const size_t weight = (size_t)num_experts * ffn * hidden_size * 2;
@@ -54,15 +54,18 @@ struct StepParts {
     rows = flags & MBX_STEP_GATHER ? 0 : kept.take(narrow);
     x1 = kept.take(wide);
     x2 = gate ? kept.take(wide) : 0;
-    hidden = kept.take(wide);
+    const bool again = flags & MBX_STEP_RECOMPUTE;
+    hidden = again ? 0 : kept.take(wide);
     product = kept.take(narrow);
     sort_bytes = mbx_sort_scratch_bytes(n ? n : 1, MBX_I32, end_bit);
     sort = forward.take(sort_bytes);
+    hidden_forward = again ? forward.take(wide) : 0;
     grad_rows = backward.take(narrow);
     d1 = backward.take(wide);
     d2 = gate ? backward.take(wide) : 0;
     table_bytes = flags & MBX_STEP_GATHER ? mbx_gmm_tn_gather_table_bytes(tokens, top_k, num_experts) : 0;
     table = backward.take(table_bytes);
+    hidden_again = again ? d1 : 0;   // before the gradient of the first product, and done with by then
   }
 };
 
@@ -153,7 +156,8 @@ int mbx_experts_step_forward(const void* x, int64_t tokens, int hidden_size, int
   char* const base = (char*)kept;
   int32_t *const indices = (int32_t*)(base + p.indices), *const bin_ids = (int32_t*)(base + p.bin_ids);
   int32_t *const slot_rows = (int32_t*)(base + p.slot_rows), *const bins = (int32_t*)(base + p.bins);
-  void *const x1 = base + p.x1, *const x2 = v1 ? base + p.x2 : nullptr, *const h = base + p.hidden, *const y = base + p.product;
+  void *const x1 = base + p.x1, *const x2 = v1 ? base + p.x2 : nullptr, *const y = base + p.product;
+  void* const h = flags & MBX_STEP_RECOMPUTE ? (char*)scratch + p.hidden_forward : base + p.hidden;
   int rc = mbx_route(expert_ids, slots, num_experts, end_bit, 0, indices, bin_ids, tokens_per_expert, bins, nullptr, slot_rows, (char*)scratch + p.sort, p.sort_bytes, stream);
   if (rc) return rc;
   if (flags & MBX_STEP_FP32_WEIGHTS) {
@@ -203,7 +207,9 @@ int mbx_experts_step_backward(const void* grad, const void* x, int64_t tokens, i
   char* const own = (char*)scratch;
   const int32_t *const indices = (const int32_t*)(base + p.indices), *const bin_ids = (const int32_t*)(base + p.bin_ids);
   const int32_t *const slot_rows = (const int32_t*)(base + p.slot_rows), *const bins = (const int32_t*)(base + p.bins);
-  const void *const x1 = base + p.x1, *const x2 = gate ? base + p.x2 : nullptr, *const h = base + p.hidden, *const y = base + p.product;
+  const void *const x1 = base + p.x1, *const x2 = gate ? base + p.x2 : nullptr, *const y = base + p.product;
+  const bool again = flags & MBX_STEP_RECOMPUTE;
+  const void* const h = again ? own + p.hidden_again : base + p.hidden;
   if (fp32) {
     w1 = base + p.weights[0];
     v1 = gate ? base + p.weights[1] : nullptr;
@@ -214,6 +220,10 @@ int mbx_experts_step_backward(const void* grad, const void* x, int64_t tokens, i
                     : mbx_gather(grad, dtype, tokens, hidden_size, top_k, indices, bins, nullptr, num_experts, weights, w_dtype, grad_rows, slots, top_k > 1 ? slot_rows : nullptr, stream);
   if (rc) return rc;
   if (dw2) {
+    if (again) {
+      rc = gate ? mbx_glu_forward(x1, x2, (void*)h, dtype, act, slots * ffn, stream) : mbx_gelu_forward(x1, (void*)h, dtype, slots * ffn, stream);
+      if (rc) return rc;
+    }
     rc = fp32 ? mbx_gmm_tn_f32(h, grad_rows, 0, nullptr, 1, nullptr, (float*)dw2, dtype, bins, num_experts, slots, ffn, hidden_size, nullptr, 0, 0, stream)
               : mbx_gmm(h, grad_rows, dw2, dtype, bins, num_experts, slots, ffn, hidden_size, MBX_TN, stream);
     if (rc) return rc;

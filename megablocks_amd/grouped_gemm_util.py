@@ -291,6 +291,17 @@ def gmm_act(a, b, batch_sizes, fuse=None, trans_b=True, keep_product=True):
     return c, c_act
 
 
+def gelu_forward(x):
+    """gelu_tanh(x), the values `gmm_act` gives of the same x where its epilogue makes them (`mbx_gelu_forward`); else torch's."""
+    if x.is_cuda and x.dtype in (torch.bfloat16, torch.float16) and x.is_contiguous() and x.numel() % 8 == 0 and x.data_ptr() % 16 == 0 and \
+            ACTIVATION_EPILOGUES:
+        out = torch.empty_like(x)
+        with _lib.device_of(x):
+            _lib.check(lib.mbx_gelu_forward(_lib.ptr(x), _lib.ptr(out), _lib.dtype_of(x), x.numel(), _lib.stream()), 'gelu_forward')
+        return out
+    return torch.nn.functional.gelu(x, approximate='tanh')
+
+
 def gmm_dact(a, b, pre, batch_sizes, c=None, fuse=None):
     """round(a[r_e] @ b[e].T) * d/dx gelu_tanh(pre[r_e]): the activation gradient of the expert MLP's backward
     (mlp.py:478-483 with gelu.py:9-13) with the multiplication in the product's epilogue where the library has a
@@ -636,7 +647,7 @@ def experts_forward(x, expert_ids, expert_weights, num_experts, end_bit, top_k, 
 # Bytes a step keeps and works in up to which `experts_step` takes it: beyond, the GPU's time is what counts, and the separate nodes give
 # their tensors back one by one.
 EXPERTS_STEP_MAX_BYTES = 1 << 29
-_STEP_GATHER, _STEP_COMBINE, _STEP_KEEP_PRODUCT, _STEP_FP32_WEIGHTS, _STEP_GATE = 1, 2, 4, 8, 16   # of include/mbx.h
+_STEP_GATHER, _STEP_COMBINE, _STEP_KEEP_PRODUCT, _STEP_FP32_WEIGHTS, _STEP_GATE, _STEP_RECOMPUTE = 1, 2, 4, 8, 16, 32   # of include/mbx.h
 
 
 class _ExpertsStep(torch.autograd.Function):
@@ -698,12 +709,13 @@ def _aligned(t):
     return t if t.data_ptr() % 16 == 0 else t.clone()
 
 
-def experts_step(x, expert_ids, expert_weights, num_experts, end_bit, top_k, w1, v1, w2, act, gather):
+def experts_step(x, expert_ids, expert_weights, num_experts, end_bit, top_k, w1, v1, w2, act, gather, recompute=False):
     """(out, tokens_per_expert) of the grouped dropless layer behind its router (dmoe.py:239-280) where a gradient is recorded: one node, and
     one call of the library each way (`mbx_experts_step_forward` / `_backward`), in place of the nodes of ops.gather, the experts and ops.scatter;
     the launches and the results are theirs, bit for bit.  None: some launch does not take the operands, or they are not plain tensors.
     w1, v1 (None: no gate), w2 as for `experts_forward`; under autocast they may be fp32 (their gradients then are).  gather: whether the experts'
-    rows are read from the tokens (`FUSED_GATHER`).  (A step the host bounds: 572 tokens, top-2 of 4 experts of [696, 856], gated, 463 -> 246 us;
+    rows are read from the tokens (`FUSED_GATHER`).  recompute: the activation's output is not kept but made again in the backward
+    (the memory-optimised experts; all of x, w1, v1, w2 want a gradient).  (A step the host bounds: 572 tokens, top-2 of 4 experts of [696, 856], gated, 463 -> 246 us;
     one the GPU bounds, 16384 tokens, 64 experts of [1024, 4096], 1364 -> 1363.)"""
     tensors = (x, expert_ids, expert_weights, w1, w2) if v1 is None else (x, expert_ids, expert_weights, w1, v1, w2)
     slots, dtype, device = expert_ids.numel(), x.dtype, x.device
@@ -723,11 +735,13 @@ def experts_step(x, expert_ids, expert_weights, num_experts, end_bit, top_k, w1,
     for w in tensors[3:]:
         if w.dtype != w_dtype or w.numel() != elements or not w.is_contiguous() or w.data_ptr() % 16:
             return None
-    flags = _STEP_GATHER if gather else 0
+    flags = (_STEP_GATHER if gather else 0) | (_STEP_RECOMPUTE if recompute else 0)
     if torch.is_autocast_enabled():
         if dtype != _lib.autocast_gpu_dtype() or w_dtype not in (dtype, torch.float32):
             return None
         if w_dtype == torch.float32:
+            if not _wants_fp32(x, w_dtype):
+                return None
             flags |= _STEP_FP32_WEIGHTS
     elif w_dtype != dtype:
         return None

@@ -192,14 +192,16 @@ class ParallelDroplessMLP(moe.ParallelMLP):
     def _one_call_step(self, x, expert_weights, top_experts):
         """grouped_forward_once as one node (gg.experts_step), where the layer and its experts are the built-in ones, nothing is traced
         or transformed, nobody looks at the experts module by itself and a gradient is recorded; else None."""
-        known = None if self.args.memory_optimized_mlp else self._one_call_experts()
+        known = self._one_call_experts()
         if known is None or router._has_hooks(self.mlp) or not _only_computed(autocast=True):
             return None
         act, w1, v1, w2 = known
-        if not any(t is not None and t.requires_grad for t in (x, expert_weights, w1, v1, w2)):
+        wanted = [t.requires_grad for t in (x, w1, v1, w2) if t is not None]
+        recompute = self.args.memory_optimized_mlp
+        if not (all(wanted) if recompute else any(wanted) or expert_weights.requires_grad):   # mlp.py:459-460, glu.py:117-118 refuse the others
             return None
         return gg.experts_step(x.view(-1, x.shape[-1]), top_experts.int(), expert_weights, self.num_experts, self.sort_end_bit,
-                               self.args.moe_top_k, w1, v1, w2, act, self._fuse_gather(x, self.args.moe_top_k))
+                               self.args.moe_top_k, w1, v1, w2, act, self._fuse_gather(x, self.args.moe_top_k), recompute)
 
     def grouped_forward_once(self, x, expert_weights, top_experts):
         """dmoe.py:239-258."""

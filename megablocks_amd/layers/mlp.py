@@ -332,7 +332,7 @@ class MemoryOptimizedGroupedMLP(torch.autograd.Function):
 
         # Recompute the activation (kept in the graph only when its gradient is taken by autograd).
         if default_act:
-            activation_fn_out = activation_fn(sdd_out)
+            activation_fn_out = gg.gelu_forward(sdd_out)
         else:
             with torch.set_grad_enabled(True):
                 sdd_out = sdd_out.detach().requires_grad_(True)

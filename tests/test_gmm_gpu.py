@@ -1771,3 +1771,16 @@ def test_gathered_products_of_a_few_dozen_rows_per_expert(gg, tokens, experts, t
         got, want = gg.gmm_gather(src, w1, sizes, b2=v1, act=code), gg.gmm_glu(a, w1, v1, sizes, code, fuse=True)
         assert all(torch.equal(p, q) for p, q in zip(got, want)) and torch.equal(got[0], c)
         assert torch.equal(gg.gmm_gather(src, w1, sizes, b2=v1, act=code, keep_product=False)[2], got[2])
+
+
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])
+def test_gelu_forward_is_the_epilogues(gg, dtype):
+    """The pass of its own gives what the first product's epilogue stores, for every finite 16-bit value; from an address or of a
+    size it does not take, torch's values."""
+    x = torch.arange(-32768, 32768, dtype=torch.int32, device='cuda').to(torch.int16).view(dtype)
+    x = torch.where(torch.isfinite(x), x, torch.zeros_like(x)).view(-1, 8)
+    pre, act = gg.gmm_act(x, torch.eye(8, device='cuda').to(dtype)[None], torch.tensor([x.shape[0]]), fuse=True)
+    assert torch.equal(pre, x) and torch.equal(gg.gelu_forward(pre), act)
+    for odd in (pre.flatten()[1:9], pre.flatten()[:7], pre[:, ::2], pre.float()):
+        assert torch.equal(gg.gelu_forward(odd), torch.nn.functional.gelu(odd, approximate='tanh'))
+    assert gg.gelu_forward(pre[:0]).shape == (0, 8)

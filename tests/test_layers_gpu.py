@@ -1314,18 +1314,19 @@ def test_dmoe_forward_from_one_call_is_the_separate_calls(monkeypatch, mlp_type,
 @pytest.mark.parametrize('tokens,hs,ffn,ne,top_k,mode', [
     (1, 64, 200, 1, 1, 'bf16'), (5, 136, 264, 12, 6, 'bf16'), (300, 256, 520, 8, 1, 'fp16'), (1029, 64, 704, 64, 8, 'bf16'),
     (777, 72, 200, 16, 2, 'fp16'), (300, 256, 520, 8, 1, 'amp'), (5, 128, 264, 12, 6, 'amp'), (777, 72, 200, 16, 2, 'amp'),
+    (300, 256, 520, 8, 1, 'memopt'), (5, 128, 264, 12, 6, 'memopt'), (777, 72, 200, 16, 2, 'memopt amp'),
     (3, 64, 192, 4, 2, 'none'), (3, 60, 200, 4, 2, 'none'), (3, 64, 200, 16, 9, 'none')])
 def test_dmoe_step_from_one_call_is_the_separate_nodes(monkeypatch, mlp_type, tokens, hs, ffn, ne, top_k, mode):
     """A training step's experts as one node and one call each way: the output and every gradient bit for bit those of the separate
-    nodes, whatever wants a gradient, with the row gather forced on and off, fp32 parameters under autocast, strided and int64
+    nodes (the memory-optimised ones too), whatever wants a gradient, with the row gather forced on and off, fp32 parameters under autocast, strided and int64
     assignments, a strided gradient, saved tensors that hooks have moved about; a second backward through a kept graph; 'none': sizes
     left to the separate nodes."""
     from megablocks_amd import grouped_gemm_util as gg
     from megablocks_amd.layers.dmoe import dMoE
     torch.manual_seed(tokens)
-    amp, dtype = mode == 'amp', torch.float16 if mode == 'fp16' else torch.bfloat16
+    amp, memopt, dtype = 'amp' in mode, 'memopt' in mode, torch.float16 if mode == 'fp16' else torch.bfloat16
     layer = dMoE(_args(hidden_size=hs, ffn_hidden_size=ffn, moe_num_experts=ne, moe_top_k=top_k, mlp_type=mlp_type, bf16=not amp and mode != 'fp16',
-                       fp16=mode == 'fp16'))
+                       fp16=mode == 'fp16', memory_optimized_mlp=memopt))
     x = torch.randn(tokens, 1, hs, device='cuda').to(dtype)
     ids = torch.rand(tokens, ne, device='cuda').topk(top_k).indices
     weights = torch.rand(tokens, top_k, device='cuda').to(torch.float32 if amp else dtype)
@@ -1360,6 +1361,8 @@ def test_dmoe_step_from_one_call_is_the_separate_nodes(monkeypatch, mlp_type, to
     wide_ids[:, ::2] = ids
     forms = [('all', ids.int(), None), ('all', wide_ids[:, ::2], misplaced), (('x',), ids, None), (('weights',), ids, None),
              (('w2',), ids, None), (('w1', 'weights'), ids, None), (('v1', 'x') if mlp_type == 'glu' else ('w1', 'x'), ids, None)]
+    if memopt:   # all of them want a gradient, or the experts refuse; the combine's weights may not
+        forms = forms[:2] + [(('x', 'w1', 'v1', 'w2'), ids, None)]
     for gather in ('auto', '1', '0'):
         monkeypatch.setattr(gg, 'FUSED_GATHER', gather)
         monkeypatch.setattr(gg, 'experts_step', lambda *a: seen.append(call(*a)) or seen[-1])

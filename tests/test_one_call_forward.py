@@ -184,7 +184,7 @@ def test_other_layers_steps_are_not(stepped, change):
 
 
 @pytest.mark.parametrize('kw', [dict(cls=_Layer), dict(activation_fn=F.relu), dict(memory_optimized_mlp=True)])
-def test_steps_of_other_classes_activations_and_schedules_are_not(stepped, kw):
+def test_steps_of_other_classes_and_activations_and_memory_optimized_ones_without_all_gradients_are_not(stepped, kw):
     assert _layer(**kw)._one_call_step(*_inputs()) is None
     assert not stepped
 
