@@ -459,6 +459,16 @@ int mbx_router_backward(const void* grad_weights, const void* grad_scores, const
  * piece). */
 int mbx_sum_parts(const float* parts, int num_parts, int64_t pitch, void* out, int dtype, int64_t n, mbx_stream_t stream);
 
+/* The sums of the router's auxiliary losses and their gradients.  out[0] = scale * sum over i < n of values[i] * counts[i % period]
+ * (megablocks/layers/moe.py:69-89 for one layer: values the scores [tokens, period], counts the tokens per expert), or with counts NULL of
+ * values[i]^2 (megablocks/layers/router.py:37-42: values the logsumexp of the logits; period 1), in fp32.  scratch: mbx_loss_scratch_bytes(n) bytes (0: NULL).
+ * Gradient: out[i] (of type dtype) = grad[0] * scale * counts[i % period], or grad[0] * scale * 2 values[i]. */
+size_t mbx_loss_scratch_bytes(int64_t n);
+int mbx_loss_sum(const void* values, int dtype, const int32_t* counts, int64_t n, int period, float scale, float* out, float* scratch,
+                 mbx_stream_t stream);
+int mbx_loss_gradient(const float* grad, const void* values, int dtype, const int32_t* counts, int64_t n, int period, float scale, void* out,
+                      mbx_stream_t stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -279,6 +279,66 @@ sum_parts_kernel(const float* __restrict__ parts, int num_parts, int64_t pitch, 
     if (i + t < n) ((E*)out_)[i + t] = Elem<DT>::from_f32(sum[t]);
 }
 
+// The sums of the auxiliary losses: values[i] counts[i % period] (the load-balancing loss: scores and tokens per expert), or without
+// counts values[i]^2 (the z-loss).  A sum of up to kLossOneBlock values is one workgroup's, a longer one is cut into runs of kLossRun for a workgroup
+// each, whose sums a second launch adds in order.  What bounds a loss of a small model is the number of launches: as torch's operations the two losses
+// are ten of 1 - 7 us forward and ten backward, each with a node of its own (a step of 1024 tokens, 8 experts, the host in its slower mode: 825 us with
+// them, 695 with these four).
+constexpr int kLossThreads = 1024, kLossOneBlock = 32 * kLossThreads, kLossRun = 8 * kLossThreads, kLossParts = 256;
+
+__device__ __forceinline__ float block_sum(float v) {   // in thread 0
+  __shared__ float sums[kLossThreads / kWave];
+  v = wave_sum(v);
+  if (lane_id() == 0) sums[threadIdx.x / kWave] = v;
+  __syncthreads();
+  if (threadIdx.x >= kWave) return 0.f;
+  return wave_sum(threadIdx.x < kLossThreads / kWave ? sums[threadIdx.x] : 0.f);
+}
+
+template <int DT>
+__global__ void __launch_bounds__(kLossThreads)
+loss_sum_kernel(const void* __restrict__ values_, const int32_t* __restrict__ counts, int64_t n, int period, float scale, float* __restrict__ out) {
+  typedef typename Elem<DT>::type E;
+  const E* const values = (const E*)values_;
+  const int64_t stride = (int64_t)gridDim.x * kLossThreads;
+  int64_t i = (int64_t)blockIdx.x * kLossThreads + threadIdx.x;
+  int e = (int)(i % period);
+  const int step = (int)(stride % period);
+  float sum = 0.f;
+#pragma unroll 8
+  for (; i < n; i += stride) {
+    const float v = Elem<DT>::to_f32(values[i]);
+    sum += v * (counts ? (float)counts[e] : v);
+    e += step;
+    e = e >= period ? e - period : e;
+  }
+  sum = block_sum(sum);
+  if (threadIdx.x == 0) out[blockIdx.x] = scale * sum;
+}
+
+__global__ void __launch_bounds__(kLossThreads) loss_parts_kernel(const float* __restrict__ parts, int count, float scale, float* __restrict__ out) {
+  const float sum = block_sum(threadIdx.x < (unsigned)count ? parts[threadIdx.x] : 0.f);
+  if (threadIdx.x == 0) *out = scale * sum;
+}
+
+// The sums' gradients: grad scale counts[i % period], or without counts grad scale 2 values[i].
+template <int DT>
+__global__ void __launch_bounds__(256)
+loss_gradient_kernel(const float* __restrict__ grad, const void* __restrict__ values_, const int32_t* __restrict__ counts, int64_t n, int period,
+                     float scale, void* __restrict__ out_) {
+  typedef typename Elem<DT>::type E;
+  const float g = *grad * scale;
+  const int64_t stride = (int64_t)gridDim.x * 256;
+  int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  int e = (int)(i % period);
+  const int step = (int)(stride % period);
+  for (; i < n; i += stride) {
+    ((E*)out_)[i] = Elem<DT>::from_f32(counts ? g * (float)counts[e] : g * (2.f * Elem<DT>::to_f32(((const E*)values_)[i])));
+    e += step;
+    e = e >= period ? e - period : e;
+  }
+}
+
 static inline unsigned token_grid(int64_t tokens) {
   int64_t blocks = ceil_div(tokens, kTokenWaves);
   if (blocks > 256 * 8) blocks = 256 * 8;
@@ -384,6 +444,43 @@ int mbx_sum_parts(const float* parts, int num_parts, int64_t pitch, void* out, i
   if (dtype == MBX_BF16) sum_parts_kernel<MBX_BF16><<<(unsigned)blocks, kTokenThreads, 0, s>>>(parts, num_parts, pitch, out, n);
   else if (dtype == MBX_F16) sum_parts_kernel<MBX_F16><<<(unsigned)blocks, kTokenThreads, 0, s>>>(parts, num_parts, pitch, out, n);
   else sum_parts_kernel<MBX_F32><<<(unsigned)blocks, kTokenThreads, 0, s>>>(parts, num_parts, pitch, out, n);
+  return launch_status();
+}
+
+int mbx_loss_sum(const void* values, int dtype, const int32_t* counts, int64_t n, int period, float scale, float* out, float* scratch,
+                 mbx_stream_t stream) {
+  if (n < 0 || period <= 0 || (dtype != MBX_BF16 && dtype != MBX_F16 && dtype != MBX_F32)) return MBX_EINVAL;
+  if (!out || (n > 0 && !values)) return MBX_EINVAL;
+  if (n > kLossOneBlock && !scratch) return MBX_ESCRATCH;
+  hipStream_t s = as_stream(stream);
+  const int64_t runs = ceil_div(n, kLossRun);
+  const unsigned blocks = n <= kLossOneBlock ? 1u : (unsigned)(runs < kLossParts ? runs : kLossParts);
+  float* const to = blocks > 1 ? scratch : out;
+  const float by = blocks > 1 ? 1.f : scale;
+  switch (dtype) {
+    case MBX_BF16: loss_sum_kernel<MBX_BF16><<<blocks, kLossThreads, 0, s>>>(values, counts, n, period, by, to); break;
+    case MBX_F16: loss_sum_kernel<MBX_F16><<<blocks, kLossThreads, 0, s>>>(values, counts, n, period, by, to); break;
+    default: loss_sum_kernel<MBX_F32><<<blocks, kLossThreads, 0, s>>>(values, counts, n, period, by, to); break;
+  }
+  if (blocks > 1) loss_parts_kernel<<<1, kLossThreads, 0, s>>>(scratch, (int)blocks, scale, out);
+  return launch_status();
+}
+
+size_t mbx_loss_scratch_bytes(int64_t n) { return n > kLossOneBlock ? kLossParts * sizeof(float) : 0; }
+
+int mbx_loss_gradient(const float* grad, const void* values, int dtype, const int32_t* counts, int64_t n, int period, float scale, void* out,
+                      mbx_stream_t stream) {
+  if (n < 0 || period <= 0 || (dtype != MBX_BF16 && dtype != MBX_F16 && dtype != MBX_F32)) return MBX_EINVAL;
+  if (n == 0) return 0;
+  if (!grad || !out || (!counts && !values)) return MBX_EINVAL;
+  hipStream_t s = as_stream(stream);
+  const int64_t wanted = ceil_div(n, 256);
+  const unsigned blocks = (unsigned)(wanted < 2048 ? wanted : 2048);
+  switch (dtype) {
+    case MBX_BF16: loss_gradient_kernel<MBX_BF16><<<blocks, 256, 0, s>>>(grad, values, counts, n, period, scale, out); break;
+    case MBX_F16: loss_gradient_kernel<MBX_F16><<<blocks, 256, 0, s>>>(grad, values, counts, n, period, scale, out); break;
+    default: loss_gradient_kernel<MBX_F32><<<blocks, 256, 0, s>>>(grad, values, counts, n, period, scale, out); break;
+  }
   return launch_status();
 }
 

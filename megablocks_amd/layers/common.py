@@ -23,3 +23,12 @@ def cast_if_autocast_enabled(tensor):
             raise NotImplementedError()
         return tensor.to(dtype=target)
     return tensor
+
+
+def only_computed(autocast: bool = False) -> bool:
+    """Whether operations are carried out as they are called and nothing else: not traced, compiled, transformed (torch.func),
+    differentiated forward or, unless `autocast` says that the caller sees to that, cast, all of which act on torch's operators and see
+    nothing of a raw launch.  A torch that does not say counts as one that is doing it."""
+    return not ((not autocast and torch.is_autocast_enabled()) or torch.compiler.is_compiling() or torch.jit.is_tracing() or
+                getattr(torch._C, '_are_functorch_transforms_active', lambda: True)() or
+                getattr(torch.autograd.forward_ad, '_current_level', 0) >= 0)   # -1: outside of any dual level

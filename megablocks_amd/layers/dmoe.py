@@ -16,13 +16,7 @@ from megablocks_amd.layers.glu import GroupedGLU, _activation_code
 from megablocks_amd.layers.mlp import DEFAULT_ACTIVATION_FN, GroupedMLP, Topology
 
 
-def _only_computed(autocast: bool = False) -> bool:
-    """Whether operations are carried out as they are called and nothing else: not traced, compiled, transformed (torch.func),
-    differentiated forward or, unless `autocast` says that the caller sees to that, cast, all of which act on torch's operators and see
-    nothing of a raw launch.  A torch that does not say counts as one that is doing it."""
-    return not ((not autocast and torch.is_autocast_enabled()) or torch.compiler.is_compiling() or torch.jit.is_tracing() or
-                getattr(torch._C, '_are_functorch_transforms_active', lambda: True)() or
-                getattr(torch.autograd.forward_ad, '_current_level', 0) >= 0)   # -1: outside of any dual level
+_only_computed = common.only_computed
 
 
 def promote_scalar(x):

@@ -42,6 +42,11 @@ def batched_load_balancing_loss(args: Arguments):
     assert all((x.ndim == 1 and x.numel() == args.moe_num_experts for x in tokens_per_expert))
     tokens = expert_scores[0].shape[0]
     assert all(((x.ndim == 2 and x.shape[1] == args.moe_num_experts and x.shape[0] == tokens) for x in expert_scores))
+    scale = (args.moe_num_experts * args.moe_loss_weight) / (args.num_layers * tokens * args.moe_top_k) if tokens else 0.0
+    if layers and tokens and all(args.moe_lbl_in_fp32 or x.dtype == torch.float32 for x in expert_scores) and \
+            router.LossSums.takes(expert_scores, tokens_per_expert):
+        sums = router.LossSums.apply([scale / tokens] * layers, tokens_per_expert, *expert_scores)
+        return sums.view(()) if layers == 1 else sums.sum()
     expert_scores = torch.cat(expert_scores, dim=1)
     if args.moe_lbl_in_fp32:
         expert_scores = expert_scores.float()

@@ -24,6 +24,54 @@ def _save_router_logits(logits: torch.Tensor, args: Arguments, lse=None):
     _ROUTER_LOGITS.append((logits, lse))
 
 
+class LossSums(torch.autograd.Function):
+    """[scales[l] * sum(values[l] * counts[l]) for l] with counts[l] a row for every row of values[l], or (counts None) * sum(values[l]^2): the
+    sums of the auxiliary losses (moe.py:69-89, router.py:37-42), fp32, a launch each (two for long ones) forward and backward."""
+
+    @staticmethod
+    def takes(values, counts) -> bool:
+        """Plain contiguous tensors on the GPU, the counts int32, and nothing that acts on torch's operators at work (autocast does not
+        cast these)."""
+        plain = lambda t, device: type(t) is torch.Tensor and t.is_cuda and t.device == device and t.is_contiguous()
+        device = values[0].device
+        return all(plain(v, device) and v.dtype in _lib.DTYPE and v.numel() for v in values) and \
+            (counts is None or all(plain(c, device) and c.dtype == torch.int32 for c in counts)) and common.only_computed(autocast=True)
+
+    @staticmethod
+    def forward(ctx: Any, scales, counts, *values):
+        out = torch.empty(len(values), dtype=torch.float32, device=values[0].device)
+        with _lib.device_of(out):
+            for l, v in enumerate(values):
+                nbytes = _lib.lib.mbx_loss_scratch_bytes(v.numel())
+                scratch = torch.empty(nbytes, dtype=torch.uint8, device=v.device) if nbytes else None
+                _lib.check(_lib.lib.mbx_loss_sum(_lib.ptr(v), _lib.dtype_of(v), None if counts is None else _lib.ptr(counts[l]), v.numel(),
+                                                 1 if counts is None else v.shape[1], scales[l], out.data_ptr() + 4 * l, _lib.ptr(scratch),
+                                                 _lib.stream()), 'loss_sum')
+        ctx.save_for_backward(*(values if counts is None else counts))
+        ctx.scales, ctx.counted, ctx.like = scales, counts is not None, [(v.shape, v.dtype) for v in values]
+        return out
+
+    @staticmethod
+    def backward(ctx: Any, grad):
+        grads = []
+        with _lib.device_of(grad):
+            grad = grad.float().contiguous()
+            for l, (saved, scale, (shape, dtype)) in enumerate(zip(ctx.saved_tensors, ctx.scales, ctx.like)):
+                if not ctx.needs_input_grad[2 + l]:
+                    g = None
+                elif torch.is_grad_enabled() or not _has_memory(grad):   # differentiated itself, or over a batch of gradients
+                    g = grad[l] * scale * saved.float() if ctx.counted else grad[l] * (2 * scale) * saved.float()
+                    g = g.to(dtype).expand(shape)
+                else:
+                    saved = saved.contiguous()
+                    g = torch.empty(shape, dtype=dtype, device=grad.device)
+                    _lib.check(_lib.lib.mbx_loss_gradient(grad.data_ptr() + 4 * l, None if ctx.counted else _lib.ptr(saved), _lib.DTYPE[dtype],
+                                                          _lib.ptr(saved) if ctx.counted else None, g.numel(),
+                                                          shape[1] if ctx.counted else 1, scale, _lib.ptr(g), _lib.stream()), 'loss_gradient')
+                grads.append(g)
+        return (None, None, *grads)
+
+
 def clear_router_zloss():
     _ROUTER_LOGITS.clear()
 
@@ -34,6 +82,9 @@ def batched_router_zloss(args: Arguments):
         import warnings
         warnings.warn('Call to batched_router_zloss, but moe_zloss_weight=0')
         return 0
+    if _ROUTER_LOGITS and all(lse is not None and (args.moe_zloss_in_fp32 or logits.dtype == torch.float32) for logits, lse in _ROUTER_LOGITS) and \
+            LossSums.takes([lse for _, lse in _ROUTER_LOGITS], None):
+        return LossSums.apply([args.moe_zloss_weight / lse.numel() for _, lse in _ROUTER_LOGITS], None, *(lse for _, lse in _ROUTER_LOGITS))
     terms = []
     for logits, lse in _ROUTER_LOGITS:
         if lse is None:

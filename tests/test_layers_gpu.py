@@ -1021,6 +1021,56 @@ def test_auxiliary_losses_match_oracle(dtype, in_fp32, tokens, hs, ne, top_k, la
     assert moe.get_load_balancing_loss() == [] and moe.batched_load_balancing_loss(_args(moe_loss_weight=0.0)) == 0.0
 
 
+@pytest.mark.parametrize('dtype', [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize('tokens,experts,layers', [(1, 1, 1), (4096, 8, 1), (4097, 8, 1), (300, 12, 3), (70000, 64, 1), (33, 512, 2)])
+def test_sums_of_the_auxiliary_losses(monkeypatch, dtype, tokens, experts, layers):
+    """LossSums against fp64, values and gradients, on both sides of where a sum is cut over workgroups: sums of non-negative terms, 2^-24 times
+    the length of the longest chain (a thread's terms and ten steps of a tree, twice); the same from torch's operations, and where the
+    backward is differentiated or runs over a batch of gradients."""
+    from megablocks_amd.layers import common, router
+    torch.manual_seed(tokens)
+    scores = [torch.rand(tokens, experts, device='cuda').to(dtype) for _ in range(layers)]
+    counts = [torch.randint(0, 5 * tokens + 2, (experts,), device='cuda', dtype=torch.int32) for _ in range(layers)]
+    lse = [torch.rand(tokens, device='cuda') + 1 for _ in range(layers)]
+    scales, weight = [0.5 / (l + 1) for l in range(layers)], torch.rand(layers, device='cuda') + 1
+    chain = -(-tokens * experts // (256 * 1024)) + 32 + 20
+    for values, c in ((scores, counts), (lse, None)):
+        assert router.LossSums.takes(values, c)
+        leaves = [v.clone().requires_grad_(True) for v in values]
+        got = router.LossSums.apply(scales, c, *leaves)
+        grads = torch.autograd.grad(got, leaves, weight, retain_graph=True)
+        again = torch.autograd.grad(got, leaves, weight, create_graph=True)
+        batch = torch.autograd.grad(got, leaves, torch.stack([weight, 2 * weight]), is_grads_batched=True)
+        for l in range(layers):
+            v = values[l].double()
+            want = scales[l] * ((v * c[l].double()).sum() if c else (v * v).sum())
+            assert abs(float(got[l]) - float(want)) <= chain * 2.0 ** -24 * abs(float(want))
+            dwant = float(weight[l]) * scales[l] * (c[l].double().expand_as(v) if c else 2 * v)
+            step = 2.0 ** -8 if grads[l].dtype == torch.bfloat16 else 2.0 ** -22
+            for g in (grads[l], again[l], batch[l][0], batch[l][1] / 2):
+                assert g.dtype == values[l].dtype and g.shape == v.shape and bool(((g.double() - dwant).abs() <= step * dwant.abs()).all())
+        assert again[0].requires_grad or c is not None
+    # the layers' functions, with these sums and without
+    layer_args = _args(hidden_size=64, ffn_hidden_size=128, moe_num_experts=experts, moe_top_k=1, moe_loss_weight=0.1, moe_zloss_weight=1e-3, num_layers=layers,
+                       moe_lbl_in_fp32=True, moe_zloss_in_fp32=True)
+    from megablocks_amd.layers import moe
+    results = []
+    for fused in (True, False):
+        monkeypatch.setattr(common, 'only_computed', lambda autocast=False: fused)
+        moe.clear_load_balancing_loss()
+        router.clear_router_zloss()
+        leaves = [t.clone().requires_grad_(True) for t in (*scores, *lse)]
+        for l in range(layers):
+            moe.save_load_balancing_loss((counts[l], leaves[l]))
+            router._save_router_logits(leaves[l], layer_args, leaves[layers + l])
+        lbl, z = moe.batched_load_balancing_loss(layer_args), router.batched_router_zloss(layer_args)
+        results.append([lbl, z, *torch.autograd.grad([lbl, z.sum()], leaves)])
+    moe.clear_load_balancing_loss()
+    router.clear_router_zloss()
+    for a, b in zip(*results):
+        assert a.shape == b.shape and a.dtype == b.dtype and rel_err(a, b) < (4e-3 if a.dtype == torch.bfloat16 else 2e-6)
+
+
 def test_load_balancing_loss_closed_forms_on_the_layer():
     """Evenly loaded experts give loss_weight whatever the scores (uniform_expert_assignment makes them even);
     the wrong number of saved layers raises as moe.py:42-60 does."""
