@@ -195,6 +195,12 @@ int mbx_binned_scatter(const void* x, int dtype, int64_t tokens, int hidden, int
                        const void* weights, int w_dtype, void* out, void* scratch,
                        size_t scratch_bytes, mbx_stream_t stream);
 
+/* mbx_binned_scatter from a slot -> row map of the sorted assignments (mbx_slot_rows without padded bins, or mbx_route's) and their bins, instead of the
+ * assignments: no scratch, and no launches that turn them into a map.  num_bins > 0. */
+int mbx_binned_scatter_rows(const void* x, int dtype, int64_t tokens, int hidden, int top_k, const int32_t* slot_rows,
+                            const int32_t* bins, int num_bins, int capacity, const void* weights, int w_dtype, void* out,
+                            mbx_stream_t stream);
+
 /* megablocks/backend/kernels.py:521-543 `binned_scatter_wgrad`: wgrad[slot] =
  * <x[e, j], grad[slot / top_k]> for kept slots, 0 for dropped ones. */
 int mbx_binned_scatter_wgrad(const void* x, const void* grad, int dtype, int64_t tokens,

@@ -68,6 +68,11 @@ def forget_slot_rows(indices):
         pass
 
 
+def _kept_slot_rows(indices, key):
+    cached = getattr(indices, '_mbx_slot_rows', None)
+    return cached[1] if cached is not None and cached[0] == key else None
+
+
 def _slot_rows(indices, bin_ids, bins, padded_bins):
     """int32 [n_slots]: the row of the expert-major (optionally padded) buffer that holds each slot.  One map
     serves all gathers and scatters of a routing decision, forward and backward, so it is kept on the `indices`
@@ -78,9 +83,9 @@ def _slot_rows(indices, bin_ids, bins, padded_bins):
     contain the kernels that build its map."""
     capturing = torch.cuda.is_current_stream_capturing()
     key = _slot_rows_key(indices, bins, padded_bins)
-    cached = getattr(indices, '_mbx_slot_rows', None)
-    if not capturing and cached is not None and cached[0] == key:
-        return cached[1]
+    rows = None if capturing else _kept_slot_rows(indices, key)
+    if rows is not None:
+        return rows
     n_slots = indices.shape[0]
     rows = _scratch(n_slots, indices.device)
     with _lib.device_of(indices):
@@ -303,6 +308,13 @@ def binned_scatter(x, indices, weights, bins, top_k):
     indices, bins = _lib.as_i32(indices), _lib.as_i32(bins)
     wp, wdt, weights = _w(weights)
     out = torch.empty((tokens, hidden_size), dtype=x.dtype, device=x.device)
+    # the map that came with the routing, if these are its assignments and bins (see _slot_rows)
+    rows = None if not num_experts or torch.cuda.is_current_stream_capturing() else _kept_slot_rows(indices, _slot_rows_key(indices, bins, None))
+    if rows is not None:
+        with _lib.device_of(x):
+            _lib.check(lib.mbx_binned_scatter_rows(_lib.ptr(x), _lib.dtype_of(x), tokens, hidden_size, top_k, _lib.ptr(rows), _lib.ptr(bins),
+                                                   num_experts, expert_capacity, wp, wdt, _lib.ptr(out), _lib.stream()), 'binned_scatter')
+        return out
     scratch = _scratch(n_slots, x.device)
     with _lib.device_of(x):
         _lib.check(lib.mbx_binned_scatter(_lib.ptr(x), _lib.dtype_of(x), tokens, hidden_size, top_k, _lib.ptr(indices),

@@ -237,6 +237,29 @@ def test_binned_ops(kernels, sl, hs, ne, top_k, cap_factor, dtype):
     assert rel_err(wg, oracle.binned_scatter_wgrad(want, grad, indices, bins, top_k)) < 1e-2
 
 
+@pytest.mark.parametrize('sl,hs,ne,top_k,cap', [(1, 64, 1, 1, 1), (257, 72, 4, 1, 40), (257, 72, 4, 2, 200), (100, 64, 32, 8, 0), (500, 63, 130, 4, 9), (40, 64, 8, 1, 1000)])
+@pytest.mark.parametrize('weighted', [False, True])
+def test_binned_scatter_from_the_routings_map(kernels, sl, hs, ne, top_k, cap, weighted):
+    """The map that came with the routing instead of one of the binned rows: bit for bit the same, with dropped slots, empty experts, no capacity; a map
+    that belongs to other bins or rewritten assignments is not used."""
+    from megablocks_amd.ops import routing
+    torch.manual_seed(sl + ne)
+    ids = (torch.rand(sl * top_k, device='cuda') ** 2 * ne).int().clamp_(max=ne - 1)
+    end_bit = max(int(np.ceil(np.log2(ne))), 1)
+    indices, _, _, bins, _ = routing.route(ids, ne, end_bit)
+    assert kernels._kept_slot_rows(indices, kernels._slot_rows_key(indices, bins, None)) is not None
+    x = torch.randn(ne, cap, hs, device='cuda').half()
+    w = torch.rand(sl * top_k, device='cuda').half() if weighted else None
+    plain = indices.clone()
+    want = kernels.binned_scatter(x, plain, w, bins, top_k)
+    assert torch.equal(kernels.binned_scatter(x, indices, w, bins, top_k), want)
+    other = bins.clone()
+    other[:-1] = 0
+    assert torch.equal(kernels.binned_scatter(x, indices, w, other, top_k), kernels.binned_scatter(x, plain, w, other, top_k))
+    indices.copy_(indices.flip(0))
+    assert torch.equal(kernels.binned_scatter(x, indices, w, bins, top_k), kernels.binned_scatter(x, plain.flip(0), w, bins, top_k))
+
+
 @pytest.mark.parametrize('sl,hs,ne,top_k,cap', [(1, 8, 1, 1, 1), (77, 520, 3, 2, 5), (300, 2056, 8, 1, 60), (513, 129, 64, 4, 20), (2000, 768, 32, 1, 62)])
 @pytest.mark.parametrize('dtype,w_dtype', [(torch.bfloat16, torch.bfloat16), (torch.float16, torch.float32), (torch.float32, torch.float32), (torch.float16, None)])
 def test_both_gradients_of_binned_scatter_in_one_pass(kernels, sl, hs, ne, top_k, cap, dtype, w_dtype):
