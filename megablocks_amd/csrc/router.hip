@@ -238,10 +238,107 @@ router_backward_kernel(const void* __restrict__ grad_weights_, const void* __res
   }
 }
 
+// out[t] = add[t] + grad_logits[t] @ weight, the input's gradient of the router's linear layer on top of the experts': fp32 sums, rounded
+// once.  What bounds it: one reading of `add` and one writing of `out` (a product of its own and the addition read and write 2 1/2 times as much):
+// 16384 x 1024 and 64 experts 17 us (4.1 TB/s; two passes 17.5 + 17.5), 24576 x 2048 and 16 experts 41 (4.9 TB/s; 36 + 45), 16384 x 768, 32: 12 (18.3 + 12.5).
+// A wave has 64 columns and keeps their weights, all experts', in registers as operands (KT 16-byte pieces for each 16 columns); it then goes
+// through tokens, two sixteens at a time so that eight 16-byte loads are under way.  An operand of 16 columns has every eighth group of four
+// of 32: a lane's results of two products are eight columns in a row then, a 16-byte piece of its token's row of `add` and `out`.
+// ALIGNED: experts % 8 == 0, rows of grad_logits are whole 16-byte pieces.
+constexpr int kInputGradColumns = 64, kInputGradTokens = 32, kInputGradMaxExperts = 128, kInputGradBlocks = 512;
+typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+template <int DT>
+__device__ __forceinline__ f32x4_t mfma_16x16x32(const u32x4_t& a, const u32x4_t& b, const f32x4_t& c) {
+  typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+  typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
+  if constexpr (DT == MBX_BF16) return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
+  else return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, a), __builtin_bit_cast(f16x8_t, b), c, 0, 0, 0);
+}
+template <int DT, int KT, bool ALIGNED>
+__global__ void __launch_bounds__(kTokenThreads)
+router_input_gradient_kernel(const uint16_t* __restrict__ grad_logits, const uint16_t* __restrict__ weight, const uint16_t* __restrict__ add,
+                             int64_t tokens, int hidden, int num_experts, uint16_t* __restrict__ out) {
+  typedef typename Elem<DT>::type E;
+  const int lane = lane_id(), row = lane % 16, group = lane / 16;
+  const int c0 = ((int)blockIdx.x * kTokenWaves + (int)(threadIdx.x / kWave)) * kInputGradColumns;
+  if (c0 >= hidden) return;
+  // eight experts from `first` on of a row of n, past the last one zero
+  const auto pack = [&](const uint16_t* p, int64_t step, int first) {
+    uint32_t v[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) v[q] = p[(first + q < num_experts ? first + q : num_experts - 1) * step];   // one load after the other, no branches
+#pragma unroll
+    for (int q = 0; q < 8; ++q) v[q] = first + q < num_experts ? v[q] : 0u;
+    return u32x4_t{v[0] | v[1] << 16, v[2] | v[3] << 16, v[4] | v[5] << 16, v[6] | v[7] << 16};
+  };
+  struct Rows { u32x4_t g[2][KT], v[2][2]; };
+  const auto fetch = [&](int64_t t0, Rows& r) {
+    auto& g = r.g;
+    auto& v = r.v;
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int64_t t = t0 + 16 * u + row;
+#pragma unroll
+      for (int kt = 0; kt < KT; ++kt) {
+        const int first = 32 * kt + 8 * group;
+        if constexpr (ALIGNED) g[u][kt] = t < tokens && first < num_experts ? *(const u32x4_t*)(grad_logits + t * num_experts + first) : u32x4_t{0, 0, 0, 0};
+        else g[u][kt] = t < tokens ? pack(grad_logits + t * num_experts, 1, first) : u32x4_t{0, 0, 0, 0};
+      }
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const int column = c0 + 32 * i + 8 * group;
+        v[u][i] = t < tokens && column < hidden ? *(const u32x4_t*)(add + t * hidden + column) : u32x4_t{0, 0, 0, 0};
+      }
+    }
+  };
+  int64_t t0 = (int64_t)blockIdx.y * kInputGradTokens;
+  const int64_t step = (int64_t)gridDim.y * kInputGradTokens;
+  Rows next;
+  fetch(t0, next);
+  u32x4_t w[2][2][KT];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+      const int column = c0 + 32 * i + 8 * (row / 4) + 4 * half + row % 4;
+#pragma unroll
+      for (int kt = 0; kt < KT; ++kt) w[i][half][kt] = pack(weight + (column < hidden ? column : 0), hidden, 32 * kt + 8 * group);
+    }
+  for (; t0 < tokens; t0 += step) {
+    const Rows now = next;
+    fetch(t0 + step, next);
+    const auto& g = now.g;
+    const auto& v = now.v;
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int64_t t = t0 + 16 * u + row;
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        f32x4_t acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+        for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+          for (int half = 0; half < 2; ++half) acc[half] = mfma_16x16x32<DT>(w[i][half][kt], g[u][kt], acc[half]);
+        const int column = c0 + 32 * i + 8 * group;
+        if (t >= tokens || column >= hidden) continue;
+        u32x4_t r;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const uint32_t pair = v[u][i][q];
+          const float low = Elem<DT>::to_f32(__builtin_bit_cast(E, (uint16_t)pair)) + acc[q / 2][2 * q % 4];
+          const float high = Elem<DT>::to_f32(__builtin_bit_cast(E, (uint16_t)(pair >> 16))) + acc[q / 2][2 * q % 4 + 1];
+          r[q] = (uint32_t)__builtin_bit_cast(uint16_t, Elem<DT>::from_f32(low)) | (uint32_t)__builtin_bit_cast(uint16_t, Elem<DT>::from_f32(high)) << 16;
+        }
+        *(u32x4_t*)(out + t * hidden + column) = r;
+      }
+    }
+  }
+}
+
 // out[i] = sum over the parts, in fp32, rounded once.  A block takes 64 runs of four values; each of its four waves adds up a
 // quarter of the parts, eight loads under way, and the first puts the quarters together, in order.  What bounds it: one reading of the
 // parts (64 of 64 x 1024, 16.8 MB: 5 us; torch's sum of as many 16-bit values 9.9, and the cast of its result 4.8).
-typedef float f32x4_t __attribute__((ext_vector_type(4)));
 template <int DT>
 __global__ void __launch_bounds__(kTokenThreads)
 sum_parts_kernel(const float* __restrict__ parts, int num_parts, int64_t pitch, void* __restrict__ out_, int64_t n) {
@@ -430,6 +527,38 @@ int mbx_router_backward(const void* grad_weights, const void* grad_scores, const
   hipStream_t s = as_stream(stream);
   MBX_ROUTER_DISPATCH(router_backward_kernel, grad_weights, grad_scores, scores, indices, tokens, num_experts, top_k,
                       norm_p, grad_logits, grad_lse);
+  return launch_status();
+}
+
+int mbx_router_input_gradient(const void* grad_logits, const void* weight, const void* add, int dtype, int64_t tokens, int hidden,
+                              int num_experts, void* out, mbx_stream_t stream) {
+  if (tokens < 0 || hidden <= 0 || num_experts <= 0 || (dtype != MBX_BF16 && dtype != MBX_F16 && dtype != MBX_F32)) return MBX_EINVAL;
+  if (tokens == 0) return 0;
+  if (!grad_logits || !weight || !add || !out) return MBX_EINVAL;
+  if (dtype == MBX_F32 || hidden % 8 || num_experts > kInputGradMaxExperts || (((uintptr_t)add | (uintptr_t)out) & 15u)) return MBX_EUNSUPPORTED;
+  hipStream_t s = as_stream(stream);
+  const bool aligned = num_experts % 8 == 0 && ((uintptr_t)grad_logits & 15u) == 0;
+  // two waves to a SIMD where there are tokens for as many: each reads all experts' weights of its columns first (us with 256 / 512 / 1024 / 2048
+  // workgroups: 16384 x 1024, 64 experts 17.8 / 17.1 / 19.0 / 22.7; 16384 x 768, 32 experts 14.6 / 12.2 / 12.7 / 13.0)
+  const int64_t columns = ceil_div(hidden, kTokenWaves * kInputGradColumns), pieces = ceil_div(tokens, kInputGradTokens), most = ceil_div(kInputGradBlocks, columns);
+  const dim3 grid((unsigned)columns, (unsigned)(pieces < most ? pieces : most));
+#define MBX_INPUT_GRAD(DT, KT)                                                                                                                    \
+  do {                                                                                                                                            \
+    if (aligned) router_input_gradient_kernel<DT, KT, true><<<grid, kTokenThreads, 0, s>>>((const uint16_t*)grad_logits, (const uint16_t*)weight, \
+                                                                                          (const uint16_t*)add, tokens, hidden, num_experts, (uint16_t*)out); \
+    else router_input_gradient_kernel<DT, KT, false><<<grid, kTokenThreads, 0, s>>>((const uint16_t*)grad_logits, (const uint16_t*)weight,        \
+                                                                                   (const uint16_t*)add, tokens, hidden, num_experts, (uint16_t*)out); \
+  } while (0)
+#define MBX_INPUT_GRAD_DT(DT)                        \
+  do {                                               \
+    if (num_experts <= 32) MBX_INPUT_GRAD(DT, 1);    \
+    else if (num_experts <= 64) MBX_INPUT_GRAD(DT, 2); \
+    else MBX_INPUT_GRAD(DT, 4);                      \
+  } while (0)
+  if (dtype == MBX_BF16) MBX_INPUT_GRAD_DT(MBX_BF16);
+  else MBX_INPUT_GRAD_DT(MBX_F16);
+#undef MBX_INPUT_GRAD_DT
+#undef MBX_INPUT_GRAD
   return launch_status();
 }
 

@@ -265,6 +265,63 @@ def test_router_linear_gradients_against_fp64(tokens, hidden, experts, dtype, we
     assert rel_err(weight.grad.double(), g.double().t() @ x.detach().double()) < (sums if exact else rounding)
 
 
+@pytest.mark.parametrize('tokens,hidden,experts', [(1, 8, 1), (31, 72, 8), (33, 264, 12), (65, 64, 32), (1025, 1032, 40), (2000, 328, 33), (5003, 520, 128), (70000, 264, 64)])
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])
+def test_input_gradient_of_the_router_on_top_of_the_experts(tokens, hidden, experts, dtype):
+    """Against fp64: fp32 sums of the terms rounded once (half a step, 2^-8 or 2^-11 of the value's power of two)."""
+    from megablocks_amd.layers import router as r
+    torch.manual_seed(tokens)
+    other = torch.randn(tokens, hidden, device='cuda').to(dtype)
+    weight, grad = torch.randn(experts, hidden, device='cuda').to(dtype), torch.randn(tokens, experts, device='cuda').to(dtype)
+    with torch.no_grad():
+        got = r._input_gradient_on(other, grad, weight)
+    want = other.double() + grad.double() @ weight.double()
+    terms = other.double().abs() + grad.double().abs() @ weight.double().abs()
+    half_step = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+    assert ((got.double() - want).abs() <= half_step * want.abs() * (1 + 1e-3) + (experts + 1) * 2.0 ** -24 * terms + 2.0 ** -25).all()
+
+
+@pytest.mark.parametrize('kind', ['dMoE', 'MoE', 'glu', 'autocast', 'top1'])
+def test_experts_gradient_of_the_tokens_comes_back_through_the_router(monkeypatch, kind):
+    """The layer with one gradient of its input, formed by the router's node, against the layer whose two are added up by autograd: the
+    same but for a rounding less; a hook on the router keeps it to its own gradient."""
+    from megablocks_amd.layers import router as r
+    from megablocks_amd.layers.arguments import Arguments
+    from megablocks_amd.layers.dmoe import dMoE
+    from megablocks_amd.layers.moe import MoE
+    torch.manual_seed(3)
+    autocast = kind == 'autocast'
+    args = Arguments(hidden_size=264, ffn_hidden_size=256, moe_num_experts=8, moe_top_k=1 if kind == 'top1' else 2, device='cuda', bf16=not autocast, fp16=False,
+                     mlp_type='glu' if kind == 'glu' else 'mlp', mlp_impl='grouped', moe_capacity_factor=1, moe_loss_weight=0)
+    layer = (MoE if kind == 'MoE' else dMoE)(args)
+    x = torch.randn(1100, 1, 264, device='cuda').to(torch.float32 if autocast else torch.bfloat16).requires_grad_(True)
+    dy = torch.randn(1100, 1, 264, device='cuda').bfloat16()
+    launched = []
+    launch = r._input_gradient_on
+    monkeypatch.setattr(r, '_input_gradient_on', lambda *a: launched.append(launch(*a)) or launched[-1])
+
+    def gradients():
+        launched.clear()
+        layer.zero_grad()
+        x.grad = None
+        with torch.autocast('cuda', dtype=torch.bfloat16, enabled=autocast):
+            out = layer(x)
+        (out[0] if isinstance(out, tuple) else out).backward(dy)
+        return [x.grad] + [p.grad for p in layer.parameters() if p.grad is not None], [t is not None for t in launched]
+    got, fused = gradients()
+    assert fused == [True]
+    seen = []
+    hook = layer.router.register_full_backward_hook(lambda module, gin, gout: seen.append(gin))
+    want, fused = gradients()
+    hook.remove()
+    assert fused == [] and len(seen) == 1
+    assert len(got) == len(want) > 3
+    for g, w in zip(got, want):
+        assert g.dtype == w.dtype and rel_err(g, w) < 2.0 ** -8
+    for g, w in zip(got[1:], want[1:]):
+        assert torch.equal(g, w)
+
+
 @pytest.mark.parametrize('tokens,hidden', [(4096, 256), (1100, 70)])
 def test_router_products_keep_out_of_the_experts_statistics(monkeypatch, tokens, hidden):
     """Per-launch timing (bench.py) sums up launches by name: those of the router's gradients have names of their own."""
