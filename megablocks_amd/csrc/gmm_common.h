@@ -71,6 +71,15 @@ int gmm_mid(const DmaCall& call);
 constexpr int kMinCutTiles = 32;
 // A cut tile has up to kMaxKSplit parts of at least kMinPartTiles K tiles.
 constexpr int kMaxKSplit = 8, kMinPartTiles = 8;
+// Behind full rounds the tail's tiles are cut along the reduction into three parts and more from kMinTailCutTiles K tiles on, into two from kMinTailHalvesTiles:
+// below, half-height tiles, where a launch has them, take less (8 experts of 1024 rows, [k, 2304 / 2560 / 2816 / 3072], i.e. tails cut into 8 / 4 / 2 / 2 parts, operands out of
+// memory, us cut and not: k = 1024 69 / 50 and 73 / 50 (2 parts); 2048 85 / 80, 95 / 85, 93 / 81, 101 / 84; 4096 160 / 143, 153 / 151, 153 / 145, 162 / 152; 5120 192 / 182,
+// 183 / 193, 188 / 184, 195 / 192; 6144 199 / 213, 205 / 225, 224 / 215, 226 / 229; 8192 245 / 271, 254 / 293, 289 / 280, 302 / 294; 10240 305 / 344, 313 / 365, 354 / 352,
+// 369 / 378; 14336 404 / 467, 436 / 501, 481 / 488, 508 / 544).
+constexpr int kMinTailCutTiles = 80, kMinTailHalvesTiles = 160;
+__host__ __device__ constexpr bool cut_pays(int full_rounds /* 0: there are no half-height tiles to take instead */, int parts, int k_tiles) {
+  return parts >= 2 && (full_rounds == 0 || k_tiles >= (parts >= 3 ? kMinTailCutTiles : kMinTailHalvesTiles));
+}
 
 // NN / NT launches of gmm_dma.h's kernel are tiled with the half-height tile only up to kHalfHeightRows rows per expert on average, and
 // up to kMixedRows unless full tiles with a half-height last one make kMixedRounds rounds (gmm_rows.h).

@@ -1366,7 +1366,7 @@ gmm_rows_kernel(const uint16_t* __restrict__ a, const uint16_t* __restrict__ b, 
       s_ = s_ > kMaxKSplit ? kMaxKSplit : s_;
       s_ = s_ > nk_all / kMinPartTiles ? nk_all / kMinPartTiles : s_;
       s_ = (int64_t)s_ * rest > ws_capacity ? ws_capacity / rest : s_;
-      ksplit = s_ < 2 ? 1 : s_;
+      ksplit = cut_pays(kSplit ? full_rounds : 0, s_, nk_all) ? s_ : 1;
     }
   }
   const bool split = ksplit == 1 && kSplit && rest > 0 && 2 * rest <= P;

@@ -51,6 +51,10 @@ def _sizes(groups, rows, seed, empty=()):
     return sizes
 
 
+def _units():
+    return torch.cuda.get_device_properties(0).multi_processor_count
+
+
 def _ref_gpu(a, b, sizes, trans_a, trans_b):
     a, b = a.float(), b.float()
     outs, start = [], 0
@@ -352,6 +356,20 @@ def test_gmm_tail_cut_along_the_reduction(gg, row_tiles, col_tiles, k, dtype):
     assert torch.equal(out, plain)
     assert _lib.lib.mbx_gmm_ws(_lib.ptr(a), _lib.ptr(b), _lib.ptr(a2), None, _lib.ptr(out), _lib.dtype_of(a), _lib.ptr(bins), groups,
                                rows, k, n, _lib.NN, None, 0, _lib.stream()) == _lib.EINVAL
+
+
+@pytest.mark.parametrize('column_tiles,k_tiles,cut', [(20, 79, False), (20, 80, True), (24, 159, False), (24, 160, True)])   # tails of 64 and 128 tiles: four parts, two
+def test_gmm_tail_behind_full_rounds_is_cut_along_long_reductions_only(gg, monkeypatch, column_tiles, k_tiles, cut):
+    """Sixteen row tiles: a full round and a tail.  Not cut, the launch computes what it does without a workspace, to the bit; cut, another order of the sums."""
+    sizes, k, n = torch.tensor([1024] * 4), 64 * k_tiles, 256 * column_tiles
+    torch.manual_seed(k_tiles)
+    a = torch.randn(4096, k, device='cuda').bfloat16()
+    b = torch.empty(4, k, n, device='cuda', dtype=torch.bfloat16).normal_(0, k ** -0.5)
+    got = gg.gmm(a, b, sizes)
+    ref = _ref_gpu(a, b, sizes, False, False)
+    assert rel_err(got, ref) < TOL and max_block_err(got, ref) < 2 * TOL
+    monkeypatch.setattr(gg, 'GMM_WORKSPACE', False)
+    assert torch.equal(gg.gmm(a, b, sizes), got) != (cut and _units() == 256)
 
 
 MIXED_ROWS = [  # per-expert row counts around the boundaries between full (256-row) and half-height (128-row) tiles
