@@ -186,7 +186,7 @@ class ParallelDroplessMLP(moe.ParallelMLP):
     def _one_call_step(self, x, expert_weights, top_experts):
         """grouped_forward_once as one node (gg.experts_step), where the layer and its experts are the built-in ones, nothing is traced
         or transformed, nobody looks at the experts module by itself and a gradient is recorded; else None."""
-        known = self._one_call_experts()
+        known = self._one_call_experts() if x.dtype in (torch.bfloat16, torch.float16) else None
         if known is None or router._has_hooks(self.mlp) or not _only_computed(autocast=True):
             return None
         act, w1, v1, w2 = known

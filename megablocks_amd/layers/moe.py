@@ -162,8 +162,9 @@ class MoE(torch.nn.Module):
         # LearnedRouter hangs the int32 copy of its indices, which its kernel writes anyway, on the int64 tensor it
         # returns; the routing takes that copy (no cast, moe.py:160) unless something has replaced or rewritten the
         # indices on the way here.
-        if type(self.router) is router.LearnedRouter and self.router.shares(x):
-            scores, expert_weights, top_experts, x = self.router.forward_and_tokens(x)
+        module = self.router
+        if torch.is_grad_enabled() and type(module) is router.LearnedRouter and module.shares(x):
+            scores, expert_weights, top_experts, x = module.forward_and_tokens(x)
         else:
-            scores, expert_weights, top_experts = self.router(x)
+            scores, expert_weights, top_experts = module(x)
         return self.experts(x, scores, expert_weights, router.int32_indices(top_experts))

@@ -405,9 +405,7 @@ class LearnedRouter(torch.nn.Module):
         return torch.topk(scores, self.args.moe_top_k, dim=-1)
 
     def forward(self, x: torch.Tensor):
-        return self._attach(*self.route(x))
-
-    def _attach(self, scores, expert_weights, expert_indices, expert_indices32):
+        scores, expert_weights, expert_indices, expert_indices32 = self.route(x)
         if expert_indices32 is not None:
             # out of band: the same indices as int32, valid while the int64 tensor is the one returned here, unmodified
             expert_indices._mbx_int32 = (expert_indices32, expert_indices._version)
@@ -422,20 +420,26 @@ class LearnedRouter(torch.nn.Module):
 
     def forward_and_tokens(self, x: torch.Tensor):
         """forward(x), and x again for the experts: their gradient of it comes back through the router's (_RouterLinearAndTokens)."""
-        *routed, tokens = self._route(x, _RouterLinearAndTokens)
-        return (*self._attach(*routed), tokens.view(x.shape))
+        tokens = None
+
+        def linear(x2d, weight):
+            nonlocal tokens
+            logits, tokens = _RouterLinearAndTokens.apply(x2d, weight)
+            return logits
+
+        scores, expert_weights, expert_indices, expert_indices32 = self.route(x, linear)
+        if expert_indices32 is not None:   # as in forward
+            expert_indices._mbx_int32 = (expert_indices32, expert_indices._version)
+        return scores, expert_weights, expert_indices, x if tokens is None else tokens.view(x.shape)
 
     @staticmethod
     def _takes_linear(x: torch.Tensor) -> bool:
         return x.is_cuda and x.dtype in (torch.bfloat16, torch.float16) and x.numel() >= 4 * _RouterLinear.PIECE_ROWS * x.shape[-1]
 
-    def route(self, x: torch.Tensor):
+    def route(self, x: torch.Tensor, linear=_RouterLinear.apply):
         """forward's (scores, expert_weights, expert_indices) and, where the router kernel wrote them, the indices as
-        int32 (else None): the layer routes with those and skips the cast of moe.py:160."""
-        return self._route(x)[:4]
-
-    def _route(self, x: torch.Tensor, linear=_RouterLinear):
-        """route, and what `linear` has returned besides the logits (None where another product has formed them)."""
+        int32 (else None): the layer routes with those and skips the cast of moe.py:160.  linear: what forms the logits of more than a few
+        16-bit rows on the GPU."""
         if self.training and self.args.moe_jitter_eps is not None:
             x = x * self.jitter(x)
         x2d = x.view(-1, x.shape[-1])
@@ -443,12 +447,9 @@ class LearnedRouter(torch.nn.Module):
         if FUSED_SOFTMAX_TOPK and args.moe_zloss_weight == 0 and not args.uniform_expert_assignment:
             for node in (_LinearSoftmaxTopK, _RecordedLinearSoftmaxTopK):   # without gradients, with
                 if node.supported(x2d, self.layer, args.moe_top_k):
-                    return (*node.apply(x2d, self.layer.weight, args.moe_top_k, args.moe_normalize_expert_weights or 0), None)
-        tokens = None
+                    return node.apply(x2d, self.layer.weight, args.moe_top_k, args.moe_normalize_expert_weights or 0)
         if self._takes_linear(x2d):
-            logits = linear.apply(x2d, self.layer.weight)
-            if linear is _RouterLinearAndTokens:
-                logits, tokens = logits
+            logits = linear(x2d, self.layer.weight)
         else:
             logits = self.layer(x2d)
         saved_logits, lse = logits, None
@@ -470,4 +471,4 @@ class LearnedRouter(torch.nn.Module):
         if self.args.uniform_expert_assignment:
             expert_indices = _UniformExpertAssignment.apply(expert_indices, self.args.moe_num_experts)
             expert_indices32 = None
-        return scores, expert_weights, expert_indices, expert_indices32, tokens
+        return scores, expert_weights, expert_indices, expert_indices32
