@@ -201,17 +201,22 @@ __global__ void fill_kernel(int32_t* __restrict__ p, int64_t n, int32_t v) {
 
 // Zero-fill the rows of an expert-major buffer that no slot owns (padding; a sorted position whose index is not a
 // slot), for the kernels that write such a buffer slot by slot.  Lane l of a wave looks at row base + l, and the
-// wave clears the rows its ballot names; wave `wave_id` of `waves` takes every waves-th group of 64 rows.
+// wave clears the rows its ballot names; wave `wave_id` of `waves` takes every waves-th group of rows.  With padding the groups are
+// of twice a wave's share of the rows, so that half of the waves or more look and none is left with 64 rows to clear when the others are done
+// (2000 tokens of 2056 columns, top-4 of 64 experts padded to 128, fp16: gather 25.1 -> 17.6 us; 4191 of 4096, top-8 of 128: 90 -> 85); without it
+// there is next to nothing to clear and 64 rows cost one look.
 template <int DT>
 __device__ __forceinline__ void zero_unowned_rows(typename Elem<DT>::type* __restrict__ out, int64_t out_rows, int hidden,
                                                   const int32_t* __restrict__ indices, const int32_t* __restrict__ bins,
                                                   const int32_t* __restrict__ padded_bins, int num_bins, int n_slots,
                                                   int64_t wave_id, int64_t waves) {
   const int lane = lane_id();
-  for (int64_t base = wave_id * kWave; base < out_rows; base += waves * kWave) {
+  const int64_t share = (out_rows + waves - 1) / waves;
+  const int group = padded_bins != nullptr && 2 * share < kWave ? (int)(2 * share) : kWave;
+  for (int64_t base = wave_id * group; base < out_rows; base += waves * group) {
     const int64_t row = base + lane;
     bool empty = false;
-    if (row < out_rows) {
+    if (lane < group && row < out_rows) {
       const int pos = slot_of_row((int)row, bins, padded_bins, num_bins, n_slots);
       const int sl = pos >= 0 ? indices[pos] : -1;
       empty = sl < 0 || sl >= n_slots;
@@ -228,9 +233,12 @@ __device__ __forceinline__ void zero_unowned_rows(typename Elem<DT>::type* __res
 // ------------------------------------------------------------------ gather, one wave per token
 // The token's row is read once (the row-major kernel reads it once per slot, from wherever in the expert-major
 // order that slot landed) and written to the rows of its top_k slots, inv[t * top_k + j] (-1: none).  Then
-// the rows that no slot owns are zero-filled.  The stores are non-temporal (the expert-major copy is top_k times the
-// tokens and is not read by this kernel: keeping it out of the caches is worth a fifth of the kernel's time); the loads
-// are not: the tokens are a matrix that fits the last-level cache and that a kernel before or after this one touches as
+// the rows that no slot owns are zero-filled.  What bounds it: the stores, 5.0 TB/s of reads and writes from memory, 5.8 in a layer's step.
+// Nothing here is non-temporal.  Not the stores: past the caches they are slower themselves, more so where rows are no whole 128-byte
+// lines, whose ends then leave in pieces, and the kernel that reads the rows next finds none of them in the last-level cache (us, non-temporal / plain:
+// 32768 rows of 4096 bytes to 6 x as many 190 / 162, of 4080 bytes, out of memory, 266 / 208; 16384 of 2048 bytes to 4 x as many 27.5 and the
+// combine that reads them 40.7 / 26.6 and 33.3; 57407 of 1088 bytes to twice as many 30.2 and 54.2 / 35.4 and 49.4).  Not the loads: the
+// tokens are a matrix that fits the last-level cache and that a kernel before or after this one touches as
 // well (the producer of the tokens, the router; in the backward pass the router-weight gradient reads the same rows of
 // the output gradient right afterwards), and a non-temporal load does not find them there (32768 rows of 4 KiB into
 // 6 x as many: 153 us from a hot source with plain loads, 187 us with non-temporal ones).
@@ -281,7 +289,7 @@ gather_tokens_kernel(const void* __restrict__ x_, int64_t tokens, int hidden, in
             for (int q = 0; q < EV; ++q) f[q] *= scale;
             w = Vec16<DT>::pack(f);
           }
-          __builtin_nontemporal_store(w, dst + c);
+          dst[c] = w;
         }
       }
     }

@@ -172,6 +172,31 @@ def test_gather_and_padded_gather(kernels, sl, hs, ne, top_k, dtype):
     assert torch.equal(got.cpu(), oracle.padded_gather(x, indices, bin_ids, w, bins, pbins, top_k))
 
 
+@pytest.mark.parametrize('tokens,ne,top_k,block', [
+    (3, 2, 2, 128),        # a wave's share of the rows is 64 and more: groups of 64
+    (10, 64, 8, 128),
+    (1000, 128, 8, 128),   # 17 rows: groups of 34
+    (4096, 4, 2, 128),     # 3 rows: groups of 6
+    (4096, 2, 2, 2),       # next to no padding
+])
+def test_padded_gather_clears_every_row_no_slot_owns(kernels, tokens, ne, top_k, block):
+    x = torch.randn(tokens, 72).bfloat16()
+    ids = torch.rand(tokens, ne).argsort(dim=1)[:, :top_k].flatten().int()
+    bin_ids, indices = oracle.sort(ids)
+    indices[::7] = tokens * top_k + 5      # a sorted position that is no slot: its row is one of zeros too
+    counts = oracle.histogram(ids, ne)
+    bins, pbins = counts.cumsum(0).int(), ((counts + block - 1) // block * block).cumsum(0).int()
+    poison = torch.full((int(pbins[-1]), 72), float('nan'), dtype=x.dtype, device='cuda')
+    del poison                             # the output's memory
+    got = kernels.padded_gather(dev(x), dev(indices), dev(bin_ids), None, dev(bins), dev(pbins), top_k).cpu()
+    want = torch.zeros_like(got)
+    for i, s in enumerate(indices.tolist()):
+        e = int(bin_ids[i])
+        if s < tokens * top_k:
+            want[i - (int(bins[e - 1]) if e else 0) + (int(pbins[e - 1]) if e else 0)] = x[s // top_k]
+    assert torch.equal(got, want)
+
+
 @pytest.mark.parametrize('sl,hs,ne,top_k', PERMUTE_CASES)
 @pytest.mark.parametrize('dtype', [torch.float16, torch.bfloat16, torch.float32])
 def test_scatter_and_padded_scatter(kernels, sl, hs, ne, top_k, dtype):
