@@ -462,9 +462,10 @@ int mbx_router_backward(const void* grad_weights, const void* grad_scores, const
 
 /* out[t, :] = add[t, :] + grad_logits[t, :] @ weight, fp32 sums rounded once: the input gradient of the router's linear layer (weight [num_experts, hidden],
  * megablocks/layers/router.py:96) added to the experts'.  All contiguous, 16-bit, hidden a multiple of 8, at most 128 experts, add and out 16-byte
- * aligned (else MBX_EUNSUPPORTED).  out must not overlap the others. */
+ * aligned (else MBX_EUNSUPPORTED).  out must not overlap the others.  padded (or NULL): gets grad_logits with zeros up to a multiple of 8 experts,
+ * [tokens, that many], 16-byte aligned. */
 int mbx_router_input_gradient(const void* grad_logits, const void* weight, const void* add, int dtype, int64_t tokens, int hidden,
-                              int num_experts, void* out, mbx_stream_t stream);
+                              int num_experts, void* out, void* padded, mbx_stream_t stream);
 
 /* out[i] = parts[0][i] + ... + parts[num_parts - 1][i] for i < n, in fp32, rounded once to `dtype`; part p starts at parts + p pitch.
  * The weight gradient of the router's linear layer from those of equal pieces of the batch (mbx_gmm_tn_f32, one group a

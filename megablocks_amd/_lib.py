@@ -76,7 +76,7 @@ _SIGNATURES = {
     'mbx_loss_scratch_bytes': (_sz, [_i64]),
     'mbx_loss_sum': (_i, [_vp, _i, _vp, _i64, _i, ctypes.c_float, _vp, _vp, _vp]),
     'mbx_loss_gradient': (_i, [_vp, _vp, _i, _vp, _i64, _i, ctypes.c_float, _vp, _vp]),
-    'mbx_router_input_gradient': (_i, [_vp, _vp, _vp, _i, _i64, _i, _i, _vp, _vp]),
+    'mbx_router_input_gradient': (_i, [_vp, _vp, _vp, _i, _i64, _i, _i, _vp, _vp, _vp]),
     'mbx_sum_parts': (_i, [_vp, _i, _i64, _vp, _i, _i64, _vp]),
     'mbx_router_backward': (_i, [_vp, _vp, _vp, _vp, _i, _i64, _i, _i, ctypes.c_float, _vp, _vp, _vp]),
 }

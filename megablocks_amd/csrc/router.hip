@@ -244,7 +244,9 @@ router_backward_kernel(const void* __restrict__ grad_weights_, const void* __res
 // A wave has 64 columns and keeps their weights, all experts', in registers as operands (KT 16-byte pieces for each 16 columns); it then goes
 // through tokens, two sixteens at a time so that eight 16-byte loads are under way.  An operand of 16 columns has every eighth group of four
 // of 32: a lane's results of two products are eight columns in a row then, a 16-byte piece of its token's row of `add` and `out`.
-// ALIGNED: experts % 8 == 0, rows of grad_logits are whole 16-byte pieces.
+// ALIGNED: experts % 8 == 0, rows of grad_logits are whole 16-byte pieces.  Where they are not, the rows with zeros up to whole pieces, which the
+// kernels have in registers, can be written to `padded` on the way: the weight's gradient wants them like that (a fill and a strided copy of
+// 10 us otherwise, 3001 tokens, 12 experts).
 constexpr int kInputGradColumns = 64, kInputGradTokens = 32, kInputGradMaxExperts = 128, kInputGradBlocks = 512;
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
@@ -258,7 +260,7 @@ __device__ __forceinline__ f32x4_t mfma_16x16x32(const u32x4_t& a, const u32x4_t
 template <int DT, int KT, bool ALIGNED>
 __global__ void __launch_bounds__(kTokenThreads)
 router_input_gradient_kernel(const uint16_t* __restrict__ grad_logits, const uint16_t* __restrict__ weight, const uint16_t* __restrict__ add,
-                             int64_t tokens, int hidden, int num_experts, uint16_t* __restrict__ out) {
+                             int64_t tokens, int hidden, int num_experts, uint16_t* __restrict__ out, uint16_t* __restrict__ padded) {
   typedef typename Elem<DT>::type E;
   const int lane = lane_id(), row = lane % 16, group = lane / 16;
   const int c0 = ((int)blockIdx.x * kTokenWaves + (int)(threadIdx.x / kWave)) * kInputGradColumns;
@@ -310,6 +312,19 @@ router_input_gradient_kernel(const uint16_t* __restrict__ grad_logits, const uin
     fetch(t0 + step, next);
     const auto& g = now.g;
     const auto& v = now.v;
+    if constexpr (!ALIGNED) {
+      if (padded != nullptr && c0 == 0) {
+        const int pitch = (num_experts + 7) & ~7;
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+          for (int kt = 0; kt < KT; ++kt) {
+            const int64_t t = t0 + 16 * u + row;
+            const int first = 32 * kt + 8 * group;
+            if (t < tokens && first < pitch) *(u32x4_t*)(padded + t * pitch + first) = g[u][kt];
+          }
+      }
+    }
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
       const int64_t t = t0 + 16 * u + row;
@@ -531,13 +546,13 @@ int mbx_router_backward(const void* grad_weights, const void* grad_scores, const
 }
 
 int mbx_router_input_gradient(const void* grad_logits, const void* weight, const void* add, int dtype, int64_t tokens, int hidden,
-                              int num_experts, void* out, mbx_stream_t stream) {
+                              int num_experts, void* out, void* padded, mbx_stream_t stream) {
   if (tokens < 0 || hidden <= 0 || num_experts <= 0 || (dtype != MBX_BF16 && dtype != MBX_F16 && dtype != MBX_F32)) return MBX_EINVAL;
   if (tokens == 0) return 0;
   if (!grad_logits || !weight || !add || !out) return MBX_EINVAL;
-  if (dtype == MBX_F32 || hidden % 8 || num_experts > kInputGradMaxExperts || (((uintptr_t)add | (uintptr_t)out) & 15u)) return MBX_EUNSUPPORTED;
+  if (dtype == MBX_F32 || hidden % 8 || num_experts > kInputGradMaxExperts || (((uintptr_t)add | (uintptr_t)out | (uintptr_t)padded) & 15u)) return MBX_EUNSUPPORTED;
   hipStream_t s = as_stream(stream);
-  const bool aligned = num_experts % 8 == 0 && ((uintptr_t)grad_logits & 15u) == 0;
+  const bool aligned = num_experts % 8 == 0 && ((uintptr_t)grad_logits & 15u) == 0 && !padded;
   // two waves to a SIMD where there are tokens for as many: each reads all experts' weights of its columns first (us with 256 / 512 / 1024 / 2048
   // workgroups: 16384 x 1024, 64 experts 17.8 / 17.1 / 19.0 / 22.7; 16384 x 768, 32 experts 14.6 / 12.2 / 12.7 / 13.0)
   const int64_t columns = ceil_div(hidden, kTokenWaves * kInputGradColumns), pieces = ceil_div(tokens, kInputGradTokens), most = ceil_div(kInputGradBlocks, columns);
@@ -545,9 +560,9 @@ int mbx_router_input_gradient(const void* grad_logits, const void* weight, const
 #define MBX_INPUT_GRAD(DT, KT)                                                                                                                    \
   do {                                                                                                                                            \
     if (aligned) router_input_gradient_kernel<DT, KT, true><<<grid, kTokenThreads, 0, s>>>((const uint16_t*)grad_logits, (const uint16_t*)weight, \
-                                                                                          (const uint16_t*)add, tokens, hidden, num_experts, (uint16_t*)out); \
+                                                                                          (const uint16_t*)add, tokens, hidden, num_experts, (uint16_t*)out, (uint16_t*)nullptr); \
     else router_input_gradient_kernel<DT, KT, false><<<grid, kTokenThreads, 0, s>>>((const uint16_t*)grad_logits, (const uint16_t*)weight,        \
-                                                                                   (const uint16_t*)add, tokens, hidden, num_experts, (uint16_t*)out); \
+                                                                                   (const uint16_t*)add, tokens, hidden, num_experts, (uint16_t*)out, (uint16_t*)padded); \
   } while (0)
 #define MBX_INPUT_GRAD_DT(DT)                        \
   do {                                               \

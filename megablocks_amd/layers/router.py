@@ -179,16 +179,19 @@ class _RouterLinearAndTokens(torch.autograd.Function):
         if grad is None:
             return grad_tokens, None
         grad = grad.to(x.dtype)
-        dx = _input_gradient_on(grad_tokens, grad, weight) if want_x and grad_tokens is not None else None
+        tokens, experts = grad.shape
+        padded = torch.empty((tokens, experts + -experts % 8), dtype=grad.dtype, device=grad.device) if want_weight and experts % 8 else None
+        dx = _input_gradient_on(grad_tokens, grad, weight, padded) if want_x and grad_tokens is not None else None
         fused = dx is not None
-        plain, dw = _linear_gradients(grad, x, weight, ctx.weight_dtype, want_x and not fused, want_weight)
+        plain, dw = _linear_gradients(grad, x, weight, ctx.weight_dtype, want_x and not fused, want_weight, padded if fused else None)
         if not fused and want_x:
             dx = plain if grad_tokens is None else plain + grad_tokens
         return dx, dw
 
 
-def _input_gradient_on(other, grad, weight):
-    """other + grad @ weight, in one pass over `other`, rounded once; None where the kernel does not take the call."""
+def _input_gradient_on(other, grad, weight, padded=None):
+    """other + grad @ weight, in one pass over `other`, rounded once; None where the kernel does not take the call.  padded: gets `grad` with zeros up to
+    a multiple of 8 columns."""
     if torch.is_grad_enabled() or not all(type(t) is torch.Tensor and _has_memory(t) for t in (other, grad)):
         return None
     tokens, experts = grad.shape
@@ -198,7 +201,7 @@ def _input_gradient_on(other, grad, weight):
     grad, out = grad.contiguous(), torch.empty_like(other)
     with _lib.device_of(other):
         _lib.check(_lib.lib.mbx_router_input_gradient(_lib.ptr(grad), _lib.ptr(weight), _lib.ptr(other), _lib.dtype_of(other), tokens, other.shape[1],
-                                                      experts, _lib.ptr(out), _lib.stream()), 'router_input_gradient')
+                                                      experts, _lib.ptr(out), _lib.ptr(padded), _lib.stream()), 'router_input_gradient')
     return out
 
 
@@ -214,8 +217,9 @@ def _has_memory(t: torch.Tensor) -> bool:
     return True
 
 
-def _linear_gradients(grad, x, weight, weight_dtype, want_x, want_weight):
-    """(dx, dweight) of `x @ weight^T`, all 16-bit of one type on the GPU; dweight in `weight_dtype`."""
+def _linear_gradients(grad, x, weight, weight_dtype, want_x, want_weight, padded=None):
+    """(dx, dweight) of `x @ weight^T`, all 16-bit of one type on the GPU; dweight in `weight_dtype`.  padded: `grad` with zeros up to a multiple of
+    8 experts, where the caller has it."""
     from megablocks_amd import grouped_gemm_util as gg
     if torch.is_grad_enabled() or not _has_memory(grad):
         # a backward that is differentiated itself (create_graph), or runs over a batch of gradients at once (is_grads_batched)
@@ -232,7 +236,7 @@ def _linear_gradients(grad, x, weight, weight_dtype, want_x, want_weight):
     if want_weight:
         pieces = sizes.shape[0]
         if experts % 8:
-            grad = torch.nn.functional.pad(grad, (0, -experts % 8))
+            grad = torch.nn.functional.pad(grad, (0, -experts % 8)) if padded is None else padded
         # [pieces, E, h]; a single piece's sums are rounded by the product itself
         parts = gg.weight_gradient(grad, x.contiguous(), sizes, torch.float32 if pieces > 1 else None, _record_as='router_wgrad')
         if pieces == 1 or parts.dtype != torch.float32:

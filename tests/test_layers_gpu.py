@@ -281,6 +281,21 @@ def test_input_gradient_of_the_router_on_top_of_the_experts(tokens, hidden, expe
     assert ((got.double() - want).abs() <= half_step * want.abs() * (1 + 1e-3) + (experts + 1) * 2.0 ** -24 * terms + 2.0 ** -25).all()
 
 
+@pytest.mark.parametrize('tokens,experts', [(1, 1), (33, 12), (1031, 4), (77, 36), (40, 127)])
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])
+def test_input_gradient_of_the_router_leaves_padded_rows(tokens, experts, dtype):
+    """Rows of no whole 16-byte pieces come back with zeros up to that, and nothing behind the last."""
+    from megablocks_amd.layers import router as r
+    torch.manual_seed(tokens)
+    other = torch.randn(tokens, 520, device='cuda').to(dtype)
+    weight, grad = torch.randn(experts, 520, device='cuda').to(dtype), torch.randn(tokens, experts, device='cuda').to(dtype)
+    wide = torch.full((tokens + 16, experts + -experts % 8), float('nan'), device='cuda', dtype=dtype)
+    with torch.no_grad():
+        got = r._input_gradient_on(other, grad, weight, wide[:tokens])
+        assert torch.equal(got, r._input_gradient_on(other, grad, weight))
+    assert torch.equal(wide[:tokens], torch.nn.functional.pad(grad, (0, -experts % 8))) and wide[tokens:].isnan().all()
+
+
 @pytest.mark.parametrize('kind', ['dMoE', 'MoE', 'glu', 'autocast', 'top1'])
 def test_experts_gradient_of_the_tokens_comes_back_through_the_router(monkeypatch, kind):
     """The layer with one gradient of its input, formed by the router's node, against the layer whose two are added up by autograd: the
