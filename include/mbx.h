@@ -328,6 +328,10 @@ int mbx_gmm_hidden(const void* x, int64_t x_rows, const int32_t* indices, int to
 int mbx_gmm_scatter(const void* a, const void* b, void* c, void* out, int dtype, const int32_t* bins, int num_groups,
                     int64_t rows, int k, int n, const int32_t* indices, const void* weights, int w_dtype, int64_t tokens,
                     mbx_stream_t stream);
+/* The same with a workspace, as mbx_gmm_ws: bit-identical to mbx_gmm_ws with it followed by mbx_scatter where the same kernel takes both. */
+int mbx_gmm_scatter_ws(const void* a, const void* b, void* c, void* out, int dtype, const int32_t* bins, int num_groups,
+                       int64_t rows, int k, int n, const int32_t* indices, const void* weights, int w_dtype, int64_t tokens,
+                       void* workspace, size_t workspace_bytes, mbx_stream_t stream);
 
 /* What follows the router in the dropless layer's forward where no gradient is recorded (megablocks/layers/dmoe.py:239-280 over
  * mlp.py:499-523 / glu.py:173-205), enqueued by one call: mbx_route, mbx_gmm_hidden, mbx_gmm_ws and mbx_scatter (with fused_combine

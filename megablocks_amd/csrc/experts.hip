@@ -123,7 +123,7 @@ int mbx_experts_forward(const void* x, int64_t tokens, int hidden_size, int dtyp
   }
   if (rc) return rc;
   if (top_k == 1 && fused_combine) {
-    rc = mbx_gmm_scatter(h, w2, nullptr, out, dtype, bins, num_experts, slots, ffn, hidden_size, indices, weights, w_dtype, tokens, stream);
+    rc = mbx_gmm_scatter_ws(h, w2, nullptr, out, dtype, bins, num_experts, slots, ffn, hidden_size, indices, weights, w_dtype, tokens, workspace, workspace_bytes, stream);
     if (rc != MBX_EUNSUPPORTED) return rc;
   }
   rc = mbx_gmm_ws(h, w2, nullptr, nullptr, y, dtype, bins, num_experts, slots, ffn, hidden_size, MBX_NN, workspace, workspace_bytes, stream);
@@ -185,7 +185,7 @@ int mbx_experts_step_forward(const void* x, int64_t tokens, int hidden_size, int
   }
   if (rc) return rc;
   if (top_k == 1 && flags & MBX_STEP_COMBINE) {
-    rc = mbx_gmm_scatter(h, w2, flags & MBX_STEP_KEEP_PRODUCT ? y : nullptr, out, dtype, bins, num_experts, slots, ffn, hidden_size, indices, weights, w_dtype, tokens, stream);
+    rc = mbx_gmm_scatter_ws(h, w2, flags & MBX_STEP_KEEP_PRODUCT ? y : nullptr, out, dtype, bins, num_experts, slots, ffn, hidden_size, indices, weights, w_dtype, tokens, workspace, workspace_bytes, stream);
     if (rc != MBX_EUNSUPPORTED) return rc;
   }
   rc = mbx_gmm_ws(h, w2, nullptr, nullptr, y, dtype, bins, num_experts, slots, ffn, hidden_size, MBX_NN, workspace, workspace_bytes, stream);

@@ -852,6 +852,12 @@ int mbx_gmm_hidden(const void* x, int64_t x_rows, const int32_t* indices, int to
 int mbx_gmm_scatter(const void* a, const void* b, void* c, void* out, int dtype, const int32_t* bins, int num_groups,
                     int64_t rows, int k, int n, const int32_t* indices, const void* weights, int w_dtype, int64_t tokens,
                     mbx_stream_t stream) {
+  return mbx_gmm_scatter_ws(a, b, c, out, dtype, bins, num_groups, rows, k, n, indices, weights, w_dtype, tokens, nullptr, 0, stream);
+}
+
+int mbx_gmm_scatter_ws(const void* a, const void* b, void* c, void* out, int dtype, const int32_t* bins, int num_groups,
+                       int64_t rows, int k, int n, const int32_t* indices, const void* weights, int w_dtype, int64_t tokens,
+                       void* workspace, size_t workspace_bytes, mbx_stream_t stream) {
   if (num_groups < 0 || rows < 0 || k < 0 || n < 0 || tokens < 0) return MBX_EINVAL;
   if (dtype != MBX_BF16 && dtype != MBX_F16 && dtype != MBX_F32) return MBX_EINVAL;
   if (weights && w_dtype != MBX_BF16 && w_dtype != MBX_F16 && w_dtype != MBX_F32) return MBX_EINVAL;
@@ -872,6 +878,7 @@ int mbx_gmm_scatter(const void* a, const void* b, void* c, void* out, int dtype,
   call.epi = dma::kEpiCombine;
   call.extra = out;
   call.combine = combine;
+  call.ws = Workspace{workspace, workspace_bytes};
   return gmm_dma(call);
 }
 

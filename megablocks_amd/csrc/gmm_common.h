@@ -39,7 +39,7 @@ struct GatherRows {
 //   epi / extra / out2: an epilogue (dma::kEpi*) and its second output / input, third output; kEpiDglu*: a2 is x2; kEpiGlu*: b2 is
 //   the second matrix;
 //   gather: rows of `a` (NT; no epilogue, kEpiAct or kEpiGlu*) or of `b` (TN) picked through the sorted assignments;
-//   ws: device memory the launch may use for the parts of tiles it cuts along the reduction (NN without epilogue).
+//   ws: device memory the launch may use for the parts of tiles it cuts along the reduction (NN without epilogue or with the combine).
 struct DmaCall {
   const void *a, *b;
   void* c;
@@ -77,8 +77,14 @@ constexpr int kMaxKSplit = 8, kMinPartTiles = 8;
 // 183 / 193, 188 / 184, 195 / 192; 6144 199 / 213, 205 / 225, 224 / 215, 226 / 229; 8192 245 / 271, 254 / 293, 289 / 280, 302 / 294; 10240 305 / 344, 313 / 365, 354 / 352,
 // 369 / 378; 14336 404 / 467, 436 / 501, 481 / 488, 508 / 544).
 constexpr int kMinTailCutTiles = 80, kMinTailHalvesTiles = 160;
-__host__ __device__ constexpr bool cut_pays(int full_rounds /* 0: there are no half-height tiles to take instead */, int parts, int k_tiles) {
-  return parts >= 2 && (full_rounds == 0 || k_tiles >= (parts >= 3 ? kMinTailCutTiles : kMinTailHalvesTiles));
+// Launches of half-height tiles only have nothing to take instead, but two parts pay from kMinHalfHeightHalvesTiles K tiles on (160 launches, 4 - 128
+// experts of 30 - 320 rows, with the combine; cut / not: two parts of up to 23 K tiles 1.035, 24 - 31 1.015, 32 - 39 0.99, 40 - 47 0.96, beyond 0.93; three 0.96 - 0.86,
+// more 0.92 - 0.72).
+constexpr int kMinHalfHeightHalvesTiles = 40;
+__host__ __device__ constexpr bool cut_pays(bool half_height_only, int full_rounds, int parts, int k_tiles) {
+  if (parts < 2 || full_rounds == 0) return parts >= 2;
+  if (half_height_only) return parts >= 3 || k_tiles >= kMinHalfHeightHalvesTiles;
+  return k_tiles >= (parts >= 3 ? kMinTailCutTiles : kMinTailHalvesTiles);
 }
 
 // NN / NT launches of gmm_dma.h's kernel are tiled with the half-height tile only up to kHalfHeightRows rows per expert on average, and

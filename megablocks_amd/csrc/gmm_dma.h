@@ -1352,13 +1352,13 @@ gmm_rows_kernel(const uint16_t* __restrict__ a, const uint16_t* __restrict__ b, 
   // The last, partly filled round.  Its `rest` tiles leave P - rest compute units idle for a whole tile's time, which
   // with long reductions and few rounds is a large part of the launch (a Mixtral-shaped second product: 1088 tiles on
   // 256 compute units, 4.25 rounds).  When at most half of the compute units would be busy:
-  //   * with a workspace (kSplitK launches: NN, no epilogue): every tail tile is cut along the reduction into
+  //   * with a workspace (kSplitK launches: NN, no epilogue or the combine): every tail tile is cut along the reduction into
   //     `ksplit` = P / rest parts, one per workgroup, each a full-size tile over a `ksplit`-th of the K tiles.  A part
   //     writes its fp32 accumulators to the workspace and counts itself in; the workgroup that finds it was the last
   //     adds the parts up in part order (so the sum does not depend on who was last), rounds and stores the tile.
   //     Nobody waits for anybody.  The tail then takes 1 / ksplit of a round plus the reduction;
   //   * else the tail's tiles are cut into two half-height tiles each (TS), which take 0.7 of a full tile's time.
-  constexpr bool kSplitK = B_MC && EPI == kEpiNone && !GATHER;
+  constexpr bool kSplitK = B_MC && (EPI == kEpiNone || EPI == kEpiCombine) && !GATHER;
   int ksplit = 1;
   if constexpr (kSplitK) {
     if (ws_parts != nullptr && rest > 0 && 2 * rest <= P) {
@@ -1366,7 +1366,7 @@ gmm_rows_kernel(const uint16_t* __restrict__ a, const uint16_t* __restrict__ b, 
       s_ = s_ > kMaxKSplit ? kMaxKSplit : s_;
       s_ = s_ > nk_all / kMinPartTiles ? nk_all / kMinPartTiles : s_;
       s_ = (int64_t)s_ * rest > ws_capacity ? ws_capacity / rest : s_;
-      ksplit = cut_pays(kSplit ? full_rounds : 0, s_, nk_all) ? s_ : 1;
+      ksplit = cut_pays(!kSplit, full_rounds, s_, nk_all) ? s_ : 1;
     }
   }
   const bool split = ksplit == 1 && kSplit && rest > 0 && 2 * rest <= P;
@@ -1386,6 +1386,18 @@ gmm_rows_kernel(const uint16_t* __restrict__ a, const uint16_t* __restrict__ b, 
     int t_ = (int)((int64_t)p_ * nk_all / ksplit);
     if (DUAL && t_ - nk1 < T::SB + 1 && nk1 - t_ < T::SB + 1) t_ = nk1;
     return t_;
+  };
+  // the assignment of tile row threadIdx.x (top_k = 1: the token itself) of the tile with first row row0
+  auto combine_of = [&](int row0, int end) -> Combine {
+    Combine combine;
+    combine.out = extra;
+    combine.weights = combine_weights;
+    combine.w_dtype = combine_w_dtype;
+    combine.tokens = combine_tokens;
+    const int row = row0 + (int)threadIdx.x;
+    combine.row_exists = row < end;
+    combine.token = slots[combine.row_exists ? row : end - 1];
+    return combine;
   };
   // the tile with first row row0 of expert e (rows start .. end - 1), column tile tn
   auto compute_tile = [&](int e, int end, int tn, int row0, bool use_ts) {
@@ -1505,6 +1517,8 @@ gmm_rows_kernel(const uint16_t* __restrict__ a, const uint16_t* __restrict__ b, 
           __syncthreads();
           const bool last = *flag == ksplit - 1;  // uniform
           if (last) {
+            Combine combine;
+            if constexpr (EPI == kEpiCombine) combine = combine_of(row0, end);
             // The sum of the parts, in part order whoever came last, goes straight to the staging area of the store:
             // one row of product tiles at a time, the parts of up to four workgroups in flight together.
             constexpr int kRowsAtOnce = 1, kTilesAtOnce = kRowsAtOnce * T::TN;   // rows of product tiles per batch of loads
@@ -1540,7 +1554,7 @@ gmm_rows_kernel(const uint16_t* __restrict__ a, const uint16_t* __restrict__ b, 
               __builtin_amdgcn_sched_barrier(0);
             });
             if (threadIdx.x == 0) ws_counters[tile] = 0;   // as the launch found it
-            block_store<DT, T, kEpiNone, true>(acc, c + (int64_t)row0 * n, n, 0, end - row0, g.b_r0, n, lds);
+            block_store<DT, T, EPI, true>(acc, EPI == kEpiCombine && c == nullptr ? nullptr : c + (int64_t)row0 * n, n, 0, end - row0, g.b_r0, n, lds, nullptr, nullptr, nullptr, combine);
           }
           MBX_TICK(r, 4);
           tile_done();
@@ -1575,16 +1589,7 @@ gmm_rows_kernel(const uint16_t* __restrict__ a, const uint16_t* __restrict__ b, 
       // the last row tile of an expert, when at most half full, is computed as a half-height tile as well
       use_ts = kSplit && (use_ts || end - row0 <= half_limit);
       Combine combine;
-      if constexpr (EPI == kEpiCombine) {
-        // the assignment of tile row threadIdx.x (top_k = 1: the token itself), on its way during the main loop
-        combine.out = extra;
-        combine.weights = combine_weights;
-        combine.w_dtype = combine_w_dtype;
-        combine.tokens = combine_tokens;
-        const int row = row0 + (int)threadIdx.x;
-        combine.row_exists = row < end;
-        combine.token = slots[combine.row_exists ? row : end - 1];
-      }
+      if constexpr (EPI == kEpiCombine) combine = combine_of(row0, end);   // on its way during the main loop
       if (use_ts) {
         block_gemm<DT, false, B_MC, TS, DUAL, EPI, false, KTAIL>(g, c_tile, n, 0, end - row0, g.b_r0, n, lds, e_tile, p_tile, o_tile, combine);
       } else {

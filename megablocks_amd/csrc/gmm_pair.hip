@@ -282,7 +282,7 @@ bool gmm_pair_takes(const DmaCall& q) {
   double there = (nn ? 1.3 : 0.5) + full * tile;
   if (left > 0) {
     const double parts = fmin(fmin((double)kMaxKSplit, floor(units / left)), floor(nk / kMinPartTiles));
-    const bool cut = may_cut && 2 * left <= units && (full > 0 || nk >= kMinCutTiles) && cut_pays(half ? 0 : (int)full, (int)parts, (int)nk);
+    const bool cut = may_cut && 2 * left <= units && (full > 0 || nk >= kMinCutTiles) && cut_pays(half, (int)full, (int)parts, (int)nk);
     there += cut ? tile / parts + 21 : 2 * left <= units && full > 0 && !half ? 0.75 * tile : tile;
   }
   there = fmax(there, (nn ? 1.3 : 0.5) + mb / (nn ? 5.4 : 4.6));

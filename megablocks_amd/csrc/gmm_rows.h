@@ -46,7 +46,7 @@ int launch_rows(const DmaCall& call) {
   const int64_t tiles = (ceil_div(rows, T::BM) + num_groups) * tiles_n;   // the row counts are only known on the device
   if (tiles > 0x7fffffff) return MBX_ERANGE;
   // launches that may cut their tiles along the reduction want the compute units that have no tile for the parts
-  const bool may_cut = layout == MBX_NN && epi == dma::kEpiNone && ws.base != nullptr && (dual ? 2 : 1) * ceil_div(k, T::BK) >= kMinCutTiles;
+  const bool may_cut = layout == MBX_NN && (epi == dma::kEpiNone || epi == dma::kEpiCombine) && ws.base != nullptr && (dual ? 2 : 1) * ceil_div(k, T::BK) >= kMinCutTiles;
   const unsigned grid = (unsigned)persistent_grid(may_cut ? (int64_t)1 << 30 : tiles);
   // An expert's last row tile, when at most half full, is computed with the half-height tile -- unless a row of tiles is
   // longer than the run of tiles an XCD's workgroups take per round: the half-height tiles of such a row fill whole
@@ -86,7 +86,7 @@ int launch_rows(const DmaCall& call) {
     int rc = allow_lds(kern, lds);                                                                    \
     if (rc) return rc;                                                                                \
     kern<<<grid, T::THREADS, lds, s>>>(ap, bp, cp, bins, num_groups, rows, k, n, tiles_n, ap2, bp2, (uint16_t*)extra, (uint16_t*)out2,  \
-                                       combine.indices, nullptr, 1, 0, 0u, 0, half_limit, nullptr, nullptr, 0,          \
+                                       combine.indices, nullptr, 1, 0, 0u, 0, half_limit, ws_counters, ws_parts, ws_capacity, \
                                        combine.weights, combine.w_dtype, combine.tokens);             \
   } while (0)
   if constexpr (KTAIL) {

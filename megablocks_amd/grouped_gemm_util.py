@@ -563,7 +563,7 @@ class CombinedRows:
 def gmm_scatter(a, b, batch_sizes, combine: CombinedRows, keep_product=True):
     """(y, out): y[r_e] = a[r_e] @ b[e], the experts' second product (mlp.py:523, glu.py:205), and out =
     ops.scatter(y, indices, bin_ids, weights, bins, top_k = 1) (dmoe.py:280), the combine written by the product's
-    store phase (`mbx_gmm_scatter`; bit-identical to the two steps).  y is None when `keep_product` is False and the
+    store phase (`mbx_gmm_scatter_ws`; bit-identical to the two steps).  y is None when `keep_product` is False and the
     launch did not have to write it (nothing will differentiate).  Shapes the kernel does not take: two steps."""
     _lib.require_cuda(a, b, combine.indices, combine.weights)
     if a.ndim != 2 or b.ndim != 3 or a.dtype != b.dtype or b.shape[1] != a.shape[1]:
@@ -582,9 +582,10 @@ def gmm_scatter(a, b, batch_sizes, combine: CombinedRows, keep_product=True):
         out = torch.empty((combine.tokens, n), dtype=a.dtype, device=a.device)
         w = None if weights is None else weights.contiguous()
         with _lib.device_of(a), _lib.record('gmm_nn_scatter', rows=rows, k=k, n=n, elem=a.element_size(), groups=groups) as rec:
-            rc = lib.mbx_gmm_scatter(_lib.ptr(a), _lib.ptr(b), _lib.ptr(y), _lib.ptr(out), _lib.dtype_of(a), _lib.ptr(bins),
-                                     groups, rows, k, n, _lib.ptr(indices.contiguous()), _lib.ptr(w),
-                                     0 if w is None else _lib.dtype_of(w), combine.tokens, _lib.stream())
+            ws, ws_bytes = _workspace(a.device)
+            rc = lib.mbx_gmm_scatter_ws(_lib.ptr(a), _lib.ptr(b), _lib.ptr(y), _lib.ptr(out), _lib.dtype_of(a), _lib.ptr(bins),
+                                        groups, rows, k, n, _lib.ptr(indices.contiguous()), _lib.ptr(w),
+                                        0 if w is None else _lib.dtype_of(w), combine.tokens, ws, ws_bytes, _lib.stream())
             if rc == _lib.EUNSUPPORTED:
                 rec.cancel()
     if rc == _lib.EUNSUPPORTED:

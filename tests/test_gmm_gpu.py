@@ -1368,6 +1368,39 @@ def test_products_of_few_tiles_are_the_general_kernels(gg, monkeypatch, row_kern
 
 
 @pytest.mark.parametrize('counts,k,n', [
+    ([100, 0, 128, 60], 4096, 520),            # no full round, half-height tiles: eight parts
+    ([700, 20, 300], 4104, 264),               # full tiles, a reduction that ends inside a K tile
+    ([250, 270] * 32, 4096, 1024),             # behind two rounds of half-height tiles: two parts
+    ([250, 270] * 32, 2048, 1024),             # ... of too few K tiles: not cut
+    ([1024] * 8, 5184, 2304),                  # behind a full round: eight parts
+    ([1024] * 8, 2048, 2304),                  # ... where half-height tiles are shorter: not cut
+])
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])
+def test_combine_in_the_store_phase_of_tiles_cut_along_the_reduction(gg, monkeypatch, row_kernel, counts, k, n, dtype):
+    """Product and combined output, with and without the product kept, are those of the cut product and the combine after it, bit for
+    bit, on the last of three launches too, which find the counters as the first did."""
+    torch.manual_seed(k + n)
+    sizes = torch.tensor(counts)
+    groups, rows = len(counts), int(sizes.sum())
+    a = torch.randn(rows, k, device='cuda').to(dtype)
+    w = (torch.randn(groups, k, n, device='cuda') / k ** 0.5).to(dtype)
+    order = torch.randperm(rows, device='cuda').int()
+    bins = torch.cumsum(sizes.cuda(), 0).int()
+    bin_ids = torch.repeat_interleave(torch.arange(groups), sizes).int().cuda()
+    combine = gg.CombinedRows(order, bin_ids, bins, torch.rand(rows, device='cuda').to(dtype))
+    row_kernel(1)
+    y = gg.backend.gmm(a, w, sizes)
+    want = combine.scatter(y)
+    for keep in (True, False, True):
+        got, out = gg.gmm_scatter(a, w, sizes, combine, keep_product=keep)
+        assert torch.equal(out, want) and (torch.equal(got, y) if keep else got is None)
+    monkeypatch.setattr(gg, 'GMM_WORKSPACE', False)
+    whole, out = gg.gmm_scatter(a, w, sizes, combine)
+    assert torch.equal(whole, y) == (k == 2048)   # the other launches were cut
+    assert rel_err(y, whole) < TOL and rel_err(want, out) < TOL
+
+
+@pytest.mark.parametrize('counts,k,n', [
     ([0, 1, 16, 17, 33, 2, 0, 0, 3, 5, 1, 0], 2048, 136),      # experts around the 16 rows a workgroup takes
     ([1] + [0] * 7, 4096, 1024), ([3, 0, 0, 1] + [0] * 60, 2048, 1408), ([2] * 16, 200, 264), ([1, 2, 1, 4] * 20, 2728, 72),
     ([5] * 8, 64, 64), ([8] * 3, 8, 8),
