@@ -83,9 +83,9 @@ def _slot_rows(indices, bin_ids, bins, padded_bins):
     contain the kernels that build its map."""
     capturing = torch.cuda.is_current_stream_capturing()
     key = _slot_rows_key(indices, bins, padded_bins)
-    rows = None if capturing else _kept_slot_rows(indices, key)
-    if rows is not None:
-        return rows
+    cached = getattr(indices, '_mbx_slot_rows', None)   # _kept_slot_rows, without the call: five times a layer step
+    if not capturing and cached is not None and cached[0] == key:
+        return cached[1]
     n_slots = indices.shape[0]
     rows = _scratch(n_slots, indices.device)
     with _lib.device_of(indices):
