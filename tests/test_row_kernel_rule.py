@@ -29,7 +29,9 @@ def kernel():
     # more than eight rounds: few rows, the activation's gradient, narrow products
     (_lib.NT, 151, 67, 320, 5504, ACT), (_lib.NT, 105, 137, 576, 8000, ACT), (_lib.NT, 97, 10059, 128, 64, PLAIN),
     # a long reduction next to a mostly empty wide tile
-    (_lib.NN, 36, 825, 7768, 64, PLAIN)])
+    (_lib.NN, 36, 825, 7768, 64, PLAIN),
+    # half-height tiles whose last round two short parts would not shorten
+    (_lib.NN, 64, 227, 1216, 1344, PLAIN)])
 def test_launches_of_few_tiles(kernel, layout, experts, rows, k, n, epi):
     """Measured 6 - 50 % shorter in the kernel for few tiles than in the general one."""
     assert kernel(layout, experts, rows, k, n, epi) == FEW_TILES
