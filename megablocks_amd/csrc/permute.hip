@@ -329,7 +329,7 @@ struct BoundedRows {
 };
 
 // ------------------------------------------------------------------ combine (scatter)
-// out[t] = sum_j round(x[inv[t*k+j]] * w[t*k+j]); one wave per token, or per kCombineSegment
+// out[t] = sum_j round(x[inv[t*k+j]] * w[t*k+j]); one wave per token, or per `segment`
 // columns of a token (`parts` waves) where the tokens alone would leave the chip idle.  Each product is
 // rounded to the storage type before the fp32 sum, as the reference's scaled copy into a
 // [tokens, top_k, hidden] buffer followed by sum(dim=1) does.
@@ -339,7 +339,7 @@ struct BoundedRows {
 constexpr int kCombineSegment = 512;   // one 16-byte access per lane at 16 bits, two at fp32
 template <int DT, bool VEC, int BATCH>
 __global__ void __launch_bounds__(kRowThreads)
-combine_kernel(const void* __restrict__ x_, int64_t tokens, int hidden, int parts, int top_k, const int32_t* __restrict__ inv_,
+combine_kernel(const void* __restrict__ x_, int64_t tokens, int hidden, int parts, int segment, int top_k, const int32_t* __restrict__ inv_,
                const void* __restrict__ weights, int w_dtype, void* __restrict__ out_,
                const int32_t* __restrict__ row_limit_ptr, int row_limit_value, const int32_t* __restrict__ binned, int num_bins, int capacity) {
   typedef typename Elem<DT>::type E;
@@ -353,8 +353,8 @@ combine_kernel(const void* __restrict__ x_, int64_t tokens, int hidden, int part
   const int64_t items = tokens * parts;
   for (int64_t item = (int64_t)blockIdx.x * kRowWaves + wave; item < items; item += (int64_t)gridDim.x * kRowWaves) {
     const int64_t t = parts == 1 ? item : item / parts;
-    const int col0 = parts == 1 ? 0 : (int)(item - t * parts) * kCombineSegment;       // parts > 1: this wave's segment
-    const int cols = parts == 1 ? hidden : hidden - col0 < kCombineSegment ? hidden - col0 : kCombineSegment;
+    const int col0 = parts == 1 ? 0 : (int)(item - t * parts) * segment;       // parts > 1: this wave's segment
+    const int cols = parts == 1 ? hidden : hidden - col0 < segment ? hidden - col0 : segment;
     const E* const x = x_base + col0;
     E* dst = out + t * hidden + col0;
     const int64_t s0 = t * top_k;
@@ -481,10 +481,14 @@ wgrad_kernel(const void* __restrict__ x_, const void* __restrict__ grad_, int64_
 // One wave per token reads grad[t] once, and for each of its slots reads x[row], accumulates the dot product
 // in the order wgrad_kernel does and writes the dx row: N h e bytes of reads through L2 and one launch less
 // than the two kernels.  Then the rows of dx that no slot owns are zero-filled, as in gather_tokens_kernel.
-// WRITE = false: only dw (a read-only pass; dx is left to gather_tokens_kernel).
+// WRITE = false: only dw (a read-only pass; dx is left to gather_tokens_kernel).  Up to kSlotTokens tokens a wave per slot then: `tokens` is their
+// number, top_k 1, and `share` slots have a token's row of `grad` between them, which is read again, out of the L2.  With a wave per token such a pass
+// is a few waves' chain of latencies (us, with the gather of dx, wave per token / per slot: 700 tokens of 4096 columns, top-8 51 / 28, top-2 20.6 / 16.2; 1500, top-8
+// 65 / 49; 3000 of 2688, top-8 67 / 64; 4200 of 768, top-4 21.2 / 22.4).  The sums keep their order.
+constexpr int64_t kSlotTokens = 4096;   // four waves to a SIMD
 template <int DT, int BATCH, bool WRITE>
 __global__ void __launch_bounds__(kRowThreads)
-scatter_backward_kernel(const void* __restrict__ grad_, const void* __restrict__ x_, int64_t tokens, int hidden, int top_k,
+scatter_backward_kernel(const void* __restrict__ grad_, const void* __restrict__ x_, int64_t tokens, int hidden, int top_k, int share,
                         const int32_t* __restrict__ indices, const int32_t* __restrict__ inv,
                         const int32_t* __restrict__ bins, const int32_t* __restrict__ padded_bins, int num_bins,
                         const void* __restrict__ weights, int w_dtype, void* __restrict__ dx_, int64_t out_rows,
@@ -499,7 +503,7 @@ scatter_backward_kernel(const void* __restrict__ grad_, const void* __restrict__
   const int nvec = hidden / EV;
   const int64_t wave_id = (int64_t)blockIdx.x * kRowWaves + wave, waves = (int64_t)gridDim.x * kRowWaves;
   for (int64_t t = wave_id; t < tokens; t += waves) {
-    const u32x4* g = (const u32x4*)(grad + t * hidden);
+    const u32x4* g = (const u32x4*)(grad + (share == 1 ? t : t / share) * hidden);
     const int64_t s0 = t * top_k;
     int my_row = lane < top_k ? inv[s0 + lane] : -1;
     my_row = my_row < out_rows ? my_row : -1;             // x and dx have out_rows rows
@@ -782,9 +786,11 @@ static int launch_combine(const void* x, int dtype, int64_t tokens, int hidden, 
                           hipStream_t s, const int32_t* binned = nullptr, int num_bins = 0, int capacity = 0) {
   const bool vec = can_vec(dtype, hidden, x, out);
   // Fewer tokens than the chip has SIMDs: a wave per segment of the row.  5 tokens of 2048 columns, top-6: 8.7 us with a wave
-  // per token, one load after the other's latency, 4.5 with four; from 1024 tokens on every SIMD has a wave of its own.
-  const int parts = tokens < 1024 && hidden > kCombineSegment ? (int)ceil_div(hidden, kCombineSegment) : 1;
-#define CALL_B(DT, V, B) combine_kernel<DT, V, B><<<row_grid(tokens * parts), kRowThreads, 0, s>>>(x, tokens, hidden, parts, top_k, inv, weights, w_dtype, out, limit_ptr, limit_value, binned, num_bins, capacity)
+  // per token, one load after the other's latency, 4.5 with four.  With one or two tokens to a SIMD a wave per 1024 columns (us, without / with: 1100
+  // tokens of 2688, top-4 14.8 / 12.0, 1100 of 2048, top-2 9.6 / 8.8, 1500 of 4096, top-8 30.5 / 27.4; 2200 of 3200, top-2 15.1 / 15.8, 3000 16.8 / 18.8).
+  const int segment = tokens < 1024 ? kCombineSegment : 2 * kCombineSegment;
+  const int parts = tokens < 2048 && hidden > segment ? (int)ceil_div(hidden, segment) : 1;
+#define CALL_B(DT, V, B) combine_kernel<DT, V, B><<<row_grid(tokens * parts), kRowThreads, 0, s>>>(x, tokens, hidden, parts, segment, top_k, inv, weights, w_dtype, out, limit_ptr, limit_value, binned, num_bins, capacity)
 #define CALL(DT, V)                            \
   do {                                         \
     if (top_k == 1) CALL_B(DT, V, 1);          \
@@ -874,7 +880,7 @@ int mbx_scatter_backward(const void* grad, const void* x, int dtype, int64_t tok
   if (!grad || !x || !indices || !weights || !grad_x || !wgrad || (padded_bins && !bins)) return MBX_EINVAL;
   hipStream_t s = as_stream(stream);
   const unsigned grid = row_grid(tokens > out_rows / kWave ? tokens : out_rows / kWave);
-#define CALL(DT, B, W) scatter_backward_kernel<DT, B, W><<<grid, kRowThreads, 0, s>>>(grad, x, tokens, hidden, top_k, indices, slot_rows, bins, padded_bins, num_bins, weights, w_dtype, grad_x, out_rows, wgrad)
+#define CALL(DT, B, W) scatter_backward_kernel<DT, B, W><<<grid, kRowThreads, 0, s>>>(grad, x, tokens, hidden, top_k, 1, indices, slot_rows, bins, padded_bins, num_bins, weights, w_dtype, grad_x, out_rows, wgrad)
 #define CALL_DT(DT)                        \
   do {                                     \
     if (top_k == 1) CALL(DT, 1, true);     \
@@ -882,7 +888,9 @@ int mbx_scatter_backward(const void* grad, const void* x, int dtype, int64_t tok
       const int64_t items = tokens * ceil_div((int64_t)hidden * dtype_bytes(dtype) / 16, 4 * kWave);                       \
       const unsigned ggrid = row_grid(items > out_rows / kWave ? items : out_rows / kWave);                               \
       gather_tokens_kernel<DT><<<ggrid, kRowThreads, 0, s>>>(grad, tokens, hidden, top_k, indices, slot_rows, bins, padded_bins, num_bins, weights, w_dtype, grad_x, out_rows); \
-      if (top_k == 2) CALL(DT, 2, false);  \
+      if (tokens <= kSlotTokens)           \
+        scatter_backward_kernel<DT, 1, false><<<row_grid(tokens * top_k), kRowThreads, 0, s>>>(grad, x, tokens * top_k, hidden, 1, top_k, indices, slot_rows, bins, padded_bins, num_bins, weights, w_dtype, grad_x, out_rows, wgrad); \
+      else if (top_k == 2) CALL(DT, 2, false); \
       else if (top_k <= 4) CALL(DT, 4, false); \
       else CALL(DT, 8, false);             \
     }                                      \

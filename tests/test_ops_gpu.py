@@ -429,6 +429,23 @@ def test_c_abi_gather_and_scatter_without_a_prebuilt_map(kernels, padded):
     assert lib.mbx_scatter(*args, None, 0, _lib.stream()) == -2                      # neither a map nor scratch
 
 
+@pytest.mark.parametrize('sl,hs,top_k', [(1023, 1032, 2), (1024, 1024, 4), (1025, 1032, 8), (2047, 2056, 4), (2048, 1032, 2), (4096, 72, 3),
+                                         (4097, 72, 2), (4097, 136, 4), (4100, 72, 8)])
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float32])
+def test_combine_and_its_gradients_around_the_lines_of_their_splits(kernels, sl, hs, top_k, dtype):
+    """Waves of a token's combine by segments of its row, of the weights' gradient by slots, and by tokens: all on both sides of the
+    token counts that choose, the combine against the oracle, the gradients against the two kernels bit for bit."""
+    indices, bin_ids, bins, _ = _routing(sl, 16, top_k, seed=sl)
+    x, grad, w = torch.randn(sl * top_k, hs).to(dtype), torch.randn(sl, hs).to(dtype), torch.rand(sl * top_k).to(dtype)
+    args = dev(indices), dev(bin_ids)
+    got = kernels.scatter(dev(x), *args, dev(w), dev(bins), top_k)
+    # the products are rounded as the storage type says, the sums of up to 8 of them taken in fp32 in another order than the oracle's
+    assert rel_err(got, oracle.scatter(x, indices, bin_ids, w, bins, top_k)) < (4e-3 if dtype == torch.bfloat16 else 1e-6)
+    dx, dw = kernels.scatter_backward(dev(x), dev(grad), *args, dev(w), dev(bins), None, top_k)
+    assert torch.equal(dx, kernels.gather(dev(grad), *args, dev(w), dev(bins), top_k))
+    assert torch.equal(dw, kernels.scatter_wgrad(dev(x), dev(grad), *args, dev(bins), top_k))
+
+
 @pytest.mark.parametrize('sl,hs,ne,top_k', [(1024, 256, 8, 1), (1000, 4096, 8, 2), (777, 264, 5, 3), (2048, 2048, 64, 6),
                                             (512, 1024, 16, 8), (300, 100, 4, 2), (256, 128, 32, 9)])
 @pytest.mark.parametrize('padded', [False, True])
