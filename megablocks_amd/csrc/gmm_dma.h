@@ -1517,6 +1517,7 @@ gmm_rows_kernel(const uint16_t* __restrict__ a, const uint16_t* __restrict__ b, 
           __syncthreads();
           const bool last = *flag == ksplit - 1;  // uniform
           if (last) {
+            __syncthreads();                     // every wave has read the flag, which lies where the first staged tile goes
             Combine combine;
             if constexpr (EPI == kEpiCombine) combine = combine_of(row0, end);
             // The sum of the parts, in part order whoever came last, goes straight to the staging area of the store:

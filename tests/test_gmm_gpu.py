@@ -1400,6 +1400,30 @@ def test_combine_in_the_store_phase_of_tiles_cut_along_the_reduction(gg, monkeyp
     assert rel_err(y, whole) < TOL and rel_err(want, out) < TOL
 
 
+@pytest.mark.parametrize('combined', [False, True])
+def test_tiles_cut_along_the_reduction_are_the_same_every_time(gg, row_kernel, combined):
+    """The workgroup that comes last puts the sum of the parts where the count of the parts was: every one of many launches gives the same
+    bits and leaves the counters at zero.  32 tiles of eight parts fill the chip with such hand-overs."""
+    from megablocks_amd import _lib
+    torch.manual_seed(5)
+    sizes, k, n = torch.tensor([1000, 1024]), 4096, 1024
+    a = torch.randn(2024, k, device='cuda').bfloat16()
+    w = (torch.randn(2, k, n, device='cuda') / k ** 0.5).bfloat16()
+    bins = torch.cumsum(sizes.cuda(), 0).int()
+    bin_ids = torch.repeat_interleave(torch.arange(2), sizes).int().cuda()
+    combine = gg.CombinedRows(torch.randperm(2024, device='cuda').int(), bin_ids, bins, torch.rand(2024, device='cuda').bfloat16())
+    row_kernel(1)
+    run = (lambda: gg.gmm_scatter(a, w, sizes, combine)[1]) if combined else (lambda: gg.backend.gmm(a, w, sizes))
+    first = run()
+    y = gg.backend.gmm(a, w, sizes)
+    assert max_block_err(y, _ref_gpu(a, w, sizes, False, False)) < 2 * TOL
+    assert torch.equal(first, combine.scatter(y) if combined else y)
+    different = sum((run() != first).any().int() for _ in range(100))
+    assert int(different) == 0
+    ws = gg._workspaces[(torch.cuda.current_device(), _lib.stream().value)]
+    assert int(ws[:4096].count_nonzero()) == 0
+
+
 @pytest.mark.parametrize('counts,k,n', [
     ([0, 1, 16, 17, 33, 2, 0, 0, 3, 5, 1, 0], 2048, 136),      # experts around the 16 rows a workgroup takes
     ([1] + [0] * 7, 4096, 1024), ([3, 0, 0, 1] + [0] * 60, 2048, 1408), ([2] * 16, 200, 264), ([1, 2, 1, 4] * 20, 2728, 72),
