@@ -1,25 +1,29 @@
-// Grouped GEMM in fp32 on the 16-bit matrix instructions.  Reductions of more than kThreeParts terms: a value, times a power of two of its
-// row's (column's), is the sum of two fp16 parts (22 bits and the sign of the second), and the three products of parts that reach 2^-22 of a
-// product are summed in fp32 (v_mfma_f32_16x16x32_f16).  Shorter ones: three bf16 parts (24 bits), six products, no scale
-// (v_mfma_f32_16x16x32_bf16).  Chunk below has the splitting, Scale the scales.
+// Grouped GEMM in fp32 on the bf16 matrix instruction: every value is split into three bf16 parts (24 bits, Chunk below), and the
+// six products of parts that reach 2^-18 of a product are summed in fp32 (v_mfma_f32_16x16x32_bf16).
 //
-// What bounds it: the power the matrix cores draw, and next to them the splitting.  The fp32 instruction (v_mfma_f32_16x16x4_f32) does 256 FLOP
-// per cycle and compute unit, the 16-bit ones 4096, a third of which is 1365 and a sixth 683.  A workgroup converts a value once, on its way to the LDS, and
-// its waves multiply parts: two values of fp16 parts take two multiplications, two conversions, two exact rests and a maximum (2.5 cycles of a
-// SIMD the multiplications, 4.4 the others; v_fma_mixlo / mixhi_f16, which would do scale, rest and conversion at once, 8.3: 3 % slower).
-// 4096^3: 403 / 412 / 411 us NT / NN / TN = 334 - 341 TFLOP/s on normal values at 1.8 GHz (zeros, at 2.4 GHz: 284 - 321), with three bf16 parts
-// 642 / 626 / 607, torch.mm 1067 - 1071.  8 experts of 1024 +- 30 rows, [1024, 4096]: 307 / 309 / 252 against 429 / 433 / 358; without the conversions 216 / 211 / 172
-// (and wrong).  The element-wise kernel of gmm.hip, which serves every alignment, takes 947 / 983 / 882.  Launches of a dozen K tiles or less, whose time is the
-// latency of a K tile's way through registers and LDS, gain less (64 experts of 64, [1024, 1408]: 134 / 126 / 180 -> 116 / 105 / 173).
+// What bounds it: the matrix cores and the power they draw.  The fp32 instruction (v_mfma_f32_16x16x4_f32) does 256 FLOP
+// per cycle and compute unit, the bf16 one 4096, a sixth of which is 683.  Next to a product there is room for two vector-ALU
+// instructions per SIMD (measured: 2 are free, 3 cost a fifth, 4 half of the rate), and a value takes six to become parts.  So a
+// workgroup converts a value once, on its way to the LDS, and its waves multiply parts: 1.7 instructions per product.  When every
+// wave converted what it read, 4 per product, the matrix cores were busy 45 - 50 % of the time, now 55 - 59 %, at 2.0 GHz instead
+// of 2.1.  8 experts of 1024 +- 30 rows, [1024, 4096], normal values: 376 / 379 / 352 us NT / NN / TN (operands in the last-level cache or
+// not) against 460 / 459 / 408 that way and 947 / 983 / 882 in the element-wise kernel of gmm.hip, which serves every alignment; 4096^3: 626 /
+// 643 / 646 us, 220 - 213 TFLOP/s, against 799 / 802 / 783 (torch.mm: 1067 - 1071).  On the fp32 instruction the first three were some 40 %
+// longer than here.  Reductions of a dozen K tiles or less in small launches, whose time is the latency of a K tile's way through registers and
+// LDS, are 1 - 3 us longer than when operands went to the LDS directly (24 experts of 74, [128, 256], NT: 13.3 / 10.5).  Keeping the
+// pipeline filled across a workgroup's tiles changed nothing; cutting the parts off instead of rounding them is 3 % faster and up to a third less exact.
 //
-// How exact: relative error (2-norm) against fp64 3.6e-7 over k = 1024, 7.2e-7 over 4096 (three bf16 parts: 4.9e-7 and 1.0e-6; a chain of fp32 fused
-// multiply-adds: 5.7e-7 and 1.15e-6).  An accumulator is rounded three times per 32 k, and that outweighs what the parts leave out from
-// some hundred terms on: 160 terms 1.60e-7 (three bf16 parts 1.75e-7), 128: 1.48e-7 (1.53e-7), 64: 1.19e-7 (0.93e-7); hence kThreeParts.  The small
-// tile, which puts its sums aside every 256 terms: 2.0e-7 over 1024 and 4096 terms (2.3e-7).  These are errors of a row: a value below 2^-13 of
-// the largest of its row's first values keeps fewer than 22 bits, 2^-34 of that largest value being what the second part resolves.
+// How exact: three parts hold all 24 bits of a value; the three products of parts not taken come to less than 2^-25 of a product,
+// and an accumulator is rounded six times per 32 k instead of 32 times.  Relative error (2-norm) against fp64: 4.8e-7 over
+// k = 1024, 9.8e-7 over 4096, where a chain of fp32 fused multiply-adds shows 5.7e-7 and 1.15e-6; 3.1e-8 over eight terms (5.4e-8).
+// The small tile, which puts its sums aside every 256 terms: 2.3e-7 over 1024 terms of which a launch that is cut into four parts made
+// 2.3e-7 too, 2.4e-7 over 4096 (3.5e-7 cut into eight).
 // The error of a single product is larger than that chain's, up to 2.6 2^-24 of it instead of one: sums of one or two terms,
-// and those that the parts do not serve (infinities; with bf16 parts values next to the largest or the smallest), are formed on the fp32
+// and those that the parts do not serve (infinities, NaN, values next to the largest or the smallest), are formed on the fp32
 // instruction: multiply().
+// Why not two fp16 parts of a value times a power of two of its row, and three products (4096^3: 403 / 412 / 411 us): they hold 22 bits, fewer
+// below 2^-13 of the row's largest value and none below 2^-35, and a sum whose large values meet zeros of the other operand is made of just those
+// (off by up to 0.14 of the sum of its terms' magnitudes).  No check of the operands or the result finds such a sum.
 //
 // Tile: 128 x 256 per workgroup of eight waves, two to a SIMD, K tiles of 32 in two stages of 72 KiB; 256 x 128 for TN products
 // whose edges it leaves less empty (12 experts of 500 rows, [2728, 1032]: 252 -> 212 us); 64 x 128, 36 KiB a stage and two
@@ -27,7 +31,7 @@
 // K tile ahead: while K tile kt is multiplied, kt + 1 is converted and written to the other stage, and the loads of kt + 2 go
 // out into the registers that frees.  One barrier per K tile.
 //
-// LDS layout: the parts of an operand tile, each [row][32 k]: 64-byte rows, the 16-byte chunk of k = 8 q .. 8 q + 7 of
+// LDS layout: the three parts of an operand tile, each [row][32 k] bf16: 64-byte rows, the 16-byte chunk of k = 8 q .. 8 q + 7 of
 // row r at position q ^ x(r) (chunk_at), which neither the reads (16 rows, one chunk) nor the writes (64 rows of one chunk, or
 // 16 whole rows) find in the same banks; x = (r >> 2) & 3 alone costs 14 % of the cycles in conflicts.  An operand whose reduction
 // dimension is contiguous (KC) is loaded in 16-byte pieces, two to a chunk; one whose reduction dimension is strided (MC) in
@@ -59,9 +63,7 @@ struct Shape {
   static constexpr int WN = BM == 256 ? 2 : 4, WM = 8 / WN;                      // waves along the columns, the rows
   static constexpr int TM = BM / WM / 16, TN = BN / WN / 16;                     // 16 x 16 accumulator tiles of a wave
   static constexpr uint32_t kPlaneBytes = (BM + BN) * kRowBytes, kStageBytes = 3 * kPlaneBytes;
-  static constexpr uint32_t kExponentsAt = 2 * kStageBytes;                      // behind the stages: the exponents of the rows' scales
-  static constexpr int kA = BM == 256 ? 2 : 1, kB = BN / 128, kChunks = kA + kB; // chunks of A and of B a thread converts
-  static constexpr size_t kLdsBytes = 2 * kStageBytes + (BM + BN) * 4;
+  static constexpr size_t kLdsBytes = 2 * kStageBytes;
   static constexpr size_t kPartBytes = (size_t)BM * BN * 4;                      // one tile's accumulators in the workspace
   static constexpr int kPerUnit = kLdsBytes > 80 * 1024 ? 1 : 2;                 // workgroups that share a compute unit
   // K tiles after which the sums so far are put aside and new ones begun (0: never).  Launches of few tiles get the small tile
@@ -87,83 +89,38 @@ struct Args {
 };
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef int i32x4 __attribute__((ext_vector_type(4)));
 typedef const __attribute__((address_space(3))) u32x4* lds_in;
 typedef __attribute__((address_space(3))) u32x4* lds_out;
 typedef __attribute__((address_space(3))) u32x2* lds_out_half;
 
-template <int PARTS>
 __device__ __forceinline__ f32x4 mfma(u32x4 a, u32x4 b, f32x4 c) {
-  if constexpr (PARTS == 2) return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
-  else return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
-}
-
-// Two values as fp16, rounded to nearest.
-__device__ __forceinline__ uint32_t fp16_pair(float a, float b) {
-  uint32_t d;
-  asm("v_cvt_pk_f16_f32 %0, %1, %2" : "=v"(d) : "v"(a), "v"(b));
-  return d;
-}
-// What fp16_pair() leaves of either value, exactly.
-__device__ __forceinline__ float rest_of_low(float a, uint32_t pair) {
-  float d;
-  asm("v_fma_mix_f32 %0, %1, 1.0, -%2 op_sel_hi:[0,0,1]" : "=v"(d) : "v"(a), "v"(pair));
-  return d;
-}
-__device__ __forceinline__ float rest_of_high(float b, uint32_t pair) {
-  float d;
-  asm("v_fma_mix_f32 %0, %1, 1.0, -%2 op_sel:[0,0,1] op_sel_hi:[0,0,1]" : "=v"(d) : "v"(b), "v"(pair));
-  return d;
-}
-
-// the largest of |a|, |b| and m
-__device__ __forceinline__ float larger(float a, float b, float m) {
-  asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(m) : "v"(a), "v"(b));
-  return m;
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }
 
 // V (8 or 4) consecutive k of one row (column) of an operand on their way from memory to the LDS: the chunk of one thread.
-// step() forms the parts, two fp16 ones of the value times its row's scale (the sum differs from it by up to 2^-23 of it) or three bf16 ones of the
-// value (2^-27): every part is the rest the parts before it leave (the differences are exact), rounded to nearest.  In kSteps steps of a few
-// instructions, to be put between products: step V / 2 q + p forms part q of the values 2 p and 2 p + 1, the last of a part stores it.
-template <int V, uint32_t PLANE, int PARTS>
+// step() forms the three bf16 parts, v = part 0 + part 1 + part 2 up to 2^-27 |v|: every part is the rest the parts before
+// it leave (the differences are exact), rounded to nearest.  In kSteps steps of a few instructions, to be put between
+// products: step V / 2 q + p forms part q of the values 2 p and 2 p + 1, the last of a part stores it.
+template <int V, uint32_t PLANE>
 struct Chunk {
-  static constexpr int kPairs = V / 2, kSteps = PARTS * kPairs;
+  static constexpr int kPairs = V / 2, kSteps = 3 * kPairs;
   float v[V];
   uint32_t part[kPairs];
 
   template <int X>
-  __device__ __forceinline__ void step(float scale, float& largest, lds_ptr to) {   // largest: magnitude seen
+  __device__ __forceinline__ void step(float& largest, lds_ptr to) {   // largest: magnitude seen
     constexpr int q = X / kPairs, p = X % kPairs;
-    if constexpr (q == 0) largest = larger(v[2 * p], v[2 * p + 1], largest);
-    if constexpr (PARTS == 2) {
-      if constexpr (q == 0) {
-        v[2 * p] *= scale;
-        v[2 * p + 1] *= scale;
-      }
-      part[p] = fp16_pair(v[2 * p], v[2 * p + 1]);
-      if constexpr (q == 0) {
-        v[2 * p] = rest_of_low(v[2 * p], part[p]);
-        v[2 * p + 1] = rest_of_high(v[2 * p + 1], part[p]);
-      }
-    } else {
-      part[p] = pack2<MBX_BF16>(v[2 * p], v[2 * p + 1]);
-      if constexpr (q < 2) {
-        v[2 * p] -= __uint_as_float(part[p] << 16);
-        v[2 * p + 1] -= __uint_as_float(part[p] & 0xffff0000u);
-      }
+    if constexpr (q == 0) asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(largest) : "v"(v[2 * p]), "v"(v[2 * p + 1]));
+    const uint32_t both = pack2<MBX_BF16>(v[2 * p], v[2 * p + 1]);
+    part[p] = both;
+    if constexpr (q < 2) {
+      v[2 * p] -= __uint_as_float(both << 16);
+      v[2 * p + 1] -= __uint_as_float(both & 0xffff0000u);
     }
     if constexpr (p == kPairs - 1) {
       if constexpr (V == 8) *(lds_out)(to + q * PLANE) = u32x4{part[0], part[1], part[2], part[3]};
       else *(lds_out_half)(to + q * PLANE) = u32x2{part[0], part[1]};
     }
-  }
-  __device__ __forceinline__ float largest_of() const {
-    float m = 0.f;
-#pragma unroll
-    for (int p = 0; p < kPairs; ++p) m = larger(v[2 * p], v[2 * p + 1], m);
-    return m;
   }
   // for the fp32 instruction: the values as they are, k 0 .. 3 of eight to one plane, 4 .. 7 to the next
   __device__ __forceinline__ void store_as_is(lds_ptr to, int half) const {
@@ -185,53 +142,22 @@ __device__ __forceinline__ void clear(typename S::Acc& acc) {
     for (int j = 0; j < S::TN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 }
 
-// The pairs of parts that are multiplied, pass by pass, and which part of an operand is read during a pass (-1: none; in the last pass
-// the next K tile's).  A part is read while the products that last took its registers are past.
-template <int PARTS> struct Order;
-template <> struct Order<1> { static constexpr int kPasses = 1, a[] = {0}, b[] = {0}, read_a[] = {0}, read_b[] = {0}; };   // (unused)
-template <> struct Order<2> { static constexpr int kPasses = 3, a[] = {1, 0, 0}, b[] = {0, 0, 1}, read_a[] = {0, -1, 1}, read_b[] = {-1, 1, 0}; };
-template <> struct Order<3> {
-  static constexpr int kPasses = 6, a[] = {1, 0, 2, 0, 1, 0}, b[] = {1, 2, 0, 1, 0, 0};
-  static constexpr int read_a[] = {0, 2, -1, -1, -1, 1}, read_b[] = {2, 0, -1, -1, -1, 1};
-};
-
-// The scale of a row of A (column of B) within a tile, 2^x with x in the LDS at kExponentsAt, brings its largest magnitude
-//   * kFirst: among its first two K tiles to 2^9 .. 2^10, which leaves 64 times that for the values to come: nobody reads an operand twice
-//     to know its largest value.  A row that exceeds it, or whose first values are all zero and later ones are not, shows at the end, and
-//     the tile is multiplied again,
-//   * kExact: among all its values, known by then, to 2^14 .. 2^15.  (8 experts of 1024, [1024, 4096], one such value in every row: 270 / 264 /
-//     247 -> 400 / 414 / 397 us NT / NN / TN; one infinity in every tile 691 / 711 / 708.)
-struct Scale {
-  float by;
-  bool some;   // whether the values it was made from were not all zero
-};
-enum Attempt { kFirst, kExact };
-constexpr int kTopFirst = 10, kTopExact = 15;
-constexpr float kFp16Max = 65504.f;
-
-// acc += A_tile * B_tile over K tiles [g.kt0, g.kt1), of PARTS parts a value; 1: of the values, on the fp32 instruction.
-// largest: the largest magnitude of every chunk's row this thread has seen (PARTS == 2: as == kExact takes the scales from it; 3: updated).
-// Returns (PARTS == 2) whether a scale did not fit, in this thread's chunks.
-template <bool A_MC, bool B_MC, typename S, bool DUAL, int PARTS>
-__device__ __forceinline__ bool multiply_as(const Args& g, typename S::Acc& acc, char* lds_generic, Attempt as, float (&largest)[S::kChunks]) {
-  constexpr bool FP32 = PARTS == 1;
-  constexpr int TM = S::TM, TN = S::TN, kA = S::kA, kB = S::kB, kChunks = S::kChunks;
+// acc += A_tile * B_tile over K tiles [g.kt0, g.kt1); largest: the largest magnitude among the operands (unless FP32)
+template <bool A_MC, bool B_MC, typename S, bool DUAL, bool FP32>
+__device__ __forceinline__ void multiply_as(const Args& g, typename S::Acc& acc, char* lds_generic, float& largest) {
+  constexpr int TM = S::TM, TN = S::TN, kA = S::BM == 256 ? 2 : 1, kB = S::BN / 128, kChunks = kA + kB;   // chunks of a thread
   constexpr int kAV = S::BM == 64 ? 4 : 8;
-  if (g.kt0 >= g.kt1) return false;
+  if (g.kt0 >= g.kt1) return;
   const lds_ptr lds = (lds_ptr)lds_generic;
-  // a copy the compiler cannot see through: what depends on the lane alone would else be worked out once, ahead of the loop over tiles, for
-  // every form of this function, and not fit into the registers
-  uint32_t thread = threadIdx.x;
-  asm volatile("" : "+v"(thread));
-  const int wave = __builtin_amdgcn_readfirstlane(thread / kWave), lane = thread % kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = lane_id();
 
   // This thread's chunks: k = 8 q .. 8 q + 7 of rows r and r + 128 of A and of B; BM = 64: one half of eight k of a row of A.
   auto chunk_at = [&](int row, int q) -> uint32_t {
     const int b = row >> 2 & 3, x = (((b << 1 ^ b) & 2) | b >> 1) ^ (row >> 1 & 1);
     return (uint32_t)row * kRowBytes + (uint32_t)((q ^ x) << 4);
   };
-  const int kc_r = thread >> 2, kc_q = thread & 3;                    // four lanes a row: 128 bytes of it
-  const int half_r = A_MC ? lane : thread >> 3, half_k = 4 * (A_MC ? wave : thread & 7);   // eight lanes a row; 64 columns per load
+  const int kc_r = threadIdx.x >> 2, kc_q = threadIdx.x & 3;                    // four lanes a row: 128 bytes of it
+  const int half_r = A_MC ? lane : threadIdx.x >> 3, half_k = 4 * (A_MC ? wave : threadIdx.x & 7);   // eight lanes a row; 64 columns per load
   const int mc_r = lane + 64 * (wave >> 2), mc_q = wave & 3;                    // 64 consecutive columns per load
   const uint32_t a_to = kAV == 4 ? chunk_at(half_r, half_k >> 3) + (half_k & 4 ? 8u : 0u) : A_MC ? chunk_at(mc_r, mc_q) : chunk_at(kc_r, kc_q);
   const uint32_t b_to = S::BM * kRowBytes + (B_MC ? chunk_at(mc_r, mc_q) : chunk_at(kc_r, kc_q));
@@ -242,11 +168,10 @@ __device__ __forceinline__ bool multiply_as(const Args& g, typename S::Acc& acc,
                                : (uint32_t)(g.b_r0 + kc_r) * g.b_ld + (uint32_t)kc_q * 32u;
   const uint32_t a_step = A_MC ? kBK * g.a_ld : kBK * 4u, b_step = B_MC ? kBK * g.b_ld : kBK * 4u;   // per K tile
 
-  typedef Chunk<kAV, S::kPlaneBytes, PARTS> ChunkA;
-  typedef Chunk<8, S::kPlaneBytes, PARTS> ChunkB;
+  typedef Chunk<kAV, S::kPlaneBytes> ChunkA;
+  typedef Chunk<8, S::kPlaneBytes> ChunkB;
   ChunkA ca[kA];
   ChunkB cb[kB];
-  Scale scale[kChunks];
   uint32_t a_at = 0, b_at = 0, past_half = 0, past_low = 0, past_high = 0;
   __amdgpu_buffer_rsrc_t ra = g.rsrc_a, rb = g.rsrc_b;
   auto load_at = [&](int kt) {
@@ -295,8 +220,7 @@ __device__ __forceinline__ bool multiply_as(const Args& g, typename S::Acc& acc,
   const uint32_t frag_lane = chunk_at(lane & 15, lane >> 4);
   const uint32_t fa_at = (uint32_t)S::row(wave) * kRowBytes + frag_lane;
   const uint32_t fb_at = (uint32_t)(S::BM + S::column(wave)) * kRowBytes + frag_lane;
-  constexpr int kPlanes = FP32 ? 2 : PARTS;
-  u32x4 fa[kPlanes][TM], fb[kPlanes][TN];
+  u32x4 fa[3][TM], fb[3][TN];
   auto read_a = [&](auto qi, auto ii, uint32_t stage) {
     constexpr int q = decltype(qi)::value, i = decltype(ii)::value;
     fa[q][i] = *(lds_in)(lds + (fa_at + stage) + (q * S::kPlaneBytes + i * 16 * kRowBytes));
@@ -311,6 +235,7 @@ __device__ __forceinline__ bool multiply_as(const Args& g, typename S::Acc& acc,
   };
   constexpr std::integral_constant<int, 0> c0{};
   constexpr std::integral_constant<int, 1> c1{};
+  constexpr std::integral_constant<int, 2> c2{};
 
   // K tile kt0 into stage 0, K tile kt0 + 1 under way
   {
@@ -326,58 +251,15 @@ __device__ __forceinline__ bool multiply_as(const Args& g, typename S::Acc& acc,
     for (int c = 0; c < kA; ++c) load_a(c, ca[c]);
 #pragma unroll
     for (int c = 0; c < kB; ++c) load_b(c, cb[c]);
-    if constexpr (PARTS == 2) {
-      // the largest magnitude of every row (column): of its values so far, or (kExact) of all of them, which the attempt before left
-      // behind.  Its pieces meet in stage 1, which nothing is in yet.
-      typedef __attribute__((address_space(3))) float* lds_float;
-      const lds_float pieces = (lds_float)(lds + S::kStageBytes);
-      auto a_piece = [&](int c) { return kAV == 4 ? (A_MC ? wave : thread & 7) * S::BM + half_r : (A_MC ? mc_q * S::BM + mc_r : kc_q * S::BM + kc_r) + 128 * c; };
-      constexpr int kAPieces = kAV == 4 ? 8 : 4;
-      auto b_piece = [&](int c) { return kAPieces * S::BM + (B_MC ? mc_q * S::BN + mc_r : kc_q * S::BN + kc_r) + 128 * c; };
-      if (as == kFirst) {
-#pragma unroll
-        for (int c = 0; c < kA; ++c) pieces[a_piece(c)] = __builtin_fmaxf(first_a[c].largest_of(), ca[c].largest_of());
-#pragma unroll
-        for (int c = 0; c < kB; ++c) pieces[b_piece(c)] = __builtin_fmaxf(first_b[c].largest_of(), cb[c].largest_of());
-      } else {
-#pragma unroll
-        for (int c = 0; c < kA; ++c) pieces[a_piece(c)] = largest[c];
-#pragma unroll
-        for (int c = 0; c < kB; ++c) pieces[b_piece(c)] = largest[kA + c];
-      }
-      barrier();
-      const int top = as == kFirst ? kTopFirst : kTopExact;
-      auto scale_of = [&](int at, int step, int number, int row) {
-        float m = pieces[at];
-#pragma unroll
-        for (int q = 1; q < number; ++q) m = __builtin_fmaxf(m, pieces[at + q * step]);
-        const int e = m > 0.f ? top - __builtin_amdgcn_frexp_expf(m) : 0;
-        const int x = e > 127 ? 127 : e;
-        ((__attribute__((address_space(3))) int*)(lds + S::kExponentsAt))[row] = x;   // the same from every thread of a row
-        return Scale{__uint_as_float((uint32_t)(x + 127) << 23), m > 0.f};
-      };
-#pragma unroll
-      for (int c = 0; c < kA; ++c) {
-        const int row = (kAV == 4 ? half_r : A_MC ? mc_r : kc_r) + 128 * c;
-        scale[c] = scale_of(row, S::BM, kAPieces, row);
-      }
-#pragma unroll
-      for (int c = 0; c < kB; ++c) {
-        const int row = (B_MC ? mc_r : kc_r) + 128 * c;
-        scale[kA + c] = scale_of(kAPieces * S::BM + row, S::BN, 4, S::BM + row);
-      }
-#pragma unroll
-      for (int c = 0; c < kChunks; ++c) largest[c] = 0.f;
-    }
     dma::static_for<kA>([&](auto ci) {
       constexpr int c = decltype(ci)::value;
       if constexpr (FP32) first_a[c].store_as_is(a_chunk_to(c, 0), (half_k & 4) != 0);
-      else dma::static_for<ChunkA::kSteps>([&](auto xi) { first_a[c].template step<decltype(xi)::value>(scale[c].by, largest[c], a_chunk_to(c, 0)); });
+      else dma::static_for<ChunkA::kSteps>([&](auto xi) { first_a[c].template step<decltype(xi)::value>(largest, a_chunk_to(c, 0)); });
     });
     dma::static_for<kB>([&](auto ci) {
       constexpr int c = decltype(ci)::value;
       if constexpr (FP32) first_b[c].store_as_is(b_chunk_to(c, 0), 0);
-      else dma::static_for<ChunkB::kSteps>([&](auto xi) { first_b[c].template step<decltype(xi)::value>(scale[kA + c].by, largest[kA + c], b_chunk_to(c, 0)); });
+      else dma::static_for<ChunkB::kSteps>([&](auto xi) { first_b[c].template step<decltype(xi)::value>(largest, b_chunk_to(c, 0)); });
     });
   }
   barrier();
@@ -416,46 +298,53 @@ __device__ __forceinline__ bool multiply_as(const Args& g, typename S::Acc& acc,
       put_aside(kt);
       barrier();
     }
-    return false;
+    return;
   }
 
-  // The products of a K tile go by pairs of parts.  The parts of the first pass are read ahead of the loop's head, the others one or
-  // more passes before the products that take them; between the products of all passes but the last stand the conversions
+  // The products of a K tile go by pairs of parts, the small ones first.  Parts 1 are read ahead of the loop's head, the other
+  // parts a pass before the products that take them; between the products of the first five passes stand the conversions
   // of K tile kt + 1 (and, when a chunk is converted, the loads of kt + 2 into its registers); the barrier stands where all
   // waves have read this stage and written the other, with the last pass still to be multiplied behind it.
-  typedef Order<PARTS> O;
-  constexpr int kPasses = O::kPasses, kPass = TM * TN, kConvert = (kPasses - 1) * kPass - 2;
-  constexpr int kWorkA = kA * ChunkA::kSteps, kWork = kWorkA + kB * ChunkB::kSteps;
-  dma::static_for<TM>([&](auto ii) { read_a(std::integral_constant<int, O::a[0]>{}, ii, 0); });
-  dma::static_for<TN>([&](auto ji) { read_b(std::integral_constant<int, O::b[0]>{}, ji, 0); });
+  constexpr int kPass = TM * TN, kConvert = 5 * kPass - 2, kWorkA = kA * ChunkA::kSteps, kWork = kWorkA + kB * ChunkB::kSteps;
+  constexpr int pa[6] = {1, 0, 2, 0, 1, 0}, pb[6] = {1, 2, 0, 1, 0, 0};
+  dma::static_for<TM>([&](auto ii) { read_a(c1, ii, 0); });
+  dma::static_for<TN>([&](auto ji) { read_b(c1, ji, 0); });
   for (int kt = g.kt0; kt < g.kt1; ++kt) {
     const uint32_t next = S::kStageBytes - stage;
     load_at(kt + 2);
-    dma::static_for<kPasses>([&](auto pi) {
+    dma::static_for<6>([&](auto pi) {
       constexpr int pass = decltype(pi)::value;
-      constexpr bool last = pass == kPasses - 1;
-      constexpr int ra = O::read_a[pass], rb = O::read_b[pass], kReadsA = ra < 0 ? 0 : TM, kReads = kReadsA + (rb < 0 ? 0 : TN);
-      if constexpr (last) barrier();
+      if constexpr (pass == 5) barrier();
       dma::static_for<kPass>([&](auto mi) {
         constexpr int m = decltype(mi)::value, i = m / TN, j = m % TN, at = pass * kPass + m;
-        // reads, spread over the pass; the last pass's are the next K tile's
-        constexpr int f0 = m * kReads / kPass, f1 = (m + 1) * kReads / kPass;
-        dma::static_for<f1 - f0>([&](auto oi) {
-          constexpr int f = f0 + decltype(oi)::value;
-          if constexpr (f < kReadsA) read_a(std::integral_constant<int, ra>{}, std::integral_constant<int, f>{}, last ? next : stage);
-          else read_b(std::integral_constant<int, rb>{}, std::integral_constant<int, f - kReadsA>{}, last ? next : stage);
-        });
-        acc[i][j] = mfma<PARTS>(fb[O::b[pass]][j], fa[O::a[pass]][i], acc[i][j]);
+        // the next pass's (pass 5: the next K tile's) operands: TM + TN reads over the pass
+        constexpr int f0 = m * (TM + TN) / kPass, f1 = (m + 1) * (TM + TN) / kPass;
+        if constexpr (pass < 2 || pass == 5)
+          dma::static_for<f1 - f0>([&](auto oi) {
+            constexpr int f = f0 + decltype(oi)::value;
+            if constexpr (f < TM) {
+              constexpr std::integral_constant<int, f> fi{};
+              if constexpr (pass == 0) read_a(c0, fi, stage);
+              if constexpr (pass == 1) read_a(c2, fi, stage);
+              if constexpr (pass == 5) read_a(c1, fi, next);
+            } else {
+              constexpr std::integral_constant<int, f - TM> fi{};
+              if constexpr (pass == 0) read_b(c2, fi, stage);
+              if constexpr (pass == 1) read_b(c0, fi, stage);
+              if constexpr (pass == 5) read_b(c1, fi, next);
+            }
+          });
+        acc[i][j] = mfma(fb[pb[pass]][j], fa[pa[pass]][i], acc[i][j]);
         constexpr int x0 = at * kWork / kConvert, x1 = (at + 1) * kWork / kConvert < kWork ? (at + 1) * kWork / kConvert : kWork;
         dma::static_for<(x1 > x0 ? x1 - x0 : 0)>([&](auto oi) {
           constexpr int x = x0 + decltype(oi)::value;
           if constexpr (x < kWorkA) {
             constexpr int c = x / ChunkA::kSteps, y = x % ChunkA::kSteps;
-            ca[c].template step<y>(scale[c].by, largest[c], a_chunk_to(c, next));
+            ca[c].template step<y>(largest, a_chunk_to(c, next));
             if constexpr (y == ChunkA::kSteps - 1) load_a(c, ca[c]);
           } else {
             constexpr int c = (x - kWorkA) / ChunkB::kSteps, y = (x - kWorkA) % ChunkB::kSteps;
-            cb[c].template step<y>(scale[kA + c].by, largest[kA + c], b_chunk_to(c, next));
+            cb[c].template step<y>(largest, b_chunk_to(c, next));
             if constexpr (y == ChunkB::kSteps - 1) load_b(c, cb[c]);
           }
         });
@@ -465,51 +354,6 @@ __device__ __forceinline__ bool multiply_as(const Args& g, typename S::Acc& acc,
     stage = next;
     put_aside(kt);
   }
-  bool off = false;
-  if constexpr (PARTS == 2)
-#pragma unroll
-    for (int c = 0; c < kChunks; ++c) off |= !(largest[c] * scale[c].by < kFp16Max) || (!scale[c].some && largest[c] > 0.f);
-  return off;
-}
-
-// acc times the scales of its row and of its column, backwards
-template <typename S>
-__device__ __forceinline__ void unscale(typename S::Acc& acc, char* lds_generic) {
-  typedef const __attribute__((address_space(3))) int* lds_int;
-  uint32_t thread = threadIdx.x;
-  asm volatile("" : "+v"(thread));
-  const int wave = thread / kWave, lane = thread % kWave;
-  const lds_ptr exponents = (lds_ptr)lds_generic + S::kExponentsAt;
-  i32x4 xb[S::TN];
-#pragma unroll
-  for (int j = 0; j < S::TN; ++j) xb[j] = *(const __attribute__((address_space(3))) i32x4*)(exponents + 4 * (S::BM + S::column(wave) + 16 * j + 4 * (lane >> 4)));
-#pragma unroll
-  for (int i = 0; i < S::TM; ++i) {
-    const int xa = *(lds_int)(exponents + 4 * (S::row(wave) + 16 * i + (lane & 15)));
-#pragma unroll
-    for (int j = 0; j < S::TN; ++j)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) acc[i][j][r] = __builtin_amdgcn_ldexpf(acc[i][j][r], -(xa + xb[j][r]));
-  }
-}
-
-// acc = A_tile * B_tile over K tiles [g.kt0, g.kt1) of two fp16 parts a value; false (and acc zero) where an operand of the tile has an infinity.
-// A NaN stays a NaN through scale and parts, in the rows and columns it belongs to.
-template <bool A_MC, bool B_MC, typename S, bool DUAL>
-__device__ __forceinline__ bool multiply_scaled(const Args& g, typename S::Acc& acc, char* lds) {
-  float largest[S::kChunks];
-  Attempt as = kFirst;
-#pragma unroll 1   // one copy of the code: two take registers of each other
-  while (__syncthreads_or(multiply_as<A_MC, B_MC, S, DUAL, 2>(g, acc, lds, as, largest)) && as == kFirst) {
-    bool infinite = false;
-#pragma unroll
-    for (int c = 0; c < S::kChunks; ++c) infinite |= largest[c] == INFINITY;
-    clear<S>(acc);
-    if (__syncthreads_or(infinite)) return false;
-    as = kExact;
-  }
-  unscale<S>(acc, lds);
-  return true;
 }
 
 // Whether one of the values a tile multiplies over K tiles [g.kt0, g.kt1) is so small that its parts lose some of it, zeros
@@ -552,14 +396,17 @@ __device__ __forceinline__ bool any_small(const Args& g, const __amdgpu_buffer_r
   return smallest < __float_as_uint(kSmall) - 1u;
 }
 
-// Whether the sums of three bf16 parts a value are to be formed again on the fp32 instruction, which takes every value as it is, because
+// acc = A_tile * B_tile over K tiles [g.kt0, g.kt1), on the split operands (multiply()); a second time on the fp32 instruction,
+// which takes every value as it is, where
 //   * a sum comes out infinite, NaN or of a magnitude below kTiny, or an operand is kHuge or more.  The splitting of an
 //     infinity, or of a value that rounds to one, leaves NaN parts, so no such sum stays unnoticed.  Parts of a value below
 //     kSmall can fall below the normal range: next to operands below kHuge its products are below kTiny, and what they
 //     lose (2^-134 of the value, 2^-96 of a product) is 2^-32 of any sum that stays;
 //   * a sum comes out zero and the tile has such a value, whose parts may all have been zero.  Zero sums are common (rows that
 //     pad an expert), so the values are looked at before the tile is repeated.
-// Of the sums only those that are stored count: rows below m_lim, columns below n_lim.
+// Of the sums only those that are stored count: rows below m_lim, columns below n_lim.  A launch that is formed twice throughout
+// (operands of 2^-60 and less next to others of order one, or of 2^40) takes 993 / 1013 / 954 us NT / NN / TN for 8 experts of 1024
+// rows, [1024, 4096], instead of 376 / 379 / 352; the element-wise kernel takes 947 / 983 / 882 for any values.
 constexpr float kTiny = 0x1p-64f, kHuge = 0x1p38f;
 
 template <bool A_MC, bool B_MC, typename S, bool DUAL>
@@ -603,30 +450,19 @@ __device__ __forceinline__ bool sums_need_fp32(const Args& g, const typename S::
 
 // A reduction of one or two terms goes to the fp32 instruction at once: its result is rounded once or twice there, and the
 // products of parts that are left out, and what the bf16 instruction drops of a sum, are more than that (largest error over the
-// sum of the magnitudes, 2^-24: 1.0 / 2.6 over one term, 1.9 / 2.6 over two, 2.5 / 2.3 over three, 3.7 / 2.1 over eight).  Up to kThreeParts
-// terms: see the head of this file; there the stores bound the launch and the second three products cost next to nothing (32 experts of
-// 128, [1024, 2048], TN: 152 us, of 160: 146).
-constexpr int kThreeParts = 128, kFewTerms = 2;
+// sum of the magnitudes, 2^-24: 1.0 / 2.6 over one term, 1.9 / 2.6 over two, 2.5 / 2.3 over three, 3.7 / 2.1 over eight).
+constexpr int kFewTerms = 2;
 
-// acc = A_tile * B_tile over K tiles [g.kt0, g.kt1).  SHORT: whether the reduction may be of kThreeParts terms or fewer.
-template <bool A_MC, bool B_MC, typename S, bool DUAL, bool SHORT>
+template <bool A_MC, bool B_MC, typename S, bool DUAL>
 __device__ __forceinline__ void multiply(const Args& g, typename S::Acc& acc, int m_lim, int n_lim, char* lds) {
   clear<S>(acc);
-  float largest[S::kChunks];
-  const int terms = DUAL ? 2 * g.k : g.k;
-  if (!SHORT || (A_MC && terms > kThreeParts)) {
-    if (multiply_scaled<A_MC, B_MC, S, DUAL>(g, acc, lds)) return;
-  } else if (!A_MC || terms > kFewTerms) {   // NN / NT: k is a multiple of 4
-#pragma unroll
-    for (int c = 0; c < S::kChunks; ++c) largest[c] = 0.f;
-    multiply_as<A_MC, B_MC, S, DUAL, 3>(g, acc, lds, kFirst, largest);
-    float operand = 0.f;
-#pragma unroll
-    for (int c = 0; c < S::kChunks; ++c) operand = __builtin_fmaxf(operand, largest[c]);
+  float operand = 0.f;
+  if (!A_MC || g.k > kFewTerms) {   // NN / NT: k is a multiple of 4
+    multiply_as<A_MC, B_MC, S, DUAL, false>(g, acc, lds, operand);
     if (!sums_need_fp32<A_MC, B_MC, S, DUAL>(g, acc, operand, m_lim, n_lim)) return;
     clear<S>(acc);
   }
-  multiply_as<A_MC, B_MC, S, DUAL, 1>(g, acc, lds, kFirst, largest);
+  multiply_as<A_MC, B_MC, S, DUAL, true>(g, acc, lds, operand);
 }
 
 // c[m][n] = acc for the tile's rows below m_lim and columns below n (n a multiple of 4, c 16-byte aligned)
@@ -691,7 +527,7 @@ __device__ __forceinline__ bool join_parts(typename S::Acc& acc, int tile, int t
 // last round that would leave at least half of the workgroups idle are cut along the reduction when there is a
 // workspace: with four and a half rounds of long reductions (8 experts of 1024 rows: 4.4 rounds NT, 1.1 NN) the tail
 // would otherwise take as long as a full round.
-template <bool B_MC, typename S, bool DUAL, bool SHORT>
+template <bool B_MC, typename S, bool DUAL>
 __global__ void __launch_bounds__(kThreads, 2 * S::kPerUnit)
 gmm_f32_rows_kernel(const float* __restrict__ a, const float* __restrict__ b, float* __restrict__ c, const int32_t* __restrict__ bins,
                     int num_groups, int64_t rows, int k, int n, int tiles_n, const float* __restrict__ a2, const float* __restrict__ b2,
@@ -747,7 +583,7 @@ gmm_f32_rows_kernel(const float* __restrict__ a, const float* __restrict__ b, fl
     g.kt0 = cut ? (int)((int64_t)part * nk / ksplit) : 0;
     g.kt1 = cut ? (int)((int64_t)(part + 1) * nk / ksplit) : nk;
     typename S::Acc acc;
-    multiply<false, B_MC, S, DUAL, SHORT>(g, acc, end - row0, n - g.b_r0, lds);
+    multiply<false, B_MC, S, DUAL>(g, acc, end - row0, n - g.b_r0, lds);
     if (!cut || join_parts<S>(acc, id - full_rounds * P, rest, part, ksplit, ws_counters, ws_parts, lds))
       store<S>(acc, c + (int64_t)row0 * n, n, end - row0, g.b_r0, n);
     tile_done();
@@ -797,7 +633,7 @@ gmm_f32_tn_kernel(const float* __restrict__ a, const float* __restrict__ b, floa
   g.kt0 = (int)((int64_t)part * nk / ksplit);
   g.kt1 = (int)((int64_t)(part + 1) * nk / ksplit);
   typename S::Acc acc;
-  multiply<true, true, S, false, true>(g, acc, k - g.a_r0, n - g.b_r0, lds);
+  multiply<true, true, S, false>(g, acc, k - g.a_r0, n - g.b_r0, lds);
   if (ksplit > 1 && !join_parts<S>(acc, tile, total, part, ksplit, ws_counters, ws_parts, lds)) return;
   store<S>(acc, c + ((int64_t)e * k + g.a_r0) * n, n, k - g.a_r0, g.b_r0, n);
 }
@@ -807,7 +643,7 @@ int launch_rows(const float* a, const float* b, float* c, const int32_t* bins, i
                 const float* b2, const Workspace& lent, int units, hipStream_t s) {
   WorkspaceParts ws(lent, S::kPartBytes);
   if (units > (int)kWorkspaceCounters) ws.parts = nullptr;   // at most half of the workgroups' tiles are cut
-  auto kern = (DUAL ? 2 : 1) * (int64_t)k > kThreeParts ? gmm_f32_rows_kernel<B_MC, S, DUAL, false> : gmm_f32_rows_kernel<B_MC, S, DUAL, true>;
+  auto kern = gmm_f32_rows_kernel<B_MC, S, DUAL>;
   const int rc = allow_lds(kern, S::kLdsBytes);
   if (rc) return rc;
   kern<<<(unsigned)(S::kPerUnit * units), kThreads, S::kLdsBytes, s>>>(a, b, c, bins, num_groups, rows, k, n, (int)ceil_div(n, S::BN), a2, b2,
