@@ -123,6 +123,11 @@ def stream():
     return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
 
 
+def stream_of(t):
+    """The handle of the current stream of `t`'s device."""
+    return _raw_stream(t.get_device()) if _raw_stream is not None else torch.cuda.current_stream(t.device).cuda_stream
+
+
 class _Nothing:
     """The context of a launch that needs none."""
     __slots__ = ()

@@ -42,7 +42,7 @@ def _scratch(n_slots, device):
 
 
 def _slot_rows_key(indices, bins, padded_bins):
-    return (indices._version, bins.data_ptr(), bins._version,
+    return (_lib.stream_of(indices), indices._version, bins.data_ptr(), bins._version,
             None if padded_bins is None else (padded_bins.data_ptr(), padded_bins._version))
 
 
@@ -79,7 +79,9 @@ def _slot_rows(indices, bin_ids, bins, padded_bins):
     tensor and reused while `indices`, `bins` and `padded_bins` are the same unmodified tensors ("unmodified" as
     torch sees it, by `_version`: a caller that rewrites them through raw pointers or by replaying a captured graph
     into them must pass new tensors, or delete the `_mbx_slot_rows` attribute).  A caller that builds a new `indices` tensor for every
-    call gets a new map for every call.  Under stream capture nothing is reused or kept: a captured graph has to
+    call gets a new map for every call.  Calls on another stream than the map's get one of their own: whoever uses `indices` there
+    waits for that tensor and says that it is in use, and knows nothing of a map, which may have been built since and whose memory
+    goes back to its stream with `indices`.  Under stream capture nothing is reused or kept: a captured graph has to
     contain the kernels that build its map."""
     capturing = torch.cuda.is_current_stream_capturing()
     key = _slot_rows_key(indices, bins, padded_bins)

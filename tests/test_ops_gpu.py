@@ -285,6 +285,37 @@ def test_binned_scatter_from_the_routings_map(kernels, sl, hs, ne, top_k, cap, w
     assert torch.equal(kernels.binned_scatter(x, indices, w, bins, top_k), kernels.binned_scatter(x, plain.flip(0), w, bins, top_k))
 
 
+def test_a_map_is_used_on_its_own_stream_only(kernels):
+    """Whoever uses the assignments on a second stream waits for them and marks them as in use there; a map kept from the first, which nobody could
+    mark, is not read there, by none of the operators, and one made there is not read on the first."""
+    from megablocks_amd.ops import routing
+    torch.manual_seed(3)
+    indices, bin_ids, _, bins, _ = routing.route((torch.rand(600, device='cuda') * 8).int(), 8, 3)
+    x, binned = torch.randn(300, 64, device='cuda').half(), torch.randn(8, 50, 64, device='cuda').half()
+    w = torch.rand(600, device='cuda').half()
+
+    def calls():
+        y = kernels.gather(x, indices, bin_ids, None, bins, 2)
+        return y, kernels.scatter(y, indices, bin_ids, w, bins, 2), kernels.binned_scatter(binned, indices, w, bins, 2)
+
+    def map_on(stream):
+        with torch.cuda.stream(stream):
+            return kernels._kept_slot_rows(indices, kernels._slot_rows_key(indices, bins, None))
+
+    here, there = torch.cuda.current_stream(), torch.cuda.Stream()
+    kept = map_on(here)
+    assert kept is not None and map_on(there) is None
+    want = calls()
+    assert map_on(here) is kept
+    there.wait_stream(here)
+    with torch.cuda.stream(there):
+        got = calls()
+    here.wait_stream(there)
+    assert map_on(here) is None and map_on(there) is not kept
+    assert all(torch.equal(a, b) for a, b in zip(got, want)) and all(torch.equal(a, b) for a, b in zip(calls(), want))
+    torch.cuda.synchronize()
+
+
 @pytest.mark.parametrize('sl,hs,ne,top_k,cap', [(1, 8, 1, 1, 1), (77, 520, 3, 2, 5), (300, 2056, 8, 1, 60), (513, 129, 64, 4, 20), (2000, 768, 32, 1, 62)])
 @pytest.mark.parametrize('dtype,w_dtype', [(torch.bfloat16, torch.bfloat16), (torch.float16, torch.float32), (torch.float32, torch.float32), (torch.float16, None)])
 def test_both_gradients_of_binned_scatter_in_one_pass(kernels, sl, hs, ne, top_k, cap, dtype, w_dtype):
