@@ -40,7 +40,8 @@ struct Parts {
 // A training step's three buffers: what the forward keeps for the backward, and what either needs for itself.
 struct StepParts {
   Layout kept, forward, backward;
-  size_t indices, bin_ids, bins, slot_rows, weights[3], rows, x1, x2, hidden, product;   // kept
+  size_t indices, bin_ids, bins, slot_rows, weights[3], rows, x1, x2, hidden;             // kept
+  size_t product;                                                                        // kept with MBX_STEP_KEEP_PRODUCT, else the forward's own
   size_t sort, sort_bytes, hidden_forward;                                               // forward
   size_t grad_rows, d1, d2, table, table_bytes, hidden_again;                            // backward
   StepParts(int64_t tokens, int top_k, int num_experts, int end_bit, int hidden_size, int ffn, bool gate, int flags) {
@@ -56,10 +57,11 @@ struct StepParts {
     x2 = gate ? kept.take(wide) : 0;
     const bool again = flags & MBX_STEP_RECOMPUTE;
     hidden = again ? 0 : kept.take(wide);
-    product = kept.take(narrow);
+    if (flags & MBX_STEP_KEEP_PRODUCT) product = kept.take(narrow);
     sort_bytes = mbx_sort_scratch_bytes(n ? n : 1, MBX_I32, end_bit);
     sort = forward.take(sort_bytes);
     hidden_forward = again ? forward.take(wide) : 0;
+    if (!(flags & MBX_STEP_KEEP_PRODUCT)) product = forward.take(narrow);
     grad_rows = backward.take(narrow);
     d1 = backward.take(wide);
     d2 = gate ? backward.take(wide) : 0;
@@ -156,7 +158,8 @@ int mbx_experts_step_forward(const void* x, int64_t tokens, int hidden_size, int
   char* const base = (char*)kept;
   int32_t *const indices = (int32_t*)(base + p.indices), *const bin_ids = (int32_t*)(base + p.bin_ids);
   int32_t *const slot_rows = (int32_t*)(base + p.slot_rows), *const bins = (int32_t*)(base + p.bins);
-  void *const x1 = base + p.x1, *const x2 = v1 ? base + p.x2 : nullptr, *const y = base + p.product;
+  void *const x1 = base + p.x1, *const x2 = v1 ? base + p.x2 : nullptr;
+  void* const y = (flags & MBX_STEP_KEEP_PRODUCT ? base : (char*)scratch) + p.product;
   void* const h = flags & MBX_STEP_RECOMPUTE ? (char*)scratch + p.hidden_forward : base + p.hidden;
   int rc = mbx_route(expert_ids, slots, num_experts, end_bit, 0, indices, bin_ids, tokens_per_expert, bins, nullptr, slot_rows, (char*)scratch + p.sort, p.sort_bytes, stream);
   if (rc) return rc;
@@ -207,7 +210,7 @@ int mbx_experts_step_backward(const void* grad, const void* x, int64_t tokens, i
   char* const own = (char*)scratch;
   const int32_t *const indices = (const int32_t*)(base + p.indices), *const bin_ids = (const int32_t*)(base + p.bin_ids);
   const int32_t *const slot_rows = (const int32_t*)(base + p.slot_rows), *const bins = (const int32_t*)(base + p.bins);
-  const void *const x1 = base + p.x1, *const x2 = gate ? base + p.x2 : nullptr, *const y = base + p.product;
+  const void *const x1 = base + p.x1, *const x2 = gate ? base + p.x2 : nullptr, *const y = base + p.product;   // y: with MBX_STEP_KEEP_PRODUCT only
   const bool again = flags & MBX_STEP_RECOMPUTE;
   const void* const h = again ? own + p.hidden_again : base + p.hidden;
   if (fp32) {

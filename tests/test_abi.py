@@ -52,6 +52,19 @@ def test_error_strings_and_scratch_sizes():
         assert sizes == sorted(sizes)
 
 
+@pytest.mark.parametrize('top_k,flags', [(1, 2), (2, 0), (2, 32), (4, 1), (1, 2 | 8)])
+def test_a_step_keeps_the_second_product_only_for_the_gradient_of_the_weights(top_k, flags):
+    """MBX_STEP_KEEP_PRODUCT (4) holds [tokens top_k, hidden] from the forward to the backward; without it the product is the forward's own."""
+    from megablocks_amd._lib import lib
+    tokens, hidden, ffn = 512, 256, 1024
+
+    def sizes(f):
+        return [lib.mbx_experts_step_bytes(tokens, top_k, 8, 3, hidden, ffn, 1, f, which) for which in (0, 1, 2)]
+    product = tokens * top_k * hidden * 2
+    without, with_ = sizes(flags), sizes(flags | 4)
+    assert with_[0] - without[0] == product and without[1] - with_[1] == product and with_[2] == without[2]
+
+
 def test_argument_errors_are_reported_without_touching_the_gpu():
     from megablocks_amd._lib import lib
     assert lib.mbx_histogram(None, 7, 1, 1, 4, None, None) == -1           # bad itype / null out
