@@ -147,8 +147,10 @@ int mbx_experts_step_forward(const void* x, int64_t tokens, int hidden_size, int
   if (!sizes_ok(tokens, top_k, num_experts, end_bit, hidden_size, ffn)) return MBX_EINVAL;
   const int64_t slots = tokens * top_k;
   // what the launches of the backward take, which cannot go another way any more: 16-bit whole 16-byte pieces of rows, four K tiles to an
-  // operand pair of the gate's input gradient, more than a half-height tile of the indexed weight gradient, up to eight experts a token
+  // operand pair of the gate's input gradient, more than a half-height tile of the indexed weight gradient, up to eight experts a token, 256
+  // rows of an operand below 2 GiB (the gate's two halves of a tile: half a tile more)
   if ((dtype != MBX_BF16 && dtype != MBX_F16) || slots == 0 || hidden_size == 0 || hidden_size % 8 || ffn % 8 || ffn <= 192 || top_k > 8 ||
+      ffn >= (1 << 22) - 128 || hidden_size >= 1 << 22 ||
       slots * (int64_t)(hidden_size > ffn ? hidden_size : ffn) * 2 >= (int64_t)1 << 31 || (int64_t)hidden_size * ffn * 2 >= (int64_t)1 << 30)
     return MBX_EUNSUPPORTED;
   if (!x || !expert_ids || !weights || !w1 || !w2 || !out || !tokens_per_expert) return MBX_EINVAL;

@@ -651,6 +651,11 @@ EXPERTS_STEP_MAX_BYTES = 1 << 29
 _STEP_GATHER, _STEP_COMBINE, _STEP_KEEP_PRODUCT, _STEP_FP32_WEIGHTS, _STEP_GATE, _STEP_RECOMPUTE = 1, 2, 4, 8, 16, 32   # of include/mbx.h
 
 
+def _step_takes(hidden, ffn):
+    """Whether every launch of a step takes experts of these sizes: `mbx_experts_step_forward`'s own line, drawn ahead of the call."""
+    return hidden % 8 == 0 and ffn % 8 == 0 and 192 < ffn < (1 << 22) - 128 and 0 < ffn * hidden < 1 << 29
+
+
 class _ExpertsStep(torch.autograd.Function):
     """(out, tokens_per_expert) of `experts_step`; sizes: (num_experts, end_bit, top_k, ffn, act, flags, bytes kept)."""
 
@@ -731,7 +736,7 @@ def experts_step(x, expert_ids, expert_weights, num_experts, end_bit, top_k, w1,
             expert_weights.numel() != slots or expert_weights.dtype not in _lib.DTYPE:
         return None
     ffn = elements // (num_experts * hidden)
-    if hidden % 8 or ffn % 8 or ffn <= 192 or ffn * hidden >= 1 << 29 or not _use_epilogue(None, x, slots, ffn):
+    if not _step_takes(hidden, ffn) or not _use_epilogue(None, x, slots, ffn):
         return None
     for w in tensors[3:]:
         if w.dtype != w_dtype or w.numel() != elements or not w.is_contiguous() or w.data_ptr() % 16:

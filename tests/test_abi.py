@@ -65,6 +65,20 @@ def test_a_step_keeps_the_second_product_only_for_the_gradient_of_the_weights(to
     assert with_[0] - without[0] == product and without[1] - with_[1] == product and with_[2] == without[2]
 
 
+@pytest.mark.parametrize('hidden,ffn,taken', [
+    (64, 192, False), (64, 200, True), (60, 200, False), (64, 204, False), (8, (1 << 22) - 136, True),
+    (8, (1 << 22) - 128, False), (8, 1 << 22, False),    # 256 rows of 2^22 columns: 2 GiB, which the products leave to the kernels without epilogues
+    (1 << 21, 208, True), (1 << 22, 200, False), (1 << 15, 1 << 14, False)])
+def test_sizes_a_step_takes_are_the_librarys(hidden, ffn, taken):
+    """What the layer gives to the one call and what that call takes are one line: it has no other way left once it is chosen."""
+    from megablocks_amd import grouped_gemm_util as gg
+    from megablocks_amd._lib import lib, EUNSUPPORTED, EINVAL
+    assert gg._step_takes(hidden, ffn) == taken
+    # without operands: sizes that are taken are refused for that only
+    code = lib.mbx_experts_step_forward(None, 2, hidden, 0, None, 1, None, 0, 1, 1, None, None, None, ffn, 1, 0, None, None, None, 0, None, 0, None, 0, None)
+    assert code == (EINVAL if taken else EUNSUPPORTED)
+
+
 def test_argument_errors_are_reported_without_touching_the_gpu():
     from megablocks_amd._lib import lib
     assert lib.mbx_histogram(None, 7, 1, 1, 4, None, None) == -1           # bad itype / null out
