@@ -476,10 +476,17 @@ int mbx_router_input_gradient(const void* grad_logits, const void* weight, const
  * piece). */
 int mbx_sum_parts(const float* parts, int num_parts, int64_t pitch, void* out, int dtype, int64_t n, mbx_stream_t stream);
 
-/* The sums of the router's auxiliary losses and their gradients.  out[0] = scale * sum over i < n of values[i] * counts[i % period]
- * (megablocks/layers/moe.py:69-89 for one layer: values the scores [tokens, period], counts the tokens per expert), or with counts NULL of
- * values[i]^2 (megablocks/layers/router.py:37-42: values the logsumexp of the logits; period 1), in fp32.  scratch: mbx_loss_scratch_bytes(n) bytes (0: NULL).
- * Gradient: out[i] (of type dtype) = grad[0] * scale * counts[i % period], or grad[0] * scale * 2 values[i]. */
+/* The sums of the router's auxiliary losses and their gradients, of all layers that saved something.  out[l] = scales[l] * sum over i < n[l] of
+ * values[l][i] * counts[l][i % period] (megablocks/layers/moe.py:69-89: values the scores [tokens, period], counts the tokens per expert), or with counts NULL
+ * of values[l][i]^2 (megablocks/layers/router.py:37-42: values the logsumexp of the logits; period 1), in fp32.  scratch: mbx_loss_sums_scratch_bytes(the
+ * largest n[l], layers) bytes (0: NULL).  Gradient: out[l][i] (of type dtype) = grad[l] * scales[l] * counts[l][i % period] (values may be NULL), or
+ * grad[l] * scales[l] * 2 values[l][i]; out[l] NULL: not wanted.  The arrays of pointers, n and scales are in host memory, read before the call returns. */
+size_t mbx_loss_sums_scratch_bytes(int64_t n, int layers);
+int mbx_loss_sums(const void* const* values, int dtype, const int32_t* const* counts, const int64_t* n, const float* scales, int layers,
+                  int period, float* out, float* scratch, mbx_stream_t stream);
+int mbx_loss_gradients(const float* grad, const void* const* values, int dtype, const int32_t* const* counts, const int64_t* n, const float* scales,
+                       int layers, int period, void* const* out, mbx_stream_t stream);
+/* The same of one layer. */
 size_t mbx_loss_scratch_bytes(int64_t n);
 int mbx_loss_sum(const void* values, int dtype, const int32_t* counts, int64_t n, int period, float scale, float* out, float* scratch,
                  mbx_stream_t stream);

@@ -77,6 +77,9 @@ _SIGNATURES = {
     'mbx_loss_scratch_bytes': (_sz, [_i64]),
     'mbx_loss_sum': (_i, [_vp, _i, _vp, _i64, _i, ctypes.c_float, _vp, _vp, _vp]),
     'mbx_loss_gradient': (_i, [_vp, _vp, _i, _vp, _i64, _i, ctypes.c_float, _vp, _vp]),
+    'mbx_loss_sums_scratch_bytes': (_sz, [_i64, _i]),
+    'mbx_loss_sums': (_i, [_vp, _i, _vp, _vp, _vp, _i, _i, _vp, _vp, _vp]),
+    'mbx_loss_gradients': (_i, [_vp, _vp, _i, _vp, _vp, _vp, _i, _i, _vp, _vp]),
     'mbx_router_input_gradient': (_i, [_vp, _vp, _vp, _i, _i64, _i, _i, _vp, _vp, _vp]),
     'mbx_sum_parts': (_i, [_vp, _i, _i64, _vp, _i, _i64, _vp]),
     'mbx_router_backward': (_i, [_vp, _vp, _vp, _vp, _i, _i64, _i, _i, ctypes.c_float, _vp, _vp, _vp]),

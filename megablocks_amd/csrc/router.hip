@@ -392,11 +392,24 @@ sum_parts_kernel(const float* __restrict__ parts, int num_parts, int64_t pitch, 
 }
 
 // The sums of the auxiliary losses: values[i] counts[i % period] (the load-balancing loss: scores and tokens per expert), or without
-// counts values[i]^2 (the z-loss).  A sum of up to kLossOneBlock values is one workgroup's, a longer one is cut into runs of kLossRun for a workgroup
-// each, whose sums a second launch adds in order.  What bounds a loss of a small model is the number of launches: as torch's operations the two losses
-// are ten of 1 - 7 us forward and ten backward, each with a node of its own (a step of 1024 tokens, 8 experts, the host in its slower mode: 825 us with
-// them, 695 with these four).
-constexpr int kLossThreads = 1024, kLossOneBlock = 32 * kLossThreads, kLossRun = 8 * kLossThreads, kLossParts = 256;
+// counts values[i]^2 (the z-loss), for all saved layers by one launch, a row of workgroups each.  A layer's sum of up to kLossOneBlock values is one
+// workgroup's, a longer one is cut into runs of kLossRun for a workgroup each, whose sums a second launch adds in order.  What bounds the losses is the
+// number of launches and the calls behind them: as torch's operations the two are ten of 1 - 7 us forward and ten backward for a layer, each with a node of
+// its own (a step of 1024 tokens, 8 experts, the host in its slower mode: 825 us with them, 695 with these four); with a launch and a call for every layer
+// the z-loss of 32 took 1400 us of the host's time each way together, with one for all 1105, torch's operations 2166.
+constexpr int kLossThreads = 1024, kLossOneBlock = 32 * kLossThreads, kLossRun = 8 * kLossThreads, kLossParts = 256, kLossLayers = 64;
+
+struct LossLayers {   // of one launch, in its arguments
+  const void* values[kLossLayers];
+  const int32_t* counts[kLossLayers];
+  void* out[kLossLayers];   // the gradients
+  int64_t n[kLossLayers];
+  float scale[kLossLayers];
+};
+
+__host__ __device__ constexpr int loss_blocks(int64_t n) {
+  return n <= kLossOneBlock ? 1 : n > (int64_t)kLossParts * kLossRun ? kLossParts : (int)((n + kLossRun - 1) / kLossRun);
+}
 
 __device__ __forceinline__ float block_sum(float v) {   // in thread 0
   __shared__ float sums[kLossThreads / kWave];
@@ -408,11 +421,15 @@ __device__ __forceinline__ float block_sum(float v) {   // in thread 0
 }
 
 template <int DT>
-__global__ void __launch_bounds__(kLossThreads)
-loss_sum_kernel(const void* __restrict__ values_, const int32_t* __restrict__ counts, int64_t n, int period, float scale, float* __restrict__ out) {
+__global__ void __launch_bounds__(kLossThreads) loss_sum_kernel(const LossLayers layers, int period, float* __restrict__ out, float* __restrict__ parts) {
   typedef typename Elem<DT>::type E;
-  const E* const values = (const E*)values_;
-  const int64_t stride = (int64_t)gridDim.x * kLossThreads;
+  const int layer = blockIdx.y;
+  const int64_t n = layers.n[layer];
+  const int blocks = loss_blocks(n);
+  if ((int)blockIdx.x >= blocks) return;
+  const E* __restrict__ const values = (const E*)layers.values[layer];
+  const int32_t* __restrict__ const counts = layers.counts[layer];
+  const int64_t stride = (int64_t)blocks * kLossThreads;
   int64_t i = (int64_t)blockIdx.x * kLossThreads + threadIdx.x;
   int e = (int)(i % period);
   const int step = (int)(stride % period);
@@ -425,27 +442,35 @@ loss_sum_kernel(const void* __restrict__ values_, const int32_t* __restrict__ co
     e = e >= period ? e - period : e;
   }
   sum = block_sum(sum);
-  if (threadIdx.x == 0) out[blockIdx.x] = scale * sum;
+  if (threadIdx.x != 0) return;
+  if (blocks == 1) out[layer] = layers.scale[layer] * sum;
+  else parts[layer * kLossParts + blockIdx.x] = sum;
 }
 
-__global__ void __launch_bounds__(kLossThreads) loss_parts_kernel(const float* __restrict__ parts, int count, float scale, float* __restrict__ out) {
-  const float sum = block_sum(threadIdx.x < (unsigned)count ? parts[threadIdx.x] : 0.f);
-  if (threadIdx.x == 0) *out = scale * sum;
+__global__ void __launch_bounds__(kLossThreads) loss_parts_kernel(const LossLayers layers, const float* __restrict__ parts, float* __restrict__ out) {
+  const int layer = blockIdx.x, blocks = loss_blocks(layers.n[layer]);
+  if (blocks == 1) return;
+  const float sum = block_sum((int)threadIdx.x < blocks ? parts[layer * kLossParts + threadIdx.x] : 0.f);
+  if (threadIdx.x == 0) out[layer] = layers.scale[layer] * sum;
 }
 
 // The sums' gradients: grad scale counts[i % period], or without counts grad scale 2 values[i].
 template <int DT>
-__global__ void __launch_bounds__(256)
-loss_gradient_kernel(const float* __restrict__ grad, const void* __restrict__ values_, const int32_t* __restrict__ counts, int64_t n, int period,
-                     float scale, void* __restrict__ out_) {
+__global__ void __launch_bounds__(256) loss_gradient_kernel(const float* __restrict__ grad, const LossLayers layers, int period) {
   typedef typename Elem<DT>::type E;
-  const float g = *grad * scale;
+  const int layer = blockIdx.y;
+  E* __restrict__ const out = (E*)layers.out[layer];
+  if (out == nullptr) return;
+  const E* __restrict__ const values = (const E*)layers.values[layer];
+  const int32_t* __restrict__ const counts = layers.counts[layer];
+  const int64_t n = layers.n[layer];
+  const float g = grad[layer] * layers.scale[layer];
   const int64_t stride = (int64_t)gridDim.x * 256;
   int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   int e = (int)(i % period);
   const int step = (int)(stride % period);
   for (; i < n; i += stride) {
-    ((E*)out_)[i] = Elem<DT>::from_f32(counts ? g * (float)counts[e] : g * (2.f * Elem<DT>::to_f32(((const E*)values_)[i])));
+    out[i] = Elem<DT>::from_f32(counts ? g * (float)counts[e] : g * (2.f * Elem<DT>::to_f32(values[i])));
     e += step;
     e = e >= period ? e - period : e;
   }
@@ -591,41 +616,85 @@ int mbx_sum_parts(const float* parts, int num_parts, int64_t pitch, void* out, i
   return launch_status();
 }
 
-int mbx_loss_sum(const void* values, int dtype, const int32_t* counts, int64_t n, int period, float scale, float* out, float* scratch,
-                 mbx_stream_t stream) {
-  if (n < 0 || period <= 0 || (dtype != MBX_BF16 && dtype != MBX_F16 && dtype != MBX_F32)) return MBX_EINVAL;
-  if (!out || (n > 0 && !values)) return MBX_EINVAL;
-  if (n > kLossOneBlock && !scratch) return MBX_ESCRATCH;
-  hipStream_t s = as_stream(stream);
-  const int64_t runs = ceil_div(n, kLossRun);
-  const unsigned blocks = n <= kLossOneBlock ? 1u : (unsigned)(runs < kLossParts ? runs : kLossParts);
-  float* const to = blocks > 1 ? scratch : out;
-  const float by = blocks > 1 ? 1.f : scale;
-  switch (dtype) {
-    case MBX_BF16: loss_sum_kernel<MBX_BF16><<<blocks, kLossThreads, 0, s>>>(values, counts, n, period, by, to); break;
-    case MBX_F16: loss_sum_kernel<MBX_F16><<<blocks, kLossThreads, 0, s>>>(values, counts, n, period, by, to); break;
-    default: loss_sum_kernel<MBX_F32><<<blocks, kLossThreads, 0, s>>>(values, counts, n, period, by, to); break;
+size_t mbx_loss_sums_scratch_bytes(int64_t n, int layers) { return n > kLossOneBlock && layers > 0 ? (size_t)layers * kLossParts * sizeof(float) : 0; }
+
+int mbx_loss_sums(const void* const* values, int dtype, const int32_t* const* counts, const int64_t* n, const float* scales, int layers,
+                  int period, float* out, float* scratch, mbx_stream_t stream) {
+  if (layers < 0 || period <= 0 || (dtype != MBX_BF16 && dtype != MBX_F16 && dtype != MBX_F32)) return MBX_EINVAL;
+  if (layers == 0) return 0;
+  if (!out || !values || !n || !scales) return MBX_EINVAL;
+  for (int l = 0; l < layers; ++l) {
+    if (n[l] < 0 || (n[l] > 0 && !values[l]) || (counts && n[l] > 0 && !counts[l])) return MBX_EINVAL;
+    if (n[l] > kLossOneBlock && !scratch) return MBX_ESCRATCH;
   }
-  if (blocks > 1) loss_parts_kernel<<<1, kLossThreads, 0, s>>>(scratch, (int)blocks, scale, out);
+  hipStream_t s = as_stream(stream);
+  for (int first = 0; first < layers; first += kLossLayers) {
+    LossLayers of = {};
+    const int count = layers - first < kLossLayers ? layers - first : kLossLayers;
+    int blocks = 1;
+    for (int l = 0; l < count; ++l) {
+      of.values[l] = values[first + l];
+      of.counts[l] = counts ? counts[first + l] : nullptr;
+      of.n[l] = n[first + l];
+      of.scale[l] = scales[first + l];
+      blocks = loss_blocks(of.n[l]) > blocks ? loss_blocks(of.n[l]) : blocks;
+    }
+    float* const to = out + first;
+    float* const parts = scratch ? scratch + (int64_t)first * kLossParts : nullptr;
+    const dim3 grid((unsigned)blocks, (unsigned)count);
+    switch (dtype) {
+      case MBX_BF16: loss_sum_kernel<MBX_BF16><<<grid, kLossThreads, 0, s>>>(of, period, to, parts); break;
+      case MBX_F16: loss_sum_kernel<MBX_F16><<<grid, kLossThreads, 0, s>>>(of, period, to, parts); break;
+      default: loss_sum_kernel<MBX_F32><<<grid, kLossThreads, 0, s>>>(of, period, to, parts); break;
+    }
+    if (blocks > 1) loss_parts_kernel<<<(unsigned)count, kLossThreads, 0, s>>>(of, parts, to);
+  }
   return launch_status();
 }
 
-size_t mbx_loss_scratch_bytes(int64_t n) { return n > kLossOneBlock ? kLossParts * sizeof(float) : 0; }
+int mbx_loss_gradients(const float* grad, const void* const* values, int dtype, const int32_t* const* counts, const int64_t* n, const float* scales,
+                       int layers, int period, void* const* out, mbx_stream_t stream) {
+  if (layers < 0 || period <= 0 || (dtype != MBX_BF16 && dtype != MBX_F16 && dtype != MBX_F32)) return MBX_EINVAL;
+  if (layers == 0) return 0;
+  if (!grad || !out || !n || !scales || (!counts && !values)) return MBX_EINVAL;
+  for (int l = 0; l < layers; ++l)
+    if (n[l] < 0 || (out[l] && n[l] > 0 && !(counts ? (const void*)counts[l] : values[l]))) return MBX_EINVAL;
+  hipStream_t s = as_stream(stream);
+  for (int first = 0; first < layers; first += kLossLayers) {
+    LossLayers of = {};
+    const int count = layers - first < kLossLayers ? layers - first : kLossLayers;
+    int64_t most = 0;
+    for (int l = 0; l < count; ++l) {
+      of.values[l] = counts ? nullptr : values[first + l];
+      of.counts[l] = counts ? counts[first + l] : nullptr;
+      of.out[l] = out[first + l];
+      of.n[l] = n[first + l];
+      of.scale[l] = scales[first + l];
+      if (of.out[l] && of.n[l] > most) most = of.n[l];
+    }
+    if (most == 0) continue;
+    const int64_t wanted = ceil_div(most, 256);
+    const dim3 grid((unsigned)(wanted < 2048 ? wanted : 2048), (unsigned)count);
+    switch (dtype) {
+      case MBX_BF16: loss_gradient_kernel<MBX_BF16><<<grid, 256, 0, s>>>(grad + first, of, period); break;
+      case MBX_F16: loss_gradient_kernel<MBX_F16><<<grid, 256, 0, s>>>(grad + first, of, period); break;
+      default: loss_gradient_kernel<MBX_F32><<<grid, 256, 0, s>>>(grad + first, of, period); break;
+    }
+  }
+  return launch_status();
+}
+
+size_t mbx_loss_scratch_bytes(int64_t n) { return mbx_loss_sums_scratch_bytes(n, 1); }
+
+int mbx_loss_sum(const void* values, int dtype, const int32_t* counts, int64_t n, int period, float scale, float* out, float* scratch,
+                 mbx_stream_t stream) {
+  return mbx_loss_sums(&values, dtype, counts ? &counts : nullptr, &n, &scale, 1, period, out, scratch, stream);
+}
 
 int mbx_loss_gradient(const float* grad, const void* values, int dtype, const int32_t* counts, int64_t n, int period, float scale, void* out,
                       mbx_stream_t stream) {
-  if (n < 0 || period <= 0 || (dtype != MBX_BF16 && dtype != MBX_F16 && dtype != MBX_F32)) return MBX_EINVAL;
-  if (n == 0) return 0;
-  if (!grad || !out || (!counts && !values)) return MBX_EINVAL;
-  hipStream_t s = as_stream(stream);
-  const int64_t wanted = ceil_div(n, 256);
-  const unsigned blocks = (unsigned)(wanted < 2048 ? wanted : 2048);
-  switch (dtype) {
-    case MBX_BF16: loss_gradient_kernel<MBX_BF16><<<blocks, 256, 0, s>>>(grad, values, counts, n, period, scale, out); break;
-    case MBX_F16: loss_gradient_kernel<MBX_F16><<<blocks, 256, 0, s>>>(grad, values, counts, n, period, scale, out); break;
-    default: loss_gradient_kernel<MBX_F32><<<blocks, 256, 0, s>>>(grad, values, counts, n, period, scale, out); break;
-  }
-  return launch_status();
+  if (n > 0 && !out) return MBX_EINVAL;
+  return mbx_loss_gradients(grad, &values, dtype, counts ? &counts : nullptr, &n, &scale, 1, period, &out, stream);
 }
 
 }  // extern "C"

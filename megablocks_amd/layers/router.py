@@ -2,6 +2,7 @@
 GEMM), except for its gradients on large 16-bit batches, which go through the grouped kernels;
 softmax, top-k and the renormalisation of the selected weights are one HIP kernel each way.  The outputs
 feed the HIP routing kernels."""
+import ctypes
 from typing import Any
 
 import torch
@@ -26,49 +27,56 @@ def _save_router_logits(logits: torch.Tensor, args: Arguments, lse=None):
 
 class LossSums(torch.autograd.Function):
     """[scales[l] * sum(values[l] * counts[l]) for l] with counts[l] a row for every row of values[l], or (counts None) * sum(values[l]^2): the
-    sums of the auxiliary losses (moe.py:69-89, router.py:37-42), fp32, a launch each (two for long ones) forward and backward."""
+    sums of the auxiliary losses (moe.py:69-89, router.py:37-42), fp32, of all layers by one launch (two for long ones) forward and one backward."""
 
     @staticmethod
     def takes(values, counts) -> bool:
-        """Plain contiguous tensors on the GPU, the counts int32, and nothing that acts on torch's operators at work (autocast does not
-        cast these)."""
-        plain = lambda t, device: type(t) is torch.Tensor and t.is_cuda and t.device == device and t.is_contiguous()
-        device = values[0].device
-        return all(plain(v, device) and v.dtype in _lib.DTYPE and v.numel() for v in values) and \
-            (counts is None or all(plain(c, device) and c.dtype == torch.int32 for c in counts)) and common.only_computed(autocast=True)
+        """Plain contiguous tensors on the GPU, the values of one type, the counts int32, and nothing that acts on torch's operators at work (autocast
+        does not cast these)."""
+        device, dtype = values[0].device, values[0].dtype
+        plain = lambda t, dtype: type(t) is torch.Tensor and t.dtype == dtype and t.device == device and t.is_contiguous()
+        return values[0].is_cuda and dtype in _lib.DTYPE and all(plain(v, dtype) and v.numel() for v in values) and \
+            (counts is None or all(plain(c, torch.int32) for c in counts)) and common.only_computed(autocast=True)
+
+    @staticmethod
+    def _arrays(sizes, scales):
+        return (ctypes.c_int64 * len(sizes))(*sizes), (ctypes.c_float * len(scales))(*scales)
+
+    @staticmethod
+    def _pointers(tensors):
+        return (ctypes.c_void_p * len(tensors))(*map(_lib.ptr, tensors))
 
     @staticmethod
     def forward(ctx: Any, scales, counts, *values):
-        out = torch.empty(len(values), dtype=torch.float32, device=values[0].device)
+        first, layers = values[0], len(values)
+        period = 1 if counts is None else first.shape[1]
+        sizes = [v.numel() for v in values]
+        out = torch.empty(layers, dtype=torch.float32, device=first.device)
+        nbytes = _lib.lib.mbx_loss_sums_scratch_bytes(max(sizes), layers)
+        scratch = torch.empty(nbytes, dtype=torch.uint8, device=first.device) if nbytes else None
         with _lib.device_of(out):
-            for l, v in enumerate(values):
-                nbytes = _lib.lib.mbx_loss_scratch_bytes(v.numel())
-                scratch = torch.empty(nbytes, dtype=torch.uint8, device=v.device) if nbytes else None
-                _lib.check(_lib.lib.mbx_loss_sum(_lib.ptr(v), _lib.dtype_of(v), None if counts is None else _lib.ptr(counts[l]), v.numel(),
-                                                 1 if counts is None else v.shape[1], scales[l], out.data_ptr() + 4 * l, _lib.ptr(scratch),
-                                                 _lib.stream()), 'loss_sum')
+            _lib.check(_lib.lib.mbx_loss_sums(LossSums._pointers(values), _lib.dtype_of(first), None if counts is None else LossSums._pointers(counts),
+                                              *LossSums._arrays(sizes, scales), layers, period, _lib.ptr(out), _lib.ptr(scratch), _lib.stream()),
+                       'loss_sums')
         ctx.save_for_backward(*(values if counts is None else counts))
-        ctx.scales, ctx.counted, ctx.like = scales, counts is not None, [(v.shape, v.dtype) for v in values]
+        ctx.scales, ctx.counted, ctx.period, ctx.shapes, ctx.dtype = scales, counts is not None, period, [v.shape for v in values], first.dtype
         return out
 
     @staticmethod
     def backward(ctx: Any, grad):
-        grads = []
+        saved, wanted, layers = ctx.saved_tensors, ctx.needs_input_grad[2:], len(ctx.shapes)
+        grad = grad.float().contiguous()
+        if torch.is_grad_enabled() or not _has_memory(grad):   # differentiated itself, or over a batch of gradients
+            by = [scale if ctx.counted else 2 * scale for scale in ctx.scales]
+            return (None, None, *((grad[l] * by[l] * saved[l].float()).to(ctx.dtype).expand(ctx.shapes[l]) if wanted[l] else None
+                                  for l in range(layers)))
+        saved = [t.contiguous() for t in saved]
+        grads = [torch.empty(shape, dtype=ctx.dtype, device=grad.device) if want else None for shape, want in zip(ctx.shapes, wanted)]
+        pointers = LossSums._pointers(saved)
         with _lib.device_of(grad):
-            grad = grad.float().contiguous()
-            for l, (saved, scale, (shape, dtype)) in enumerate(zip(ctx.saved_tensors, ctx.scales, ctx.like)):
-                if not ctx.needs_input_grad[2 + l]:
-                    g = None
-                elif torch.is_grad_enabled() or not _has_memory(grad):   # differentiated itself, or over a batch of gradients
-                    g = grad[l] * scale * saved.float() if ctx.counted else grad[l] * (2 * scale) * saved.float()
-                    g = g.to(dtype).expand(shape)
-                else:
-                    saved = saved.contiguous()
-                    g = torch.empty(shape, dtype=dtype, device=grad.device)
-                    _lib.check(_lib.lib.mbx_loss_gradient(grad.data_ptr() + 4 * l, None if ctx.counted else _lib.ptr(saved), _lib.DTYPE[dtype],
-                                                          _lib.ptr(saved) if ctx.counted else None, g.numel(),
-                                                          shape[1] if ctx.counted else 1, scale, _lib.ptr(g), _lib.stream()), 'loss_gradient')
-                grads.append(g)
+            _lib.check(_lib.lib.mbx_loss_gradients(_lib.ptr(grad), None if ctx.counted else pointers, _lib.DTYPE[ctx.dtype],
+                                                   pointers if ctx.counted else None, *LossSums._arrays([s.numel() for s in ctx.shapes], ctx.scales),
+                                                   layers, ctx.period, LossSums._pointers(grads), _lib.stream()), 'loss_gradients')
         return (None, None, *grads)
 
 

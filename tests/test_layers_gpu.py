@@ -1094,16 +1094,21 @@ def test_auxiliary_losses_match_oracle(dtype, in_fp32, tokens, hs, ne, top_k, la
 
 
 @pytest.mark.parametrize('dtype', [torch.float32, torch.bfloat16])
-@pytest.mark.parametrize('tokens,experts,layers', [(1, 1, 1), (4096, 8, 1), (4097, 8, 1), (300, 12, 3), (70000, 64, 1), (33, 512, 2)])
+@pytest.mark.parametrize('tokens,experts,layers', [(1, 1, 1), (4096, 8, 1), (4097, 8, 1), (300, 12, 3), (70000, 64, 1), (33, 512, 2), (40, 8, 64),
+                                                   (9000, 4, 66)])
 def test_sums_of_the_auxiliary_losses(monkeypatch, dtype, tokens, experts, layers):
     """LossSums against fp64, values and gradients, on both sides of where a sum is cut over workgroups: sums of non-negative terms, 2^-24 times
     the length of the longest chain (a thread's terms and ten steps of a tree, twice); the same from torch's operations, and where the
-    backward is differentiated or runs over a batch of gradients."""
+    backward is differentiated or runs over a batch of gradients.  However many layers: one call of the library each way (beyond 64, two launches of it)."""
+    from megablocks_amd import _lib
     from megablocks_amd.layers import common, router
+    calls = []
+    for name in ('mbx_loss_sums', 'mbx_loss_gradients'):
+        monkeypatch.setattr(_lib.lib, name, lambda *a, name=name, call=getattr(_lib.lib, name): calls.append(name) or call(*a))
     torch.manual_seed(tokens)
     scores = [torch.rand(tokens, experts, device='cuda').to(dtype) for _ in range(layers)]
     counts = [torch.randint(0, 5 * tokens + 2, (experts,), device='cuda', dtype=torch.int32) for _ in range(layers)]
-    lse = [torch.rand(tokens, device='cuda') + 1 for _ in range(layers)]
+    lse = [torch.rand(tokens + l, device='cuda') + 1 for l in range(layers)]
     scales, weight = [0.5 / (l + 1) for l in range(layers)], torch.rand(layers, device='cuda') + 1
     chain = -(-tokens * experts // (256 * 1024)) + 32 + 20
     for values, c in ((scores, counts), (lse, None)):
@@ -1111,6 +1116,8 @@ def test_sums_of_the_auxiliary_losses(monkeypatch, dtype, tokens, experts, layer
         leaves = [v.clone().requires_grad_(True) for v in values]
         got = router.LossSums.apply(scales, c, *leaves)
         grads = torch.autograd.grad(got, leaves, weight, retain_graph=True)
+        assert calls == ['mbx_loss_sums', 'mbx_loss_gradients']
+        calls.clear()
         again = torch.autograd.grad(got, leaves, weight, create_graph=True)
         batch = torch.autograd.grad(got, leaves, torch.stack([weight, 2 * weight]), is_grads_batched=True)
         for l in range(layers):
@@ -1135,7 +1142,9 @@ def test_sums_of_the_auxiliary_losses(monkeypatch, dtype, tokens, experts, layer
         for l in range(layers):
             moe.save_load_balancing_loss((counts[l], leaves[l]))
             router._save_router_logits(leaves[l], layer_args, leaves[layers + l])
+        calls.clear()
         lbl, z = moe.batched_load_balancing_loss(layer_args), router.batched_router_zloss(layer_args)
+        assert len(calls) == (0 if not fused else 2 if layers <= moe.LOSS_SUMS_MAX_LAYERS else 1)
         results.append([lbl, z, *torch.autograd.grad([lbl, z.sum()], leaves)])
     moe.clear_load_balancing_loss()
     router.clear_router_zloss()
