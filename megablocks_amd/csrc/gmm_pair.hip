@@ -270,7 +270,9 @@ bool gmm_pair_takes(const DmaCall& q) {
   auto row_tiles = [&](double height) { return experts * (average > 64 ? average / height + 0.5 : 1.0); };   // the row counts vary
   // here: a round is two tiles to a compute unit, which one by itself works off in little more than half the time
   const double tiles = row_tiles(128) * ceil(n / 128), rounds = floor(tiles / (2 * units)), rest = tiles / (2 * units) - rounds;
-  const bool may_cut = nn && q.epi == dma::kEpiNone && q.ws.base;
+  // gmm_dma.h's kernel cuts the combine's tails as the plain product's (120 combines, 4 - 128 experts of 17 - 1500 rows, mostly where it matters, over the
+  // shorter of the two: judged as cut 1.04, as never cut 1.13; 4 of 104, [13120, 512]: 58 us there, 130 here)
+  const bool may_cut = nn && (q.epi == dma::kEpiNone || q.epi == dma::kEpiCombine) && q.ws.base;
   const double line = gain_line(q, may_cut, nk, average, tiles / (2 * units));
   double here = 4.8 + rounds * nk * 1.2;
   if (rest > 0) here += nk * (rest <= 0.5 ? 0.56 : 0.56 + 0.64 * (2 * rest - 1));

@@ -563,7 +563,7 @@ class CombinedRows:
 def gmm_scatter(a, b, batch_sizes, combine: CombinedRows, keep_product=True):
     """(y, out): y[r_e] = a[r_e] @ b[e], the experts' second product (mlp.py:523, glu.py:205), and out =
     ops.scatter(y, indices, bin_ids, weights, bins, top_k = 1) (dmoe.py:280), the combine written by the product's
-    store phase (`mbx_gmm_scatter_ws`; bit-identical to the two steps).  y is None when `keep_product` is False and the
+    store phase (`mbx_gmm_scatter_ws`; bit-identical to the two steps where the same kernel takes the product without a combine).  y is None when `keep_product` is False and the
     launch did not have to write it (nothing will differentiate).  Shapes the kernel does not take: two steps."""
     _lib.require_cuda(a, b, combine.indices, combine.weights)
     if a.ndim != 2 or b.ndim != 3 or a.dtype != b.dtype or b.shape[1] != a.shape[1]:
