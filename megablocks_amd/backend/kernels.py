@@ -310,8 +310,10 @@ def binned_scatter(x, indices, weights, bins, top_k):
     indices, bins = _lib.as_i32(indices), _lib.as_i32(bins)
     wp, wdt, weights = _w(weights)
     out = torch.empty((tokens, hidden_size), dtype=x.dtype, device=x.device)
-    # the map that came with the routing, if these are its assignments and bins (see _slot_rows)
-    rows = None if not num_experts or torch.cuda.is_current_stream_capturing() else _kept_slot_rows(indices, _slot_rows_key(indices, bins, None))
+    # the map that came with the routing, if these are its assignments and bins (see _slot_rows); inference tensors have no version to tell by
+    rows = None
+    if num_experts and hasattr(indices, '_mbx_slot_rows') and not bins.is_inference() and not torch.cuda.is_current_stream_capturing():
+        rows = _kept_slot_rows(indices, _slot_rows_key(indices, bins, None))
     if rows is not None:
         with _lib.device_of(x):
             _lib.check(lib.mbx_binned_scatter_rows(_lib.ptr(x), _lib.dtype_of(x), tokens, hidden_size, top_k, _lib.ptr(rows), _lib.ptr(bins),

@@ -285,6 +285,25 @@ def test_binned_scatter_from_the_routings_map(kernels, sl, hs, ne, top_k, cap, w
     assert torch.equal(kernels.binned_scatter(x, indices, w, bins, top_k), kernels.binned_scatter(x, plain.flip(0), w, bins, top_k))
 
 
+@pytest.mark.parametrize('routed', [False, True])
+def test_binned_scatter_of_inference_tensors(kernels, routed):
+    """Assignments and bins made in inference mode, which have no version that a kept map could be told by, alone and next to ordinary ones."""
+    import megablocks_amd.ops as ops
+    from megablocks_amd.ops import routing
+    torch.manual_seed(0)
+    ids = (torch.rand(600, device='cuda') * 8).int()
+    if routed:
+        indices, _, _, bins, _ = routing.route(ids, 8, 3)
+    else:
+        indices, bins = ops.sort(ids, 3)[1], ops.inclusive_cumsum(ops.histogram(ids, 8), 0)
+    x, w = torch.randn(8, 50, 64, device='cuda').half(), torch.rand(600, device='cuda').half()
+    want = ops.binned_scatter(x, indices, w, bins, 2)
+    with torch.inference_mode():
+        i, b = indices.clone(), bins.clone()
+        forms = [(indices, bins), (i, b), (i, bins), (indices, b), (indices.long(), bins), (indices, bins.long())]
+        assert all(torch.equal(ops.binned_scatter(x, *form[:1], w, *form[1:], 2), want) for form in forms)
+
+
 def test_a_map_is_used_on_its_own_stream_only(kernels):
     """Whoever uses the assignments on a second stream waits for them and marks them as in use there; a map kept from the first, which nobody could
     mark, is not read there, by none of the operators, and one made there is not read on the first."""
