@@ -27,7 +27,8 @@ def _save_router_logits(logits: torch.Tensor, args: Arguments, lse=None):
 
 class LossSums(torch.autograd.Function):
     """[scales[l] * sum(values[l] * counts[l]) for l] with counts[l] a row for every row of values[l], or (counts None) * sum(values[l]^2): the
-    sums of the auxiliary losses (moe.py:69-89, router.py:37-42), fp32, of all layers by one launch (two for long ones) forward and one backward."""
+    sums of the auxiliary losses (moe.py:69-89, router.py:37-42), fp32, of all layers by one launch (two for long ones) forward and one backward.
+    A single layer goes without the arrays of those for many, 2 us of the host's time a call."""
 
     @staticmethod
     def takes(values, counts) -> bool:
@@ -55,9 +56,13 @@ class LossSums(torch.autograd.Function):
         nbytes = _lib.lib.mbx_loss_sums_scratch_bytes(max(sizes), layers)
         scratch = torch.empty(nbytes, dtype=torch.uint8, device=first.device) if nbytes else None
         with _lib.device_of(out):
-            _lib.check(_lib.lib.mbx_loss_sums(LossSums._pointers(values), _lib.dtype_of(first), None if counts is None else LossSums._pointers(counts),
-                                              *LossSums._arrays(sizes, scales), layers, period, _lib.ptr(out), _lib.ptr(scratch), _lib.stream()),
-                       'loss_sums')
+            if layers == 1:
+                rc = _lib.lib.mbx_loss_sum(_lib.ptr(first), _lib.dtype_of(first), None if counts is None else _lib.ptr(counts[0]), sizes[0], period,
+                                           scales[0], _lib.ptr(out), _lib.ptr(scratch), _lib.stream())
+            else:
+                rc = _lib.lib.mbx_loss_sums(LossSums._pointers(values), _lib.dtype_of(first), None if counts is None else LossSums._pointers(counts),
+                                            *LossSums._arrays(sizes, scales), layers, period, _lib.ptr(out), _lib.ptr(scratch), _lib.stream())
+            _lib.check(rc, 'loss_sums')
         ctx.save_for_backward(*(values if counts is None else counts))
         ctx.scales, ctx.counted, ctx.period, ctx.shapes, ctx.dtype = scales, counts is not None, period, [v.shape for v in values], first.dtype
         return out
@@ -72,11 +77,18 @@ class LossSums(torch.autograd.Function):
                                   for l in range(layers)))
         saved = [t.contiguous() for t in saved]
         grads = [torch.empty(shape, dtype=ctx.dtype, device=grad.device) if want else None for shape, want in zip(ctx.shapes, wanted)]
-        pointers = LossSums._pointers(saved)
         with _lib.device_of(grad):
-            _lib.check(_lib.lib.mbx_loss_gradients(_lib.ptr(grad), None if ctx.counted else pointers, _lib.DTYPE[ctx.dtype],
-                                                   pointers if ctx.counted else None, *LossSums._arrays([s.numel() for s in ctx.shapes], ctx.scales),
-                                                   layers, ctx.period, LossSums._pointers(grads), _lib.stream()), 'loss_gradients')
+            if layers == 1:
+                values, counts = (None, _lib.ptr(saved[0])) if ctx.counted else (_lib.ptr(saved[0]), None)
+                rc = _lib.lib.mbx_loss_gradient(_lib.ptr(grad), values, _lib.DTYPE[ctx.dtype], counts, ctx.shapes[0].numel(), ctx.period, ctx.scales[0],
+                                                _lib.ptr(grads[0]), _lib.stream())
+            else:
+                pointers = LossSums._pointers(saved)
+                values, counts = (None, pointers) if ctx.counted else (pointers, None)
+                rc = _lib.lib.mbx_loss_gradients(_lib.ptr(grad), values, _lib.DTYPE[ctx.dtype], counts,
+                                                 *LossSums._arrays([s.numel() for s in ctx.shapes], ctx.scales), layers, ctx.period,
+                                                 LossSums._pointers(grads), _lib.stream())
+            _lib.check(rc, 'loss_gradients')
         return (None, None, *grads)
 
 

@@ -1099,11 +1099,12 @@ def test_auxiliary_losses_match_oracle(dtype, in_fp32, tokens, hs, ne, top_k, la
 def test_sums_of_the_auxiliary_losses(monkeypatch, dtype, tokens, experts, layers):
     """LossSums against fp64, values and gradients, on both sides of where a sum is cut over workgroups: sums of non-negative terms, 2^-24 times
     the length of the longest chain (a thread's terms and ten steps of a tree, twice); the same from torch's operations, and where the
-    backward is differentiated or runs over a batch of gradients.  However many layers: one call of the library each way (beyond 64, two launches of it)."""
+    backward is differentiated or runs over a batch of gradients.  However many layers: one call of the library each way (beyond 64, two launches of it;
+    a single layer's has no arrays of pointers)."""
     from megablocks_amd import _lib
     from megablocks_amd.layers import common, router
-    calls = []
-    for name in ('mbx_loss_sums', 'mbx_loss_gradients'):
+    calls, both = [], ['mbx_loss_sum', 'mbx_loss_gradient'] if layers == 1 else ['mbx_loss_sums', 'mbx_loss_gradients']
+    for name in ('mbx_loss_sum', 'mbx_loss_gradient', 'mbx_loss_sums', 'mbx_loss_gradients'):
         monkeypatch.setattr(_lib.lib, name, lambda *a, name=name, call=getattr(_lib.lib, name): calls.append(name) or call(*a))
     torch.manual_seed(tokens)
     scores = [torch.rand(tokens, experts, device='cuda').to(dtype) for _ in range(layers)]
@@ -1116,7 +1117,7 @@ def test_sums_of_the_auxiliary_losses(monkeypatch, dtype, tokens, experts, layer
         leaves = [v.clone().requires_grad_(True) for v in values]
         got = router.LossSums.apply(scales, c, *leaves)
         grads = torch.autograd.grad(got, leaves, weight, retain_graph=True)
-        assert calls == ['mbx_loss_sums', 'mbx_loss_gradients']
+        assert calls == both
         calls.clear()
         again = torch.autograd.grad(got, leaves, weight, create_graph=True)
         batch = torch.autograd.grad(got, leaves, torch.stack([weight, 2 * weight]), is_grads_batched=True)
