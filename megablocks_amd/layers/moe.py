@@ -26,11 +26,6 @@ def clear_load_balancing_loss():
     _LOAD_BALANCING_LOSS.clear()
 
 
-# Layers up to which the loss takes router.LossSums: a layer is an input of its node and a gradient tensor of its own there, where torch joins the scores
-# first (host time of the loss and its backward, us, here / torch: 1 layer 137 / 158, 2 178 / 182, 4 240 / 237, 8 363 / 341, 32 1126 / 1001).
-LOSS_SUMS_MAX_LAYERS = 2
-
-
 def batched_load_balancing_loss(args: Arguments):
     """moe.py:32-89: loss_weight * E / (layers * tokens * top_k) * <tokens_per_expert, mean scores>."""
     if args.moe_loss_weight == 0:
@@ -48,10 +43,11 @@ def batched_load_balancing_loss(args: Arguments):
     tokens = expert_scores[0].shape[0]
     assert all(((x.ndim == 2 and x.shape[1] == args.moe_num_experts and x.shape[0] == tokens) for x in expert_scores))
     scale = (args.moe_num_experts * args.moe_loss_weight) / (args.num_layers * tokens * args.moe_top_k) if tokens else 0.0
-    if 0 < layers <= LOSS_SUMS_MAX_LAYERS and tokens and all(args.moe_lbl_in_fp32 or x.dtype == torch.float32 for x in expert_scores) and \
+    # One layer: in many, each is an input of the sums' node and a gradient tensor of its own there, where torch joins the scores first (host time of the
+    # loss and its backward, us, by the sums / by torch, two boxes: 1 layer 107 / 119, 2 144 / 138 and 178 / 182, 4 169 / 166 and 240 / 237, 32 1126 / 1001)
+    if layers == 1 and tokens and (args.moe_lbl_in_fp32 or expert_scores[0].dtype == torch.float32) and \
             router.LossSums.takes(expert_scores, tokens_per_expert):
-        sums = router.LossSums.apply([scale / tokens] * layers, tokens_per_expert, *expert_scores)
-        return sums.view(()) if layers == 1 else sums.sum()
+        return router.LossSums.apply([scale / tokens], tokens_per_expert, *expert_scores).view(())
     expert_scores = torch.cat(expert_scores, dim=1)
     if args.moe_lbl_in_fp32:
         expert_scores = expert_scores.float()
