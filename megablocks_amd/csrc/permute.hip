@@ -237,8 +237,8 @@ __device__ __forceinline__ void zero_unowned_rows(typename Elem<DT>::type* __res
 // Nothing here is non-temporal.  Not the stores: past the caches they are slower themselves, more so where rows are no whole 128-byte
 // lines, whose ends then leave in pieces, and the kernel that reads the rows next finds none of them in the last-level cache (us, non-temporal / plain:
 // 32768 rows of 4096 bytes to 6 x as many 190 / 162, of 4080 bytes, out of memory, 266 / 208; 16384 of 2048 bytes to 4 x as many 27.5 and the
-// combine that reads them 40.7 / 26.6 and 33.3; 57407 of 1088 bytes to twice as many 30.2 and 54.2 / 35.4 and 49.4).  Not the loads: the
-// tokens are a matrix that fits the last-level cache and that a kernel before or after this one touches as
+// combine that reads them 40.7 / 26.6 and 33.3 back to back, 28.3 and 35.6 / 29.3 and 32.1 among the other launches of a pass with its gradients;
+// 57407 of 1088 bytes to twice as many 30.2 and 54.2 / 35.4 and 49.4).  Not the loads: the tokens are a matrix that fits the last-level cache and that a kernel before or after this one touches as
 // well (the producer of the tokens, the router; in the backward pass the router-weight gradient reads the same rows of
 // the output gradient right afterwards), and a non-temporal load does not find them there (32768 rows of 4 KiB into
 // 6 x as many: 153 us from a hot source with plain loads, 187 us with non-temporal ones).
