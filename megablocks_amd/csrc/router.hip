@@ -396,15 +396,19 @@ sum_parts_kernel(const float* __restrict__ parts, int num_parts, int64_t pitch, 
 // workgroup's, a longer one is cut into runs of kLossRun for a workgroup each, whose sums a second launch adds in order.  What bounds the losses is the
 // number of launches and the calls behind them: as torch's operations the two are ten of 1 - 7 us forward and ten backward for a layer, each with a node of
 // its own (a step of 1024 tokens, 8 experts, the host in its slower mode: 825 us with them, 695 with these four); with a launch and a call for every layer
-// the z-loss of 32 took 1400 us of the host's time each way together, with one for all 1105, torch's operations 2166.
+// the z-loss of 32 took 1400 us of the host's time each way together, with one for all 1105, torch's operations 2166 (a faster host 487, torch's
+// 1602 - 1966; of 2 layers 134, torch's 177).
 constexpr int kLossThreads = 1024, kLossOneBlock = 32 * kLossThreads, kLossRun = 8 * kLossThreads, kLossParts = 256, kLossLayers = 64;
 
-struct LossLayers {   // of one launch, in its arguments
-  const void* values[kLossLayers];
-  const int32_t* counts[kLossLayers];
-  void* out[kLossLayers];   // the gradients
-  int64_t n[kLossLayers];
-  float scale[kLossLayers];
+// Of one launch, in its arguments: MOST is 1 or kLossLayers.  One layer has arguments of its own: with the 2.3 KB of those for many every launch of its step took
+// longer on the host (1024 tokens, 8 experts, medians of 12 processes: forward of the layer 280.0 -> 276.6 us, each loss 1.2 less).
+template <int MOST>
+struct LossLayers {
+  const void* values[MOST];
+  const int32_t* counts[MOST];
+  void* out[MOST];   // the gradients
+  int64_t n[MOST];
+  float scale[MOST];
 };
 
 __host__ __device__ constexpr int loss_blocks(int64_t n) {
@@ -420,8 +424,8 @@ __device__ __forceinline__ float block_sum(float v) {   // in thread 0
   return wave_sum(threadIdx.x < kLossThreads / kWave ? sums[threadIdx.x] : 0.f);
 }
 
-template <int DT>
-__global__ void __launch_bounds__(kLossThreads) loss_sum_kernel(const LossLayers layers, int period, float* __restrict__ out, float* __restrict__ parts) {
+template <int DT, int MOST>
+__global__ void __launch_bounds__(kLossThreads) loss_sum_kernel(const LossLayers<MOST> layers, int period, float* __restrict__ out, float* __restrict__ parts) {
   typedef typename Elem<DT>::type E;
   const int layer = blockIdx.y;
   const int64_t n = layers.n[layer];
@@ -447,7 +451,8 @@ __global__ void __launch_bounds__(kLossThreads) loss_sum_kernel(const LossLayers
   else parts[layer * kLossParts + blockIdx.x] = sum;
 }
 
-__global__ void __launch_bounds__(kLossThreads) loss_parts_kernel(const LossLayers layers, const float* __restrict__ parts, float* __restrict__ out) {
+template <int MOST>
+__global__ void __launch_bounds__(kLossThreads) loss_parts_kernel(const LossLayers<MOST> layers, const float* __restrict__ parts, float* __restrict__ out) {
   const int layer = blockIdx.x, blocks = loss_blocks(layers.n[layer]);
   if (blocks == 1) return;
   const float sum = block_sum((int)threadIdx.x < blocks ? parts[layer * kLossParts + threadIdx.x] : 0.f);
@@ -455,8 +460,8 @@ __global__ void __launch_bounds__(kLossThreads) loss_parts_kernel(const LossLaye
 }
 
 // The sums' gradients: grad scale counts[i % period], or without counts grad scale 2 values[i].
-template <int DT>
-__global__ void __launch_bounds__(256) loss_gradient_kernel(const float* __restrict__ grad, const LossLayers layers, int period) {
+template <int DT, int MOST>
+__global__ void __launch_bounds__(256) loss_gradient_kernel(const float* __restrict__ grad, const LossLayers<MOST> layers, int period) {
   typedef typename Elem<DT>::type E;
   const int layer = blockIdx.y;
   E* __restrict__ const out = (E*)layers.out[layer];
@@ -473,6 +478,51 @@ __global__ void __launch_bounds__(256) loss_gradient_kernel(const float* __restr
     out[i] = Elem<DT>::from_f32(counts ? g * (float)counts[e] : g * (2.f * Elem<DT>::to_f32(values[i])));
     e += step;
     e = e >= period ? e - period : e;
+  }
+}
+
+// A launch of up to MOST layers (two for long sums); parts: kLossParts floats a layer
+template <int MOST>
+static void launch_loss_sums(const void* const* values, int dtype, const int32_t* const* counts, const int64_t* n, const float* scales, int count, int period,
+                             float* out, float* parts, hipStream_t s) {
+  LossLayers<MOST> of = {};
+  int blocks = 1;
+  for (int l = 0; l < count; ++l) {
+    of.values[l] = values[l];
+    of.counts[l] = counts ? counts[l] : nullptr;
+    of.n[l] = n[l];
+    of.scale[l] = scales[l];
+    blocks = loss_blocks(n[l]) > blocks ? loss_blocks(n[l]) : blocks;
+  }
+  const dim3 grid((unsigned)blocks, (unsigned)count);
+  switch (dtype) {
+    case MBX_BF16: loss_sum_kernel<MBX_BF16, MOST><<<grid, kLossThreads, 0, s>>>(of, period, out, parts); break;
+    case MBX_F16: loss_sum_kernel<MBX_F16, MOST><<<grid, kLossThreads, 0, s>>>(of, period, out, parts); break;
+    default: loss_sum_kernel<MBX_F32, MOST><<<grid, kLossThreads, 0, s>>>(of, period, out, parts); break;
+  }
+  if (blocks > 1) loss_parts_kernel<MOST><<<(unsigned)count, kLossThreads, 0, s>>>(of, parts, out);
+}
+
+template <int MOST>
+static void launch_loss_gradients(const float* grad, const void* const* values, int dtype, const int32_t* const* counts, const int64_t* n, const float* scales,
+                                  int count, int period, void* const* out, hipStream_t s) {
+  LossLayers<MOST> of = {};
+  int64_t most = 0;
+  for (int l = 0; l < count; ++l) {
+    of.values[l] = counts ? nullptr : values[l];
+    of.counts[l] = counts ? counts[l] : nullptr;
+    of.out[l] = out[l];
+    of.n[l] = n[l];
+    of.scale[l] = scales[l];
+    if (out[l] && n[l] > most) most = n[l];
+  }
+  if (most == 0) return;
+  const int64_t wanted = ceil_div(most, 256);
+  const dim3 grid((unsigned)(wanted < 2048 ? wanted : 2048), (unsigned)count);
+  switch (dtype) {
+    case MBX_BF16: loss_gradient_kernel<MBX_BF16, MOST><<<grid, 256, 0, s>>>(grad, of, period); break;
+    case MBX_F16: loss_gradient_kernel<MBX_F16, MOST><<<grid, 256, 0, s>>>(grad, of, period); break;
+    default: loss_gradient_kernel<MBX_F32, MOST><<<grid, 256, 0, s>>>(grad, of, period); break;
   }
 }
 
@@ -627,28 +677,11 @@ int mbx_loss_sums(const void* const* values, int dtype, const int32_t* const* co
     if (n[l] < 0 || (n[l] > 0 && !values[l]) || (counts && n[l] > 0 && !counts[l])) return MBX_EINVAL;
     if (n[l] > kLossOneBlock && !scratch) return MBX_ESCRATCH;
   }
-  hipStream_t s = as_stream(stream);
-  for (int first = 0; first < layers; first += kLossLayers) {
-    LossLayers of = {};
-    const int count = layers - first < kLossLayers ? layers - first : kLossLayers;
-    int blocks = 1;
-    for (int l = 0; l < count; ++l) {
-      of.values[l] = values[first + l];
-      of.counts[l] = counts ? counts[first + l] : nullptr;
-      of.n[l] = n[first + l];
-      of.scale[l] = scales[first + l];
-      blocks = loss_blocks(of.n[l]) > blocks ? loss_blocks(of.n[l]) : blocks;
-    }
-    float* const to = out + first;
-    float* const parts = scratch ? scratch + (int64_t)first * kLossParts : nullptr;
-    const dim3 grid((unsigned)blocks, (unsigned)count);
-    switch (dtype) {
-      case MBX_BF16: loss_sum_kernel<MBX_BF16><<<grid, kLossThreads, 0, s>>>(of, period, to, parts); break;
-      case MBX_F16: loss_sum_kernel<MBX_F16><<<grid, kLossThreads, 0, s>>>(of, period, to, parts); break;
-      default: loss_sum_kernel<MBX_F32><<<grid, kLossThreads, 0, s>>>(of, period, to, parts); break;
-    }
-    if (blocks > 1) loss_parts_kernel<<<(unsigned)count, kLossThreads, 0, s>>>(of, parts, to);
-  }
+  if (layers == 1) launch_loss_sums<1>(values, dtype, counts, n, scales, 1, period, out, scratch, as_stream(stream));
+  else
+    for (int first = 0; first < layers; first += kLossLayers)
+      launch_loss_sums<kLossLayers>(values + first, dtype, counts ? counts + first : nullptr, n + first, scales + first, layers - first < kLossLayers ? layers - first : kLossLayers,
+                                    period, out + first, scratch ? scratch + (int64_t)first * kLossParts : nullptr, as_stream(stream));
   return launch_status();
 }
 
@@ -659,28 +692,11 @@ int mbx_loss_gradients(const float* grad, const void* const* values, int dtype, 
   if (!grad || !out || !n || !scales || (!counts && !values)) return MBX_EINVAL;
   for (int l = 0; l < layers; ++l)
     if (n[l] < 0 || (out[l] && n[l] > 0 && !(counts ? (const void*)counts[l] : values[l]))) return MBX_EINVAL;
-  hipStream_t s = as_stream(stream);
-  for (int first = 0; first < layers; first += kLossLayers) {
-    LossLayers of = {};
-    const int count = layers - first < kLossLayers ? layers - first : kLossLayers;
-    int64_t most = 0;
-    for (int l = 0; l < count; ++l) {
-      of.values[l] = counts ? nullptr : values[first + l];
-      of.counts[l] = counts ? counts[first + l] : nullptr;
-      of.out[l] = out[first + l];
-      of.n[l] = n[first + l];
-      of.scale[l] = scales[first + l];
-      if (of.out[l] && of.n[l] > most) most = of.n[l];
-    }
-    if (most == 0) continue;
-    const int64_t wanted = ceil_div(most, 256);
-    const dim3 grid((unsigned)(wanted < 2048 ? wanted : 2048), (unsigned)count);
-    switch (dtype) {
-      case MBX_BF16: loss_gradient_kernel<MBX_BF16><<<grid, 256, 0, s>>>(grad + first, of, period); break;
-      case MBX_F16: loss_gradient_kernel<MBX_F16><<<grid, 256, 0, s>>>(grad + first, of, period); break;
-      default: loss_gradient_kernel<MBX_F32><<<grid, 256, 0, s>>>(grad + first, of, period); break;
-    }
-  }
+  if (layers == 1) launch_loss_gradients<1>(grad, values, dtype, counts, n, scales, 1, period, out, as_stream(stream));
+  else
+    for (int first = 0; first < layers; first += kLossLayers)
+      launch_loss_gradients<kLossLayers>(grad + first, values ? values + first : nullptr, dtype, counts ? counts + first : nullptr, n + first, scales + first,
+                                         layers - first < kLossLayers ? layers - first : kLossLayers, period, out + first, as_stream(stream));
   return launch_status();
 }
 
